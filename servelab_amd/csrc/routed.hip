@@ -375,6 +375,90 @@ __global__ __launch_bounds__(64 * WR * WC) void grouped_product_mfma_kernel(cons
 }
 
 
+// Row tiles of 16 rows where an expert has few of them, bound by the stream of the experts' matrices: a
+// workgroup takes a row tile by 16 NU columns and its eight wavefronts cut K among themselves, so that the few
+// (expert, column block) pairs of such a step still put enough loads in flight on every CU (one token of 8
+// experts of 1,024 x 2,048 was 128 wavefronts that each walked all of K).  The partial sums meet in LDS and are
+// added in the order of K.  Two products and the combine, 64 experts of 1,024 over rows of 2,048, 8 a token,
+// at 1 / 2 / 4 / 8 / 32 tokens: 48 / 51 / 78 / 113 / 146 -> 23 / 39 / 58 / 89 / 128 us (5.5 TB/s at 8 tokens).
+// Four wavefronts or 64 columns a workgroup: 27 us at one token, 103 at 8.
+constexpr int FEW_WAVES = 8;
+template <int NU, bool GATED>
+__global__ __launch_bounds__(64 * FEW_WAVES) void grouped_product_few_kernel(const Grouped a) {
+  constexpr int KW = FEW_WAVES;
+  constexpr int MATS = GATED ? 2 : 1;
+  __shared__ rt_f32x4 part[KW][NU * MATS][64];
+  int tile, cb;
+  if (!grouped_place(a, tile, cb)) return;
+  const int* tl = a.tiles + 3 * tile;
+  const int rows = min(16, tl[2]);
+  const int n0 = cb * 16 * NU;
+  if (rows <= 0 || n0 >= a.N) return;                   // (the whole workgroup)
+  const int e = tl[0], row0 = tl[1];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x & 63, i = lane & 15, gq = lane >> 4;
+  const size_t n_w = GATED ? 2 * (size_t)a.N : (size_t)a.N;
+  const __bf16* we = a.w + (size_t)e * n_w * a.K;
+  const int rr = row0 + min(i, rows - 1);
+  const size_t src = a.order != nullptr ? (size_t)(a.order[rr] / a.top) : (size_t)rr;
+  const __bf16* xp = a.x + src * a.K + 8 * gq;
+  const __bf16* wp[NU];
+  const int wstep = a.w_tiled ? 512 : 32;               // elements from one k-step to the next
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    if (a.w_tiled) wp[u] = we + (size_t)(min(n0 + 16 * u, a.N - 16) / 16) * (a.K / 32) * 512 + lane * 8;
+    else wp[u] = we + (size_t)min(n0 + 16 * u + i, a.N - 1) * a.K + 8 * gq;
+  }
+  const size_t up = (size_t)a.N * a.K;
+  rt_f32x4 acc[NU * MATS];
+#pragma unroll
+  for (int u = 0; u < NU * MATS; ++u) acc[u] = rt_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = a.K / 32, s1 = steps * (wave + 1) / KW;
+#pragma unroll 4
+  for (int s = steps * wave / KW; s < s1; ++s) {
+    const rt_bf16x8 b = *(const rt_bf16x8*)(xp + 32 * s);
+    const size_t kw = (size_t)s * wstep;
+    rt_bf16x8 w[NU * MATS];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      w[u] = __builtin_nontemporal_load((const rt_bf16x8*)(wp[u] + kw));
+      if (GATED) w[NU + u] = __builtin_nontemporal_load((const rt_bf16x8*)(wp[u] + up + kw));
+    }
+#pragma unroll
+    for (int u = 0; u < NU * MATS; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], b, acc[u], 0, 0, 0);
+  }
+#pragma unroll
+  for (int u = 0; u < NU * MATS; ++u) part[wave][u][lane] = acc[u];
+  __syncthreads();
+  if (i >= rows) return;
+  const float rs = a.row_scale != nullptr ? a.row_scale[a.order[row0 + i]] : 1.f;
+  for (int u = wave; u < NU; u += KW) {
+    if (n0 + 16 * u >= a.N) continue;
+    rt_f32x4 v = part[0][u][lane];
+#pragma unroll
+    for (int w = 1; w < KW; ++w) v += part[w][u][lane];
+    v *= rs;
+    const size_t at = (size_t)(row0 + i) * a.N + n0 + 16 * u + 4 * gq;
+    if (GATED) {
+      rt_f32x4 z = part[0][NU + u][lane];
+#pragma unroll
+      for (int w = 1; w < KW; ++w) z += part[w][NU + u][lane];
+      z *= rs;
+      rt_bf16x4 r;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) r[c] = (__bf16)sl_gated(v[c], z[c], a.act, a.limit);
+      *(rt_bf16x4*)(a.out_act + at) = r;
+    } else if (a.act) {
+      rt_bf16x4 r;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) r[c] = (__bf16)sl_act(v[c], a.act);
+      *(rt_bf16x4*)(a.out_act + at) = r;
+    } else {
+      *(rt_f32x4*)(a.out_f32 + at) = v;
+    }
+  }
+}
+
+
 // Row tiles of 128 rows with the rows of x staged in LDS: a workgroup of four wavefronts takes a row
 // tile by 64 NU columns; every wavefront owns all 128 rows by 16 NU columns (of the gate and of the
 // up matrix in the gated form).  The tile's rows of x come 64 values of k at a time into one of two
@@ -499,8 +583,8 @@ __global__ __launch_bounds__(256, 2) void grouped_product_staged_kernel(const Gr
 #endif
 
 extern "C" const char* sl_grouped_product(const void* x, const int* order, int top, const void* w, const int* tiles,
-                                          int w_tiled, int max_tiles, int tile_rows, int N, int K, int gated,
-                                          int act, float limit, const float* row_scale, void* out, hipStream_t stream) {
+                                          int w_tiled, int max_tiles, int tile_rows, int pairs, int experts, int N,
+                                          int K, int gated, int act, float limit, const float* row_scale, void* out, hipStream_t stream) {
   // gated: act(gate) * up into the activation type; else act != 0: act(W x) into the activation type;
   // else plain float sums
   SL_CHECK(max_tiles >= 0 && N > 0 && K > 0 && top >= 1, "grouped_product: sizes must be positive");
@@ -508,7 +592,9 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
            "grouped_product: unknown activation, a gate without one, or the clamped form without a gate");
   SL_CHECK(row_scale == nullptr || order != nullptr, "grouped_product: factors per row go with the pairs' order");
   SL_CHECK(tile_rows == 16 || tile_rows == 64 || tile_rows == 128, "grouped_product: row tiles hold 16, 64 or 128 rows");
-  if (max_tiles == 0) return nullptr;
+  SL_CHECK(pairs >= 0 && experts >= 0, "grouped_product: sizes must be positive");
+  if (max_tiles == 0 || pairs == 0) return nullptr;
+  max_tiles = min(max_tiles, pairs);                    // (the tiles in use come first, and each holds a pair)
   Grouped a{(const act_t*)x, order, top, (const act_t*)w, w_tiled, tiles, tile_rows / RT_ROWS, N, K,
             act ? (act_t*)out : nullptr, act ? nullptr : (float*)out, act, limit, row_scale, max_tiles, 1};
 #if !defined(SL_F32)
@@ -527,6 +613,18 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
     } else if (tile_rows == 64) {
       if (gated) grouped_product_mfma_kernel<4, 4, true, 1, 4><<<blocks(256), 256, 0, stream>>>(a);
       else grouped_product_mfma_kernel<4, 4, false, 1, 4><<<blocks(256), 256, 0, stream>>>(a);
+    } else if (pairs <= 8 * (long long)experts) {
+      // (few rows an expert: the launch is bound by the matrices' stream, see the kernel.  Under six rows an
+      // expert every one of its tiles is narrow; from there on the rows of x, read again by every column block,
+      // count: 64 experts of 1,792, 8 rows each, 433 us in blocks of 16 columns and 400 in blocks of 32.  From
+      // twelve rows on it is the kernel below that is faster: 12 rows of the 2,048 x 1,024 experts 152 against 160 us.)
+      if (pairs < 6 * (long long)experts) {
+        if (gated) grouped_product_few_kernel<1, true><<<blocks(16), 64 * FEW_WAVES, 0, stream>>>(a);
+        else grouped_product_few_kernel<1, false><<<blocks(16), 64 * FEW_WAVES, 0, stream>>>(a);
+      } else {
+        if (gated) grouped_product_few_kernel<2, true><<<blocks(32), 64 * FEW_WAVES, 0, stream>>>(a);
+        else grouped_product_few_kernel<2, false><<<blocks(32), 64 * FEW_WAVES, 0, stream>>>(a);
+      }
     } else {
       if (gated) grouped_product_mfma_kernel<1, 4, true, 1, 1><<<blocks(64), 64, 0, stream>>>(a);
       else grouped_product_mfma_kernel<1, 4, false, 1, 1><<<blocks(64), 64, 0, stream>>>(a);

@@ -451,11 +451,11 @@ class RecurrentOps:
         lib = self._lazy("routed")
         mid = self._new((n, ff))
         self._call(lib, "sl_grouped_product", _p(x), _p(routing.order), top, _p(w_gate_up.data),
-                   _p(routing.tiles), int(w_gate_up.tiled), max_tiles, routing.tile_rows, ff, K, int(bool(gated)), code,
-                   _c_float(limit), _p(routing.shares) if weigh_input else None, _p(mid))
+                   _p(routing.tiles), int(w_gate_up.tiled), max_tiles, routing.tile_rows, n, E, ff, K, int(bool(gated)),
+                   code, _c_float(limit), _p(routing.shares) if weigh_input else None, _p(mid))
         y = self._new((n, K), torch.float32)
         self._call(lib, "sl_grouped_product", _p(mid), None, 1, _p(w_down.data), _p(routing.tiles),
-                   int(w_down.tiled), max_tiles, routing.tile_rows, K, ff, 0, 0, _c_float(0.0), None,
+                   int(w_down.tiled), max_tiles, routing.tile_rows, n, E, K, ff, 0, 0, _c_float(0.0), None,
                    _p(y))
         out = self._new((T, K))
         gate_at = None

@@ -1,0 +1,39 @@
+"""The grouped products where an expert has few rows, at the sizes where their split of K and their column blocks can
+go wrong, against the plain torch form (tests/emulated_ops.py)."""
+import pytest
+import torch
+
+from emulated_ops import EmulatedOps
+from servelab_amd.kernels import HipOps
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# (tokens, experts, top, ff, width): K of one step (seven of eight wavefronts without a share), of a number of steps that
+# eight does not divide, the last column block of 32 half empty, 6 and 8 rows an expert and just beyond, every token at the
+# same experts (tiles of 16 rows full, a second one with one row)
+@pytest.mark.parametrize("T,E,top,ff,K", [(1, 4, 2, 16, 32), (3, 8, 3, 48, 352), (6, 2, 2, 48, 96), (8, 4, 4, 80, 288),
+                                          (9, 4, 4, 80, 288), (17, 3, 1, 16, 64), (1, 64, 8, 1024, 2048)])
+@pytest.mark.parametrize("form", ["gated", "plain", "weighed input"])
+def test_few_rows_an_expert(T, E, top, ff, K, form):
+    hip, emu = HipOps(torch.bfloat16, DEV), EmulatedOps(torch.bfloat16)
+    g = torch.Generator().manual_seed(T + E)
+    gated = form != "plain"
+    x = torch.randn(T, K, generator=g).bfloat16()
+    first = (torch.randn(E, (2 if gated else 1) * ff, K, generator=g) * K ** -0.5).bfloat16()
+    down = (torch.randn(E, K, ff, generator=g) * ff ** -0.5).bfloat16()
+    logits = torch.randn(T, E, generator=g)
+    if T == 17:
+        logits[:, 1] += 20.0
+    r = hip.route_tokens(logits.to(DEV), E, top, sigmoid=form == "weighed input")
+    assert r.tile_rows == 16
+    options = dict(activation="silu" if gated else "relu2", gated=gated, weigh_input=form == "weighed input")
+    want = emu.routed_experts(x, (r.chosen.cpu(), r.shares.cpu()), first, down, None, **options)
+    for a, b in ((first.to(DEV), down.to(DEV)),
+                 (hip.prepare_expert_matrices(first.to(DEV), gated=gated), hip.prepare_expert_matrices(down.to(DEV)))):
+        got = hip.routed_experts(x.to(DEV), r, a, b, None, **options).float().cpu()
+        # float sums in another order (2^-24 sqrt(K) of a sum) may round either way where the activation type is 2^-8
+        # wide: at most three roundings (the activated row, its product, the result) of a value of this size
+        bar = 3 * 2.0 ** -8 * want.float().abs().max().item()
+        assert (got - want.float()).abs().max().item() <= bar
