@@ -450,6 +450,7 @@ struct MatrixScan {
   const int* slots;
   int write;
   float* out;                // [T][H][Dv]
+  float* normaliser;         // matrix LSTM: [S][H][D + 1], the new n and m until every block has read the old ones
 };
 
 enum { SCAN_DECAY = 0, SCAN_DELTA = 1, SCAN_LSTM = 2, SCAN_SSD = 3, SCAN_FORGET = 4, SCAN_DELTA_HEAD = 5 };
@@ -639,7 +640,8 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
       const int rounds = (last - first + CH - 1) / CH + 1;
       flush(rounds, first + rounds * CH);
     }
-    if (MODE == SCAN_LSTM && a.write && slice == 0 && tid == 0) *mcell = m;
+    if (MODE == SCAN_LSTM && a.write && slice == 0 && tid == 0)
+      a.normaliser[((size_t)s * a.H + h) * (a.D + 1) + a.D] = m;
     return;
   }
 
@@ -743,7 +745,14 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
     }
     __syncthreads();                      // chunk c + 1 is in LDS, chunk c's half is free
   }
-  if (a.write && (!is_n || slice == 0)) {             // (every slice carries the same n: the first writes it)
+  if (a.write && is_n) {
+    // every slice carries the same n and reads the old one when it starts, which may be after the first slice
+    // has ended: the new one waits beside the slots for normaliser_kernel
+    if (slice == 0)
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i)
+        if (r0 + i < a.D) a.normaliser[((size_t)s * a.H + h) * (a.D + 1) + r0 + i] = S[i];
+  } else if (a.write) {
     if (whole) {
 #pragma unroll
       for (int u = 0; u < ROWS / 4; ++u) {
@@ -761,12 +770,23 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
   }
 }
 
+// The matrix LSTM's n and m to their slots, behind the scan whose blocks have all read the old ones.
+__global__ void normaliser_kernel(const MatrixScan a) {
+  const int s = blockIdx.x, h = blockIdx.y;
+  float* slot = a.state + (size_t)a.slots[s] * a.state_stride + (size_t)a.H * a.Dv * a.D;
+  const float* from = a.normaliser + ((size_t)s * a.H + h) * (a.D + 1);
+  for (int d = threadIdx.x; d < a.D; d += blockDim.x) slot[(size_t)h * a.D + d] = from[d];
+  if (threadIdx.x == 0) slot[(size_t)a.H * a.D + h] = from[a.D];
+}
+
 extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride, int q_col, int k_col, int v_col,
                                       int H, int G, int D, int Dv, const float* log_decay, float q_scale,
                                       const float* gates, int gate_stride, int i_col, int f_col, float cap,
                                       const float* rates, const float* step_bias, const float* skip, const float* lower, float* state, long long state_stride,
                                       const int* cu_q, const int* positions,
-                                      const int* slots, int S, int T, int write, float* out, hipStream_t stream) {
+                                      const int* slots, int S, int T, int write, float* normaliser, float* out,
+                                      hipStream_t stream) {
+  SL_CHECK(mode != SCAN_LSTM || !write || normaliser != nullptr, "matrix_scan: room for the new normalisers is missing");
   SL_CHECK(mode >= 0 && mode <= 5, "matrix_scan: unknown mode");
   SL_CHECK(S >= 0 && T >= 0 && H > 0 && G > 0 && H % G == 0 && Dv > 0, "matrix_scan: sizes must be positive");
   SL_CHECK(D >= 1 && D <= 64 * SCAN_ROWS, "matrix_scan: at most 512 key channels a head");
@@ -795,7 +815,7 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   const bool scalar = mode == SCAN_LSTM || mode == SCAN_SSD || mode == SCAN_DELTA_HEAD;
   const size_t lds = 2 * (size_t)CH * ((scalar ? 2 : 3) * Dp + 2 * cols + 4) * sizeof(float);   // two halves
   const MatrixScan a{src, src_stride, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, gates, gate_stride,
-                     i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out};
+                     i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out, normaliser};
   const int vcols = mode == SCAN_LSTM ? cols - 1 : cols;       // (the matrix LSTM's last column group carries n)
   const dim3 grid(S, H, (Dv + vcols - 1) / vcols);
   if (mode == SCAN_DECAY) matrix_scan_kernel<SCAN_DECAY, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);
@@ -803,7 +823,10 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   else if (mode == SCAN_SSD) matrix_scan_kernel<SCAN_SSD, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);
   else if (mode == SCAN_DELTA_HEAD) matrix_scan_kernel<SCAN_DELTA_HEAD, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);
   else if (mode == SCAN_FORGET) matrix_scan_kernel<SCAN_FORGET, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);
-  else matrix_scan_kernel<SCAN_LSTM, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);
+  else {
+    matrix_scan_kernel<SCAN_LSTM, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);
+    if (write) normaliser_kernel<<<dim3(S, H), 64, 0, stream>>>(a);
+  }
   return sl_launch_status();
 }
 

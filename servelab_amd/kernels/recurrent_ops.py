@@ -180,11 +180,12 @@ class RecurrentOps:
             if gates.shape[0] != T:
                 raise KernelError("gates for another number of tokens")
         out = self._new((T, H * Dv), torch.float32)
+        normaliser = self._new((batch.num_seqs, H, D + 1), torch.float32) if mode == _SCAN_LSTM and write else None
         self._call(self._lazy("recurrent"), "sl_matrix_scan", mode, _p(src), stride, q_col, k_col, v_col, H, G,
                    D, Dv, _p(log_decay), _c_float(q_scale), _p(gates), gate_stride, i_col, f_col, _c_float(cap),
                    _p(rates), _p(step_bias), _p(skip), _p(lower), _p(state), _ll(slot_size), _p(batch.cu_q),
                    _p(batch.positions), _p(batch.state_slots),
-                   batch.num_seqs, T, int(bool(write)), _p(out))
+                   batch.num_seqs, T, int(bool(write)), _p(normaliser), _p(out))
         return out
 
     def decay_scan(self, src, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, beta_src, beta_col,
