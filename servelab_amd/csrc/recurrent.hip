@@ -779,13 +779,21 @@ __global__ void normaliser_kernel(const MatrixScan a) {
   if (threadIdx.x == 0) slot[(size_t)a.H * a.D + h] = from[a.D];
 }
 
+#include "scan_chunks.h"
+
+// Floats of the workspace that a step of T tokens in S sequences needs to be walked in chunks; 0: it cannot be.
+extern "C" long long sl_matrix_scan_workspace(int mode, int T, int S, int H, int G, int D, int Dv) {
+  return scan_chunks_layout(mode, T, S, H, G, D, Dv, nullptr, nullptr);
+}
+
+// workspace: walked in chunks (max_len: tokens of the longest sequence); nullptr: token by token.
 extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride, int q_col, int k_col, int v_col,
                                       int H, int G, int D, int Dv, const float* log_decay, float q_scale,
                                       const float* gates, int gate_stride, int i_col, int f_col, float cap,
                                       const float* rates, const float* step_bias, const float* skip, const float* lower, float* state, long long state_stride,
                                       const int* cu_q, const int* positions,
-                                      const int* slots, int S, int T, int write, float* normaliser, float* out,
-                                      hipStream_t stream) {
+                                      const int* slots, int S, int T, int write, float* normaliser, float* workspace,
+                                      int max_len, float* out, hipStream_t stream) {
   SL_CHECK(mode != SCAN_LSTM || !write || normaliser != nullptr, "matrix_scan: room for the new normalisers is missing");
   SL_CHECK(mode >= 0 && mode <= 5, "matrix_scan: unknown mode");
   SL_CHECK(S >= 0 && T >= 0 && H > 0 && G > 0 && H % G == 0 && Dv > 0, "matrix_scan: sizes must be positive");
@@ -805,6 +813,23 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   const long long need = (long long)H * Dv * D + (mode == SCAN_LSTM ? (long long)H * D + H : 0);
   SL_CHECK(need <= state_stride, "matrix_scan: the state does not fit its slot");
   if (S == 0 || T == 0) return nullptr;
+  if (workspace != nullptr) {
+    SL_CHECK((uintptr_t)workspace % 16 == 0, "matrix_scan: the workspace must be aligned");
+    SL_CHECK(max_len >= 1 && max_len <= T, "matrix_scan: the longest sequence does not fit the step");
+    const MatrixScan a{src, src_stride, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, gates, gate_stride,
+                       i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out, normaliser};
+    ScanChunks c;
+    SL_CHECK(scan_chunks_layout(mode, T, S, H, G, D, Dv, workspace, &c) > 0, "matrix_scan: at most 256 key channels a head in chunks");
+    const char* err = mode == SCAN_DECAY ? scan_in_chunks<SCAN_DECAY>(a, c, S, max_len, stream) :
+                      mode == SCAN_DELTA ? scan_in_chunks<SCAN_DELTA>(a, c, S, max_len, stream) :
+                      mode == SCAN_SSD ? scan_in_chunks<SCAN_SSD>(a, c, S, max_len, stream) :
+                      mode == SCAN_DELTA_HEAD ? scan_in_chunks<SCAN_DELTA_HEAD>(a, c, S, max_len, stream) :
+                      mode == SCAN_FORGET ? scan_in_chunks<SCAN_FORGET>(a, c, S, max_len, stream) :
+                                            scan_in_chunks<SCAN_LSTM>(a, c, S, max_len, stream);
+    if (err != nullptr) return err;
+    if (mode == SCAN_LSTM && write) normaliser_kernel<<<dim3(S, H), 64, 0, stream>>>(a);
+    return sl_launch_status();
+  }
   // (A lane owning 4 key channels instead of 8 doubles the blocks of a lone prompt and halves a lane's
   // products; measured, a token takes as long: its cost is the sums across lanes, the hand-over and
   // the waits, not the products.)

@@ -45,6 +45,13 @@ class ExpertMatrices:
 
 class RecurrentOps:
     SELECTIVE_SEGMENT = 64        # tokens of a segment of the selective scan
+    # The matrix recurrences are walked in chunks of 32 tokens (scan_chunks.h), not token by token, from this many
+    # tokens of a step's longest sequence on: the chunks' own kernels cost 20 to 30 us however short a sequence is, a
+    # token 0.2 to 0.35 us (heads of 128 x 256: 64 tokens 21 us either way, 96: 27 against 23, 256: 58 against 29).  The
+    # state-space form, whose groups of heads are prepared one head after the other, from twice as many (128
+    # tokens 35 against 40 us, 192: 50 against 45).  Several sequences keep the chip busier: eight of 64 tokens
+    # 51 against 41 us, eight of 32: 34 against 35.
+    SCAN_CHUNKS_FROM, SCAN_CHUNKS_FROM_GROUPED, SCAN_CHUNKS_FROM_MANY, SCAN_MANY_TOKENS = 80, 160, 48, 400
     ROUTED_WIDE_TILE_ROWS = 48    # rows an expert has on average from which row tiles hold 64 rows
 
     # ------------------------------------------------- norm on an output
@@ -181,11 +188,19 @@ class RecurrentOps:
                 raise KernelError("gates for another number of tokens")
         out = self._new((T, H * Dv), torch.float32)
         normaliser = self._new((batch.num_seqs, H, D + 1), torch.float32) if mode == _SCAN_LSTM and write else None
-        self._call(self._lazy("recurrent"), "sl_matrix_scan", mode, _p(src), stride, q_col, k_col, v_col, H, G,
+        lib = self._lazy("recurrent")
+        workspace, longest = None, int(getattr(batch, "max_q_len", T))
+        alone = self.SCAN_CHUNKS_FROM_GROUPED if mode == _SCAN_SSD else self.SCAN_CHUNKS_FROM
+        if longest >= (alone if T < self.SCAN_MANY_TOKENS else min(alone, self.SCAN_CHUNKS_FROM_MANY)):
+            size = self._lib[lib].sl_matrix_scan_workspace
+            size.restype = ctypes.c_longlong
+            floats = size(mode, T, batch.num_seqs, H, G, D, Dv)
+            workspace = self._new((floats,), torch.float32) if floats else None
+        self._call(lib, "sl_matrix_scan", mode, _p(src), stride, q_col, k_col, v_col, H, G,
                    D, Dv, _p(log_decay), _c_float(q_scale), _p(gates), gate_stride, i_col, f_col, _c_float(cap),
                    _p(rates), _p(step_bias), _p(skip), _p(lower), _p(state), _ll(slot_size), _p(batch.cu_q),
                    _p(batch.positions), _p(batch.state_slots),
-                   batch.num_seqs, T, int(bool(write)), _p(normaliser), _p(out))
+                   batch.num_seqs, T, int(bool(write)), _p(normaliser), _p(workspace), longest, _p(out))
         return out
 
     def decay_scan(self, src, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, beta_src, beta_col,

@@ -46,3 +46,102 @@ def test_normalisers_of_a_full_decode_batch():
     # 128 products of a head's read-out, over a divisor that is at least 1e-6 and mostly near one
     close(o1, o2, 2e-5)
     close(s1, s2, 2e-5)
+
+
+Q_LENS, STARTS, SLOTS = [1, 31, 32, 33, 7, 100, 64], [0, 5, 0, 7, 300, 0, 9], [4, 0, 5, 2, 1, 6, 3]
+
+
+def scan_case(mode, H, G, D, Dv, strong):
+    """The call of ``mode`` on seeded inputs: (function of a kernel table, a state and a batch on a device) and the slot size."""
+    g = torch.Generator().manual_seed(H * D + Dv)
+    T = sum(Q_LENS)
+    width = 2 * G * D + H * Dv
+    src = torch.randn(T, width, generator=g)
+    if "delta" in mode:                                    # (unit vectors, as the convolution in front of it makes them)
+        heads = src[:, :2 * G * D].view(T, 2 * G, D)
+        src[:, :2 * G * D] = (heads / heads.norm(dim=-1, keepdim=True)).flatten(1)
+    gates = torch.randn(T, 2 * H, generator=g) * (4.0 if strong else 1.0)
+    rates = torch.log(1.0 + 15.0 * torch.rand(H, generator=g))
+    bias = torch.full((H,), 2.0 if strong else -3.0)
+    log_decay = -torch.rand(T, H * D, generator=g) * (12.0 if strong else 0.1)
+    if strong:
+        log_decay[torch.rand(T, H * D, generator=g) < 0.05] = -1e4
+    lower = torch.zeros(H * D) if strong else torch.rand(H * D, generator=g) * 0.9
+    cols = (0, G * D, 2 * G * D)
+
+    def call(ops, state, batch, device):
+        d = lambda t: t.to(device)
+        if mode == "decay":
+            return ops.decay_scan(d(src), *cols, H, G, D, Dv, d(log_decay), 0.7, None, 0, state, batch, True)
+        if mode == "delta":
+            return ops.decay_scan(d(src), *cols, H, G, D, Dv, d(log_decay), 0.7, d(gates), H, state, batch, True)
+        if mode == "delta, decay a head":
+            return ops.head_delta_scan(d(src), *cols, H, G, D, Dv, d(gates), 0, H, d(rates), d(bias), state, batch, True)
+        if mode == "state space":
+            return ops.ssd_scan(d(src), 2 * G * D, G * D, 0, H, G, D, Dv, d(gates), H, d(rates), d(bias), d(rates), state,
+                                batch, True)
+        if mode == "forget":
+            z = src.clone()
+            z[:, G * D:2 * G * D] *= 30.0 if strong else 1.0
+            return ops.forget_scan(d(z), 0, G * D, 2 * G * D, H, D, Dv, d(lower), state, batch, True, q_scale=0.5)
+        buf = torch.cat([src, gates], 1)
+        return ops.mlstm_scan(d(buf), *cols, width, width + H, H, D, Dv, 15.0, D ** -0.5, state, batch, True)
+    return call, H * D * Dv + (H * D + H if mode == "lstm" else 0), torch.cat([src, gates], 1)
+
+
+def lstm_read_outs(buf, state, H, D, Dv):
+    """The matrix LSTM's read-outs in float64 and what their errors are measured by: with o = N / d, N = S^T q and d = |n q|
+    or more, the terms that are added up for N over d, and o times those for n q over d (n q may cancel)."""
+    buf, state = buf.double(), torch.nan_to_num(state.double())
+    width, out, scale = 2 * H * D + H * Dv, [], []
+    at = 0
+    for n_tok, start, slot in zip(Q_LENS, STARTS, SLOTS):
+        row = state[slot] * (start > 0)
+        S, n, m = row[:H * D * Dv].view(H, Dv, D).transpose(1, 2), row[H * D * Dv:H * D * Dv + H * D].view(H, D), \
+            row[H * D * Dv + H * D:H * D * Dv + H * D + H]
+        for t in range(at, at + n_tok):
+            q, k, v = buf[t, :H * D].view(H, D) * D ** -0.5, buf[t, H * D:2 * H * D].view(H, D), buf[t, 2 * H * D:width].view(H, Dv)
+            i = 15 * torch.tanh(buf[t, width:width + H] / 15)
+            f = torch.nn.functional.logsigmoid(15 * torch.tanh(buf[t, width + H:width + 2 * H] / 15))
+            new = torch.maximum(f + m, i)
+            keep, add, m = torch.exp(f + m - new), torch.exp(i - new), new
+            S = keep[:, None, None] * S + add[:, None, None] * k[:, :, None] * v[:, None, :]
+            n = keep[:, None] * n + add[:, None] * k
+            d = torch.maximum((n * q).sum(-1).abs(), torch.exp(-m))[:, None] + 1e-6
+            o = (S * q[:, :, None]).sum(1) / d
+            out.append(o.flatten())
+            scale.append(((S * q[:, :, None]).abs().sum(1) / d + o.abs() * (n * q).abs().sum(-1)[:, None] / d).flatten())
+        at += n_tok
+    return torch.stack(out), torch.stack(scale)
+
+
+# heads of one, two, three and four blocks of 64 key channels, odd sizes, value channels that no slice divides
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 2, 128, 256), (3, 3, 20, 24), (2, 2, 72, 15), (1, 1, 200, 33), (2, 1, 256, 16), (4, 2, 64, 40)])
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("mode", ["decay", "delta", "delta, decay a head", "state space", "forget", "lstm"])
+def test_scan_in_chunks(mode, strong, H, G, D, Dv):
+    """Sequences of one token up to several chunks, at their starts (their slots hold NaN) and going on, with weak decays and with
+    ones that end a state at once."""
+    if mode in ("forget", "lstm"):
+        G = H
+    hip, emu = HipOps(torch.float32, DEV), EmulatedOps(torch.float32)
+    hip.SCAN_CHUNKS_FROM = hip.SCAN_CHUNKS_FROM_GROUPED = hip.SCAN_CHUNKS_FROM_MANY = 1
+    call, size, buf = scan_case(mode, H, G, D, Dv, strong)
+    g = torch.Generator().manual_seed(5)
+    state = torch.randn(len(SLOTS), size + 3, generator=g) * 0.3
+    for slot, start in zip(SLOTS, STARTS):
+        if start == 0:
+            state[slot] = float("nan")
+    s1, s2 = state.clone().to(DEV), state.clone()
+    o1 = call(hip, s1, sequences(Q_LENS, STARTS, SLOTS, DEV), DEV)
+    host = sequences(Q_LENS, STARTS, SLOTS, "cpu")
+    host.q_lens, host.starts = Q_LENS, STARTS
+    o2 = call(emu, s2, host, "cpu")
+    # both sides are float32: sums of up to 256 + 32 terms a chunk, as in the tests of the walk token by token
+    if mode == "lstm":                                     # (2^-24 a rounding, chains of at most 64 of them on either side of the /)
+        want, scale = lstm_read_outs(buf, state, H, D, Dv)
+        assert ((o1.cpu().double() - want).abs() <= 1e-6 + 64 * 2.0 ** -24 * scale).all()
+    else:
+        close(o1, o2, 2e-5)
+    close(s1[:, :size], s2[:, :size], 2e-5)
+    assert torch.equal(torch.nan_to_num(s1.cpu()[:, size:], 9.0), torch.nan_to_num(state[:, size:], 9.0))
