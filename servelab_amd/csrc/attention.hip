@@ -116,6 +116,8 @@ __global__ __launch_bounds__(64) void attention_general_kernel(
 // them together and every key row and value column is fetched once for all of
 // them (the kernel above fetches it once per head).
 constexpr int GROUP_HEADS = 8;
+constexpr int PIECE = 16 / sizeof(act_t);
+struct __attribute__((aligned(16))) att_piece { act_t v[PIECE]; };
 
 __global__ __launch_bounds__(64) void attention_general_group_kernel(
     const act_t* __restrict__ qkv, int row_stride, const act_t* __restrict__ kc,
@@ -132,6 +134,7 @@ __global__ __launch_bounds__(64) void attention_general_group_kernel(
   const int s = tok_seq[t], p = positions[t];
   const int lo = window > 0 ? (p - window + 1 > 0 ? p - window + 1 : 0) : 0;
   const int* table = block_tables + (size_t)s * max_pages;
+  const bool aligned = ((uintptr_t)kc | (uintptr_t)vc) % 16 == 0, whole = aligned && D % PIECE == 0;
   for (int idx = lane; idx < GROUP_HEADS * D; idx += 64)      // rows past nheads: zeros, results never stored
     qs[idx / D][idx % D] = idx / D < nheads
         ? to_f(qkv[(size_t)t * row_stride + (size_t)(h0 + idx / D) * D + idx % D]) : 0.f;
@@ -157,10 +160,22 @@ __global__ __launch_bounds__(64) void attention_general_group_kernel(
     if (valid) {
       const int pg = table[r / page];
       const act_t* kr = kc + (((size_t)pg * nkv + kvh) * page + r % page) * D;
-      for (int d = 0; d < D; ++d) {
-        const float kv = to_f(kr[d]);
+      // (rows of whole 16-byte pieces: a lane's row is its own, so its loads are as wide as they can be, eight in flight)
+      if (whole) {
+#pragma unroll 8
+        for (int d = 0; d < D; d += PIECE) {
+          const att_piece kv = *(const att_piece*)(kr + d);
 #pragma unroll
-        for (int h = 0; h < GROUP_HEADS; ++h) dot[h] += qs[h][d] * kv;
+          for (int j = 0; j < PIECE; ++j)
+#pragma unroll
+            for (int h = 0; h < GROUP_HEADS; ++h) dot[h] += qs[h][d + j] * to_f(kv.v[j]);
+        }
+      } else {
+        for (int d = 0; d < D; ++d) {
+          const float kv = to_f(kr[d]);
+#pragma unroll
+          for (int h = 0; h < GROUP_HEADS; ++h) dot[h] += qs[h][d] * kv;
+        }
       }
     }
     float alpha[GROUP_HEADS];
@@ -190,10 +205,22 @@ __global__ __launch_bounds__(64) void attention_general_group_kernel(
         const int d = lane + 64 * i;
         if (d < D) {
           const act_t* vr = vbase + (size_t)d * page;
-          for (int j = 0; j < page; ++j) {
-            const float v = to_f(vr[j]);
+          // (a channel's keys of a page lie together: pages of 16, 32 or 64 keys are whole pieces)
+          if (aligned) {
+#pragma unroll 4
+            for (int j = 0; j < page; j += PIECE) {
+              const att_piece v = *(const att_piece*)(vr + j);
 #pragma unroll
-            for (int h = 0; h < GROUP_HEADS; ++h) acc[h][i] += ps[h][pb + j] * v;
+              for (int e = 0; e < PIECE; ++e)
+#pragma unroll
+                for (int h = 0; h < GROUP_HEADS; ++h) acc[h][i] += ps[h][pb + j + e] * to_f(v.v[e]);
+            }
+          } else {
+            for (int j = 0; j < page; ++j) {
+              const float v = to_f(vr[j]);
+#pragma unroll
+              for (int h = 0; h < GROUP_HEADS; ++h) acc[h][i] += ps[h][pb + j] * v;
+            }
           }
         }
       }
@@ -401,6 +428,147 @@ __global__ __launch_bounds__(TILE_THREADS) void attention_general_tile_kernel(
     if (j < nd16) o[16 * j] = from_f<act_t>(acc[j] * inv);
 }
 
+#if defined(SL_F32)
+// ---------------------------------------------------------------------------
+// Prompt portions in float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 factors and sums), for head sizes in
+// steps of 16 fixed at compile time.  A workgroup of four wavefronts owns 64 columns, (token, head of the group) pairs of
+// one sequence and one kv head, a wavefront 16 of them, and walks blocks of 32 keys, staged in LDS as K [32][D + 4] and
+// V^T [D][36]; the next block travels from the pages to registers meanwhile.  S^T = K Q^T, softmax with a running
+// maximum per column, O^T += V^T P^T: a lane's scores of a 16 x 16 block (keys 4 (lane / 16) .. + 3 of column lane % 16) are the
+// second product's operand as they are.  What bounds it is the matrix instructions: 1.05 MFLOP a block and workgroup at
+// D 128, 0.6 TFLOP/s a CU.  One prompt of 333 tokens and two shorter ones, 12 heads on 2, D 128: 287 us with the FMA tiles.
+// ---------------------------------------------------------------------------
+typedef float att_v4 __attribute__((ext_vector_type(4)));
+
+template <int D>
+__global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
+    const float* __restrict__ qkv, int row_stride, const float* __restrict__ kc, const float* __restrict__ vc,
+    const int* __restrict__ block_tables, int max_pages, const int* __restrict__ cu_q, const int* __restrict__ positions,
+    int nh, int nkv, int page, float scale, int window, float* __restrict__ out) {
+  constexpr int KR = D + 4, VR = 36, NP = D / 32;      // row lengths; 16-byte pieces of K and of V^T a thread stages of a block
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* ks = lds;                                     // [32][KR]
+  float* vt = ks + 32 * KR;                            // [D][VR]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, gq = lane >> 4;
+  const int seq = blockIdx.z, kvh = blockIdx.y, g = nh / nkv;
+  const int q0 = cu_q[seq], qlen = cu_q[seq + 1] - q0, ncols = qlen * g;
+  // (tiles of late tokens see the most keys: they come first)
+  const int tile = (int)gridDim.x - 1 - (int)blockIdx.x, c0 = tile * 64;
+  if (c0 >= ncols) return;
+  const int pos0 = positions[q0];
+  const int* table = block_tables + (size_t)seq * max_pages;
+  const int c_last = min(c0 + 63, ncols - 1);
+  const int kmax = pos0 + c_last / g;
+  const int kmin = window > 0 ? max(0, pos0 + c0 / g - window + 1) : 0;
+  const int cw = c0 + 16 * wave;
+  const bool wave_live = cw < ncols;
+  const int c = min(cw + n, ncols - 1);                // (a column past the last is computed like the last, never stored)
+  const int tok = c / g, head = kvh * g + c % g, pos_c = pos0 + tok;
+  const int lo_c = window > 0 ? max(0, pos_c - window + 1) : 0;
+  att_v4 qf[D / 16];
+  {
+    const float* q = qkv + (size_t)(q0 + tok) * row_stride + (size_t)head * D + 4 * gq;
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) qf[j] = *(const att_v4*)(q + 16 * j);
+  }
+  att_v4 o[D / 16];
+#pragma unroll
+  for (int j = 0; j < D / 16; ++j) o[j] = att_v4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  att_v4 kr[NP], vr[NP];
+  // Keys outside [kmin, kmax] are staged as zeros: a slot that holds no visible key, or a released page, may hold anything.
+  auto fetch = [&](int kbase) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int idx = tid + 256 * i;
+      const int key = kbase + idx / (D / 4), d4 = idx % (D / 4);
+      kr[i] = att_v4{0.f, 0.f, 0.f, 0.f};
+      if (key >= kmin && key <= kmax)
+        kr[i] = *(const att_v4*)(kc + (((size_t)table[key / page] * nkv + kvh) * page + key % page) * D + 4 * d4);
+      const int d = idx / 8, key0 = kbase + 4 * (idx % 8);
+      vr[i] = att_v4{0.f, 0.f, 0.f, 0.f};
+      if (key0 + 3 >= kmin && key0 <= kmax) {          // (page sizes are multiples of 16: four keys share a page)
+        vr[i] = *(const att_v4*)(vc + (((size_t)table[key0 / page] * nkv + kvh) * D + d) * page + key0 % page);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (key0 + e < kmin || key0 + e > kmax) vr[i][e] = 0.f;
+      }
+    }
+  };
+  const int b0 = kmin / 32, b1 = kmax / 32;
+  fetch(32 * b0);
+  for (int b = b0; b <= b1; ++b) {
+    const int kbase = 32 * b;
+    __syncthreads();                                   // the last block's readers are done
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int idx = tid + 256 * i;
+      *(att_v4*)(ks + (idx / (D / 4)) * KR + 4 * (idx % (D / 4))) = kr[i];
+      *(att_v4*)(vt + (idx / 8) * VR + 4 * (idx % 8)) = vr[i];
+    }
+    __syncthreads();
+    if (b < b1) fetch(kbase + 32);
+    if (!wave_live) continue;                          // (a wavefront without columns only helps staging)
+    att_v4 s[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      att_v4 sum[2] = {};
+      const float* kp = ks + (16 * kt + n) * KR + 4 * gq;
+#pragma unroll
+      for (int j = 0; j < D / 16; ++j) {
+        const att_v4 kv = *(const att_v4*)(kp + 16 * j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], qf[j][i], sum[j & 1], 0, 0, 0);
+      }
+      s[kt] = sum[0] + sum[1];
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = kbase + 16 * kt + 4 * gq + i;
+        s[kt][i] = key >= lo_c && key <= pos_c ? s[kt][i] * scale : -INFINITY;
+        top = fmaxf(top, s[kt][i]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float mn = fmaxf(m, top);
+    // a column that has seen no key yet keeps m = -inf: nothing to rescale, nothing to add
+    const float alpha = mn == -INFINITY ? 1.f : expf(m - mn);
+    float psum = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kt][i] = s[kt][i] == -INFINITY ? 0.f : expf(s[kt][i] - mn);
+        psum += s[kt][i];
+      }
+    l = l * alpha + psum;                              // (this lane's keys; the column's four lanes are added at the end)
+    m = mn;
+#pragma unroll
+    for (int dd = 0; dd < D / 16; ++dd) {
+      att_v4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        const att_v4 vv = *(const att_v4*)(vt + (16 * dd + n) * VR + 16 * kt + 4 * gq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], s[kt][i], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[dd][i] = fmaf(o[dd][i], alpha, acc[i]);
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (cw + n >= ncols) return;
+  const float inv = 1.f / l;
+  float* to = out + ((size_t)(q0 + tok) * nh + head) * D + 4 * gq;
+#pragma unroll
+  for (int dd = 0; dd < D / 16; ++dd) *(att_v4*)(to + 16 * dd) = o[dd] * inv;
+}
+#endif
+
 // Sequences [0, num_seqs) of the batch, prompt portions of at most max_q_len
 // tokens each (their tokens come first in the batch).  D % 16 == 0.
 extern "C" const char* sl_attention_general_tiles(
@@ -418,6 +586,21 @@ extern "C" const char* sl_attention_general_tiles(
   const long long tiles = (cols + TILE_COLS - 1) / TILE_COLS;
   SL_CHECK(tiles <= 1 << 30, "attention tiles: too many column tiles");
   const dim3 grid((unsigned)tiles, nkv, num_seqs);
+#if defined(SL_F32)
+  // (head sizes of the shapes served; from 32 columns on a tile of 64 is filled well enough to win at every length measured)
+  if ((D == 64 || D == 128) && cols >= 32 && row_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)kc % 16 == 0 &&
+      (uintptr_t)vc % 16 == 0 && (uintptr_t)out % 16 == 0) {
+    const dim3 wide((unsigned)((cols + 63) / 64), nkv, num_seqs);
+    const size_t room = sizeof(float) * ((size_t)32 * (D + 4) + (size_t)D * 36);
+    auto run = [&](auto kernel) {
+      kernel<<<wide, 256, room, stream>>>((const float*)qkv, row_stride, (const float*)kc, (const float*)vc, block_tables,
+                                          max_pages, cu_q, positions, nh, nkv, page, scale, window, (float*)out);
+    };
+    if (D == 64) run(attention_f32_mfma_kernel<64>);
+    else run(attention_f32_mfma_kernel<128>);
+    return sl_launch_status();
+  }
+#endif
   const int KB = D <= 128 ? 32 : 16;
   const size_t bytes = sizeof(float) * ((size_t)TILE_COLS * D + (size_t)KB * (D + 4) + (size_t)KB * (D + 1) +
                                         (size_t)TILE_COLS * KB);

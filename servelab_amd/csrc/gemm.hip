@@ -72,6 +72,76 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(
   }
 }
 
+#if defined(SL_F32)
+// The same with K cut among the four wavefronts of a workgroup, which then own NC columns together: a matrix of few rows
+// still has a workgroup for every CU, and a lane's running sums are a quarter as long (1,536 columns of 8,960 at 1 / 3 / 8
+// rows: 22 / 39 / 60 -> 11 / 15 / 23 us, 5.0 TB/s at one row; errors halve).  STREAM: W is read past the caches, which
+// pays where it is far larger than they are (151,936 columns of 1,536 at one row 152 -> 129 us).
+template <int MB, int NC, bool STREAM>
+__global__ __launch_bounds__(256) void gemm_rows_split_kernel(
+    const act_t* __restrict__ x, const act_t* __restrict__ w, const float* __restrict__ bias,
+    void* __restrict__ y, int M, int N, int K) {
+  typedef float rows_v4 __attribute__((ext_vector_type(4)));
+  __shared__ float part[4][MB * NC];
+  const int lane = threadIdx.x % SL_WAVE, wave = threadIdx.x / SL_WAVE;
+  const int n0 = blockIdx.x * NC;
+  const act_t* wr[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) wr[c] = w + (size_t)(n0 + c < N ? n0 + c : N - 1) * K;
+  float acc[MB][NC];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[i][c] = 0.f;
+#pragma unroll 2
+  for (int k = threadIdx.x * SL_VEC; k < K; k += 256 * SL_VEC) {
+    float wf[NC][SL_VEC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      vec_t wv;
+      const rows_v4 raw = STREAM ? __builtin_nontemporal_load((const rows_v4*)(wr[c] + k)) : *(const rows_v4*)(wr[c] + k);
+      __builtin_memcpy(&wv, &raw, 16);
+#pragma unroll
+      for (int j = 0; j < SL_VEC; ++j) wf[c][j] = to_f(wv.v[j]);
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const vec_t xv = *(const vec_t*)(x + (size_t)min(i, M - 1) * K + k);
+#pragma unroll
+      for (int j = 0; j < SL_VEC; ++j) {
+        const float xf = to_f(xv.v[j]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[i][c] += wf[c][j] * xf;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const float s = wave_sum(acc[i][c]);
+      if (lane == 0) part[wave][i * NC + c] = s;
+    }
+  __syncthreads();
+  if (threadIdx.x < MB * NC) {
+    const int i = threadIdx.x / NC, c = threadIdx.x % NC;
+    if (i < M && n0 + c < N) {
+      const float s = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
+      ((float*)y)[(size_t)i * N + n0 + c] = s + (bias != nullptr ? bias[n0 + c] : 0.f);
+    }
+  }
+}
+template <int NC, bool STREAM>
+static const char* rows_split(const act_t* x, const act_t* w, const float* bias, void* y, int M, int N, int K, hipStream_t stream) {
+  const int grid = (N + NC - 1) / NC;
+  if (M == 1) gemm_rows_split_kernel<1, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else if (M == 2) gemm_rows_split_kernel<2, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else if (M <= 4) gemm_rows_split_kernel<4, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else gemm_rows_split_kernel<8, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  return sl_launch_status();
+}
+#endif
+
 // The same product with the rows of x staged through LDS: the eight wavefronts of a workgroup own
 // four columns each and share every chunk of x, so x leaves the cache hierarchy once per 32 columns
 // of W instead of once per 4 (with 8 rows of x that was twice the bytes of W itself, and what the
@@ -147,6 +217,16 @@ extern "C" const char* sl_gemm_rows(const void* x, const void* w, const float* b
   const act_t* ww = (const act_t*)w;
   // (measured, float32, 7B shape: from 4 rows on the staged form wins, 8 rows 139 -> 113 us for gate/up and
   // 176 -> 114 us for down, 16 rows 281 -> 172 and 494 -> 174 us; with 1 to 3 rows it loses up to 18 us of 44)
+#if defined(SL_F32)
+  // (measured, us, one form against the next: 1,536 columns of 1,536 / 8,960 at 3 rows 9.9 / 39 -> 5.8 / 15 with two
+  // columns a workgroup; 3,584 of 18,944 at 1 / 3 / 8 rows 44 / 74 / 111 -> 42 / 47 / 62 with four.  Of many columns a
+  // wavefront each has enough to do from three rows on unless its rows are long: 151,936 of 1,536 at 3 rows 163
+  // against 177, 37,888 of 3,584 102 against 88; at 1 / 2 rows 93 / 99 -> 75 / 78.)
+  if (M <= 8 && N <= 2048) return rows_split<2, true>(xx, ww, bias, y, M, N, K, stream);
+  if (M <= 8 && N <= 4096) return rows_split<4, false>(xx, ww, bias, y, M, N, K, stream);
+  if (M == 1) return rows_split<2, true>(xx, ww, bias, y, M, N, K, stream);
+  if (M == 2 || (M <= 4 && K >= 2048)) return rows_split<4, true>(xx, ww, bias, y, M, N, K, stream);
+#endif
   constexpr int SHARED_MAX_M = sizeof(act_t) == 4 ? 16 : 8;   // (16 rows of bfloat16 spill registers)
   if (shared && M >= 4 && M <= SHARED_MAX_M) {
     // (eight wavefronts a workgroup also for matrices of few rows: four, for twice the workgroups, measured
@@ -274,7 +354,7 @@ constexpr int FK = 16, FS = FK + 1;
 template <int TI, int TJ, int WM, int WN>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
-    float* __restrict__ y, int M, int N, int K) {
+    float* __restrict__ y, int M, int N, int K, int nsplit) {
   static_assert(WM * WN == 4, "four wavefronts");
   constexpr int FM = 32 * TI * WM, FN = 32 * TJ * WN;
   constexpr int XL = (FM * 4 + 255) / 256, WL = (FN * 4 + 255) / 256;    // 16-byte loads a thread makes per chunk
@@ -334,14 +414,22 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
       }
     }
   };
-  const int nchunks = K / FK;
-  load(0);
-  store(0);
+  constexpr int SEG = SEGMENT_K / FK;                 // chunks a running sum takes
+  // this share of K: whole segments (the last share also what is left over), results to its own [M, N]
+  const int segs = (K / FK + SEG - 1) / SEG;
+  const int first = (int)((long long)segs * blockIdx.z / nsplit) * SEG;
+  const int behind = (int)((long long)segs * (blockIdx.z + 1) / nsplit) * SEG;
+  const int nchunks = behind < K / FK ? behind : K / FK;
+  if (nsplit > 1) {
+    y += (size_t)blockIdx.z * M * N;
+    bias = nullptr;
+  }
+  load(first * FK);
+  store(first & 1);
   __syncthreads();
   // operand element of this lane in a 32 x 2 step: row lane % 32, k lane / 32
   const int orow = lane & 31, ok = lane >> 5;
-  constexpr int SEG = SEGMENT_K / FK;                 // chunks a running sum takes
-  for (int c0 = 0; c0 < nchunks; c0 += SEG) {
+  for (int c0 = first; c0 < nchunks; c0 += SEG) {
     const int c1 = c0 + SEG < nchunks ? c0 + SEG : nchunks;
     for (int c = c0; c < c1; ++c) {
       const int buf = c & 1;
@@ -389,22 +477,50 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   }
 }
 
+// The shares' sums added up in their order, then the bias; VEC values a thread.
+template <int VEC>
+__global__ __launch_bounds__(256) void f32_shares_kernel(const float* __restrict__ part, const float* __restrict__ bias,
+                                                         float* __restrict__ y, long long total, int N, int nsplit) {
+  struct __attribute__((aligned(4 * VEC))) piece { float v[VEC]; };
+  const long long at = ((long long)blockIdx.x * 256 + threadIdx.x) * VEC;
+  if (at >= total) return;
+  piece sum = *(const piece*)(part + at);
+  for (int j = 1; j < nsplit; ++j) {
+    const piece p = *(const piece*)(part + j * total + at);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) sum.v[i] += p.v[i];
+  }
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) sum.v[i] += bias != nullptr ? bias[(at + i) % N] : 0.f;
+  *(piece*)(y + at) = sum;
+}
+
+// nsplit > 1: K is cut into that many shares of whole segments, whose sums wait in `part`, [nsplit, M, N].  A product of
+// few tiles (the output projection and the down projection of a short prompt) leaves most CUs idle otherwise: 849 rows
+// of x, 1,536 rows of W of 8,960: 84 tiles.
 extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const float* bias, void* y,
-                                        int M, int N, int K, hipStream_t stream) {
+                                        int M, int N, int K, int nsplit, float* part, hipStream_t stream) {
   SL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_f32_mfma: sizes must be positive");
   SL_CHECK(K % FK == 0, "gemm_f32_mfma: K must be a multiple of 16");
   SL_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
            "gemm_f32_mfma: x and W must be 16-byte aligned");
   if (M == 0) return nullptr;
+  SL_CHECK(nsplit >= 1 && nsplit <= (K + SEGMENT_K - 1) / SEGMENT_K, "gemm_f32_mfma: at most one share of K per 512 terms");
+  SL_CHECK(nsplit == 1 || (part != nullptr && (uintptr_t)part % 16 == 0 && (uintptr_t)y % 16 == 0),
+           "gemm_f32_mfma: shares of K need an aligned buffer for their sums");
   const int rows = M <= 64 ? 32 : 128;
-  const dim3 grid((N + 127) / 128, (M + rows - 1) / rows);
+  const dim3 grid((N + 127) / 128, (M + rows - 1) / rows, nsplit);
   SL_CHECK(grid.y <= 65535, "gemm_f32_mfma: more than 65535 row tiles");
+  float* to = nsplit > 1 ? part : (float*)y;
   if (M <= 64)
-    gemm_f32_mfma_kernel<1, 1, 1, 4><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias,
-                                                              (float*)y, M, N, K);
+    gemm_f32_mfma_kernel<1, 1, 1, 4><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
   else
-    gemm_f32_mfma_kernel<2, 2, 2, 2><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias,
-                                                              (float*)y, M, N, K);
+    gemm_f32_mfma_kernel<2, 2, 2, 2><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
+  if (nsplit > 1) {
+    const long long total = (long long)M * N;
+    if (N % 4 == 0) f32_shares_kernel<4><<<(unsigned)((total + 1023) / 1024), 256, 0, stream>>>(part, bias, (float*)y, total, N, nsplit);
+    else f32_shares_kernel<1><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(part, bias, (float*)y, total, N, nsplit);
+  }
   return sl_launch_status();
 }
 #endif

@@ -516,8 +516,28 @@ class ProductOps:
         M, K = x.shape
         N = w.shape[0]
         y = self._new((M, N), torch.float32)
-        self._call("gemm", "sl_gemm_f32_mfma", _p(x), _p(w), _p(bias), _p(y), M, N, K)
+        shares = self._f32_shares(M, N, K)
+        part = self._new((shares, M, N), torch.float32) if shares > 1 else None
+        self._call("gemm", "sl_gemm_f32_mfma", _p(x), _p(w), _p(bias), _p(y), M, N, K, shares, _p(part))
         return y
+
+    F32_SEGMENT = 512             # terms of a running sum of the float32 products: a share of K holds whole ones
+    F32_TILE_US_PER_TERM = 0.067  # a tile of 128 x 128 results takes this long per term of K with a CU to itself
+
+    def _f32_shares(self, M, N, K):
+        """Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated
+        time, which is the tiles' rounds over the CUs plus, for several shares, the traffic of the partial sums and
+        their addition."""
+        rows = 32 if M <= 64 else 128
+        tiles = -(-M // rows) * -(-N // 128)
+        best, least = 1, float("inf")
+        for s in range(1, min(16, -(-K // self.F32_SEGMENT)) + 1):
+            us = -(-tiles * s // self._num_cus) * (K / s) * self.F32_TILE_US_PER_TERM * (rows / 128)
+            if s > 1:
+                us += 5.0 + (s + 1) * M * N * 4 / 3e6
+            if us < 0.97 * least:
+                best, least = s, us
+        return best
 
     def library_sums(self, x, w, out_dtype=None):
         """x w^T by the library, in bfloat16 or (``out_dtype`` float32) with the

@@ -1,0 +1,65 @@
+"""The float32 table's products and prompt attention at the sizes where their forms can go wrong, against float64."""
+import pytest
+import torch
+
+from servelab_amd.kernels import HipOps
+from test_kernels_gpu import make_attention_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def relative(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+# two and four columns a workgroup (up to 2,048, up to 4,096 and more columns), rows of 1 to 8, columns that neither divides,
+# K shorter than the workgroup's step of 1,024 values and not a multiple of it
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("N,K", [(1, 4), (7, 1028), (2048, 252), (2051, 2052), (4097, 1536), (4099, 2048)])
+def test_few_rows(M, N, K):
+    ops = HipOps(torch.float32, DEV)
+    g = torch.Generator().manual_seed(M + N)
+    x, w, b = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV), torch.randn(N, generator=g).to(DEV)
+    got = ops.linear_rows(x, w, b, False)
+    # 256 running sums of K / 256 products each, added in pairs: far below 2^-24 sqrt(K) of a result
+    assert relative(got, x.double() @ w.double().T + b.double()) < 1e-6
+
+
+# rows of 32 and of 128 a tile, one share and several, a last share with what no segment of 512 divides, odd columns
+@pytest.mark.parametrize("M,N,K", [(17, 40, 528), (64, 256, 1552), (65, 130, 2048), (300, 133, 8960), (849, 1536, 1536), (70, 128, 496)])
+def test_products_in_shares_of_k(M, N, K):
+    ops = HipOps(torch.float32, DEV)
+    g = torch.Generator().manual_seed(M + N)
+    x, w, b = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV), torch.randn(N, generator=g).to(DEV)
+    want = x.double() @ w.double().T + b.double()
+    errors = {}
+    for shares in sorted({1, ops._f32_shares(M, N, K), -(-K // 512)}):
+        ops._f32_shares = lambda *_: shares
+        errors[shares] = relative(ops.linear_f32_mfma(x, w, b), want)
+    # running sums of 512 products: 2^-24 sqrt(512) of a result; shares only shorten the chain of their sums
+    assert max(errors.values()) < 1.4e-6 and all(e <= 1.05 * errors[1] for e in errors.values())
+
+
+@pytest.mark.parametrize("nh,nkv,D", [(12, 2, 128), (14, 2, 64), (4, 4, 64), (8, 1, 128)])
+@pytest.mark.parametrize("page,window", [(16, None), (32, 40), (64, 5)])
+def test_prompt_attention_on_the_matrix_cores(nh, nkv, D, page, window):
+    """Portions that start at zero and deep in their contexts, of one tile of 64 columns and several, ending inside a block of
+    32 keys and at its end; single tokens behind them take the other kernels."""
+    from emulated_ops import EmulatedOps
+    ops, emu = HipOps(torch.float32, DEV), EmulatedOps(torch.float32)
+    qkv, kc, vc, tables, batch = make_attention_case(torch.float32, nh, nkv, D, page, [(33, 33), (72, 2), (63, 32), (95, 90), (300, 40), (65, 1)])[:5]
+    got = ops.paged_attention(qkv, nh, nkv, D, kc, vc, page, tables, batch, D ** -0.5, window)
+    host = emu_batch(batch)
+    want = emu.paged_attention(qkv.cpu(), nh, nkv, D, kc.cpu(), vc.cpu(), page, tables.cpu(), host, D ** -0.5, window)
+    # float32 scores of 128 products and sums over at most 300 keys on both sides
+    assert float((got.cpu() - want).abs().max()) <= 2e-6 * max(1.0, float(want.abs().max()))
+
+
+def emu_batch(batch):
+    import copy
+    host = copy.copy(batch)
+    for name, value in vars(batch).items():
+        if torch.is_tensor(value):
+            setattr(host, name, value.cpu())
+    return host
