@@ -1834,16 +1834,16 @@ template <int N_> __device__ __forceinline__ void block_wait_loads() {
   __builtin_amdgcn_s_waitcnt((N_ & 15) | (7 << 4) | (15 << 8) | ((N_ >> 4) << 14));
 }
 
-template <int WM, int WN, int STAGES>
+template <int WM, int WN, int STAGES, bool GATED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ w, const float* __restrict__ bias,
-    void* __restrict__ y, int M, int N, int K, int out_f32, int KS) {
+    void* __restrict__ y, int M, int N, int K, int out_f32, int act, int KS) {
   constexpr int WAVES = WM * WN, BM = 64 * WM, BN = 64 * WN;
   static_assert(STAGES == 2 || STAGES == 3, "a ring of two or three stages");
   constexpr int ROWS = BM + BN;                      // rows of a stage: x, then W; 128 bytes each
   constexpr int STAGE_BYTES = ROWS * 128;
-  constexpr int LOADS = ROWS / 8 / WAVES;            // wavefront-wide loads (8 rows) a wavefront makes per chunk
-  static_assert(LOADS * 8 * WAVES == ROWS, "the rows of a stage must divide evenly over the wavefronts");
+  constexpr int LOADS = (ROWS / 8 + WAVES - 1) / WAVES;        // wavefront-wide loads (8 rows) a wavefront makes per chunk
+  static_assert(STAGES == 2 || LOADS * 8 * WAVES == ROWS, "a count of loads under way must hold for every wavefront");
   __shared__ __attribute__((aligned(1024))) char ring[STAGES * STAGE_BYTES];
   const int t = threadIdx.x, lane = t & 63, i = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1882,14 +1882,16 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
   auto fetch = [&](int c, int stage) {
     const unsigned at = ring_at + STAGE_BYTES * stage + 1024 * wave;
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j) block_load_to_lds(src[j] + 64 * (size_t)c, at + 1024 * WAVES * j);
+    for (int j = 0; j < LOADS; ++j)
+      if (LOADS * 8 * WAVES == ROWS || wave + WAVES * j < ROWS / 8)
+        block_load_to_lds(src[j] + 64 * (size_t)c, at + 1024 * WAVES * j);
   };
   // where this lane reads its operands: row R0 + i (R0 a multiple of 16), unit 4 kk + gq
   int at_kk[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) at_kk[kk] = 128 * i + 16 * ((4 * kk + gq) ^ (((i >> 1) & 7) ^ (4 * (i & 1))));
 
-  f32x4 acc[4][4];                                   // [tile of W rows][tile of x rows]
+  f32x4 acc[4][4];                                 // [tile of W rows][tile of x rows]
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -1915,10 +1917,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
     for (int kk = 0; kk < 2; ++kk) {
       bf16x8 a[4], b[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u] = *(const bf16x8*)(st + 128 * (BM + 64 * wn + 16 * u) + at_kk[kk]);
-        b[u] = *(const bf16x8*)(st + 128 * (64 * wm + 16 * u) + at_kk[kk]);
-      }
+      for (int u = 0; u < 4; ++u) a[u] = *(const bf16x8*)(st + 128 * (BM + 64 * wn + 16 * u) + at_kk[kk]);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) b[v] = *(const bf16x8*)(st + 128 * (64 * wm + 16 * v) + at_kk[kk]);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -1936,6 +1937,31 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int m = m0 + 64 * wm + 16 * v + i;
+    if constexpr (GATED) {
+      // gate and up rows lie in blocks of eight: lanes 0..31 of a tile's sums hold gates, 32..63 ups.  Two tiles
+      // trade halves, so that every lane holds four gates and their four ups.
+#pragma unroll
+      for (int u = 0; u < 4; u += 2) {
+        const int n = n0 + 64 * wn + 16 * u + 4 * gq;
+        f32x4 r0 = acc[u][v], r1 = acc[u + 1][v];
+        if (bias != nullptr) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (n + e < N) r0[e] += bias[n + e];
+            if (n + 16 + e < N) r1[e] += bias[n + 16 + e];
+          }
+        }
+        bf16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(r0[e]), __float_as_uint(r1[e]), false, false);
+          h[e] = (__bf16)(sl_act(__uint_as_float(both[0]), act) * __uint_as_float(both[1]));
+        }
+        const int o = (n0 + 64 * wn + 16 * u) / 2 + 8 * (gq >> 1) + 4 * (gq & 1);
+        if (m < M && o < N / 2) *(bf16x4*)((__bf16*)y + (size_t)m * (N / 2) + o) = h;
+      }
+      continue;
+    }
     if (m >= M) continue;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -1978,16 +2004,21 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
   }
 }
 
-// x and W row-major.  ks > 1: `part` holds ks * M * N floats; with y == nullptr they are left
+// x and W row-major.  gated (an activation): W's rows hold gate and up in blocks of eight, y [M, N / 2] = act(gate) * up
+// of the float sums (7B shape, 2,048 rows: 491 us, the library's product and the kernel that gates it 544).
+// ks > 1: `part` holds ks * M * N floats; with y == nullptr they are left
 // there for the reader to add (and the bias with them), else splitk_reduce adds them into y.
 extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* bias, void* y,
-                                     int M, int N, int K, int out_f32, int ks, int square, float* part,
+                                     int M, int N, int K, int out_f32, int gated, int ks, int square, float* part,
                                      hipStream_t stream) {
   SL_CHECK(M > 0 && N > 0 && K > 0, "gemm_block: sizes must be positive");
   SL_CHECK(K % 64 == 0, "gemm_block: K must be a multiple of 64");
   SL_CHECK(ks >= 1 && ks <= 64 && ks <= K / 64, "gemm_block: ks must be in 1..64 and <= K / 64");
   SL_CHECK(ks == 1 || part != nullptr, "gemm_block: a split of K needs the partial buffer");
   SL_CHECK(y != nullptr || ks > 1, "gemm_block: no output");
+  SL_CHECK(square == 0 || square == 256 || (square == 192 && gated), "gemm_block: tiles of 256 rows by 128 or 256, gated ones of 256 or 192 by 256");
+  SL_CHECK(!gated || (square && ks == 1 && !out_f32 && N % 16 == 0),
+           "gemm_block: a gated product takes wide tiles, whole rows of K, blocks of eight and bfloat16 results");
   SL_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_block: x and W must be 16-byte aligned");
   void* dst = ks > 1 ? (void*)part : y;
   const __bf16* xx = (const __bf16*)x;
@@ -1998,12 +2029,15 @@ extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* 
   // square: tiles of 256 x 256 (sixteen wavefronts, a ring of two stages in 128 KB of LDS) instead of
   // 256 x 128 (eight wavefronts, three stages): a workgroup pulls 512 rows for 256 x 256 of result
   // instead of 384 for 256 x 128, which is what the time of these products follows.
-  const int bn = square ? 256 : 128;
-  const long long triples = (long long)((N + bn - 1) / bn) * ((M + 255) / 256) * ks;
+  // 192: tiles of 192 x 256 (twelve wavefronts) where they leave fewer CUs idle, see the caller's rule.
+  const int bn = square ? 256 : 128, bm = square == 192 ? 192 : 256;
+  const long long triples = (long long)((N + bn - 1) / bn) * ((M + bm - 1) / bm) * ks;
   SL_CHECK(triples < (1ll << 28), "gemm_block: too many tiles");
   const dim3 grid((unsigned)(8 * ((triples + 7) / 8)));              // laid out by chiplet (see the kernel)
-  if (square) gemm_block_kernel<4, 4, 2><<<grid, 1024, 0, stream>>>(xx, ww, bias, dst, M, N, K, out_f32, ks);
-  else gemm_block_kernel<4, 2, 3><<<grid, 512, 0, stream>>>(xx, ww, bias, dst, M, N, K, out_f32, ks);
+  if (gated && square == 192) gemm_block_kernel<3, 4, 2, true><<<grid, 768, 0, stream>>>(xx, ww, bias, dst, M, N, K, 0, gated, 1);
+  else if (gated) gemm_block_kernel<4, 4, 2, true><<<grid, 1024, 0, stream>>>(xx, ww, bias, dst, M, N, K, 0, gated, 1);
+  else if (square) gemm_block_kernel<4, 4, 2, false><<<grid, 1024, 0, stream>>>(xx, ww, bias, dst, M, N, K, out_f32, 0, ks);
+  else gemm_block_kernel<4, 2, 3, false><<<grid, 512, 0, stream>>>(xx, ww, bias, dst, M, N, K, out_f32, 0, ks);
   const char* e = sl_launch_status();
   if (e || ks == 1 || y == nullptr) return e;
   const size_t total = (size_t)M * N;

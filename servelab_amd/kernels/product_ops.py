@@ -194,7 +194,8 @@ class ProductOps:
                 return self.linear_f32_mfma(x, weight.w, bias)
             return self.linear_tiled(x, weight.w, bias, out_f32)
         limit = self._few_rows_limit(weight)
-        plan = self._block_plan(M, N, K, weight)
+        plan = self._block_plan(M, N, K, weight) or (
+            defer and self.fuse_norms and not out_f32 and self._shares_plan(M, N, K, weight))
         if plan:
             # (deferred: the norm adds the partial sums)
             return self.linear_block(x, weight, bias, out_f32, plan[0],
@@ -307,6 +308,52 @@ class ProductOps:
         tiles = -(-N // 128) * -(-M // 256)
         return max(1, min(16, K // 64 // 3, self._num_cus // tiles)), False
 
+    def _shares_plan(self, M, N, K, weight):
+        """Like ``_block_plan`` for a product of more rows that the norm adds to the stream: two or
+        three shares of K in square tiles where they fill three quarters of the CUs and the tiles
+        alone would not (7B shape, down projection at 1,800 / 2,048 rows: 218 / 245 us in 2
+        shares, 334 / 362 us in the library's product; 3B shape, whose 64 tiles need 4 shares: 85
+        against 93 us, which the norm's reading of four partial sums takes back)."""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or weight.w is None
+                or K % 64 or N % 4 or N > self.BLOCK_MAX_N or K < self.BLOCK_SQUARE_MIN_K
+                or not self.BLOCK_SQUARE_MAX_M < M <= self.SHARES_MAX_M):
+            return None
+        tiles = -(-N // 256) * -(-M // 256)
+        shares = self._num_cus // tiles
+        return (shares, True) if 2 <= shares <= 3 and 4 * tiles * shares >= 3 * self._num_cus else None
+
+    def _gated_rows(self, M, N, K, weight):
+        """Rows of x a workgroup of the block kernel takes (256 or 192) for the gated product of a
+        prompt, or None where the library's product and a pass that gates it are the faster pair.
+        The kernel runs in rounds of one tile a CU, of which a half-filled one costs as much as a
+        full one; the library's own tiles leave less idle, but it writes gate and up (2 N bytes a
+        row) for the second kernel to read.  So: rows of K up to GATED_SHORT_K, where the
+        library's prologue weighs most (9728 x 896, 1,024 rows: 25.5 us, 36 in two kernels); one
+        round that fills GATED_FILL of the CUs' share (8192 x 2048, 1,400 rows: 47.1 against 51 us, at
+        900 rows and 0.55 of it 40.7 against 39); several rounds, filled to three quarters, of
+        GATED_ROUNDS_MIN_M rows and more (37888 x 3584: 1,700 rows 435 against 446 us, 2,048 rows 492
+        against 544; at 1,536 rows 395 against 348, where the library has tiles that fit)."""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
+                or not 256 <= M <= self.GATED_MAX_M or N < self.GATED_MIN_N):
+            return None
+        rounds = {rows: -(--(-N // 256) * -(-M // rows) // self._num_cus) for rows in (256, 192)}
+        rows = min(rounds, key=lambda r: rounds[r] * (r * K + 65536))
+        fill = M * N / (rounds[rows] * self._num_cus * rows * 256)
+        if K <= self.GATED_SHORT_K or (fill >= self.GATED_FILL and rounds[rows] == 1):
+            return rows
+        return rows if M >= self.GATED_ROUNDS_MIN_M and fill >= 0.75 else None
+
+    def linear_gated_block(self, x, weight, bias, rows, act):
+        """act(gate) * up of many rows over the row-major weight, tiles of ``rows`` x 256."""
+        M, K = x.shape
+        N = weight.shape[0]
+        w = self.rows_of(weight)
+        self._check(x, self.act_dtype, (M, K), "x")
+        self._check(w, self.act_dtype, (N, K), "weight")
+        y = self._new((M, N // 2))
+        self._call("gemm", "sl_gemm_block", _p(x), _p(w), _p(bias), _p(y), M, N, K, 0, int(act), 1, int(rows), None)
+        return y
+
     def linear_block(self, x, weight, bias, out_f32=False, ks=1, partial=False, square=False):
         """A few hundred rows over the row-major copy of the weight: workgroups
         own a tile of 256 rows of x by 128 rows of W (``square``: by 256) over
@@ -322,14 +369,14 @@ class ProductOps:
         part = self._new((ks, M, N), torch.float32) if ks > 1 or partial else None
         if partial:
             if ks > 1:
-                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, None, M, N, K, 0, int(ks), int(square),
+                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, None, M, N, K, 0, 0, int(ks), 256 * int(square),
                            _p(part))
             else:
-                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, _p(part), M, N, K, 1, 1, int(square), None)
+                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, _p(part), M, N, K, 1, 0, 1, 256 * int(square), None)
             return PartialSums(part, bias)
         y = self._new((M, N), torch.float32 if out_f32 else None)
         self._call("gemm", "sl_gemm_block", _p(x), _p(w), _p(bias), _p(y), M, N, K, int(out_f32),
-                   int(ks), int(square), _p(part))
+                   0, int(ks), 256 * int(square), _p(part))
         return y
 
     def linear_skinny(self, x, weight, bias, out_f32=False):
@@ -394,8 +441,8 @@ class ProductOps:
         """act(x Wg^T + bg) * (x Wu^T + bu) for a weight whose rows hold gate and up
         interleaved in blocks of ``block`` rows (``block`` = I: plain [Wg; Wu]) and a
         ``bias`` [2 I] (or None) that lies as the rows do;
-        ``activation``: "silu", "relu" or "gelu_tanh".  Few rows and a tiled weight with blocks
-        of 8: one fused kernel."""
+        ``activation``: "silu", "relu" or "gelu_tanh".  Blocks of 8 and few rows of x over
+        a tiled weight, or as many as ``_gated_rows`` takes: one fused kernel."""
         if not isinstance(weight, LinearWeight):
             weight = LinearWeight(weight)
         code = activation_code(activation, ("silu", "relu", "gelu_tanh"))      # (what the kernels take as `gated`)
@@ -423,6 +470,9 @@ class ProductOps:
             y = self._new((M, N // 2))
             self._skinny(x, weight, bias, y, M, N, K, gated=code)
             return y
+        rows = block == self.GATE_BLOCK and self._gated_rows(M, N, K, weight)
+        if rows:
+            return self.linear_gated_block(x, weight, bias, rows, code)
         return self.gate_mul(self.linear(x, weight, bias), block, activation)
 
     def gated_mlp(self, x, w_gate_up, block, w_down, defer=False, activation="silu", bias_gate_up=None,

@@ -1,0 +1,66 @@
+"""Gated products of a prompt in tiles of 256 or 192 rows of x by 256 rows of W, and the shares of K of a long-row product
+of many rows, at the sizes where their edges lie, against float64."""
+import pytest
+import torch
+
+from servelab_amd.kernels import HipOps
+from servelab_amd.kernels.ops import PartialSums
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def act64(z, name):
+    if name == "relu":
+        return z.clamp(min=0)
+    return torch.nn.functional.silu(z) if name == "silu" else torch.nn.functional.gelu(z, approximate="tanh")
+
+
+# one row of x, a tile less and more by one; half a block's tile of W, a column tile with one matrix-instruction tile, one and
+# three chunks of K
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (191, 272, 192), (193, 256, 64), (255, 528, 128), (257, 1040, 192), (385, 32, 64)])
+@pytest.mark.parametrize("act", ["silu", "relu", "gelu_tanh"])
+@pytest.mark.parametrize("rows", [192, 256])
+def test_gated_tiles(M, N, K, act, rows):
+    ops = HipOps(torch.bfloat16, DEV)
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    b = torch.randn(N, generator=g) if act != "relu" else None
+    z = x.double() @ w.double().T + (0 if b is None else b.double())
+    z = z.view(M, N // 16, 2, 8)
+    want = (act64(z[:, :, 0], act) * z[:, :, 1]).reshape(M, N // 2)
+    code = {"silu": 1, "relu": 2, "gelu_tanh": 4}[act]
+    got = ops.linear_gated_block(x.to(DEV), ops.prepare_weight(w.to(DEV)), None if b is None else b.to(DEV), rows, code)
+    # one rounding to bfloat16 (2^-9 of the value) and float sums of K terms: K 2^-24 of their absolute sum, twice
+    # (gate and up), times the other factor
+    size = (x.double().abs() @ w.double().abs().T + (0 if b is None else b.double().abs())).max().item()
+    bar = 2.0 ** -8 * want.abs() + 4 * K * 2.0 ** -24 * size * z.abs().max().item() + 1e-30
+    assert ((got.double().cpu() - want).abs() <= bar).all()
+
+
+def test_routes_of_prompts_products():
+    ops = HipOps(torch.bfloat16, DEV)
+    big = ops.prepare_weight(torch.zeros(8192, 1088, dtype=torch.bfloat16, device=DEV))
+    assert ops._gated_rows(255, 8192, 1024, big) is None and ops._gated_rows(256, 8192, 1024, big) == 192
+    assert ops._gated_rows(256, 8192, 1088, big) is None                         # a round filled to a sixth
+    assert ops._gated_rows(1536, 8192, 2048, big) == 192                         # 256 tiles of 192 rows: one full round
+    assert ops._gated_rows(1537, 8192, 2048, big) == 256                         # 224 tiles of 256
+    assert ops._gated_rows(1600, 37888, 3584, big) is None and ops._gated_rows(2048, 37888, 3584, big) == 256
+    assert ops._gated_rows(2561, 37888, 3584, big) is None and ops._gated_rows(2048, 8192, 2080, big) is None
+    x = torch.randn(300, 1024, device=DEV).bfloat16()
+    w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
+    weight = ops.prepare_weight(w)
+    assert torch.equal(ops.gated_linear(x, weight, 8), ops.linear_gated_block(x, weight, None, 192, 1))
+    # a residual delta of 1,537 and more rows: two or three shares
+    K, N, M = 8192, 1024, 1600
+    w = (torch.randn(N, K, device=DEV) * 0.02).bfloat16()
+    weight, x = ops.prepare_weight(w), torch.randn(M, K, device=DEV).bfloat16()
+    ops._num_cus = 64
+    assert ops._shares_plan(M, N, K, weight) == (2, True) and ops._shares_plan(1536, N, K, weight) is None
+    assert ops._shares_plan(2049, N, K, weight) is None and ops._shares_plan(M, 2 * N, K, weight) is None
+    delta = ops.linear(x, weight, None, defer=True)
+    assert isinstance(delta, PartialSums) and delta.parts.shape == (2, M, N)
+    want = x.double() @ w.double().T
+    # float sums of K terms: K 2^-24 of their absolute sum
+    assert ((delta.parts.double().sum(0) - want).abs() <= K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
+    assert not isinstance(ops.linear(x, weight, None), PartialSums)
