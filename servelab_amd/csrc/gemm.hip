@@ -7,6 +7,7 @@
 //                 rows of x at a time.
 //   sl_gemm_tiled any M: 64x64 LDS tiles, 4x4 outputs per thread.
 #include "common.h"
+#include "lds_loads.h"
 #include <type_traits>
 
 #if defined(SL_F32)
@@ -1823,16 +1824,7 @@ extern "C" const char* sl_untile_weight(const void* wt, void* w, int N, int K, i
 // (global_load_lds_dwordx4: a wavefront's 64 loads of 16 bytes land side by side in 1 KB), two
 // chunks in flight while the third is multiplied: at the 50 GB/s a CU pulls and 2 us of loaded
 // latency that is what keeps the stream going.  A stage holds the rows of x, then those of W, 8
-// units of 16 bytes a row; a lane can put any unit anywhere at no cost, so unit c of row r lies
-// at place c ^ f(r), f(r) = ((r >> 1) & 7) ^ 4 (r & 1): the 16 lanes that read one operand
-// column (rows r .. r + 15, same c) then touch 16 different 16-byte slots of a 256-byte line of
-// banks, and each half of them 8 different slots of a 128-byte one.
-__device__ __forceinline__ void block_load_to_lds(const void* from, unsigned lds_at) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
-}
-template <int N_> __device__ __forceinline__ void block_wait_loads() {
-  __builtin_amdgcn_s_waitcnt((N_ & 15) | (7 << 4) | (15 << 8) | ((N_ >> 4) << 14));
-}
+// units of 16 bytes a row; a lane can put any unit anywhere at no cost, so they lie as lds_place says.
 
 template <int WM, int WN, int STAGES, bool GATED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
@@ -1869,7 +1861,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
 #pragma unroll
   for (int j = 0; j < LOADS; ++j) {
     const int row = 8 * (wave + WAVES * j) + (lane >> 3);
-    const int c = (lane & 7) ^ (((row >> 1) & 7) ^ (4 * (row & 1)));
+    const int c = (lane & 7) ^ lds_place(row);
     if (row < BM) {
       const int m = m0 + row < M ? m0 + row : M - 1;           // rows past the end: the last row again, never stored
       src[j] = x + (size_t)m * K + 8 * c;
@@ -1884,12 +1876,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
 #pragma unroll
     for (int j = 0; j < LOADS; ++j)
       if (LOADS * 8 * WAVES == ROWS || wave + WAVES * j < ROWS / 8)
-        block_load_to_lds(src[j] + 64 * (size_t)c, at + 1024 * WAVES * j);
+        load_to_lds(src[j] + 64 * (size_t)c, at + 1024 * WAVES * j);
   };
   // where this lane reads its operands: row R0 + i (R0 a multiple of 16), unit 4 kk + gq
   int at_kk[2];
 #pragma unroll
-  for (int kk = 0; kk < 2; ++kk) at_kk[kk] = 128 * i + 16 * ((4 * kk + gq) ^ (((i >> 1) & 7) ^ (4 * (i & 1))));
+  for (int kk = 0; kk < 2; ++kk) at_kk[kk] = 128 * i + 16 * ((4 * kk + gq) ^ lds_place(i));
 
   f32x4 acc[4][4];                                 // [tile of W rows][tile of x rows]
 #pragma unroll
@@ -1901,9 +1893,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
     fetch(cbeg, 0);
     if (STAGES == 3 && cbeg + 1 < cend) {
       fetch(cbeg + 1, 1);
-      block_wait_loads<LOADS>();
+      wait_loads<LOADS>();
     } else {
-      block_wait_loads<0>();
+      wait_loads<0>();
     }
     __builtin_amdgcn_s_barrier();
     asm volatile("" : : : "memory");
@@ -1926,8 +1918,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
         for (int v = 0; v < 4; ++v)
           acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[v], acc[u][v], 0, 0, 0);
     }
-    if (more && STAGES == 3) block_wait_loads<LOADS>();        // all but the chunk just asked for
-    else block_wait_loads<0>();
+    if (more && STAGES == 3) wait_loads<LOADS>();        // all but the chunk just asked for
+    else wait_loads<0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" : : : "memory");
     stage = stage == STAGES - 1 ? 0 : stage + 1;

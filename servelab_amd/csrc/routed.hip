@@ -20,8 +20,9 @@
 // + experts tiles) and workgroups beyond the tiles in use leave at once, so a step is a fixed
 // list of launches that a captured graph can replay.
 #include "common.h"
+#include "lds_loads.h"
 
-#define RT_ROWS 16           // rows of a tile of the plain grouped product; a row tile holds 16, 64 or 128 rows
+#define RT_ROWS 16           // rows of a tile of the plain grouped product; a row tile holds 16 or 128 rows
 
 // ------------------------------------------------------------------ route
 // One wavefront per token.  Largest first; among equal logits the lower index wins.
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(64) void route_kernel(const float* __restrict__ log
 // ------------------------------------------------------------------ group
 // One workgroup sorts the n = tokens * top pairs by expert (counting sort in LDS).
 //   order[place] = pair (token * top + choice);  place_of[pair] = place
-//   tiles[i] = {expert, first row, rows} for i < tiles in use; rows 0 beyond
+//   tiles[i] = {expert, first row, rows} for i < tiles in use; rows 0 beyond; tiles[max_tiles][0] = tiles in use
 // Experts from E_real on have no matrices: their pairs get places but no tiles.
 __global__ __launch_bounds__(1024) void group_kernel(const int* __restrict__ chosen, int n, int E, int E_real, int max_tiles,
                                                      int tile_rows, int* __restrict__ order,
@@ -142,6 +143,7 @@ __global__ __launch_bounds__(1024) void group_kernel(const int* __restrict__ cho
       rows += count[e];
       if (e < E_real) nt += (count[e] + tile_rows - 1) / tile_rows;
     }
+    tiles[3 * max_tiles] = nt;
   }
   __syncthreads();
   for (int e = tid; e < E_real; e += blockDim.x) {
@@ -172,7 +174,7 @@ extern "C" const char* sl_route_tokens(const float* logits, int stride, int T, i
            "route_tokens: at most 4096 experts within the rows, at most 64 choices");
   SL_CHECK(E_real >= 0 && E_real <= E && (over_all || correction == nullptr),
            "route_tokens: the experts with matrices are the first of all; a correction needs shares over all");
-  SL_CHECK(tile_rows == 16 || tile_rows == 64 || tile_rows == 128, "route_tokens: row tiles hold 16, 64 or 128 rows");
+  SL_CHECK(tile_rows == 16 || tile_rows == 128, "route_tokens: row tiles hold 16 or 128 rows");
   SL_CHECK(max_tiles >= ((long long)T * top + tile_rows - 1) / tile_rows + E, "route_tokens: too few tile entries");
   if (T == 0) return nullptr;
   route_kernel<<<T, 64, 0, stream>>>(logits, stride, E, top, chosen, shares, over_all, correction, scale, sigmoid);
@@ -197,6 +199,7 @@ struct Grouped {
   int act;                   // the activation (common.h); 0 with out_f32
   float limit;               // the clamped gate's bound
   const float* row_scale;    // with order: the sums of row r are multiplied by row_scale[order[r]] first; or nullptr
+  const int* used;           // how many of the tiles are in use
   int max_tiles, col_blocks; // the matrix-core kernels' launch: max_tiles x col_blocks workgroups in a row
 };
 
@@ -211,6 +214,19 @@ __device__ __forceinline__ bool grouped_place(const Grouped& a, int& tile, int& 
   if ((int)(blockIdx.x >> 3) >= run || m >= total) return false;
   cb = m / a.max_tiles;
   tile = m - cb * a.max_tiles;
+  return true;
+}
+
+// The same for row tiles of 128 rows: only the tiles in use, and every column block of a tile before the next tile.  A die
+// then reads a tile's rows of x once for all of its columns, and has two or three experts' matrices under way (64 experts of
+// 2,048 x 1,024, gate/up, down and the sum, 8 of them a token: 256 / 1,000 / 2,048 tokens 196 / 254 / 360 us by column
+// blocks, 162 / 231 / 359 by tiles).
+__device__ __forceinline__ bool grouped_place_by_rows(const Grouped& a, int& tile, int& cb) {
+  const int total = min(*a.used, a.max_tiles) * a.col_blocks, run = (total + 7) / 8;
+  const int m = (blockIdx.x & 7) * run + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= run || m >= total) return false;
+  tile = m / a.col_blocks;
+  cb = m - tile * a.col_blocks;
   return true;
 }
 
@@ -459,123 +475,127 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void grouped_product_few_kernel(con
 }
 
 
-// Row tiles of 128 rows with the rows of x staged in LDS: a workgroup of four wavefronts takes a row
-// tile by 64 NU columns; every wavefront owns all 128 rows by 16 NU columns (of the gate and of the
-// up matrix in the gated form).  The tile's rows of x come 64 values of k at a time into one of two
-// halves of LDS (a thread brings four 16-byte pieces, asked for one step ahead); a row's eight pieces
-// are stored at piece ^ (row / 2 % 8), so that the 16 lanes of a fragment read, and the 16 of a
-// write, take every bank once.  W comes straight from memory in the tiled layout, a k-step ahead: no
-// two wavefronts of the workgroup read the same piece of it, and the CU's cache delivers a third of
-// what the unstaged kernel asks of it.  Two workgroups a CU: one computes while the other waits.
-template <int NU, bool GATED>
-__global__ __launch_bounds__(256, 2) void grouped_product_staged_kernel(const Grouped a) {
-  constexpr int NT = 8, MATS = GATED ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) __bf16 stage[2][128 * 64];
+// Row tiles of 128 rows, both operands through LDS: a workgroup of eight wavefronts takes a row tile by 256 rows of W (256
+// columns, or 128 of the gate and the same 128 of the up matrix), a wavefront 64 by 64 of it.  Prompts with a few
+// hundred rows an expert sit where the stream of the matrices and the matrix units cost about the same, so what counts is
+// that enough of both is asked for ahead: chunks of 64 values of k go straight into a ring of three LDS stages (48 KB
+// each, the rows of x as lds_place says, W as its tiles lie in memory: what a wavefront reads of a tile is 1 KB in a row),
+// two chunks under way while the third is multiplied.  Blocks of 16 rows that hold no pair are not multiplied.
+// (64 experts of 2,048 x 1,024, gate/up, down and the sum, 8 of them a token: 256 / 1,000 / 2,048 tokens 174 / 285 / 401 us
+// with x staged through registers and W a step of 32 ahead of its use, 162 / 231 / 359 here.  Chunks of 32 values of k and two
+// workgroups a CU do not fit the registers: 310 / 484 / 635.)
+template <bool GATED>
+__global__ __launch_bounds__(512) void grouped_product_staged_kernel(const Grouped a) {
+  constexpr int STAGES = 3, X_BYTES = 128 * 128, STAGE_BYTES = X_BYTES + 256 * 128, LOADS = STAGE_BYTES / 1024 / 8;
+  __shared__ __attribute__((aligned(1024))) char ring[STAGES * STAGE_BYTES];
   int tile, cb;
-  if (!grouped_place(a, tile, cb)) return;
+  if (!grouped_place_by_rows(a, tile, cb)) return;
   const int* tl = a.tiles + 3 * tile;
   const int rows = min(128, tl[2]);
   if (rows <= 0) return;                                // (the whole workgroup: no barrier is left waiting)
   const int e = tl[0], row0 = tl[1];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x & 63, i = lane & 15, gq = lane >> 4;
-  const int n0 = (cb * 4 + wave) * 16 * NU;
-  const size_t n_w = GATED ? 2 * (size_t)a.N : (size_t)a.N;
-  const __bf16* we = a.w + (size_t)e * n_w * a.K;
-  const size_t up = (size_t)a.N * a.K;
-  const __bf16* wp[NU];
+  const int lane = threadIdx.x & 63, i = lane & 15, gq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 2, wn = wave & 3;
+  const int n0 = cb * (GATED ? 128 : 256);
+  const __bf16* we = a.w + (size_t)e * (GATED ? 2 * (size_t)a.N : (size_t)a.N) * a.K;
+  // Tile t of 16 rows of W (four a column of wavefronts): the wavefront's columns, or its gate's, then its up's
+  auto column = [&](int t) { return GATED ? n0 + 16 * (2 * (t >> 2) + (t & 1)) : n0 + 16 * t; };
+  // what this lane brings of every chunk: two pieces of 8 rows of x, four pieces (32 values of k) of W's tiles
+  const char* src[LOADS];
 #pragma unroll
-  for (int u = 0; u < NU; ++u)
-    wp[u] = we + (size_t)(min(n0 + 16 * u, a.N - 16) / 16) * (a.K / 32) * 512 + lane * 8;
-  // what this thread brings: piece threadIdx % 8 of rows threadIdx / 8 + 32 j
-  const int piece = threadIdx.x & 7, rbase = threadIdx.x >> 3;
-  const __bf16* xsrc[4];
-  int xat[4];
+  for (int j = 0; j < 2; ++j) {
+    const int r = 8 * (wave + 8 * j) + (lane >> 3), rr = row0 + min(r, rows - 1);
+    const size_t from = a.order != nullptr ? (size_t)(a.order[rr] / a.top) : (size_t)rr;
+    src[j] = (const char*)(a.x + from * a.K + 8 * ((lane & 7) ^ lds_place(r)));
+  }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int r = rbase + 32 * j, rr = row0 + min(r, rows - 1);
-    const size_t src = a.order != nullptr ? (size_t)(a.order[rr] / a.top) : (size_t)rr;
-    xsrc[j] = a.x + src * a.K + 8 * piece;
-    xat[j] = r * 64 + 8 * (piece ^ ((r >> 1) & 7));
+    const int piece = wave + 8 * j, t = piece >> 1;
+    const __bf16* m = we + (GATED && (t & 2) ? (size_t)a.N * a.K : 0);
+    src[2 + j] = (const char*)(m + ((size_t)(min(column(t), a.N - 16) / 16) * (a.K / 32) + (piece & 1)) * 512 + lane * 8);
   }
-  const int fsw = (i >> 1) & 7;                         // (16 v + i) / 2 % 8
-  rt_f32x4 acc[NT][NU * MATS];
+  const unsigned ring_at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
+  auto fetch = [&](int c, int stage) {
+    const unsigned at = ring_at + STAGE_BYTES * stage + 1024 * wave;
 #pragma unroll
-  for (int v = 0; v < NT; ++v)
+    for (int j = 0; j < LOADS; ++j)
+      load_to_lds(src[j] + (size_t)c * (j < 2 ? 128 : 2048), at + 8192 * j);
+  };
+  int at_kk[2];
 #pragma unroll
-    for (int u = 0; u < NU * MATS; ++u) acc[v][u] = rt_f32x4{0.f, 0.f, 0.f, 0.f};
-  rt_bf16x8 xr[4], wcur[NU * MATS], wnext[NU * MATS];
+  for (int kk = 0; kk < 2; ++kk) at_kk[kk] = 128 * (64 * wm + i) + 16 * ((4 * kk + gq) ^ lds_place(i));
+  const int blocks = min(4, (rows - 64 * wm + 15) / 16);         // of 16 rows with a pair (none: zero or less)
+
+  rt_f32x4 acc[4][4];                                   // [tile of W][block of rows]
 #pragma unroll
-  for (int j = 0; j < 4; ++j) xr[j] = *(const rt_bf16x8*)(xsrc[j]);
+  for (int u = 0; u < 4; ++u)
 #pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    wcur[u] = *(const rt_bf16x8*)(wp[u]);
-    if (GATED) wcur[NU + u] = *(const rt_bf16x8*)(wp[u] + up);
+    for (int v = 0; v < 4; ++v) acc[u][v] = rt_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int chunks = a.K / 64;
+  fetch(0, 0);
+  if (chunks > 1) {
+    fetch(1, 1);
+    wait_loads<LOADS>();
+  } else {
+    wait_loads<0>();
   }
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+  int stage = 0;
+  for (int c = 0; c < chunks; ++c) {
+    const bool more = c + 2 < chunks;
+    if (more) fetch(c + 2, stage >= 1 ? stage - 1 : 2);          // the stage the last chunk was read from
+    const char* st = ring + STAGE_BYTES * stage;
+    auto multiply = [&](auto all) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) *(rt_bf16x8*)(&stage[0][xat[j]]) = xr[j];
-  __syncthreads();
-  const int steps = a.K / 64;
-  for (int s = 0; s < steps; ++s) {
-    if (s + 1 < steps) {
+      for (int kk = 0; kk < 2; ++kk) {
+        rt_bf16x8 w[4], x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) xr[j] = *(const rt_bf16x8*)(xsrc[j] + 64 * (s + 1));
-    }
-    const __bf16* buf = stage[s & 1] + i * 64;
+        for (int u = 0; u < 4; ++u) w[u] = *(const rt_bf16x8*)(st + X_BYTES + 1024 * (2 * (4 * wn + u) + kk) + 16 * lane);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int kstep = 2 * s + h;
-      if (kstep + 1 < 2 * steps) {
-        const size_t kw = (size_t)(kstep + 1) * 512;
+        for (int v = 0; v < 4; ++v)
+          if (all || v < blocks) x[v] = *(const rt_bf16x8*)(st + 128 * 16 * v + at_kk[kk]);
 #pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          wnext[u] = *(const rt_bf16x8*)(wp[u] + kw);
-          if (GATED) wnext[NU + u] = *(const rt_bf16x8*)(wp[u] + up + kw);
-        }
+        for (int v = 0; v < 4; ++v)
+          if (all || v < blocks) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[v], acc[u][v], 0, 0, 0);
+          }
       }
-      const int fo = 8 * ((4 * h + gq) ^ fsw);
-#pragma unroll
-      for (int v = 0; v < NT; ++v) {
-        const rt_bf16x8 b = *(const rt_bf16x8*)(buf + v * 16 * 64 + fo);
-#pragma unroll
-        for (int u = 0; u < NU * MATS; ++u)
-          acc[v][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wcur[u], b, acc[v][u], 0, 0, 0);
-      }
-#pragma unroll
-      for (int u = 0; u < NU * MATS; ++u) wcur[u] = wnext[u];
-    }
-    if (s + 1 < steps) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) *(rt_bf16x8*)(&stage[(s + 1) & 1][xat[j]]) = xr[j];
-    }
-    __syncthreads();
+    };
+    if (blocks == 4) multiply(std::true_type{});
+    else if (blocks > 0) multiply(std::false_type{});
+    if (more) wait_loads<LOADS>();                      // all but the chunk just asked for
+    else wait_loads<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+    stage = stage == 2 ? 0 : stage + 1;
   }
-  // this lane holds columns n0 + 16 u + 4 gq .. + 3 of rows 16 v + i
+  // this lane holds columns 4 gq .. + 3 of each tile of W, of rows 64 wm + 16 v + i
 #pragma unroll
-  for (int v = 0; v < NT; ++v) {
-    if (16 * v + i >= rows) continue;
-    const size_t at = (size_t)(row0 + 16 * v + i) * a.N + n0 + 4 * gq;
-    if (a.row_scale != nullptr) {
-      const float rs = a.row_scale[a.order[row0 + 16 * v + i]];
+  for (int v = 0; v < 4; ++v) {
+    const int r = 64 * wm + 16 * v + i;
+    if (r >= rows) continue;
+    const float rs = a.row_scale != nullptr ? a.row_scale[a.order[row0 + r]] : 1.f;
+    const size_t at = (size_t)(row0 + r) * a.N + 4 * gq;
 #pragma unroll
-      for (int u = 0; u < NU * MATS; ++u) {
-        acc[v][u] *= rs;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      if (n0 + 16 * u >= a.N) continue;
+    for (int u = 0; u < (GATED ? 2 : 4); ++u) {
+      const int n = column(4 * wn + u);
+      if (n >= a.N) continue;
+      const rt_f32x4 z = a.row_scale != nullptr ? acc[u][v] * rs : acc[u][v];
       if (GATED) {
-        rt_bf16x4 r;
+        const rt_f32x4 up = a.row_scale != nullptr ? acc[2 + u][v] * rs : acc[2 + u][v];
+        rt_bf16x4 h;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) r[c] = (__bf16)sl_gated(acc[v][u][c], acc[v][NU + u][c], a.act, a.limit);
-        *(rt_bf16x4*)(a.out_act + at + 16 * u) = r;
+        for (int c = 0; c < 4; ++c) h[c] = (__bf16)sl_gated(z[c], up[c], a.act, a.limit);
+        *(rt_bf16x4*)(a.out_act + at + n) = h;
       } else if (a.act) {
-        rt_bf16x4 r;
+        rt_bf16x4 h;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) r[c] = (__bf16)sl_act(acc[v][u][c], a.act);
-        *(rt_bf16x4*)(a.out_act + at + 16 * u) = r;
+        for (int c = 0; c < 4; ++c) h[c] = (__bf16)sl_act(z[c], a.act);
+        *(rt_bf16x4*)(a.out_act + at + n) = h;
       } else {
-        *(rt_f32x4*)(a.out_f32 + at + 16 * u) = acc[v][u];
+        *(rt_f32x4*)(a.out_f32 + at + n) = z;
       }
     }
   }
@@ -591,12 +611,13 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
   SL_CHECK(act >= 0 && act <= SL_ACT_CLAMPED_SWISH && (!gated || act) && (gated || act != SL_ACT_CLAMPED_SWISH),
            "grouped_product: unknown activation, a gate without one, or the clamped form without a gate");
   SL_CHECK(row_scale == nullptr || order != nullptr, "grouped_product: factors per row go with the pairs' order");
-  SL_CHECK(tile_rows == 16 || tile_rows == 64 || tile_rows == 128, "grouped_product: row tiles hold 16, 64 or 128 rows");
+  SL_CHECK(tile_rows == 16 || tile_rows == 128, "grouped_product: row tiles hold 16 or 128 rows");
   SL_CHECK(pairs >= 0 && experts >= 0, "grouped_product: sizes must be positive");
   if (max_tiles == 0 || pairs == 0) return nullptr;
+  const int* used = tiles + 3 * (size_t)max_tiles;
   max_tiles = min(max_tiles, pairs);                    // (the tiles in use come first, and each holds a pair)
   Grouped a{(const act_t*)x, order, top, (const act_t*)w, w_tiled, tiles, tile_rows / RT_ROWS, N, K,
-            act ? (act_t*)out : nullptr, act ? nullptr : (float*)out, act, limit, row_scale, max_tiles, 1};
+            act ? (act_t*)out : nullptr, act ? nullptr : (float*)out, act, limit, row_scale, used, max_tiles, 1};
 #if !defined(SL_F32)
   if (K % 32 == 0 && N % 16 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0) {
     // (a one-dimensional launch of max_tiles x col_blocks workgroups, rounded up to the eight dies)
@@ -605,14 +626,11 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
       return dim3(8 * (unsigned)((max_tiles * a.col_blocks + 7) / 8));
     };
     if (tile_rows == 128 && w_tiled && K % 64 == 0) {   // the tile's rows of x staged in LDS
-      if (gated) grouped_product_staged_kernel<2, true><<<blocks(128), 256, 0, stream>>>(a);
-      else grouped_product_staged_kernel<4, false><<<blocks(256), 256, 0, stream>>>(a);
+      if (gated) grouped_product_staged_kernel<true><<<blocks(128), 512, 0, stream>>>(a);
+      else grouped_product_staged_kernel<false><<<blocks(256), 512, 0, stream>>>(a);
     } else if (tile_rows == 128) {                      // two wavefronts along the rows, two along the columns
       if (gated) grouped_product_mfma_kernel<4, 4, true, 2, 2><<<blocks(128), 256, 0, stream>>>(a);
       else grouped_product_mfma_kernel<4, 4, false, 2, 2><<<blocks(128), 256, 0, stream>>>(a);
-    } else if (tile_rows == 64) {
-      if (gated) grouped_product_mfma_kernel<4, 4, true, 1, 4><<<blocks(256), 256, 0, stream>>>(a);
-      else grouped_product_mfma_kernel<4, 4, false, 1, 4><<<blocks(256), 256, 0, stream>>>(a);
     } else if (pairs <= 8 * (long long)experts) {
       // (few rows an expert: the launch is bound by the matrices' stream, see the kernel.  Under six rows an
       // expert every one of its tiles is narrow; from there on the rows of x, read again by every column block,

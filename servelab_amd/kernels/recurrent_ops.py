@@ -17,7 +17,7 @@ _ll = ctypes.c_longlong
 
 _EXPAND_MODES = {"plain": 0, "log_sigmoid": 1, "rate_softplus": 2, "softplus": 3}
 _SCAN_DECAY, _SCAN_DELTA, _SCAN_LSTM, _SCAN_SSD, _SCAN_FORGET, _SCAN_DELTA_HEAD = 0, 1, 2, 3, 4, 5
-_TILE_ROWS = (16, 64, 128)    # rows of a row tile of the grouped products (routed.hip)
+_TILE_ROWS = (16, 128)    # rows of a row tile of the grouped products (routed.hip)
 
 
 class Routing(NamedTuple):
@@ -52,7 +52,13 @@ class RecurrentOps:
     # tokens 35 against 40 us, 192: 50 against 45).  Several sequences keep the chip busier: eight of 64 tokens
     # 51 against 41 us, eight of 32: 34 against 35.
     SCAN_CHUNKS_FROM, SCAN_CHUNKS_FROM_GROUPED, SCAN_CHUNKS_FROM_MANY, SCAN_MANY_TOKENS = 80, 160, 48, 400
-    ROUTED_WIDE_TILE_ROWS = 48    # rows an expert has on average from which row tiles hold 64 rows
+
+    # rows an expert has on average from which row tiles hold 128 rows (64 experts, 8 and 12 rows each: gate/up, down and
+    # the sum of 2,048 x 1,024 experts 143 and 154 us in tiles of 16, 147 and 150 in tiles of 128; of 3,584 x 1,792 405
+    # and 500, 431 and 436; 8 experts of 2,048 x 5,632, 8 and 12 rows 101 and 171, 144 and 144); with fewer than
+    # ROUTED_WIDE_EXPERTS experts, whose tiles of 128 rows leave most CUs idle, only from the second number on (4
+    # experts of 1,024 x 512, 47 and 120 rows 29.7 and 31, 32 and 40)
+    ROUTED_WIDE_TILE_ROWS, ROUTED_WIDE_TILE_ROWS_OF_FEW, ROUTED_WIDE_EXPERTS = 12, 96, 8
 
     # ------------------------------------------------- norm on an output
     def add_postnorm(self, resid, y, weight, eps, mult, want_rows=True):
@@ -392,17 +398,17 @@ class RecurrentOps:
         tiles; ``routed_experts`` hands their input through)."""
         T, stride = self._f32_rows(logits, "router logits")
         n = T * top
-        # larger row tiles once an expert has that many rows on average: its matrices are then read
-        # once per 64 or 128 rows instead of once per 16
+        # larger row tiles once an expert has that many rows on average (float32 has no kernel that would use them)
         per_expert = n / (experts if with_matrices is None else max(1, int(with_matrices)))
-        tile_rows = _TILE_ROWS[2] if per_expert >= 2 * self.ROUTED_WIDE_TILE_ROWS else \
-            (_TILE_ROWS[1] if per_expert >= self.ROUTED_WIDE_TILE_ROWS else _TILE_ROWS[0])
+        line = self.ROUTED_WIDE_TILE_ROWS if experts >= self.ROUTED_WIDE_EXPERTS else self.ROUTED_WIDE_TILE_ROWS_OF_FEW
+        wide = per_expert >= line and self.act_dtype == torch.bfloat16
+        tile_rows = _TILE_ROWS[int(wide)]
         max_tiles = -(-n // tile_rows) + experts
         chosen = self._new((T, top), torch.int32)
         shares = self._new((T, top), torch.float32)
         order = self._new((n,), torch.int32)
         place_of = self._new((n,), torch.int32)
-        tiles = self._new((max_tiles, 3), torch.int32)
+        tiles = self._new((max_tiles + 1, 3), torch.int32)[:max_tiles]      # (their number in use lies behind them)
         if correction is not None:
             self._check(correction, torch.float32, (experts,), "correction")
         real = experts if with_matrices is None else int(with_matrices)

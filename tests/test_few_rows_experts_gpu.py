@@ -37,3 +37,38 @@ def test_few_rows_an_expert(T, E, top, ff, K, form):
         # wide: at most three roundings (the activated row, its product, the result) of a value of this size
         bar = 3 * 2.0 ** -8 * want.float().abs().max().item()
         assert (got - want.float()).abs().max().item() <= bar
+
+
+# tiles of 128 rows: one and two chunks of 64 values of k, more than the ring holds, a number of steps of 32 that is odd
+# (the kernel beside it); column blocks of 128 (gated) and 256 with one tile of 16, and one more than whole; 12 rows an expert
+# and less for most, a second tile of one row, every token at the same expert (the others without tiles)
+@pytest.mark.parametrize("T,E,top,ff,K,one", [(12, 8, 8, 16, 64, False), (129, 8, 8, 144, 128, False), (300, 9, 1, 272, 320, True),
+                                              (100, 16, 2, 96, 192, False), (70, 8, 2, 128, 96, False), (400, 4, 1, 64, 64, False)])
+@pytest.mark.parametrize("form", ["gated", "plain", "weighed input"])
+def test_tiles_of_128_rows(T, E, top, ff, K, one, form):
+    hip, emu = HipOps(torch.bfloat16, DEV), EmulatedOps(torch.bfloat16)
+    g = torch.Generator().manual_seed(T + E)
+    gated = form != "plain"
+    x = torch.randn(T, K, generator=g).bfloat16()
+    first = (torch.randn(E, (2 if gated else 1) * ff, K, generator=g) * K ** -0.5).bfloat16()
+    down = (torch.randn(E, K, ff, generator=g) * ff ** -0.5).bfloat16()
+    logits = torch.randn(T, E, generator=g)
+    if one:
+        logits[:, 4] += 20.0
+    r = hip.route_tokens(logits.to(DEV), E, top, sigmoid=form == "weighed input")
+    assert r.tile_rows == 128
+    options = dict(activation="silu" if gated else "relu2", gated=gated, weigh_input=form == "weighed input")
+    want = emu.routed_experts(x, (r.chosen.cpu(), r.shares.cpu()), first, down, None, **options)
+    for a, b in ((first.to(DEV), down.to(DEV)),
+                 (hip.prepare_expert_matrices(first.to(DEV), gated=gated), hip.prepare_expert_matrices(down.to(DEV)))):
+        got = hip.routed_experts(x.to(DEV), r, a, b, None, **options).float().cpu()
+        # (as above)
+        bar = 3 * 2.0 ** -8 * want.float().abs().max().item()
+        assert (got - want.float()).abs().max().item() <= bar
+
+
+def test_rows_a_tile_holds():
+    hip = HipOps(torch.bfloat16, DEV)
+    rows = lambda T, E, top: hip.route_tokens(torch.randn(T, E, device=DEV), E, top).tile_rows
+    assert (rows(11, 8, 8), rows(12, 8, 8), rows(95, 4, 4), rows(96, 4, 4)) == (16, 128, 16, 128)
+    assert HipOps(torch.float32, DEV).route_tokens(torch.randn(200, 8, device=DEV), 8, 8).tile_rows == 16
