@@ -23,6 +23,11 @@
 // the weights of 8 consecutive keys of its column: the B operand of the second product as it is.
 // A step of single tokens has few columns (the heads of a group): its blocks are cut into shares
 // over workgroups, whose wavefronts without a column only help to stage.
+//
+// The widest form (576 / 512) holds one workgroup a CU, 132 matrix instructions a block and wavefront of which the
+// three of a channel tile depend on each other: what it waits for is not hidden by another wavefront, so loads stand
+// behind no condition, four channel tiles go side by side, and the longest tiles start first (two prompts of 945 tokens, 16
+// heads: 248 us before, 160 with the three; 128 / 128, 2,048 tokens: 137 and 112).
 #include "window_attention.h"
 
 #if defined(SL_F32)
@@ -76,17 +81,25 @@ constexpr int RCH = VK ? (DK - DV) / 8 : 0;            // chunks of a key row be
 constexpr int NT = VK ? cdiv((DV / 8) * 4, THREADS) : 1;   // 8 keys x 8 channels tiles a thread (turned on their way into LDS)
 constexpr int NR = VK ? (RCH ? cdiv(32 * RCH, THREADS) : 1) : 1;
 
-__global__ __launch_bounds__(THREADS) void window_attention_mfma_kernel(const WindowAttention a) {
+// (rows of up to 128 values: four workgroups a CU, which 128 registers allow)
+__global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_mfma_kernel(const WindowAttention a) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
   __bf16* ks = lds16;                                  // [32][KROW]
   __bf16* vt = ks + 32 * KROW;                         // [DV][VROW]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, gq = lane >> 4;
   const int page = a.page, nkv = a.nkv;
-  const int seq = blockIdx.z, kvh = blockIdx.y;
+  // Workgroups start in the order of their number: without a window the tiles with the most keys to walk (the last
+  // ones) of every sequence and head first, so that the short ones fill what is left at the end.  (Read back from a
+  // lane: a division is done in vector registers, and so would be all that follows from it.)
+  const int number = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), pairs = gridDim.y * gridDim.z;
+  const bool longest = a.window == 0 && a.chunk == 0;
+  const int seq = longest ? __builtin_amdgcn_readfirstlane(number % pairs / gridDim.y) : blockIdx.z;
+  const int kvh = longest ? __builtin_amdgcn_readfirstlane(number % pairs % gridDim.y) : blockIdx.y;
+  const int item = longest ? __builtin_amdgcn_readfirstlane(gridDim.x - 1 - number / pairs) : blockIdx.x;
   const int g = a.nh / nkv;
   const int q0 = a.cu_q[seq], qlen = a.cu_q[seq + 1] - q0;
   const int ncols = qlen * g;
-  const int tile = blockIdx.x / a.nsplit, share = blockIdx.x % a.nsplit;
+  const int tile = __builtin_amdgcn_readfirstlane(item / a.nsplit), share = item - tile * a.nsplit;
   const int c0 = tile * COLS;
   if (c0 >= ncols) return;
   const int pos0 = a.positions[q0];
@@ -137,13 +150,15 @@ __global__ __launch_bounds__(THREADS) void window_attention_mfma_kernel(const Wi
     const __bf16* qp = a.q + (size_t)(q0 + tok) * a.q_stride + (size_t)head * DK + 8 * gq;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) qf[kk] = *(const bf16x8*)(qp + 32 * kk);
+    // (waited for here: left to the loop, the wait for the first use of q would be one for the next block's keys as well)
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
   }
   f32x4 o[DD];
 #pragma unroll
   for (int dd = 0; dd < DD; ++dd) o[dd] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;                        // the maximum in units of log 2
   const __bf16 zero = (__bf16)0.f;
-  const bf16x8 zeros = {zero, zero, zero, zero, zero, zero, zero, zero};
 
   // A block travels pages -> registers -> LDS; the registers are filled for block i + 1 while block i
   // is computed from LDS.
@@ -155,58 +170,53 @@ __global__ __launch_bounds__(THREADS) void window_attention_mfma_kernel(const Wi
     const int key = kbase + ((lane & 1) << 4);
     return table[(key <= kmax ? key : kbase) >> page_shift];
   };
+  // A key no column sees is replaced by one of the block that some column does: no load stands behind a
+  // condition (the compiler waits for a load where the two ways meet, and eight rows a block are then eight trips to
+  // memory in turn), and what comes in its place gets no weight.
+  auto seen_in = [&](int key, int kbase) {
+    key = min(key, kmax);
+    return key >= kmin || key < keep ? key : (kmin <= kbase + 31 ? kmin : keep - 1);
+  };
   bf16x8 kreg[NKC], vreg[NVC], treg[NT][8], rreg[NR];
   auto fetch = [&](int kbase, int asked) {
     const int pgA = __builtin_amdgcn_readlane(asked, 0), pgB = __builtin_amdgcn_readlane(asked, 1);
     auto key_row = [&](int kl) {                       // start of the cache row of key kbase + kl
-      const int pg = kl < 16 ? pgA : pgB;
-      return a.kc + (((size_t)pg * nkv + kvh) * page + ((kbase + kl) & (page - 1))) * DK;
+      const int key = seen_in(kbase + kl, kbase), pg = key < kbase + 16 ? pgA : pgB;
+      return a.kc + (((size_t)pg * nkv + kvh) * page + (key & (page - 1))) * DK;
     };
     if constexpr (!VK) {
 #pragma unroll
       for (int i = 0; i < NKC; ++i) {
-        const int idx = tid + THREADS * i, kl = idx / KCH, c8 = idx % KCH;
-        kreg[i] = zeros;
-        if (idx < 32 * KCH && loadable(kbase + kl)) kreg[i] = *(const bf16x8*)(key_row(kl) + 8 * c8);
+        const int idx = min(tid + THREADS * i, 32 * KCH - 1);
+        kreg[i] = *(const bf16x8*)(key_row(idx / KCH) + 8 * (idx % KCH));
       }
 #pragma unroll
       for (int i = 0; i < NVC; ++i) {
-        const int idx = tid + THREADS * i, d = idx / 4, k8 = idx % 4, key0 = kbase + 8 * k8;
-        vreg[i] = zeros;
-        if (idx < DV * 4 && key0 <= kmax && (key0 + 7 >= kmin || key0 < keep)) {
-          const int pg = k8 < 2 ? pgA : pgB;
-          bf16x8 v = *(const bf16x8*)(a.vc + (((size_t)pg * nkv + kvh) * DV + d) * page + (key0 & (page - 1)));
-          if (!((key0 + 7 <= kmax && key0 >= kmin) || key0 + 7 < keep)) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)                // a slot of the page that holds no visible key may hold anything
-              if (!loadable(key0 + e)) v[e] = zero;
-          }
-          vreg[i] = v;
-        }
+        const int idx = min(tid + THREADS * i, DV * 4 - 1), d = idx / 4, key0 = kbase + 8 * (idx % 4);
+        // (a chunk of 8 keys with one that is seen, else the chunk of one that is)
+        const int key = key0 <= kmax && (key0 + 7 >= kmin || key0 < keep) ? key0 : seen_in(key0, kbase) & ~7;
+        const int pg = key < kbase + 16 ? pgA : pgB;
+        vreg[i] = *(const bf16x8*)(a.vc + (((size_t)pg * nkv + kvh) * DV + d) * page + (key & (page - 1)));
       }
     } else {
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
-        const int idx = tid + THREADS * i, cb = idx / 4, kg = idx % 4;
+        const int idx = min(tid + THREADS * i, (DV / 8) * 4 - 1), cb = idx / 4, kg = idx % 4;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          treg[i][j] = zeros;
-          if (idx < (DV / 8) * 4 && loadable(kbase + 8 * kg + j))
-            treg[i][j] = *(const bf16x8*)(key_row(8 * kg + j) + 8 * cb);
-        }
+        for (int j = 0; j < 8; ++j) treg[i][j] = *(const bf16x8*)(key_row(8 * kg + j) + 8 * cb);
       }
       if constexpr (RCH > 0) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-          const int idx = tid + THREADS * i, kl = idx / RCH, c8 = DV / 8 + idx % RCH;
-          rreg[i] = zeros;
-          if (idx < 32 * RCH && loadable(kbase + kl)) rreg[i] = *(const bf16x8*)(key_row(kl) + 8 * c8);
+          const int idx = min(tid + THREADS * i, 32 * RCH - 1), kl = idx / RCH, c8 = DV / 8 + idx % RCH;
+          rreg[i] = *(const bf16x8*)(key_row(kl) + 8 * c8);
         }
       }
     }
   };
-  auto store = [&]() {
+  auto store = [&](int kbase) {
     if constexpr (!VK) {
+      const bool all_seen = kbase + 31 <= kmax && (kbase >= kmin || kbase + 31 < keep);
 #pragma unroll
       for (int i = 0; i < NKC; ++i) {
         const int idx = tid + THREADS * i, kl = idx / KCH, c8 = idx % KCH;
@@ -215,7 +225,13 @@ __global__ __launch_bounds__(THREADS) void window_attention_mfma_kernel(const Wi
 #pragma unroll
       for (int i = 0; i < NVC; ++i) {
         const int idx = tid + THREADS * i, d = idx / 4, k8 = idx % 4;
-        if (idx < DV * 4) *(bf16x8*)(vt + d * VROW + 8 * k8) = vreg[i];
+        bf16x8 v = vreg[i];
+        if (!all_seen) {                               // a slot of the page that holds no visible key may hold anything
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (!loadable(kbase + 8 * k8 + e)) v[e] = zero;
+        }
+        if (idx < DV * 4) *(bf16x8*)(vt + d * VROW + 8 * k8) = v;
       }
     } else {
 #pragma unroll
@@ -251,7 +267,7 @@ __global__ __launch_bounds__(THREADS) void window_attention_mfma_kernel(const Wi
   for (int i = i0; i < i1; ++i) {
     const int kbase = block_base(i);
     __syncthreads();                                   // the last block's readers are done
-    store();
+    store(kbase);
     __syncthreads();
     if (i + 1 < i1) {
       fetch(block_base(i + 1), asked);
@@ -322,13 +338,19 @@ __global__ __launch_bounds__(THREADS) void window_attention_mfma_kernel(const Wi
     }
     const bf16x8 p1 = __builtin_bit_cast(bf16x8, w1), p2 = __builtin_bit_cast(bf16x8, w2),
                  p3 = __builtin_bit_cast(bf16x8, w3);
+    // (four tiles of channels side by side: the three products of one depend on each other)
+    constexpr int SIDE = DD % 4 == 0 ? 4 : 1;
 #pragma unroll
-    for (int dd = 0; dd < DD; ++dd) {
-      const bf16x8 vf = *(const bf16x8*)(vt + (16 * dd + n) * VROW + 8 * gq);
-      f32x4 acc = o[dd];
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p3, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p2, acc, 0, 0, 0);
-      o[dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p1, acc, 0, 0, 0);
+    for (int dd = 0; dd < DD; dd += SIDE) {
+      bf16x8 vf[SIDE];
+#pragma unroll
+      for (int u = 0; u < SIDE; ++u) vf[u] = *(const bf16x8*)(vt + (16 * (dd + u) + n) * VROW + 8 * gq);
+#pragma unroll
+      for (int u = 0; u < SIDE; ++u) o[dd + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[u], p3, o[dd + u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < SIDE; ++u) o[dd + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[u], p2, o[dd + u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < SIDE; ++u) o[dd + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[u], p1, o[dd + u], 0, 0, 0);
     }
   }
   if (!live) return;
