@@ -72,3 +72,37 @@ def test_rows_a_tile_holds():
     rows = lambda T, E, top: hip.route_tokens(torch.randn(T, E, device=DEV), E, top).tile_rows
     assert (rows(11, 8, 8), rows(12, 8, 8), rows(95, 4, 4), rows(96, 4, 4)) == (16, 128, 16, 128)
     assert HipOps(torch.float32, DEV).route_tokens(torch.randn(200, 8, device=DEV), 8, 8).tile_rows == 16
+
+
+# one workgroup for both up to 16 tokens and 1,024 experts, two kernels beyond; experts a wavefront adds up in one, two and
+# more rounds, some without matrices, equal logits, logits of minus infinity
+@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (1, 64, 8), (16, 65, 8), (17, 65, 8), (5, 300, 64), (16, 1024, 3), (16, 1025, 3)])
+@pytest.mark.parametrize("form", ["softmax", "over all", "sigmoid"])
+def test_routes_and_their_tiles(T, E, top, form):
+    hip = HipOps(torch.bfloat16, DEV)
+    g = torch.Generator().manual_seed(T + E)
+    z = torch.randn(T, E + 2, generator=g)[:, :E]
+    if E > 1:
+        z[0, E // 2] = z[0, 0] = 3.0
+    if E > 2 * top:
+        z[0, -top:] = -torch.inf
+    real = max(1, E - 1)
+    r = hip.route_tokens(z.to(DEV), E, top, over_all=form == "over all", with_matrices=real, sigmoid=form == "sigmoid")
+    number = torch.softmax(z, -1) if form == "over all" else z
+    order = torch.sort(-number, dim=-1, stable=True).indices[:, :top]
+    assert torch.equal(r.chosen.cpu().long(), order)
+    picked = number.gather(1, order).double()
+    want = torch.sigmoid(picked) if form == "sigmoid" else (
+        picked / (picked.sum(-1, keepdim=True) + 1e-20) if form == "over all" else torch.softmax(picked, -1))
+    # exponentials and a sum of at most 64 float terms
+    assert ((r.shares.cpu().double() - want).abs() <= 1e-5 * want + 1e-7).all()
+    flat, order, place = r.chosen.cpu().flatten().long(), r.order.cpu().long(), r.place_of.cpu().long()
+    assert torch.equal(order[place], torch.arange(T * top)) and (flat[order].diff() >= 0).all()
+    tiles, first = [], 0
+    for e in range(E):
+        n = int((flat == e).sum())
+        if e < real:
+            tiles += [[e, first + i, min(r.tile_rows, n - i)] for i in range(0, n, r.tile_rows)]
+        first += n
+    got = r.tiles.cpu()
+    assert got[:len(tiles)].tolist() == tiles and (got[len(tiles):] == 0).all()
