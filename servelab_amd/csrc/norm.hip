@@ -520,6 +520,10 @@ extern "C" const char* sl_add_into(float* resid, const void* delta, long long n,
 // RMS norm on a sublayer's output: resid (float, in place) += mult * y * rsqrt(mean(y^2) + eps) * w,
 // and the stream's new rows in the activation type for the sublayer that reads them next (out == nullptr:
 // they are not wanted).  y == nullptr: only those rows.  One block per row; sums and the stream in float.
+// A row is a few trips to memory in turn, so up to NORMED_KEEP values a thread of all that is read are asked for at
+// once, before the sum, and no load stands behind a condition, which would be waited for where the ways meet (8 rows of
+// 3,584 values: 6.4 us with a loop after the sum, 4.7 here).
+constexpr int NORMED_KEEP = 8;
 __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
                                     const float* __restrict__ w, act_t* __restrict__ out, int H, float eps,
                                     float mult) {
@@ -532,14 +536,36 @@ __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __re
     return;
   }
   const act_t* yr = y + r * H;
+  act_t yk[NORMED_KEEP];
+  float xk[NORMED_KEEP], wk[NORMED_KEEP];
+#pragma unroll
+  for (int u = 0; u < NORMED_KEEP; ++u) {
+    const int i = min((int)(threadIdx.x + u * blockDim.x), H - 1);
+    yk[u] = yr[i];
+    xk[u] = x[i];
+    wk[u] = w[i];
+  }
   float ss = 0.f;
-  for (int i = threadIdx.x; i < H; i += blockDim.x) {
+#pragma unroll
+  for (int u = 0; u < NORMED_KEEP; ++u) {
+    const float v = threadIdx.x + u * blockDim.x < H ? to_f(yk[u]) : 0.f;
+    ss += v * v;
+  }
+  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = to_f(yr[i]);
     ss += v * v;
   }
   ss = block_sum(ss, scratch);
   const float inv = 1.f / sqrtf(ss / (float)H + eps);
-  for (int i = threadIdx.x; i < H; i += blockDim.x) {
+#pragma unroll
+  for (int u = 0; u < NORMED_KEEP; ++u) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i >= H) break;
+    const float v = xk[u] + mult * (to_f(yk[u]) * inv * wk[u]);
+    x[i] = v;
+    if (o != nullptr) o[i] = from_f<act_t>(v);
+  }
+  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = x[i] + mult * (to_f(yr[i]) * inv * w[i]);
     x[i] = v;
     if (o != nullptr) o[i] = from_f<act_t>(v);
@@ -559,8 +585,8 @@ extern "C" const char* sl_add_postnorm(float* resid, const void* y, const float*
 // follows at once: v = resid + y * rsqrt(mean(y^2) + eps_y) * wy, out = v * rsqrt(mean(v^2) + eps) * w.
 // rows == nullptr: every row, and v goes back to the stream; else only the listed rows are computed
 // and the stream stays as it is (the head reads few rows of the last layer's result).  One block per
-// row, up to NORMED_KEEP values a thread kept in registers between the passes; all sums in float.
-constexpr int NORMED_KEEP = 8;
+// row, up to NORMED_KEEP values a thread asked for at once, as above, and kept in registers between the passes; all
+// sums in float (2 rows of 2,048 values: 6.0 us with loads after each sum, 4.4 here).
 __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
                                           const float* __restrict__ wy, float eps_y,
                                           const int* __restrict__ rows, const float* __restrict__ w, float eps,
@@ -570,12 +596,20 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   float* x = resid + r * H;
   const act_t* yr = y + r * H;
   act_t* o = out + (size_t)blockIdx.x * H;
-  float keep[NORMED_KEEP];
+  act_t yk[NORMED_KEEP];
+  float keep[NORMED_KEEP], xk[NORMED_KEEP], wyk[NORMED_KEEP], wk[NORMED_KEEP];
+#pragma unroll
+  for (int u = 0; u < NORMED_KEEP; ++u) {
+    const int i = min((int)(threadIdx.x + u * blockDim.x), H - 1);
+    yk[u] = yr[i];
+    xk[u] = x[i];
+    wyk[u] = wy[i];
+    wk[u] = w[i];
+  }
   float ss = 0.f;
 #pragma unroll
   for (int u = 0; u < NORMED_KEEP; ++u) {
-    const int i = threadIdx.x + u * blockDim.x;
-    keep[u] = i < H ? to_f(yr[i]) : 0.f;
+    keep[u] = threadIdx.x + u * blockDim.x < H ? to_f(yk[u]) : 0.f;
     ss += keep[u] * keep[u];
   }
   for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
@@ -589,7 +623,7 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   for (int u = 0; u < NORMED_KEEP; ++u) {
     const int i = threadIdx.x + u * blockDim.x;
     if (i < H) {
-      keep[u] = x[i] + keep[u] * inv_y * wy[i];
+      keep[u] = xk[u] + keep[u] * inv_y * wyk[u];
       if (rows == nullptr) x[i] = keep[u];
       s2 += keep[u] * keep[u];
     }
@@ -604,7 +638,7 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
 #pragma unroll
   for (int u = 0; u < NORMED_KEEP; ++u) {
     const int i = threadIdx.x + u * blockDim.x;
-    if (i < H) o[i] = from_f<act_t>(keep[u] * inv * w[i]);
+    if (i < H) o[i] = from_f<act_t>(keep[u] * inv * wk[u]);
   }
   for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = rows == nullptr ? x[i] : x[i] + to_f(yr[i]) * inv_y * wy[i];
