@@ -195,7 +195,8 @@ class ProductOps:
             return self.linear_tiled(x, weight.w, bias, out_f32)
         limit = self._few_rows_limit(weight)
         plan = self._block_plan(M, N, K, weight) or (
-            defer and self.fuse_norms and not out_f32 and self._shares_plan(M, N, K, weight))
+            defer and M > self.BLOCK_SQUARE_MAX_M and self.fuse_norms and not out_f32
+            and not self._tuned_for(M, N, K) and self._shares_plan(M, N, K, weight))
         if plan:
             # (deferred: the norm adds the partial sums)
             return self.linear_block(x, weight, bias, out_f32, plan[0],
@@ -322,7 +323,7 @@ class ProductOps:
         shares = self._num_cus // tiles
         return (shares, True) if 2 <= shares <= 3 and 4 * tiles * shares >= 3 * self._num_cus else None
 
-    def _gated_rows(self, M, N, K, weight):
+    def _gated_rows(self, M, N, K):
         """Rows of x a workgroup of the block kernel takes (256 or 192) for the gated product of a
         prompt, or None where the library's product and a pass that gates it are the faster pair.
         The kernel runs in rounds of one tile a CU, of which a half-filled one costs as much as a
@@ -342,6 +343,15 @@ class ProductOps:
         if K <= self.GATED_SHORT_K or (fill >= self.GATED_FILL and rounds[rows] == 1):
             return rows
         return rows if M >= self.GATED_ROUNDS_MIN_M and fill >= 0.75 else None
+
+    def _tuned_for(self, M, N, K) -> bool:
+        """Whether the library's product of this shape was timed over its candidates (``library_tuning``; inside
+        its block: whether it is about to be).  Those shapes stay with the library, whose default pick is
+        what the rules above were measured against: tuned it is up to a quarter faster."""
+        shape = (self.library_rows(M), N, K)
+        if self._tuning:
+            self._tuned.add(shape)
+        return shape in self._tuned
 
     def linear_gated_block(self, x, weight, bias, rows, act):
         """act(gate) * up of many rows over the row-major weight, tiles of ``rows`` x 256."""
@@ -470,7 +480,8 @@ class ProductOps:
             y = self._new((M, N // 2))
             self._skinny(x, weight, bias, y, M, N, K, gated=code)
             return y
-        rows = block == self.GATE_BLOCK and self._gated_rows(M, N, K, weight)
+        rows = (M >= 256 and block == self.GATE_BLOCK and not self._tuned_for(M, N, K)
+                and self._gated_rows(M, N, K))
         if rows:
             return self.linear_gated_block(x, weight, bias, rows, code)
         return self.gate_mul(self.linear(x, weight, bias), block, activation)
@@ -656,7 +667,9 @@ class ProductOps:
         tunable.set_max_tuning_duration(int(max_ms))
         tunable.enable(True)
         tunable.tuning_enable(True)
+        self._tuning = True
         try:
             yield
         finally:
+            self._tuning = False
             tunable.tuning_enable(False)           # the choices made stay in use; nothing new is timed

@@ -40,13 +40,12 @@ def test_gated_tiles(M, N, K, act, rows):
 
 def test_routes_of_prompts_products():
     ops = HipOps(torch.bfloat16, DEV)
-    big = ops.prepare_weight(torch.zeros(8192, 1088, dtype=torch.bfloat16, device=DEV))
-    assert ops._gated_rows(255, 8192, 1024, big) is None and ops._gated_rows(256, 8192, 1024, big) == 192
-    assert ops._gated_rows(256, 8192, 1088, big) is None                         # a round filled to a sixth
-    assert ops._gated_rows(1536, 8192, 2048, big) == 192                         # 256 tiles of 192 rows: one full round
-    assert ops._gated_rows(1537, 8192, 2048, big) == 256                         # 224 tiles of 256
-    assert ops._gated_rows(1600, 37888, 3584, big) is None and ops._gated_rows(2048, 37888, 3584, big) == 256
-    assert ops._gated_rows(2561, 37888, 3584, big) is None and ops._gated_rows(2048, 8192, 2080, big) is None
+    assert ops._gated_rows(255, 8192, 1024) is None and ops._gated_rows(256, 8192, 1024) == 192
+    assert ops._gated_rows(256, 8192, 1088) is None                         # a round filled to a sixth
+    assert ops._gated_rows(1536, 8192, 2048) == 192                         # 256 tiles of 192 rows: one full round
+    assert ops._gated_rows(1537, 8192, 2048) == 256                         # 224 tiles of 256
+    assert ops._gated_rows(1600, 37888, 3584) is None and ops._gated_rows(2048, 37888, 3584) == 256
+    assert ops._gated_rows(2561, 37888, 3584) is None and ops._gated_rows(2048, 8192, 2080) is None
     x = torch.randn(300, 1024, device=DEV).bfloat16()
     w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
     weight = ops.prepare_weight(w)
@@ -64,3 +63,19 @@ def test_routes_of_prompts_products():
     # float sums of K terms: K 2^-24 of their absolute sum
     assert ((delta.parts.double().sum(0) - want).abs() <= K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
     assert not isinstance(ops.linear(x, weight, None), PartialSums)
+
+
+def test_shapes_tuned_for_the_library_stay_with_it(tmp_path):
+    ops = HipOps(torch.bfloat16, DEV)
+    w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
+    weight, x = ops.prepare_weight(w), torch.randn(300, 1024, device=DEV).bfloat16()
+    calls = []
+    gated = ops.linear_gated_block
+    ops.linear_gated_block = lambda *a: calls.append(a[0].shape[0]) or gated(*a)
+    ops._tuning = True                                        # (what the block of library_tuning sets)
+    ops.gated_linear(x, weight, 8)
+    ops._tuning = False
+    ops.gated_linear(x, weight, 8)
+    assert calls == []
+    ops.gated_linear(torch.cat([x, x]), weight, 8)            # another number of rows: not tuned
+    assert calls == [600]
