@@ -21,6 +21,7 @@
 // delta with a decay a head 605 -> 133 (32 + 106); state-space, 64 heads of 128 x 64 in 8 groups: 535 -> 116 (34 + 86).
 // The walk is bound by its chain: 1.2 to 1.6 us a chunk, of which the products are 0.6 to 0.8.
 #pragma once
+#include <type_traits>
 
 typedef float scan_v4 __attribute__((ext_vector_type(4)));
 constexpr int SCAN_CHUNK = 32;
@@ -98,6 +99,32 @@ __device__ __forceinline__ void scan_rows(int Dp, int tid, Load load, Keep keep)
   }
 }
 
+// Products of a triangle: t reads s <= t, and the zeros above the diagonal are in the matrix instruction all the same, where an
+// infinity or NaN of a later token turns them into NaN.  Whoever finds a result that is not finite (scan_odd gathers that
+// without a branch) therefore takes the products again with these sums, which leave the zeros out.  An operand's block is 16 x 16,
+// its row at lane row + 16 (column / 4), place column % 4; TRIANGLE_FIRST: `x` is the triangle, else `y` is, turned.
+__device__ __forceinline__ float scan_odd(float odd, const scan_v4& result) {
+  return fmaf((result[0] + result[1]) + (result[2] + result[3]), 0.f, odd);   // (0, or NaN from the first such result on)
+}
+template <bool TRIANGLE_FIRST>
+__device__ __forceinline__ scan_v4 scan_lower_only(const scan_v4& x, const scan_v4& y, int lane) {
+  const int n = lane & 15, r0 = 4 * (lane >> 4);
+  scan_v4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int from = 0; from < 64; from += 16)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int s = from / 4 + c;
+      const float ys = __shfl(y[c], from + n, SL_WAVE);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float xs = __shfl(x[c], from + r0 + i, SL_WAVE);
+        if (s <= (TRIANGLE_FIRST ? r0 + i : n)) sum[i] = fmaf(xs, ys, sum[i]);
+      }
+    }
+  return sum;
+}
+
 // A 32 x 32 square of LDS as the walk's first operand.
 __device__ __forceinline__ void scan_square_out(const float* As, float* out, int tid) {
   const int l = tid & 63, r = tid >> 7, j = (tid >> 6) & 1;
@@ -140,6 +167,7 @@ __device__ __forceinline__ void scan_delta_rows(const MatrixScan& a, const ScanC
     // (the first product's results lie as the second one's operand)
 #pragma unroll
     for (int i = 0; i < 4; ++i) below = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[i], acc[i], below, 0, 0, 0);
+    if (__ballot(scan_odd(0.f, below) != 0.f)) below = scan_lower_only<true>(rv, acc, lane);
 #pragma unroll
     for (int i = 0; i < 4; ++i) As[(16 + 4 * gq + i) * AR + n] = -below[i];
   }
@@ -152,38 +180,49 @@ __device__ __forceinline__ void scan_delta_rows(const MatrixScan& a, const ScanC
       rv[r][j] = *(const scan_v4*)(As + (16 * r + n) * AR + 16 * j + 4 * gq) * *(const scan_v4*)(beta + 16 * j + 4 * gq);
   const int vblocks = (a.Dv + 15) / 16;
   float* vout = c.vt + ((size_t)chunk * a.H + h) * vblocks * 512;
-  for (int blk = wave; blk < vblocks; blk += 4) {
-    const int col = 16 * blk + n;
-    float v[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = 16 * j + 4 * gq + i;
-        v[j][i] = t < nt && col < a.Dv ? a.src[(size_t)(first + t) * a.src_stride + a.v_col + h * a.Dv + col] : 0.f;
-      }
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      scan_v4 acc[2] = {};
-#pragma unroll
-      for (int j = 0; j <= r; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[r][j][i], v[j][i], acc[j], 0, 0, 0);
-      *(scan_v4*)(vout + ((size_t)blk * 2 + r) * 256 + lane * 4) = acc[0] + acc[1];
-    }
-  }
   float* wout = c.w + ((size_t)chunk * a.H + h) * blocks * 512;
-  for (int blk = wave; blk < blocks; blk += 4)          // W turned: rows are channels, columns tokens
+  float odd = 0.f;
+  auto rows = [&](auto careful) {
+    for (int blk = wave; blk < vblocks; blk += 4) {
+      const int col = 16 * blk + n;
+      scan_v4 v[2];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      scan_v4 acc[2] = {};
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int j = 0; j <= r; ++j)
+        for (int i = 0; i < 4; ++i) {
+          const int t = 16 * j + 4 * gq + i;
+          v[j][i] = t < nt && col < a.Dv ? a.src[(size_t)(first + t) * a.src_stride + a.v_col + h * a.Dv + col] : 0.f;
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(16 * j + 4 * gq + i) * row + 16 * blk + n], rv[r][j][i], acc[j], 0, 0, 0);
-      *(scan_v4*)(wout + ((size_t)blk * 2 + r) * 256 + lane * 4) = acc[0] + acc[1];
+      for (int r = 0; r < 2; ++r) {
+        scan_v4 acc[2] = {};
+#pragma unroll
+        for (int j = 0; j <= r; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[r][j][i], v[j][i], acc[j], 0, 0, 0);
+        if (careful) acc[r] = scan_lower_only<true>(rv[r][r], v[r], lane);
+        else odd = scan_odd(odd, acc[r]);
+        *(scan_v4*)(vout + ((size_t)blk * 2 + r) * 256 + lane * 4) = acc[0] + acc[1];
+      }
     }
+    for (int blk = wave; blk < blocks; blk += 4)        // W turned: rows are channels, columns tokens
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        scan_v4 acc[2] = {}, kv;
+#pragma unroll
+        for (int j = 0; j <= r; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) kv[i] = ks[(16 * j + 4 * gq + i) * row + 16 * blk + n];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], rv[r][j][i], acc[j], 0, 0, 0);
+        }
+        if (careful) acc[r] = scan_lower_only<false>(kv, rv[r][r], lane);
+        else odd = scan_odd(odd, acc[r]);
+        *(scan_v4*)(wout + ((size_t)blk * 2 + r) * 256 + lane * 4) = acc[0] + acc[1];
+      }
+  };
+  rows(std::false_type{});
+  if (__ballot(odd != 0.f)) rows(std::true_type{});
 }
 
 // One decay a head: a workgroup per (chunk, group of heads, sequence), since the products of q and k are the group's; a
@@ -391,7 +430,7 @@ __global__ __launch_bounds__(256) void scan_prepare_channel_kernel(const MatrixS
       k = in ? (1.f - bound) * (pos ? small : big) : 0.f;
       q = q * sigmoidf_(q);
     } else {
-      l = fmaxf(l, -110.f);                             // (e^-110 is 0 in float)
+      l = l < -110.f ? -110.f : l;                      // (e^-110 is 0 in float; NaN stays NaN)
     }
     qs[tt * row + d] = q * a.q_scale;
     ks[tt * row + d] = k;
@@ -560,10 +599,11 @@ __global__ __launch_bounds__(256) void scan_prepare_channel_kernel(const MatrixS
 // operand, so q^T S and W S need no exchange but the sum over the wavefronts (through LDS, one barrier a chunk).
 // The operands of the chunks ahead are asked for while one is worked on.
 template <int MODE, int TW>
-__global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, const ScanChunks c, int S, int slices) {
+__global__ __launch_bounds__(256, ScanForm<MODE>::DELTA && TW > 1 ? 1 : 2) void scan_walk_kernel(const MatrixScan a, const ScanChunks c, int S, int slices) {
   constexpr bool SCALAR = ScanForm<MODE>::SCALAR, DELTA = ScanForm<MODE>::DELTA;
   constexpr int C = SCAN_CHUNK, NP = DELTA ? 4 : 2;
   __shared__ scan_v4 part[2][4][NP][64];
+  __shared__ bool again[2];
   // Workgroups go to the eight dies in turn: the slices of a head, which read the same operands, run on one of them.
   const int die = blockIdx.x & 7, rest = blockIdx.x >> 3, slice = rest % slices, hs = rest / slices * 8 + die;
   if (hs >= S * a.H) return;
@@ -581,13 +621,16 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, cons
   float* srow = is_n ? slot + (size_t)a.H * a.Dv * a.D + (size_t)h * a.D : slot + ((size_t)h * a.Dv + (live ? col : 0)) * a.D;
   const int blocks = c.Dp / 16, vblocks = (a.Dv + 15) / 16;
   scan_v4 st[TW];
+  auto begin = [&]() {
 #pragma unroll
-  for (int b = 0; b < TW; ++b)
+    for (int b = 0; b < TW; ++b)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 16 * (wave * TW + b) + 4 * gq + i;
-      st[b][i] = !fresh && live && d < a.D ? srow[d] : 0.f;
-    }
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (wave * TW + b) + 4 * gq + i;
+        st[b][i] = !fresh && live && d < a.D ? srow[d] : 0.f;
+      }
+  };
+  begin();
   const float skip = MODE == SCAN_SSD ? a.skip[h] : 0.f;
 
   struct Chunk {
@@ -613,7 +656,7 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, cons
 #pragma unroll
       for (int j = 0; j < 2; ++j) x.v[j] = *(const scan_v4*)(vt + j * 256 + lane * 4);
     } else {
-      // (beyond the sequence's last token its row again: what multiplies it is 0)
+      // (beyond the sequence's last token its row again: it is not used)
       const int t0 = ci * C, last = len - 1 - t0;
       const float* v = a.src + (size_t)(first + t0) * a.src_stride + a.v_col + h * a.Dv;
 #pragma unroll
@@ -640,7 +683,8 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, cons
     for (int j = 0; j < 2; ++j) x.a[j] = *(const scan_v4*)(c.a + ah * 1024 + (wave & 1) * 512 + j * 256 + lane * 4);
   };
 
-  auto step = [&](int ci, Chunk& now) {
+  float odd = 0.f;
+  auto step = [&](int ci, Chunk& now, auto careful) {
     scan_v4(*buf)[NP][64] = part[ci & 1];
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
@@ -662,6 +706,13 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, cons
     __syncthreads();                                    // (the other half was read before the barrier ahead of this one)
     scan_v4 u[2] = {now.v[0], now.v[1]};
     if (is_n) u[0] = u[1] = scan_v4{1.f, 1.f, 1.f, 1.f};   // (tokens beyond the last: A and the factors of k are 0)
+    if (careful && !DELTA) {                            // (the last row again may be infinite, which 0 does not take out)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (ci * C + 16 * j + 4 * gq + i >= len) u[j][i] = 0.f;
+    }
     if (DELTA) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) u[j] -= (buf[0][2 + j][lane] + buf[1][2 + j][lane]) + (buf[2][2 + j][lane] + buf[3][2 + j][lane]);
@@ -691,7 +742,10 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, cons
         if (j <= wave)
 #pragma unroll
           for (int i = 0; i < 4; ++i) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a[j][i], u[j][i], own[j], 0, 0, 0);
+      if (careful && wave == 0) own[0] = scan_lower_only<true>(now.a[0], u[0], lane);
+      if (careful && wave == 1) own[1] = scan_lower_only<true>(now.a[1], u[1], lane);
       o += own[0] + own[1];
+      if (!careful) odd = scan_odd(odd, o);
       const int t = ci * C + 16 * wave;
       float* out = a.out + ((size_t)(first + t) * a.H + h) * a.Dv;
 #pragma unroll
@@ -717,10 +771,23 @@ __global__ __launch_bounds__(256) void scan_walk_kernel(const MatrixScan a, cons
         done = true;
         break;
       }
-      step(c0 + i, ring[i]);
+      step(c0 + i, ring[i], std::false_type{});
       ask(min(c0 + i + AHEAD, nchunks - 1), ring[i]);
     }
     if (done) break;
+  }
+  if (wave < 2) {
+    const bool any = __ballot(odd != 0.f) != 0;
+    if (lane == 0) again[wave] = any;
+  }
+  __syncthreads();
+  if (again[0] || again[1]) {                           // from the start again, a chunk at a time, the read-outs with care
+    begin();
+#pragma unroll 1
+    for (int ci = 0; ci < nchunks; ++ci) {
+      ask(ci, ring[0]);
+      step(ci, ring[0], std::true_type{});
+    }
   }
   if (!a.write || !live) return;
   float* to = srow;

@@ -145,3 +145,40 @@ def test_scan_in_chunks(mode, strong, H, G, D, Dv):
         close(o1, o2, 2e-5)
     close(s1[:, :size], s2[:, :size], 2e-5)
     assert torch.equal(torch.nan_to_num(s1.cpu()[:, size:], 9.0), torch.nan_to_num(state[:, size:], 9.0))
+
+
+# a token in the middle of a block of 16, the last one of a chunk that is not full, the last one of a sequence
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 2, 72, 15), (4, 2, 64, 40)])
+@pytest.mark.parametrize("what", ["value", "key", "decay"])
+@pytest.mark.parametrize("mode", ["decay", "delta", "delta, decay a head", "state space", "forget", "lstm"])
+def test_chunks_keep_infinities_and_nan_from_earlier_tokens(mode, what, H, G, D, Dv):
+    """What is not finite in the walk token by token is not finite in chunks, and nothing else."""
+    if mode in ("forget", "lstm"):
+        G = H
+    if mode == "forget" and what == "decay":
+        what = "key"                                       # (its decays come from the keys)
+    hip = HipOps(torch.float32, DEV)
+    call, size, _ = scan_case(mode, H, G, D, Dv, False)
+    inputs = dict(zip(call.__code__.co_freevars, (c.cell_contents for c in call.__closure__)))
+    src, gates, log_decay = inputs["src"], inputs["gates"], inputs["log_decay"]
+    first = [sum(Q_LENS[:i]) for i in range(len(Q_LENS))]
+    for t in (first[5] + 40, first[5] + 75, first[3] + 32, first[4] + 6, first[6] + 18):
+        if what == "value":
+            src[t, 2 * G * D + 3] = float("inf")
+        elif what == "key":
+            src[t, G * D + 5] = float("nan")
+        elif mode in ("decay", "delta"):
+            log_decay[t, 7] = float("nan")
+        else:
+            gates[t, H if mode != "state space" else H] = float("nan")
+    state = torch.randn(len(SLOTS), size, generator=torch.Generator().manual_seed(6)) * 0.3
+    out, states = [], []
+    for line in (1, 1 << 30):                              # in chunks, token by token
+        hip.SCAN_CHUNKS_FROM = hip.SCAN_CHUNKS_FROM_GROUPED = hip.SCAN_CHUNKS_FROM_MANY = line
+        states.append(state.clone().to(DEV))
+        out.append(call(hip, states[-1], sequences(Q_LENS, STARTS, SLOTS, DEV), DEV))
+    assert not torch.isfinite(out[1]).all()
+    for a, b in (out, states):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+        if mode != "lstm" or a is not out[0]:              # (its read-outs are quotients: measured in test_scan_in_chunks)
+            close(torch.nan_to_num(a, 0.0, 0.0, 0.0), torch.nan_to_num(b, 0.0, 0.0, 0.0), 2e-5)
