@@ -782,6 +782,7 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
 // The matrix LSTM's n and m to their slots, behind the scan whose blocks have all read the old ones.
 __global__ void normaliser_kernel(const MatrixScan a) {
   const int s = blockIdx.x, h = blockIdx.y;
+  if (a.cu_q[s + 1] <= a.cu_q[s]) return;               // (no token: nothing waits there, the slot stays as it is)
   float* slot = a.state + (size_t)a.slots[s] * a.state_stride + (size_t)a.H * a.Dv * a.D;
   const float* from = a.normaliser + ((size_t)s * a.H + h) * (a.D + 1);
   for (int d = threadIdx.x; d < a.D; d += blockDim.x) slot[(size_t)h * a.D + d] = from[d];

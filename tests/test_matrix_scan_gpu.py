@@ -182,3 +182,19 @@ def test_chunks_keep_infinities_and_nan_from_earlier_tokens(mode, what, H, G, D,
         assert torch.equal(torch.isfinite(a), torch.isfinite(b))
         if mode != "lstm" or a is not out[0]:              # (its read-outs are quotients: measured in test_scan_in_chunks)
             close(torch.nan_to_num(a, 0.0, 0.0, 0.0), torch.nan_to_num(b, 0.0, 0.0, 0.0), 2e-5)
+
+
+def test_a_sequence_without_tokens_keeps_its_normaliser():
+    """In chunks nothing is computed for it, so nothing may be copied to its slot either."""
+    H, D, Dv, q_lens, starts = 2, 20, 24, [40, 0, 33], [0, 7, 3]
+    hip = HipOps(torch.float32, DEV)
+    hip.SCAN_CHUNKS_FROM = hip.SCAN_CHUNKS_FROM_MANY = 1
+    g = torch.Generator().manual_seed(9)
+    width = 2 * H * D + H * Dv
+    buf = torch.randn(sum(q_lens), width + 2 * H, generator=g).to(DEV)
+    state = torch.randn(3, H * D * Dv + H * D + H, generator=g).to(DEV)
+    before = state.clone()
+    hip.mlstm_scan(buf, 0, H * D, 2 * H * D, width, width + H, H, D, Dv, 15.0, D ** -0.5, state,
+                   sequences(q_lens, starts, [2, 0, 1], DEV), True)
+    assert torch.equal(state[0], before[0])
+    assert (state[1:] != before[1:]).all(1).all()
