@@ -131,13 +131,14 @@ __global__ __launch_bounds__(64) void route_kernel(const Route r) { route_token(
 // ------------------------------------------------------------------ group
 // One workgroup sorts the n = tokens * top pairs by expert (counting sort in LDS: 3 E numbers at `sh`).
 //   order[place] = pair (token * top + choice);  place_of[pair] = place
-//   tiles[i] = {expert, first row, rows} for i < tiles in use; rows 0 beyond; tiles[max_tiles][0] = tiles in use
+//   tiles[i] = {expert, first row, rows} for i < tiles in use; rows 0 beyond; used[0] = tiles in use
 // Experts from E_real on have no matrices: their pairs get places but no tiles.
 struct Group {
   int n, E, E_real, max_tiles, tile_rows;
   int* order;
   int* place_of;
   int* tiles;
+  int* used;
 };
 
 __device__ __forceinline__ void group_pairs(const Group& g, const int* chosen, int* sh) {
@@ -171,7 +172,7 @@ __device__ __forceinline__ void group_pairs(const Group& g, const int* chosen, i
       rows += __shfl(up_rows, 63, SL_WAVE);
       nt += __shfl(up_tiles, 63, SL_WAVE);
     }
-    if (tid == 0) tiles[3 * g.max_tiles] = nt;
+    if (tid == 0) *g.used = nt;
     for (int i = nt + tid; i < g.max_tiles; i += 64) {
       tiles[3 * i] = 0;
       tiles[3 * i + 1] = 0;
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(1024) void route_group_kernel(const Route r, const 
 }
 
 extern "C" const char* sl_route_tokens(const float* logits, int stride, int T, int E, int top, int* chosen,
-                                       float* shares, int* order, int* place_of, int* tiles, int max_tiles,
+                                       float* shares, int* order, int* place_of, int* tiles, int* used, int max_tiles,
                                        int tile_rows, int over_all, const float* correction, float scale,
                                        int E_real, int sigmoid, hipStream_t stream) {
   SL_CHECK(!(over_all && sigmoid), "route_tokens: shares over all or sigmoids");
@@ -228,7 +229,7 @@ extern "C" const char* sl_route_tokens(const float* logits, int stride, int T, i
   SL_CHECK(max_tiles >= ((long long)T * top + tile_rows - 1) / tile_rows + E, "route_tokens: too few tile entries");
   if (T == 0) return nullptr;
   const Route r{logits, stride, E, top, chosen, shares, over_all, correction, scale, sigmoid};
-  const Group g{T * top, E, E_real, max_tiles, tile_rows, order, place_of, tiles};
+  const Group g{T * top, E, E_real, max_tiles, tile_rows, order, place_of, tiles, used};
   if (T <= 16 && E <= 1024) {
     route_group_kernel<<<1, 64 * T, (3 * E + T * top) * sizeof(int), stream>>>(r, g);
   } else {
@@ -254,7 +255,7 @@ struct Grouped {
   int act;                   // the activation (common.h); 0 with out_f32
   float limit;               // the clamped gate's bound
   const float* row_scale;    // with order: the sums of row r are multiplied by row_scale[order[r]] first; or nullptr
-  const int* used;           // how many of the tiles are in use
+  const int* used;           // how many of the tiles are in use, which then come first; nullptr: any of them may be
   int max_tiles, col_blocks; // the matrix-core kernels' launch: max_tiles x col_blocks workgroups in a row
 };
 
@@ -277,7 +278,7 @@ __device__ __forceinline__ bool grouped_place(const Grouped& a, int& tile, int& 
 // 2,048 x 1,024, gate/up, down and the sum, 8 of them a token: 256 / 1,000 / 2,048 tokens 196 / 254 / 360 us by column
 // blocks, 162 / 231 / 359 by tiles).
 __device__ __forceinline__ bool grouped_place_by_rows(const Grouped& a, int& tile, int& cb) {
-  const int total = min(*a.used, a.max_tiles) * a.col_blocks, run = (total + 7) / 8;
+  const int total = (a.used != nullptr ? min(*a.used, a.max_tiles) : a.max_tiles) * a.col_blocks, run = (total + 7) / 8;
   const int m = (blockIdx.x & 7) * run + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= run || m >= total) return false;
   tile = m / a.col_blocks;
@@ -658,8 +659,8 @@ __global__ __launch_bounds__(512) void grouped_product_staged_kernel(const Group
 #endif
 
 extern "C" const char* sl_grouped_product(const void* x, const int* order, int top, const void* w, const int* tiles,
-                                          int w_tiled, int max_tiles, int tile_rows, int pairs, int experts, int N,
-                                          int K, int gated, int act, float limit, const float* row_scale, void* out, hipStream_t stream) {
+                                          const int* used, int w_tiled, int max_tiles, int tile_rows, int pairs, int experts,
+                                          int N, int K, int gated, int act, float limit, const float* row_scale, void* out, hipStream_t stream) {
   // gated: act(gate) * up into the activation type; else act != 0: act(W x) into the activation type;
   // else plain float sums
   SL_CHECK(max_tiles >= 0 && N > 0 && K > 0 && top >= 1, "grouped_product: sizes must be positive");
@@ -669,8 +670,7 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
   SL_CHECK(tile_rows == 16 || tile_rows == 128, "grouped_product: row tiles hold 16 or 128 rows");
   SL_CHECK(pairs >= 0 && experts >= 0, "grouped_product: sizes must be positive");
   if (max_tiles == 0 || pairs == 0) return nullptr;
-  const int* used = tiles + 3 * (size_t)max_tiles;
-  max_tiles = min(max_tiles, pairs);                    // (the tiles in use come first, and each holds a pair)
+  if (used != nullptr) max_tiles = min(max_tiles, pairs);         // (the tiles in use come first, and each holds a pair)
   Grouped a{(const act_t*)x, order, top, (const act_t*)w, w_tiled, tiles, tile_rows / RT_ROWS, N, K,
             act ? (act_t*)out : nullptr, act ? nullptr : (float*)out, act, limit, row_scale, used, max_tiles, 1};
 #if !defined(SL_F32)

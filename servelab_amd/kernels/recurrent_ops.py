@@ -7,7 +7,7 @@ What is float32 here in both activation types: the input projections' sums as th
 them, gates, decays and their logarithms, unit norms, states, read-outs, router logits and
 shares, the experts' weighted sum."""
 import ctypes
-from typing import NamedTuple
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -24,13 +24,15 @@ class Routing(NamedTuple):
     """A step's routing on the device: per token the chosen experts [T, top] (int32) and their
     shares (float32); the (token, choice) pairs sorted by expert (``order`` [T top], ``place_of``
     its inverse) and the row tiles [max_tiles, 3] = (expert, first row, rows) of at most
-    ``tile_rows`` rows that the grouped products walk."""
+    ``tile_rows`` rows that the grouped products walk.  ``tiles_in_use`` [1] (int32): so many of them, the
+    first ones, hold rows; None: every one is looked at (0 rows: none to walk)."""
     chosen: torch.Tensor
     shares: torch.Tensor
     order: torch.Tensor
     place_of: torch.Tensor
     tiles: torch.Tensor
     tile_rows: int
+    tiles_in_use: Optional[torch.Tensor] = None
 
 
 class ExpertMatrices:
@@ -408,14 +410,14 @@ class RecurrentOps:
         shares = self._new((T, top), torch.float32)
         order = self._new((n,), torch.int32)
         place_of = self._new((n,), torch.int32)
-        tiles = self._new((max_tiles + 1, 3), torch.int32)[:max_tiles]      # (their number in use lies behind them)
+        tiles, used = self._new((max_tiles, 3), torch.int32), self._new((1,), torch.int32)
         if correction is not None:
             self._check(correction, torch.float32, (experts,), "correction")
         real = experts if with_matrices is None else int(with_matrices)
         self._call(self._lazy("routed"), "sl_route_tokens", _p(logits), stride, T, experts, top, _p(chosen),
-                   _p(shares), _p(order), _p(place_of), _p(tiles), max_tiles, tile_rows, int(bool(over_all)),
+                   _p(shares), _p(order), _p(place_of), _p(tiles), _p(used), max_tiles, tile_rows, int(bool(over_all)),
                    _p(correction), _c_float(scale), real, int(bool(sigmoid)))
-        return Routing(chosen, shares, order, place_of, tiles, tile_rows)
+        return Routing(chosen, shares, order, place_of, tiles, tile_rows, used)
 
     def prepare_expert_matrices(self, w, gated=False):
         """Called once per stack of expert matrices [E, N, K] at load: what ``routed_experts`` takes.
@@ -473,12 +475,12 @@ class RecurrentOps:
         lib = self._lazy("routed")
         mid = self._new((n, ff))
         self._call(lib, "sl_grouped_product", _p(x), _p(routing.order), top, _p(w_gate_up.data),
-                   _p(routing.tiles), int(w_gate_up.tiled), max_tiles, routing.tile_rows, n, E, ff, K, int(bool(gated)),
-                   code, _c_float(limit), _p(routing.shares) if weigh_input else None, _p(mid))
+                   _p(routing.tiles), _p(routing.tiles_in_use), int(w_gate_up.tiled), max_tiles, routing.tile_rows,
+                   n, E, ff, K, int(bool(gated)), code, _c_float(limit), _p(routing.shares) if weigh_input else None, _p(mid))
         y = self._new((n, K), torch.float32)
         self._call(lib, "sl_grouped_product", _p(mid), None, 1, _p(w_down.data), _p(routing.tiles),
-                   int(w_down.tiled), max_tiles, routing.tile_rows, n, E, K, ff, 0, 0, _c_float(0.0), None,
-                   _p(y))
+                   _p(routing.tiles_in_use), int(w_down.tiled), max_tiles, routing.tile_rows, n, E, K, ff, 0, 0,
+                   _c_float(0.0), None, _p(y))
         out = self._new((T, K))
         gate_at = None
         if base_gate is not None:

@@ -5,6 +5,7 @@ import torch
 
 from emulated_ops import EmulatedOps
 from servelab_amd.kernels import HipOps
+from servelab_amd.kernels.recurrent_ops import Routing
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -106,3 +107,18 @@ def test_routes_and_their_tiles(T, E, top, form):
         first += n
     got = r.tiles.cpu()
     assert got[:len(tiles)].tolist() == tiles and (got[len(tiles):] == 0).all()
+
+
+@pytest.mark.parametrize("T,tile_rows", [(5, 16), (100, 128)])
+def test_a_routing_put_together_by_a_caller(T, tile_rows):
+    """Its tiles need not come from the router's buffer, nor the ones with rows first."""
+    E, top, ff, K = 8, 2, 48, 64
+    hip = HipOps(torch.bfloat16, DEV)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, K, generator=g).bfloat16().to(DEV)
+    first = hip.prepare_expert_matrices((torch.randn(E, 2 * ff, K, generator=g) * K ** -0.5).bfloat16().to(DEV), gated=True)
+    down = hip.prepare_expert_matrices((torch.randn(E, K, ff, generator=g) * ff ** -0.5).bfloat16().to(DEV))
+    r = hip.route_tokens(torch.randn(T, E, generator=g).to(DEV), E, top)
+    assert r.tile_rows == tile_rows and r.tiles_in_use.item() == (r.tiles[:, 2] > 0).sum().item()
+    own = Routing(r.chosen, r.shares, r.order, r.place_of, r.tiles.flip(0).contiguous(), tile_rows)
+    assert torch.equal(hip.routed_experts(x, own, first, down), hip.routed_experts(x, r, first, down))
