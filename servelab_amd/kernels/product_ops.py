@@ -4,6 +4,7 @@ library for the bfloat16 table's large steps; float32 kernels for the float32 ta
 import contextlib
 import ctypes
 import os
+import re
 import tempfile
 from typing import Optional
 
@@ -11,6 +12,12 @@ import torch
 
 from .values import (Deferred, KernelError, LinearWeight, PartialSums, ScaledRows, TiledRows,
                      _c_float, _p, activation_code)
+
+
+def tuned_shapes(results):
+    """(rows, N, K) of the bfloat16 products x w^T among TunableOp's ``results`` (operation, parameters, solution, time)."""
+    found = (re.match(r"tn_(\d+)_(\d+)_(\d+)_", r[1]) for r in results if r[0].endswith("_BFloat16_TN"))
+    return {(int(m[2]), int(m[1]), int(m[3])) for m in found if m}
 
 
 class ProductOps:
@@ -345,13 +352,10 @@ class ProductOps:
         return rows if M >= self.GATED_ROUNDS_MIN_M and fill >= 0.75 else None
 
     def _tuned_for(self, M, N, K) -> bool:
-        """Whether the library's product of this shape was timed over its candidates (``library_tuning``; inside
-        its block: whether it is about to be).  Those shapes stay with the library, whose default pick is
+        """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside
+        its block: whether it may be).  Those shapes stay with the library, whose default pick is
         what the rules above were measured against: tuned it is up to a quarter faster."""
-        shape = (self.library_rows(M), N, K)
-        if self._tuning:
-            self._tuned.add(shape)
-        return shape in self._tuned
+        return self._tuning or (self.library_rows(M), N, K) in self._tuned
 
     def linear_gated_block(self, x, weight, bias, rows, act):
         """act(gate) * up of many rows over the row-major weight, tiles of ``rows`` x 256."""
@@ -615,6 +619,8 @@ class ProductOps:
             padded[:M].copy_(x)
             x = padded
         if out_dtype is None:
+            if self._tuning:
+                self._tuned.add((rows, w.shape[0], x.shape[1]))
             return torch.mm(x, w.t())[:M]
         return torch.mm(x, w.t(), out_dtype=out_dtype)[:M]
 
@@ -634,6 +640,8 @@ class ProductOps:
                 padded = self._new((rows, x.shape[1]))
                 padded[:M].copy_(x)
                 x = padded
+            if self._tuning:
+                self._tuned.add((rows, w.shape[0], x.shape[1]))
             return torch.addmm(b16, x, w.t())[:M]
         return self.library_sums(x, w, torch.float32).add_(bias).to(torch.bfloat16)
 
@@ -673,3 +681,4 @@ class ProductOps:
         finally:
             self._tuning = False
             tunable.tuning_enable(False)           # the choices made stay in use; nothing new is timed
+            self._tuned |= tuned_shapes(tunable.get_results())          # (those of the file among them)

@@ -57,7 +57,7 @@ class KernelTable:
         self.tile_few_rows = act_dtype == torch.bfloat16      # gated_mlp keeps few rows tiled by k-step
         self.weight_layout = "dual" if act_dtype == torch.bfloat16 else "rows"
         self.lower_tiles = act_dtype == torch.bfloat16        # see plan_weights
-        self._tuning, self._tuned = False, set()      # within library_tuning; the (rows, N, K) it was open for
+        self._tuning, self._tuned = False, set()      # within library_tuning; the (rows, N, K) the library was timed for
         self._untiled = None          # scratch for "tiled": the row-major form of one matrix
         self._rows_budget = 0         # bytes of row-major copies a "tiled" model may still keep (plan_weights)
         self._matrices = self._matrices_with_rows = 0

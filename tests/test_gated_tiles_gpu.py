@@ -66,16 +66,27 @@ def test_routes_of_prompts_products():
 
 
 def test_shapes_tuned_for_the_library_stay_with_it(tmp_path):
-    ops = HipOps(torch.bfloat16, DEV)
-    w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
-    weight, x = ops.prepare_weight(w), torch.randn(300, 1024, device=DEV).bfloat16()
+    """The ones whose library product was timed, here or by an earlier process; not those that went to a kernel of this table while
+    the tuning was open, nor other numbers of rows."""
+    ops, later = HipOps(torch.bfloat16, DEV), HipOps(torch.bfloat16, DEV)
+    weight = ops.prepare_weight((torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16())
+    x = torch.randn(1700, 1024, device=DEV).bfloat16()
     calls = []
-    gated = ops.linear_gated_block
-    ops.linear_gated_block = lambda *a: calls.append(a[0].shape[0]) or gated(*a)
-    ops._tuning = True                                        # (what the block of library_tuning sets)
-    ops.gated_linear(x, weight, 8)
-    ops._tuning = False
-    ops.gated_linear(x, weight, 8)
-    assert calls == []
-    ops.gated_linear(torch.cat([x, x]), weight, 8)            # another number of rows: not tuned
-    assert calls == [600]
+    for table in (ops, later):
+        table.linear_gated_block = lambda *a, own=table.linear_gated_block: calls.append(a[0].shape[0]) or own(*a)
+    try:
+        with ops.library_tuning(1, str(tmp_path / "tuned.csv")):
+            ops.gated_linear(x, weight, 8)
+            assert ops._block_plan(300, 8192, 1024, weight)
+            ops.gated_linear(x[:300], weight, 8)
+        with later.library_tuning(1, str(tmp_path / "tuned.csv")):
+            pass
+        assert calls == []
+        for table in (ops, later):
+            assert (1700, 8192, 1024) in table._tuned and (320, 8192, 1024) not in table._tuned
+            table.gated_linear(x, weight, 8)
+            assert calls == []
+            table.gated_linear(x[:1650], weight, 8)
+            assert calls.pop() == 1650
+    finally:
+        torch.cuda.tunable.enable(False)

@@ -36,3 +36,12 @@ def test_a_kernel_table_with_other_choices_gives_the_same_numbers():
     ref = x.float() @ w.float().T
     assert (ya - ref).abs().max() < 2 ** -6 * ref.abs().max()
     assert (yb - ref).abs().max() < 2 ** -6 * ref.abs().max()
+
+
+def test_shapes_among_the_library_tuner_s_results():
+    from servelab_amd.kernels.product_ops import tuned_shapes
+    results = (("GemmAndBiasTunableOp_BFloat16_TN", "tn_16384_700_2048_ld_2048_2048_16384", "Gemm_Hipblaslt_1", 0.04),
+               ("GemmTunableOp_BFloat16_TN", "tn_96_32_64_ld_64_64_96", "Default", 0.01),
+               ("GemmTunableOp_BFloat16_NN", "nn_64_64_64_ld_64_64_64", "Gemm_Hipblaslt_2", 0.01),
+               ("GemmTunableOp_float_TN", "tn_8_8_8_ld_8_8_8", "Gemm_Rocblas_3", 0.01))
+    assert tuned_shapes(results) == {(700, 16384, 2048), (32, 96, 64)} and tuned_shapes(()) == set()
