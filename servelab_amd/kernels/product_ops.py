@@ -203,7 +203,7 @@ class ProductOps:
         limit = self._few_rows_limit(weight)
         plan = self._block_plan(M, N, K, weight) or (
             defer and M > self.BLOCK_SQUARE_MAX_M and self.fuse_norms and not out_f32
-            and not self._tuned_for(M, N, K) and self._shares_plan(M, N, K, weight))
+            and not self._tuned_for(M, N, K) and self._block_reads(x, weight) and self._shares_plan(M, N, K, weight))
         if plan:
             # (deferred: the norm adds the partial sums)
             return self.linear_block(x, weight, bias, out_f32, plan[0],
@@ -331,31 +331,38 @@ class ProductOps:
         return (shares, True) if 2 <= shares <= 3 and 4 * tiles * shares >= 3 * self._num_cus else None
 
     def _gated_rows(self, M, N, K):
-        """Rows of x a workgroup of the block kernel takes (256 or 192) for the gated product of a
+        """Rows of x a workgroup of the block kernel takes (192 or 256) for the gated product of a
         prompt, or None where the library's product and a pass that gates it are the faster pair.
-        The kernel runs in rounds of one tile a CU, of which a half-filled one costs as much as a
-        full one; the library's own tiles leave less idle, but it writes gate and up (2 N bytes a
-        row) for the second kernel to read.  So: rows of K up to GATED_SHORT_K, where the
-        library's prologue weighs most (9728 x 896, 1,024 rows: 25.5 us, 36 in two kernels); one
-        round that fills GATED_FILL of the CUs' share (8192 x 2048, 1,400 rows: 47.1 against 51 us, at
-        900 rows and 0.55 of it 40.7 against 39); several rounds, filled to three quarters, of
-        GATED_ROUNDS_MIN_M rows and more (37888 x 3584: 1,700 rows 435 against 446 us, 2,048 rows 492
-        against 544; at 1,536 rows 395 against 348, where the library has tiles that fit)."""
+        The kernel saves that pass, which weighs most where rows of W are short, and loses where its whole
+        rounds of one tile a CU leave CUs idle: so rows of up to GATED_SHORT_K values, in one round whose
+        tiles are GATED_FILL of the CUs or more (GPU time, pair / kernel: 9728 x 896, 1,536 rows 37.8 / 33.1 us;
+        8192 x 1024, 2,048 rows 41.9 / 37.7; 16384 x 1024, 1,024 rows 45.7 / 39.0; 8192 x 512, 2,048 rows 31.1 / 23.2; of 94
+        such sizes of 11 shapes one is slower, by 3 %).  A round filled to a half loses (8192 x 1024, 527 rows
+        21.9 / 30.6); two rounds gain 8 % or lose 20 % as the library's tiles happen to fit.  With longer rows the matrix
+        units are the limit and the library's pick decides, which no size foretells: 2,048 rows of 37888 x 3584
+        547 / 496, of 23552 x 2048 249 / 182, but of 35840 x 3584 410 / 485, of 28672 x 4096 374 / 437, of 9216 x 3584 135 / 160,
+        of 59136 x 8192 1,550 / 1,688 (26 shapes, 1,601 to 2,304 rows: faster at 31 % of the sizes, slower at 64 %)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
-                or not 256 <= M <= self.GATED_MAX_M or N < self.GATED_MIN_N):
+                or K > self.GATED_SHORT_K or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
             return None
-        rounds = {rows: -(--(-N // 256) * -(-M // rows) // self._num_cus) for rows in (256, 192)}
-        rows = min(rounds, key=lambda r: rounds[r] * (r * K + 65536))
-        fill = M * N / (rounds[rows] * self._num_cus * rows * 256)
-        if K <= self.GATED_SHORT_K or (fill >= self.GATED_FILL and rounds[rows] == 1):
-            return rows
-        return rows if M >= self.GATED_ROUNDS_MIN_M and fill >= 0.75 else None
+        # (tiles of 192 rows from 1,024 rows of x on: with fewer they take as long as the pair, 16384 x 1024 at 700 rows 33 us
+        # either way)
+        for rows, fewest in ((192, 1024), (256, 768)):
+            tiles = -(-N // 256) * -(-M // rows)
+            if M >= fewest and self.GATED_FILL * self._num_cus <= tiles <= self._num_cus:
+                return rows
+        return None
 
     def _tuned_for(self, M, N, K) -> bool:
         """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside
         its block: whether it may be).  Those shapes stay with the library, whose default pick is
         what the rules above were measured against: tuned it is up to a quarter faster."""
         return self._tuning or (self.library_rows(M), N, K) in self._tuned
+
+    @staticmethod
+    def _block_reads(x, weight) -> bool:
+        """Whether the rows lie as the block kernel reads them, from multiples of 16 bytes on (the library takes any)."""
+        return x.data_ptr() % 16 == 0 and (weight.w is None or weight.w.data_ptr() % 16 == 0)
 
     def linear_gated_block(self, x, weight, bias, rows, act):
         """act(gate) * up of many rows over the row-major weight, tiles of ``rows`` x 256."""
@@ -484,8 +491,8 @@ class ProductOps:
             y = self._new((M, N // 2))
             self._skinny(x, weight, bias, y, M, N, K, gated=code)
             return y
-        rows = (M >= 256 and block == self.GATE_BLOCK and not self._tuned_for(M, N, K)
-                and self._gated_rows(M, N, K))
+        rows = block == self.GATE_BLOCK and self._gated_rows(M, N, K)
+        rows = rows and not self._tuned_for(M, N, K) and self._block_reads(x, weight) and rows
         if rows:
             return self.linear_gated_block(x, weight, bias, rows, code)
         return self.gate_mul(self.linear(x, weight, bias), block, activation)

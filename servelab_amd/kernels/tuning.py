@@ -93,13 +93,12 @@ class Tuning:
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
     # gated products of a prompt in the block kernel: the fewest rows of W and the most rows of x it was
-    # measured at, up to which K it always wins, how full a single round of tiles has to be, and from how many
-    # rows of x it takes several (measured sides: HipOps._gated_rows)
+    # measured at, up to which K it is taken, and how full its one round of tiles has to be (measured
+    # sides: HipOps._gated_rows)
     gated_min_n: int = 4096
     gated_max_m: int = 2560
     gated_short_k: int = 1024
-    gated_fill: float = 0.7
-    gated_rounds_min_m: int = 1601
+    gated_fill: float = 0.84
 
     # ---- few-rows consumer products on workgroups that stay
     # tiles per CU from which walking the tiles beats a workgroup per tile (gate/up: 9, head: 37;

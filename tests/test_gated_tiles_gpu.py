@@ -40,16 +40,22 @@ def test_gated_tiles(M, N, K, act, rows):
 
 def test_routes_of_prompts_products():
     ops = HipOps(torch.bfloat16, DEV)
-    assert ops._gated_rows(255, 8192, 1024) is None and ops._gated_rows(256, 8192, 1024) == 192
-    assert ops._gated_rows(256, 8192, 1088) is None                         # a round filled to a sixth
-    assert ops._gated_rows(1536, 8192, 2048) == 192                         # 256 tiles of 192 rows: one full round
-    assert ops._gated_rows(1537, 8192, 2048) == 256                         # 224 tiles of 256
-    assert ops._gated_rows(1600, 37888, 3584) is None and ops._gated_rows(2048, 37888, 3584) == 256
-    assert ops._gated_rows(2561, 37888, 3584) is None and ops._gated_rows(2048, 8192, 2080) is None
-    x = torch.randn(300, 1024, device=DEV).bfloat16()
+    gated = ops._gated_rows
+    assert ops._num_cus == 256
+    # one round of tiles, 0.84 of the CUs or more: of 192 rows from 1,024 rows of x on, else of 256
+    assert [gated(M, 8192, 1024) for M in (256, 1152, 1153, 1536, 1537, 2048, 2049)] == [None, None, 192, 192, 256, 256, None]
+    assert [gated(M, 16384, 1024) for M in (768, 769, 1024, 1025)] == [None, 256, 256, None]
+    assert [gated(M, 4096, 512) for M in (2496, 2497, 2560, 2561)] == [None, 192, 192, None]
+    assert gated(512, 32768, 512) is None and gated(1536, 8192, 1056) is None                  # few rows of x; K not in steps of 64
+    assert gated(1536, 8192, 1088) is None and gated(2048, 37888, 3584) is None                # long rows stay with the library
+    x = torch.randn(1200, 1024, device=DEV).bfloat16()
     w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
     weight = ops.prepare_weight(w)
-    assert torch.equal(ops.gated_linear(x, weight, 8), ops.linear_gated_block(x, weight, None, 192, 1))
+    fused = ops.linear_gated_block(x, weight, None, 192, 1)
+    assert torch.equal(ops.gated_linear(x, weight, 8), fused)
+    # rows that do not start at a multiple of 16 bytes stay with the library, which takes them
+    odd = torch.empty(x.numel() + 1, device=DEV, dtype=x.dtype)[1:].view(x.shape).copy_(x)
+    assert (ops.gated_linear(odd, weight, 8).float() - fused.float()).abs().max() <= 2.0 ** -7 * fused.abs().max()
     # a residual delta of 1,537 and more rows: two or three shares
     K, N, M = 8192, 1024, 1600
     w = (torch.randn(N, K, device=DEV) * 0.02).bfloat16()
