@@ -318,17 +318,19 @@ class ProductOps:
 
     def _shares_plan(self, M, N, K, weight):
         """Like ``_block_plan`` for a product of more rows that the norm adds to the stream: two or
-        three shares of K in square tiles where they fill three quarters of the CUs and the tiles
-        alone would not (7B shape, down projection at 1,800 / 2,048 rows: 218 / 245 us in 2
-        shares, 334 / 362 us in the library's product; 3B shape, whose 64 tiles need 4 shares: 85
-        against 93 us, which the norm's reading of four partial sums takes back)."""
+        three shares of K in square tiles where they fill the CUs well, two to seven eighths, three to four fifths (GPU
+        time with the norm, library's product / shares: 3584 x 18944, 1,800 / 2,048 rows 351 / 246 and 376 / 272 us in two;
+        2560 x 9728, 2,048 rows 116 / 111 in three, 2560 x 13824 160 / 146; 4096 x 14336, 1,600 / 1,984 rows 343 / 195 and
+        211 / 219).  Less well filled two shares lose: 3584 x 18944, 1,664 rows (0.77) 238 / 253, 3328 x 8192, 2,048 rows (0.81)
+        112 / 129, 3072 x 8192, 2,048 rows (0.75) 107 / 127.  Four shares gain nothing: the norm reads them all."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or weight.w is None
                 or K % 64 or N % 4 or N > self.BLOCK_MAX_N or K < self.BLOCK_SQUARE_MIN_K
                 or not self.BLOCK_SQUARE_MAX_M < M <= self.SHARES_MAX_M):
             return None
         tiles = -(-N // 256) * -(-M // 256)
         shares = self._num_cus // tiles
-        return (shares, True) if 2 <= shares <= 3 and 4 * tiles * shares >= 3 * self._num_cus else None
+        fill = tiles * shares / self._num_cus
+        return (shares, True) if (shares == 2 and fill >= 0.875) or (shares == 3 and fill >= 0.8) else None
 
     def _gated_rows(self, M, N, K):
         """Rows of x a workgroup of the block kernel takes (192 or 256) for the gated product of a

@@ -60,6 +60,12 @@ def test_routes_of_prompts_products():
     K, N, M = 8192, 1024, 1600
     w = (torch.randn(N, K, device=DEV) * 0.02).bfloat16()
     weight, x = ops.prepare_weight(w), torch.randn(M, K, device=DEV).bfloat16()
+    class Rows:
+        w = True
+    shares = lambda M, N, K: ops._shares_plan(M, N, K, Rows)
+    assert shares(1792, 3584, 18944) is None and shares(1793, 3584, 18944) == (2, True)       # 0.77 and 0.875 of the CUs
+    assert shares(1793, 3328, 8192) is None and shares(1537, 3072, 8192) == (3, True) and shares(1793, 3072, 8192) is None
+    assert shares(1537, 2560, 9728) == (3, True) and shares(2048, 2048, 11008) is None        # four shares
     ops._num_cus = 64
     assert ops._shares_plan(M, N, K, weight) == (2, True) and ops._shares_plan(1536, N, K, weight) is None
     assert ops._shares_plan(2049, N, K, weight) is None and ops._shares_plan(M, 2 * N, K, weight) is None
