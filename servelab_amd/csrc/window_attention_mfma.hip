@@ -81,21 +81,39 @@ constexpr int RCH = VK ? (DK - DV) / 8 : 0;            // chunks of a key row be
 constexpr int NT = VK ? cdiv((DV / 8) * 4, THREADS) : 1;   // 8 keys x 8 channels tiles a thread (turned on their way into LDS)
 constexpr int NR = VK ? (RCH ? cdiv(32 * RCH, THREADS) : 1) : 1;
 
+// Workgroups start in the order of their number, and numbers go to the eight dies in turn and there to the groups of CUs in
+// turn.  Without a window or chunks a tile takes as long as its keys are many, so the late tiles come first:
+// BY_LENGTH, for sequences of one length: of every sequence and head, so that the short ones fill what is left at the end;
+// BY_LENGTH_MOVED, for nearly equal ones: the same, and a sequence and head moves on by one place from tile to tile;
+// LATE_FIRST, for unequal ones: sequence by sequence.  (Among short sequences every 32nd workgroup, say, is one of the long
+// prompt's, and with BY_LENGTH all of these are one die's: a prompt of 500 tokens among 31 decoding, 16 heads on 1, 576 / 512:
+// 720 us, 127 in this order; prompts of 1,200, 300, 100 and 20 tokens 413 us, 467 moved, 195; of 1,200 and three of
+// 1,000 410 moved, 463 with early tiles first.)
+enum { IN_ORDER = 0, LATE_FIRST = 1, BY_LENGTH = 2, BY_LENGTH_MOVED = 3 };
+
 // (rows of up to 128 values: four workgroups a CU, which 128 registers allow)
-__global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_mfma_kernel(const WindowAttention a) {
+__global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_mfma_kernel(const WindowAttention a, int order) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
   __bf16* ks = lds16;                                  // [32][KROW]
   __bf16* vt = ks + 32 * KROW;                         // [DV][VROW]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, gq = lane >> 4;
   const int page = a.page, nkv = a.nkv;
-  // Workgroups start in the order of their number: without a window the tiles with the most keys to walk (the last
-  // ones) of every sequence and head first, so that the short ones fill what is left at the end.  (Read back from a
-  // lane: a division is done in vector registers, and so would be all that follows from it.)
-  const int number = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), pairs = gridDim.y * gridDim.z;
-  const bool longest = a.window == 0 && a.chunk == 0;
-  const int seq = longest ? __builtin_amdgcn_readfirstlane(number % pairs / gridDim.y) : blockIdx.z;
-  const int kvh = longest ? __builtin_amdgcn_readfirstlane(number % pairs % gridDim.y) : blockIdx.y;
-  const int item = longest ? __builtin_amdgcn_readfirstlane(gridDim.x - 1 - number / pairs) : blockIdx.x;
+  int seq = blockIdx.z, kvh = blockIdx.y, item = blockIdx.x;
+  if (order == LATE_FIRST) {
+    item = gridDim.x - 1 - blockIdx.x;
+  } else if (order == BY_LENGTH) {                     // (launched with the heads along x and the tiles along z)
+    seq = blockIdx.y;
+    kvh = blockIdx.x;
+    item = gridDim.z - 1 - blockIdx.z;
+  } else if (order == BY_LENGTH_MOVED) {
+    // (read back from a lane: a division is done in vector registers, and so would be all that follows from it)
+    const int number = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), pairs = gridDim.y * gridDim.z;
+    const int rank = __builtin_amdgcn_readfirstlane(number / pairs), moved = pairs < 8 ? rank * pairs / 8 : rank;
+    const int pair = __builtin_amdgcn_readfirstlane((number % pairs + moved) % pairs);
+    seq = __builtin_amdgcn_readfirstlane(pair / gridDim.y);
+    kvh = pair - seq * gridDim.y;
+    item = gridDim.x - 1 - rank;
+  }
   const int g = a.nh / nkv;
   const int q0 = a.cu_q[seq], qlen = a.cu_q[seq + 1] - q0;
   const int ncols = qlen * g;
@@ -150,9 +168,6 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
     const __bf16* qp = a.q + (size_t)(q0 + tok) * a.q_stride + (size_t)head * DK + 8 * gq;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) qf[kk] = *(const bf16x8*)(qp + 32 * kk);
-    // (waited for here: left to the loop, the wait for the first use of q would be one for the next block's keys as well)
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
   }
   f32x4 o[DD];
 #pragma unroll
@@ -264,6 +279,10 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
     fetch(block_base(i0), ask_pages(block_base(i0)));
     if (i0 + 1 < i1) asked = ask_pages(block_base(i0 + 1));
   }
+  // (q, asked for before the first keys, is waited for here: left to the loop, the wait for its first use would be one for the
+  // next block's keys as well)
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
   for (int i = i0; i < i1; ++i) {
     const int kbase = block_base(i);
     __syncthreads();                                   // the last block's readers are done
@@ -394,14 +413,14 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
   }
 }
 
-static const char* launch_mfma(const WindowAttention& a, dim3 grid, hipStream_t stream) {
+static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, hipStream_t stream) {
   const size_t bytes = sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW);
   if (bytes > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return hipGetErrorString(e);
   }
-  window_attention_mfma_kernel<<<grid, THREADS, bytes, stream>>>(a);
+  window_attention_mfma_kernel<<<grid, THREADS, bytes, stream>>>(a, order);
   return sl_launch_status();
 }
 
@@ -440,8 +459,13 @@ extern "C" const char* sl_window_attention_mfma(
   const long long cols = (long long)max_q_len * (nh / nkv);
   const long long tiles = (cols + COLS - 1) / COLS;
   SL_CHECK(tiles * nsplit <= 1 << 30, "window attention: too many column tiles");
-  const dim3 grid((unsigned)(tiles * nsplit), nkv, num_seqs);
-  const char* e = launch_mfma(a, grid, stream);
+  const long long full = (long long)num_seqs * max_q_len;         // tokens if every sequence had as many as the longest
+  const int order = window > 0 || chunk > 0 ? IN_ORDER :
+                    num_tokens == full && tiles * nsplit <= 65535 ? BY_LENGTH :
+                    4ll * num_tokens >= 3 * full ? BY_LENGTH_MOVED : LATE_FIRST;
+  const unsigned items = (unsigned)(tiles * nsplit);
+  const dim3 grid = order == BY_LENGTH ? dim3(nkv, num_seqs, items) : dim3(items, nkv, num_seqs);
+  const char* e = launch_mfma(a, grid, order, stream);
   if (e || nsplit == 1) return e;
   window_attention_combine_kernel<<<dim3(num_tokens, nh, (Dv + 63) / 64), 64, 0, stream>>>(
       part_o, part_ml, nsplit, nh, Dv, sinks, (const act_t*)gate, gate_stride, channel_gate, channel_stride,

@@ -48,3 +48,32 @@ def test_blocks_with_unseen_keys(H, G, Dk, Dv, in_keys, window, keep, page):
     want = torch.cat(want)
     # results of size up to a few units rounded to bfloat16 (2^-9 of the value); scores, weights and sums are float32
     assert (out.view(T, H, Dv).double().cpu() - want).abs().max() <= 2.0 ** -8 * want.abs().max() + 1e-4
+
+
+# the order in which a launch takes its tiles: sequences of one length, nearly equal ones over fewer and more than eight
+# (sequence, kv head) pairs, unequal ones; several tiles of 64 columns a sequence, the last one partly filled
+@pytest.mark.parametrize("lens", [(70, 70, 70), (75, 60, 71), (90, 3, 1), (1, 1, 1)])
+@pytest.mark.parametrize("H,G", [(4, 1), (4, 4)])
+def test_orders_of_the_tiles(H, G, lens):
+    ops = HipOps(torch.bfloat16, "cuda:0")
+    g = torch.Generator().manual_seed(H + G)
+    D, page = 64, 16
+    cached = [5, 0, 40]
+    whole = [a + b for a, b in zip(cached, lens)]
+    tables, kc, vc = paged(whole, page, G, D, D, torch.bfloat16, g)
+    keys, values = ([torch.randn(n, G, D, generator=g).bfloat16() for n in whole] for _ in range(2))
+    fill_pages(tables, kc, vc, keys, values, page)
+    q = torch.randn(sum(lens), H * D, generator=g).bfloat16()
+    cu, pos, want = [0], [], []
+    for s, (a, b) in enumerate(zip(cached, lens)):
+        rows = list(range(a, a + b))
+        want.append(plain_attention(q[cu[-1]:cu[-1] + b].view(b, H, D), keys[s], values[s], rows, D ** -0.5, None, 0, None, None, None))
+        pos += rows
+        cu.append(cu[-1] + b)
+    batch = SimpleNamespace(cu_q=dev(torch.tensor(cu, dtype=torch.int32)), positions=dev(torch.tensor(pos, dtype=torch.int32)),
+                            num_seqs=len(lens), num_tokens=cu[-1], max_q_len=max(lens), max_ctx_len=max(whole))
+    out = ops.window_attention(dev(q), 0, H, G, D, D, dev(kc), dev(vc), page, dev(tables), batch, D ** -0.5, None, 0, None,
+                               None, None, 0)
+    want = torch.cat(want)
+    # (as above)
+    assert (out.view(-1, H, D).double().cpu() - want).abs().max() <= 2.0 ** -8 * want.abs().max() + 1e-4
