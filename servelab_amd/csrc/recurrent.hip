@@ -24,6 +24,7 @@
 // State layout: S as [head][value channel][key channel] (a column of the matrix, which one
 // lane group owns, is contiguous), then what the mixer keeps besides.
 #include "common.h"
+#include <climits>
 
 __device__ __forceinline__ float softplusf_(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 __device__ __forceinline__ float logsigmoidf_(float x) { return -softplusf_(-x); }
@@ -460,6 +461,7 @@ struct MatrixScan {
   int write;
   float* out;                // [T][H][Dv]
   float* normaliser;         // matrix LSTM: [S][H][D + 1], the new n and m until every block has read the old ones
+  int line;                  // sequences of so many tokens and more are walked in chunks, the others token by token
 };
 
 enum { SCAN_DECAY = 0, SCAN_DELTA = 1, SCAN_LSTM = 2, SCAN_SSD = 3, SCAN_FORGET = 4, SCAN_DELTA_HEAD = 5 };
@@ -516,6 +518,8 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
   const int oo = og + CH * 4;                                 // [CH][cols] the walkers' read-outs
   const int g = h / (a.H / a.G);
   const int first = a.cu_q[s], last = a.cu_q[s + 1];
+  // (the whole block; as one condition of the wavefront, which costs no scratch memory)
+  if (__builtin_amdgcn_readfirstlane((last <= first) | (last - first >= a.line))) return;
   const bool fresh = a.positions[first] == 0;
   float* slot = a.state + (size_t)a.slots[s] * a.state_stride;
   const size_t nS = (size_t)a.H * a.Dv * a.D;
@@ -796,14 +800,15 @@ extern "C" long long sl_matrix_scan_workspace(int mode, int T, int S, int H, int
   return scan_chunks_layout(mode, T, S, H, G, D, Dv, nullptr, nullptr);
 }
 
-// workspace: walked in chunks (max_len: tokens of the longest sequence); nullptr: token by token.
+// workspace: sequences of `line` tokens and more are walked in chunks, which are among the first `lead` (of lead_tokens tokens,
+// the longest of max_len); `rest`: there are others, walked token by token as all of them are without a workspace.
 extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride, int q_col, int k_col, int v_col,
                                       int H, int G, int D, int Dv, const float* log_decay, float q_scale,
                                       const float* gates, int gate_stride, int i_col, int f_col, float cap,
                                       const float* rates, const float* step_bias, const float* skip, const float* lower, float* state, long long state_stride,
                                       const int* cu_q, const int* positions,
                                       const int* slots, int S, int T, int write, float* normaliser, float* workspace,
-                                      int max_len, float* out, hipStream_t stream) {
+                                      int lead, int lead_tokens, int max_len, int line, int rest, float* out, hipStream_t stream) {
   SL_CHECK(mode != SCAN_LSTM || !write || normaliser != nullptr, "matrix_scan: room for the new normalisers is missing");
   SL_CHECK(mode >= 0 && mode <= 5, "matrix_scan: unknown mode");
   SL_CHECK(S >= 0 && T >= 0 && H > 0 && G > 0 && H % G == 0 && Dv > 0, "matrix_scan: sizes must be positive");
@@ -823,22 +828,27 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   const long long need = (long long)H * Dv * D + (mode == SCAN_LSTM ? (long long)H * D + H : 0);
   SL_CHECK(need <= state_stride, "matrix_scan: the state does not fit its slot");
   if (S == 0 || T == 0) return nullptr;
+  if (workspace == nullptr) line = INT_MAX;
+  const MatrixScan a{src, src_stride, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, gates, gate_stride,
+                     i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out,
+                     normaliser, line};
   if (workspace != nullptr) {
     SL_CHECK((uintptr_t)workspace % 16 == 0, "matrix_scan: the workspace must be aligned");
-    SL_CHECK(max_len >= 1 && max_len <= T, "matrix_scan: the longest sequence does not fit the step");
-    const MatrixScan a{src, src_stride, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, gates, gate_stride,
-                       i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out, normaliser};
+    SL_CHECK(lead >= 1 && lead <= S && lead_tokens <= T && max_len >= 1 && max_len <= lead_tokens && line >= 1,
+             "matrix_scan: the sequences walked in chunks do not fit the step");
     ScanChunks c;
-    SL_CHECK(scan_chunks_layout(mode, T, S, H, G, D, Dv, workspace, &c) > 0, "matrix_scan: at most 256 key channels a head in chunks");
-    const char* err = mode == SCAN_DECAY ? scan_in_chunks<SCAN_DECAY>(a, c, S, max_len, stream) :
-                      mode == SCAN_DELTA ? scan_in_chunks<SCAN_DELTA>(a, c, S, max_len, stream) :
-                      mode == SCAN_SSD ? scan_in_chunks<SCAN_SSD>(a, c, S, max_len, stream) :
-                      mode == SCAN_DELTA_HEAD ? scan_in_chunks<SCAN_DELTA_HEAD>(a, c, S, max_len, stream) :
-                      mode == SCAN_FORGET ? scan_in_chunks<SCAN_FORGET>(a, c, S, max_len, stream) :
-                                            scan_in_chunks<SCAN_LSTM>(a, c, S, max_len, stream);
+    SL_CHECK(scan_chunks_layout(mode, lead_tokens, lead, H, G, D, Dv, workspace, &c) > 0, "matrix_scan: at most 256 key channels a head in chunks");
+    const char* err = mode == SCAN_DECAY ? scan_in_chunks<SCAN_DECAY>(a, c, lead, max_len, stream) :
+                      mode == SCAN_DELTA ? scan_in_chunks<SCAN_DELTA>(a, c, lead, max_len, stream) :
+                      mode == SCAN_SSD ? scan_in_chunks<SCAN_SSD>(a, c, lead, max_len, stream) :
+                      mode == SCAN_DELTA_HEAD ? scan_in_chunks<SCAN_DELTA_HEAD>(a, c, lead, max_len, stream) :
+                      mode == SCAN_FORGET ? scan_in_chunks<SCAN_FORGET>(a, c, lead, max_len, stream) :
+                                            scan_in_chunks<SCAN_LSTM>(a, c, lead, max_len, stream);
     if (err != nullptr) return err;
-    if (mode == SCAN_LSTM && write) normaliser_kernel<<<dim3(S, H), 64, 0, stream>>>(a);
-    return sl_launch_status();
+    if (!rest) {
+      if (mode == SCAN_LSTM && write) normaliser_kernel<<<dim3(S, H), 64, 0, stream>>>(a);
+      return sl_launch_status();
+    }
   }
   // (A lane owning 4 key channels instead of 8 doubles the blocks of a lone prompt and halves a lane's
   // products; measured, a token takes as long: its cost is the sums across lanes, the hand-over and
@@ -849,8 +859,6 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   const int CH = min(min(16, 2048 / Dp), 8 * P);       // 8 values a thread of each kind a chunk
   const bool scalar = mode == SCAN_LSTM || mode == SCAN_SSD || mode == SCAN_DELTA_HEAD;
   const size_t lds = 2 * (size_t)CH * ((scalar ? 2 : 3) * Dp + 2 * cols + 4) * sizeof(float);   // two halves
-  const MatrixScan a{src, src_stride, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, gates, gate_stride,
-                     i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out, normaliser};
   const int vcols = mode == SCAN_LSTM ? cols - 1 : cols;       // (the matrix LSTM's last column group carries n)
   const dim3 grid(S, H, (Dv + vcols - 1) / vcols);
   if (mode == SCAN_DECAY) matrix_scan_kernel<SCAN_DECAY, SCAN_ROWS><<<grid, 512, lds, stream>>>(a, P, CH);

@@ -51,7 +51,7 @@ __device__ __forceinline__ int scan_chunk_id(int first, int s, int ci) { return 
 // The matrix LSTM's gates after cap and squashing, and what a chunk does to the running maximum: m -> max(m + F, M).
 __global__ __launch_bounds__(256) void scan_gates_kernel(const MatrixScan a, const ScanChunks w) {
   const int s = blockIdx.y, first = a.cu_q[s], len = a.cu_q[s + 1] - first, t0 = blockIdx.x * SCAN_CHUNK;
-  if (t0 >= len) return;
+  if (t0 >= len || len < a.line) return;
   const int nt = min(SCAN_CHUNK, len - t0);
   for (int h = threadIdx.x / SCAN_CHUNK; h < a.H; h += 256 / SCAN_CHUNK) {
     const int tt = threadIdx.x % SCAN_CHUNK;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void scan_prepare_scalar_kernel(const MatrixSc
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int s = blockIdx.z, g = blockIdx.y, ci = blockIdx.x;
   const int first = a.cu_q[s], len = a.cu_q[s + 1] - first, t0 = ci * C;
-  if (t0 >= len) return;                                // (the whole workgroup)
+  if (t0 >= len || len < a.line) return;                // (the whole workgroup)
   const int nt = min(C, len - t0), rep = a.H / a.G;
   const int chunk = scan_chunk_id(first, s, ci);
   const int Dp = c.Dp, row = Dp + 4, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, gq = lane >> 4;
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256) void scan_prepare_channel_kernel(const MatrixS
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int s = blockIdx.z, h = blockIdx.y, ci = blockIdx.x;
   const int first = a.cu_q[s], len = a.cu_q[s + 1] - first, t0 = ci * C;
-  if (t0 >= len) return;                                // (the whole workgroup)
+  if (t0 >= len || len < a.line) return;                // (the whole workgroup)
   const int nt = min(C, len - t0), g = h / (a.H / a.G);
   const int chunk = scan_chunk_id(first, s, ci);
   const int Dp = c.Dp, row = Dp + 4, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, gq = lane >> 4;
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(256, ScanForm<MODE>::DELTA && TW > 1 ? 1 : 2) void 
   if (hs >= S * a.H) return;
   const int s = hs / a.H, h = hs - s * a.H, g = h / (a.H / a.G);
   const int first = a.cu_q[s], len = a.cu_q[s + 1] - first;
-  if (len <= 0) return;
+  if (len <= 0 || len < a.line) return;
   const int nchunks = (len + C - 1) / C, chunk0 = scan_chunk_id(first, s, 0);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 15, gq = lane >> 4;
   const int vcols = MODE == SCAN_LSTM ? 15 : 16;

@@ -47,13 +47,20 @@ class ExpertMatrices:
 
 class RecurrentOps:
     SELECTIVE_SEGMENT = 64        # tokens of a segment of the selective scan
-    # The matrix recurrences are walked in chunks of 32 tokens (scan_chunks.h), not token by token, from this many
-    # tokens of a step's longest sequence on: the chunks' own kernels cost 20 to 30 us however short a sequence is, a
-    # token 0.2 to 0.35 us (heads of 128 x 256: 64 tokens 21 us either way, 96: 27 against 23, 256: 58 against 29).  The
-    # state-space form, whose groups of heads are prepared one head after the other, from twice as many (128
-    # tokens 35 against 40 us, 192: 50 against 45).  Several sequences keep the chip busier: eight of 64 tokens
-    # 51 against 41 us, eight of 32: 34 against 35.
-    SCAN_CHUNKS_FROM, SCAN_CHUNKS_FROM_GROUPED, SCAN_CHUNKS_FROM_MANY, SCAN_MANY_TOKENS = 80, 160, 48, 400
+    # A sequence's matrix recurrence is walked in chunks of 32 tokens (scan_chunks.h), not token by token, from this many
+    # tokens of it in a step on: the chunks' own kernels cost 15 to 30 us however short it is, a token 0.2 to 0.35 us (us,
+    # token by token / in chunks: decay, 8 heads of 128 x 256, 80 tokens 25 / 25, 128 35 / 27; delta, 16 of 128 x 128, 80 35 / 35;
+    # matrix LSTM, 8 of 128 x 256, 80 33 / 27).  By SCAN_LATER more tokens where the chunks cost more or a token less (delta
+    # with a decay a head, 16 of 128 x 128, 80 31 / 34, 100 37 / 35; forget, 16 of 128 x 128, 80 25 / 27, 100 29 / 29).  The
+    # state-space form prepares a group's heads one after the other, some 15 tokens' time each: from SCAN_CHUNKS_FROM_GROUPED in
+    # groups of seven or eight, earlier and later by their number (heads of 128 x 64, 64 in 8 groups, 160 tokens 44 / 44; 112 in
+    # 8, 200 62 / 75, 300 89 / 82; 8 heads of 64 x 64 in 8, 80 24 / 15).  Several sequences that fill the
+    # CUs with more than SCAN_MANY tokens of a block's walk each go in chunks from SCAN_CHUNKS_FROM_MANY tokens on (decay as
+    # above, 7 of 60 45 / 39, 16 of 48 75 / 58, 8 of 50, just below, 41 / 40; 8 heads of 16 x 16, 16 of 48 18 / 36: far below).
+    # The other sequences of the step, its decoding ones above all, are walked token by token in a launch of their own (a
+    # prompt of 512 tokens among 64 decoding, delta, 28 heads: 330 us all token by token, 1,634 all in chunks, 167).
+    SCAN_CHUNKS_FROM, SCAN_CHUNKS_FROM_GROUPED, SCAN_CHUNKS_FROM_MANY, SCAN_MANY = 80, 160, 48, 208
+    SCAN_LATER = {_SCAN_FORGET: 1.25, _SCAN_DELTA_HEAD: 1.2}
 
     # rows an expert has on average from which row tiles hold 128 rows (64 experts, 8 and 12 rows each: gate/up, down and
     # the sum of 2,048 x 1,024 experts 143 and 154 us in tiles of 16, 147 and 150 in tiles of 128; of 3,584 x 1,792 405
@@ -197,19 +204,46 @@ class RecurrentOps:
         out = self._new((T, H * Dv), torch.float32)
         normaliser = self._new((batch.num_seqs, H, D + 1), torch.float32) if mode == _SCAN_LSTM and write else None
         lib = self._lazy("recurrent")
-        workspace, longest = None, int(getattr(batch, "max_q_len", T))
-        alone = self.SCAN_CHUNKS_FROM_GROUPED if mode == _SCAN_SSD else self.SCAN_CHUNKS_FROM
-        if longest >= (alone if T < self.SCAN_MANY_TOKENS else min(alone, self.SCAN_CHUNKS_FROM_MANY)):
+        workspace, (lead, lead_tokens, longest, line, rest) = None, self._scan_chunks(mode, batch, T, H, G, D, Dv)
+        if lead:
             size = self._lib[lib].sl_matrix_scan_workspace
             size.restype = ctypes.c_longlong
-            floats = size(mode, T, batch.num_seqs, H, G, D, Dv)
+            floats = size(mode, lead_tokens, lead, H, G, D, Dv)
             workspace = self._new((floats,), torch.float32) if floats else None
         self._call(lib, "sl_matrix_scan", mode, _p(src), stride, q_col, k_col, v_col, H, G,
                    D, Dv, _p(log_decay), _c_float(q_scale), _p(gates), gate_stride, i_col, f_col, _c_float(cap),
                    _p(rates), _p(step_bias), _p(skip), _p(lower), _p(state), _ll(slot_size), _p(batch.cu_q),
                    _p(batch.positions), _p(batch.state_slots),
-                   batch.num_seqs, T, int(bool(write)), _p(normaliser), _p(workspace), longest, _p(out))
+                   batch.num_seqs, T, int(bool(write)), _p(normaliser), _p(workspace), lead, lead_tokens, longest, line,
+                   int(rest), _p(out))
         return out
+
+    def _scan_chunks(self, mode, batch, T, H, G, D, Dv):
+        """Which sequences of a step are walked in chunks: (the first so many hold all of them; their tokens, the longest's;
+        those of at least so many tokens; whether the step has others), zeros where none is."""
+        longest = int(getattr(batch, "max_q_len", T))
+        line = self.SCAN_CHUNKS_FROM * self.SCAN_LATER.get(mode, 1)
+        if mode == _SCAN_SSD:
+            line = self.SCAN_CHUNKS_FROM_GROUPED * (H // G + 3.5) / 10.7
+        if longest < min(line, self.SCAN_CHUNKS_FROM_MANY):
+            return 0, 0, 0, 0, True
+        lens = getattr(batch, "q_lens", None)
+        if not lens or len(lens) != batch.num_seqs or sum(lens) != T:
+            lens = None                       # (a batch that does not say: its sequences are taken for long ones)
+        columns = 256 // (1 << max(0, (D + 7) // 8 - 1).bit_length()) - (mode == _SCAN_LSTM)
+        blocks = H * -(-Dv // max(1, columns))
+        several = self.SCAN_CHUNKS_FROM_MANY
+        tokens = T if lens is None else sum(n for n in lens if n >= several)
+        later = max(1.0, H / G / 4.5) if mode == _SCAN_SSD else self.SCAN_LATER.get(mode, 1)
+        if tokens * blocks >= self.SCAN_MANY * self._num_cus * later:
+            line = min(line, several)
+        line = max(1, int(line))
+        if longest < line:
+            return 0, 0, 0, 0, True
+        if lens is None:
+            return batch.num_seqs, T, longest, 1, False
+        lead = max(i for i, n in enumerate(lens) if n >= line) + 1
+        return lead, sum(lens[:lead]), longest, line, any(n < line for n in lens)
 
     def decay_scan(self, src, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, beta_src, beta_col,
                    state, batch, write):

@@ -198,3 +198,50 @@ def test_a_sequence_without_tokens_keeps_its_normaliser():
                    sequences(q_lens, starts, [2, 0, 1], DEV), True)
     assert torch.equal(state[0], before[0])
     assert (state[1:] != before[1:]).all(1).all()
+
+
+@pytest.mark.parametrize("mode", ["decay", "delta", "delta, decay a head", "state space", "forget", "lstm"])
+@pytest.mark.parametrize("order", [range(7), (5, 6, 3, 1, 2, 0, 4)])
+def test_long_sequences_in_chunks_beside_short_ones(mode, order):
+    """The two launches of such a step against all of it token by token; the long ones last and first."""
+    H, G, D, Dv = (2, 2, 72, 33) if mode in ("forget", "lstm") else (4, 2, 64, 40)
+    hip = HipOps(torch.float32, DEV)
+    call, size, _ = scan_case(mode, H, G, D, Dv, False)
+    lens, starts, slots = ([v[i] for i in order] for v in (Q_LENS, STARTS, SLOTS))
+    batch = sequences(lens, starts, slots, DEV)
+    state = torch.randn(len(slots), size, generator=torch.Generator().manual_seed(8)).to(DEV) * 0.3
+    walked, both = state.clone(), state.clone()
+    batch.q_lens = lens
+    hip.SCAN_CHUNKS_FROM = hip.SCAN_CHUNKS_FROM_GROUPED = hip.SCAN_CHUNKS_FROM_MANY = 1 << 30
+    want = call(hip, walked, batch, DEV)
+    hip.SCAN_CHUNKS_FROM = hip.SCAN_CHUNKS_FROM_GROUPED = 40
+    got = call(hip, both, batch, DEV)
+    # (float32 in another order of sums, as against the plain functions above; the matrix LSTM's read-outs are quotients)
+    close(got, want, 2e-5 if mode != "lstm" else 1e-3)
+    close(both, walked, 2e-5)
+
+
+def test_normalisers_of_a_long_portion():
+    """More than 64 chunks, whose running maxima are put together 64 at a time, behind a context; against float64."""
+    H, D, Dv, T = 2, 20, 24, 2100
+    hip = HipOps(torch.float32, DEV)
+    g = torch.Generator().manual_seed(11)
+    width = 2 * H * D + H * Dv
+    buf = torch.randn(T, width + 2 * H, generator=g) * 0.5
+    buf[:, width + H:] += 4.0                              # (weak decays: a maximum is carried over many chunks)
+    buf[3, width:width + H] = 14.0
+    state = torch.randn(1, H * D * Dv + H * D + H, generator=g) * 0.3
+    state[0, -H:] = 5.0
+    s1 = state.clone().to(DEV)
+    hip.mlstm_scan(buf.to(DEV), 0, H * D, 2 * H * D, width, width + H, H, D, Dv, 15.0, D ** -0.5, s1, sequences([T], [9], [0], DEV), True)
+    row = state[0].double()
+    S, n, m = row[:H * D * Dv].view(H, Dv, D), row[H * D * Dv:-H].view(H, D), row[-H:]
+    for t in buf.double():
+        k, v = t[H * D:2 * H * D].view(H, D), t[2 * H * D:width].view(H, Dv)
+        i = 15 * torch.tanh(t[width:width + H] / 15)
+        f = torch.nn.functional.logsigmoid(15 * torch.tanh(t[width + H:] / 15))
+        new = torch.maximum(f + m, i)
+        keep, add, m = torch.exp(f + m - new), torch.exp(i - new), new
+        S, n = keep[:, None, None] * S + add[:, None, None] * v[:, :, None] * k[:, None], keep[:, None] * n + add[:, None] * k
+    want = torch.cat([S.flatten(), n.flatten(), m])
+    assert float((s1[0].double().cpu() - want).norm() / want.norm()) < 1e-5          # (chains of some hundred tokens)
