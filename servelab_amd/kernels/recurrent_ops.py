@@ -65,9 +65,13 @@ class RecurrentOps:
     # rows an expert has on average from which row tiles hold 128 rows (64 experts, 8 and 12 rows each: gate/up, down and
     # the sum of 2,048 x 1,024 experts 143 and 154 us in tiles of 16, 147 and 150 in tiles of 128; of 3,584 x 1,792 405
     # and 500, 431 and 436; 8 experts of 2,048 x 5,632, 8 and 12 rows 101 and 171, 144 and 144); with fewer than
-    # ROUTED_WIDE_EXPERTS experts, whose tiles of 128 rows leave most CUs idle, only from the second number on (4
-    # experts of 1,024 x 512, 47 and 120 rows 29.7 and 31, 32 and 40)
+    # ROUTED_WIDE_EXPERTS experts, or ones so small that a tile an expert makes fewer than ROUTED_WIDE_WORKGROUPS workgroups,
+    # only from the second number on (4 experts of 1,024 x 512, 47 and 120 rows 29.7 and 31, 32 and 40; 8 of them, 32
+    # rows 30.6 and 32.4).  The staged kernel that wins there takes rows in steps of 64 values; rows of an odd number of 32 values
+    # go to the one before it, from ROUTED_WIDE_TILE_ROWS_ODD rows on (64 experts of 2,080 x 1,024, 12 / 24 / 48 rows 160 / 189 /
+    # 262 in tiles of 16, 214 / 223 / 255 in tiles of 128; 8 of 4,128 x 1,056, 12 rows 122 and 169)
     ROUTED_WIDE_TILE_ROWS, ROUTED_WIDE_TILE_ROWS_OF_FEW, ROUTED_WIDE_EXPERTS = 12, 96, 8
+    ROUTED_WIDE_TILE_ROWS_ODD, ROUTED_WIDE_WORKGROUPS = 48, 64
 
     # ------------------------------------------------- norm on an output
     def add_postnorm(self, resid, y, weight, eps, mult, want_rows=True):
@@ -423,22 +427,33 @@ class RecurrentOps:
                 _p(batch.tok_seq), _p(batch.state_slots), batch.num_seqs, int(bool(write)))
 
     # ------------------------------------------------------- routed experts
+    def expert_tile_rows(self, pairs, w_gate_up, gated=True):
+        """Rows of a row tile (16 or 128) for a step of ``pairs`` (token, choice) pairs over the experts of ``w_gate_up``:
+        what ``route_tokens`` takes as ``tile_rows``."""
+        experts, N, K = w_gate_up.shape
+        blocks = -(-(N // 2 if gated else N) // 128)
+        few = experts < self.ROUTED_WIDE_EXPERTS or experts * blocks < self.ROUTED_WIDE_WORKGROUPS
+        line = self.ROUTED_WIDE_TILE_ROWS_OF_FEW if few else \
+            (self.ROUTED_WIDE_TILE_ROWS if K % 64 == 0 else self.ROUTED_WIDE_TILE_ROWS_ODD)
+        return _TILE_ROWS[int(pairs >= line * experts and self.act_dtype == torch.bfloat16)]
+
     def route_tokens(self, logits, experts, top, over_all=False, correction=None, scale=1.0, with_matrices=None,
-                     sigmoid=False):
+                     sigmoid=False, tile_rows=None):
         """The ``top`` largest of each row's first ``experts`` logits (float32; among equals the
         lower index) with the softmax over them, and the step's (token, choice) pairs sorted by
         expert for the grouped products.  ``over_all``: what is compared is the softmax over all
         ``experts`` logits plus ``correction`` [experts] (None: nothing), and a chosen expert's
         share is its softmax value over the sum of the chosen ones' (+ 1e-20), times ``scale``.
         ``sigmoid``: a chosen expert's share is the sigmoid of its logit.  ``with_matrices``: only the first so many experts have matrices (the others get no row
-        tiles; ``routed_experts`` hands their input through)."""
+        tiles; ``routed_experts`` hands their input through).  ``tile_rows``: what ``expert_tile_rows`` says of the
+        experts' matrices (None: by their number alone)."""
         T, stride = self._f32_rows(logits, "router logits")
         n = T * top
         # larger row tiles once an expert has that many rows on average (float32 has no kernel that would use them)
-        per_expert = n / (experts if with_matrices is None else max(1, int(with_matrices)))
-        line = self.ROUTED_WIDE_TILE_ROWS if experts >= self.ROUTED_WIDE_EXPERTS else self.ROUTED_WIDE_TILE_ROWS_OF_FEW
-        wide = per_expert >= line and self.act_dtype == torch.bfloat16
-        tile_rows = _TILE_ROWS[int(wide)]
+        if tile_rows is None:
+            per_expert = n / (experts if with_matrices is None else max(1, int(with_matrices)))
+            line = self.ROUTED_WIDE_TILE_ROWS if experts >= self.ROUTED_WIDE_EXPERTS else self.ROUTED_WIDE_TILE_ROWS_OF_FEW
+            tile_rows = _TILE_ROWS[int(per_expert >= line and self.act_dtype == torch.bfloat16)]
         max_tiles = -(-n // tile_rows) + experts
         chosen = self._new((T, top), torch.int32)
         shares = self._new((T, top), torch.float32)

@@ -118,19 +118,22 @@ class RoutedExperts(FeedForward):
     def forward(self, x):
         ops = self.rt.ops
         logits = ops.linear(x, self.w_router, self.b_router, out_f32=True)
+        tiles = {}                                     # (how the kernel table cuts the experts' rows)
+        if hasattr(ops, "expert_tile_rows"):
+            tiles["tile_rows"] = ops.expert_tile_rows(x.shape[0] * self.top, self.w_gate_up, self.gated)
         if self.routing == "shares":
             routing = ops.route_tokens(logits, self.outputs, self.top, over_all=True,
                                        correction=self.route_correction, scale=self.route_scale,
-                                       with_matrices=self.experts)
+                                       with_matrices=self.experts, **tiles)
             base = ops.materialize(self.shared.forward(x)) if self.shared is not None else None
             return ops.routed_experts(x, routing, self.w_gate_up, self.w_down, base, activation=self.activation,
                                       gated=self.gated, base_gate=logits if self.shared_gate else None,
                                       base_gate_col=self.outputs, limit=self.limit,
                                       pass_through=self.pass_through > 0)
         if self.routing == "sigmoid":
-            routing = ops.route_tokens(logits, self.experts, self.top, sigmoid=True)
+            routing = ops.route_tokens(logits, self.experts, self.top, sigmoid=True, **tiles)
         else:
-            routing = ops.route_tokens(logits, self.experts, self.top)
+            routing = ops.route_tokens(logits, self.experts, self.top, **tiles)
         base = ops.materialize(self.shared.forward(x)) if self.shared is not None else None
         if self.weigh == "input":
             return ops.routed_experts(x, routing, self.w_gate_up, self.w_down, base, activation=self.activation,

@@ -122,3 +122,20 @@ def test_a_routing_put_together_by_a_caller(T, tile_rows):
     assert r.tile_rows == tile_rows and r.tiles_in_use.item() == (r.tiles[:, 2] > 0).sum().item()
     own = Routing(r.chosen, r.shares, r.order, r.place_of, r.tiles.flip(0).contiguous(), tile_rows)
     assert torch.equal(hip.routed_experts(x, own, first, down), hip.routed_experts(x, r, first, down))
+
+
+def test_tiles_asked_for_by_the_matrices():
+    """Rows of an odd number of 32 values stay in tiles of 16 where the staged kernel cannot take them; either gives the same."""
+    T, E, top, ff, K = 70, 8, 2, 1024, 96
+    hip = HipOps(torch.bfloat16, DEV)
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(T, K, generator=g).bfloat16().to(DEV)
+    first = hip.prepare_expert_matrices((torch.randn(E, 2 * ff, K, generator=g) * K ** -0.5).bfloat16().to(DEV), gated=True)
+    down = hip.prepare_expert_matrices((torch.randn(E, K, ff, generator=g) * ff ** -0.5).bfloat16().to(DEV))
+    logits = torch.randn(T, E, generator=g).to(DEV)
+    rows = hip.expert_tile_rows(T * top, first)
+    r, wide = (hip.route_tokens(logits, E, top, tile_rows=n) for n in (rows, None))
+    assert (r.tile_rows, wide.tile_rows) == (16, 128)
+    got, want = (hip.routed_experts(x, v, first, down).float() for v in (r, wide))
+    # (as above)
+    assert (got - want).abs().max() <= 3 * 2.0 ** -8 * want.abs().max()
