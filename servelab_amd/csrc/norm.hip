@@ -520,10 +520,10 @@ extern "C" const char* sl_add_into(float* resid, const void* delta, long long n,
 // RMS norm on a sublayer's output: resid (float, in place) += mult * y * rsqrt(mean(y^2) + eps) * w,
 // and the stream's new rows in the activation type for the sublayer that reads them next (out == nullptr:
 // they are not wanted).  y == nullptr: only those rows.  One block per row; sums and the stream in float.
-// A row is a few trips to memory in turn, so up to NORMED_KEEP values a thread of all that is read are asked for at
-// once, before the sum, and no load stands behind a condition, which would be waited for where the ways meet (8 rows of
-// 3,584 values: 6.4 us with a loop after the sum, 4.7 here).
-constexpr int NORMED_KEEP = 8;
+// A row is a few trips to memory in turn, so up to KEEP (1, 2, 4 or 8: what a row needs) values a thread of all that is read are
+// asked for at once, before the sum, and no load stands behind a condition, which would be waited for where the ways meet (8
+// rows of 3,584 values: 6.4 us with a loop after the sum, 4.7 here; 2,048 rows of 64: 3.4 us, 4.6 with eight loads, 3.3 here).
+template <int KEEP>
 __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
                                     const float* __restrict__ w, act_t* __restrict__ out, int H, float eps,
                                     float mult) {
@@ -536,10 +536,10 @@ __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __re
     return;
   }
   const act_t* yr = y + r * H;
-  act_t yk[NORMED_KEEP];
-  float xk[NORMED_KEEP], wk[NORMED_KEEP];
+  act_t yk[KEEP];
+  float xk[KEEP], wk[KEEP];
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const int i = min((int)(threadIdx.x + u * blockDim.x), H - 1);
     yk[u] = yr[i];
     xk[u] = x[i];
@@ -547,25 +547,25 @@ __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __re
   }
   float ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const float v = threadIdx.x + u * blockDim.x < H ? to_f(yk[u]) : 0.f;
     ss += v * v;
   }
-  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
+  for (int i = threadIdx.x + KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = to_f(yr[i]);
     ss += v * v;
   }
   ss = block_sum(ss, scratch);
   const float inv = 1.f / sqrtf(ss / (float)H + eps);
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const int i = threadIdx.x + u * blockDim.x;
     if (i >= H) break;
     const float v = xk[u] + mult * (to_f(yk[u]) * inv * wk[u]);
     x[i] = v;
     if (o != nullptr) o[i] = from_f<act_t>(v);
   }
-  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
+  for (int i = threadIdx.x + KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = x[i] + mult * (to_f(yr[i]) * inv * w[i]);
     x[i] = v;
     if (o != nullptr) o[i] = from_f<act_t>(v);
@@ -577,7 +577,12 @@ extern "C" const char* sl_add_postnorm(float* resid, const void* y, const float*
   SL_CHECK(T >= 0 && H > 0, "add_postnorm: sizes must be positive");
   SL_CHECK(y != nullptr || out != nullptr, "add_postnorm: nothing to do");
   if (T == 0) return nullptr;
-  add_postnorm_kernel<<<T, H >= 2048 ? 512 : 256, 0, stream>>>(resid, (const act_t*)y, w, (act_t*)out, H, eps, mult);
+  const int threads = H >= 2048 ? 512 : 256, need = (H + threads - 1) / threads;
+  auto run = [&](auto kernel) { kernel<<<T, threads, 0, stream>>>(resid, (const act_t*)y, w, (act_t*)out, H, eps, mult); };
+  if (need <= 1) run(add_postnorm_kernel<1>);
+  else if (need <= 2) run(add_postnorm_kernel<2>);
+  else if (need <= 4) run(add_postnorm_kernel<4>);
+  else run(add_postnorm_kernel<8>);
   return sl_launch_status();
 }
 
@@ -585,8 +590,9 @@ extern "C" const char* sl_add_postnorm(float* resid, const void* y, const float*
 // follows at once: v = resid + y * rsqrt(mean(y^2) + eps_y) * wy, out = v * rsqrt(mean(v^2) + eps) * w.
 // rows == nullptr: every row, and v goes back to the stream; else only the listed rows are computed
 // and the stream stays as it is (the head reads few rows of the last layer's result).  One block per
-// row, up to NORMED_KEEP values a thread asked for at once, as above, and kept in registers between the passes; all
+// row, up to KEEP values a thread asked for at once, as above, and kept in registers between the passes; all
 // sums in float (2 rows of 2,048 values: 6.0 us with loads after each sum, 4.4 here).
+template <int KEEP>
 __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
                                           const float* __restrict__ wy, float eps_y,
                                           const int* __restrict__ rows, const float* __restrict__ w, float eps,
@@ -596,10 +602,10 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   float* x = resid + r * H;
   const act_t* yr = y + r * H;
   act_t* o = out + (size_t)blockIdx.x * H;
-  act_t yk[NORMED_KEEP];
-  float keep[NORMED_KEEP], xk[NORMED_KEEP], wyk[NORMED_KEEP], wk[NORMED_KEEP];
+  act_t yk[KEEP];
+  float keep[KEEP], xk[KEEP], wyk[KEEP], wk[KEEP];
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const int i = min((int)(threadIdx.x + u * blockDim.x), H - 1);
     yk[u] = yr[i];
     xk[u] = x[i];
@@ -608,11 +614,11 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   }
   float ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     keep[u] = threadIdx.x + u * blockDim.x < H ? to_f(yk[u]) : 0.f;
     ss += keep[u] * keep[u];
   }
-  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
+  for (int i = threadIdx.x + KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = to_f(yr[i]);
     ss += v * v;
   }
@@ -620,7 +626,7 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   const float inv_y = 1.f / sqrtf(ss / (float)H + eps_y);
   float s2 = 0.f;
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const int i = threadIdx.x + u * blockDim.x;
     if (i < H) {
       keep[u] = xk[u] + keep[u] * inv_y * wyk[u];
@@ -628,7 +634,7 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
       s2 += keep[u] * keep[u];
     }
   }
-  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
+  for (int i = threadIdx.x + KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = x[i] + to_f(yr[i]) * inv_y * wy[i];
     if (rows == nullptr) x[i] = v;
     s2 += v * v;
@@ -636,11 +642,11 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   s2 = block_sum(s2, scratch);
   const float inv = 1.f / sqrtf(s2 / (float)H + eps);
 #pragma unroll
-  for (int u = 0; u < NORMED_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const int i = threadIdx.x + u * blockDim.x;
     if (i < H) o[i] = from_f<act_t>(keep[u] * inv * wk[u]);
   }
-  for (int i = threadIdx.x + NORMED_KEEP * blockDim.x; i < H; i += blockDim.x) {
+  for (int i = threadIdx.x + KEEP * blockDim.x; i < H; i += blockDim.x) {
     const float v = rows == nullptr ? x[i] : x[i] + to_f(yr[i]) * inv_y * wy[i];
     o[i] = from_f<act_t>(v * inv * w[i]);
   }
@@ -652,8 +658,14 @@ extern "C" const char* sl_add_normed_rmsnorm(float* resid, const void* y, const 
   SL_CHECK(R >= 0 && H > 0, "add_normed_rmsnorm: sizes must be positive");
   SL_CHECK(y != nullptr && wy != nullptr && w != nullptr, "add_normed_rmsnorm: the output and both gains are required");
   if (R == 0) return nullptr;
-  add_normed_rmsnorm_kernel<<<R, H >= 2048 ? 512 : 256, 0, stream>>>(resid, (const act_t*)y, wy, eps_y, rows, w,
-                                                                    eps, (act_t*)out, H);
+  const int threads = H >= 2048 ? 512 : 256, need = (H + threads - 1) / threads;
+  auto run = [&](auto kernel) {
+    kernel<<<R, threads, 0, stream>>>(resid, (const act_t*)y, wy, eps_y, rows, w, eps, (act_t*)out, H);
+  };
+  if (need <= 1) run(add_normed_rmsnorm_kernel<1>);
+  else if (need <= 2) run(add_normed_rmsnorm_kernel<2>);
+  else if (need <= 4) run(add_normed_rmsnorm_kernel<4>);
+  else run(add_normed_rmsnorm_kernel<8>);
   return sl_launch_status();
 }
 

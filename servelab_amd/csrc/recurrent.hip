@@ -348,35 +348,45 @@ __global__ __launch_bounds__(256) void stream_conv_kernel(const ShortConv a, act
 
 // One token a sequence: everything between a sublayer's output and the next mixer's rows in one launch.
 // x += y / sqrt(mean(y^2) + eps) * wy (y == nullptr: x as it is), the convolution over x and the slot's
-// last inputs, and the slot moved on by one.  A block takes a channel a thread of a token, so that the slot is read and
-// rewritten without a barrier; every block of a token adds up all of its y (7 KB) for the norm.  What bounds it is the
-// trips to memory in a row: all that a channel needs is asked for before that sum (8 tokens of 3,584
-// channels, four taps: 10.6 us with a block a token, whose threads took their channels one after the other, 4.8 here).
-// The sums run in the order of the kernels for longer steps.
+// last inputs, and the slot moved on by one.  A block takes slices of a token's channels, a channel a thread, so that the slot is
+// read and rewritten without a barrier; every block of a token adds up all of its y (7 KB) for the norm.  What bounds it is the
+// trips to memory in a row: all that a channel of the first slice needs is asked for before that sum (8 tokens of 3,584
+// channels, four taps: 10.6 us with a block a token, whose threads took their channels one after the other, 4.8 here).  Tokens that
+// fill the chip with fewer blocks get fewer (300 of 3,584, two / four taps: 10.8 / 11.8 us with a slice a block, 7.6 / 10.6
+// with a block a token, 8.2 / 9.9 here).  The sums run in the order of the kernels for longer steps.
+// (LOOP apart from the one slice: a loop about the loads costs that 0.5 us.)
 constexpr int STREAM_KEEP = 8, STREAM_TAPS = 3;
+template <bool LOOP>
 __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid, const act_t* __restrict__ y,
                                    const float* __restrict__ wy, float eps, int write, act_t* __restrict__ out) {
   __shared__ float scratch[16];
   const int t = blockIdx.x, H = a.C, back = a.taps - 1;
-  const int own = blockIdx.y * blockDim.x + threadIdx.x, c = min(own, H - 1);
   float* x = resid + (size_t)t * H;
   const act_t* yr = y != nullptr ? y + (size_t)t * H : nullptr;
   const int s = a.tok_seq[t];
   const bool fresh = a.positions[t] == 0;
   float* keep_in = a.state + (size_t)a.slots[s] * a.state_stride + a.state_off;
-  float v = x[c], yv = 0.f, gain = 0.f;
+  float v, yv = 0.f, gain = 0.f, w_own;
   float past[STREAM_TAPS], w[STREAM_TAPS];
-  if (back > 0) {
+  auto ask = [&](int c) {
+    v = x[c];
+    if (back > 0) {
 #pragma unroll
-    for (int j = 0; j < STREAM_TAPS; ++j) {            // (past the taps: the last again, not used)
-      past[j] = keep_in[(size_t)min(j, back - 1) * H + c];
-      w[j] = a.w[(size_t)min(j, back) * H + c];
+      for (int j = 0; j < STREAM_TAPS; ++j) {          // (past the taps: the last again, not used)
+        past[j] = keep_in[(size_t)min(j, back - 1) * H + c];
+        w[j] = a.w[(size_t)min(j, back) * H + c];
+      }
     }
-  }
-  const float w_own = a.w[(size_t)back * H + c];
+    w_own = a.w[(size_t)back * H + c];
+    if (yr != nullptr) {
+      yv = to_f(yr[c]);
+      gain = wy[c];
+    }
+  };
+  const int first = blockIdx.y * blockDim.x + threadIdx.x;
+  ask(min(first, H - 1));
+  float inv = 0.f;
   if (yr != nullptr) {
-    yv = to_f(yr[c]);
-    gain = wy[c];
     float ss = 0.f;
 #pragma unroll
     for (int u = 0; u < STREAM_KEEP; ++u) {
@@ -389,26 +399,36 @@ __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid,
       ss += z * z;
     }
     ss = block_sum(ss, scratch);
-    v += yv * (1.f / sqrtf(ss / (float)H + eps)) * gain;
-    if (own < H) x[c] = v;
+    inv = 1.f / sqrtf(ss / (float)H + eps);
   }
-  if (own >= H) return;
-  float acc = 0.f;
+  auto channel = [&](int c) {
+    if (yr != nullptr) {
+      v += yv * inv * gain;
+      x[c] = v;
+    }
+    float acc = 0.f;
 #pragma unroll
-  for (int j = 0; j < STREAM_TAPS; ++j) {
-    if (j >= back) break;
-    const float p = fresh ? 0.f : past[j];
-    if (!fresh) acc += w[j] * p;
-    if (write && j > 0) keep_in[(size_t)(j - 1) * H + c] = p;
-  }
-  for (int j = STREAM_TAPS; j < back; ++j) {
-    const float p = fresh ? 0.f : keep_in[(size_t)j * H + c];
-    if (!fresh) acc += a.w[(size_t)j * H + c] * p;
-    if (write) keep_in[(size_t)(j - 1) * H + c] = p;
-  }
-  acc += w_own * v;
-  if (write && back > 0) keep_in[(size_t)(back - 1) * H + c] = v;
-  out[(size_t)t * H + c] = from_f<act_t>(v + acc);
+    for (int j = 0; j < STREAM_TAPS; ++j) {
+      if (j >= back) break;
+      const float p = fresh ? 0.f : past[j];
+      if (!fresh) acc += w[j] * p;
+      if (write && j > 0) keep_in[(size_t)(j - 1) * H + c] = p;
+    }
+    for (int j = STREAM_TAPS; j < back; ++j) {
+      const float p = fresh ? 0.f : keep_in[(size_t)j * H + c];
+      if (!fresh) acc += a.w[(size_t)j * H + c] * p;
+      if (write) keep_in[(size_t)(j - 1) * H + c] = p;
+    }
+    acc += w_own * v;
+    if (write && back > 0) keep_in[(size_t)(back - 1) * H + c] = v;
+    out[(size_t)t * H + c] = from_f<act_t>(v + acc);
+  };
+  if (first < H) channel(first);
+  if (LOOP)
+    for (int c = first + gridDim.y * blockDim.x; c < H; c += gridDim.y * blockDim.x) {
+      ask(c);
+      channel(c);
+    }
 }
 
 // single: every sequence of the step has one token; y (with wy, eps) is taken in that form only.
@@ -426,8 +446,13 @@ extern "C" const char* sl_stream_conv(float* resid, int C, int taps, const float
                     slots, 0, 0, 0, 0.f, 1.f, 0, nullptr, nullptr, 0};
   if (single) {
     const int threads = C >= 2048 ? 1024 : (C >= 512 ? 512 : 256);
-    stream_step_kernel<<<dim3(T, (C + threads - 1) / threads), threads, 0, stream>>>(a, resid, (const act_t*)y, wy, eps,
-                                                                                     write, (act_t*)out);
+    // a block a slice while the blocks fit the chip together: 32 wavefronts on each of 256 CUs
+    const int all = (C + threads - 1) / threads, slices = max(1, min(all, 2048 * 256 / threads / T));
+    auto run = [&](auto kernel) {
+      kernel<<<dim3(T, slices), threads, 0, stream>>>(a, resid, (const act_t*)y, wy, eps, write, (act_t*)out);
+    };
+    if (slices == all) run(stream_step_kernel<false>);
+    else run(stream_step_kernel<true>);
     return sl_launch_status();
   }
   const bool whole = C % 4 == 0 && (uintptr_t)resid % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0;
