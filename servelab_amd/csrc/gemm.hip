@@ -77,7 +77,9 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(
 // The same with K cut among the four wavefronts of a workgroup, which then own NC columns together: a matrix of few rows
 // still has a workgroup for every CU, and a lane's running sums are a quarter as long (1,536 columns of 8,960 at 1 / 3 / 8
 // rows: 22 / 39 / 60 -> 11 / 15 / 23 us, 5.0 TB/s at one row; errors halve).  STREAM: W is read past the caches, which
-// pays where it is far larger than they are (151,936 columns of 1,536 at one row 152 -> 129 us).
+// pays where it is larger than the 32 MB of the dies' L2 (us, through them / past them: 37,888 columns of 3,584 at 1 / 3 rows
+// 84.5 / 94.3 and 74.8 / 86.8, 3,584 of 18,944 51 / 57 and 46 / 54, 2,048 of 11,008 18.2 / 22.6 and 16.4 / 21.3) and costs
+// where it is smaller (896 of 4,864 at 3 rows 7.2 and 8.3, 1,536 of 1,536 5.4 and 6.0, 3,072 of 1,024 at 4 rows 7.5 and 8.0).
 template <int MB, int NC, bool STREAM>
 __global__ __launch_bounds__(256) void gemm_rows_split_kernel(
     const act_t* __restrict__ x, const act_t* __restrict__ w, const float* __restrict__ bias,
@@ -140,6 +142,11 @@ static const char* rows_split(const act_t* x, const act_t* w, const float* bias,
   else if (M <= 4) gemm_rows_split_kernel<4, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
   else gemm_rows_split_kernel<8, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
   return sl_launch_status();
+}
+template <int NC>
+static const char* rows_split(const act_t* x, const act_t* w, const float* bias, void* y, int M, int N, int K, hipStream_t stream) {
+  return (long long)N * K >= 8 << 20 ? rows_split<NC, true>(x, w, bias, y, M, N, K, stream)
+                                     : rows_split<NC, false>(x, w, bias, y, M, N, K, stream);
 }
 #endif
 
@@ -216,17 +223,19 @@ extern "C" const char* sl_gemm_rows(const void* x, const void* w, const float* b
   const int waves = 4;
   const act_t* xx = (const act_t*)x;
   const act_t* ww = (const act_t*)w;
-  // (measured, float32, 7B shape: from 4 rows on the staged form wins, 8 rows 139 -> 113 us for gate/up and
-  // 176 -> 114 us for down, 16 rows 281 -> 172 and 494 -> 174 us; with 1 to 3 rows it loses up to 18 us of 44)
+  // (the staged form against a wavefront's columns, float32, 7B shape: from 4 rows on it wins, 8 rows 139 -> 113 us for
+  // gate/up and 176 -> 114 us for down, 16 rows 281 -> 172 and 494 -> 174 us; with 1 to 3 rows it loses up to 18 us of 44)
 #if defined(SL_F32)
-  // (measured, us, one form against the next: 1,536 columns of 1,536 / 8,960 at 3 rows 9.9 / 39 -> 5.8 / 15 with two
-  // columns a workgroup; 3,584 of 18,944 at 1 / 3 / 8 rows 44 / 74 / 111 -> 42 / 47 / 62 with four.  Of many columns a
+  // (measured, us, a wavefront's columns against a workgroup's: 1,536 columns of 1,536 / 8,960 at 3 rows 9.9 / 39 -> 5.8 / 15
+  // with two columns a workgroup; 3,584 of 18,944 at 1 / 3 / 8 rows 44 / 74 / 111 -> 42 / 47 / 62 with four.  Of many columns a
   // wavefront each has enough to do from three rows on unless its rows are long: 151,936 of 1,536 at 3 rows 163
-  // against 177, 37,888 of 3,584 102 against 88; at 1 / 2 rows 93 / 99 -> 75 / 78.)
-  if (M <= 8 && N <= 2048) return rows_split<2, true>(xx, ww, bias, y, M, N, K, stream);
-  if (M <= 8 && N <= 4096) return rows_split<4, false>(xx, ww, bias, y, M, N, K, stream);
-  if (M == 1) return rows_split<2, true>(xx, ww, bias, y, M, N, K, stream);
-  if (M == 2 || (M <= 4 && K >= 2048)) return rows_split<4, true>(xx, ww, bias, y, M, N, K, stream);
+  // against 177, 37,888 of 3,584 102 against 88; at 1 / 2 rows 93 / 99 -> 75 / 78.  Short rows leave the workgroup's 1,024
+  // values a step empty: 8,192 columns of 64 at 1 / 2 rows 3.1 / 4.3 and 4.7 / 6.8, 4,096 of 512 at 1 / 8 rows 3.6 / 11.2 and 4.2 /
+  // 12.4, 3,072 of 1,024 at one 4.1 and 4.7, 6,000 of 640 4.7 and 5.3.)
+  if (M <= 8 && N <= 2048 && K >= 512) return rows_split<2>(xx, ww, bias, y, M, N, K, stream);
+  if (M <= 8 && N <= 4096 && K >= (M == 1 ? 1536 : 1024)) return rows_split<4>(xx, ww, bias, y, M, N, K, stream);
+  if (M == 1 && N > 4096 && K >= 768) return rows_split<2>(xx, ww, bias, y, M, N, K, stream);
+  if (N > 4096 && ((M == 2 && K >= 512) || (M <= 4 && K >= 2048))) return rows_split<4>(xx, ww, bias, y, M, N, K, stream);
 #endif
   constexpr int SHARED_MAX_M = sizeof(act_t) == 4 ? 16 : 8;   // (16 rows of bfloat16 spill registers)
   if (shared && M >= 4 && M <= SHARED_MAX_M) {
@@ -352,7 +361,7 @@ constexpr int FK = 16, FS = FK + 1;
 // step of 95 ms against 129 ms with the large tiles and 175 ms with the FMA
 // tiles; at 8 rows the wavefront-per-column kernel is twice as fast as either:
 // 8 KB of W per barrier is too little in flight to stream it).
-template <int TI, int TJ, int WM, int WN>
+template <int TI, int TJ, int WM, int WN, bool SHARES>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
     float* __restrict__ y, int M, int N, int K, int nsplit) {
@@ -418,10 +427,10 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   constexpr int SEG = SEGMENT_K / FK;                 // chunks a running sum takes
   // this share of K: whole segments (the last share also what is left over), results to its own [M, N]
   const int segs = (K / FK + SEG - 1) / SEG;
-  const int first = (int)((long long)segs * blockIdx.z / nsplit) * SEG;
-  const int behind = (int)((long long)segs * (blockIdx.z + 1) / nsplit) * SEG;
+  const int first = SHARES ? (int)((unsigned)segs * blockIdx.z / (unsigned)nsplit) * SEG : 0;
+  const int behind = SHARES ? (int)((unsigned)segs * (blockIdx.z + 1) / (unsigned)nsplit) * SEG : segs * SEG;
   const int nchunks = behind < K / FK ? behind : K / FK;
-  if (nsplit > 1) {
+  if (SHARES) {
     y += (size_t)blockIdx.z * M * N;
     bias = nullptr;
   }
@@ -513,10 +522,15 @@ extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const floa
   const dim3 grid((N + 127) / 128, (M + rows - 1) / rows, nsplit);
   SL_CHECK(grid.y <= 65535, "gemm_f32_mfma: more than 65535 row tiles");
   float* to = nsplit > 1 ? part : (float*)y;
-  if (M <= 64)
-    gemm_f32_mfma_kernel<1, 1, 1, 4><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
-  else
-    gemm_f32_mfma_kernel<2, 2, 2, 2><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
+  auto run = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit); };
+  // (one share apart: products of short rows take 6 to 8 % longer in a kernel that could take several)
+  if (M <= 64) {
+    if (nsplit > 1) run(gemm_f32_mfma_kernel<1, 1, 1, 4, true>);
+    else run(gemm_f32_mfma_kernel<1, 1, 1, 4, false>);
+  } else {
+    if (nsplit > 1) run(gemm_f32_mfma_kernel<2, 2, 2, 2, true>);
+    else run(gemm_f32_mfma_kernel<2, 2, 2, 2, false>);
+  }
   if (nsplit > 1) {
     const long long total = (long long)M * N;
     if (N % 4 == 0) f32_shares_kernel<4><<<(unsigned)((total + 1023) / 1024), 256, 0, stream>>>(part, bias, (float*)y, total, N, nsplit);

@@ -604,9 +604,10 @@ class ProductOps:
         their addition."""
         rows = 32 if M <= 64 else 128
         tiles = -(-M // rows) * -(-N // 128)
-        best, least = 1, float("inf")
-        for s in range(1, min(16, -(-K // self.F32_SEGMENT)) + 1):
-            us = -(-tiles * s // self._num_cus) * (K / s) * self.F32_TILE_US_PER_TERM * (rows / 128)
+        best, least, segments = 1, float("inf"), -(-K // self.F32_SEGMENT)
+        for s in range(1, min(16, segments) + 1):
+            terms = min(K, -(-segments // s) * self.F32_SEGMENT)          # of the longest share
+            us = -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM * (rows / 128)
             if s > 1:
                 us += 5.0 + (s + 1) * M * N * 4 / 3e6
             if us < 0.97 * least:

@@ -63,3 +63,9 @@ def emu_batch(batch):
         if torch.is_tensor(value):
             setattr(host, name, value.cpu())
     return host
+
+
+def test_shares_cost_what_the_longest_one_takes():
+    ops = HipOps(torch.float32, DEV)
+    assert ops._f32_shares(512, 9728, 896) == 1                # two segments of 512 and 384 terms: as long as three rounds of 512
+    assert ops._f32_shares(849, 1536, 8960) > 1 and ops._f32_shares(64, 256, 512) == 1
