@@ -1,12 +1,14 @@
 // Loads that go from global memory straight into LDS (global_load_lds_dwordx4): a wavefront's 64 loads of 16
 // bytes land side by side in 1 KB at `lds_at`.  They pass the registers by, so the compiler neither counts
-// nor waits for them: wait_loads<N> returns once at most the N youngest loads of the wavefront are under way.
+// nor waits for them: wait_loads<N> returns once at most the N youngest loads of the wavefront are under way, and
+// its reads of LDS are done: behind the barrier that follows, another wavefront's loads may land where they read (the
+// compiler moves products of the last reads, and the wait for these with them, behind a barrier).
 #pragma once
 __device__ __forceinline__ void load_to_lds(const void* from, unsigned lds_at) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
 }
 template <int N_> __device__ __forceinline__ void wait_loads() {
-  __builtin_amdgcn_s_waitcnt((N_ & 15) | (7 << 4) | (15 << 8) | ((N_ >> 4) << 14));
+  __builtin_amdgcn_s_waitcnt((N_ & 15) | (7 << 4) | ((N_ >> 4) << 14));
 }
 // Rows of 128 bytes in LDS, eight units of 16 bytes each: unit c of row r lies at place c ^ lds_place(r), so that the 16
 // lanes that read unit c of rows r .. r + 15 touch 16 different 16-byte slots of a 256-byte line of banks, and each half of
