@@ -340,17 +340,31 @@ class ProductOps:
         tiles are GATED_FILL of the CUs or more (GPU time, pair / kernel: 9728 x 896, 1,536 rows 37.8 / 33.1 us;
         8192 x 1024, 2,048 rows 41.9 / 37.7; 16384 x 1024, 1,024 rows 45.7 / 39.0; 8192 x 512, 2,048 rows 31.1 / 23.2; of 94
         such sizes of 11 shapes one is slower, by 3 %).  A round filled to a half loses (8192 x 1024, 527 rows
-        21.9 / 30.6); two rounds gain 8 % or lose 20 % as the library's tiles happen to fit.  With longer rows the matrix
-        units are the limit and the library's pick decides, which no size foretells: 2,048 rows of 37888 x 3584
-        547 / 496, of 23552 x 2048 249 / 182, but of 35840 x 3584 410 / 485, of 28672 x 4096 374 / 437, of 9216 x 3584 135 / 160,
-        of 59136 x 8192 1,550 / 1,688 (26 shapes, 1,601 to 2,304 rows: faster at 31 % of the sizes, slower at 64 %)."""
+        21.9 / 30.6); two rounds gain 8 % or lose 20 % as the library's tiles happen to fit.
+
+        With longer rows the matrix units are the limit, and the library is the faster one where its pick fills its
+        rounds, which it was seen to do where 192 or 224 divides N (2,048 rows of 35840 x 3584 410 / 485, of 28672 x 4096
+        374 / 437); where it does not, it idles as the kernel does and pays for the pass on top (of 37888 x 3584 547 / 496, of
+        22016 x 2048 196 / 181, of 23552 x 2048 249 / 182).  So: N that neither divides, and several rounds of tiles
+        of 256 x 256 whose last one is filled by GATED_LAST_ROUND; rows of up to GATED_LONG_K
+        values and GATED_LONG_ROWS rows of x, where this was measured (124 sizes of 28 shapes: 12 % faster on average, but slower
+        at a fifth of them, by up to 15 %, since the pick is not known: 15104 x 2048, 2,048 rows 109 / 121; of 284 sizes
+        outside the rule 30 % are faster, and the average is 3 % slower).  The sums meet the activation unrounded, so that it
+        is the more exact form as well.  Shapes that were tuned stay with the library (``_tuned_for``)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
-                or K > self.GATED_SHORT_K or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
+                or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
             return None
+        columns = -(-N // 256)
+        if K > self.GATED_SHORT_K:
+            rounds, last = divmod(columns * -(-M // 256), self._num_cus)
+            least, most = self.GATED_LAST_ROUND
+            fits = (K <= self.GATED_LONG_K and self.GATED_LONG_ROWS[0] <= M <= self.GATED_LONG_ROWS[1] and N % 192 and N % 224
+                    and rounds and least * self._num_cus <= last <= most * self._num_cus)
+            return 256 if fits else None
         # (tiles of 192 rows from 1,024 rows of x on: with fewer they take as long as the pair, 16384 x 1024 at 700 rows 33 us
         # either way)
         for rows, fewest in ((192, 1024), (256, 768)):
-            tiles = -(-N // 256) * -(-M // rows)
+            tiles = columns * -(-M // rows)
             if M >= fewest and self.GATED_FILL * self._num_cus <= tiles <= self._num_cus:
                 return rows
         return None
@@ -494,8 +508,7 @@ class ProductOps:
             self._skinny(x, weight, bias, y, M, N, K, gated=code)
             return y
         rows = block == self.GATE_BLOCK and self._gated_rows(M, N, K)
-        rows = rows and not self._tuned_for(M, N, K) and self._block_reads(x, weight) and rows
-        if rows:
+        if rows and not self._tuned_for(M, N, K) and self._block_reads(x, weight):
             return self.linear_gated_block(x, weight, bias, rows, code)
         return self.gate_mul(self.linear(x, weight, bias), block, activation)
 

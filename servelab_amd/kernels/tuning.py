@@ -92,13 +92,16 @@ class Tuning:
     block_square_max_m: int = 1536
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
-    # gated products of a prompt in the block kernel: the fewest rows of W and the most rows of x it was
-    # measured at, up to which K it is taken, and how full its one round of tiles has to be (measured
-    # sides: HipOps._gated_rows)
+    # gated products of a prompt in the block kernel (measured sides: HipOps._gated_rows): the fewest rows of W and the
+    # most rows of x it was measured at; rows of up to gated_short_k values, in one round of tiles filled by gated_fill; ...
     gated_min_n: int = 4096
     gated_max_m: int = 2560
     gated_short_k: int = 1024
     gated_fill: float = 0.84
+    # ... longer ones, up to gated_long_k values and for so many rows of x, in several rounds, the last filled so far
+    gated_long_k: int = 5120
+    gated_long_rows: tuple = (1537, 2048)
+    gated_last_round: tuple = (0.55, 0.95)
 
     # ---- few-rows consumer products on workgroups that stay
     # tiles per CU from which walking the tiles beats a workgroup per tile (gate/up: 9, head: 37;

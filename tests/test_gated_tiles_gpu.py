@@ -47,7 +47,11 @@ def test_routes_of_prompts_products():
     assert [gated(M, 16384, 1024) for M in (768, 769, 1024, 1025)] == [None, 256, 256, None]
     assert [gated(M, 4096, 512) for M in (2496, 2497, 2560, 2561)] == [None, 192, 192, None]
     assert gated(512, 32768, 512) is None and gated(1536, 8192, 1056) is None                  # few rows of x; K not in steps of 64
-    assert gated(1536, 8192, 1088) is None and gated(2048, 37888, 3584) is None                # long rows stay with the library
+    # longer rows: several rounds, the last one more than half filled, and no tile of the library's that divides N
+    assert [gated(M, 37888, 3584) for M in (1536, 1792, 1793, 2048, 2049)] == [None, None, 256, 256, None]
+    assert [gated(M, 27392, 2560) for M in (1536, 1537, 1792, 1793)] == [None, 256, 256, None]
+    assert gated(2048, 35840, 3584) is None and gated(2048, 24576, 3072) is None               # 160 times 224, 128 times 192
+    assert gated(2048, 9216, 3584) is None and gated(1536, 8192, 1088) is None and gated(2048, 37888, 5184) is None
     x = torch.randn(1200, 1024, device=DEV).bfloat16()
     w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
     weight = ops.prepare_weight(w)
