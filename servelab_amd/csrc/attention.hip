@@ -436,7 +436,9 @@ __global__ __launch_bounds__(TILE_THREADS) void attention_general_tile_kernel(
 // V^T [D][36]; the next block travels from the pages to registers meanwhile.  S^T = K Q^T, softmax with a running
 // maximum per column, O^T += V^T P^T: a lane's scores of a 16 x 16 block (keys 4 (lane / 16) .. + 3 of column lane % 16) are the
 // second product's operand as they are.  What bounds it is the matrix instructions: 1.05 MFLOP a block and workgroup at
-// D 128, 0.6 TFLOP/s a CU.  One prompt of 333 tokens and two shorter ones, 12 heads on 2, D 128: 287 us with the FMA tiles.
+// D 128, 0.6 TFLOP/s a CU.  One prompt of 333 tokens and two shorter ones, 12 heads on 2, D 128: 287 us with the FMA tiles,
+// 71 here.  The second product multiplies the zero weights of keys that a column does not see too, which an infinite or NaN
+// value turns into NaN: a wavefront with a result that is not finite takes its columns again key by key, over seen keys alone.
 // ---------------------------------------------------------------------------
 typedef float att_v4 __attribute__((ext_vector_type(4)));
 
@@ -561,6 +563,39 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  float odd = 0.f;                                     // (0, or NaN where a result is not finite)
+#pragma unroll
+  for (int dd = 0; dd < D / 16; ++dd) odd = fmaf((o[dd][0] + o[dd][1]) + (o[dd][2] + o[dd][3]), 0.f, odd);
+  if (__ballot(odd != 0.f)) {
+#pragma unroll
+    for (int dd = 0; dd < D / 16; ++dd) o[dd] = att_v4{0.f, 0.f, 0.f, 0.f};
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll 1
+    for (int key = kmin; key <= kmax; ++key) {
+      const size_t at = (size_t)table[key / page] * nkv + kvh;
+      const float* kp = kc + (at * page + key % page) * D + 4 * gq;
+      const float* vp = vc + (at * D + 4 * gq) * page + key % page;
+      float sc = 0.f;                                  // this lane's quarter of the channels: those that it holds of q and o
+#pragma unroll
+      for (int j = 0; j < D / 16; ++j) {
+        const att_v4 kv = *(const att_v4*)(kp + 16 * j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc = fmaf(qf[j][i], kv[i], sc);
+      }
+      sc += __shfl_xor(sc, 16, 64);
+      sc += __shfl_xor(sc, 32, 64);
+      if (key < lo_c || key > pos_c) continue;
+      sc *= scale;
+      const float mn = fmaxf(m, sc), alpha = mn == -INFINITY ? 1.f : expf(m - mn), p = sc == -INFINITY ? 0.f : expf(sc - mn);
+      l = fmaf(l, alpha, p);
+      m = mn;
+#pragma unroll
+      for (int dd = 0; dd < D / 16; ++dd)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[dd][i] = fmaf(p, vp[(16 * dd + i) * page], o[dd][i] * alpha);
+    }
+  }
   if (cw + n >= ncols) return;
   const float inv = 1.f / l;
   float* to = out + ((size_t)(q0 + tok) * nh + head) * D + 4 * gq;

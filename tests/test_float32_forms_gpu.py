@@ -56,6 +56,25 @@ def test_prompt_attention_on_the_matrix_cores(nh, nkv, D, page, window):
     assert float((got.cpu() - want).abs().max()) <= 2e-6 * max(1.0, float(want.abs().max()))
 
 
+@pytest.mark.parametrize("nh,nkv,D", [(12, 2, 128), (4, 4, 64)])
+@pytest.mark.parametrize("window", [None, 9])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_prompt_attention_beside_values_that_are_not_finite(nh, nkv, D, window, value):
+    """One key's value at position 50 reaches the tokens that see it, in its kv head and channel, and no other result."""
+    ops, page = HipOps(torch.float32, DEV), 16
+    lens = [(72, 72), (40, 40)]
+    qkv, kc, vc, tables, batch = make_attention_case(torch.float32, nh, nkv, D, page, lens)[:5]
+    run = lambda: ops.paged_attention(qkv, nh, nkv, D, kc, vc, page, tables, batch, D ** -0.5, window).view(-1, nh, D)
+    want = run()
+    vc[int(tables[0, 50 // page]), 0, 3, 50 % page] = value
+    got = run()
+    reached = torch.zeros_like(want, dtype=torch.bool)
+    reached[50:72 if window is None else 50 + window, :nh // nkv, 3] = True
+    assert torch.equal(~torch.isfinite(got), reached)
+    # the same products in another order of sums over at most 72 keys
+    assert float((got - want)[~reached].abs().max()) <= 2e-6 * max(1.0, float(want.abs().max()))
+
+
 def emu_batch(batch):
     import copy
     host = copy.copy(batch)
