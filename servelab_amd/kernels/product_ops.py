@@ -338,9 +338,10 @@ class ProductOps:
         The kernel saves that pass, which weighs most where rows of W are short, and loses where its whole
         rounds of one tile a CU leave CUs idle: so rows of up to GATED_SHORT_K values, in one round whose
         tiles are GATED_FILL of the CUs or more (GPU time, pair / kernel: 9728 x 896, 1,536 rows 37.8 / 33.1 us;
-        8192 x 1024, 2,048 rows 41.9 / 37.7; 16384 x 1024, 1,024 rows 45.7 / 39.0; 8192 x 512, 2,048 rows 31.1 / 23.2; of 94
-        such sizes of 11 shapes one is slower, by 3 %).  A round filled to a half loses (8192 x 1024, 527 rows
-        21.9 / 30.6); two rounds gain 8 % or lose 20 % as the library's tiles happen to fit.
+        8192 x 1024, 2,048 rows 41.9 / 37.7; 16384 x 1024, 1,024 rows 45.7 / 39.0; 8192 x 512, 2,048 rows 31.1 / 23.2; 11008 x
+        512, 820 rows 50.3 / 20.5; 9728 x 896, 1,000 rows 36.3 / 28.1; 32768 x 1024, 300 rows 36.0 / 34.0; of some 300 such sizes of
+        40 shapes none is more than 4 % slower from GATED_MIN_M rows of x on, at 256 rows and fewer up to 10 %).  A round filled to
+        a half loses (8192 x 1024, 527 rows 21.9 / 30.6); two rounds gain 8 % or lose 20 % as the library's tiles happen to fit.
 
         With longer rows the matrix units are the limit, and the library is the faster one where its pick fills its
         rounds, which it was seen to do where 192 or 224 divides N (2,048 rows of 35840 x 3584 410 / 485, of 28672 x 4096
@@ -361,11 +362,9 @@ class ProductOps:
             fits = (K <= self.GATED_LONG_K and self.GATED_LONG_ROWS[0] <= M <= self.GATED_LONG_ROWS[1] and N % 192 and N % 224
                     and rounds and least * self._num_cus <= last <= most * self._num_cus)
             return 256 if fits else None
-        # (tiles of 192 rows from 1,024 rows of x on: with fewer they take as long as the pair, 16384 x 1024 at 700 rows 33 us
-        # either way)
-        for rows, fewest in ((192, 1024), (256, 768)):
+        for rows in (192, 256):
             tiles = columns * -(-M // rows)
-            if M >= fewest and self.GATED_FILL * self._num_cus <= tiles <= self._num_cus:
+            if M >= self.GATED_MIN_M and self.GATED_FILL * self._num_cus <= tiles <= self._num_cus:
                 return rows
         return None
 

@@ -92,9 +92,10 @@ class Tuning:
     block_square_max_m: int = 1536
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
-    # gated products of a prompt in the block kernel (measured sides: HipOps._gated_rows): the fewest rows of W and the
-    # most rows of x it was measured at; rows of up to gated_short_k values, in one round of tiles filled by gated_fill; ...
+    # gated products of a prompt in the block kernel (measured sides: HipOps._gated_rows): the fewest rows of W, the
+    # fewest and the most rows of x; rows of up to gated_short_k values, in one round of tiles filled by gated_fill; ...
     gated_min_n: int = 4096
+    gated_min_m: int = 257
     gated_max_m: int = 2560
     gated_short_k: int = 1024
     gated_fill: float = 0.84
