@@ -234,6 +234,8 @@ class RecurrentOps:
         lens = getattr(batch, "q_lens", None)
         if not lens or len(lens) != batch.num_seqs or sum(lens) != T:
             lens = None                       # (a batch that does not say: its sequences are taken for long ones)
+        else:
+            longest = max(lens)               # (max_q_len may be a bound)
         columns = 256 // (1 << max(0, (D + 7) // 8 - 1).bit_length()) - (mode == _SCAN_LSTM)
         blocks = H * -(-Dv // max(1, columns))
         several = self.SCAN_CHUNKS_FROM_MANY

@@ -48,5 +48,12 @@ def test_long_and_short_sequences():
     assert split(DECAY, [48] * 9 + [47] * 2 + [1]) == (9, 432, 48, 48, True)
 
 
+def test_a_bound_for_the_longest_sequence():
+    batch = SimpleNamespace(num_seqs=3, max_q_len=512, q_lens=[70, 20, 1])
+    assert Table()._scan_chunks(DECAY, batch, 91, 8, 8, 128, 256) == NONE
+    batch.q_lens = [90, 20, 1]
+    assert Table()._scan_chunks(DECAY, batch, 111, 8, 8, 128, 256) == (1, 90, 90, 80, True)
+
+
 def test_a_batch_that_does_not_say():
     assert split(DECAY, [79], told=False) == NONE and split(DECAY, [80, 1], told=False) == (2, 81, 80, 1, False)
