@@ -26,7 +26,7 @@
 
 // ------------------------------------------------------------------ route
 // One wavefront per token; lane k < top gets the expert of the k-th choice.  Largest first; among equal logits the lower
-// index wins.
+// index wins.  NaN counts as -infinity there, so that a choice is an expert whatever the row holds; its share is NaN.
 // over_all: the numbers compared are softmax(z)[e] + correction[e] over all E, and a chosen
 // expert's share is softmax(z)[e] / (sum over the chosen + 1e-20) * scale.  sigmoid: the logits are
 // compared, and a chosen expert's share is the sigmoid of its own.
@@ -60,8 +60,8 @@ __device__ __forceinline__ int route_token(const Route& r, size_t t, int lane) {
   float mine = 0.f;                            // lane k keeps the k-th largest logit
   int mine_e = 0;
   auto number = [&](int e) -> float {          // what the experts are compared by
-    const float v = z[e];
-    return over_all ? expf(v - zmax) * inv_sum + (correction != nullptr ? correction[e] : 0.f) : v;
+    const float v = z[e], c = over_all ? expf(v - zmax) * inv_sum + (correction != nullptr ? correction[e] : 0.f) : v;
+    return c == c ? c : -INFINITY;
   };
   float kept[4];                               // a lane's first four numbers stay in registers (E <= 256: all)
 #pragma unroll
@@ -93,7 +93,7 @@ __device__ __forceinline__ int route_token(const Route& r, size_t t, int lane) {
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) at = min(at, __shfl_xor(at, o, SL_WAVE));
     }
-    best = most;
+    best = most == -INFINITY && !over_all ? z[at] : most;
     if (at % 64 == lane) taken |= 1ull << (at / 64);
     if (lane == k) {
       mine = best;

@@ -75,6 +75,30 @@ def test_rows_a_tile_holds():
     assert HipOps(torch.float32, DEV).route_tokens(torch.randn(200, 8, device=DEV), 8, 8).tile_rows == 16
 
 
+@pytest.mark.parametrize("T,E,top", [(4, 64, 8), (16, 300, 4), (17, 64, 8), (4, 5, 5)])
+@pytest.mark.parametrize("form", ["softmax", "over all", "sigmoid"])
+def test_routes_of_logits_that_are_not_numbers(T, E, top, form):
+    """Every choice is an expert, NaN behind all numbers, and its row's shares say so; other rows are as without such a row."""
+    hip = HipOps(torch.bfloat16, DEV)
+    z = torch.randn(T, E, generator=torch.Generator().manual_seed(E))
+    route = lambda z: hip.route_tokens(z.to(DEV), E, top, over_all=form == "over all", sigmoid=form == "sigmoid")
+    before = route(z)
+    z[1] = torch.nan
+    z[2, top - 1:] = torch.nan                                        # one number too few
+    z[3, E - 1] = torch.nan
+    r = route(z)
+    number = torch.where(z.isnan() | (z.isnan().any(-1, keepdim=True) if form == "over all" else False), -torch.inf, z)
+    assert torch.equal(r.chosen.cpu().long(), torch.sort(-number, dim=-1, stable=True).indices[:, :top])
+    odd = z.gather(1, r.chosen.cpu().long()).isnan()
+    if form != "sigmoid":                                             # (a share takes in the chosen ones' sum, or that of all)
+        odd = (z.isnan() if form == "over all" else odd).any(-1, keepdim=True).expand(T, top)
+    assert torch.equal(r.shares.cpu().isnan(), odd)
+    same = [t for t in range(T) if t not in (1, 2, 3)]
+    assert torch.equal(r.chosen[same], before.chosen[same]) and torch.equal(r.shares[same], before.shares[same])
+    flat, order = r.chosen.cpu().flatten().long(), r.order.cpu().long()
+    assert torch.equal(order[r.place_of.cpu().long()], torch.arange(T * top)) and (flat[order].diff() >= 0).all()
+
+
 # one workgroup for both up to 16 tokens and 1,024 experts, two kernels beyond; experts a wavefront adds up in one, two and
 # more rounds, some without matrices, equal logits, logits of minus infinity
 @pytest.mark.parametrize("T,E,top", [(1, 1, 1), (1, 64, 8), (16, 65, 8), (17, 65, 8), (5, 300, 64), (16, 1024, 3), (16, 1025, 3)])
