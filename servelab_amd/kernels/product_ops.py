@@ -335,13 +335,15 @@ class ProductOps:
     def _gated_rows(self, M, N, K):
         """Rows of x a workgroup of the block kernel takes (192 or 256) for the gated product of a
         prompt, or None where the library's product and a pass that gates it are the faster pair.
-        The kernel saves that pass, which weighs most where rows of W are short, and loses where its whole
-        rounds of one tile a CU leave CUs idle: so rows of up to GATED_SHORT_K values, in one round whose
-        tiles are GATED_FILL of the CUs or more (GPU time, pair / kernel: 9728 x 896, 1,536 rows 37.8 / 33.1 us;
-        8192 x 1024, 2,048 rows 41.9 / 37.7; 16384 x 1024, 1,024 rows 45.7 / 39.0; 8192 x 512, 2,048 rows 31.1 / 23.2; 11008 x
-        512, 820 rows 50.3 / 20.5; 9728 x 896, 1,000 rows 36.3 / 28.1; 32768 x 1024, 300 rows 36.0 / 34.0; of some 300 such sizes of
-        40 shapes none is more than 4 % slower from GATED_MIN_M rows of x on, at 256 rows and fewer up to 10 %).  A round filled to
-        a half loses (8192 x 1024, 527 rows 21.9 / 30.6); two rounds gain 8 % or lose 20 % as the library's tiles happen to fit.
+        The kernel saves that pass, which weighs most where rows of W are short, and loses where its rounds of one tile a CU
+        leave many CUs idle: so rows of up to GATED_SHORT_K values, in as few rounds as either tile gives (of 192 rows where
+        that is the same), if a single round is filled by GATED_FILL[0] and the last of several by GATED_FILL[1] (GPU time, pair /
+        kernel: 9728 x 896, 1,000 rows 36.3 / 28.1 us, 1,536 rows 37.3 / 34.1, 2,048 rows 62.7 / 57.8; 8192 x 1024, 2,048 rows 41.9 / 37.7;
+        16384 x 1024, 1,024 rows 45.7 / 39.0).  Rows of up to GATED_SHORTEST_K values win from GATED_SHORTEST_FILL of one round on
+        (11008 x 512, 820 rows 50.3 / 20.5; 9728 x 512, 2,048 rows 54.1 / 34.4).  Of 660 such sizes of 60 shapes the kernel takes 0.65,
+        0.68, 0.88, 0.93 and 0.94 of the pair's time on average with rows of 256, 512, 768, 896 and 1,024 values and at most 1.11
+        (14336 x 1024, 1,200 rows; 24576 x 768, 700 rows).  Less well filled it loses (8192 x 1024, 527 rows 21.9 / 30.6; 9728 x
+        896, 1,600 rows 45.8 / 56.4; 24576 x 1024, 527 rows, 1.4 of the pair's time), and with 256 rows of x and fewer by up to 10 %.
 
         With longer rows the matrix units are the limit, and the library is the faster one where its pick fills its
         rounds, which it was seen to do where 192 or 224 divides N (2,048 rows of 35840 x 3584 410 / 485, of 28672 x 4096
@@ -362,11 +364,15 @@ class ProductOps:
             fits = (K <= self.GATED_LONG_K and self.GATED_LONG_ROWS[0] <= M <= self.GATED_LONG_ROWS[1] and N % 192 and N % 224
                     and rounds and least * self._num_cus <= last <= most * self._num_cus)
             return 256 if fits else None
-        for rows in (192, 256):
-            tiles = columns * -(-M // rows)
-            if M >= self.GATED_MIN_M and self.GATED_FILL * self._num_cus <= tiles <= self._num_cus:
-                return rows
-        return None
+        if M < self.GATED_MIN_M:
+            return None
+        tiles = {rows: columns * -(-M // rows) for rows in (192, 256)}
+        rounds = {rows: -(-n // self._num_cus) for rows, n in tiles.items()}
+        rows = 192 if rounds[192] == rounds[256] else 256
+        last = tiles[rows] / self._num_cus - (rounds[rows] - 1)
+        if K <= self.GATED_SHORTEST_K:
+            return rows if rounds[rows] > 1 or last >= self.GATED_SHORTEST_FILL else None
+        return rows if last >= self.GATED_FILL[rounds[rows] > 1] else None
 
     def _tuned_for(self, M, N, K) -> bool:
         """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside

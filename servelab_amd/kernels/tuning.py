@@ -93,12 +93,15 @@ class Tuning:
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
     # gated products of a prompt in the block kernel (measured sides: HipOps._gated_rows): the fewest rows of W, the
-    # fewest and the most rows of x; rows of up to gated_short_k values, in one round of tiles filled by gated_fill; ...
+    # fewest and the most rows of x; rows of up to gated_short_k values, in one round of tiles filled so far or in several
+    # whose last is; rows of up to gated_shortest_k values, in one round filled so far or in any several; ...
     gated_min_n: int = 4096
     gated_min_m: int = 257
     gated_max_m: int = 2560
     gated_short_k: int = 1024
-    gated_fill: float = 0.84
+    gated_fill: tuple = (0.7, 0.4)
+    gated_shortest_k: int = 512
+    gated_shortest_fill: float = 0.5
     # ... longer ones, up to gated_long_k values and for so many rows of x, in several rounds, the last filled so far
     gated_long_k: int = 5120
     gated_long_rows: tuple = (1537, 2048)
