@@ -335,15 +335,17 @@ class ProductOps:
     def _gated_rows(self, M, N, K):
         """Rows of x a workgroup of the block kernel takes (192 or 256) for the gated product of a
         prompt, or None where the library's product and a pass that gates it are the faster pair.
-        The kernel saves that pass, which weighs most where rows of W are short, and loses where its rounds of one tile a CU
-        leave many CUs idle: so rows of up to GATED_SHORT_K values, in as few rounds as either tile gives (of 192 rows where
-        that is the same), if a single round is filled by GATED_FILL[0] and the last of several by GATED_FILL[1] (GPU time, pair /
-        kernel: 9728 x 896, 1,000 rows 36.3 / 28.1 us, 1,536 rows 37.3 / 34.1, 2,048 rows 62.7 / 57.8; 8192 x 1024, 2,048 rows 41.9 / 37.7;
-        16384 x 1024, 1,024 rows 45.7 / 39.0).  Rows of up to GATED_SHORTEST_K values win from GATED_SHORTEST_FILL of one round on
-        (11008 x 512, 820 rows 50.3 / 20.5; 9728 x 512, 2,048 rows 54.1 / 34.4).  Of 660 such sizes of 60 shapes the kernel takes 0.65,
-        0.68, 0.88, 0.93 and 0.94 of the pair's time on average with rows of 256, 512, 768, 896 and 1,024 values and at most 1.11
-        (14336 x 1024, 1,200 rows; 24576 x 768, 700 rows).  Less well filled it loses (8192 x 1024, 527 rows 21.9 / 30.6; 9728 x
-        896, 1,600 rows 45.8 / 56.4; 24576 x 1024, 527 rows, 1.4 of the pair's time), and with 256 rows of x and fewer by up to 10 %.
+        The kernel saves that pass and the host the library's call, some 25 us a layer. Rows of up to GATED_SHORT_K values
+        therefore always take it: such models' prompts wait for the host at nearly every size (whole passes, pair / kernel: 24
+        layers of the 0.5B shape, 9728 x 896, 260 / 600 / 1,000 / 1,700 / 2,048 tokens 4,893 / 4,194, 3,837 / 3,356, 4,116 /
+        3,604, 4,184 / 3,901 and 4,381 / 4,191 us, three prompts of 1,500 12,818 / 11,166; 12 layers of 4096 x 1024, 256 and
+        2,048 tokens 2,063 / 1,823 and 2,133 / 1,862, of 24576 x 1024, 527 tokens 1,930 / 1,846). By GPU time alone it wins
+        where its last round of one tile a CU is well filled and loses elsewhere, by less than that call (9728 x 896, 300 /
+        1,000 / 1,600 / 2,048 rows 21.7 / 28.2, 36.3 / 28.1, 45.8 / 56.4 and 62.7 / 57.8 us; 4096 x 1024, 256 rows 11.7 / 23.4).
+        Tiles are as high as their estimated time says. Rows of up to GATED_ONE_ROUND_K values take it where one round of tiles
+        is GATED_FILL useful (the 1.5B shape, 17920 x 1536, 12 layers, 527 / 700 / 768 tokens 1,994 / 1,828, 2,081 / 2,041 and
+        2,119 / 2,089; GPU time 42 / 47, 51 / 49 and 52 / 51 a product; with 2,048 values the kernel is 5 to 20 % slower there,
+        17920 x 2048, 768 rows 57 / 62).
 
         With longer rows the matrix units are the limit, and the library is the faster one where its pick fills its
         rounds, which it was seen to do where 192 or 224 divides N (2,048 rows of 35840 x 3584 410 / 485, of 28672 x 4096
@@ -358,21 +360,16 @@ class ProductOps:
                 or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
             return None
         columns = -(-N // 256)
-        if K > self.GATED_SHORT_K:
-            rounds, last = divmod(columns * -(-M // 256), self._num_cus)
-            least, most = self.GATED_LAST_ROUND
-            fits = (K <= self.GATED_LONG_K and self.GATED_LONG_ROWS[0] <= M <= self.GATED_LONG_ROWS[1] and N % 192 and N % 224
-                    and rounds and least * self._num_cus <= last <= most * self._num_cus)
-            return 256 if fits else None
-        if M < self.GATED_MIN_M:
-            return None
-        tiles = {rows: columns * -(-M // rows) for rows in (192, 256)}
-        rounds = {rows: -(-n // self._num_cus) for rows, n in tiles.items()}
-        rows = 192 if rounds[192] == rounds[256] else 256
-        last = tiles[rows] / self._num_cus - (rounds[rows] - 1)
-        if K <= self.GATED_SHORTEST_K:
-            return rows if rounds[rows] > 1 or last >= self.GATED_SHORTEST_FILL else None
-        return rows if last >= self.GATED_FILL[rounds[rows] > 1] else None
+        if M >= self.GATED_MIN_M and K <= self.GATED_ONE_ROUND_K:
+            rounds = {rows: -(-columns * -(-M // rows) // self._num_cus) for rows in (256, 192)}
+            rows = min(rounds, key=lambda r: rounds[r] * (r * K + 65536))
+            if K <= self.GATED_SHORT_K or (rounds[rows] == 1 and M * N >= self.GATED_FILL * self._num_cus * rows * 256):
+                return rows
+        rounds, last = divmod(columns * -(-M // 256), self._num_cus)
+        least, most = self.GATED_LAST_ROUND
+        fits = (K <= self.GATED_LONG_K and self.GATED_LONG_ROWS[0] <= M <= self.GATED_LONG_ROWS[1] and N % 192 and N % 224
+                and rounds and least * self._num_cus <= last <= most * self._num_cus)
+        return 256 if fits else None
 
     def _tuned_for(self, M, N, K) -> bool:
         """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside

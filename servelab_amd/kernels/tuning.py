@@ -93,15 +93,14 @@ class Tuning:
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
     # gated products of a prompt in the block kernel (measured sides: HipOps._gated_rows): the fewest rows of W, the
-    # fewest and the most rows of x; rows of up to gated_short_k values, in one round of tiles filled so far or in several
-    # whose last is; rows of up to gated_shortest_k values, in one round filled so far or in any several; ...
+    # fewest and the most rows of x; rows of up to gated_short_k values, or up to gated_one_round_k in one round of tiles of
+    # which so much is useful; ...
     gated_min_n: int = 4096
-    gated_min_m: int = 257
+    gated_min_m: int = 256
     gated_max_m: int = 2560
     gated_short_k: int = 1024
-    gated_fill: tuple = (0.7, 0.4)
-    gated_shortest_k: int = 512
-    gated_shortest_fill: float = 0.5
+    gated_one_round_k: int = 1536
+    gated_fill: float = 0.7
     # ... longer ones, up to gated_long_k values and for so many rows of x, in several rounds, the last filled so far
     gated_long_k: int = 5120
     gated_long_rows: tuple = (1537, 2048)

@@ -42,22 +42,18 @@ def test_routes_of_prompts_products():
     ops = HipOps(torch.bfloat16, DEV)
     gated = ops._gated_rows
     assert ops._num_cus == 256
-    # the fewer rounds of tiles, of 192 rows if equal; one filled to 0.7 or several with the last filled to 0.4
-    assert [gated(M, 8192, 1024) for M in (256, 960, 961, 1536, 1537, 2048, 2049, 2112, 2113)] == \
-        [None, None, 192, 192, 256, 256, None, None, 192]
-    assert [gated(M, 9728, 896) for M in (768, 769, 1152, 1153, 1536, 1537, 1728, 1729, 2496, 2497, 2560, 2561)] == \
-        [None, 192, 192, 256, 256, None, None, 192, 192, 256, 256, None]
-    assert [gated(M, 16384, 1024) for M in (384, 385, 768, 769, 1024, 1025)] == [None, 192, 192, 256, 256, 192]
-    # rows of 512 values: half a round, or several however filled
-    assert [gated(M, 4096, 512) for M in (1344, 1345, 2560, 2561)] == [None, 192, 192, None]
-    assert [gated(M, 32768, 512) for M in (256, 257, 384, 385, 512, 513, 768, 769)] == [None, 192, 192, 256, 256, 192, 192, 256]
-    assert gated(384, 16384, 512) == 192 and gated(384, 16384, 576) is None
-    assert gated(1536, 8192, 1056) is None                                                     # K not in steps of 64
+    # rows of up to 1,024 values: always, in the tiles that take fewer or shorter rounds
+    assert [gated(M, 8192, 1024) for M in (255, 256, 1536, 1537, 2048, 2049, 2560, 2561)] == [None, 192, 192, 256, 256, 192, 192, None]
+    assert [gated(M, 9728, 896) for M in (256, 1152, 1153, 1536, 1537)] == [192, 192, 256, 256, 192]
+    assert gated(256, 4096, 64) == 192 and gated(256, 4095, 1024) is None and gated(1536, 8192, 1000) is None
+    # up to 1,536: one round, 0.7 of it useful
+    assert [gated(M, 17920, 1536) for M in (491, 492, 576, 577, 655, 656, 768, 769)] == [None, 192, 192, None, None, 256, 256, None]
+    assert gated(1536, 8192, 1536) == 192 and gated(1536, 8192, 1600) is None and gated(1536, 8192, 1056) is None
     # longer rows: several rounds, the last one more than half filled, and no tile of the library's that divides N
     assert [gated(M, 37888, 3584) for M in (1536, 1792, 1793, 2048, 2049)] == [None, None, 256, 256, None]
     assert [gated(M, 27392, 2560) for M in (1536, 1537, 1792, 1793)] == [None, 256, 256, None]
     assert gated(2048, 35840, 3584) is None and gated(2048, 24576, 3072) is None               # 160 times 224, 128 times 192
-    assert gated(2048, 9216, 3584) is None and gated(1536, 8192, 1088) is None and gated(2048, 37888, 5184) is None
+    assert gated(2048, 9216, 3584) is None and gated(1536, 8192, 1664) is None and gated(2048, 37888, 5184) is None
     x = torch.randn(1200, 1024, device=DEV).bfloat16()
     w = (torch.randn(8192, 1024, device=DEV) * 0.03).bfloat16()
     weight = ops.prepare_weight(w)
