@@ -76,11 +76,11 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(
 #if defined(SL_F32)
 // The same with K cut among the four wavefronts of a workgroup, which then own NC columns together: a matrix of few rows
 // still has a workgroup for every CU, and a lane's running sums are a quarter as long (1,536 columns of 8,960 at 1 / 3 / 8
-// rows: 22 / 39 / 60 -> 11 / 15 / 23 us, 5.0 TB/s at one row; errors halve).  STREAM: W is read past the caches, which
-// pays where it is larger than the 32 MB of the dies' L2 (us, through them / past them: 37,888 columns of 3,584 at 1 / 3 rows
-// 84.5 / 94.3 and 74.8 / 86.8, 3,584 of 18,944 51 / 57 and 46 / 54, 2,048 of 11,008 18.2 / 22.6 and 16.4 / 21.3) and costs
-// where it is smaller (896 of 4,864 at 3 rows 7.2 and 8.3, 1,536 of 1,536 5.4 and 6.0, 3,072 of 1,024 at 4 rows 7.5 and 8.0).
-template <int MB, int NC, bool STREAM>
+// rows: 22 / 39 / 60 -> 11 / 15 / 23 us, 5.0 TB/s at one row; errors halve).  W is read past the caches: a model reads every
+// matrix once a step, and by the next one it has left them (us over matrices in turn, 1.2 GB in all, through the caches / past them:
+// 896 of 896 at one row 3.2 and 2.9, 1,536 of 1,536 at 1 / 8 rows 4.1 / 8.4 and 3.8 / 8.1, 2,560 of 2,048 6.7 / 14.5 and 6.2 / 14.2, 3,584
+// of 3,584 11.7 / 23.3 and 11.2 / 23.2; one matrix again and again is faster through them, 896 of 4,864 at 3 rows 7.2 and 8.3).
+template <int MB, int NC>
 __global__ __launch_bounds__(256) void gemm_rows_split_kernel(
     const act_t* __restrict__ x, const act_t* __restrict__ w, const float* __restrict__ bias,
     void* __restrict__ y, int M, int N, int K) {
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void gemm_rows_split_kernel(
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       vec_t wv;
-      const rows_v4 raw = STREAM ? __builtin_nontemporal_load((const rows_v4*)(wr[c] + k)) : *(const rows_v4*)(wr[c] + k);
+      const rows_v4 raw = __builtin_nontemporal_load((const rows_v4*)(wr[c] + k));
       __builtin_memcpy(&wv, &raw, 16);
 #pragma unroll
       for (int j = 0; j < SL_VEC; ++j) wf[c][j] = to_f(wv.v[j]);
@@ -134,19 +134,14 @@ __global__ __launch_bounds__(256) void gemm_rows_split_kernel(
     }
   }
 }
-template <int NC, bool STREAM>
-static const char* rows_split(const act_t* x, const act_t* w, const float* bias, void* y, int M, int N, int K, hipStream_t stream) {
-  const int grid = (N + NC - 1) / NC;
-  if (M == 1) gemm_rows_split_kernel<1, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  else if (M == 2) gemm_rows_split_kernel<2, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  else if (M <= 4) gemm_rows_split_kernel<4, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  else gemm_rows_split_kernel<8, NC, STREAM><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  return sl_launch_status();
-}
 template <int NC>
 static const char* rows_split(const act_t* x, const act_t* w, const float* bias, void* y, int M, int N, int K, hipStream_t stream) {
-  return (long long)N * K >= 8 << 20 ? rows_split<NC, true>(x, w, bias, y, M, N, K, stream)
-                                     : rows_split<NC, false>(x, w, bias, y, M, N, K, stream);
+  const int grid = (N + NC - 1) / NC;
+  if (M == 1) gemm_rows_split_kernel<1, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else if (M == 2) gemm_rows_split_kernel<2, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else if (M <= 4) gemm_rows_split_kernel<4, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else gemm_rows_split_kernel<8, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  return sl_launch_status();
 }
 #endif
 
