@@ -1835,16 +1835,15 @@ extern "C" const char* sl_untile_weight(const void* wt, void* w, int N, int K, i
 // latency that is what keeps the stream going.  A stage holds the rows of x, then those of W, 8
 // units of 16 bytes a row; a lane can put any unit anywhere at no cost, so they lie as lds_place says.
 
-template <int WM, int WN, int STAGES, bool GATED>
+template <int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ w, const float* __restrict__ bias,
-    void* __restrict__ y, int M, int N, int K, int out_f32, int act, int KS) {
-  constexpr int WAVES = WM * WN, BM = 64 * WM, BN = 64 * WN;
-  static_assert(STAGES == 2 || STAGES == 3, "a ring of two or three stages");
+    void* __restrict__ y, int M, int N, int K, int out_f32, int KS) {
+  constexpr int WAVES = WM * WN, BM = 64 * WM, BN = 64 * WN, STAGES = 3;
   constexpr int ROWS = BM + BN;                      // rows of a stage: x, then W; 128 bytes each
   constexpr int STAGE_BYTES = ROWS * 128;
-  constexpr int LOADS = (ROWS / 8 + WAVES - 1) / WAVES;        // wavefront-wide loads (8 rows) a wavefront makes per chunk
-  static_assert(STAGES == 2 || LOADS * 8 * WAVES == ROWS, "a count of loads under way must hold for every wavefront");
+  constexpr int LOADS = ROWS / 8 / WAVES;            // wavefront-wide loads (8 rows) a wavefront makes per chunk
+  static_assert(LOADS * 8 * WAVES == ROWS, "a count of loads under way must hold for every wavefront");
   __shared__ __attribute__((aligned(1024))) char ring[STAGES * STAGE_BYTES];
   const int t = threadIdx.x, lane = t & 63, i = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1883,9 +1882,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
   auto fetch = [&](int c, int stage) {
     const unsigned at = ring_at + STAGE_BYTES * stage + 1024 * wave;
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j)
-      if (LOADS * 8 * WAVES == ROWS || wave + WAVES * j < ROWS / 8)
-        load_to_lds(src[j] + 64 * (size_t)c, at + 1024 * WAVES * j);
+    for (int j = 0; j < LOADS; ++j) load_to_lds(src[j] + 64 * (size_t)c, at + 1024 * WAVES * j);
   };
   // where this lane reads its operands: row R0 + i (R0 a multiple of 16), unit 4 kk + gq
   int at_kk[2];
@@ -1900,7 +1897,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
 
   if (cbeg < cend) {
     fetch(cbeg, 0);
-    if (STAGES == 3 && cbeg + 1 < cend) {
+    if (cbeg + 1 < cend) {
       fetch(cbeg + 1, 1);
       wait_loads<LOADS>();
     } else {
@@ -1927,7 +1924,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
         for (int v = 0; v < 4; ++v)
           acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[v], acc[u][v], 0, 0, 0);
     }
-    if (more && STAGES == 3) wait_loads<LOADS>();        // all but the chunk just asked for
+    if (more) wait_loads<LOADS>();        // all but the chunk just asked for
     else wait_loads<0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" : : : "memory");
@@ -1938,31 +1935,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int m = m0 + 64 * wm + 16 * v + i;
-    if constexpr (GATED) {
-      // gate and up rows lie in blocks of eight: lanes 0..31 of a tile's sums hold gates, 32..63 ups.  Two tiles
-      // trade halves, so that every lane holds four gates and their four ups.
-#pragma unroll
-      for (int u = 0; u < 4; u += 2) {
-        const int n = n0 + 64 * wn + 16 * u + 4 * gq;
-        f32x4 r0 = acc[u][v], r1 = acc[u + 1][v];
-        if (bias != nullptr) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (n + e < N) r0[e] += bias[n + e];
-            if (n + 16 + e < N) r1[e] += bias[n + 16 + e];
-          }
-        }
-        bf16x4 h;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(r0[e]), __float_as_uint(r1[e]), false, false);
-          h[e] = (__bf16)(sl_act(__uint_as_float(both[0]), act) * __uint_as_float(both[1]));
-        }
-        const int o = (n0 + 64 * wn + 16 * u) / 2 + 8 * (gq >> 1) + 4 * (gq & 1);
-        if (m < M && o < N / 2) *(bf16x4*)((__bf16*)y + (size_t)m * (N / 2) + o) = h;
-      }
-      continue;
-    }
     if (m >= M) continue;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -2005,40 +1977,55 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_block_kernel(
   }
 }
 
+#include "gemm_rounds.h"
+
+template <int T>
+static void rounds(const __bf16* x, const __bf16* w, const float* bias, void* y, int M, int N, int K, int out_f32, int gated,
+                   int act, int ks, hipStream_t stream) {
+  const long long items = (long long)((N + 255) / 256) * ((M + 64 * T - 1) / (64 * T)) * ks;
+  const int cus = device_cus() & ~7;
+  const long long even = 8 * ((items + 7) / 8);
+  const dim3 grid((unsigned)(cus >= 8 && cus < even ? cus : even));
+  if (gated) gemm_rounds_kernel<T, ROUNDS_GATED><<<grid, 512, 0, stream>>>(x, w, bias, y, M, N, K, gated, 1);
+  else if (out_f32 || ks > 1) gemm_rounds_kernel<T, ROUNDS_F32><<<grid, 512, 0, stream>>>(x, w, bias, y, M, N, K, 0, ks);
+  else gemm_rounds_kernel<T, ROUNDS_BF16><<<grid, 512, 0, stream>>>(x, w, bias, y, M, N, K, act, 1);
+}
+
 // x and W row-major.  gated (an activation): W's rows hold gate and up in blocks of eight, y [M, N / 2] = act(gate) * up
-// of the float sums (8192 x 1024, 2,048 rows: 37.7 us, the library's product and the kernel that gates it 41.9).
+// of the float sums; act: y = act(x W^T + bias), bfloat16.
 // ks > 1: `part` holds ks * M * N floats; with y == nullptr they are left
 // there for the reader to add (and the bias with them), else splitk_reduce adds them into y.
+// square: rows of x a tile, 256 or 192, by 256 of W (gemm_rounds.h); 0: tiles of 256 x 128.
 extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* bias, void* y,
-                                     int M, int N, int K, int out_f32, int gated, int ks, int square, float* part,
+                                     int M, int N, int K, int out_f32, int gated, int act, int ks, int square, float* part,
                                      hipStream_t stream) {
   SL_CHECK(M > 0 && N > 0 && K > 0, "gemm_block: sizes must be positive");
-  SL_CHECK(K % 64 == 0, "gemm_block: K must be a multiple of 64");
+  SL_CHECK(K % 64 == 0 && K <= (1 << 22), "gemm_block: K must be a multiple of 64, 4 M at most");
   SL_CHECK(ks >= 1 && ks <= 64 && ks <= K / 64, "gemm_block: ks must be in 1..64 and <= K / 64");
   SL_CHECK(ks == 1 || part != nullptr, "gemm_block: a split of K needs the partial buffer");
   SL_CHECK(y != nullptr || ks > 1, "gemm_block: no output");
-  SL_CHECK(square == 0 || square == 256 || (square == 192 && gated), "gemm_block: tiles of 256 rows by 128 or 256, gated ones of 256 or 192 by 256");
+  SL_CHECK(square == 0 || square == 256 || square == 192, "gemm_block: tiles of 256 rows by 128 or 256, or of 192 by 256");
   SL_CHECK(!gated || (square && ks == 1 && !out_f32 && N % 16 == 0),
            "gemm_block: a gated product takes wide tiles, whole rows of K, blocks of eight and bfloat16 results");
+  SL_CHECK(!act || (square && ks == 1 && !out_f32 && !gated), "gemm_block: an activation takes wide tiles, whole rows of K and bfloat16 results");
   SL_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_block: x and W must be 16-byte aligned");
   void* dst = ks > 1 ? (void*)part : y;
+  const float* b = ks > 1 ? nullptr : bias;
   const __bf16* xx = (const __bf16*)x;
   const __bf16* ww = (const __bf16*)w;
   // (Tiles of 64 x 256 and 128 x 256 for fewer rows of x were built and measured: alone they beat the
   // LDS-staged kernel above, in a decode step of 24 to 128 requests they lost 2-5 % tokens/s to it,
   // so that kernel keeps those rows and this one starts where it ends.)
-  // square: tiles of 256 x 256 (sixteen wavefronts, a ring of two stages in 128 KB of LDS) instead of
-  // 256 x 128 (eight wavefronts, three stages): a workgroup pulls 512 rows for 256 x 256 of result
-  // instead of 384 for 256 x 128, which is what the time of these products follows.
-  // 192: tiles of 192 x 256 (twelve wavefronts) where those fill a round of the CUs, see the caller's rule.
   const int bn = square ? 256 : 128, bm = square == 192 ? 192 : 256;
   const long long triples = (long long)((N + bn - 1) / bn) * ((M + bm - 1) / bm) * ks;
-  SL_CHECK(triples < (1ll << 28), "gemm_block: too many tiles");
-  const dim3 grid((unsigned)(8 * ((triples + 7) / 8)));              // laid out by chiplet (see the kernel)
-  if (gated && square == 192) gemm_block_kernel<3, 4, 2, true><<<grid, 768, 0, stream>>>(xx, ww, bias, dst, M, N, K, 0, gated, 1);
-  else if (gated) gemm_block_kernel<4, 4, 2, true><<<grid, 1024, 0, stream>>>(xx, ww, bias, dst, M, N, K, 0, gated, 1);
-  else if (square) gemm_block_kernel<4, 4, 2, false><<<grid, 1024, 0, stream>>>(xx, ww, bias, dst, M, N, K, out_f32, 0, ks);
-  else gemm_block_kernel<4, 2, 3, false><<<grid, 512, 0, stream>>>(xx, ww, bias, dst, M, N, K, out_f32, 0, ks);
+  SL_CHECK(triples < (1ll << 24), "gemm_block: too many tiles");
+  if (square) {
+    if (square == 192) rounds<3>(xx, ww, b, dst, M, N, K, out_f32, gated, act, ks, stream);
+    else rounds<4>(xx, ww, b, dst, M, N, K, out_f32, gated, act, ks, stream);
+  } else {
+    const dim3 grid((unsigned)(8 * ((triples + 7) / 8)));              // laid out by chiplet (see the kernel)
+    gemm_block_kernel<4, 2><<<grid, 512, 0, stream>>>(xx, ww, b, dst, M, N, K, out_f32, ks);
+  }
   const char* e = sl_launch_status();
   if (e || ks == 1 || y == nullptr) return e;
   const size_t total = (size_t)M * N;

@@ -7,6 +7,10 @@
 __device__ __forceinline__ void load_to_lds(const void* from, unsigned lds_at) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
 }
+// The same from a base that all lanes share and an offset of the lane's own.
+__device__ __forceinline__ void load_to_lds(unsigned offset, const void* base, unsigned lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" : : "v"(offset), "s"(lds_at), "s"(base) : "m0");
+}
 template <int N_> __device__ __forceinline__ void wait_loads() {
   __builtin_amdgcn_s_waitcnt((N_ & 15) | (7 << 4) | ((N_ >> 4) << 14));
 }

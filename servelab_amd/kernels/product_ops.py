@@ -333,28 +333,18 @@ class ProductOps:
         return (shares, True) if (shares == 2 and fill >= 0.875) or (shares == 3 and fill >= 0.8) else None
 
     def _gated_rows(self, M, N, K):
-        """Rows of x a workgroup of the block kernel takes (192 or 256) for the gated product of a
-        prompt, or None where the library's product and a pass that gates it are the faster pair.
-        The kernel saves that pass and the host the library's call, some 25 us a layer. Rows of up to GATED_SHORT_K values
-        therefore always take it: such models' prompts wait for the host at nearly every size (whole passes, pair / kernel: 24
-        layers of the 0.5B shape, 9728 x 896, 260 / 600 / 1,000 / 1,700 / 2,048 tokens 4,893 / 4,194, 3,837 / 3,356, 4,116 /
-        3,604, 4,184 / 3,901 and 4,381 / 4,191 us, three prompts of 1,500 12,818 / 11,166; 12 layers of 4096 x 1024, 256 and
-        2,048 tokens 2,063 / 1,823 and 2,133 / 1,862, of 24576 x 1024, 527 tokens 1,930 / 1,846). By GPU time alone it wins
-        where its last round of one tile a CU is well filled and loses elsewhere, by less than that call (9728 x 896, 300 /
-        1,000 / 1,600 / 2,048 rows 21.7 / 28.2, 36.3 / 28.1, 45.8 / 56.4 and 62.7 / 57.8 us; 4096 x 1024, 256 rows 11.7 / 23.4).
-        Tiles are as high as their estimated time says. Rows of up to GATED_ONE_ROUND_K values take it where one round of tiles
-        is GATED_FILL useful (the 1.5B shape, 17920 x 1536, 12 layers, 527 / 700 / 768 tokens 1,994 / 1,828, 2,081 / 2,041 and
-        2,119 / 2,089; GPU time 42 / 47, 51 / 49 and 52 / 51 a product; with 2,048 values the kernel is 5 to 20 % slower there,
-        17920 x 2048, 768 rows 57 / 62).
-
-        With longer rows the matrix units are the limit, and the library is the faster one where its pick fills its
-        rounds, which it was seen to do where 192 or 224 divides N (2,048 rows of 35840 x 3584 410 / 485, of 28672 x 4096
-        374 / 437); where it does not, it idles as the kernel does and pays for the pass on top (of 37888 x 3584 547 / 496, of
-        22016 x 2048 196 / 181, of 23552 x 2048 249 / 182).  So: N that neither divides, and several rounds of tiles
-        of 256 x 256 whose last one is filled by GATED_LAST_ROUND; rows of up to GATED_LONG_K
-        values and GATED_LONG_ROWS rows of x, where this was measured (124 sizes of 28 shapes: 12 % faster on average, but slower
-        at a fifth of them, by up to 15 %, since the pick is not known: 15104 x 2048, 2,048 rows 109 / 121; of 284 sizes
-        outside the rule 30 % are faster, and the average is 3 % slower).  The sums meet the activation unrounded, so that it
+        """Rows of x a workgroup takes (192 or 256) for the gated product of a prompt at sizes that take the tiles whatever their
+        estimated rate (``_prompt_tiles``) says, or None.  The kernel saves the pass that gates the library's product and the
+        host the library's call, some 25 us a layer.  Rows of up to GATED_SHORT_K values
+        therefore always take it: such models' prompts wait for the host at nearly every size (whole passes, pair / kernel as it
+        was with sixteen wavefronts: 24 layers of the 0.5B shape, 9728 x 896, 260 / 600 / 1,000 / 1,700 / 2,048 tokens 4,893 / 4,194,
+        3,837 / 3,356, 4,116 / 3,604, 4,184 / 3,901 and 4,381 / 4,191 us; 12 layers of 4096 x 1024, 256 and
+        2,048 tokens 2,063 / 1,823 and 2,133 / 1,862).  By GPU time alone it wins there as well now (9728 x 896, 300 / 1,000 /
+        1,600 / 2,048 rows 38 / 19, 35 / 22, 60 / 38 and 66 / 40 us).  Rows of up to GATED_ONE_ROUND_K values take it where one
+        round of tiles is GATED_FILL useful (17920 x 1536, 527 / 640 / 768 rows 38 / 31, 43 / 38 and 46 / 39 us a product), and
+        longer ones, up to GATED_LONG_K values at GATED_LONG_ROWS rows of x, in several rounds of tiles of 256 x 256 whose last
+        one is filled by GATED_LAST_ROUND where neither 192 nor 224 divides N, at which the library's picks idle (2,048 rows of
+        37888 x 3584 542 / 422, of 22016 x 2048 196 / 151).  The sums meet the activation unrounded, so that it
         is the more exact form as well.  Shapes that were tuned stay with the library (``_tuned_for``)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
                 or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
@@ -370,6 +360,34 @@ class ProductOps:
         fits = (K <= self.GATED_LONG_K and self.GATED_LONG_ROWS[0] <= M <= self.GATED_LONG_ROWS[1] and N % 192 and N % 224
                 and rounds and least * self._num_cus <= last <= most * self._num_cus)
         return 256 if fits else None
+
+    # rows of x a tile -> us of a launch, of a round of tiles, of a chunk of 64 values of k with few CUs busy, and what all of
+    # them add to a chunk (they share the power): fitted to 168 gated products of 12 shapes, 260 to 2,048 rows of x; 3 % rms, 12 % at worst
+    TILE_US = {256: (1.8, 6.0, 0.92, 0.49), 192: (2.5, 4.0, 0.74, 0.39)}
+
+    def _tiles_us(self, rows, M, N, K, ks=1):
+        """Estimated time of a product in tiles of ``rows`` rows of x by 256 of W."""
+        launch, tile, chunk, shared = self.TILE_US[rows]
+        items = -(-N // 256) * -(-M // rows) * ks
+        rounds = -(-items // self._num_cus)
+        return launch + rounds * (tile + K / ks / 64 * (chunk + shared * items / (rounds * self._num_cus)))
+
+    def _tile_rows(self, M, N, K, ks=1):
+        """Rows of x a workgroup takes, the ones that take less time by estimate (of the 168 products 0.04 % slower on
+        average than the better one of both, 2 % at worst)."""
+        return min(self.TILE_US, key=lambda rows: self._tiles_us(rows, M, N, K, ks))
+
+    def _prompt_tiles(self, M, N, K):
+        """Rows of x a tile for a product of a prompt whose results the library would leave to a second pass (a gate or an
+        activation), or None where its product and the pass are the faster pair: where the tiles' estimated rate is below
+        PROMPT_MIN_TFLOPS, which is where they leave CUs idle.  Over the 168 products (rows of 896 to 5,120 values) the
+        kernel at 750 and more takes 0.90 of the pair's time on average, 1.12 at worst (640 x 28672 x 4096, 148 against 141
+        us); at 700 9216 x 3584 with 640 rows of x is among them (56 against 45), at 900 the average is 0.92."""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
+                or N < self.GATED_MIN_N or not self.GATED_MIN_M <= M <= self.GATED_MAX_M or K > self.PROMPT_MAX_K):
+            return None
+        rows = self._tile_rows(M, N, K)
+        return rows if 2e-6 * M * N * K >= self.PROMPT_MIN_TFLOPS * self._tiles_us(rows, M, N, K) else None
 
     def _tuned_for(self, M, N, K) -> bool:
         """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside
@@ -390,12 +408,12 @@ class ProductOps:
         self._check(x, self.act_dtype, (M, K), "x")
         self._check(w, self.act_dtype, (N, K), "weight")
         y = self._new((M, N // 2))
-        self._call("gemm", "sl_gemm_block", _p(x), _p(w), _p(bias), _p(y), M, N, K, 0, int(act), 1, int(rows), None)
+        self._call("gemm", "sl_gemm_block", _p(x), _p(w), _p(bias), _p(y), M, N, K, 0, int(act), 0, 1, int(rows), None)
         return y
 
     def linear_block(self, x, weight, bias, out_f32=False, ks=1, partial=False, square=False):
         """A few hundred rows over the row-major copy of the weight: workgroups
-        own a tile of 256 rows of x by 128 rows of W (``square``: by 256) over
+        own a tile of 256 rows of x by 128 rows of W (``square``: of 256 or 192, ``_tile_rows``, by 256) over
         one of ``ks`` shares of K.  ``partial``: the product comes back as
         ``PartialSums`` for its reader to add up."""
         M, K = x.shape
@@ -405,17 +423,18 @@ class ProductOps:
             raise KernelError("linear_block needs the row-major copy of the weight")
         self._check(x, self.act_dtype, (M, K), "x")
         self._check(w, self.act_dtype, (N, K), "weight")
+        rows = self._tile_rows(M, N, K, ks) if square else 0
         part = self._new((ks, M, N), torch.float32) if ks > 1 or partial else None
         if partial:
             if ks > 1:
-                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, None, M, N, K, 0, 0, int(ks), 256 * int(square),
+                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, None, M, N, K, 0, 0, 0, int(ks), rows,
                            _p(part))
             else:
-                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, _p(part), M, N, K, 1, 0, 1, 256 * int(square), None)
+                self._call("gemm", "sl_gemm_block", _p(x), _p(w), None, _p(part), M, N, K, 1, 0, 0, 1, rows, None)
             return PartialSums(part, bias)
         y = self._new((M, N), torch.float32 if out_f32 else None)
         self._call("gemm", "sl_gemm_block", _p(x), _p(w), _p(bias), _p(y), M, N, K, int(out_f32),
-                   0, int(ks), 256 * int(square), _p(part))
+                   0, 0, int(ks), rows, _p(part))
         return y
 
     def linear_skinny(self, x, weight, bias, out_f32=False):
@@ -509,7 +528,7 @@ class ProductOps:
             y = self._new((M, N // 2))
             self._skinny(x, weight, bias, y, M, N, K, gated=code)
             return y
-        rows = block == self.GATE_BLOCK and self._gated_rows(M, N, K)
+        rows = block == self.GATE_BLOCK and (self._prompt_tiles(M, N, K) or self._gated_rows(M, N, K))
         if rows and not self._tuned_for(M, N, K) and self._block_reads(x, weight):
             return self.linear_gated_block(x, weight, bias, rows, code)
         return self.gate_mul(self.linear(x, weight, bias), block, activation)

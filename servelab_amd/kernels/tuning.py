@@ -101,6 +101,9 @@ class Tuning:
     gated_short_k: int = 1024
     gated_one_round_k: int = 1536
     gated_fill: float = 0.7
+    # ... any rows of up to prompt_max_k values whose tiles are estimated at this rate or more (HipOps._prompt_tiles) ...
+    prompt_max_k: int = 8192
+    prompt_min_tflops: float = 750.0
     # ... longer ones, up to gated_long_k values and for so many rows of x, in several rounds, the last filled so far
     gated_long_k: int = 5120
     gated_long_rows: tuple = (1537, 2048)

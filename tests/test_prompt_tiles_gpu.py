@@ -1,0 +1,67 @@
+"""Products of prompts on workgroups that walk their tiles (gemm_rounds.h), where a workgroup takes several tiles, where a tile is
+one chunk of K, and the activation at values that are not ordinary numbers."""
+import pytest
+import torch
+
+from servelab_amd.kernels import HipOps
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# 261 and 348 tiles on 256 CUs, a number of tiles that eight does not divide, tiles of one, two and three chunks
+@pytest.mark.parametrize("M,N,K", [(700, 22064, 64), (700, 22064, 192), (600, 32800, 128)])
+@pytest.mark.parametrize("rows", [192, 256])
+def test_workgroups_walk_several_tiles(M, N, K, rows):
+    ops = HipOps(torch.bfloat16, DEV)
+    assert -(-M // rows) * -(-N // 256) > ops._num_cus
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    z = x.double() @ w.double().T
+    ops.TILE_US = {rows: ops.TILE_US[rows]}
+    parts = ops.linear_block(x.to(DEV), w.to(DEV), None, ks=1, partial=True, square=True).parts[0]
+    # float sums of K terms: K 2^-24 of their absolute sum
+    bar = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((parts.double().cpu() - z).abs() <= bar).all()
+    half = ops.linear_block(x.to(DEV), w.to(DEV), None, square=True)
+    assert torch.equal(half, parts.bfloat16())
+    pair = z.view(M, N // 16, 2, 8)
+    want = (torch.nn.functional.silu(pair[:, :, 0]) * pair[:, :, 1]).reshape(M, N // 2)
+    got = ops.linear_gated_block(x.to(DEV), ops.prepare_weight(w.to(DEV)), None, rows, 1)
+    # one rounding to bfloat16, and the sums' error in the gate (whose slope is 1.1 at most) and in its up product
+    size = bar.max().item() * 2.2 * z.abs().max().item()
+    assert ((got.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + size).all()
+
+
+def test_gates_that_are_not_ordinary_numbers():
+    ops = HipOps(torch.bfloat16, DEV)
+    inf, nan = float("inf"), float("nan")
+    gates = torch.tensor([inf, -inf, nan, 0.0, -0.0, 1e38, -1e38, 1e-40, -80.0, -87.0, -100.0, 100.0, 20.0, -20.0, 1.0, -1.0])
+    ups = torch.tensor([1.5, -2.0])
+    N = 2 * len(gates) * 16
+    bias = torch.empty(N // 16, 2, 8)
+    bias[:, 0] = gates.repeat(2)[:, None]
+    bias[:, 1] = ups.repeat_interleave(len(gates))[:, None]
+    x, w = torch.zeros(8, 64, device=DEV).bfloat16(), torch.zeros(N, 64, device=DEV).bfloat16()
+    got = ops.linear_gated_block(x, ops.prepare_weight(w), bias.view(-1).to(DEV), 256, 1).view(8, N // 16, 8)[3, :, 5].double().cpu()
+    want = (torch.nn.functional.silu(gates).double()[None] * ups[:, None]).view(-1)
+    assert torch.equal(got.isnan(), want.isnan())
+    keep = ~want.isnan() & want.isfinite()
+    # one rounding to bfloat16; results below the smallest normal float may be zero
+    assert ((got - want).abs()[keep] <= 2.0 ** -8 * want.abs()[keep] + 2.0 ** -125).all()
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+
+
+def test_routes_by_estimated_rate():
+    ops = HipOps(torch.bfloat16, DEV)
+    tiles = ops._prompt_tiles
+    # well filled rounds, in the height that takes less time; part-filled ones stay with the library
+    assert [tiles(M, 37888, 3584) for M in (300, 400, 527, 1000, 2048, 2560)] == [None, 192, 192, 256, 256, 256]
+    assert [tiles(M, 9216, 3584) for M in (640, 900, 1536)] == [None, 192, 256]
+    assert tiles(255, 37888, 3584) is None and tiles(2561, 37888, 3584) is None and tiles(2048, 37888, 3600) is None
+    assert tiles(2048, 4080, 3584) is None and tiles(2048, 37888, 8256) is None
+    # either height gives the same sums
+    x = torch.randn(527, 512, device=DEV).bfloat16()
+    w = (torch.randn(22016, 512, device=DEV) * 0.05).bfloat16()
+    weight = ops.prepare_weight(w)
+    assert torch.equal(ops.linear_gated_block(x, weight, None, 192, 1), ops.linear_gated_block(x, weight, None, 256, 1))
