@@ -1995,7 +1995,8 @@ static void rounds(const __bf16* x, const __bf16* w, const float* bias, void* y,
 // of the float sums; act: y = act(x W^T + bias), bfloat16.
 // ks > 1: `part` holds ks * M * N floats; with y == nullptr they are left
 // there for the reader to add (and the bias with them), else splitk_reduce adds them into y.
-// square: rows of x a tile, 256 or 192, by 256 of W (gemm_rounds.h); 0: tiles of 256 x 128.
+// square: rows of x a tile, 256 or 192, by 256 of W (gemm_rounds.h); 0: tiles of 256 x 128, which take
+// any N and stand in where the others' stores of 16 bytes do not fit.
 extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* bias, void* y,
                                      int M, int N, int K, int out_f32, int gated, int act, int ks, int square, float* part,
                                      hipStream_t stream) {
@@ -2007,7 +2008,9 @@ extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* 
   SL_CHECK(square == 0 || square == 256 || square == 192, "gemm_block: tiles of 256 rows by 128 or 256, or of 192 by 256");
   SL_CHECK(!gated || (square && ks == 1 && !out_f32 && N % 16 == 0),
            "gemm_block: a gated product takes wide tiles, whole rows of K, blocks of eight and bfloat16 results");
-  SL_CHECK(!act || (square && ks == 1 && !out_f32 && !gated), "gemm_block: an activation takes wide tiles, whole rows of K and bfloat16 results");
+  SL_CHECK(!act || (square && ks == 1 && !out_f32 && !gated && N % 8 == 0),
+           "gemm_block: an activation takes wide tiles, whole rows of K, bfloat16 results and columns in eights");
+  if (N % (out_f32 || ks > 1 ? 4 : 8)) square = 0;       // (the wide tiles store 16 bytes at a time; the others any number)
   SL_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_block: x and W must be 16-byte aligned");
   void* dst = ks > 1 ? (void*)part : y;
   const float* b = ks > 1 ? nullptr : bias;

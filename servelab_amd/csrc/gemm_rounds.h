@@ -17,8 +17,8 @@
 //    its slot during the next one; a barrier a half.  Five slots (all of the LDS) gain nothing, nor do four
 //    wavefronts of 128 x 128, which read a third less from the LDS.
 //  - Consecutive products differ in one operand only (2 % of the power).
-//  - The rows of W lie in a tile so that a lane's results are sixteen consecutive columns: 32 bytes a store, and a gate and
-//    its up product are in one lane.
+//  - The rows of W lie in a tile so that four lanes' results are 64 bytes of a row of y in one store of 16 bytes each, and a gate
+//    and its up product are in one lane.
 //  - A workgroup's loads run on over the end of its tile, so the next tile starts without waiting for memory.
 #pragma once
 
@@ -43,7 +43,7 @@ __device__ __forceinline__ float fast_silu(float z) {
   return z * __builtin_amdgcn_rcpf(1.f + fmaf(e, lost * 0.693147181f, e));
 }
 
-enum { ROUNDS_BF16 = 0, ROUNDS_F32 = 1, ROUNDS_GATED = 2 };            // what is written: KIND
+enum { ROUNDS_BF16 = 0, ROUNDS_F32 = 1, ROUNDS_GATED = 2 };            // what is written: KIND; N % 8, 4 and 16 == 0
 
 template <int T, int KIND>
 __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
@@ -84,7 +84,8 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j) {          // row s of half j / 2: tile u of a wavefront's four, row r of the matrix instruction
       const int s = 8 * (wave + 8 * (j & 1)) + (lane >> 3), r = s & 15, u = 2 * (j >> 1) + (s >> 4 & 1);
-      const int n = 64 * (s >> 5) + 16 * (r >> 2) + 4 * u + (r & 3);
+      const int n = 64 * (s >> 5) + (KIND == ROUNDS_GATED ? 16 * (r >> 2) + 4 * u + (r & 3)
+                                     : KIND == ROUNDS_BF16 ? 32 * (u >> 1) + 8 * (r >> 2) + 4 * (u & 1) + (r & 3) : 16 * u + r);
       at_w[j] = (unsigned)(n < last_n ? n : last_n) * (unsigned)(2 * K) + 16 * ((lane & 7) ^ lds_place(s));
     }
   };
@@ -197,9 +198,11 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
       advance();
     }
 
-    // lane: row m of x, sixteen consecutive rows n of W
-    const int lane = lane_here();
-    const int n = n0 + 64 * wn + 16 * (lane >> 4);
+    // lane: row m of x; of tile b the four rows of W from column(b) on
+    const int lane = lane_here(), g = lane >> 4, nw = n0 + 64 * wn;
+    auto column = [&](int b) {
+      return nw + (KIND == ROUNDS_GATED ? 16 * g + 4 * b : KIND == ROUNDS_BF16 ? 32 * (b >> 1) + 8 * g + 4 * (b & 1) : 16 * b + 4 * g);
+    };
 #pragma unroll
     for (int a = 0; a < 2 * T; ++a) {
       const int m = m0 + (a < 2 * T0 ? 32 * T0 * wm + 16 * a : 64 * T0 + 32 * T1 * wm + 16 * (a - 2 * T0)) + (lane & 15);
@@ -211,11 +214,12 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
         if (bias != nullptr) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (n + 4 * b + e < N) r[b][e] += bias[n + 4 * b + e];
+            if (column(b) < N) r[b][e] += bias[column(b) + e];
         }
       }
-      if (m >= M || n >= N) continue;
+      if (m >= M) continue;
       if constexpr (KIND == ROUNDS_GATED) {
+        const int n = column(0);
         bf16x8 h;                          // (gate and up rows lie in blocks of eight: gates first, then their ups)
         if (act == SL_ACT_SILU) {
 #pragma unroll
@@ -224,36 +228,27 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
 #pragma unroll
           for (int e = 0; e < 8; ++e) h[e] = (__bf16)(sl_act(r[e >> 2][e & 3], act) * r[2 + (e >> 2)][e & 3]);
         }
-        *(bf16x8*)((__bf16*)y + (size_t)m * (N / 2) + n / 2) = h;
+        if (n < N) *(bf16x8*)((__bf16*)y + (size_t)m * (N / 2) + n / 2) = h;
       } else if constexpr (KIND == ROUNDS_F32) {
-        float* o = (float*)y + ((size_t)share * M + m) * N + n;
-        if (N % 4 == 0) {
+        float* o = (float*)y + ((size_t)share * M + m) * N;
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            if (n + 4 * q < N) *(f32x4*)(o + 4 * q) = r[q];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            if (n + e < N) o[e] = r[e >> 2][e & 3];
+        for (int b = 0; b < 4; ++b) {
+          const int n = column(b);
+          if (n < N) *(f32x4*)(o + n) = r[b];
         }
       } else {
-        __bf16* o = (__bf16*)y + (size_t)m * N + n;
+        __bf16* o = (__bf16*)y + (size_t)m * N;
         if (act) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) r[e >> 2][e & 3] = sl_act(r[e >> 2][e & 3], act);
         }
-        if (N % 8 == 0 && n + 16 <= N) {
 #pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            bf16x8 h;
+        for (int p = 0; p < 2; ++p) {
+          const int n = column(2 * p);
+          bf16x8 h;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) h[e] = (__bf16)r[2 * q + (e >> 2)][e & 3];
-            *(bf16x8*)(o + 8 * q) = h;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            if (n + e < N) o[e] = (__bf16)r[e >> 2][e & 3];
+          for (int e = 0; e < 8; ++e) h[e] = (__bf16)r[2 * p + (e >> 2)][e & 3];
+          if (n < N) *(bf16x8*)(o + n) = h;
         }
       }
     }

@@ -65,3 +65,38 @@ def test_routes_by_estimated_rate():
     w = (torch.randn(22016, 512, device=DEV) * 0.05).bfloat16()
     weight = ops.prepare_weight(w)
     assert torch.equal(ops.linear_gated_block(x, weight, None, 192, 1), ops.linear_gated_block(x, weight, None, 256, 1))
+
+
+# ragged rows of x and of W, both heights
+@pytest.mark.parametrize("M,N,K,act", [(300, 4112, 128, "relu2"), (257, 1000, 192, "silu"), (385, 264, 64, "gelu_tanh"), (193, 520, 64, "relu")])
+@pytest.mark.parametrize("rows", [192, 256])
+def test_activation_of_the_sums(M, N, K, act, rows):
+    ops = HipOps(torch.bfloat16, DEV)
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    b = torch.randn(N, generator=g)
+    z = x.double() @ w.double().T + b.double()
+    want = {"relu2": lambda t: t.clamp(min=0) ** 2, "relu": lambda t: t.clamp(min=0), "silu": torch.nn.functional.silu,
+            "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}[act](z)
+    code = {"silu": 1, "relu": 2, "relu2": 3, "gelu_tanh": 4}[act]
+    weight = ops.prepare_weight(w.to(DEV))
+    got = ops.linear_activated_block(x.to(DEV), weight, b.to(DEV), rows, code)
+    # one rounding to bfloat16; float sums of K terms: K 2^-24 of their absolute sum, times the activation's slope there
+    size = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + b.double().abs())
+    slope = 2 * z.abs() + size if act == "relu2" else 1.2
+    assert ((got.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + slope * size + 2.0 ** -20).all()
+
+
+def test_activated_prompts_take_the_tiles():
+    ops = HipOps(torch.bfloat16, DEV)
+    w = (torch.randn(18944, 256, device=DEV) * 0.06).bfloat16()
+    weight = ops.prepare_weight(w)
+    x = torch.randn(1852, 256, device=DEV).bfloat16()
+    ops.PROMPT_MIN_TFLOPS = 100.0                # (short rows: an estimated rate of 480 TFLOP/s)
+    assert ops._prompt_tiles(1852, 18944, 256)
+    got = ops.activated_linear(x, weight, "relu2")
+    assert torch.equal(got, ops.linear_activated_block(x, weight, None, 256, 3))
+    odd = torch.empty(x.numel() + 1, device=DEV, dtype=x.dtype)[1:].view(x.shape).copy_(x)
+    plain = ops.activated_linear(odd, weight, "relu2")
+    # (the library's product is rounded before the square as well)
+    assert ((plain.float() - got.float()).abs() <= 2.0 ** -6 * got.float().abs() + 2.0 ** -12).all()
