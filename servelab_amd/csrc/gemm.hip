@@ -930,16 +930,6 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
   }
 }
 
-// CUs of the current device (asked once per device).
-static int device_cus() {
-  static int cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cus[dev] == 0 &&
-      hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  return cus[dev];
-}
-
 // wt: W in the tiled layout, ceil(N / 16) * 16 rows (rows beyond N are zero).
 // At most 16 rows.  Fusion: in_parts != nullptr makes x un-normalised rows
 // (consumer), resid != nullptr makes the result a delta of the stream (producer).

@@ -22,27 +22,11 @@
 //  - A workgroup's loads run on over the end of its tile, so the next tile starts without waiting for memory.
 #pragma once
 
-// the lane's number, worked out where it stands: kept in no register through the loop, which has none to spare
-__device__ __forceinline__ int lane_here() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
-  return l;
-}
 __device__ __forceinline__ const __bf16* same_in_all_lanes(const __bf16* p) {
   const unsigned long long v = (unsigned long long)p;
   const unsigned long long hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32));
   return (const __bf16*)((hi << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)v));
 }
-// z sigmoid(z) on the exponential unit: 2^t with what t lost in its rounding put back, so that the error stays a few units
-// in the last place at any z; the whole tile's activation takes 4 us instead of 7 through expf and a division
-__device__ __forceinline__ float fast_silu(float z) {
-  const float x = __builtin_amdgcn_fmed3f(-z, -126.f, 126.f);          // (finite: an infinite z gives z * 1 or z * 0)
-  const float t = x * 1.44269504088896341f;
-  const float lost = fmaf(x, 1.44269504088896341f, -t);
-  const float e = __builtin_amdgcn_exp2f(t);
-  return z * __builtin_amdgcn_rcpf(1.f + fmaf(e, lost * 0.693147181f, e));
-}
-
 enum { ROUNDS_BF16 = 0, ROUNDS_F32 = 1, ROUNDS_GATED = 2 };            // what is written: KIND; N % 8, 4 and 16 == 0
 
 template <int T, int KIND>

@@ -18,3 +18,9 @@ template <int N_> __device__ __forceinline__ void wait_loads() {
 // lanes that read unit c of rows r .. r + 15 touch 16 different 16-byte slots of a 256-byte line of banks, and each half of
 // them 8 different slots of a 128-byte one.
 __device__ __forceinline__ int lds_place(int r) { return ((r >> 1) & 7) ^ (4 * (r & 1)); }
+// The lane's number, worked out where it stands: kept in no register through a loop that has none to spare.
+__device__ __forceinline__ int lane_here() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+  return l;
+}

@@ -22,7 +22,7 @@
 #include "common.h"
 #include "lds_loads.h"
 
-#define RT_ROWS 16           // rows of a tile of the plain grouped product; a row tile holds 16 or 128 rows
+#define RT_ROWS 16           // rows of a tile of the plain grouped product; a row tile holds 16, 128 or 256 rows
 
 // ------------------------------------------------------------------ route
 // One wavefront per token; lane k < top gets the expert of the k-th choice.  Largest first; among equal logits the lower
@@ -225,7 +225,7 @@ extern "C" const char* sl_route_tokens(const float* logits, int stride, int T, i
            "route_tokens: at most 4096 experts within the rows, at most 64 choices");
   SL_CHECK(E_real >= 0 && E_real <= E && (over_all || correction == nullptr),
            "route_tokens: the experts with matrices are the first of all; a correction needs shares over all");
-  SL_CHECK(tile_rows == 16 || tile_rows == 128, "route_tokens: row tiles hold 16 or 128 rows");
+  SL_CHECK(tile_rows == 16 || tile_rows == 128 || tile_rows == 256, "route_tokens: row tiles hold 16, 128 or 256 rows");
   SL_CHECK(max_tiles >= ((long long)T * top + tile_rows - 1) / tile_rows + E, "route_tokens: too few tile entries");
   if (T == 0) return nullptr;
   const Route r{logits, stride, E, top, chosen, shares, over_all, correction, scale, sigmoid};
@@ -273,18 +273,10 @@ __device__ __forceinline__ bool grouped_place(const Grouped& a, int& tile, int& 
   return true;
 }
 
-// The same for row tiles of 128 rows: only the tiles in use, and every column block of a tile before the next tile.  A die
+// Row tiles of 128 rows instead take only the tiles in use, and every column block of a tile before the next tile.  A die
 // then reads a tile's rows of x once for all of its columns, and has two or three experts' matrices under way (64 experts of
 // 2,048 x 1,024, gate/up, down and the sum, 8 of them a token: 256 / 1,000 / 2,048 tokens 196 / 254 / 360 us by column
 // blocks, 162 / 231 / 359 by tiles).
-__device__ __forceinline__ bool grouped_place_by_rows(const Grouped& a, int& tile, int& cb) {
-  const int total = (a.used != nullptr ? min(*a.used, a.max_tiles) : a.max_tiles) * a.col_blocks, run = (total + 7) / 8;
-  const int m = (blockIdx.x & 7) * run + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= run || m >= total) return false;
-  tile = m / a.col_blocks;
-  cb = m - tile * a.col_blocks;
-  return true;
-}
 
 // 256 threads: thread (row = tid / 16, lane16 = tid % 16) owns columns lane16 + 16 u, u < 4, of a
 // 16 x 64 tile.  x and W go through LDS in chunks of 32 values of k; sums are float.
@@ -531,129 +523,245 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void grouped_product_few_kernel(con
 }
 
 
-// Row tiles of 128 rows, both operands through LDS: a workgroup of eight wavefronts takes a row tile by 256 rows of W (256
-// columns, or 128 of the gate and the same 128 of the up matrix), a wavefront 64 by 64 of it.  Prompts with a few
-// hundred rows an expert sit where the stream of the matrices and the matrix units cost about the same, so what counts is
-// that enough of both is asked for ahead: chunks of 64 values of k go straight into a ring of three LDS stages (48 KB
-// each, the rows of x as lds_place says, W as its tiles lie in memory: what a wavefront reads of a tile is 1 KB in a row),
-// two chunks under way while the third is multiplied.  Blocks of 16 rows that hold no pair are not multiplied.
-// (64 experts of 2,048 x 1,024, gate/up, down and the sum, 8 of them a token: 256 / 1,000 / 2,048 tokens 174 / 285 / 401 us
-// with x staged through registers and W a step of 32 ahead of its use, 162 / 231 / 359 here.  Chunks of 32 values of k and two
-// workgroups a CU do not fit the registers: 310 / 484 / 635.)
-template <bool GATED>
-__global__ __launch_bounds__(512) void grouped_product_staged_kernel(const Grouped a) {
-  constexpr int STAGES = 3, X_BYTES = 128 * 128, STAGE_BYTES = X_BYTES + 256 * 128, LOADS = STAGE_BYTES / 1024 / 8;
-  __shared__ __attribute__((aligned(1024))) char ring[STAGES * STAGE_BYTES];
-  int tile, cb;
-  if (!grouped_place_by_rows(a, tile, cb)) return;
-  const int* tl = a.tiles + 3 * tile;
-  const int rows = min(128, tl[2]);
-  if (rows <= 0) return;                                // (the whole workgroup: no barrier is left waiting)
-  const int e = tl[0], row0 = tl[1];
-  const int lane = threadIdx.x & 63, i = lane & 15, gq = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 2, wn = wave & 3;
-  const int n0 = cb * (GATED ? 128 : 256);
-  const __bf16* we = a.w + (size_t)e * (GATED ? 2 * (size_t)a.N : (size_t)a.N) * a.K;
-  // Tile t of 16 rows of W (four a column of wavefronts): the wavefront's columns, or its gate's, then its up's
-  auto column = [&](int t) { return GATED ? n0 + 16 * (2 * (t >> 2) + (t & 1)) : n0 + 16 * t; };
-  // what this lane brings of every chunk: two pieces of 8 rows of x, four pieces (32 values of k) of W's tiles
-  const char* src[LOADS];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = 8 * (wave + 8 * j) + (lane >> 3), rr = row0 + min(r, rows - 1);
-    const size_t from = a.order != nullptr ? (size_t)(a.order[rr] / a.top) : (size_t)rr;
-    src[j] = (const char*)(a.x + from * a.K + 8 * ((lane & 7) ^ lds_place(r)));
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int piece = wave + 8 * j, t = piece >> 1;
-    const __bf16* m = we + (GATED && (t & 2) ? (size_t)a.N * a.K : 0);
-    src[2 + j] = (const char*)(m + ((size_t)(min(column(t), a.N - 16) / 16) * (a.K / 32) + (piece & 1)) * 512 + lane * 8);
-  }
-  const unsigned ring_at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
-  auto fetch = [&](int c, int stage) {
-    const unsigned at = ring_at + STAGE_BYTES * stage + 1024 * wave;
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j)
-      load_to_lds(src[j] + (size_t)c * (j < 2 ? 128 : 2048), at + 8192 * j);
-  };
-  int at_kk[2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk) at_kk[kk] = 128 * (64 * wm + i) + 16 * ((4 * kk + gq) ^ lds_place(i));
-  const int blocks = min(4, (rows - 64 * wm + 15) / 16);         // of 16 rows with a pair (none: zero or less)
-
-  rt_f32x4 acc[4][4];                                   // [tile of W][block of rows]
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[u][v] = rt_f32x4{0.f, 0.f, 0.f, 0.f};
+// Row tiles of R = 128 or 256 rows, both operands through LDS: eight wavefronts take a row tile by 256 rows of W (256
+// columns, or 128 of the gate and the same 128 of the up matrix), a wavefront R / 2 by 64 of it, and walk their (row tile, column
+// block) items, at most a workgroup a CU.  As in the products of whole prompts (gemm_rounds.h) a chunk of 64 values of k is
+// two halves, R / 2 rows of x and half of W each; a half's operands are read into registers while the one before it is multiplied,
+// in an order laid down instruction by instruction, and six halves of 24 KB, or four of 32, are on the way in the ring.  What
+// bounds it at 128 rows is that ring: the matrices come from memory, two microseconds away, and three chunks of 512 ns of matrix
+// work ahead do not cover that (about 1.1 us a chunk whatever the order of the items; a chunk of 256 rows takes 1.3).
+// The trips that start an item (its row tile, where its rows lie, the rows) are as long as several chunks, so a workgroup
+// looks up BATCH items ahead and its loads run on from one item into the next.
+// A prompt of 2,048 tokens, 8 of 64 experts of 1,024 over rows of 2,048 a token: gate/up 229 -> 176 us, down 134 -> 111 (of which
+// its 134 MB of float rows and 268 MB of matrices are 70), against an item a workgroup, 128 rows each, and a ring of three whole chunks
+// behind one barrier; 128 rows walked like this: 196 and 118.
+// Halves of the rows without a pair are not multiplied.  HALF: results in bfloat16, and the rows of W are picked from two tiles
+// so that a lane holds eight columns in a row; odd tiles lie in LDS with their rows four places on, off the other's banks.
+template <int R, bool GATED, bool HALF>
+__global__ __launch_bounds__(512, 2) void grouped_product_walk_kernel(const Grouped a) {
+  constexpr int X_BYTES = 64 * R, SLOT = X_BYTES + 16384, SLOTS = R == 128 ? 6 : 4, BATCH = 12;
+  constexpr int XL = R / 128, LOADS = XL + 2;            // loads of 64 rows a half holds, a wavefront's loads of a half
+  constexpr int XT = R / 64;                            // a wavefront's tiles of 16 rows in a half
+  static_assert(R == 128 || R == 256, "row tiles of 128 or 256 rows");
+  __shared__ __attribute__((aligned(1024))) char ring[SLOTS * SLOT];
+  __shared__ int from[BATCH][R];                      // of an item's rows: the row of x
+  __shared__ float scale[BATCH][R];                   // and the factor of its sums
+  __shared__ int what[BATCH][4];                        // expert, first row, rows, column block
+  __shared__ int found;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wm = wave >> 2, wn = wave & 3;
+  // (every column block of a tile before the next tile; a die's items are a contiguous run, a workgroup takes every `step`-th of them)
+  const int total = (a.used != nullptr ? min(*a.used, a.max_tiles) : a.max_tiles) * a.col_blocks, run = (total + 7) / 8;
+  const int first = (int)(blockIdx.x & 7) * run, end = min(first + run, total), step = (int)gridDim.x >> 3;
   const int chunks = a.K / 64;
-  fetch(0, 0);
-  if (chunks > 1) {
-    fetch(1, 1);
-    wait_loads<LOADS>();
-  } else {
-    wait_loads<0>();
+  const unsigned ring_at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring + 1024 * wave;
+  int at_x[2], at_wt;                                   // where this lane reads its operands in a slot
+  {
+    const int lane = threadIdx.x & 63, i = lane & 15, gq = lane >> 4;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) at_x[kk] = 128 * (16 * XT * wm + i) + 16 * ((4 * kk + gq) ^ lds_place(i));
+    const int odd = HALF ? i >> 3 : 0, row = HALF ? (8 * (i >> 2 & 1) + (i & 3)) ^ (4 * odd) : i;
+    at_wt = X_BYTES + 2048 * (2 * wn + odd) + 16 * (16 * gq + row);
   }
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" : : : "memory");
-  int stage = 0;
-  for (int c = 0; c < chunks; ++c) {
-    const bool more = c + 2 < chunks;
-    if (more) fetch(c + 2, stage >= 1 ? stage - 1 : 2);          // the stage the last chunk was read from
-    const char* st = ring + STAGE_BYTES * stage;
-    auto multiply = [&](auto all) {
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        rt_bf16x8 w[4], x[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) w[u] = *(const rt_bf16x8*)(st + X_BYTES + 1024 * (2 * (4 * wn + u) + kk) + 16 * lane);
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          if (all || v < blocks) x[v] = *(const rt_bf16x8*)(st + 128 * 16 * v + at_kk[kk]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          if (all || v < blocks) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[v], acc[u][v], 0, 0, 0);
-          }
-      }
-    };
-    if (blocks == 4) multiply(std::true_type{});
-    else if (blocks > 0) multiply(std::false_type{});
-    if (more) wait_loads<LOADS>();                      // all but the chunk just asked for
-    else wait_loads<0>();
+  auto operand = [&](int at) { return *(const rt_bf16x8*)(ring + at); };
+  auto w_at = [&](int b, int kk) { return HALF ? (at_wt ^ (64 * b)) + 1024 * kk : at_wt + 2048 * b + 1024 * kk; };
+  auto barrier = [&]() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" : : : "memory");
-    stage = stage == 2 ? 0 : stage + 1;
-  }
-  // this lane holds columns 4 gq .. + 3 of each tile of W, of rows 64 wm + 16 v + i
+  };
+  auto next = [&](unsigned at) { return at == SLOT * (SLOTS - 1) ? 0u : at + SLOT; };
+
+  for (int base = first + (int)(blockIdx.x >> 3); base < end; base += BATCH * step) {
+    if (wave == 0) {                                    // the next items that have rows
+      const int lane = threadIdx.x & 63, it = base + lane * step;
+      int e = 0, row0 = 0, rows = 0, cb = 0;
+      if (lane < BATCH && it < end) {
+        const int tile = it / a.col_blocks;
+        cb = it - tile * a.col_blocks;
+        e = a.tiles[3 * tile], row0 = a.tiles[3 * tile + 1], rows = min(R, a.tiles[3 * tile + 2]);
+      }
+      const unsigned long long live = __ballot(rows > 0);
+      if (rows > 0) {
+        const int p = __popcll(live & ((1ull << lane) - 1));
+        what[p][0] = e, what[p][1] = row0, what[p][2] = rows, what[p][3] = cb;
+      }
+      if (lane == 0) found = __popcll(live);
+    }
+    __syncthreads();
+    const int items = __builtin_amdgcn_readfirstlane(found);
+    for (int q = threadIdx.x; q < items * R; q += 512) {
+      const int k = q / R, r = q % R, rr = what[k][1] + min(r, what[k][2] - 1);
+      const int pair = a.order != nullptr ? a.order[rr] : rr;
+      from[k][r] = a.order != nullptr ? pair / a.top : rr;
+      scale[k][r] = a.row_scale != nullptr ? a.row_scale[pair] : 1.f;
+    }
+    __syncthreads();
+    if (items == 0) continue;
+
+    int load_item = 0, load_left;
+    const __bf16 *load_x, *load_w;
+    unsigned from_x[2 * XL], from_w[4];                 // of each half
+    auto open = [&](int k) {
+      const int lane = lane_here();
+      const int e = __builtin_amdgcn_readfirstlane(what[k][0]), cb = __builtin_amdgcn_readfirstlane(what[k][3]);
+      const int n0 = cb * (GATED ? 128 : 256);
+      load_left = chunks;
+      load_x = a.x;
+      load_w = a.w + (size_t)e * (GATED ? 2 * (size_t)a.N : (size_t)a.N) * a.K;
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = 64 * wm + 16 * v + i;
-    if (r >= rows) continue;
-    const float rs = a.row_scale != nullptr ? a.row_scale[a.order[row0 + r]] : 1.f;
-    const size_t at = (size_t)(row0 + r) * a.N + 4 * gq;
+      for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int u = 0; u < (GATED ? 2 : 4); ++u) {
-      const int n = column(4 * wn + u);
-      if (n >= a.N) continue;
-      const rt_f32x4 z = a.row_scale != nullptr ? acc[u][v] * rs : acc[u][v];
-      if (GATED) {
-        const rt_f32x4 up = a.row_scale != nullptr ? acc[2 + u][v] * rs : acc[2 + u][v];
-        rt_bf16x4 h;
+        for (int j = 0; j < XL; ++j) {
+          const int r = 64 * j + 8 * wave + (lane >> 3);
+          from_x[XL * h + j] = (unsigned)from[k][R / 2 * h + r] * (unsigned)(2 * a.K) + 16 * ((lane & 7) ^ lds_place(r));
+        }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) h[c] = (__bf16)sl_gated(z[c], up[c], a.act, a.limit);
-        *(rt_bf16x4*)(a.out_act + at + n) = h;
-      } else if (a.act) {
-        rt_bf16x4 h;
+        for (int j = 0; j < 2; ++j) {                   // 1 KB: a tile of 16 rows of W by 32 of k, tiles 2 h and 2 h + 1 of each wn
+          const int piece = wave + 8 * j, t = piece >> 1;
+          const int col = GATED ? n0 + 32 * (t >> 1) + 16 * (t & 1) : n0 + 64 * (t >> 1) + 32 * h + 16 * (t & 1);
+          from_w[2 * h + j] = ((unsigned)(min(col, a.N - 16) / 16) * (unsigned)(a.K / 32) + (piece & 1)) * 1024u
+                              + 16 * (HALF && (t & 1) ? lane ^ 4 : lane) + (GATED && h ? 2u * (unsigned)a.N * (unsigned)a.K : 0u);
+        }
+      }
+    };
+    auto load = [&](int h, int j, unsigned slot) {
+      if (j < XL) load_to_lds(from_x[XL * h + j], load_x, ring_at + slot + 8192 * j);
+      else load_to_lds(from_w[2 * h + j - XL], load_w, ring_at + slot + X_BYTES + 8192 * (j - XL));
+    };
+    auto advance = [&]() {
+      if (--load_left > 0) {
+        load_x += 64;
+        load_w += 1024;
+      } else if (load_item + 1 < items) {
+        open(++load_item);
+      }                                                 // (past the last chunk: that one again, which nothing reads)
+    };
+    open(0);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) h[c] = (__bf16)sl_act(z[c], a.act);
-        *(rt_bf16x4*)(a.out_act + at + n) = h;
+    for (int s = 0; s < SLOTS; ++s) {
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) load(s & 1, j, SLOT * s);
+      if (s & 1) advance();
+    }
+    rt_bf16x8 x0[XT][2], x1[XT][2], w0[2][2], w1[2][2]; // [tile of 16 rows][k-step of 32]
+    rt_f32x4 acc[2 * XT][4];                            // [tile of 16 rows, of the first half, then the second][tile of W]
+#pragma unroll
+    for (int v = 0; v < 2 * XT; ++v)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[v][u] = rt_f32x4{0.f, 0.f, 0.f, 0.f};
+    wait_loads<LOADS * (SLOTS - 1)>();
+    barrier();
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) w0[b][kk] = operand(w_at(b, kk));
+#pragma unroll
+      for (int v = 0; v < XT; ++v) x0[v][kk] = operand(at_x[kk] + 2048 * v);
+    }
+    asm volatile("" : : : "memory");
+    wait_loads<LOADS * (SLOTS - 2)>();
+    barrier();
+    int read_at = SLOT;                                 // slot of the half that is read next
+    unsigned load_at = 0;                               // slot of the half that is loaded next: the one read before
+
+    for (int item = 0; item < items; ++item) {
+      const int rows = __builtin_amdgcn_readfirstlane(what[item][2]);
+      auto chunk = [&](auto both) {                     // (a loop of its own for each: the registers do not reach for one that branches)
+        // the first half of the rows; W's second half and the other rows arrive in registers
+        constexpr int P = 8 * XT, R0 = 4 + 2 * XT;      // products, reads
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+#pragma unroll
+          for (int r = 0; r < R0; ++r) {
+            if (r * (P * 3 / 4) / R0 != p) continue;
+            const int q = r < 4 ? 0 : r - 4;
+            if (r < 4) w1[r & 1][r >> 1] = operand(w_at(r & 1, r >> 1) + read_at);
+            else x1[q % XT][q / XT] = operand(at_x[q / XT] + read_at + 2048 * (q % XT));
+          }
+#pragma unroll
+          for (int j = 0; j < LOADS; ++j)
+            if (j * P / LOADS == p) load(0, j, load_at);
+          const int h = p / (4 * XT), j = p % (4 * XT), kk = j / (2 * XT), v = j / 2 % XT, b = (j ^ v) & 1;
+          acc[v][2 * h + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h ? w1[b][kk] : w0[b][kk], x0[v][kk], acc[v][2 * h + b], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("" : : : "memory");
+        wait_loads<LOADS * (SLOTS - 2)>();                  // the half that is read next is there
+        barrier();
+        read_at = (int)next(read_at);
+        load_at = next(load_at);
+        // the other rows; the first halves of the next chunk arrive
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+#pragma unroll
+          for (int r = 0; r < 2 * XT; ++r)
+            if (r * (P / 2) / (2 * XT) == p) x0[r % XT][r / XT] = operand(at_x[r / XT] + read_at + 2048 * (r % XT));
+#pragma unroll
+          for (int r = 0; r < 4; ++r)                 // (their first half's products are done)
+            if (P / 2 + r * (P / 4) / 4 == p) w0[r & 1][r >> 1] = operand(w_at(r & 1, r >> 1) + read_at);
+#pragma unroll
+          for (int j = 0; j < LOADS; ++j)
+            if (j * P / LOADS == p) load(1, j, load_at);
+          const int h = p / (4 * XT), j = p % (4 * XT), kk = j / (2 * XT), v = j / 2 % XT, b = (j ^ v) & 1;
+          if (decltype(both)::value)
+            acc[XT + v][2 * h + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h ? w1[b][kk] : w0[b][kk], x1[v][kk], acc[XT + v][2 * h + b], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("" : : : "memory");
+        wait_loads<LOADS * (SLOTS - 2)>();
+        barrier();
+        read_at = (int)next(read_at);
+        load_at = next(load_at);
+        advance();
+      };
+      if (rows > R / 2) {
+        for (int c = 0; c < chunks; ++c) chunk(std::true_type{});
       } else {
-        *(rt_f32x4*)(a.out_f32 + at + n) = z;
+        for (int c = 0; c < chunks; ++c) chunk(std::false_type{});
+      }
+      // this lane: row i of a tile of rows; of W rows 4 gq .. + 3 of each tile, or (HALF) 8 gq .. + 7 of each two
+      const int lane = lane_here(), i = lane & 15, gq = lane >> 4, row0 = __builtin_amdgcn_readfirstlane(what[item][1]);
+      const int n0 = __builtin_amdgcn_readfirstlane(what[item][3]) * (GATED ? 128 : 256);
+#pragma unroll
+      for (int v = 0; v < 2 * XT; ++v) {
+        const int r = R / 2 * (v / XT) + 16 * XT * wm + 16 * (v % XT) + i;
+        const float rs = scale[item][r];
+        const size_t at = (size_t)(row0 + r) * a.N;
+        rt_f32x4 z[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          z[u] = acc[v][u] * rs;
+          acc[v][u] = rt_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (r >= rows) continue;
+        if constexpr (GATED) {
+          const int n = n0 + 32 * wn + 8 * gq;
+          rt_bf16x8 h;
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            const float g = z[c >> 2][c & 3], up = z[2 + (c >> 2)][c & 3];
+            h[c] = (__bf16)sl_gated(g, up, a.act, a.limit);
+          }
+          if (n < a.N) *(rt_bf16x8*)(a.out_act + at + n) = h;
+        } else if constexpr (HALF) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const int n = n0 + 64 * wn + 32 * q + 8 * gq;
+            rt_bf16x8 h;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) h[c] = (__bf16)sl_act(z[2 * q + (c >> 2)][c & 3], a.act);
+            if (n < a.N) *(rt_bf16x8*)(a.out_act + at + n) = h;
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int n = n0 + 64 * wn + 16 * u + 4 * gq;
+            if (n < a.N) *(rt_f32x4*)(a.out_f32 + at + n) = z[u];
+          }
+        }
       }
     }
+    wait_loads<0>();                                    // (loads past the last chunk still land in the ring)
+    __syncthreads();
   }
 }
 #endif
@@ -667,7 +775,7 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
   SL_CHECK(act >= 0 && act <= SL_ACT_CLAMPED_SWISH && (!gated || act) && (gated || act != SL_ACT_CLAMPED_SWISH),
            "grouped_product: unknown activation, a gate without one, or the clamped form without a gate");
   SL_CHECK(row_scale == nullptr || order != nullptr, "grouped_product: factors per row go with the pairs' order");
-  SL_CHECK(tile_rows == 16 || tile_rows == 128, "grouped_product: row tiles hold 16 or 128 rows");
+  SL_CHECK(tile_rows == 16 || tile_rows == 128 || tile_rows == 256, "grouped_product: row tiles hold 16, 128 or 256 rows");
   SL_CHECK(pairs >= 0 && experts >= 0, "grouped_product: sizes must be positive");
   if (max_tiles == 0 || pairs == 0) return nullptr;
   if (used != nullptr) max_tiles = min(max_tiles, pairs);         // (the tiles in use come first, and each holds a pair)
@@ -680,9 +788,24 @@ extern "C" const char* sl_grouped_product(const void* x, const int* order, int t
       a.col_blocks = (N + cols - 1) / cols;
       return dim3(8 * (unsigned)((max_tiles * a.col_blocks + 7) / 8));
     };
-    if (tile_rows == 128 && w_tiled && K % 64 == 0) {   // the tile's rows of x staged in LDS
-      if (gated) grouped_product_staged_kernel<true><<<blocks(128), 512, 0, stream>>>(a);
-      else grouped_product_staged_kernel<false><<<blocks(256), 512, 0, stream>>>(a);
+    const unsigned long long rows = order != nullptr ? pairs / top : pairs;
+    if (tile_rows >= 128 && w_tiled && K % 64 == 0 && rows * K < (1ull << 31) && (gated ? 2ull : 1ull) * N * K < (1ull << 31)) {
+      // (operands' offsets in 32 bits)
+      const int cus = device_cus() & ~7;
+      dim3 grid = blocks(gated ? 128 : 256);
+      if (cus >= 8 && grid.x > (unsigned)cus) grid.x = cus;
+      if (tile_rows == 128) {
+        if (gated) grouped_product_walk_kernel<128, true, true><<<grid, 512, 0, stream>>>(a);
+        else if (act) grouped_product_walk_kernel<128, false, true><<<grid, 512, 0, stream>>>(a);
+        else grouped_product_walk_kernel<128, false, false><<<grid, 512, 0, stream>>>(a);
+      } else {
+        if (gated) grouped_product_walk_kernel<256, true, true><<<grid, 512, 0, stream>>>(a);
+        else if (act) grouped_product_walk_kernel<256, false, true><<<grid, 512, 0, stream>>>(a);
+        else grouped_product_walk_kernel<256, false, false><<<grid, 512, 0, stream>>>(a);
+      }
+    } else if (tile_rows == 256) {                      // four wavefronts along the rows
+      if (gated) grouped_product_mfma_kernel<4, 4, true, 4, 1><<<blocks(64), 256, 0, stream>>>(a);
+      else grouped_product_mfma_kernel<4, 4, false, 4, 1><<<blocks(64), 256, 0, stream>>>(a);
     } else if (tile_rows == 128) {                      // two wavefronts along the rows, two along the columns
       if (gated) grouped_product_mfma_kernel<4, 4, true, 2, 2><<<blocks(128), 256, 0, stream>>>(a);
       else grouped_product_mfma_kernel<4, 4, false, 2, 2><<<blocks(128), 256, 0, stream>>>(a);

@@ -17,7 +17,7 @@ _ll = ctypes.c_longlong
 
 _EXPAND_MODES = {"plain": 0, "log_sigmoid": 1, "rate_softplus": 2, "softplus": 3}
 _SCAN_DECAY, _SCAN_DELTA, _SCAN_LSTM, _SCAN_SSD, _SCAN_FORGET, _SCAN_DELTA_HEAD = 0, 1, 2, 3, 4, 5
-_TILE_ROWS = (16, 128)    # rows of a row tile of the grouped products (routed.hip)
+_TILE_ROWS = (16, 128, 256)    # rows of a row tile of the grouped products (routed.hip)
 
 
 class Routing(NamedTuple):
@@ -72,6 +72,12 @@ class RecurrentOps:
     # 262 in tiles of 16, 214 / 223 / 255 in tiles of 128; 8 of 4,128 x 1,056, 12 rows 122 and 169)
     ROUTED_WIDE_TILE_ROWS, ROUTED_WIDE_TILE_ROWS_OF_FEW, ROUTED_WIDE_EXPERTS = 12, 96, 8
     ROUTED_WIDE_TILE_ROWS_ODD, ROUTED_WIDE_WORKGROUPS = 48, 64
+    # ... and from which they hold 256, where such tiles, as many as the average expert needs, make ROUTED_TALL_WORKGROUPS items
+    # of the first product (two rounds of 256 CUs): a matrix is then read for twice the rows (gate/up, down and the sum in tiles of
+    # 128 / 256 rows: 64 experts of 2,048 x 1,024, 62 / 125 / 200 / 256 / 512 rows each 167 / 172, 216 / 199, 256 / 236, 337 / 319
+    # and 586 / 576 us; of 3,584 x 1,792 490 / 503, 629 / 575, 794 / 678, 946 / 912 and 1,626 / 1,411; 8 of 2,048 x 4,096, 125 /
+    # 250 / 325 / 400 / 512 rows, the first three one round, 144 / 149, 191 / 207, 211 / 218, 248 / 234 and 317 / 272)
+    ROUTED_TALL_TILE_ROWS, ROUTED_TALL_WORKGROUPS = 100, 512
 
     # ------------------------------------------------- norm on an output
     def add_postnorm(self, resid, y, weight, eps, mult, want_rows=True):
@@ -437,7 +443,11 @@ class RecurrentOps:
         few = experts < self.ROUTED_WIDE_EXPERTS or experts * blocks < self.ROUTED_WIDE_WORKGROUPS
         line = self.ROUTED_WIDE_TILE_ROWS_OF_FEW if few else \
             (self.ROUTED_WIDE_TILE_ROWS if K % 64 == 0 else self.ROUTED_WIDE_TILE_ROWS_ODD)
-        return _TILE_ROWS[int(pairs >= line * experts and self.act_dtype == torch.bfloat16)]
+        wide = pairs >= line * experts and self.act_dtype == torch.bfloat16
+        if (wide and pairs >= self.ROUTED_TALL_TILE_ROWS * experts and getattr(w_gate_up, "tiled", False) and K % 64 == 0
+                and experts * blocks * -(-pairs // (256 * experts)) >= self.ROUTED_TALL_WORKGROUPS):
+            return _TILE_ROWS[2]
+        return _TILE_ROWS[int(wide)]
 
     def route_tokens(self, logits, experts, top, over_all=False, correction=None, scale=1.0, with_matrices=None,
                      sigmoid=False, tile_rows=None):

@@ -163,3 +163,49 @@ def test_tiles_asked_for_by_the_matrices():
     got, want = (hip.routed_experts(x, v, first, down).float() for v in (r, wide))
     # (as above)
     assert (got - want).abs().max() <= 3 * 2.0 ** -8 * want.abs().max()
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("gated,act", [(True, "silu"), (False, "relu2")])
+def test_workgroups_that_walk_more_items_than_they_look_up(gated, act, rows):
+    """Tiles of 128 and 256 rows: 104 row tiles (of 128) of 32 column blocks, of which a workgroup of 256 looks up twelve at a time; an
+    expert without rows, one with a single row and one with half a tile among them."""
+    hip = HipOps(torch.bfloat16, DEV)
+    E, ff, K = 6, 4096 if gated else 8192, 64
+    g = torch.Generator().manual_seed(3)
+    counts = [6400, 0, 1, 64, 6399, 300] if rows == 128 else [12800, 0, 1, 128, 12799, 600]
+    chosen = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(sum(counts), generator=g)].view(-1, 1)
+    T = chosen.shape[0]
+    logits = torch.full((T, E), -30.0).scatter_(1, chosen, 5.0)
+    x = torch.randn(T, K, generator=g).bfloat16()
+    w1 = (torch.randn(E, 2 * ff if gated else ff, K, generator=g) * K ** -0.5).bfloat16()
+    w2 = (torch.randn(E, K, ff, generator=g) * ff ** -0.5).bfloat16()
+    first, second = hip.prepare_expert_matrices(w1.to(DEV), gated), hip.prepare_expert_matrices(w2.to(DEV))
+    r = hip.route_tokens(logits.to(DEV), E, 1, tile_rows=rows)
+    assert r.tiles_in_use.item() * (ff // 128 if gated else ff // 256) > 12 * hip._num_cus
+    got = hip.routed_experts(x.to(DEV), r, first, second, activation=act, gated=gated).float().cpu()
+    for e in range(E):
+        at = (chosen[:, 0] == e).nonzero()[:, 0]
+        z = x[at].double() @ w1[e].double().T
+        h = torch.nn.functional.silu(z[:, :ff]) * z[:, ff:] if gated else z.clamp(min=0) ** 2
+        want = h @ w2[e].double().T
+        # what lies between the products and the result are rounded to bfloat16: 2^-9 of a value each, the first as often as it is added
+        bar = 2.0 ** -8 * want.abs() + 2.0 ** -8 * (h.abs() @ w2[e].double().abs().T)
+        assert ((got[at].double() - want).abs() <= bar).all(), e
+
+
+@pytest.mark.parametrize("T,E,top,ff,K", [(400, 3, 2, 128, 64), (700, 2, 1, 272, 192), (257, 1, 1, 64, 128), (900, 3, 3, 96, 96)])
+def test_tiles_of_256_rows_are_as_those_of_128(T, E, top, ff, K):
+    """The same sums in the same order, gated and activated, with factors on the sums, row-major matrices and rows of an odd number of
+    32 values (the kernel beside it) among them."""
+    hip = HipOps(torch.bfloat16, DEV)
+    torch.manual_seed(T)
+    x, logits = torch.randn(T, K, device=DEV).bfloat16(), torch.randn(T, E, device=DEV)
+    for gated, act in ((True, "silu"), (False, "relu2")):
+        w1 = (torch.randn(E, 2 * ff if gated else ff, K, device=DEV) * K ** -0.5).bfloat16()
+        w2 = (torch.randn(E, K, ff, device=DEV) * ff ** -0.5).bfloat16()
+        for a, b in ((hip.prepare_expert_matrices(w1, gated), hip.prepare_expert_matrices(w2)), (w1, w2)):
+            for weigh in (False, True):
+                r = [hip.route_tokens(logits, E, top, tile_rows=rows) for rows in (128, 256)]
+                narrow, wide = (hip.routed_experts(x, q, a, b, activation=act, gated=gated, weigh_input=weigh) for q in r)
+                assert torch.equal(narrow, wide)
