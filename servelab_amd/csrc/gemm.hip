@@ -482,6 +482,121 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   }
 }
 
+// The same for more rows, K in chunks of 32: four wavefronts own 128 x 128, a wavefront 64 x 64, two workgroups a CU.  Bound by the
+// matrix units (64 cycles a v_mfma_f32_32x32x2_f32, 157 TFLOP/s): chunks go from memory straight into a ring of two LDS stages
+// (rows of 128 bytes as lds_place says), a lane reads four values of k of its row at once, and the matrix instruction takes its two
+// k's from the halves' lanes: value j of both, so eight k's are four instructions a tile, in another order of the terms.
+// 849 rows, 17920 x 1536 444 -> 424 us (110 TFLOP/s; two rounds of two workgroups a CU), 1536 x 8960 in three shares 250 -> 222;
+// 2,048 rows, 37888 x 3584 4,733 -> 4,279 (130), against chunks of 16 through registers and single words.  What is left: the two
+// workgroups of a CU begin, end and come to their barriers together (some 25 us a round; a higher wave priority for one of them
+// changes nothing).
+template <bool SHARES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    float* __restrict__ y, int M, int N, int K, int nsplit) {
+  constexpr int CK = 32, STAGE = 256 * 128;
+  __shared__ __attribute__((aligned(1024))) char ring[2 * STAGE];      // rows of x, then those of W
+  const int t = threadIdx.x, lane = t & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 1, wn = wave & 1;
+  // a chiplet takes a contiguous eighth of the (share, column tile, row tile) triples, row tiles fastest
+  const int gx = (N + 127) / 128, gy = (M + 127) / 128, total = gx * gy * nsplit, per = (total + 7) / 8;
+  const int triple = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || triple >= total) return;        // (the whole workgroup)
+  const int share = triple / (gx * gy), m0 = triple % gy * 128, n0 = triple / gy % gx * 128;
+  constexpr int SEG = SEGMENT_K / CK;                 // chunks a running sum takes
+  const int chunks = K / CK, segs = (chunks + SEG - 1) / SEG;
+  const int first = SHARES ? (int)((unsigned)segs * share / (unsigned)nsplit) * SEG : 0;
+  const int behind = SHARES ? (int)((unsigned)segs * (share + 1) / (unsigned)nsplit) * SEG : segs * SEG;
+  const int last = behind < chunks ? behind : chunks;
+  if (SHARES) {
+    y += (size_t)share * M * N;
+    bias = nullptr;
+  }
+  // what this lane brings of every chunk: unit (lane % 8) ^ place of rows 8 (wave + 4 j) + lane / 8; rows past the end: the last
+  const float* src[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int r = 8 * (wave + 4 * (j & 3)) + (lane >> 3), c = (lane & 7) ^ lds_place(r);
+    if (j < 4) src[j] = x + (size_t)(m0 + r < M ? m0 + r : M - 1) * K + 4 * c;
+    else src[j] = w + (size_t)(n0 + r < N ? n0 + r : N - 1) * K + 4 * c;
+  }
+  const unsigned ring_at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring + 1024 * wave;
+  auto load = [&](int j, int c, int stage) { load_to_lds(src[j] + CK * (size_t)c, ring_at + STAGE * stage + 4096 * j); };
+  auto barrier = [&]() {
+    asm volatile("" : : : "memory");
+    wait_loads<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+  };
+  int at[4];                                           // this lane's four values of eight k's: row lane % 32, unit 2 g + half
+#pragma unroll
+  for (int g = 0; g < 4; ++g) at[g] = 128 * (lane & 31) + 16 * ((2 * g + half) ^ lds_place(lane & 15));
+  const int x_at = 128 * 64 * wm, w_at = 128 * (128 + 64 * wn);
+  f32x16 acc[2][2], sum[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = sum[i][j][r] = 0.f;
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  f32x4 a[2][2], b[2][2];                              // [set][tile]
+  auto operands = [&](int set, int g, int stage) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a[set][i] = *(const f32x4*)(ring + STAGE * stage + x_at + 4096 * i + at[g]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) b[set][i] = *(const f32x4*)(ring + STAGE * stage + w_at + 4096 * i + at[g]);
+  };
+#pragma unroll
+  for (int j = 0; j < 8; ++j) load(j, first, first & 1);
+  barrier();
+  for (int c0 = first; c0 < last; c0 += SEG) {
+    const int c1 = c0 + SEG < last ? c0 + SEG : last;
+    for (int c = c0; c < c1; ++c) {
+      const int stage = c & 1, ahead = c + 1 < last ? c + 1 : c;       // (at the end the last chunk again, which nothing reads)
+      operands(0, 0, stage);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (g < 3) operands((g + 1) & 1, g + 1, stage);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (g < 2) load(4 * g + k, ahead, stage ^ 1);
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              acc[i][j ^ i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g & 1][i][k], b[g & 1][j ^ i][k], acc[i][j ^ i], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      barrier();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        sum[i][j] += acc[i][j];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      }
+  }
+  // element r of a tile: row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = n0 + 64 * wn + 32 * j + (lane & 31);
+    if (n >= N) continue;
+    const float bv = bias != nullptr ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = m0 + 64 * wm + 32 * i + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (m < M) y[(size_t)m * N + n] = sum[i][j][r] + bv;
+      }
+  }
+}
+
 // The shares' sums added up in their order, then the bias; VEC values a thread.
 template <int VEC>
 __global__ __launch_bounds__(256) void f32_shares_kernel(const float* __restrict__ part, const float* __restrict__ bias,
@@ -522,6 +637,12 @@ extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const floa
   if (M <= 64) {
     if (nsplit > 1) run(gemm_f32_mfma_kernel<1, 1, 1, 4, true>);
     else run(gemm_f32_mfma_kernel<1, 1, 1, 4, false>);
+  } else if (K % 32 == 0) {
+    const long long triples = (long long)grid.x * grid.y * nsplit;
+    SL_CHECK(triples < (1ll << 24), "gemm_f32_mfma: too many tiles");
+    const dim3 line((unsigned)(8 * ((triples + 7) / 8)));
+    if (nsplit > 1) gemm_f32_ring_kernel<true><<<line, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
+    else gemm_f32_ring_kernel<false><<<line, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
   } else {
     if (nsplit > 1) run(gemm_f32_mfma_kernel<2, 2, 2, 2, true>);
     else run(gemm_f32_mfma_kernel<2, 2, 2, 2, false>);
@@ -1985,7 +2106,7 @@ static void rounds(const __bf16* x, const __bf16* w, const float* bias, void* y,
 // of the float sums; act: y = act(x W^T + bias), bfloat16.
 // ks > 1: `part` holds ks * M * N floats; with y == nullptr they are left
 // there for the reader to add (and the bias with them), else splitk_reduce adds them into y.
-// square: rows of x a tile, 256 or 192, by 256 of W (gemm_rounds.h); 0: tiles of 256 x 128, which take
+// square: rows of x a tile, 256, 192 or 128, by 256 of W (gemm_rounds.h); 0: tiles of 256 x 128, which take
 // any N and stand in where the others' stores of 16 bytes do not fit.
 extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* bias, void* y,
                                      int M, int N, int K, int out_f32, int gated, int act, int ks, int square, float* part,
@@ -1995,7 +2116,7 @@ extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* 
   SL_CHECK(ks >= 1 && ks <= 64 && ks <= K / 64, "gemm_block: ks must be in 1..64 and <= K / 64");
   SL_CHECK(ks == 1 || part != nullptr, "gemm_block: a split of K needs the partial buffer");
   SL_CHECK(y != nullptr || ks > 1, "gemm_block: no output");
-  SL_CHECK(square == 0 || square == 256 || square == 192, "gemm_block: tiles of 256 rows by 128 or 256, or of 192 by 256");
+  SL_CHECK(square == 0 || square == 256 || square == 192 || square == 128, "gemm_block: tiles of 256 rows by 128, or of 256, 192 or 128 by 256");
   SL_CHECK(!gated || (square && ks == 1 && !out_f32 && N % 16 == 0),
            "gemm_block: a gated product takes wide tiles, whole rows of K, blocks of eight and bfloat16 results");
   SL_CHECK(!act || (square && ks == 1 && !out_f32 && !gated && N % 8 == 0),
@@ -2009,11 +2130,12 @@ extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* 
   // (Tiles of 64 x 256 and 128 x 256 for fewer rows of x were built and measured: alone they beat the
   // LDS-staged kernel above, in a decode step of 24 to 128 requests they lost 2-5 % tokens/s to it,
   // so that kernel keeps those rows and this one starts where it ends.)
-  const int bn = square ? 256 : 128, bm = square == 192 ? 192 : 256;
+  const int bn = square ? 256 : 128, bm = square ? square : 256;
   const long long triples = (long long)((N + bn - 1) / bn) * ((M + bm - 1) / bm) * ks;
   SL_CHECK(triples < (1ll << 24), "gemm_block: too many tiles");
   if (square) {
-    if (square == 192) rounds<3>(xx, ww, b, dst, M, N, K, out_f32, gated, act, ks, stream);
+    if (square == 128) rounds<2>(xx, ww, b, dst, M, N, K, out_f32, gated, act, ks, stream);
+    else if (square == 192) rounds<3>(xx, ww, b, dst, M, N, K, out_f32, gated, act, ks, stream);
     else rounds<4>(xx, ww, b, dst, M, N, K, out_f32, gated, act, ks, stream);
   } else {
     const dim3 grid((unsigned)(8 * ((triples + 7) / 8)));              // laid out by chiplet (see the kernel)

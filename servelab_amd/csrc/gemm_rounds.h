@@ -34,8 +34,9 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ w, const float* __restrict__ bias,
     void* __restrict__ y, int M, int N, int K, int act, int KS) {
   constexpr int T0 = (T + 1) / 2, T1 = T / 2, BM = 64 * T, BN = 256;   // halves of the tile: 64 T0 and 64 T1 rows of x, 128 of W
-  constexpr int SLOT = 8192 * (T0 + 2), SLOTS = 4;
+  constexpr int SLOT = 8192 * (T0 + 2), SLOTS = T == 2 ? 6 : 4;
   constexpr int HALF0 = T0 + 2, HALF1 = T1 + 2;                        // loads a wavefront makes of a half
+  constexpr int AHEAD = (HALF0 + HALF1) * (SLOTS - 2) / 2;             // that are younger than those of the half read next
   __shared__ __attribute__((aligned(1024))) char ring[SLOTS * SLOT];
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
     at_wt[kk] = at + 4096 * wn + 8192 * T0;
   }
   auto operand = [&](int at) { return *(const bf16x8*)(ring + at); };
-  wait_loads<2 * HALF1 + HALF0>();
+  wait_loads<AHEAD + HALF1>();
   barrier();
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
     for (int a = 0; a < 2 * T0; ++a) x0[a][kk] = operand(at_x0[kk] + 2048 * a);
   }
   asm volatile("" : : : "memory");
-  wait_loads<HALF0 + HALF1>();
+  wait_loads<AHEAD>();
   barrier();
   int read_at = SLOT;                      // slot of the half that is read next
   unsigned load_at = 0;                    // slot of the half that is loaded next: the one read before
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
       asm volatile("" : : : "memory");
-      wait_loads<HALF0 + HALF1>();         // the half that is read next is there: of the loads, one of each half is younger
+      wait_loads<AHEAD>();         // the half that is read next is there: of the loads, one of each half is younger
       barrier();
       read_at = next(read_at);
       load_at = next(load_at);
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
       asm volatile("" : : : "memory");
-      wait_loads<HALF0 + HALF1>();
+      wait_loads<AHEAD>();
       barrier();
       read_at = next(read_at);
       load_at = next(load_at);

@@ -363,7 +363,8 @@ class ProductOps:
 
     # rows of x a tile -> us of a launch, of a round of tiles, of a chunk of 64 values of k with few CUs busy, and what all of
     # them add to a chunk (they share the power): fitted to 168 gated products of 12 shapes, 260 to 2,048 rows of x; 3 % rms, 12 % at worst
-    TILE_US = {256: (1.8, 6.0, 0.92, 0.49), 192: (2.5, 4.0, 0.74, 0.39)}
+    # (the ones of 128 rows, with six halves on the way where the others have four, to 20)
+    TILE_US = {256: (1.8, 6.0, 0.92, 0.49), 192: (2.5, 4.0, 0.74, 0.39), 128: (1.0, 3.5, 0.68, 0.20)}
 
     def _tiles_us(self, rows, M, N, K, ks=1):
         """Estimated time of a product in tiles of ``rows`` rows of x by 256 of W."""
@@ -373,8 +374,9 @@ class ProductOps:
         return launch + rounds * (tile + K / ks / 64 * (chunk + shared * items / (rounds * self._num_cus)))
 
     def _tile_rows(self, M, N, K, ks=1):
-        """Rows of x a workgroup takes, the ones that take less time by estimate (of the 168 products 0.04 % slower on
-        average than the better one of both, 2 % at worst)."""
+        """Rows of x a workgroup takes, the ones that take the least time by estimate (256 or 192: of the 168 products 0.04 %
+        slower on average than the better one of both, 2 % at worst; 128 where those leave CUs idle: 22016 x 2048 at 527 / 640 rows
+        72 / 56 and 77 / 57 us, 9216 x 3584 at 768 58 / 46)."""
         return min(self.TILE_US, key=lambda rows: self._tiles_us(rows, M, N, K, ks))
 
     def _prompt_tiles(self, M, N, K):
@@ -428,7 +430,7 @@ class ProductOps:
 
     def linear_block(self, x, weight, bias, out_f32=False, ks=1, partial=False, square=False):
         """A few hundred rows over the row-major copy of the weight: workgroups
-        own a tile of 256 rows of x by 128 rows of W (``square``: of 256 or 192, ``_tile_rows``, by 256) over
+        own a tile of 256 rows of x by 128 rows of W (``square``: of 256, 192 or 128, ``_tile_rows``, by 256) over
         one of ``ks`` shares of K.  ``partial``: the product comes back as
         ``PartialSums`` for its reader to add up."""
         M, K = x.shape
@@ -648,7 +650,9 @@ class ProductOps:
         return y
 
     F32_SEGMENT = 512             # terms of a running sum of the float32 products: a share of K holds whole ones
-    F32_TILE_US_PER_TERM = 0.067  # a tile of 128 x 128 results takes this long per term of K with a CU to itself
+    F32_TILE_US_PER_TERM = 0.067  # a tile of 32 x 128 results takes a quarter of this per term of K with a CU to itself
+    # a tile of 128 x 128: us, and us per term of K, with a CU to itself and beside another (fitted to 12 products)
+    F32_TILE_ALONE, F32_TILE_PAIR = (3.0, 0.060), (25.0, 0.1215)
 
     def _f32_shares(self, M, N, K):
         """Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated
@@ -657,9 +661,14 @@ class ProductOps:
         rows = 32 if M <= 64 else 128
         tiles = -(-M // rows) * -(-N // 128)
         best, least, segments = 1, float("inf"), -(-K // self.F32_SEGMENT)
+
+        def two_a_cu(items, terms):                  # rounds of two tiles a CU, the last one of single ones if they suffice
+            alone, pair = (us + per * terms for us, per in (self.F32_TILE_ALONE, self.F32_TILE_PAIR))
+            whole, rest = divmod(items, 2 * self._num_cus)
+            return whole * pair + (0.0 if not rest else alone if rest <= self._num_cus else pair)
         for s in range(1, min(16, segments) + 1):
             terms = min(K, -(-segments // s) * self.F32_SEGMENT)          # of the longest share
-            us = -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM * (rows / 128)
+            us = two_a_cu(tiles * s, terms) if rows == 128 else -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM / 4
             if s > 1:
                 us += 5.0 + (s + 1) * M * N * 4 / 3e6
             if us < 0.97 * least:

@@ -88,3 +88,17 @@ def test_shares_cost_what_the_longest_one_takes():
     ops = HipOps(torch.float32, DEV)
     assert ops._f32_shares(512, 9728, 896) == 1                # two segments of 512 and 384 terms: as long as three rounds of 512
     assert ops._f32_shares(849, 1536, 8960) > 1 and ops._f32_shares(64, 256, 512) == 1
+
+
+# rows that end a tile of 128 and pass it by one, odd columns, one chunk of 32, a chunk past a segment of 512, a last share of one chunk
+@pytest.mark.parametrize("M,N,K", [(65, 1, 32), (128, 127, 544), (129, 130, 1056), (255, 129, 96), (1025, 1100, 64)])
+def test_products_in_chunks_of_32(M, N, K):
+    ops = HipOps(torch.float32, DEV)
+    g = torch.Generator().manual_seed(M)
+    x, w, b = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g), torch.randn(N, generator=g)
+    want, size = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    for shares in {1, -(-K // 512)}:
+        ops._f32_shares = lambda *_: shares
+        got = ops.linear_f32_mfma(x.to(DEV), w.to(DEV), b.to(DEV)).cpu()
+        # running sums of up to 512 products: no further off than 512 roundings of 2^-24 of their absolute sum
+        assert ((got.double() - want).abs() <= min(K, 512) * 2.0 ** -24 * size).all()

@@ -11,7 +11,7 @@ DEV = "cuda:0"
 
 # 261 and 348 tiles on 256 CUs, a number of tiles that eight does not divide, tiles of one, two and three chunks
 @pytest.mark.parametrize("M,N,K", [(700, 22064, 64), (700, 22064, 192), (600, 32800, 128)])
-@pytest.mark.parametrize("rows", [192, 256])
+@pytest.mark.parametrize("rows", [128, 192, 256])
 def test_workgroups_walk_several_tiles(M, N, K, rows):
     ops = HipOps(torch.bfloat16, DEV)
     assert -(-M // rows) * -(-N // 256) > ops._num_cus
@@ -56,20 +56,22 @@ def test_routes_by_estimated_rate():
     ops = HipOps(torch.bfloat16, DEV)
     tiles = ops._prompt_tiles
     # well filled rounds, in the height that takes less time; part-filled ones stay with the library
-    assert [tiles(M, 37888, 3584) for M in (300, 400, 527, 1000, 2048, 2560)] == [None, 192, 192, 256, 256, 256]
-    assert [tiles(M, 9216, 3584) for M in (640, 900, 1536)] == [None, 192, 256]
+    assert [tiles(M, 37888, 3584) for M in (260, 400, 527, 1000, 2048, 2560)] == [None, 192, 192, 256, 256, 256]
+    assert [tiles(M, 22016, 2048) for M in (400, 527, 640, 768)] == [256, 128, 128, 192]
+    assert [tiles(M, 9216, 3584) for M in (527, 640, 900, 1536)] == [None, 128, 192, 256]
     assert tiles(255, 37888, 3584) is None and tiles(2561, 37888, 3584) is None and tiles(2048, 37888, 3600) is None
     assert tiles(2048, 4080, 3584) is None and tiles(2048, 37888, 8256) is None
     # either height gives the same sums
     x = torch.randn(527, 512, device=DEV).bfloat16()
     w = (torch.randn(22016, 512, device=DEV) * 0.05).bfloat16()
     weight = ops.prepare_weight(w)
-    assert torch.equal(ops.linear_gated_block(x, weight, None, 192, 1), ops.linear_gated_block(x, weight, None, 256, 1))
+    whole = ops.linear_gated_block(x, weight, None, 256, 1)
+    assert torch.equal(ops.linear_gated_block(x, weight, None, 192, 1), whole) and torch.equal(ops.linear_gated_block(x, weight, None, 128, 1), whole)
 
 
 # ragged rows of x and of W, both heights
 @pytest.mark.parametrize("M,N,K,act", [(300, 4112, 128, "relu2"), (257, 1000, 192, "silu"), (385, 264, 64, "gelu_tanh"), (193, 520, 64, "relu")])
-@pytest.mark.parametrize("rows", [192, 256])
+@pytest.mark.parametrize("rows", [128, 192, 256])
 def test_activation_of_the_sums(M, N, K, act, rows):
     ops = HipOps(torch.bfloat16, DEV)
     g = torch.Generator().manual_seed(M)
