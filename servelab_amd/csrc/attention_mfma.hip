@@ -974,6 +974,7 @@ extern "C" const char* sl_attention_mfma(
   SL_CHECK(((uintptr_t)qkv % 16) == 0 && ((uintptr_t)kc % 16) == 0 && ((uintptr_t)vc % 16) == 0,
            "attention_mfma: operands must be 16-byte aligned");
   SL_CHECK(window >= 0 && nsplit >= 1 && max_q_len >= 1, "attention_mfma: bad window, split or length");
+  SL_CHECK(out != nullptr || (nsplit > 1 && max_q_len == 1 && !group && ctx_stats == nullptr), "attention_mfma: no output, and no shares of one to leave");
   SL_CHECK(nkv <= 65535 && num_seqs <= 65535, "attention_mfma: grid too large");
   if (num_seqs == 0) return nullptr;
   const int g = nh / nkv;
@@ -1025,7 +1026,7 @@ extern "C" const char* sl_attention_mfma(
     }
 #undef SL_SPLIT
     const char* e = sl_launch_status();
-    if (e) return e;
+    if (e || out == nullptr) return e;               // (out == nullptr: the shares are left to their reader)
     if (one_length) attention_combine_kernel<true><<<dim3(num_seqs, nh), 64, 0, stream>>>(
         part_o, part_ml, nsplit, nh, part_row0, (__bf16*)out, out_rows);
     else attention_combine_kernel<false><<<dim3(num_seqs, nh), 64, 0, stream>>>(
@@ -1085,5 +1086,14 @@ extern "C" const char* sl_attention_mfma(
                                                                     part_row0, (__bf16*)out, out_rows);
     }
   }
+  return sl_launch_status();
+}
+
+// Shares that a split launch over `rows` single tokens left (out == nullptr) into plain rows.
+extern "C" const char* sl_attention_combine(const float* part_o, const float* part_ml, int nsplit, int nh, int rows, void* out,
+                                            hipStream_t stream) {
+  SL_CHECK(part_o != nullptr && part_ml != nullptr && out != nullptr, "attention_combine: shares and a result");
+  SL_CHECK(rows > 0 && nh > 0 && nh <= 65535 && nsplit >= 1 && nsplit <= 64 * COMBINE_PER_LANE, "attention_combine: bad sizes");
+  attention_combine_kernel<false><<<dim3(rows, nh), 64, 0, stream>>>(part_o, part_ml, nsplit, nh, 0, (__bf16*)out, 0);
   return sl_launch_status();
 }

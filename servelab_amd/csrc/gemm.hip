@@ -702,6 +702,7 @@ __device__ __forceinline__ bf16x8 stream_load(const __bf16* p) {
 #define SL_MAX_PARTS_PER_THREAD 16      // 32 * 16 parts of 16 columns: rows of up to 8192 values
                                         // (8 per thread, and fewer registers, for rows of up to 4096)
 
+#define SL_MAX_SHARES 8
 struct NormFusion {
   const float* in_parts;     // CONSUMER: [in_nparts][16] sums of squares by row
   int in_nparts;
@@ -725,6 +726,14 @@ struct NormFusion {
   int pair_x;                // at most 8 rows and one tile a workgroup: a load of x takes two k-steps (see stream_k2)
   int gate_act;              // gated forms: the activation of the gate (common.h: 1 silu, 2 relu); plain form: the
                              // activation of the result (0: none)
+};
+
+// SHARES: x is the attention's result, still in shares of its keys, which every workgroup merges on its way: partial outputs
+// [M, K / D, shares, D] and (maximum, sum) [M, K / D, shares, 2], D = 1 << head_bits.
+struct KeyShares {
+  const float* o;
+  const float2* ml;
+  int shares, head_bits;
 };
 
 // Rotary embedding and the write to the cache pages fused into the q/k/v
@@ -751,11 +760,11 @@ struct RopeStore {
 // CU pulls, and halving them shows (MI355X, gate/up of the 7B shape at 16 rows:
 // 66 us with one tile).  Matrices with few tiles keep one tile per workgroup so
 // that every CU has work.
-template <bool GATED, bool CONSUMER, bool PRODUCER, int PARTS, bool ROPE = false, int NT = 1, int WAVES = 8>
+template <bool GATED, bool CONSUMER, bool PRODUCER, int PARTS, bool ROPE = false, int NT = 1, int WAVES = 8, bool SHARES = false>
 __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ wt, const float* __restrict__ bias,
     void* __restrict__ y, int M, int N, int K, int out_f32, const NormFusion F,
-    const RopeStore R = RopeStore{}) {
+    const std::conditional_t<SHARES, KeyShares, RopeStore> R) {
   constexpr int U = NT == 1 ? 8 : 4;
   static_assert(WAVES == 8 || !CONSUMER, "the shares of the sums of squares are laid out for 512 threads");
   __shared__ f32x4 red[NT][WAVES][64];
@@ -806,7 +815,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
   // (ROPE: the bias, the angle's cosine and sine and the cache row of this thread's element)
   float b_pre[NT], c_pre[NT], s_pre[NT];
   int slot_pre = 0;
-  if (ROPE) {
+  if constexpr (ROPE) {
     if (threadIdx.x < 256 && em < M && R.slots != nullptr) slot_pre = R.slots[em];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -936,7 +945,47 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
     if (F.x_tiled) stream_k(std::true_type{}, th_tag);
     else stream_k(std::false_type{}, th_tag);
   };
-  if constexpr (!PRODUCER) {
+  if constexpr (SHARES) {
+    // A thread merges the shares of a channel, everything it needs asked for at once behind the first of W, into rows of
+    // bfloat16 in LDS.  (Merged by the lanes that multiply, sixteen (row, share) pairs to a load, it took 7 us a layer of the 0.5B
+    // shape more than the merging kernel that it saves.)
+    constexpr int KB = 4, J = SL_MAX_SHARES;
+    extern __shared__ __bf16 merged[];                        // [M][K]
+    auto w_of = [&](int k) { return stream_load(wp[0] + (size_t)32 * th * k); };
+    bf16x8 a[KB];
+#pragma unroll
+    for (int u = 0; u < KB; ++u) a[u] = w_of(ks0 + u < ks1 ? ks0 + u : ks1 - 1);
+    for (int c = threadIdx.x; c < M * K; c += 64 * WAVES) {
+      const size_t at = (size_t)(c >> R.head_bits) * R.shares;          // (rows of K values: whole heads)
+      const float* o = R.o + (at << R.head_bits) + (c & ((1 << R.head_bits) - 1));
+      float v[J], top = -INFINITY, sum = 0.f, all = 0.f;
+      float2 ml[J];
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int q = j < R.shares ? j : R.shares - 1;
+        v[j] = o[(size_t)q << R.head_bits];
+        ml[j] = R.ml[at + q];
+      }
+#pragma unroll
+      for (int j = 0; j < J; ++j) top = fmaxf(top, ml[j].x);
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const float wgt = j < R.shares && ml[j].x != -INFINITY ? __builtin_amdgcn_exp2f(ml[j].x - top) : 0.f;   // (maxima are in units of log 2)
+        all += wgt * ml[j].y;
+        sum += wgt * v[j];
+      }
+      merged[c] = (__bf16)(sum * (1.f / all));
+    }
+    __syncthreads();
+    const __bf16* row = merged + (size_t)(i < M ? i : M - 1) * K + 8 * gq;
+    for (int ks = ks0; ks < ks1; ks += KB) {
+#pragma unroll
+      for (int u = 0; u < KB; ++u) {
+        if (ks + u >= ks1) break;
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ks == ks0 ? a[u] : w_of(ks + u), *(const bf16x8*)(row + 32 * (ks + u)), acc[0], 0, 0, 0);
+      }
+    }
+  } else if constexpr (!PRODUCER) {
     stream_th(std::integral_constant<int, 16>{});
   } else {
     if (th == 16) stream_th(std::integral_constant<int, 16>{});
@@ -945,7 +994,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
     else if (th == 10) stream_th(std::integral_constant<int, 10>{});
     else stream_th(std::integral_constant<int, 8>{});
   }
-  if constexpr (NT == 1) {
+  if constexpr (NT == 1 && !SHARES) {
     if (M <= 8 && F.pair_x) {         // column m + 8 of the odd k-steps' sums belongs to column m
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[0][r] += __shfl(acc_odd[r], lane + 8, 64);
@@ -1008,7 +1057,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
 #pragma unroll
       for (int wv = 0; wv < WAVES; ++wv) s += red[t][wv][m + 16 * (n_local / 4)][n_local % 4];
       if (CONSUMER && live) s *= inv_of(m);
-      if (ROPE) {
+      if constexpr (ROPE) {
         s += b_pre[t];
         const float partner = __shfl_xor(s, 8, 64);      // the other half of the pair, same row
         if (!live) continue;
@@ -1127,14 +1176,37 @@ extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float
   }
   // a matrix with fewer tiles than the chip has CUs leaves each CU one workgroup: sixteen
   // wavefronts then have twice the loads in flight (7B shape, batch 1: 349 -> 356 tok/s)
-  if (producer && (int)grid.x <= device_cus() && K >= 2048) gemm_skinny_kernel<false, false, true, 1, false, 1, 16><<<grid, 1024, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F);
-  else if (producer) gemm_skinny_kernel<false, false, true, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F);
-  else if (consumer && gated && few) gemm_skinny_kernel<true, true, false, 8><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F);
-  else if (consumer && gated) gemm_skinny_kernel<true, true, false, 16><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F);
-  else if (consumer && few) gemm_skinny_kernel<false, true, false, 8><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F);
-  else if (consumer) gemm_skinny_kernel<false, true, false, 16><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F);
-  else if (gated) gemm_skinny_kernel<true, false, false, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F);
-  else gemm_skinny_kernel<false, false, false, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F);
+  if (producer && (int)grid.x <= device_cus() && K >= 2048) gemm_skinny_kernel<false, false, true, 1, false, 1, 16><<<grid, 1024, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
+  else if (producer) gemm_skinny_kernel<false, false, true, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
+  else if (consumer && gated && few) gemm_skinny_kernel<true, true, false, 8><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
+  else if (consumer && gated) gemm_skinny_kernel<true, true, false, 16><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
+  else if (consumer && few) gemm_skinny_kernel<false, true, false, 8><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
+  else if (consumer) gemm_skinny_kernel<false, true, false, 16><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
+  else if (gated) gemm_skinny_kernel<true, false, false, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
+  else gemm_skinny_kernel<false, false, false, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
+  return sl_launch_status();
+}
+
+// A producer (see sl_gemm_skinny) whose x is attention that is still in shares of its keys: M rows of K = heads * head_dim values,
+// partial outputs [M, heads, shares, head_dim] and (maximum, sum) [M, heads, shares, 2] as the attention's split launch
+// leaves them.  The kernel that merges them, 2.5 to 4.5 us a layer for a few thousand values, is saved; every
+// workgroup reads all shares instead, which is why few of them are taken (24 layers of 896 values at 300 keys, four tokens 2,871 ->
+// 2,770 us).
+extern "C" const char* sl_gemm_skinny_shares(const float* shares_o, const float* shares_ml, int shares, int head_dim, const void* wt,
+                                             const float* bias, void* y, int M, int N, int K, float* resid, const float* next_w,
+                                             float* out_parts, int y_tiled, int th, hipStream_t stream) {
+  SL_CHECK(M > 0 && N > 0 && K > 0 && K % 32 == 0, "gemm_skinny_shares: sizes must be positive, K in steps of 32");
+  SL_CHECK(head_dim >= 32 && (head_dim & (head_dim - 1)) == 0 && K % head_dim == 0, "gemm_skinny_shares: heads of a power of two, 32 at least");
+  SL_CHECK(shares >= 2 && shares <= SL_MAX_SHARES, "gemm_skinny_shares: 2 to 8 shares");
+  SL_CHECK(M <= 16 && M * K <= 16384, "gemm_skinny_shares: at most 16 rows, of 16,384 values together");
+  SL_CHECK(shares_o != nullptr && shares_ml != nullptr && resid != nullptr && next_w != nullptr && out_parts != nullptr,
+           "gemm_skinny_shares: a producer over shares needs them, the stream, the next gain and a parts buffer");
+  SL_CHECK(((uintptr_t)shares_o % 16) == 0 && ((uintptr_t)shares_ml % 8) == 0 && ((uintptr_t)wt % 16) == 0, "gemm_skinny_shares: shares and W must be 16-byte aligned");
+  SL_CHECK(th >= 8 && th <= 16 && th % 2 == 0 && (!y_tiled || N % 32 == 0), "gemm_skinny_shares: tiles of 8 to 16 rows, tiled results of N % 32 == 0");
+  const NormFusion F{nullptr, 0, 0.f, nullptr, resid, next_w, out_parts, 0, y_tiled, th, 0, 0};
+  const KeyShares R{shares_o, (const float2*)shares_ml, shares, __builtin_ctz(head_dim)};
+  gemm_skinny_kernel<false, false, true, 1, false, 1, 16, true><<<(N + th - 1) / th, 1024, 2 * M * K, stream>>>(
+      nullptr, (const __bf16*)wt, bias, y, M, N, K, 0, F, R);
   return sl_launch_status();
 }
 

@@ -6,7 +6,7 @@ import ctypes
 import torch
 
 from . import build
-from .values import (KernelError, LinearWeight, PartialSums, RotationPlan, ScaledRows, TiledRows,
+from .values import (AttentionShares, Deferred, KernelError, LinearWeight, PartialSums, RotationPlan, ScaledRows, TiledRows,
                      _RopeStore, _c_float, _p, _ptr)
 
 
@@ -210,12 +210,43 @@ class AttentionOps:
                  and batch.num_prefill_seqs == 0 and batch.num_seqs == T and w_out.tiled is not None
                  and w_out.shape[1] == nh * D
                  and self._mfma_attention_fits(D, nh // nkv, block_tables.shape[1], page_size, batch))
+        shares = defer and self._shares_for_projection(T, nh, nkv, D, block_tables, page_size, batch, window, w_out)
         attn = self.paged_attention(qkv, nh, nkv, D, k_cache, v_cache, page_size, block_tables,
-                                    batch, scale, window, _tiled_out=tiled)
-        return self.linear(attn, w_out, bias, defer=defer)
+                                    batch, scale, window, _tiled_out=tiled and not shares, _leave_shares=bool(shares))
+        return Deferred(attn, w_out, bias) if shares else self.linear(attn, w_out, bias, defer=defer)
+
+    def _shares_for_projection(self, T, nh, nkv, D, block_tables, page_size, batch, window, w_out):
+        """Into how many shares of its keys the attention of a step of single tokens is cut, where the output projection may merge
+        them (its kernel adds to the stream as well): 0 where it may not.  Every workgroup of the projection reads all shares, so
+        their values are bounded by SHARES_MAX_VALUES; rows of up to SHARES_MAX_K values are one trip to
+        memory for a wavefront.  A layer of the 0.5B shape, merged by a kernel of its own / here, 1 request at 280 / 300 / 400 keys 29.8 /
+        28.8, 30.4 / 28.8 and 29.9 / 29.1 us, 2 requests 30.7 / 29.9, 30.1 / 30.4 and 30.8 / 30.4, 4 and 8 the same either way; of
+        the 1.5B shape, 1 request at 280 46.7 / 43.9; of the 3B shape the same either way."""
+        K, N = nh * D, w_out.shape[0]
+        if not (self.act_dtype == torch.bfloat16 and self.fuse_norms and self.merge_shares and batch.max_q_len == 1
+                and batch.num_prefill_seqs == 0 and batch.num_seqs == T and 0 < T <= min(8, self._fused_rows(N)) and N <= 8192
+                and w_out.tiled is not None and w_out.shape[1] == K and K <= self.SHARES_MAX_K and D & (D - 1) == 0
+                and self._mfma_attention_fits(D, nh // nkv, block_tables.shape[1], page_size, batch)
+                and not (self.SHARES_OF_ONE_LENGTH and getattr(batch, "ctx_stats", None) is not None)):
+            return 0
+        lib = self._attention_lib(D)
+        blocks = -(-batch.max_ctx_len // 32)
+        if window:
+            blocks = min(blocks, -(-int(window) // 32) + 1)
+        fits = nh // nkv <= int(self._lib[lib].sl_attention_mfma_group_heads())
+        launches = self._decode_launches(T, nkv, blocks, D, fits, int(self._lib[lib].sl_attention_mfma_max_splits()))
+        shares = launches[0][3] if len(launches) == 1 and not launches[0][2] else 1
+        return shares if 1 < shares <= 8 and T * shares * K <= self.SHARES_MAX_VALUES else 0
+
+    def combine_shares(self, a):
+        """Plain rows of attention that is in shares."""
+        T, nh, shares, D = a.o.shape
+        out = self._new(a.shape)
+        self._call(self._attention_lib(D), "sl_attention_combine", _p(a.o), _p(a.ml), shares, nh, T, _p(out))
+        return out
 
     def paged_attention(self, qkv, nh, nkv, D, k_cache, v_cache, page_size, block_tables,
-                        batch, scale, window, _tiled_out=False):
+                        batch, scale, window, _tiled_out=False, _leave_shares=False):
         T = qkv.shape[0]
         S, max_pages = block_tables.shape
         self._check(qkv, self.act_dtype, (T, (nh + 2 * nkv) * D), "qkv")
@@ -227,6 +258,8 @@ class AttentionOps:
             raise KernelError(f"block tables hold {S} sequences, the batch {batch.num_seqs}")
         if batch.max_ctx_len > max_pages * page_size:
             raise KernelError("block table is shorter than the context")
+        if _leave_shares:
+            return self._attention_mfma(qkv, nh, nkv, D, k_cache, v_cache, page_size, block_tables, batch, scale, window, None)
         out = self._new((T, nh * D))
         if self._mfma_attention_fits(D, nh // nkv, max_pages, page_size, batch):
             self._attention_mfma(qkv, nh, nkv, D, k_cache, v_cache, page_size, block_tables,
@@ -468,3 +501,5 @@ class AttentionOps:
                 self._call(lib, name, *common, n_pre + first, count, 1, *tail, nsplit, 0, 0, _p(out),
                            _p(part_o), _p(part_ml), n_pre_tok + first, count if nsplit > 1 else 0, 0,
                            int(out_rows), int(group), _p(stats) if aim else None, aim)
+                if out is None:               # (one launch in shares, see _shares_for_projection)
+                    return AttentionShares(part_o, part_ml)

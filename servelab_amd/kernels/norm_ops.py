@@ -4,7 +4,7 @@ import ctypes
 
 import torch
 
-from .values import (Deferred, KernelError, PartialSums, ScaledRows, TiledRows, _c_float, _p,
+from .values import (AttentionShares, Deferred, KernelError, PartialSums, ScaledRows, TiledRows, _c_float, _p,
                      activation_code)
 
 
@@ -124,15 +124,21 @@ class NormOps:
         N = weight.shape[0]
         if tuple(resid.shape) != (M, N):
             raise KernelError(f"a delta of shape {[M, N]} does not fit the stream {list(resid.shape)}")
-        self._check(x.data if isinstance(x, TiledRows) else x, self.act_dtype, None, "x")
+        shares = isinstance(x, AttentionShares)
+        if not shares:
+            self._check(x.data if isinstance(x, TiledRows) else x, self.act_dtype, None, "x")
         if d.bias is not None:
             self._check(d.bias, torch.float32, (N,), "bias")
         out = self._new((M, N))
-        th = self._producer_copy(weight, M)[1]
+        wt, th = self._producer_copy(weight, M)
         parts = self._new((-(-N // th), 16), torch.float32)
         tiled = M if self.tile_few_rows and M > 1 and N % 32 == 0 else 0     # for the products that read the rows
-        self._skinny(x, weight, d.bias, out, M, N, K, resid=resid, next_gain=gain, out_parts=parts,
-                     y_tiled=bool(tiled))
+        if shares:
+            self._call("gemm", "sl_gemm_skinny_shares", _p(x.o), _p(x.ml), x.o.shape[2], x.o.shape[3], _p(wt), _p(d.bias), _p(out),
+                       M, N, K, _p(resid), _p(gain), _p(parts), int(bool(tiled)), th)
+        else:
+            self._skinny(x, weight, d.bias, out, M, N, K, resid=resid, next_gain=gain, out_parts=parts,
+                         y_tiled=bool(tiled))
         return ScaledRows(out, parts, eps, tiled=tiled)
 
     def silu_mul(self, gate_up, block=None):

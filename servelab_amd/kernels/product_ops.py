@@ -10,7 +10,7 @@ from typing import Optional
 
 import torch
 
-from .values import (Deferred, KernelError, LinearWeight, PartialSums, ScaledRows, TiledRows,
+from .values import (AttentionShares, Deferred, KernelError, LinearWeight, PartialSums, ScaledRows, TiledRows,
                      _c_float, _p, activation_code)
 
 
@@ -175,6 +175,8 @@ class ProductOps:
             if weight.tiled is not None and weight.shape == (weight.shape[0], x.shape[1]):
                 return self._linear_scaled(x, weight, bias, out_f32, False)
             x = self.finish_scaled_rows(x)      # (a matrix the fused kernels do not take: rows of odd length)
+        if isinstance(x, AttentionShares):
+            x = self.combine_shares(x)
         M, K = x.shape
         N = weight.shape[0]
         if isinstance(x, TiledRows) and not (defer and self.fuse_norms and not out_f32 and N <= 8192):

@@ -54,6 +54,7 @@ class KernelTable:
         self._resident_k = {}
         self.fuse_norms = act_dtype == torch.bfloat16
         self.fuse_rope = act_dtype == torch.bfloat16
+        self.merge_shares = act_dtype == torch.bfloat16       # the output projection merges attention that is in few shares
         self.tile_few_rows = act_dtype == torch.bfloat16      # gated_mlp keeps few rows tiled by k-step
         self.weight_layout = "dual" if act_dtype == torch.bfloat16 else "rows"
         self.lower_tiles = act_dtype == torch.bfloat16        # see plan_weights

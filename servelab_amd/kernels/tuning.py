@@ -146,6 +146,10 @@ class Tuning:
     # 3.92 -> 3.84 ms (in shares), 60 at 2,048 keys 4.98 -> 4.81 ms (merged); 48 at 1,024 keys 3.95 ms merged, 4.03 in shares.
     group_attention_fill: float = 1.0
     group_attention_from: tuple = ((8, 1 / 1024), (16, 0.45), (32, 0.7), (64, 0.85), (128, 0.97), (1 << 30, 1.01))
+    # attention in shares that the output projection merges (HipOps._shares_for_projection): the longest rows, and the most values
+    # of all rows' shares together (32 KB, which every workgroup of the projection reads)
+    shares_max_k: int = 2048
+    shares_max_values: int = 8192
     # With more pairs than CUs the form is taken by an estimate of the launch's time, whose constants
     # are fitted to 63 launches of 288 to 1,024 pairs over contexts of 640 to 4,096 (3.5 % rms; the form
     # taken is 0.8 % slower than the best measured one on average, 6 % at worst).  The keys and values

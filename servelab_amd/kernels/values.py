@@ -81,6 +81,17 @@ class TiledRows:
         return self.data.view(K // 32, M, 32).permute(1, 0, 2).reshape(M, K)
 
 
+class AttentionShares:
+    """The attention of a few single tokens, still in shares of its keys: partial outputs ``o`` [T, heads, shares, D] and ``ml``
+    [T, heads, shares, 2], for the output projection that merges them (``HipOps.attend_and_project``).  Never leaves the kernel
+    table."""
+    __slots__ = ("o", "ml", "shape")
+
+    def __init__(self, o, ml):
+        self.o, self.ml = o, ml
+        self.shape = (o.shape[0], o.shape[1] * o.shape[3])
+
+
 class PartialSums:
     """A product whose K was split over workgroups, left as float partial sums
     ``parts`` [ks, T, N] with the bias not yet added, for a reader that adds
