@@ -660,7 +660,7 @@ struct Stage2 { static constexpr int value = 2; };
 // and the loads would never be more than one block ahead.  The waits are explicit instead
 // (wait_loads below; the loads complete in order).
 __device__ __forceinline__ void load_to_lds(const void* from, unsigned lds_at) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
 }
 
 // s_waitcnt vmcnt(n) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14, the other counters left at their maxima)

@@ -3,9 +3,10 @@
 // nor waits for them: wait_loads<N> returns once at most the N youngest loads of the wavefront are under way, and
 // its reads of LDS are done: behind the barrier that follows, another wavefront's loads may land where they read (the
 // compiler moves products of the last reads, and the wait for these with them, behind a barrier).
+// (M0 holds the place in LDS; a load that reads it may not follow the instruction that writes it without a wait state between.)
 #pragma once
 __device__ __forceinline__ void load_to_lds(const void* from, unsigned lds_at) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_at) : "m0");
 }
 // The same from a base that all lanes share and an offset of the lane's own.
 __device__ __forceinline__ void load_to_lds(unsigned offset, const void* base, unsigned lds_at) {
