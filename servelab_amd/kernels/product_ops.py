@@ -347,7 +347,7 @@ class ProductOps:
         longer ones, up to GATED_LONG_K values at GATED_LONG_ROWS rows of x, in several rounds of tiles of 256 x 256 whose last
         one is filled by GATED_LAST_ROUND where neither 192 nor 224 divides N, at which the library's picks idle (2,048 rows of
         37888 x 3584 542 / 422, of 22016 x 2048 196 / 151).  The sums meet the activation unrounded, so that it
-        is the more exact form as well.  Shapes that were tuned stay with the library (``_tuned_for``)."""
+        is the more exact form as well.  Shapes that were tuned may stay with the library (``_tiles_beat_tuned``)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
                 or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
             return None
@@ -398,6 +398,13 @@ class ProductOps:
         its block: whether it may be).  Those shapes stay with the library, whose default pick is
         what the rules above were measured against: tuned it is up to a quarter faster."""
         return self._tuning or (self.library_rows(M), N, K) in self._tuned
+
+    def _tiles_beat_tuned(self, M, N, K) -> bool:
+        """Whether a gated or activated product that may take the tiles does: a shape that was tuned stays with the library and its
+        pass below an estimated rate of PROMPT_TUNED_TFLOPS.  From there on the tiles are the faster pair also against the tuned pick
+        (us, tuned / tiles: 37888 x 3584 at 544 / 1,024 / 2,048 rows 172 / 138, 269 / 246 and 456 / 458, 22016 x 2048 at 2,048 184 /
+        157, 17920 x 1536 136 / 121, 55296 x 5120 951 / 865, 28672 x 4096 397 / 375, 18944 x 3584 with relu squared 263 / 267)."""
+        return not self._tuned_for(M, N, K) or 2e-6 * M * N * K >= self.PROMPT_TUNED_TFLOPS * self._tiles_us(self._tile_rows(M, N, K), M, N, K)
 
     @staticmethod
     def _block_reads(x, weight) -> bool:
@@ -548,7 +555,7 @@ class ProductOps:
             self._skinny(x, weight, bias, y, M, N, K, gated=code)
             return y
         rows = block == self.GATE_BLOCK and (self._prompt_tiles(M, N, K) or self._gated_rows(M, N, K))
-        if rows and not self._tuned_for(M, N, K) and self._block_reads(x, weight):
+        if rows and self._tiles_beat_tuned(M, N, K) and self._block_reads(x, weight):
             return self.linear_gated_block(x, weight, bias, rows, code)
         return self.gate_mul(self.linear(x, weight, bias), block, activation)
 
@@ -582,7 +589,7 @@ class ProductOps:
         N = weight.shape[0]
         if M > self._few_rows_limit(weight) or M == 0:
             rows = self._prompt_tiles(M, N, K)
-            if rows and weight.shape == (N, K) and not self._tuned_for(M, N, K) and self._block_reads(x, weight):
+            if rows and weight.shape == (N, K) and self._tiles_beat_tuned(M, N, K) and self._block_reads(x, weight):
                 return self.linear_activated_block(x, weight, bias, rows, code)
             return self.activate(self.linear(x, weight, bias), activation)
         self._check(x, self.act_dtype, None, "x")

@@ -104,6 +104,8 @@ class Tuning:
     # ... any rows of up to prompt_max_k values whose tiles are estimated at this rate or more (HipOps._prompt_tiles) ...
     prompt_max_k: int = 8192
     prompt_min_tflops: float = 750.0
+    # ... at this one also where the library's product of the shape was tuned (HipOps._tiles_beat_tuned) ...
+    prompt_tuned_tflops: float = 1000.0
     # ... longer ones, up to gated_long_k values and for so many rows of x, in several rounds, the last filled so far
     gated_long_k: int = 5120
     gated_long_rows: tuple = (1537, 2048)

@@ -102,3 +102,15 @@ def test_activated_prompts_take_the_tiles():
     plain = ops.activated_linear(odd, weight, "relu2")
     # (the library's product is rounded before the square as well)
     assert ((plain.float() - got.float()).abs() <= 2.0 ** -6 * got.float().abs() + 2.0 ** -12).all()
+
+
+def test_tuned_shapes_whose_tiles_are_faster_still():
+    ops = HipOps(torch.bfloat16, DEV)
+    rate = lambda M, N, K: 2e-6 * M * N * K / ops._tiles_us(ops._tile_rows(M, N, K), M, N, K)
+    shape, small = (2048, 37888, 3584), (1700, 8192, 1024)
+    assert rate(*shape) > ops.PROMPT_TUNED_TFLOPS > rate(*small)
+    assert ops._tiles_beat_tuned(*shape) and ops._tiles_beat_tuned(*small)                # (nothing was tuned)
+    ops._tuned = {shape, small}
+    assert ops._tiles_beat_tuned(*shape) and not ops._tiles_beat_tuned(*small)
+    ops._tuned, ops._tuning = set(), True
+    assert ops._tiles_beat_tuned(*shape) and not ops._tiles_beat_tuned(*small)
