@@ -252,6 +252,135 @@ __global__ __launch_bounds__(64) void attention_general_group_kernel(
   }
 }
 
+// The same for single tokens whose keys are shared out over wavefronts (and so are few a wavefront): blocks of 16 keys, four lanes a
+// key, each a quarter of its channels, and everything of a block asked for at once, the next block's keys and values while this one's
+// are multiplied.  A block of 64 keys, a lane each, is 10 trips to memory and a chain of 96 exchanges between lanes
+// for one wavefront, and 333 keys make six of them a pair of heads, on 256 CUs.
+// With its combine kernel, us a layer, before / here: 12 heads on 2 of 128, 1 request at 40 / 333 / 4,000 keys 26 / 16, 28 / 16 and 28 / 28,
+// 3 at 333 29 / 17, 6 at 600 29 / 18; 14 on 2 of 64, 1 and 6 requests 18 / 11 and 19 / 12.  It takes most of a SIMD's registers, so
+// that it pays while every wavefront has a SIMD to itself (16 requests at 4,000 keys, 2,048 wavefronts: 42 / 58); heads of 256
+// do not fit them (1 request at 4,000: 46 / 57).
+template <bool MAX> __device__ __forceinline__ float over_keys(float v) {      // 16 keys, the four lanes of a key alike
+  auto meet = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+  v = meet(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));   // the other key of two
+  v = meet(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true)));   // the other two of four
+  v = meet(v, __shfl_xor(v, 16, 64));
+  return meet(v, __shfl_xor(v, 32, 64));
+}
+template <int HD>
+__global__ __launch_bounds__(64) void attention_few_keys_kernel(
+    const act_t* __restrict__ qkv, int row_stride, const act_t* __restrict__ kc,
+    const act_t* __restrict__ vc, const int* __restrict__ block_tables, int max_pages,
+    const int* __restrict__ tok_seq, const int* __restrict__ positions, int nh, int nkv,
+    int page, float scale, int window, int nsplit, float* __restrict__ part_o, float* __restrict__ part_ml) {
+  constexpr int KU = HD / (4 * PIECE), VI = (HD + 63) / 64, VU = 16 / PIECE;   // pieces of a key a lane holds; channels, pieces of each
+  static_assert(KU * 4 * PIECE == HD, "four lanes a key, whole pieces");
+  __shared__ __attribute__((aligned(16))) float qs[GROUP_HEADS][HD];
+  __shared__ __attribute__((aligned(16))) float ps[GROUP_HEADS][16];
+  const int t = blockIdx.x, lane = threadIdx.x, key = lane >> 2, part = lane & 3;
+  const int g = nh / nkv, chunks = (g + GROUP_HEADS - 1) / GROUP_HEADS;
+  const int kvh = blockIdx.y / chunks, h0 = kvh * g + (blockIdx.y % chunks) * GROUP_HEADS;
+  const int nheads = kvh * g + g - h0 < GROUP_HEADS ? kvh * g + g - h0 : GROUP_HEADS;
+  const int s = tok_seq[t], p = positions[t];
+  const int lo = window > 0 ? (p - window + 1 > 0 ? p - window + 1 : 0) : 0;
+  const int* table = block_tables + (size_t)s * max_pages;
+  const int first = lo / 16, nblk = p / 16 + 1 - first;
+  const int b0 = first + (int)((long long)nblk * blockIdx.z / nsplit);
+  const int b1 = first + (int)((long long)nblk * (blockIdx.z + 1) / nsplit);
+  float m[GROUP_HEADS], l[GROUP_HEADS], acc[GROUP_HEADS][VI];
+#pragma unroll
+  for (int h = 0; h < GROUP_HEADS; ++h) {
+    m[h] = -INFINITY;
+    l[h] = 0.f;
+#pragma unroll
+    for (int i = 0; i < VI; ++i) acc[h][i] = 0.f;
+  }
+  struct block { att_piece k[KU], v[VI][VU]; };
+  auto load = [&](int b) {                              // (16 keys lie in one page; every key of a page is there to be read)
+    block r;
+    const size_t row = (size_t)table[16 * b / page] * nkv + kvh;
+    const int at = 16 * b % page;
+    const act_t* kr = kc + (row * page + at + key) * HD + PIECE * part;
+#pragma unroll
+    for (int u = 0; u < KU; ++u) r.k[u] = *(const att_piece*)(kr + 4 * PIECE * u);
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      const int d = lane + 64 * i < HD ? lane + 64 * i : HD - 1;
+#pragma unroll
+      for (int u = 0; u < VU; ++u) r.v[i][u] = *(const att_piece*)(vc + (row * HD + d) * page + at + PIECE * u);
+    }
+    return r;
+  };
+  block now;
+  if (b0 < b1) {
+    now = load(b0);
+    for (int idx = lane; idx < GROUP_HEADS * HD; idx += 64)     // rows past nheads: zeros, results never stored
+      qs[idx / HD][idx % HD] = idx / HD < nheads
+          ? to_f(qkv[(size_t)t * row_stride + (size_t)(h0 + idx / HD) * HD + idx % HD]) : 0.f;
+  }
+  __syncthreads();
+  for (int b = b0; b < b1; ++b) {
+    block ahead = now;
+    if (b + 1 < b1) ahead = load(b + 1);
+    const int r = 16 * b + key;
+    const bool valid = r >= lo && r <= p;
+    float dot[GROUP_HEADS];
+#pragma unroll
+    for (int h = 0; h < GROUP_HEADS; ++h) dot[h] = 0.f;
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+#pragma unroll
+      for (int h = 0; h < GROUP_HEADS; ++h)
+#pragma unroll
+        for (int j = 0; j < PIECE; ++j) dot[h] += qs[h][PIECE * (part + 4 * u) + j] * to_f(now.k[u].v[j]);
+#pragma unroll
+    for (int h = 0; h < GROUP_HEADS; ++h) {
+      float d = dot[h];
+      d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0xB1, 0xf, 0xf, true));
+      d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x4E, 0xf, 0xf, true));
+      const float sc = valid ? d * scale : -INFINITY;
+      const float mn = fmaxf(m[h], over_keys<true>(sc));        // every block holds a visible key
+      const float alpha = expf(m[h] - mn), pr = valid ? expf(sc - mn) : 0.f;      // exp(-inf) = 0 on the first block
+      l[h] = l[h] * alpha + over_keys<false>(pr);
+      m[h] = mn;
+      if (part == 0) ps[h][key] = pr;
+#pragma unroll
+      for (int i = 0; i < VI; ++i) acc[h][i] *= alpha;
+    }
+    __syncthreads();
+    const bool whole = 16 * b >= lo && 16 * b + 15 <= p;        // (a weight of 0 times what lies in an unseen place may be no number)
+#pragma unroll
+    for (int u = 0; u < VU; ++u)
+#pragma unroll
+      for (int e = 0; e < PIECE; ++e) {
+        const int j = PIECE * u + e;
+        const bool seen = whole || (16 * b + j >= lo && 16 * b + j <= p);
+#pragma unroll
+        for (int i = 0; i < VI; ++i) {
+          const float v = seen ? to_f(now.v[i][u].v[e]) : 0.f;
+#pragma unroll
+          for (int h = 0; h < GROUP_HEADS; ++h) acc[h][i] += ps[h][j] * v;
+        }
+      }
+    __syncthreads();
+    now = ahead;
+  }
+#pragma unroll
+  for (int h = 0; h < GROUP_HEADS; ++h) {
+    if (h >= nheads) break;
+    const size_t row = ((size_t)t * nh + h0 + h) * nsplit + blockIdx.z;
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      const int d = lane + 64 * i;
+      if (d < HD) part_o[row * HD + d] = acc[h][i];
+    }
+    if (lane == 0) {
+      part_ml[row * 2] = m[h];
+      part_ml[row * 2 + 1] = l[h];
+    }
+  }
+}
+
 // out[t, h, :] = sum_j w_j o_j / sum_j w_j l_j,  w_j = exp(m_j - max m); a share
 // without keys has m = -inf and l = 0 and drops out.  One wavefront per (t, h).
 __global__ __launch_bounds__(64) void attention_general_combine_kernel(
@@ -670,7 +799,16 @@ extern "C" const char* sl_attention_general(
   const int g = nh / nkv;
   if (g > 1) {                                       // the heads of a group together
     const int chunks = (g + GROUP_HEADS - 1) / GROUP_HEADS;
-    attention_general_group_kernel<<<dim3(T, nkv * chunks, nsplit), 64, 0, stream>>>(
+    const bool aligned = (((uintptr_t)kc | (uintptr_t)vc) % 16) == 0;
+    auto few = [&](auto kernel) {
+      kernel<<<dim3(T, nkv * chunks, nsplit), 64, 0, stream>>>((const act_t*)qkv, row_stride, (const act_t*)kc, (const act_t*)vc,
+          block_tables, max_pages, tok_seq, positions, nh, nkv, page, scale, window, nsplit, part_o, part_ml);
+    };
+    // (by the numbers of tokens and shares only, so that a captured step and an eager one add up in the same order)
+    const bool alone = nsplit > 1 && aligned && (long long)T * nkv * chunks * nsplit <= 4ll * device_cus();
+    if (alone && D == 64) few(attention_few_keys_kernel<64>);
+    else if (alone && D == 128) few(attention_few_keys_kernel<128>);
+    else attention_general_group_kernel<<<dim3(T, nkv * chunks, nsplit), 64, 0, stream>>>(
         (const act_t*)qkv, row_stride, (const act_t*)kc, (const act_t*)vc, block_tables, max_pages,
         tok_seq, positions, nh, nkv, D, page, scale, window, (act_t*)out, nsplit, part_o, part_ml);
   } else {

@@ -102,3 +102,25 @@ def test_products_in_chunks_of_32(M, N, K):
         got = ops.linear_f32_mfma(x.to(DEV), w.to(DEV), b.to(DEV)).cpu()
         # running sums of up to 512 products: no further off than 512 roundings of 2^-24 of their absolute sum
         assert ((got.double() - want).abs() <= min(K, 512) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,D", [(12, 2, 128), (14, 2, 64), (20, 2, 64), (2, 1, 128)])
+@pytest.mark.parametrize("page,window", [(16, None), (32, 40), (64, 5)])
+def test_single_tokens_in_blocks_of_16_keys(dtype, nh, nkv, D, page, window):
+    """One key and one more or less than a block, a page and a share of several blocks; more heads than a wavefront takes; what lies
+    behind a sequence's last key may be no number."""
+    from emulated_ops import EmulatedOps
+    ops, emu = HipOps(dtype, DEV), EmulatedOps(dtype)
+    ops.use_mfma_attention = False
+    lengths = [1, 16, 17] if nh == 20 else [1, 15, 1100, 65]
+    qkv, kc, vc, tables, batch = make_attention_case(dtype, nh, nkv, D, page, [(n, 1) for n in lengths])[:5]
+    ops.GENERAL_ATTENTION_WAVES = 1024                         # (as many wavefronts as have a SIMD to themselves)
+    host = emu_batch(batch)
+    want = emu.paged_attention(qkv.cpu(), nh, nkv, D, kc.cpu(), vc.cpu(), page, tables.cpu(), host, D ** -0.5, window)
+    for i, n in enumerate(lengths):                            # the unused places of each last page
+        last = int(tables[i, (n - 1) // page])
+        kc[last, :, (n - 1) % page + 1:], vc[last, :, :, (n - 1) % page + 1:] = float("nan"), float("inf")
+    got = ops.paged_attention(qkv, nh, nkv, D, kc, vc, page, tables, batch, D ** -0.5, window)
+    # float32 scores of 128 products and sums over at most 1,100 keys; bfloat16: one rounding
+    assert float((got.float().cpu() - want.float()).abs().max()) <= (3e-6 if dtype == torch.float32 else 2.0 ** -7) * max(1.0, float(want.abs().max()))
