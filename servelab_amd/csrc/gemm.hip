@@ -615,6 +615,18 @@ __global__ __launch_bounds__(256) void f32_shares_kernel(const float* __restrict
   *(piece*)(y + at) = sum;
 }
 
+// Whether a float32 product of more than 64 rows is left to the kernel of three workgroups a CU: the ring's two leave a last
+// round of at most one workgroup a CU to pairs again, which takes as long as a whole one.  That shows where terms are few and
+// rounds are few (us, ring / registers, 256 CUs; tiles times shares of so many terms): 756 of 512 145 / 120, 672 148 / 122,
+// 1,260 208 / 195, 768 of 1,024 272 / 226; not at 1,152 of 512 184 / 195, 672 of 1,024 210 / 225, 1,280 of 1,024 352 / 370,
+// 700 of 1,536 307 / 328.
+static bool f32_last_round_of_threes(long long triples, int terms) {
+  const long long cus = device_cus(), whole = triples / (2 * cus), rest = triples % (2 * cus);
+  if (terms > 1024 || rest == 0 || rest > cus) return false;
+  const bool most = 4 * rest > 3 * cus;
+  return terms <= 512 ? whole == 1 || (whole == 2 && most) : whole == 1 && most;
+}
+
 // nsplit > 1: K is cut into that many shares of whole segments, whose sums wait in `part`, [nsplit, M, N].  A product of
 // few tiles (the output projection and the down projection of a short prompt) leaves most CUs idle otherwise: 849 rows
 // of x, 1,536 rows of W of 8,960: 84 tiles.
@@ -631,14 +643,15 @@ extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const floa
   const int rows = M <= 64 ? 32 : 128;
   const dim3 grid((N + 127) / 128, (M + rows - 1) / rows, nsplit);
   SL_CHECK(grid.y <= 65535, "gemm_f32_mfma: more than 65535 row tiles");
+  const long long triples = (long long)grid.x * grid.y * nsplit;
+  const int segments = (K + SEGMENT_K - 1) / SEGMENT_K, longest = min(K, (segments + nsplit - 1) / nsplit * SEGMENT_K);
   float* to = nsplit > 1 ? part : (float*)y;
   auto run = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit); };
   // (one share apart: products of short rows take 6 to 8 % longer in a kernel that could take several)
   if (M <= 64) {
     if (nsplit > 1) run(gemm_f32_mfma_kernel<1, 1, 1, 4, true>);
     else run(gemm_f32_mfma_kernel<1, 1, 1, 4, false>);
-  } else if (K % 32 == 0) {
-    const long long triples = (long long)grid.x * grid.y * nsplit;
+  } else if (K % 32 == 0 && !f32_last_round_of_threes(triples, longest)) {
     SL_CHECK(triples < (1ll << 24), "gemm_f32_mfma: too many tiles");
     const dim3 line((unsigned)(8 * ((triples + 7) / 8)));
     if (nsplit > 1) gemm_f32_ring_kernel<true><<<line, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);

@@ -659,9 +659,7 @@ class ProductOps:
         return y
 
     F32_SEGMENT = 512             # terms of a running sum of the float32 products: a share of K holds whole ones
-    F32_TILE_US_PER_TERM = 0.067  # a tile of 32 x 128 results takes a quarter of this per term of K with a CU to itself
-    # a tile of 128 x 128: us, and us per term of K, with a CU to itself and beside another (fitted to 12 products)
-    F32_TILE_ALONE, F32_TILE_PAIR = (3.0, 0.060), (25.0, 0.1215)
+    F32_TILE_US_PER_TERM = 0.067  # a tile of 128 x 128 results takes this long per term of K with a CU to itself
 
     def _f32_shares(self, M, N, K):
         """Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated
@@ -670,14 +668,9 @@ class ProductOps:
         rows = 32 if M <= 64 else 128
         tiles = -(-M // rows) * -(-N // 128)
         best, least, segments = 1, float("inf"), -(-K // self.F32_SEGMENT)
-
-        def two_a_cu(items, terms):                  # rounds of two tiles a CU, the last one of single ones if they suffice
-            alone, pair = (us + per * terms for us, per in (self.F32_TILE_ALONE, self.F32_TILE_PAIR))
-            whole, rest = divmod(items, 2 * self._num_cus)
-            return whole * pair + (0.0 if not rest else alone if rest <= self._num_cus else pair)
         for s in range(1, min(16, segments) + 1):
             terms = min(K, -(-segments // s) * self.F32_SEGMENT)          # of the longest share
-            us = two_a_cu(tiles * s, terms) if rows == 128 else -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM / 4
+            us = -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM * (rows / 128)
             if s > 1:
                 us += 5.0 + (s + 1) * M * N * 4 / 3e6
             if us < 0.97 * least:

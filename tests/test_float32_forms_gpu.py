@@ -104,6 +104,21 @@ def test_products_in_chunks_of_32(M, N, K):
         assert ((got.double() - want).abs() <= min(K, 512) * 2.0 ** -24 * size).all()
 
 
+# two row tiles of 256 to 385 column tiles: whole rounds of two workgroups a CU, one tile more, at most one a CU and one more than that
+@pytest.mark.parametrize("columns", [256, 257, 384, 385])
+@pytest.mark.parametrize("K,shares", [(96, 1), (544, 1), (544, 2)])
+def test_products_around_rounds_of_tiles(columns, K, shares):
+    ops = HipOps(torch.float32, DEV)
+    M, N = 129, columns * 128 // shares - 1
+    g = torch.Generator().manual_seed(columns)
+    x, w, b = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV), torch.randn(N, generator=g).to(DEV)
+    ops._f32_shares = lambda *_: shares
+    got = ops.linear_f32_mfma(x, w, b).double()
+    want, size = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    # running sums of up to 512 products: no further off than 512 roundings of 2^-24 of their absolute sum
+    assert ((got - want).abs() <= min(K, 512) * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,D", [(12, 2, 128), (14, 2, 64), (20, 2, 64), (2, 1, 128)])
 @pytest.mark.parametrize("page,window", [(16, None), (32, 40), (64, 5)])
