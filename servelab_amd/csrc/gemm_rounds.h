@@ -208,7 +208,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rounds_kernel(
         bf16x8 h;                          // (gate and up rows lie in blocks of eight: gates first, then their ups)
         if (act == SL_ACT_SILU) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) h[e] = (__bf16)(fast_silu(r[e >> 2][e & 3]) * r[2 + (e >> 2)][e & 3]);
+          for (int e = 0; e < 8; ++e) h[e] = (__bf16)(sl_act(r[e >> 2][e & 3], SL_ACT_SILU) * r[2 + (e >> 2)][e & 3]);
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) h[e] = (__bf16)(sl_act(r[e >> 2][e & 3], act) * r[2 + (e >> 2)][e & 3]);

@@ -209,3 +209,35 @@ def test_tiles_of_256_rows_are_as_those_of_128(T, E, top, ff, K):
                 r = [hip.route_tokens(logits, E, top, tile_rows=rows) for rows in (128, 256)]
                 narrow, wide = (hip.routed_experts(x, q, a, b, activation=act, gated=gated, weigh_input=weigh) for q in r)
                 assert torch.equal(narrow, wide)
+
+
+# three and six rows an expert, some hundred in row tiles of each height
+@pytest.mark.parametrize("T,rows", [(3, 16), (7, 16), (40, 16), (400, 16), (400, 128), (400, 256)])
+@pytest.mark.parametrize("tiled", [True, False])
+def test_every_gate_of_an_expert_is_its_sigmoid_times_itself(T, rows, tiled):
+    """Rows of x that pick a column of the gate matrix, which holds every bfloat16 from -200 to 200 of 2^-20 and more; the second product hands
+    its input on."""
+    hip = HipOps(torch.bfloat16, DEV)
+    size = 512
+    halves = torch.arange(-32768, 32768).to(torch.int16).view(torch.bfloat16)
+    halves = halves[(halves.float().abs() <= 200) & (halves.float().abs() >= 2.0 ** -20)]
+    strong = halves[(halves < -80) & (halves >= -130)]                 # (in every column, so that the first three hold them too)
+    gate = torch.empty(size, size, dtype=torch.bfloat16)
+    gate[:len(strong)] = strong[:, None]
+    rest = size - len(strong)
+    gate[len(strong):] = halves.repeat(-(-rest * size // len(halves)))[:rest * size].view(size, rest).T
+    assert len(strong) > 90 and set(gate.view(torch.int16).flatten().tolist()) == set(halves.view(torch.int16).tolist())
+    up = torch.zeros_like(gate) + 1.5
+    x = torch.zeros(T, size, device=DEV).bfloat16()
+    x[torch.arange(T), torch.arange(T)] = 1
+    first, second = torch.cat([gate, up])[None].to(DEV), torch.eye(size, device=DEV).bfloat16()[None]
+    if tiled:
+        first, second = hip.prepare_expert_matrices(first, True), hip.prepare_expert_matrices(second)
+    r = hip.route_tokens(torch.zeros(T, 1, device=DEV), 1, 1, tile_rows=rows)
+    got = hip.routed_experts(x, r, first, second).double().cpu()
+    z = gate.double().T[:T]
+    want = 1.5 * z / (1 + torch.exp(-z))
+    assert got.isfinite().all()
+    # two roundings to bfloat16, of what lies between the products and of the result; zero where e^-z is no float any more
+    assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -120).all()
+    assert (got[z < -88.7229] == 0).all()

@@ -52,6 +52,35 @@ def test_gates_that_are_not_ordinary_numbers():
     assert torch.equal(got[want.isinf()], want[want.isinf()])
 
 
+def gates_to_sweep():
+    """Every bfloat16 from -200 to 200 of 2^-20 and more, floats closely around where e^-z passes the largest float and its half, and
+    between."""
+    halves = torch.arange(-32768, 32768).to(torch.int16).view(torch.bfloat16).float()
+    halves = halves[(halves.abs() <= 200) & (halves.abs() >= 2.0 ** -20)]
+    near = [(torch.tensor(z).view(torch.int32) + torch.arange(-300, 300, dtype=torch.int32)).view(torch.float32)
+            for z in (-88.7228394, -88.0296936, -87.3365479)]
+    return torch.cat([halves, *near, torch.linspace(-131.0, -79.0, 4001), -torch.logspace(2.0, 38.5, 200)])
+
+
+@pytest.mark.parametrize("rows", [128, 192, 256])
+def test_every_gate_is_its_sigmoid_times_itself(rows):
+    ops = HipOps(torch.bfloat16, DEV)
+    gates = gates_to_sweep()
+    gates = torch.cat([gates, gates.new_ones(-len(gates) % 8)])
+    N = 2 * len(gates)
+    bias = torch.full((N // 16, 2, 8), 1.5)
+    bias[:, 0] = gates.view(-1, 8)
+    x, w = torch.zeros(3, 64, device=DEV).bfloat16(), torch.zeros(N, 64, device=DEV).bfloat16()
+    got = ops.linear_gated_block(x, ops.prepare_weight(w), bias.view(-1).to(DEV), rows, 1).double().cpu()
+    z = gates.double()
+    want = 1.5 * z / (1 + torch.exp(-z))
+    assert got.isfinite().all()
+    # one rounding to bfloat16; below -88.72, where e^-z is no float any more, the result is zero instead of 1.5 x 2.6e-37 at most
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -120).all()
+    below = z < -88.7229
+    assert below.sum() > 1000 and (got[:, below] == 0).all()
+
+
 def test_routes_by_estimated_rate():
     ops = HipOps(torch.bfloat16, DEV)
     tiles = ops._prompt_tiles
