@@ -7,6 +7,7 @@
 //                 rows of x at a time.
 //   sl_gemm_tiled any M: 64x64 LDS tiles, 4x4 outputs per thread.
 #include "common.h"
+#include "k_steps.h"
 #include "lds_loads.h"
 #include <type_traits>
 
@@ -790,7 +791,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
   const int th = PRODUCER ? F.th : 16;
   const int ntiles = (N + th - 1) / th;
   const int KT = K / 32;
-  const int ks0 = (int)((long long)KT * wave / WAVES), ks1 = (int)((long long)KT * (wave + 1) / WAVES);
+  const int ks0 = first_k_step(KT, wave, WAVES), ks1 = first_k_step(KT, wave + 1, WAVES);
   const __bf16* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -966,8 +967,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
     extern __shared__ __bf16 merged[];                        // [M][K]
     auto w_of = [&](int k) { return stream_load(wp[0] + (size_t)32 * th * k); };
     bf16x8 a[KB];
-#pragma unroll
-    for (int u = 0; u < KB; ++u) a[u] = w_of(ks0 + u < ks1 ? ks0 + u : ks1 - 1);
+    ask_ahead<KB>(ks0, ks1, [&](int u, int k) { a[u] = w_of(k); });
     for (int c = threadIdx.x; c < M * K; c += 64 * WAVES) {
       const size_t at = (size_t)(c >> R.head_bits) * R.shares;          // (rows of K values: whole heads)
       const float* o = R.o + (at << R.head_bits) + (c & ((1 << R.head_bits) - 1));
@@ -1437,7 +1437,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(
   const int ntiles = (N + 15) / 16;
   const int tile0 = blockIdx.x * NT;
   const int KT = K / 32;
-  const int ks0 = (int)((long long)KT * wave / WAVES), ks1 = (int)((long long)KT * (wave + 1) / WAVES);
+  const int ks0 = first_k_step(KT, wave, WAVES), ks1 = first_k_step(KT, wave + 1, WAVES);
   const __bf16* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
