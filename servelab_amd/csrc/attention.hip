@@ -339,8 +339,9 @@ __global__ __launch_bounds__(64) void attention_few_keys_kernel(
       d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0xB1, 0xf, 0xf, true));
       d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x4E, 0xf, 0xf, true));
       const float sc = valid ? d * scale : -INFINITY;
-      const float mn = fmaxf(m[h], over_keys<true>(sc));        // every block holds a visible key
-      const float alpha = expf(m[h] - mn), pr = valid ? expf(sc - mn) : 0.f;      // exp(-inf) = 0 on the first block
+      const float mn = fmaxf(m[h], over_keys<true>(sc));
+      const float from = mn == -INFINITY ? 0.f : mn;            // (16 keys may well have no score above minus infinity: they weigh nothing)
+      const float alpha = expf(m[h] - from), pr = valid ? expf(sc - from) : 0.f;  // exp(-inf) = 0 on the first block
       l[h] = l[h] * alpha + over_keys<false>(pr);
       m[h] = mn;
       if (part == 0) ps[h][key] = pr;

@@ -139,3 +139,25 @@ def test_single_tokens_in_blocks_of_16_keys(dtype, nh, nkv, D, page, window):
     got = ops.paged_attention(qkv, nh, nkv, D, kc, vc, page, tables, batch, D ** -0.5, window)
     # float32 scores of 128 products and sums over at most 1,100 keys; bfloat16: one rounding
     assert float((got.float().cpu() - want.float()).abs().max()) <= (3e-6 if dtype == torch.float32 else 2.0 ** -7) * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,unseen", [(64, [(0, 16)]), (128, [(0, 48)]), (64, [(16, 32), (96, 112)])])
+def test_single_tokens_with_blocks_of_keys_that_weigh_nothing(dtype, D, unseen):
+    """Scores of minus infinity for whole blocks of 16 keys, the first of a share among them: they weigh nothing."""
+    ops = HipOps(dtype, DEV)
+    ops.use_mfma_attention, ops.GENERAL_ATTENTION_WAVES = False, 1024
+    nh, nkv, n = 4, 2, 250
+    qkv, kc, vc, tables, batch = make_attention_case(dtype, nh, nkv, D, 16, [(n, 1)])[:5]
+    qkv[0, :nh * D:D] = 1.0
+    keys, values = kc[tables[0].long()].transpose(1, 2).reshape(-1, nkv, D), vc[tables[0].long()].permute(0, 3, 1, 2).reshape(-1, nkv, D)
+    for first, behind in unseen:
+        for k in range(first, behind):
+            kc[int(tables[0, k // 16]), :, k % 16, 0] = float("-inf")
+            keys[k, :, 0] = float("-inf")
+    got = ops.paged_attention(qkv, nh, nkv, D, kc, vc, 16, tables, batch, D ** -0.5, None).double().cpu()
+    q = qkv[0, :nh * D].double().cpu().view(nkv, nh // nkv, D)
+    scores = torch.einsum("ghd,kgd->ghk", q, keys[:n].double().cpu()) * D ** -0.5
+    want = torch.einsum("ghk,kgd->ghd", scores.softmax(-1), values[:n].double().cpu()).reshape(1, nh * D)
+    # float32 scores of 128 products and sums over at most 250 keys; bfloat16: one rounding
+    assert float((got - want).abs().max()) <= (3e-6 if dtype == torch.float32 else 2.0 ** -7) * max(1.0, float(want.abs().max()))
