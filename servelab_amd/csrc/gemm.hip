@@ -622,8 +622,10 @@ __global__ __launch_bounds__(256) void f32_shares_kernel(const float* __restrict
 // 1,260 208 / 195, 768 of 1,024 272 / 226; not at 1,152 of 512 184 / 195, 672 of 1,024 210 / 225, 1,280 of 1,024 352 / 370,
 // 700 of 1,536 307 / 328.
 static bool f32_last_round_of_threes(long long triples, int terms) {
-  const long long cus = device_cus(), whole = triples / (2 * cus), rest = triples % (2 * cus);
-  if (terms > 1024 || rest == 0 || rest > cus) return false;
+  const long long cus = device_cus();
+  if (cus <= 0 || terms > 1024) return false;                          // (no answer: the ring does not depend on it)
+  const long long whole = triples / (2 * cus), rest = triples % (2 * cus);
+  if (rest == 0 || rest > cus) return false;
   const bool most = 4 * rest > 3 * cus;
   return terms <= 512 ? whole == 1 || (whole == 2 && most) : whole == 1 && most;
 }
