@@ -2194,12 +2194,12 @@ static void rounds(const __bf16* x, const __bf16* w, const float* bias, void* y,
 // ks > 1: `part` holds ks * M * N floats; with y == nullptr they are left
 // there for the reader to add (and the bias with them), else splitk_reduce adds them into y.
 // square: rows of x a tile, 256, 192 or 128, by 256 of W (gemm_rounds.h); 0: tiles of 256 x 128, which take
-// any N and stand in where the others' stores of 16 bytes do not fit.
+// any N and stand in where the others' stores of 16 bytes or their offsets of 32 bits do not fit.
 extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* bias, void* y,
                                      int M, int N, int K, int out_f32, int gated, int act, int ks, int square, float* part,
                                      hipStream_t stream) {
   SL_CHECK(M > 0 && N > 0 && K > 0, "gemm_block: sizes must be positive");
-  SL_CHECK(K % 64 == 0 && K <= (1 << 22), "gemm_block: K must be a multiple of 64, 4 M at most");
+  SL_CHECK(K % 64 == 0, "gemm_block: K must be a multiple of 64");
   SL_CHECK(ks >= 1 && ks <= 64 && ks <= K / 64, "gemm_block: ks must be in 1..64 and <= K / 64");
   SL_CHECK(ks == 1 || part != nullptr, "gemm_block: a split of K needs the partial buffer");
   SL_CHECK(y != nullptr || ks > 1, "gemm_block: no output");
@@ -2208,7 +2208,10 @@ extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* 
            "gemm_block: a gated product takes wide tiles, whole rows of K, blocks of eight and bfloat16 results");
   SL_CHECK(!act || (square && ks == 1 && !out_f32 && !gated && N % 8 == 0),
            "gemm_block: an activation takes wide tiles, whole rows of K, bfloat16 results and columns in eights");
-  if (N % (out_f32 || ks > 1 ? 4 : 8)) square = 0;       // (the wide tiles store 16 bytes at a time; the others any number)
+  // (the wide tiles store 16 bytes at a time and reach 255 rows of W from their first with 32 bits; the others any number)
+  const bool wide = (uintptr_t)(ks > 1 ? (void*)part : y) % 16 == 0 && K <= (1 << 22);
+  SL_CHECK(wide || !(gated || act), "gemm_block: a gate or an activation takes results on 16 bytes and K of 4 M at most");
+  if (!wide || N % (out_f32 || ks > 1 ? 4 : 8)) square = 0;
   SL_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_block: x and W must be 16-byte aligned");
   void* dst = ks > 1 ? (void*)part : y;
   const float* b = ks > 1 ? nullptr : bias;

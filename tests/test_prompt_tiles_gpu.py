@@ -1,9 +1,11 @@
 """Products of prompts on workgroups that walk their tiles (gemm_rounds.h), where a workgroup takes several tiles, where a tile is
 one chunk of K, and the activation at values that are not ordinary numbers."""
+import ctypes
+
 import pytest
 import torch
 
-from servelab_amd.kernels import HipOps
+from servelab_amd.kernels import HipOps, KernelError
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -143,3 +145,23 @@ def test_tuned_shapes_whose_tiles_are_faster_still():
     assert ops._tiles_beat_tuned(*shape) and not ops._tiles_beat_tuned(*small)
     ops._tuned, ops._tuning = set(), True
     assert ops._tiles_beat_tuned(*shape) and not ops._tiles_beat_tuned(*small)
+
+
+def test_products_that_the_wide_tiles_cannot_take():
+    """Rows whose offsets pass 32 bits, and results that start 8 bytes past a multiple of 16: the tiles of 256 x 128 stand in."""
+    ops = HipOps(torch.bfloat16, DEV)
+    K = (1 << 22) + 64
+    x, w = torch.randn(2, K, device=DEV).bfloat16(), torch.randn(8, K, device=DEV).bfloat16()
+    got = ops.linear_block(x, w, None, ks=1, partial=True, square=True).parts[0].double()
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # 131,074 additions in a row, each off by 2^-24 of the absolute sum at most: 2^-15.5 of it as a random walk, 2^-13 with room
+    assert ((got - want).abs() <= 2.0 ** -13 * size).all()
+    x, w = torch.randn(257, 128, device=DEV).bfloat16(), torch.randn(264, 128, device=DEV).bfloat16()
+    y = torch.zeros(257 * 264 + 4, device=DEV).bfloat16()[4:].view(257, 264)
+    assert y.data_ptr() % 16 == 8
+    ops._call("gemm", "sl_gemm_block", *(ctypes.c_void_p(v.data_ptr()) for v in (x, w)), None, ctypes.c_void_p(y.data_ptr()),
+              257, 264, 128, 0, 0, 0, 1, 256, None)
+    assert torch.equal(y, ops.linear_block(x, w, None))
+    with pytest.raises(KernelError, match="16 bytes"):
+        ops._call("gemm", "sl_gemm_block", *(ctypes.c_void_p(v.data_ptr()) for v in (x, w)), None, ctypes.c_void_p(y.data_ptr()),
+                  257, 264, 128, 0, 0, 3, 1, 256, None)
