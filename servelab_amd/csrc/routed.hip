@@ -273,11 +273,6 @@ __device__ __forceinline__ bool grouped_place(const Grouped& a, int& tile, int& 
   return true;
 }
 
-// Row tiles of 128 rows instead take only the tiles in use, and every column block of a tile before the next tile.  A die
-// then reads a tile's rows of x once for all of its columns, and has two or three experts' matrices under way (64 experts of
-// 2,048 x 1,024, gate/up, down and the sum, 8 of them a token: 256 / 1,000 / 2,048 tokens 196 / 254 / 360 us by column
-// blocks, 162 / 231 / 359 by tiles).
-
 // 256 threads: thread (row = tid / 16, lane16 = tid % 16) owns columns lane16 + 16 u, u < 4, of a
 // 16 x 64 tile.  x and W go through LDS in chunks of 32 values of k; sums are float.
 template <bool GATED>
@@ -549,7 +544,8 @@ __global__ __launch_bounds__(512, 2) void grouped_product_walk_kernel(const Grou
   __shared__ int what[BATCH][4];                        // expert, first row, rows, column block
   __shared__ int found;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wm = wave >> 2, wn = wave & 3;
-  // (every column block of a tile before the next tile; a die's items are a contiguous run, a workgroup takes every `step`-th of them)
+  // Only the tiles in use, every column block of a tile before the next tile: a die, whose items are a contiguous run, reads a tile's
+  // rows of x once for all of its columns and has two or three experts' matrices under way.  A workgroup takes every `step`-th.
   const int total = (a.used != nullptr ? min(*a.used, a.max_tiles) : a.max_tiles) * a.col_blocks, run = (total + 7) / 8;
   const int first = (int)(blockIdx.x & 7) * run, end = min(first + run, total), step = (int)gridDim.x >> 3;
   const int chunks = a.K / 64;
@@ -736,11 +732,12 @@ __global__ __launch_bounds__(512, 2) void grouped_product_walk_kernel(const Grou
         if constexpr (GATED) {
           const int n = n0 + 32 * wn + 8 * gq;
           rt_bf16x8 h;
+          auto gate = [&](int act) {
 #pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            const float g = z[c >> 2][c & 3], up = z[2 + (c >> 2)][c & 3];
-            h[c] = (__bf16)sl_gated(g, up, a.act, a.limit);
-          }
+            for (int c = 0; c < 8; ++c) h[c] = (__bf16)sl_gated(z[c >> 2][c & 3], z[2 + (c >> 2)][c & 3], act, a.limit);
+          };
+          if (a.act == SL_ACT_SILU) gate(SL_ACT_SILU);  // (no branches between the eight chains of operations)
+          else gate(a.act);
           if (n < a.N) *(rt_bf16x8*)(a.out_act + at + n) = h;
         } else if constexpr (HALF) {
 #pragma unroll
