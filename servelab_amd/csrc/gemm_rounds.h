@@ -4,8 +4,8 @@
 // What bounds it: power.  The matrix units alone, on random data, run 2.0 PFLOP/s at 2.1 GHz with v_mfma_f32_16x16x32 and
 // 1.7 at 1.75 GHz with v_mfma_f32_32x32x16 (2.43 at 2.4 GHz on zeros), so what counts beside the cycles is what else moves.
 // A chunk of 64 values of k (2,048 cycles of matrix work for T = 4) takes 2,350 to 2,450 cycles at 1.8 to 1.9 GHz; without
-// the loads it takes 2,130, without the LDS reads as well 2,080.  2,048 rows: 37888 x 3584 gated 496 -> 420 us (1.32
-// PFLOP/s), 3584 x 18944 in two shares of K 247 -> 220 us, against sixteen wavefronts of 64 x 64 each, which loaded, read and
+// the loads it takes 2,130, without the LDS reads as well 2,080.  2,048 rows: 37888 x 3584 gated 512 -> 465 us (1.20
+// PFLOP/s; 1.30 on another card), 13 us of them the activation, which nothing runs beside, 3584 x 18944 in two shares of K 247 -> 220 us, against sixteen wavefronts of 64 x 64 each, which loaded, read and
 // multiplied a chunk in turn behind one barrier.
 //
 //  - The order of a chunk is laid down instruction by instruction: products of operands that arrived before the last

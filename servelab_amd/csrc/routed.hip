@@ -527,9 +527,9 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void grouped_product_few_kernel(con
 // work ahead do not cover that (about 1.1 us a chunk whatever the order of the items; a chunk of 256 rows takes 1.3).
 // The trips that start an item (its row tile, where its rows lie, the rows) are as long as several chunks, so a workgroup
 // looks up BATCH items ahead and its loads run on from one item into the next.
-// A prompt of 2,048 tokens, 8 of 64 experts of 1,024 over rows of 2,048 a token: gate/up 229 -> 176 us, down 134 -> 111 (of which
+// A prompt of 2,048 tokens, 8 of 64 experts of 1,024 over rows of 2,048 a token: gate/up 232 -> 177 us, down 134 -> 109 (of which
 // its 134 MB of float rows and 268 MB of matrices are 70), against an item a workgroup, 128 rows each, and a ring of three whole chunks
-// behind one barrier; 128 rows walked like this: 196 and 118.
+// behind one barrier; 128 rows walked like this: 209 and 126.
 // Halves of the rows without a pair are not multiplied.  HALF: results in bfloat16, and the rows of W are picked from two tiles
 // so that a lane holds eight columns in a row; odd tiles lie in LDS with their rows four places on, off the other's banks.
 template <int R, bool GATED, bool HALF>

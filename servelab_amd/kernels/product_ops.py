@@ -342,11 +342,11 @@ class ProductOps:
         was with sixteen wavefronts: 24 layers of the 0.5B shape, 9728 x 896, 260 / 600 / 1,000 / 1,700 / 2,048 tokens 4,893 / 4,194,
         3,837 / 3,356, 4,116 / 3,604, 4,184 / 3,901 and 4,381 / 4,191 us; 12 layers of 4096 x 1024, 256 and
         2,048 tokens 2,063 / 1,823 and 2,133 / 1,862).  By GPU time alone it wins there as well now (9728 x 896, 300 / 1,000 /
-        1,600 / 2,048 rows 38 / 19, 35 / 22, 60 / 38 and 66 / 40 us).  Rows of up to GATED_ONE_ROUND_K values take it where one
-        round of tiles is GATED_FILL useful (17920 x 1536, 527 / 640 / 768 rows 38 / 31, 43 / 38 and 46 / 39 us a product), and
+        1,600 / 2,048 rows 35 / 22, 37 / 25, 43 / 42 and 59 / 43 us).  Rows of up to GATED_ONE_ROUND_K values take it where one
+        round of tiles is GATED_FILL useful (17920 x 1536, 527 / 640 / 768 rows 38 / 33, 45 / 41 and 47 / 42 us a product), and
         longer ones, up to GATED_LONG_K values at GATED_LONG_ROWS rows of x, in several rounds of tiles of 256 x 256 whose last
         one is filled by GATED_LAST_ROUND where neither 192 nor 224 divides N, at which the library's picks idle (2,048 rows of
-        37888 x 3584 542 / 422, of 22016 x 2048 196 / 151).  The sums meet the activation unrounded, so that it
+        37888 x 3584 543 / 429, of 22016 x 2048 193 / 153).  The sums meet the activation unrounded, so that it
         is the more exact form as well.  Shapes that were tuned may stay with the library (``_tiles_beat_tuned``)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
                 or N < self.GATED_MIN_N or M > self.GATED_MAX_M):
@@ -364,8 +364,9 @@ class ProductOps:
         return 256 if fits else None
 
     # rows of x a tile -> us of a launch, of a round of tiles, of a chunk of 64 values of k with few CUs busy, and what all of
-    # them add to a chunk (they share the power): fitted to 168 gated products of 12 shapes, 260 to 2,048 rows of x; 3 % rms, 12 % at worst
-    # (the ones of 128 rows, with six halves on the way where the others have four, to 20)
+    # them add to a chunk (they share the power): fitted to 168 gated products of 12 shapes, 260 to 2,048 rows of x, with a cheaper activation than is taken
+    # now; against 153 of them as they are 4 % rms and 12 % at worst (7 and 15 for the ones of 128 rows, with six halves on the way where
+    # the others have four) but for rows of 896 values, which take up to a fifth longer, and no other choice would gain more than 0.1 % on average
     TILE_US = {256: (1.8, 6.0, 0.92, 0.49), 192: (2.5, 4.0, 0.74, 0.39), 128: (1.0, 3.5, 0.68, 0.20)}
 
     def _tiles_us(self, rows, M, N, K, ks=1):
@@ -376,17 +377,17 @@ class ProductOps:
         return launch + rounds * (tile + K / ks / 64 * (chunk + shared * items / (rounds * self._num_cus)))
 
     def _tile_rows(self, M, N, K, ks=1):
-        """Rows of x a workgroup takes, the ones that take the least time by estimate (256 or 192: of the 168 products 0.04 %
-        slower on average than the better one of both, 2 % at worst; 128 where those leave CUs idle: 22016 x 2048 at 527 / 640 rows
-        72 / 56 and 77 / 57 us, 9216 x 3584 at 768 58 / 46)."""
+        """Rows of x a workgroup takes, the ones that take the least time by estimate (of 125 products 0.12 % slower on average than the best height,
+        9 % at worst, 1000 x 22016 x 2048; 128 where the others leave CUs idle: 22016 x 2048 at 527 / 640 rows
+        75 / 58 us both times, 9216 x 3584 at 768 57 / 48)."""
         return min(self.TILE_US, key=lambda rows: self._tiles_us(rows, M, N, K, ks))
 
     def _prompt_tiles(self, M, N, K):
         """Rows of x a tile for a product of a prompt whose results the library would leave to a second pass (a gate or an
         activation), or None where its product and the pass are the faster pair: where the tiles' estimated rate is below
-        PROMPT_MIN_TFLOPS, which is where they leave CUs idle.  Over the 168 products (rows of 896 to 5,120 values) the
-        kernel at 750 and more takes 0.90 of the pair's time on average, 1.12 at worst (640 x 28672 x 4096, 148 against 141
-        us); at 700 9216 x 3584 with 640 rows of x is among them (56 against 45), at 900 the average is 0.92."""
+        PROMPT_MIN_TFLOPS, which is where they leave CUs idle.  Of 153 products (rows of 896 to 5,120 values) the
+        kernel at 750 and more takes 0.91 of the pair's time on average, 1.11 at worst (600 x 27648 x 3584, 128 against 116
+        us); at 700 9216 x 3584 with 640 rows of x is among them (56 against 45)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 16
                 or N < self.GATED_MIN_N or not self.GATED_MIN_M <= M <= self.GATED_MAX_M or K > self.PROMPT_MAX_K):
             return None
@@ -402,8 +403,8 @@ class ProductOps:
     def _tiles_beat_tuned(self, M, N, K) -> bool:
         """Whether a gated or activated product that may take the tiles does: a shape that was tuned stays with the library and its
         pass below an estimated rate of PROMPT_TUNED_TFLOPS.  From there on the tiles are the faster pair also against the tuned pick
-        (us, tuned / tiles: 37888 x 3584 at 544 / 1,024 / 2,048 rows 172 / 138, 269 / 246 and 456 / 458, 22016 x 2048 at 2,048 184 /
-        157, 17920 x 1536 136 / 121, 55296 x 5120 951 / 865, 28672 x 4096 397 / 375, 18944 x 3584 with relu squared 263 / 267)."""
+        (us, tuned / tiles: 37888 x 3584 at 544 / 1,024 / 2,048 rows 176 / 150, 279 / 259 and 469 / 475, 22016 x 2048 at 2,048 187 /
+        169, 17920 x 1536 137 / 130, 55296 x 5120 973 / 909, 28672 x 4096 407 / 394, 18944 x 3584 with relu squared 267 / 273)."""
         return not self._tuned_for(M, N, K) or 2e-6 * M * N * K >= self.PROMPT_TUNED_TFLOPS * self._tiles_us(self._tile_rows(M, N, K), M, N, K)
 
     @staticmethod

@@ -436,8 +436,9 @@ class RecurrentOps:
 
     # ------------------------------------------------------- routed experts
     def expert_tile_rows(self, pairs, w_gate_up, gated=True):
-        """Rows of a row tile (16 or 128) for a step of ``pairs`` (token, choice) pairs over the experts of ``w_gate_up``:
-        what ``route_tokens`` takes as ``tile_rows``."""
+        """Rows of a row tile for a step of ``pairs`` (token, choice) pairs over the experts of ``w_gate_up``: what
+        ``route_tokens`` takes as ``tile_rows``.  16, or 128 from so many rows an expert on as the lines above say, or 256 where an expert
+        has ROUTED_TALL_TILE_ROWS, the matrices are tiled, K is a multiple of 64 and two rounds of such tiles fill the CUs."""
         experts, N, K = w_gate_up.shape
         blocks = -(-(N // 2 if gated else N) // 128)
         few = experts < self.ROUTED_WIDE_EXPERTS or experts * blocks < self.ROUTED_WIDE_WORKGROUPS

@@ -92,8 +92,8 @@ class Tuning:
     block_square_max_m: int = 1536
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
-    # gated products of a prompt in the block kernel (measured sides: HipOps._gated_rows): the fewest rows of W, the
-    # fewest and the most rows of x; rows of up to gated_short_k values, or up to gated_one_round_k in one round of tiles of
+    # gated and activated products of a prompt in the tiles of gemm_rounds.h (measured sides: HipOps._gated_rows): the fewest rows
+    # of W, the fewest and the most rows of x; rows of up to gated_short_k values, or up to gated_one_round_k in one round of tiles of
     # which so much is useful; ...
     gated_min_n: int = 4096
     gated_min_m: int = 256
