@@ -2,8 +2,8 @@
 // the host.
 #pragma once
 
-// Wavefront `wave` of `waves` takes k-steps [first_k_step(wave), first_k_step(wave + 1)) of `steps`: none where there are fewer
-// steps than wavefronts before it.
+// Wavefront `wave` of `waves` takes k-steps [first_k_step(wave), first_k_step(wave + 1)) of `steps`; with
+// fewer steps than wavefronts some have none.
 constexpr int first_k_step(int steps, int wave, int waves) { return (int)((long long)steps * wave / waves); }
 
 // What a wavefront of [first, behind) asks for ahead of its loop: load(u, k) for the first N of its k-steps, the last one again past
