@@ -739,7 +739,6 @@ struct NormFusion {
   // and its re-read of x, so a matrix whose 16-row tiles do not go round the CUs evenly gets lower tiles
   // that do (N = 5120 on 256 CUs: 512 tiles of 10 rows instead of 320 of 16).  Other forms: 16.
   int th;
-  int pair_x;                // at most 8 rows and one tile a workgroup: a load of x takes two k-steps (see stream_k2)
   int gate_act;              // gated forms: the activation of the gate (common.h: 1 silu, 2 relu); plain form: the
                              // activation of the result (0: none)
 };
@@ -771,360 +770,18 @@ struct RopeStore {
   float qscale;              // q heads are multiplied by this before their rounding (1: as they are)
 };
 
-// NT tiles (16 columns of y each) per workgroup share every load of x: with 8
-// to 16 rows the re-reads of x through L1 are a third to a half of all bytes a
-// CU pulls, and halving them shows (MI355X, gate/up of the 7B shape at 16 rows:
-// 66 us with one tile).  Matrices with few tiles keep one tile per workgroup so
-// that every CU has work.
-template <bool GATED, bool CONSUMER, bool PRODUCER, int PARTS, bool ROPE = false, int NT = 1, int WAVES = 8, bool SHARES = false>
-__global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(
-    const __bf16* __restrict__ x, const __bf16* __restrict__ wt, const float* __restrict__ bias,
-    void* __restrict__ y, int M, int N, int K, int out_f32, const NormFusion F,
-    const std::conditional_t<SHARES, KeyShares, RopeStore> R) {
-  constexpr int U = NT == 1 ? 8 : 4;
-  static_assert(WAVES == 8 || !CONSUMER, "the shares of the sums of squares are laid out for 512 threads");
-  __shared__ f32x4 red[NT][WAVES][64];
-  __shared__ float wsum[WAVES][16];
-  // the wavefront's index as a scalar: what depends on it (its share of K, its tiles) then steers
-  // real branches; matrix instructions ignore the execution mask, so they must not sit under a
-  // condition the compiler takes for divergent and may turn into masking
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int lane = threadIdx.x % 64, i = lane & 15, gq = lane >> 4;
-  const int th = PRODUCER ? F.th : 16;
-  const int ntiles = (N + th - 1) / th;
-  const int KT = K / 32;
-  const int ks0 = first_k_step(KT, wave, WAVES), ks1 = first_k_step(KT, wave + 1, WAVES);
-  const __bf16* wp[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int tile = blockIdx.x * NT + t < ntiles ? blockIdx.x * NT + t : ntiles - 1;
-    // (lanes of rows a lower tile does not have read its last row; their columns of the result are dropped)
-    wp[t] = wt + ((size_t)tile * KT * (4 * th) + gq * th + (i < th ? i : th - 1)) * 8;
-  }
-  int xrow = i < M ? i : M - 1;
-  if (CONSUMER && F.rows != nullptr) xrow = F.rows[xrow];
-  const __bf16* xp = F.x_tiled ? x + (size_t)xrow * 32 + 8 * gq : x + (size_t)xrow * K + 8 * gq;
-  const size_t xstep = F.x_tiled ? (size_t)F.x_tiled * 32 : 32;     // elements from one k-step of a row to the next
-  // Loads that only the epilogue needs are issued here, before W streams, so
-  // that their latency is hidden: the consumer's share of the sums of squares
-  // (thread t takes parts t / 16, t / 16 + 32, ... of row t % 16) and the
-  // producer's elements of the stream and of the next gain.
-  float pv[PARTS];
-  if (CONSUMER) {
-#pragma unroll
-    for (int j = 0; j < PARTS; ++j) {
-      const int p = threadIdx.x / 16 + 32 * j;
-      pv[j] = p < F.in_nparts ? F.in_parts[p * 16 + i] : 0.f;
-    }
-  }
-  const int em = threadIdx.x / 16;                                   // epilogue row of threads < 256
-  float r_old[NT], g_next[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int en = (blockIdx.x * NT + t) * th + threadIdx.x % 16;
-    r_old[t] = g_next[t] = 0.f;
-    if (PRODUCER && threadIdx.x < 256 && em < M && (int)(threadIdx.x % 16) < th && en < N) {
-      r_old[t] = F.resid[(size_t)em * N + en];
-      g_next[t] = F.next_w[en];
-    }
-  }
-  // (ROPE: the bias, the angle's cosine and sine and the cache row of this thread's element)
-  float b_pre[NT], c_pre[NT], s_pre[NT];
-  int slot_pre = 0;
-  if constexpr (ROPE) {
-    if (threadIdx.x < 256 && em < M && R.slots != nullptr) slot_pre = R.slots[em];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int en = (blockIdx.x * NT + t) * 16 + threadIdx.x % 16;
-      b_pre[t] = 0.f;
-      c_pre[t] = 1.f;
-      s_pre[t] = 0.f;
-      if (threadIdx.x < 256 && em < M && en < N) {
-        if (bias != nullptr) b_pre[t] = bias[en];
-        const int hd = en / R.D, p = en % R.D;
-        if (R.cosv != nullptr && hd < R.nh + R.nkv && p < R.rot) {
-          const int j = 8 * (p / 16) + p % 8, half = R.rot / 2;
-          c_pre[t] = R.cosv[(size_t)em * half + j];
-          s_pre[t] = R.sinv[(size_t)em * half + j];
-        }
-      }
-    }
-  }
-  f32x4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // The K loop, written once for plain rows of x (a constant step from one k-step to the next,
-  // folded into the loads' offsets) and once for rows laid out by k-step.
-  auto stream_k = [&](auto tiled_tag, auto th_tag) {
-    const size_t xs_ = decltype(tiled_tag)::value ? xstep : (size_t)32;
-    constexpr size_t WS = 32 * decltype(th_tag)::value;             // elements of W from one k-step of a tile to the next
-    int ks = ks0;
-    for (; ks + U <= ks1; ks += U) {
-      bf16x8 a[NT][U];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) a[t][u] = stream_load(wp[t] + WS * (size_t)(ks + u));
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bf16x8 bv = *(const bf16x8*)(xp + xs_ * (size_t)(ks + u));
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][u], bv, acc[t], 0, 0, 0);
-      }
-    }
-    if (ks < ks1) {
-      // the last k-steps, fewer than U: all their loads are issued before the
-      // first product, so they cost one trip to memory, not one each
-      bf16x8 a[NT][U], bv[U];
-#pragma unroll
-      for (int u = 0; u < U - 1; ++u)
-        if (ks + u < ks1) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t) a[t][u] = stream_load(wp[t] + WS * (size_t)(ks + u));
-          bv[u] = *(const bf16x8*)(xp + xs_ * (size_t)(ks + u));
-        }
-#pragma unroll
-      for (int u = 0; u < U - 1; ++u)
-        if (ks + u < ks1) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][u], bv[u], acc[t], 0, 0, 0);
-        }
-    }
-  };
-  // The same loop for at most 8 rows of x and one tile: a load of x takes two k-steps.  The matrix
-  // instruction has 16 columns for the rows of x; with at most 8 rows the lanes of columns 8..15 load the
-  // same rows one k-step further on, the products of even k-steps go to one accumulator (columns 0..7
-  // valid) and those of odd k-steps to a second (columns 8..15 valid), and the second is added to the
-  // first at the end.  Half as many loads of x: a load takes a place in the CU's queue of outstanding
-  // requests whatever its size, and that queue is what these kernels run on.
-  f32x4 acc_odd = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto stream_k2 = [&](auto tiled_tag, auto th_tag) {
-    static_assert(NT == 1 && U % 2 == 0, "two k-steps a load of x: one tile, an even number of loads in flight");
-    const size_t xs_ = decltype(tiled_tag)::value ? xstep : (size_t)32;
-    constexpr size_t WS = 32 * decltype(th_tag)::value;
-    int row = (i & 7) < M ? (i & 7) : M - 1;
-    if (CONSUMER && F.rows != nullptr) row = F.rows[row];
-    const __bf16* x0 = (F.x_tiled ? x + (size_t)row * 32 + 8 * gq : x + (size_t)row * K + 8 * gq);
-    const __bf16* x2 = x0 + (i >= 8 ? xs_ : 0);          // columns 8..15: one k-step further
-    int ks = ks0;
-    for (; ks + U <= ks1; ks += U) {
-      bf16x8 a[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) a[u] = stream_load(wp[0] + WS * (size_t)(ks + u));
-#pragma unroll
-      for (int u = 0; u < U; u += 2) {
-        const bf16x8 bv = *(const bf16x8*)(x2 + xs_ * (size_t)(ks + u));
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], bv, acc[0], 0, 0, 0);
-        acc_odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u + 1], bv, acc_odd, 0, 0, 0);
-      }
-    }
-    if (ks < ks1) {
-      // the last k-steps, fewer than U, in one trip to memory; an odd one at the end has its x in all
-      // 16 columns (nothing lies one k-step further that would be this wavefront's, or the row's)
-      bf16x8 a[U], bv[U / 2], last;
-#pragma unroll
-      for (int u = 0; u < U - 1; ++u)
-        if (ks + u < ks1) a[u] = stream_load(wp[0] + WS * (size_t)(ks + u));
-#pragma unroll
-      for (int u = 0; u + 1 < U - 1; u += 2)
-        if (ks + u + 1 < ks1) bv[u / 2] = *(const bf16x8*)(x2 + xs_ * (size_t)(ks + u));
-      const bool odd = (ks1 - ks) & 1;
-      if (odd) last = *(const bf16x8*)(x0 + xs_ * (size_t)(ks1 - 1));
-#pragma unroll
-      for (int u = 0; u + 1 < U - 1; u += 2)
-        if (ks + u + 1 < ks1) {
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], bv[u / 2], acc[0], 0, 0, 0);
-          acc_odd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u + 1], bv[u / 2], acc_odd, 0, 0, 0);
-        }
-      if (odd) {
-        // (its W is a[ks1 - 1 - ks]: picked by a chain of selects, the index is the same for the wavefront)
-        bf16x8 w_last = a[0];
-#pragma unroll
-        for (int u = 1; u < U - 1; ++u)
-          if (ks + u == ks1 - 1) w_last = a[u];
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_last, last, acc[0], 0, 0, 0);
-      }
-    }
-  };
-  // (each form of the loop is straight-line code with constant steps; the tile height is a run-time
-  // choice only for producers)
-  auto stream_th = [&](auto th_tag) {
-    if constexpr (NT == 1) {
-      if (M <= 8 && F.pair_x) {
-        if (F.x_tiled) stream_k2(std::true_type{}, th_tag);
-        else stream_k2(std::false_type{}, th_tag);
-        return;
-      }
-    }
-    if (F.x_tiled) stream_k(std::true_type{}, th_tag);
-    else stream_k(std::false_type{}, th_tag);
-  };
-  if constexpr (SHARES) {
-    // A thread merges the shares of a channel, everything it needs asked for at once behind the first of W, into rows of
-    // bfloat16 in LDS.  (Merged by the lanes that multiply, sixteen (row, share) pairs to a load, it took 7 us a layer of the 0.5B
-    // shape more than the merging kernel that it saves.)
-    constexpr int KB = 4, J = SL_MAX_SHARES;
-    extern __shared__ __bf16 merged[];                        // [M][K]
-    auto w_of = [&](int k) { return stream_load(wp[0] + (size_t)32 * th * k); };
-    bf16x8 a[KB];
-    ask_ahead<KB>(ks0, ks1, [&](int u, int k) { a[u] = w_of(k); });
-    for (int c = threadIdx.x; c < M * K; c += 64 * WAVES) {
-      const size_t at = (size_t)(c >> R.head_bits) * R.shares;          // (rows of K values: whole heads)
-      const float* o = R.o + (at << R.head_bits) + (c & ((1 << R.head_bits) - 1));
-      float v[J], top = -INFINITY, sum = 0.f, all = 0.f;
-      float2 ml[J];
-#pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int q = j < R.shares ? j : R.shares - 1;
-        v[j] = o[(size_t)q << R.head_bits];
-        ml[j] = R.ml[at + q];
-      }
-#pragma unroll
-      for (int j = 0; j < J; ++j) top = fmaxf(top, ml[j].x);
-#pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const float wgt = j < R.shares && ml[j].x != -INFINITY ? __builtin_amdgcn_exp2f(ml[j].x - top) : 0.f;   // (maxima are in units of log 2)
-        all += wgt * ml[j].y;
-        sum += wgt * v[j];
-      }
-      merged[c] = (__bf16)(sum * (1.f / all));
-    }
-    __syncthreads();
-    const __bf16* row = merged + (size_t)(i < M ? i : M - 1) * K + 8 * gq;
-    for (int ks = ks0; ks < ks1; ks += KB) {
-#pragma unroll
-      for (int u = 0; u < KB; ++u) {
-        if (ks + u >= ks1) break;
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ks == ks0 ? a[u] : w_of(ks + u), *(const bf16x8*)(row + 32 * (ks + u)), acc[0], 0, 0, 0);
-      }
-    }
-  } else if constexpr (!PRODUCER) {
-    stream_th(std::integral_constant<int, 16>{});
-  } else {
-    if (th == 16) stream_th(std::integral_constant<int, 16>{});
-    else if (th == 14) stream_th(std::integral_constant<int, 14>{});
-    else if (th == 12) stream_th(std::integral_constant<int, 12>{});
-    else if (th == 10) stream_th(std::integral_constant<int, 10>{});
-    else stream_th(std::integral_constant<int, 8>{});
-  }
-  if constexpr (NT == 1 && !SHARES) {
-    if (M <= 8 && F.pair_x) {         // column m + 8 of the odd k-steps' sums belongs to column m
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[0][r] += __shfl(acc_odd[r], lane + 8, 64);
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) red[t][wave][lane] = acc[t];
-  if (CONSUMER) {            // this wavefront's share of the sums of squares, by row
-    float sacc = 0.f;
-#pragma unroll
-    for (int j = 0; j < PARTS; ++j) sacc += pv[j];
-    sacc += __shfl_xor(sacc, 16, 64);
-    sacc += __shfl_xor(sacc, 32, 64);
-    if (lane < 16) wsum[wave][lane] = sacc;
-  }
-  __syncthreads();
-  auto inv_of = [&](int m) {   // rsqrt(mean x^2 + eps) of the row of x behind result row m
-    const int tok = F.rows != nullptr ? F.rows[m] : m;
-    float ss = 0.f;
-#pragma unroll
-    for (int wv = 0; wv < WAVES; ++wv) ss += wsum[wv][tok];
-    return rsqrtf(ss / (float)K + F.eps);
-  };
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int tile = blockIdx.x * NT + t;
-    if (tile >= ntiles) break;
-    const int n0 = tile * th;
-    // lane (m + 16 (n_local / 4)) holds y[m, n_local] in element n_local % 4
-    if (GATED) {
-      if (threadIdx.x < 128) {
-        const int m = threadIdx.x / 8, j = threadIdx.x % 8;
-        const int n = tile * 8 + j;
-        if (m < M && n < N / 2) {
-          float gsum = 0.f, usum = 0.f;
-#pragma unroll
-          for (int wv = 0; wv < WAVES; ++wv) {
-            gsum += red[t][wv][m + 16 * (j / 4)][j % 4];
-            usum += red[t][wv][m + 16 * (2 + j / 4)][j % 4];
-          }
-          if (CONSUMER) {
-            const float inv = inv_of(m);
-            gsum *= inv;
-            usum *= inv;
-          }
-          if (bias != nullptr) {                  // (the bias lies as the rows do: 8 gates, their 8 ups)
-            gsum += bias[tile * 16 + j];
-            usum += bias[tile * 16 + 8 + j];
-          }
-          const size_t at = F.y_tiled ? (size_t)(n / 32) * (M * 32) + m * 32 + n % 32 : (size_t)m * (N / 2) + n;
-          ((__bf16*)y)[at] = (__bf16)(sl_act(gsum, F.gate_act) * usum);
-        }
-      }
-      continue;
-    }
-    if (threadIdx.x < 256) {
-      const int m = em, n_local = threadIdx.x % 16, n = n0 + n_local;
-      const bool live = m < M && n_local < th && n < N;
-      float s = 0.f;
-#pragma unroll
-      for (int wv = 0; wv < WAVES; ++wv) s += red[t][wv][m + 16 * (n_local / 4)][n_local % 4];
-      if (CONSUMER && live) s *= inv_of(m);
-      if constexpr (ROPE) {
-        s += b_pre[t];
-        const float partner = __shfl_xor(s, 8, 64);      // the other half of the pair, same row
-        if (!live) continue;
-        const int hd = n / R.D, p = n % R.D;
-        const int slot = slot_pre;
-        if (hd < R.nh + R.nkv) {
-          float val = s;
-          if (R.cosv != nullptr && p < R.rot)
-            val = p % 16 < 8 ? s * c_pre[t] - partner * s_pre[t] : s * c_pre[t] + partner * s_pre[t];
-          if (hd < R.nh) {
-            ((__bf16*)y)[(size_t)m * N + n] = (__bf16)(val * R.qscale);
-          } else if (R.slots != nullptr) {
-            R.kc[(((size_t)(slot / R.page) * R.nkv + (hd - R.nh)) * R.page + slot % R.page) * R.D + p] = (__bf16)val;
-          }
-        } else if (R.slots != nullptr) {
-          R.vc[(((size_t)(slot / R.page) * R.nkv + (hd - R.nh - R.nkv)) * R.D + p) * R.page + slot % R.page] = (__bf16)s;
-        }
-        continue;
-      }
-      if (live && bias != nullptr) s += bias[n];
-      if (PRODUCER) {
-        float sq = 0.f;
-        if (live) {
-          const float r = r_old[t] + s;
-          F.resid[(size_t)m * N + n] = r;
-          const size_t at = F.y_tiled ? (size_t)(n / 32) * (M * 32) + m * 32 + n % 32 : (size_t)m * N + n;
-          ((__bf16*)y)[at] = (__bf16)(r * g_next[t]);
-          sq = r * r;
-        }
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);     // over the 16 columns of row m
-        if (n_local == 0) F.out_parts[(size_t)tile * 16 + m] = sq;
-      } else if (live) {
-        if (!CONSUMER && F.gate_act) s = sl_act(s, F.gate_act);
-        const size_t at = !CONSUMER && F.y_tiled ? (size_t)(n / 32) * (M * 32) + m * 32 + n % 32 : (size_t)m * N + n;
-        if (out_f32) ((float*)y)[at] = s;
-        else ((__bf16*)y)[at] = (__bf16)s;
-      }
-    }
-  }
-}
+#include "gemm_few.h"
 
 // wt: W in the tiled layout, ceil(N / 16) * 16 rows (rows beyond N are zero).
 // At most 16 rows.  Fusion: in_parts != nullptr makes x un-normalised rows
 // (consumer), resid != nullptr makes the result a delta of the stream (producer).
-// pair_tiles: two tiles of W per workgroup.  th: rows of W per tile (16, or what sl_tile_weight was given
-// for a producer's matrix).
+// tiles: of W per workgroup, 1 or 2, or 0 for half of one.  th: rows of W per tile (16, or what sl_tile_weight was given
+// for a producer's matrix).  pair_x: up to 8 rows, a load of x takes two k-steps.
 extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float* bias, void* y,
                                       int M, int N, int K, int out_f32, int gated,
                                       const float* in_parts, int in_nparts, float eps,
                                       const int* rows, float* resid, const float* next_w,
-                                      float* out_parts, const RopeStore* rope, int pair_tiles,
+                                      float* out_parts, const RopeStore* rope, int tiles,
                                       int x_tiled, int y_tiled, int th, int pair_x, int act, hipStream_t stream) {
   SL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_skinny: sizes must be positive");
   SL_CHECK(M <= 16, "gemm_skinny: at most 16 rows");
@@ -1146,17 +803,16 @@ extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float
   SL_CHECK(th == 16 || (producer && th >= 8 && th < 16 && th % 2 == 0),
            "gemm_skinny: tiles of 16 rows, or of 8, 10, 12 or 14 for a producer");
   if (M == 0) return nullptr;
-  const dim3 grid((N + th - 1) / th);
-  const __bf16* xx = (const __bf16*)x;
-  const __bf16* ww = (const __bf16*)wt;
   SL_CHECK(x_tiled >= 0 && (x_tiled == 0 || rows != nullptr || x_tiled == M),
            "gemm_skinny: x tiled by k-step has as many rows as the product, or rows are picked from it");
   SL_CHECK(!y_tiled || (gated && (N / 2) % 32 == 0) || ((resid != nullptr || act) && N % 32 == 0),
            "gemm_skinny: a tiled result is a gated, an activated or a producer's, of a multiple of 32 columns");
-  const NormFusion F{in_parts, in_nparts, eps, rows, resid, next_w, out_parts, x_tiled, y_tiled, th, pair_x, gated ? gated : act};
-  const bool few = in_nparts <= 32 * 8;
+  SL_CHECK(tiles >= 0 && tiles <= 2 && (tiles > 0 || (!gated && !consumer && rope == nullptr && th == 16)),
+           "gemm_skinny: half a tile a workgroup goes with plain products and producers over tiles of 16 rows");
+  FewRows A{(const __bf16*)x, (const __bf16*)wt, bias, y, M, N, K, out_f32, {}, {}, {}};
+  A.F = NormFusion{in_parts, in_nparts, eps, rows, resid, next_w, out_parts, x_tiled, y_tiled, th, gated ? gated : act};
   if (rope != nullptr) {
-    const RopeStore R = *rope;
+    const RopeStore& R = A.R = *rope;
     SL_CHECK(!gated && !producer && !out_f32, "gemm_skinny: q/k/v with rotary is a plain or a consumer product");
     SL_CHECK(R.D % 16 == 0 && R.nh > 0 && R.nkv > 0 && N == (R.nh + 2 * R.nkv) * R.D,
              "gemm_skinny: q/k/v columns must be (heads + 2 kv heads) * head_dim, head_dim % 16 == 0");
@@ -1165,40 +821,16 @@ extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float
              "gemm_skinny: the rotated width must be a multiple of 16, at most head_dim");
     SL_CHECK(R.slots == nullptr || (R.kc != nullptr && R.vc != nullptr && R.page > 0),
              "gemm_skinny: cache rows need the pages");
-    const dim3 grid2(((N + 15) / 16 + 1) / 2);
-    if (pair_tiles) {
-      if (!consumer) gemm_skinny_kernel<false, false, false, 1, true, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, R);
-      else if (few) gemm_skinny_kernel<false, true, false, 8, true, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, R);
-      else gemm_skinny_kernel<false, true, false, 16, true, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, R);
-    } else {
-      if (!consumer) gemm_skinny_kernel<false, false, false, 1, true><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, R);
-      else if (few) gemm_skinny_kernel<false, true, false, 8, true><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, R);
-      else gemm_skinny_kernel<false, true, false, 16, true><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, R);
-    }
-    return sl_launch_status();
   }
-  const RopeStore none{};
-  if (pair_tiles) {                              // two tiles per workgroup
-    const dim3 grid2((grid.x + 1) / 2);
-    if (producer) gemm_skinny_kernel<false, false, true, 1, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-    else if (consumer && gated && few) gemm_skinny_kernel<true, true, false, 8, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-    else if (consumer && gated) gemm_skinny_kernel<true, true, false, 16, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-    else if (consumer && few) gemm_skinny_kernel<false, true, false, 8, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
-    else if (consumer) gemm_skinny_kernel<false, true, false, 16, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
-    else if (gated) gemm_skinny_kernel<true, false, false, 1, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-    else gemm_skinny_kernel<false, false, false, 1, false, 2><<<grid2, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
-    return sl_launch_status();
-  }
-  // a matrix with fewer tiles than the chip has CUs leaves each CU one workgroup: sixteen
-  // wavefronts then have twice the loads in flight (7B shape, batch 1: 349 -> 356 tok/s)
-  if (producer && (int)grid.x <= device_cus() && K >= 2048) gemm_skinny_kernel<false, false, true, 1, false, 1, 16><<<grid, 1024, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-  else if (producer) gemm_skinny_kernel<false, false, true, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-  else if (consumer && gated && few) gemm_skinny_kernel<true, true, false, 8><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-  else if (consumer && gated) gemm_skinny_kernel<true, true, false, 16><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-  else if (consumer && few) gemm_skinny_kernel<false, true, false, 8><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
-  else if (consumer) gemm_skinny_kernel<false, true, false, 16><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
-  else if (gated) gemm_skinny_kernel<true, false, false, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, 0, F, none);
-  else gemm_skinny_kernel<false, false, false, 1><<<grid, 512, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32, F, none);
+  const bool wide = M > 8 || !pair_x || tiles == 2, rp = rope != nullptr;
+  const int pairs = (K / 64 + 7) / 8;            // pairs of k-steps a wavefront takes at most: up to 8 in one trip to memory
+  if (wide && tiles == 2) launch_few_rows<true, 2, 2>(A, gated, rp, stream);
+  else if (wide && tiles == 1) launch_few_rows<true, 1, 4>(A, gated, rp, stream);
+  else if (wide) launch_few_rows<true, 0, 4>(A, gated, rp, stream);
+  else if (tiles == 0 && pairs > 4 && pairs <= 8) launch_few_rows<false, 0, 8>(A, gated, rp, stream);
+  else if (tiles == 0) launch_few_rows<false, 0, 4>(A, gated, rp, stream);
+  else if (pairs > 4 && !consumer) launch_few_rows<false, 1, 8>(A, gated, rp, stream);
+  else launch_few_rows<false, 1, 4>(A, gated, rp, stream);
   return sl_launch_status();
 }
 
@@ -1209,19 +841,21 @@ extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float
 // 2,770 us).
 extern "C" const char* sl_gemm_skinny_shares(const float* shares_o, const float* shares_ml, int shares, int head_dim, const void* wt,
                                              const float* bias, void* y, int M, int N, int K, float* resid, const float* next_w,
-                                             float* out_parts, int y_tiled, int th, hipStream_t stream) {
+                                             float* out_parts, int y_tiled, int th, int halves, hipStream_t stream) {
   SL_CHECK(M > 0 && N > 0 && K > 0 && K % 32 == 0, "gemm_skinny_shares: sizes must be positive, K in steps of 32");
   SL_CHECK(head_dim >= 32 && (head_dim & (head_dim - 1)) == 0 && K % head_dim == 0, "gemm_skinny_shares: heads of a power of two, 32 at least");
   SL_CHECK(shares >= 2 && shares <= SL_MAX_SHARES, "gemm_skinny_shares: 2 to 8 shares");
-  SL_CHECK(M <= 16 && M * K <= 16384, "gemm_skinny_shares: at most 16 rows, of 16,384 values together");
+  SL_CHECK(M <= 8 && M * K <= 16384, "gemm_skinny_shares: at most 8 rows, of 16,384 values together");
   SL_CHECK(shares_o != nullptr && shares_ml != nullptr && resid != nullptr && next_w != nullptr && out_parts != nullptr,
            "gemm_skinny_shares: a producer over shares needs them, the stream, the next gain and a parts buffer");
   SL_CHECK(((uintptr_t)shares_o % 16) == 0 && ((uintptr_t)shares_ml % 8) == 0 && ((uintptr_t)wt % 16) == 0, "gemm_skinny_shares: shares and W must be 16-byte aligned");
-  SL_CHECK(th >= 8 && th <= 16 && th % 2 == 0 && (!y_tiled || N % 32 == 0), "gemm_skinny_shares: tiles of 8 to 16 rows, tiled results of N % 32 == 0");
-  const NormFusion F{nullptr, 0, 0.f, nullptr, resid, next_w, out_parts, 0, y_tiled, th, 0, 0};
-  const KeyShares R{shares_o, (const float2*)shares_ml, shares, __builtin_ctz(head_dim)};
-  gemm_skinny_kernel<false, false, true, 1, false, 1, 16, true><<<(N + th - 1) / th, 1024, 2 * M * K, stream>>>(
-      nullptr, (const __bf16*)wt, bias, y, M, N, K, 0, F, R);
+  SL_CHECK(th >= 8 && th <= 16 && th % 2 == 0 && (th == 16 || !halves) && (!y_tiled || N % 32 == 0), "gemm_skinny_shares: tiles of 8 to 16 rows, tiled results of N % 32 == 0");
+  FewRows A{nullptr, (const __bf16*)wt, bias, y, M, N, K, 0, {}, {}, {}};
+  A.F = NormFusion{nullptr, 0, 0.f, nullptr, resid, next_w, out_parts, 0, y_tiled, th, 0};
+  A.S = KeyShares{shares_o, (const float2*)shares_ml, shares, __builtin_ctz(head_dim)};
+  const int tiles = (N + th - 1) / th;
+  if (halves) gemm_few_kernel<false, 0, false, false, true, 1, false, 4, 16, true><<<2 * tiles, 1024, 2 * M * K, stream>>>(A);
+  else gemm_few_kernel<false, 1, false, false, true, 1, false, 4, 16, true><<<tiles, 1024, 2 * M * K, stream>>>(A);
   return sl_launch_status();
 }
 
@@ -1392,7 +1026,7 @@ extern "C" const char* sl_gemm_resident(const void* x, const void* wt, const flo
   SL_CHECK(!y_tiled || (gated && (N / 2) % 32 == 0), "gemm_resident: a tiled result is a gated one of a multiple of 32 columns");
   SL_CHECK(x_tiled >= 0 && (x_tiled == 0 || rows != nullptr || x_tiled == M),
            "gemm_resident: x tiled by k-step has as many rows as the product, or rows are picked from it");
-  const NormFusion F{in_parts, in_nparts, eps, rows, nullptr, nullptr, nullptr, x_tiled, y_tiled, 0, 0, gated};
+  const NormFusion F{in_parts, in_nparts, eps, rows, nullptr, nullptr, nullptr, x_tiled, y_tiled, 0, gated};
   const __bf16* xx = (const __bf16*)x;
   const __bf16* ww = (const __bf16*)wt;
 #define SL_RESIDENT(G, NS, R)                                                                   \

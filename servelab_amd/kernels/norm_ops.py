@@ -131,11 +131,12 @@ class NormOps:
             self._check(d.bias, torch.float32, (N,), "bias")
         out = self._new((M, N))
         wt, th = self._producer_copy(weight, M)
-        parts = self._new((-(-N // th), 16), torch.float32)
+        tiles = self._tiles_a_workgroup(M, N, K, th, False)
+        parts = self._new((-(-N // th) if tiles else 2 * -(-N // 16), 16), torch.float32)     # one a workgroup and tile
         tiled = M if self.tile_few_rows and M > 1 and N % 32 == 0 else 0     # for the products that read the rows
         if shares:
             self._call("gemm", "sl_gemm_skinny_shares", _p(x.o), _p(x.ml), x.o.shape[2], x.o.shape[3], _p(wt), _p(d.bias), _p(out),
-                       M, N, K, _p(resid), _p(gain), _p(parts), int(bool(tiled)), th)
+                       M, N, K, _p(resid), _p(gain), _p(parts), int(bool(tiled)), th, int(tiles == 0))
         else:
             self._skinny(x, weight, d.bias, out, M, N, K, resid=resid, next_gain=gain, out_parts=parts,
                          y_tiled=bool(tiled))

@@ -31,7 +31,7 @@ class Tuning:
     lower_tiles_memory_share: float = 0.55
     lower_tiles_min_gain: float = 0.15
 
-    # few-rows products of at most 8 rows load x for two k-steps at once (gemm.hip, stream_k2)
+    # few-rows products of at most 8 rows load x for two k-steps at once (gemm_few.h)
     pair_x_loads: bool = True
     # Up to how many rows a step takes the few-rows kernels with the residual add, the norm and the
     # rotation fused in (16 at most: the rows of one matrix instruction), by the width of the residual
