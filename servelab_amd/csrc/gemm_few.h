@@ -306,7 +306,7 @@ template <bool WIDE, int TILES, int U>
 static void launch_few_rows(const FewRows& A, bool gated, bool rope, hipStream_t stream) {
   const bool consumer = A.F.in_parts != nullptr, producer = A.F.resid != nullptr, few = A.F.in_nparts <= 32 * 8;
   const int tiles = (A.N + A.F.th - 1) / A.F.th;
-  const dim3 grid(TILES == 0 ? 2 * tiles : (tiles + TILES - 1) / TILES);
+  const dim3 grid(TILES == 0 ? 2 * tiles : TILES == 1 ? tiles : (tiles + 1) / 2);
 #define SL_FEW(GATED, CONSUMER, PRODUCER, PARTS, ROPE) \
   gemm_few_kernel<WIDE, TILES, GATED, CONSUMER, PRODUCER, PARTS, ROPE, U><<<grid, 512, 0, stream>>>(A)
   if constexpr (TILES > 0) {

@@ -216,7 +216,8 @@ class ProductOps:
         limit = self._few_rows_limit(weight)
         plan = self._block_plan(M, N, K, weight) or (
             defer and M > self.BLOCK_SQUARE_MAX_M and self.fuse_norms and not out_f32
-            and not self._tuned_for(M, N, K) and self._block_reads(x, weight) and self._shares_plan(M, N, K, weight))
+            and not self._tuned_for(M, N, K) and self._block_reads(x, weight)
+            and (self._shares_plan(M, N, K, weight) or self._shares_by_estimate(M, N, K, weight)))
         if plan:
             # (deferred: the norm adds the partial sums)
             return self.linear_block(x, weight, bias, out_f32, plan[0],
@@ -344,6 +345,22 @@ class ProductOps:
         shares = self._num_cus // tiles
         fill = tiles * shares / self._num_cus
         return (shares, True) if (shares == 2 and fill >= 0.875) or (shares == 3 and fill >= 0.8) else None
+
+    def _shares_by_estimate(self, M, N, K, weight):
+        """The sizes that ``_shares_plan`` leaves: two to eight shares in wide tiles, as many as take the least time by estimate
+        (the product's, ``_tiles_us``, and SHARE_US for every million sums written and read again).  us with the norm that adds
+        them, the library's product / the shares: 2048 x 11008 at 1,792 / 1,930 / 2,048 rows 109 / 82, 105 / 88 and 110 / 92 in
+        four, 2048 x 8192 at 2,048 81 / 76, 1536 x 8960 78 / 67 in five, 3584 x 18944 at 1,792 320 / 216 in two; 3072 x 8192
+        at 1,930 106 / 107.  Rows of 5,632 values and less gain nothing (2048 x 5632 at 2,048 64 / 62, 896 x 4864 34 / 33)."""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or weight.w is None
+                or K % 64 or N % 4 or N > self.BLOCK_MAX_N or K < self.BLOCK_SQUARE_MIN_K
+                or not self.BLOCK_SQUARE_MAX_M < M <= self.SHARES_MAX_M):
+            return None
+        tiles = -(-N // 256) * -(-M // 256)
+        plans = [ks for ks in range(2, 9) if tiles * ks <= self._num_cus]
+        if not plans:
+            return None
+        return min(plans, key=lambda ks: self._tiles_us(self._tile_rows(M, N, K, ks), M, N, K, ks) + self.SHARE_US * 1e-6 * ks * M * N), True
 
     def _gated_rows(self, M, N, K):
         """Rows of x a workgroup takes (192 or 256) for the gated product of a prompt at sizes that take the tiles whatever their

@@ -92,6 +92,8 @@ class Tuning:
     block_square_max_m: int = 1536
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
+    # what a million float32 sums of a share cost that are written and read again by the norm (us)
+    share_us: float = 0.9
     # gated and activated products of a prompt in the tiles of gemm_rounds.h (measured sides: HipOps._gated_rows): the fewest rows
     # of W, the fewest and the most rows of x; rows of up to gated_short_k values, or up to gated_one_round_k in one round of tiles of
     # which so much is useful; ...
