@@ -1,7 +1,8 @@
 // Shared definitions of the servelab_amd kernels (gfx950, 64-wide wavefronts).
 //
 // Every source is compiled twice: with -DSL_F32 the activation type is float
-// (the true 32-bit path: no reduced-precision matrix instruction anywhere),
+// (the true 32-bit path: nothing is rounded to fewer bits; products of many rows
+// multiply their operands as exact sums of bfloat16 terms, gemm_f32_split.h),
 // without it the activation type is bfloat16.  Accumulation, softmax, norms
 // and rotation are float in both.
 //

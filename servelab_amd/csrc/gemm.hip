@@ -483,120 +483,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   }
 }
 
-// The same for more rows, K in chunks of 32: four wavefronts own 128 x 128, a wavefront 64 x 64, two workgroups a CU.  Bound by the
-// matrix units (64 cycles a v_mfma_f32_32x32x2_f32, 157 TFLOP/s): chunks go from memory straight into a ring of two LDS stages
-// (rows of 128 bytes as lds_place says), a lane reads four values of k of its row at once, and the matrix instruction takes its two
-// k's from the halves' lanes: value j of both, so eight k's are four instructions a tile, in another order of the terms.
-// 849 rows, 17920 x 1536 444 -> 424 us (110 TFLOP/s; two rounds of two workgroups a CU), 1536 x 8960 in three shares 250 -> 222;
-// 2,048 rows, 37888 x 3584 4,733 -> 4,279 (130), against chunks of 16 through registers and single words.  What is left: the two
-// workgroups of a CU begin, end and come to their barriers together (some 25 us a round; a higher wave priority for one of them
-// changes nothing).
-template <bool SHARES>
-__global__ __launch_bounds__(256, 2) void gemm_f32_ring_kernel(
-    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
-    float* __restrict__ y, int M, int N, int K, int nsplit) {
-  constexpr int CK = 32, STAGE = 256 * 128;
-  __shared__ __attribute__((aligned(1024))) char ring[2 * STAGE];      // rows of x, then those of W
-  const int t = threadIdx.x, lane = t & 63, half = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 1, wn = wave & 1;
-  // a chiplet takes a contiguous eighth of the (share, column tile, row tile) triples, row tiles fastest
-  const int gx = (N + 127) / 128, gy = (M + 127) / 128, total = gx * gy * nsplit, per = (total + 7) / 8;
-  const int triple = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per || triple >= total) return;        // (the whole workgroup)
-  const int share = triple / (gx * gy), m0 = triple % gy * 128, n0 = triple / gy % gx * 128;
-  constexpr int SEG = SEGMENT_K / CK;                 // chunks a running sum takes
-  const int chunks = K / CK, segs = (chunks + SEG - 1) / SEG;
-  const int first = SHARES ? (int)((unsigned)segs * share / (unsigned)nsplit) * SEG : 0;
-  const int behind = SHARES ? (int)((unsigned)segs * (share + 1) / (unsigned)nsplit) * SEG : segs * SEG;
-  const int last = behind < chunks ? behind : chunks;
-  if (SHARES) {
-    y += (size_t)share * M * N;
-    bias = nullptr;
-  }
-  // what this lane brings of every chunk: unit (lane % 8) ^ place of rows 8 (wave + 4 j) + lane / 8; rows past the end: the last
-  const float* src[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int r = 8 * (wave + 4 * (j & 3)) + (lane >> 3), c = (lane & 7) ^ lds_place(r);
-    if (j < 4) src[j] = x + (size_t)(m0 + r < M ? m0 + r : M - 1) * K + 4 * c;
-    else src[j] = w + (size_t)(n0 + r < N ? n0 + r : N - 1) * K + 4 * c;
-  }
-  const unsigned ring_at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring + 1024 * wave;
-  auto load = [&](int j, int c, int stage) { load_to_lds(src[j] + CK * (size_t)c, ring_at + STAGE * stage + 4096 * j); };
-  auto barrier = [&]() {
-    asm volatile("" : : : "memory");
-    wait_loads<0>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" : : : "memory");
-  };
-  int at[4];                                           // this lane's four values of eight k's: row lane % 32, unit 2 g + half
-#pragma unroll
-  for (int g = 0; g < 4; ++g) at[g] = 128 * (lane & 31) + 16 * ((2 * g + half) ^ lds_place(lane & 15));
-  const int x_at = 128 * 64 * wm, w_at = 128 * (128 + 64 * wn);
-  f32x16 acc[2][2], sum[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = sum[i][j][r] = 0.f;
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  f32x4 a[2][2], b[2][2];                              // [set][tile]
-  auto operands = [&](int set, int g, int stage) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) a[set][i] = *(const f32x4*)(ring + STAGE * stage + x_at + 4096 * i + at[g]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) b[set][i] = *(const f32x4*)(ring + STAGE * stage + w_at + 4096 * i + at[g]);
-  };
-#pragma unroll
-  for (int j = 0; j < 8; ++j) load(j, first, first & 1);
-  barrier();
-  for (int c0 = first; c0 < last; c0 += SEG) {
-    const int c1 = c0 + SEG < last ? c0 + SEG : last;
-    for (int c = c0; c < c1; ++c) {
-      const int stage = c & 1, ahead = c + 1 < last ? c + 1 : c;       // (at the end the last chunk again, which nothing reads)
-      operands(0, 0, stage);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        if (g < 3) operands((g + 1) & 1, g + 1, stage);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          if (g < 2) load(4 * g + k, ahead, stage ^ 1);
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-              acc[i][j ^ i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g & 1][i][k], b[g & 1][j ^ i][k], acc[i][j ^ i], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      barrier();
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        sum[i][j] += acc[i][j];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-      }
-  }
-  // element r of a tile: row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int n = n0 + 64 * wn + 32 * j + (lane & 31);
-    if (n >= N) continue;
-    const float bv = bias != nullptr ? bias[n] : 0.f;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + 64 * wm + 32 * i + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (m < M) y[(size_t)m * N + n] = sum[i][j][r] + bv;
-      }
-  }
-}
+#include "gemm_f32_split.h"
 
 // The shares' sums added up in their order, then the bias; VEC values a thread.
 template <int VEC>
@@ -616,18 +503,19 @@ __global__ __launch_bounds__(256) void f32_shares_kernel(const float* __restrict
   *(piece*)(y + at) = sum;
 }
 
-// Whether a float32 product of more than 64 rows is left to the kernel of three workgroups a CU: the ring's two leave a last
-// round of at most one workgroup a CU to pairs again, which takes as long as a whole one.  That shows where terms are few and
-// rounds are few (us, ring / registers, 256 CUs; tiles times shares of so many terms): 756 of 512 145 / 120, 672 148 / 122,
-// 1,260 208 / 195, 768 of 1,024 272 / 226; not at 1,152 of 512 184 / 195, 672 of 1,024 210 / 225, 1,280 of 1,024 352 / 370,
-// 700 of 1,536 307 / 328.
-static bool f32_last_round_of_threes(long long triples, int terms) {
-  const long long cus = device_cus();
-  if (cus <= 0 || terms > 1024) return false;                          // (no answer: the ring does not depend on it)
-  const long long whole = triples / (2 * cus), rest = triples % (2 * cus);
-  if (rest == 0 || rest > cus) return false;
-  const bool most = 4 * rest > 3 * cus;
-  return terms <= 512 ? whole == 1 || (whole == 2 && most) : whole == 1 && most;
+// Estimated time of a product of split operands, `columns` (256 or 128) a workgroup, nsplit shares of up to `terms` terms: rounds of
+// tiles over the CUs, and what a chunk of 32 takes alone and more on all CUs.  us measured / estimated: 849 rows, 17920 x 1536 242 /
+// 245 and 288 / 290; 1536 x 1536 in three shares of 512 56 / 43 and 38 / 31 (14 of them the sums' way); 333 rows, 2048 x 1536 in one 103 /
+// 102 and 62 / 62; 1,024 rows, 8192 x 1536 122 / 128 and 137 / 148; 600 rows, 3584 x 3584 212 / 239 and 129 / 152.
+static float f32_split_us(int columns, int M, int N, int terms, int nsplit, int cus) {
+  if (cus <= 0) return 0.f;                            // (no device answers)
+  const float tiles = (float)((N + columns - 1) / columns) * ((M + 127) / 128) * nsplit;
+  const float rounds = ceilf(tiles / cus), fill = tiles / (rounds * cus), chunks = (terms + 31) / 32;
+  return columns == 256 ? 8.f + rounds * chunks * (1.9f + 0.6f * fill) : 6.f + rounds * chunks * (1.08f + 0.4f * fill);
+}
+// The better of the two, for the choice of nsplit.
+extern "C" float sl_gemm_f32_split_us(int M, int N, int terms, int nsplit, int cus) {
+  return fminf(f32_split_us(256, M, N, terms, nsplit, cus), f32_split_us(128, M, N, terms, nsplit, cus));
 }
 
 // nsplit > 1: K is cut into that many shares of whole segments, whose sums wait in `part`, [nsplit, M, N].  A product of
@@ -643,23 +531,29 @@ extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const floa
   SL_CHECK(nsplit >= 1 && nsplit <= (K + SEGMENT_K - 1) / SEGMENT_K, "gemm_f32_mfma: at most one share of K per 512 terms");
   SL_CHECK(nsplit == 1 || (part != nullptr && (uintptr_t)part % 16 == 0 && (uintptr_t)y % 16 == 0),
            "gemm_f32_mfma: shares of K need an aligned buffer for their sums");
+  const bool split = M > 64 && K % 32 == 0;
   const int rows = M <= 64 ? 32 : 128;
   const dim3 grid((N + 127) / 128, (M + rows - 1) / rows, nsplit);
   SL_CHECK(grid.y <= 65535, "gemm_f32_mfma: more than 65535 row tiles");
-  const long long triples = (long long)grid.x * grid.y * nsplit;
-  const int segments = (K + SEGMENT_K - 1) / SEGMENT_K, longest = min(K, (segments + nsplit - 1) / nsplit * SEGMENT_K);
   float* to = nsplit > 1 ? part : (float*)y;
   auto run = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit); };
   // (one share apart: products of short rows take 6 to 8 % longer in a kernel that could take several)
   if (M <= 64) {
     if (nsplit > 1) run(gemm_f32_mfma_kernel<1, 1, 1, 4, true>);
     else run(gemm_f32_mfma_kernel<1, 1, 1, 4, false>);
-  } else if (K % 32 == 0 && !f32_last_round_of_threes(triples, longest)) {
-    SL_CHECK(triples < (1ll << 24), "gemm_f32_mfma: too many tiles");
-    const dim3 line((unsigned)(8 * ((triples + 7) / 8)));
-    if (nsplit > 1) gemm_f32_ring_kernel<true><<<line, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
-    else gemm_f32_ring_kernel<false><<<line, 256, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
-  } else {
+  } else if (split) {
+    auto launch = [&](auto kernel, int bn) -> const char* {
+      const long long triples = (long long)((N + bn - 1) / bn) * ((M + 127) / 128) * nsplit;
+      SL_CHECK(triples < (1ll << 24), "gemm_f32_mfma: too many tiles");
+      kernel<<<dim3((unsigned)(8 * ((triples + 7) / 8))), 512, 0, stream>>>((const float*)x, (const float*)w, bias, to, M, N, K, nsplit);
+      return nullptr;
+    };
+    const int segments = (K + SEGMENT_K - 1) / SEGMENT_K, longest = min(K, (segments + nsplit - 1) / nsplit * SEGMENT_K), cus = device_cus();
+    const bool wide = f32_split_us(256, M, N, longest, nsplit, cus) <= f32_split_us(128, M, N, longest, nsplit, cus);
+    const char* e = nsplit > 1 ? (wide ? launch(gemm_f32_split_kernel<4, true>, 256) : launch(gemm_f32_split_kernel<2, true>, 128))
+                               : (wide ? launch(gemm_f32_split_kernel<4, false>, 256) : launch(gemm_f32_split_kernel<2, false>, 128));
+    if (e) return e;
+  } else {                                             // (rows that end in half a chunk of 32)
     if (nsplit > 1) run(gemm_f32_mfma_kernel<2, 2, 2, 2, true>);
     else run(gemm_f32_mfma_kernel<2, 2, 2, 2, false>);
   }

@@ -1,0 +1,199 @@
+// Float32 products of more than 64 rows on the bfloat16 matrix units: y[M, N] = x[M, K] W[N, K]^T, K % 32 == 0.  Included by gemm.hip.
+//
+// An operand is three bfloat16 terms, each what the ones before left over, rounded to nearest: 8 + 8 + 8 bits of significand, so
+// that together they are the float itself (above 2^-109 in size; below, what a third term loses lies under 2^-133).  A product is the
+// six products of terms down to 2^-18 of it; the three left out are at most 2^-26 of it together, a quarter of a float's rounding.
+// Products of bfloat16 are exact in float, and a matrix instruction adds 32 of them to the running sum at once.  It rounds that sum down,
+// not to nearest: left so, every result lay 5e-8 to 6e-7 of their spread too low, and the logits of a 6-layer model 3.1e-6 off
+// instead of 2.8e-6.  Hence runs of RUN chunks are summed apart, every other one with x's sign turned, whose sums are
+// subtracted.  Error of a result against 64 bits 2.6e-7 for 4.1e-7 with float32 instructions and sums of 512 terms (30 sizes,
+// inputs of several distributions), of those logits 2.4e-6 for 2.9e-6.
+// A result that is not finite is worked out again term by term: an infinite operand's rests are NaN.
+//
+// Bound by the matrix units, six instructions of 16 cycles in the place of eight of 32 (16 x 16 results, 32 terms), and their power:
+// 2.3 us a chunk of 32 k on all CUs, 1.9 on one.  A workgroup of eight wavefronts, one a CU, owns 128 rows of x by 256 of W, a
+// wavefront 64 x 64.  A chunk goes from memory to registers, is split there once for the workgroup, and lies in LDS as three planes of
+// rows of 64 bytes (a wavefront's read of an operand is 1 KB in a row); two stages.  The order of a chunk is laid down
+// instruction by instruction: left to itself the compiler converts in front of all products and loads behind them (294 us
+// below, 272 laid down).  849 rows, 17920 x 1536 444 -> 272 us (172 TFLOP/s), 1536 x 8960 in six shares 205 -> 128; 2,048 rows, 37888 x
+// 3584 4,380 -> 2,620 (212); 266 products of 65 to 2,048 rows take 0.72 of the time on average, 0.97 at worst, against
+// v_mfma_f32_32x32x2_f32.
+#pragma once
+#include <utility>
+
+typedef __bf16 split_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float split_f32x4 __attribute__((ext_vector_type(4)));
+typedef float split_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 split_bf16x2 __attribute__((ext_vector_type(2)));
+
+// Eight floats as three bfloat16 each, v = t0 + t1 + t2: every term is what the ones before left over, rounded to nearest.
+__device__ __forceinline__ void split_terms(const split_f32x4 (&v)[2], split_bf16x8 (&t)[3]) {
+  unsigned u[3][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    split_f32x2 r = {v[e >> 1][2 * (e & 1)], v[e >> 1][2 * (e & 1) + 1]};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      u[p][e] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, split_bf16x2));
+      if (p < 2) {
+        r[0] -= __uint_as_float(u[p][e] << 16);
+        r[1] -= __uint_as_float(u[p][e] & 0xffff0000u);
+      }
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) __builtin_memcpy(&t[p], u[p], 16);
+}
+
+// f(0), f(1), ..: each with its number as a constant.
+template <class F, int... I> __device__ __forceinline__ void in_order(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F> __device__ __forceinline__ void in_order(F f) { in_order(f, std::make_integer_sequence<int, N>{}); }
+
+// B: tiles of 16 columns a wavefront takes, 4 or 2: a workgroup 256 columns or 128.
+template <int B, bool SHARES>
+__global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    float* __restrict__ y, int M, int N, int K, int nsplit) {
+  constexpr int BM = 128, BN = 64 * B, CK = 32, ITEMS = 1 + B / 2, ROWS = BM + BN, PLANE = ROWS * 64, STAGE = 3 * PLANE;
+  __shared__ __attribute__((aligned(1024))) char stages[2 * STAGE];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 2, wn = wave & 3;
+  // a chiplet takes a contiguous eighth of the (share, column tile, row tile) triples, row tiles fastest
+  const int gx = (N + BN - 1) / BN, gy = (M + BM - 1) / BM, total = gx * gy * nsplit, per = (total + 7) / 8;
+  const int triple = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || triple >= total) return;        // (the whole workgroup)
+  const int share = triple / (gx * gy), m0 = triple % gy * BM, n0 = triple / gy % gx * BN;
+  constexpr int SEG = SEGMENT_K / CK;
+  const int chunks = K / CK, segs = (chunks + SEG - 1) / SEG;
+  const int first = SHARES ? (int)((unsigned)segs * share / (unsigned)nsplit) * SEG : 0;
+  const int behind = SHARES ? (int)((unsigned)segs * (share + 1) / (unsigned)nsplit) * SEG : segs * SEG;
+  const int last = behind < chunks ? behind : chunks;
+  if (SHARES) {
+    y += (size_t)share * M * N;
+    bias = nullptr;
+  }
+  // what this thread brings of every chunk: eight values of k, t % 4, of rows t / 4 + 128 j; rows past the end: the last
+  const float* src[ITEMS];
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    const int r = (t >> 2) + 128 * j;
+    src[j] = (j == 0 ? x + (size_t)(m0 + r < M ? m0 + r : M - 1) * K : w + (size_t)(n0 + r - BM < N ? n0 + r - BM : N - 1) * K) +
+             8 * (t & 3) + CK * (size_t)first;
+  }
+  split_f32x4 v[ITEMS][2];
+  auto load = [&](int j) {
+    v[j][0] = *(const split_f32x4*)src[j];
+    v[j][1] = *(const split_f32x4*)(src[j] + 4);
+    src[j] += CK;
+  };
+  // chunks of a run of RUN that are multiplied with -x, from the first on every other run
+  constexpr int RUN = 8;
+  auto sign_of = [&](int c) { return (c - first) / RUN & 1 ? 1.f : -1.f; };
+  auto store = [&](int stage, int j) {
+    split_bf16x8 terms[3];
+    if (j == 0) v[0][0] *= sign_of(first), v[0][1] *= sign_of(first);
+    split_terms(v[j], terms);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *(split_bf16x8*)(stages + stage * STAGE + p * PLANE + 8192 * j + 16 * t) = terms[p];
+  };
+  split_f32x4 acc[4][B], sum[4][B];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < B; ++b) acc[a][b] = sum[a][b] = split_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int at = 64 * (lane & 15) + 16 * (lane >> 4), x_at = at + 4096 * wm, w_at = at + 64 * BM + 1024 * B * wn;
+  int asked = first;                                   // chunks asked for; past the last one that one again
+  auto ask = [&](int j) {
+    load(j);
+    if (asked + 1 >= last) src[j] -= CK;
+  };
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) ask(j);
+  ++asked;
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    store(0, j);
+    ask(j);
+  }
+  ++asked;
+  __syncthreads();
+  int c = first, stage = 0;
+  while (c < last) {
+    const int c1 = c + RUN < last ? c + RUN : last;
+    const float sign = sign_of(c);
+    for (; c < c1; ++c, stage ^= 1) {
+      const char* from = stages + stage * STAGE;
+      char* to = stages + (stage ^ 1) * STAGE + 16 * t;
+      split_bf16x8 x0[4], x1[4], w0[B], w1[B];
+      auto read = [&](int p, int where, int a) { return *(const split_bf16x8*)(from + p * PLANE + where + 1024 * a); };
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        if (a < B) w0[a] = read(0, w_at, a);
+        x0[a] = read(0, x_at, a);
+      }
+      constexpr int P = 24 * B, S = 12 * ITEMS, S0 = 3 * B / 2, SPAN = P - 2 * B;      // products; steps of the conversion, the first one's place
+      const float sign_next = sign_of(c + 1);
+      unsigned u[3][4];
+      split_f32x2 r;
+      in_order<P>([&](auto slot) __attribute__((always_inline)) {
+        constexpr int i = decltype(slot)::value;
+        // products of the terms: 0 0, 0 1, 1 1, 1 0, 0 2, 2 0 of x and W; the third terms take the second ones' registers
+        constexpr int part = i / (4 * B), a = i / B % 4, b = a & 1 ? B - 1 - i % B : i % B;
+        if constexpr (i < B) w1[i] = read(1, w_at, i);
+        if constexpr (i >= 4 * B && i < 4 * B + 4) x1[i - 4 * B] = read(1, x_at, i - 4 * B);
+        if constexpr (i >= 12 * B && i < 13 * B) w1[i - 12 * B] = read(2, w_at, i - 12 * B);
+        if constexpr (i >= 16 * B && i < 16 * B + 4) x1[i - 16 * B] = read(2, x_at, i - 16 * B);
+        constexpr int s = (S * (i - S0) + SPAN - 1) / SPAN;              // the next chunk's conversion: item s / 12, pair s / 3 % 4, term s % 3
+        if constexpr (i >= S0 && s < S && S0 + s * SPAN / S == i) {
+          constexpr int q = s / 12, e = s / 3 % 4, p = s % 3;
+          if constexpr (p == 0) {
+            r = split_f32x2{v[q][e >> 1][2 * (e & 1)], v[q][e >> 1][2 * (e & 1) + 1]};
+            if constexpr (q == 0) r *= sign_next;
+          }
+          u[p][e] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, split_bf16x2));
+          if constexpr (p < 2) {
+            r[0] -= __uint_as_float(u[p][e] << 16);
+            r[1] -= __uint_as_float(u[p][e] & 0xffff0000u);
+          }
+          if constexpr (e == 3) __builtin_memcpy(to + p * PLANE + 8192 * q, u[p], 16);
+          if constexpr (e == 3 && p == 2) ask(q);
+        }
+        const split_bf16x8 xv = part == 0 || part == 1 || part == 4 ? x0[a] : x1[a], wv = part == 0 || part == 3 || part == 5 ? w0[b] : w1[b];
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xv, acc[a][b], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      ++asked;
+      __syncthreads();
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        sum[a][b] += sign * acc[a][b];
+        acc[a][b] = split_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  // lane: row lane % 16 of x's tile, four rows of W's from 4 (lane / 16) on
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int m = m0 + 64 * wm + 16 * a + (lane & 15);
+    if (m >= M) continue;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int n = n0 + 16 * B * wn + 16 * b + 4 * (lane >> 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) continue;
+        float s = sum[a][b][e];
+        if (!(fabsf(s) < INFINITY)) {
+          // an operand that is not finite, or beyond the largest bfloat16, or a sum past the largest float: term by term
+          s = 0.f;
+          const float* xr = x + (size_t)m * K;
+          const float* wr = w + (size_t)(n + e) * K;
+          for (int k = CK * first; k < CK * last; ++k) s = fmaf(xr[k], wr[k], s);
+        }
+        y[(size_t)m * N + n + e] = s + (bias != nullptr ? bias[n + e] : 0.f);
+      }
+    }
+  }
+}

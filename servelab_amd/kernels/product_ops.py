@@ -675,8 +675,9 @@ class ProductOps:
     F32_MFMA_MIN_M = 17           # float32 products of this many rows or more run on the matrix cores
 
     def linear_f32_mfma(self, x, w, bias):
-        """Float32 product by float32 matrix instructions (float32 inputs and sums,
-        no reduced-precision mode); K % 16 == 0."""
+        """Float32 product on the matrix cores, K % 16 == 0: more than 64 rows and K % 32 == 0 by products of
+        three bfloat16 terms an operand, which together are the float (gemm_f32_split.h: closer to 64 bits than
+        float32 instructions), else by float32 instructions; float32 sums."""
         if self.act_dtype != torch.float32:
             raise KernelError("linear_f32_mfma is for the float32 table only")
         M, K = x.shape
@@ -688,18 +689,24 @@ class ProductOps:
         return y
 
     F32_SEGMENT = 512             # terms of a running sum of the float32 products: a share of K holds whole ones
-    F32_TILE_US_PER_TERM = 0.067  # a tile of 128 x 128 results takes this long per term of K with a CU to itself
+    F32_TILE_US_PER_TERM = 0.067  # a tile of 128 x 128 results takes this long per term of K with a CU to itself (float32 instructions)
 
     def _f32_shares(self, M, N, K):
         """Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated
         time, which is the tiles' rounds over the CUs plus, for several shares, the traffic of the partial sums and
         their addition."""
-        rows = 32 if M <= 64 else 128
+        rows, split = 32 if M <= 64 else 128, M > 64 and K % 32 == 0
         tiles = -(-M // rows) * -(-N // 128)
         best, least, segments = 1, float("inf"), -(-K // self.F32_SEGMENT)
+        if split:
+            estimate = self._lib["gemm"].sl_gemm_f32_split_us
+            estimate.restype = ctypes.c_float
         for s in range(1, min(16, segments) + 1):
             terms = min(K, -(-segments // s) * self.F32_SEGMENT)          # of the longest share
-            us = -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM * (rows / 128)
+            if split:
+                us = estimate(M, N, terms, s, self._num_cus)
+            else:
+                us = -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM * (rows / 128)
             if s > 1:
                 us += 5.0 + (s + 1) * M * N * 4 / 3e6
             if us < 0.97 * least:

@@ -1,0 +1,64 @@
+"""Float32 products of three bfloat16 terms an operand: both widths of a workgroup at the edges of tiles, chunks and shares, values of
+every size, and operands that are not finite."""
+import pytest
+import torch
+
+from servelab_amd.kernels import HipOps
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def draws(M, N, K, spread):
+    """Values whose sizes are spread over 2^-spread .. 2^spread."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    two = lambda *s: torch.exp2((torch.rand(s, generator=g, device=DEV) * 2 - 1) * spread)
+    return x * two(M, K), w * two(N, K)
+
+
+# a row and a column past a tile of 128, past one of 256 (the wide form where many tiles fill the CUs), one chunk of 32, a chunk past a
+# segment of 512, a last share of one chunk
+@pytest.mark.parametrize("M,N,K", [(129, 129, 32), (70, 257, 544), (900, 8193, 96), (1025, 8191, 1056), (128, 256, 1536)])
+@pytest.mark.parametrize("spread", [0, 12])
+def test_sums_of_terms(M, N, K, spread):
+    ops = HipOps(torch.float32, DEV)
+    x, w = draws(M, N, K, spread)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    for shares in {1, -(-K // 512)}:
+        ops._f32_shares = lambda *_: shares
+        got = ops.linear_f32_mfma(x, w, None).double()
+        # six roundings of the running sum a chunk of 32, at most 16 chunks a sum, the sums' own, and 2^-26 of every product left out
+        bar = (6 * min(K // 32, 16) + K // 512 + 2) * 2.0 ** -24 + 2.0 ** -26
+        assert ((got - want).abs() <= bar * size).all()
+
+
+def test_both_widths_are_chosen():
+    ops = HipOps(torch.float32, DEV)
+    lib = ops._lib["gemm"]
+    import ctypes
+    lib.sl_gemm_f32_split_us.restype = ctypes.c_float
+    assert ops._f32_shares(849, 1536, 8960) > 1
+    # the estimate of one round of wide tiles on every CU lies below two of narrow ones, that of half as many tiles above one of them
+    full, half = lib.sl_gemm_f32_split_us(1024, 8192, 1536, 1, 256), lib.sl_gemm_f32_split_us(512, 8192, 1536, 1, 256)
+    assert full == 8 + 48 * 2.5 and abs(half - (6 + 48 * 1.48)) < 1e-3
+    assert lib.sl_gemm_f32_split_us(512, 8192, 1536, 1, 0) == 0
+
+
+@pytest.mark.parametrize("M,N,K,shares", [(130, 300, 1056, 1), (130, 300, 1056, 3), (1024, 8192, 64, 1)])
+def test_operands_that_are_not_finite_or_hardly(M, N, K, shares):
+    ops = HipOps(torch.float32, DEV)
+    ops._f32_shares = lambda *_: shares
+    x, w = draws(M, N, K, 0)
+    w *= 2.0 ** -8
+    clean = x.double() @ w.double().T
+    x[5, 7], x[6, 8], x[70, 0] = float("inf"), float("-inf"), 3.4e38          # (the last is past the largest bfloat16)
+    w[3, 9], w[200, 11] = float("nan"), float("inf")
+    w[:, 7][4], w[9, 8] = 0.5, 0.0                                            # exact in one term; infinity times zero
+    want = x.double() @ w.double().T
+    got = ops.linear_f32_mfma(x, w, None)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(want))
+    there = torch.isfinite(want)
+    size = torch.where(torch.isfinite(x), x, 0).double().abs() @ torch.where(torch.isfinite(w), w, 0).double().abs().T
+    assert ((got.double() - want).abs()[there] <= (K * 2.0 ** -24 * size)[there]).all() and there.sum() > 0.9 * clean.numel()
