@@ -1765,4 +1765,27 @@ extern "C" const char* sl_gemm_block(const void* x, const void* w, const float* 
   splitk_reduce_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(part, bias, y, M, N, ks, out_f32);
   return sl_launch_status();
 }
+
+#include "gemm_even.h"
+
+// y [M, N], bfloat16 or float32, = x W^T + bias over the tiled copy of W: tiles of 128 rows of x by `columns` (96, 128, .. 224) of W.
+extern "C" const char* sl_gemm_even(const void* x, const void* wt, const float* bias, void* y, int M, int N, int K, int out_f32,
+                                    int columns, hipStream_t stream) {
+  SL_CHECK(M > 0 && N > 0 && K > 0 && K % 64 == 0 && K <= (1 << 22), "gemm_even: positive sizes, K a multiple of 64 and 4 M at most");
+  SL_CHECK(columns >= 96 && columns <= 224 && columns % 32 == 0, "gemm_even: tiles of 96 to 224 columns in steps of 32");
+  SL_CHECK(N % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)wt % 16 == 0, "gemm_even: columns in fours, operands and results on 16 bytes");
+  const long long tiles = (long long)((N + columns - 1) / columns) * ((M + 127) / 128);
+  SL_CHECK(tiles < (1ll << 24), "gemm_even: too many tiles");
+  const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)));
+  switch (columns / 32) {
+#define SL_EVEN(B)                                                                                                                    \
+  case B:                                                                                                                             \
+    if (out_f32) gemm_even_kernel<B, EVEN_F32><<<grid, 256, 0, stream>>>((const __bf16*)x, (const __bf16*)wt, bias, y, M, N, K);     \
+    else gemm_even_kernel<B, EVEN_BF16><<<grid, 256, 0, stream>>>((const __bf16*)x, (const __bf16*)wt, bias, y, M, N, K);            \
+    break;
+    SL_EVEN(3) SL_EVEN(4) SL_EVEN(5) SL_EVEN(6) SL_EVEN(7)
+#undef SL_EVEN
+  }
+  return sl_launch_status();
+}
 #endif

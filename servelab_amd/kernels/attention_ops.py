@@ -100,10 +100,14 @@ class AttentionOps:
                 qkv = product
             elif (self.act_dtype == torch.bfloat16 and not isinstance(x, ScaledRows)
                     and M > self._few_rows_limit(weight)):
-                # many rows: the library keeps the float32 sums, and the rotation kernel adds the
+                # many rows: the library, or the product of even tiles, keeps the float32 sums, and the rotation kernel adds the
                 # float32 bias, rotates and rounds once, exactly as the fused few-rows kernel does
                 self._check(x, self.act_dtype, (M, K), "x")
-                sums = self.library_sums(x, self.rows_of(weight), torch.float32)
+                columns = self._even_columns(M, N, K)
+                if columns and weight.tiled is not None and not self._tuned_for(M, N, K) and x.data_ptr() % 16 == 0:
+                    sums = self.linear_even(x, weight, None, columns, True)
+                else:
+                    sums = self.library_sums(x, self.rows_of(weight), torch.float32)
                 qkv = self._new((M, N))
                 self.rope_store(qkv, nh, nkv, D, cos, sin, slots, k_cache, v_cache, page_size,
                                 True, split=PartialSums(sums.unsqueeze(0), bias), rot_dim=rot,

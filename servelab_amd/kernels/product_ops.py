@@ -228,6 +228,9 @@ class ProductOps:
                                    target=self.MID_DEFERRED_WORKGROUPS)
         if M <= limit:
             return self.linear_skinny(x, weight, bias, out_f32)
+        columns = self._even_columns(M, N, K)
+        if columns and weight.tiled is not None and not self._tuned_for(M, N, K) and x.data_ptr() % 16 == 0:
+            return self.linear_even(x, weight, bias, columns, out_f32)
         if out_f32 and limit:
             # float32 results of many rows (the head for more requests than the few-rows kernels take,
             # logits of every position).  With a row-major copy of W: the library's product with its
@@ -251,6 +254,34 @@ class ProductOps:
                 return self.linear_rows(x, w, bias, out_f32)
             return self.linear_tiled(x, w, bias, out_f32)
         return self.linear_library(x, w, bias)
+
+    def _even_columns(self, M, N, K):
+        """Columns of y a workgroup takes in the product of tiles that go round the CUs once (``sl_gemm_even``, 128 rows of x), the
+        fewest that do, or 0 where the product is not its own: matrices of 512 rows and more with rows of up to EVEN_MAX_K values,
+        tiles of up to 192 columns, or 224 on nine tenths of the CUs, and with rows of more than EVEN_SHORT_K values seven
+        tenths of the CUs busy.  Of 162 such products (896 to 7,168 rows, 513 to 2,048 rows of x) the library's default pick takes
+        1.32 times as long on average, 0.93 at worst (700 x 4096 x 4096); the shortest wait for the host there, 20 us a call.
+        us, library / here: 2,048 rows of x, 3584 x 3584 52 / 48, 2560 x 2048 26 / 24; 527 rows 4608 x 3584 29 / 26.
+        Longer rows and idle CUs: 527 rows, 2048 x 8192 43 / 46, 1536 x 8960 37 / 48; 1,500 rows, 4096 x 4096 49 / 54 in 224
+        columns on 0.89 of the CUs; two rounds: 2,048 rows, 4608 x 3584 60 / 76."""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 4 or N < self.EVEN_MIN_N
+                or K > self.EVEN_MAX_K):
+            return 0
+        rows = -(-M // 128)
+        for columns in range(96, 225, 32):
+            fill = rows * -(-N // columns) / self._num_cus
+            if fill <= 1:
+                return columns if (columns < 224 or fill >= 0.9) and (K <= self.EVEN_SHORT_K or fill >= 0.7) else 0
+        return 0
+
+    def linear_even(self, x, weight, bias, columns, out_f32=False):
+        """y = x W^T (+ bias) of many rows over the tiled copy of the weight, tiles of 128 x ``columns``."""
+        M, K = x.shape
+        N = weight.shape[0]
+        self._check(x, self.act_dtype, (M, K), "x")
+        y = self._new((M, N), torch.float32 if out_f32 else None)
+        self._call("gemm", "sl_gemm_even", _p(x), _p(weight.tiled), _p(bias), _p(y), M, N, K, int(out_f32), int(columns))
+        return y
 
     def linear_wide(self, x, weight, bias, out_f32=False, gated=False, act=0):
         M, K = x.shape

@@ -92,6 +92,10 @@ class Tuning:
     block_square_max_m: int = 1536
     # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
     shares_max_m: int = 2048
+    # products of more rows than the kernels above take in tiles that go round the CUs once (HipOps._even_columns)
+    even_min_n: int = 512
+    even_max_k: int = 4096
+    even_short_k: int = 2048
     # what a million float32 sums of a share cost that are written and read again by the norm (us)
     share_us: float = 0.9
     # gated and activated products of a prompt in the tiles of gemm_rounds.h (measured sides: HipOps._gated_rows): the fewest rows
