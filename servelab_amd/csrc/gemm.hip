@@ -76,11 +76,10 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(
 
 #if defined(SL_F32)
 // The same with K cut among the four wavefronts of a workgroup, which then own NC columns together: a matrix of few rows
-// still has a workgroup for every CU, and a lane's running sums are a quarter as long (1,536 columns of 8,960 at 1 / 3 / 8
-// rows: 22 / 39 / 60 -> 11 / 15 / 23 us, 5.0 TB/s at one row; errors halve).  W is read past the caches: a model reads every
+// still has a workgroup for every CU, and a lane's running sums are a quarter as long (1,536 columns of 8,960 at one row:
+// 22 -> 11 us, 5.0 TB/s; errors halve).  W is read past the caches: a model reads every
 // matrix once a step, and by the next one it has left them (us over matrices in turn, 1.2 GB in all, through the caches / past them:
-// 896 of 896 at one row 3.2 and 2.9, 1,536 of 1,536 at 1 / 8 rows 4.1 / 8.4 and 3.8 / 8.1, 2,560 of 2,048 6.7 / 14.5 and 6.2 / 14.2, 3,584
-// of 3,584 11.7 / 23.3 and 11.2 / 23.2; one matrix again and again is faster through them, 896 of 4,864 at 3 rows 7.2 and 8.3).
+// 896 of 896 at one row 3.2 and 2.9, 1,536 of 1,536 4.1 and 3.8, 2,560 of 2,048 6.7 and 6.2, 3,584 of 3,584 11.7 and 11.2).
 template <int MB, int NC>
 __global__ __launch_bounds__(256) void gemm_rows_split_kernel(
     const act_t* __restrict__ x, const act_t* __restrict__ w, const float* __restrict__ bias,
@@ -139,17 +138,16 @@ template <int NC>
 static const char* rows_split(const act_t* x, const act_t* w, const float* bias, void* y, int M, int N, int K, hipStream_t stream) {
   const int grid = (N + NC - 1) / NC;
   if (M == 1) gemm_rows_split_kernel<1, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  else if (M == 2) gemm_rows_split_kernel<2, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  else if (M <= 4) gemm_rows_split_kernel<4, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
-  else gemm_rows_split_kernel<8, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else gemm_rows_split_kernel<2, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
   return sl_launch_status();
 }
-#endif
+
+#include "gemm_f32_few.h"
+#else
 
 // The same product with the rows of x staged through LDS: the eight wavefronts of a workgroup own
 // four columns each and share every chunk of x, so x leaves the cache hierarchy once per 32 columns
-// of W instead of once per 4 (with 8 rows of x that was twice the bytes of W itself, and what the
-// float32 decode step spent most of its time pulling).  A lane keeps its own running sums over its
+// of W instead of once per 4 (with 8 rows of x that was twice the bytes of W itself).  A lane keeps its own running sums over its
 // share of K, as above.
 template <int MB>
 __global__ __launch_bounds__(512) void gemm_rows_shared_kernel(
@@ -208,7 +206,9 @@ __global__ __launch_bounds__(512) void gemm_rows_shared_kernel(
     }
 }
 
-// `shared`: 4 to 16 rows of x (to 8 of bfloat16) go through LDS once per 32 columns (gemm_rows_shared_kernel).
+#endif
+
+// `shared`, bfloat16: 4 to 8 rows of x go through LDS once per 32 columns (gemm_rows_shared_kernel).
 extern "C" const char* sl_gemm_rows(const void* x, const void* w, const float* bias, void* y,
                                     int M, int N, int K, int out_f32, int shared, hipStream_t stream) {
   SL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_rows: sizes must be positive");
@@ -219,32 +219,36 @@ extern "C" const char* sl_gemm_rows(const void* x, const void* w, const float* b
   const int waves = 4;
   const act_t* xx = (const act_t*)x;
   const act_t* ww = (const act_t*)w;
-  // (the staged form against a wavefront's columns, float32, 7B shape: from 4 rows on it wins, 8 rows 139 -> 113 us for
-  // gate/up and 176 -> 114 us for down, 16 rows 281 -> 172 and 494 -> 174 us; with 1 to 3 rows it loses up to 18 us of 44)
 #if defined(SL_F32)
-  // (measured, us, a wavefront's columns against a workgroup's: 1,536 columns of 1,536 / 8,960 at 3 rows 9.9 / 39 -> 5.8 / 15
-  // with two columns a workgroup; 3,584 of 18,944 at 1 / 3 / 8 rows 44 / 74 / 111 -> 42 / 47 / 62 with four.  Of many columns a
-  // wavefront each has enough to do from three rows on unless its rows are long: 151,936 of 1,536 at 3 rows 163
-  // against 177, 37,888 of 3,584 102 against 88; at 1 / 2 rows 93 / 99 -> 75 / 78.  Short rows leave the workgroup's 1,024
-  // values a step empty: 8,192 columns of 64 at 1 / 2 rows 3.1 / 4.3 and 4.7 / 6.8, 4,096 of 512 at 1 / 8 rows 3.6 / 11.2 and 4.2 /
-  // 12.4, 3,072 of 1,024 at one 4.1 and 4.7, 6,000 of 640 4.7 and 5.3.)
-  if (M <= 8 && N <= 2048 && K >= 512) return rows_split<2>(xx, ww, bias, y, M, N, K, stream);
-  if (M <= 8 && N <= 4096 && K >= (M == 1 ? 1536 : 1024)) return rows_split<4>(xx, ww, bias, y, M, N, K, stream);
+  // Three rows and more go through the matrix units, sixteen at a time (gemm_f32_few.h; two rows there are no faster than here: 17920 x 1536
+  // 20.1 us for 19.4, 1536 x 8960 13.4 for 13.0).
+  for (int m0 = 0; M > 2 && m0 < M; m0 += 16) {
+    const int rows = min(16, M - m0);
+    float* to = (float*)y + (size_t)m0 * N;
+    if (rows <= 4) gemm_f32_few<1>(xx + (size_t)m0 * K, ww, bias, to, rows, N, K, stream);
+    else if (rows <= 8) gemm_f32_few<2>(xx + (size_t)m0 * K, ww, bias, to, rows, N, K, stream);
+    else gemm_f32_few<4>(xx + (size_t)m0 * K, ww, bias, to, rows, N, K, stream);
+  }
+  if (M > 2) return sl_launch_status();
+  // (measured, us, a wavefront's columns against a workgroup's: 3,584 columns of 18,944 at one row 44 -> 42 with four columns a
+  // workgroup, 37,888 of 3,584 at 1 / 2 rows 93 / 99 -> 75 / 78.  Short rows leave the workgroup's 1,024
+  // values a step empty: 8,192 columns of 64 at 1 / 2 rows 3.1 / 4.3 and 4.7 / 6.8, 4,096 of 512 at one 3.6 and 4.2,
+  // 3,072 of 1,024 at one 4.1 and 4.7, 6,000 of 640 4.7 and 5.3.)
+  if (N <= 2048 && K >= 512) return rows_split<2>(xx, ww, bias, y, M, N, K, stream);
+  if (N <= 4096 && K >= (M == 1 ? 1536 : 1024)) return rows_split<4>(xx, ww, bias, y, M, N, K, stream);
   if (M == 1 && N > 4096 && K >= 768) return rows_split<2>(xx, ww, bias, y, M, N, K, stream);
-  if (N > 4096 && ((M == 2 && K >= 512) || (M <= 4 && K >= 2048))) return rows_split<4>(xx, ww, bias, y, M, N, K, stream);
-#endif
-  constexpr int SHARED_MAX_M = sizeof(act_t) == 4 ? 16 : 8;   // (16 rows of bfloat16 spill registers)
-  if (shared && M >= 4 && M <= SHARED_MAX_M) {
-    // (eight wavefronts a workgroup also for matrices of few rows: four, for twice the workgroups, measured
-    // slower: down of the 7B shape at 8 / 16 rows 125 / 214 us against 114 / 174)
+  if (N > 4096 && M == 2 && K >= 512) return rows_split<4>(xx, ww, bias, y, M, N, K, stream);
+#else
+  // (the staged form against a wavefront's columns: from 4 rows on it wins)
+  if (shared && M >= 4 && M <= 8) {                    // (16 rows spill registers)
     const int threads = 512;
     const int cols = 4 * threads / SL_WAVE;
     const dim3 grid((N + cols - 1) / cols);
     if (M <= 4) gemm_rows_shared_kernel<4><<<grid, threads, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
-    else if (M <= 8) gemm_rows_shared_kernel<8><<<grid, threads, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
-    else if constexpr (SHARED_MAX_M == 16) gemm_rows_shared_kernel<16><<<grid, threads, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
+    else gemm_rows_shared_kernel<8><<<grid, threads, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
     return sl_launch_status();
   }
+#endif
   // one row of x: a column per wavefront keeps the most wavefronts in flight;
   // more rows: 4 columns per wavefront share each load of x
   if (M == 1) {
@@ -253,8 +257,10 @@ extern "C" const char* sl_gemm_rows(const void* x, const void* w, const float* b
   }
   const dim3 grid((N + 4 * waves - 1) / (4 * waves));
   if (M == 2) gemm_rows_kernel<2, 4><<<grid, waves * SL_WAVE, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
+#if !defined(SL_F32)
   else if (M <= 4) gemm_rows_kernel<4, 4><<<grid, waves * SL_WAVE, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
   else gemm_rows_kernel<8, 4><<<grid, waves * SL_WAVE, 0, stream>>>(xx, ww, bias, y, M, N, K, out_f32);
+#endif
   return sl_launch_status();
 }
 
