@@ -524,6 +524,9 @@ extern "C" float sl_gemm_f32_split_us(int M, int N, int terms, int nsplit, int c
   return fminf(f32_split_us(256, M, N, terms, nsplit, cus), f32_split_us(128, M, N, terms, nsplit, cus));
 }
 
+constexpr int SPLIT_MIN_K = 512;
+extern "C" int sl_gemm_f32_split_min_k() { return SPLIT_MIN_K; }
+
 // nsplit > 1: K is cut into that many shares of whole segments, whose sums wait in `part`, [nsplit, M, N].  A product of
 // few tiles (the output projection and the down projection of a short prompt) leaves most CUs idle otherwise: 849 rows
 // of x, 1,536 rows of W of 8,960: 84 tiles.
@@ -537,7 +540,9 @@ extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const floa
   SL_CHECK(nsplit >= 1 && nsplit <= (K + SEGMENT_K - 1) / SEGMENT_K, "gemm_f32_mfma: at most one share of K per 512 terms");
   SL_CHECK(nsplit == 1 || (part != nullptr && (uintptr_t)part % 16 == 0 && (uintptr_t)y % 16 == 0),
            "gemm_f32_mfma: shares of K need an aligned buffer for their sums");
-  const bool split = M > 64 && K % 32 == 0;
+  // (three terms from 512 values of k on: at 32 and 64 their error is 1.17e-7 and 1.46e-7 of a result, of float32 instructions 1.03e-7
+  // and 1.44e-7, and below 512 the runs of either sign are unequal, so that results lie 4e-9 to 1.4e-8 of their spread too low)
+  const bool split = M > 64 && K % 32 == 0 && K >= SPLIT_MIN_K;
   const int rows = M <= 64 ? 32 : 128;
   const dim3 grid((N + 127) / 128, (M + rows - 1) / rows, nsplit);
   SL_CHECK(grid.y <= 65535, "gemm_f32_mfma: more than 65535 row tiles");
@@ -559,7 +564,7 @@ extern "C" const char* sl_gemm_f32_mfma(const void* x, const void* w, const floa
     const char* e = nsplit > 1 ? (wide ? launch(gemm_f32_split_kernel<4, true>, 256) : launch(gemm_f32_split_kernel<2, true>, 128))
                                : (wide ? launch(gemm_f32_split_kernel<4, false>, 256) : launch(gemm_f32_split_kernel<2, false>, 128));
     if (e) return e;
-  } else {                                             // (rows that end in half a chunk of 32)
+  } else {                                             // (short rows, and rows that end in half a chunk of 32)
     if (nsplit > 1) run(gemm_f32_mfma_kernel<2, 2, 2, 2, true>);
     else run(gemm_f32_mfma_kernel<2, 2, 2, 2, false>);
   }

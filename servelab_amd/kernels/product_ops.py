@@ -706,9 +706,9 @@ class ProductOps:
     F32_MFMA_MIN_M = 17           # float32 products of this many rows or more run on the matrix cores
 
     def linear_f32_mfma(self, x, w, bias):
-        """Float32 product on the matrix cores, K % 16 == 0: more than 64 rows and K % 32 == 0 by products of
+        """Float32 product on the matrix cores, K % 16 == 0: more than 64 rows, K % 32 == 0 and 512 at least by products of
         three bfloat16 terms an operand, which together are the float (gemm_f32_split.h: closer to 64 bits than
-        float32 instructions), else by float32 instructions; float32 sums."""
+        float32 instructions there), else by float32 instructions; float32 sums."""
         if self.act_dtype != torch.float32:
             raise KernelError("linear_f32_mfma is for the float32 table only")
         M, K = x.shape
@@ -726,7 +726,8 @@ class ProductOps:
         """Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated
         time, which is the tiles' rounds over the CUs plus, for several shares, the traffic of the partial sums and
         their addition."""
-        rows, split = 32 if M <= 64 else 128, M > 64 and K % 32 == 0
+        rows = 32 if M <= 64 else 128
+        split = M > 64 and K % 32 == 0 and K >= self._lib["gemm"].sl_gemm_f32_split_min_k()
         tiles = -(-M // rows) * -(-N // 128)
         best, least, segments = 1, float("inf"), -(-K // self.F32_SEGMENT)
         if split:

@@ -17,9 +17,9 @@ def draws(M, N, K, spread):
     return x * two(M, K), w * two(N, K)
 
 
-# a row and a column past a tile of 128, past one of 256 (the wide form where many tiles fill the CUs), one chunk of 32, a chunk past a
-# segment of 512, a last share of one chunk
-@pytest.mark.parametrize("M,N,K", [(129, 129, 32), (70, 257, 544), (900, 8193, 96), (1025, 8191, 1056), (128, 256, 1536)])
+# a row and a column past a tile of 128, past one of 256 (the wide form where many tiles fill the CUs), the shortest rows of three terms and
+# the longest of float32 instructions, a chunk past a segment of 512, a last share of one chunk
+@pytest.mark.parametrize("M,N,K", [(129, 129, 32), (129, 129, 480), (129, 129, 512), (70, 257, 544), (900, 8193, 608), (1025, 8191, 1056), (128, 256, 1536)])
 @pytest.mark.parametrize("spread", [0, 12])
 def test_sums_of_terms(M, N, K, spread):
     ops = HipOps(torch.float32, DEV)
@@ -45,7 +45,7 @@ def test_both_widths_are_chosen():
     assert lib.sl_gemm_f32_split_us(512, 8192, 1536, 1, 0) == 0
 
 
-@pytest.mark.parametrize("M,N,K,shares", [(130, 300, 1056, 1), (130, 300, 1056, 3), (1024, 8192, 64, 1)])
+@pytest.mark.parametrize("M,N,K,shares", [(130, 300, 1056, 1), (130, 300, 1056, 3), (1024, 8192, 512, 1)])
 def test_operands_that_are_not_finite_or_hardly(M, N, K, shares):
     ops = HipOps(torch.float32, DEV)
     ops._f32_shares = lambda *_: shares
