@@ -880,23 +880,47 @@ void attention_mfma_shared_kernel(const AttnParams P) {
 // output, and what lies in their place may be anything (a kernel of its own: the test costs the
 // plain one 1.9 of its 5.4 us for one request of the 7B shape in 16 shares).
 constexpr int COMBINE_PER_LANE = 4;
-template <bool SKIP>
+template <bool SKIP, int BATCH>
 __global__ __launch_bounds__(64) void attention_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, int nsplit, int nh,
     int part_row0, __bf16* __restrict__ out, int out_rows) {
   __shared__ float ws[64 * COMBINE_PER_LANE];
   const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
   const size_t base = ((size_t)r * nh + h) * nsplit;
-  float m[COMBINE_PER_LANE], l[COMBINE_PER_LANE], top = -INFINITY;
+  const float* po = part_o + base * D;
+  // A lane takes channels lane, lane + 64, ...; the partial outputs of BATCH shares are asked for
+  // together, all channels of a lane at once, the first of them with the maxima, the next before the last are added up (a batch
+  // is a trip to memory: with eight shares a batch
+  // and the channels one after the other, 64 shares took 2 us longer than 32; with the last shares
+  // below a whole batch one by one, 21 took 3 us longer than 16 or 24).  Added in the order of the
+  // shares, whatever the batches.  (Past the last channel that one again, never stored.)
+  constexpr int DI = (D + 63) / 64;
+  float v[BATCH][DI];
+  auto ask = [&](int j) {
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) {
+      const float* row = po + (size_t)(j + u < nsplit ? j + u : nsplit - 1) * D;
+#pragma unroll
+      for (int di = 0; di < DI; ++di) v[u][di] = row[64 * di + 64 <= D ? lane + 64 * di : min(lane + 64 * di, D - 1)];
+    }
+  };
+  float m[COMBINE_PER_LANE], l[COMBINE_PER_LANE];
 #pragma unroll
   for (int i = 0; i < COMBINE_PER_LANE; ++i) {
-    const int j = lane + 64 * i;
     m[i] = -INFINITY;
     l[i] = 0.f;
-    if (j < nsplit) {
-      m[i] = part_ml[(base + j) * 2];
-      l[i] = part_ml[(base + j) * 2 + 1];
+    if (64 * i < nsplit) {                              // (the same for all lanes)
+      const size_t at = (base + min(lane + 64 * i, nsplit - 1)) * 2;
+      m[i] = part_ml[at];
+      l[i] = part_ml[at + 1];
     }
+  }
+  ask(0);
+  __builtin_amdgcn_sched_barrier(0);
+  float top = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < COMBINE_PER_LANE; ++i) {
+    if (lane + 64 * i >= nsplit) m[i] = -INFINITY, l[i] = 0.f;
     top = fmaxf(top, m[i]);
   }
   const float mx = wave_max(top);
@@ -910,31 +934,23 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(
   const float denom = wave_sum(mine);
   __syncthreads();
   const float inv = 1.f / denom;
-  const float* po = part_o + base * D;
-  // A lane takes channels lane, lane + 64, ...; the partial outputs of sixteen shares are asked for
-  // together, all channels of a lane at once (a batch is a trip to memory: with eight shares a batch
-  // and the channels one after the other, 64 shares took 2 us longer than 32; with the last shares
-  // below a whole batch one by one, 21 took 3 us longer than 16 or 24).  Added in the order of the
-  // shares, whatever the batches.
-  constexpr int DI = (D + 63) / 64, BATCH = 16;
   float acc[DI];
 #pragma unroll
   for (int di = 0; di < DI; ++di) acc[di] = 0.f;
   for (int j = 0; j < nsplit; j += BATCH) {
-    float v[BATCH][DI];
+    float now[BATCH][DI];
 #pragma unroll
-    for (int u = 0; u < BATCH; ++u) {
-      const float* row = po + (size_t)(j + u < nsplit ? j + u : nsplit - 1) * D;
+    for (int u = 0; u < BATCH; ++u)
 #pragma unroll
-      for (int di = 0; di < DI; ++di) v[u][di] = 64 * di + 64 <= D || lane + 64 * di < D ? row[lane + 64 * di] : 0.f;
-    }
+      for (int di = 0; di < DI; ++di) now[u][di] = v[u][di];
+    if (j + BATCH < nsplit) ask(j + BATCH);
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
       // (no branch here: under one the compiler may move each load down to its use; beyond the last share the
       // weight is 0 and the value that of the last share)
       const float w = j + u < nsplit ? ws[j + u] : 0.f;
 #pragma unroll
-      for (int di = 0; di < DI; ++di) acc[di] += SKIP && w == 0.f ? 0.f : w * v[u][di];
+      for (int di = 0; di < DI; ++di) acc[di] += SKIP && w == 0.f ? 0.f : w * now[u][di];
     }
   }
 #pragma unroll
@@ -942,6 +958,14 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(
     const int d = lane + 64 * di;
     if (d < D) out[out_index(out_rows, nh, (size_t)(part_row0 + r), h * D + d)] = (__bf16)(acc[di] * inv);
   }
+}
+// (a prompt's two to four shares: four loads a channel and not sixteen; 2,048 rows of 16 heads of 128 in two shares 15.7 -> 11.4 us)
+template <bool SKIP>
+static void attention_combine(const float* part_o, const float* part_ml, int nsplit, int nh, int rows, int part_row0, __bf16* out,
+                              int out_rows, hipStream_t stream) {
+  auto run = [&](auto kernel) { kernel<<<dim3(rows, nh), 64, 0, stream>>>(part_o, part_ml, nsplit, nh, part_row0, out, out_rows); };
+  if (nsplit <= 4) run(attention_combine_kernel<SKIP, 4>);
+  else run(attention_combine_kernel<SKIP, 16>);
 }
 
 extern "C" int sl_attention_mfma_max_splits() { return 64 * COMBINE_PER_LANE; }
@@ -1027,10 +1051,8 @@ extern "C" const char* sl_attention_mfma(
 #undef SL_SPLIT
     const char* e = sl_launch_status();
     if (e || out == nullptr) return e;               // (out == nullptr: the shares are left to their reader)
-    if (one_length) attention_combine_kernel<true><<<dim3(num_seqs, nh), 64, 0, stream>>>(
-        part_o, part_ml, nsplit, nh, part_row0, (__bf16*)out, out_rows);
-    else attention_combine_kernel<false><<<dim3(num_seqs, nh), 64, 0, stream>>>(
-        part_o, part_ml, nsplit, nh, part_row0, (__bf16*)out, out_rows);
+    if (one_length) attention_combine<true>(part_o, part_ml, nsplit, nh, num_seqs, part_row0, (__bf16*)out, out_rows, stream);
+    else attention_combine<false>(part_o, part_ml, nsplit, nh, num_seqs, part_row0, (__bf16*)out, out_rows, stream);
     return sl_launch_status();
   }
   // Prompt portions.  The workgroups that share a block through LDS, or one
@@ -1082,8 +1104,7 @@ extern "C" const char* sl_attention_mfma(
     if (nsplit > 1) {
       const char* e = sl_launch_status();
       if (e) return e;
-      attention_combine_kernel<false><<<dim3(part_rows, nh), 64, 0, stream>>>(part_o, part_ml, nsplit, nh,
-                                                                    part_row0, (__bf16*)out, out_rows);
+      attention_combine<false>(part_o, part_ml, nsplit, nh, part_rows, part_row0, (__bf16*)out, out_rows, stream);
     }
   }
   return sl_launch_status();
@@ -1094,6 +1115,6 @@ extern "C" const char* sl_attention_combine(const float* part_o, const float* pa
                                             hipStream_t stream) {
   SL_CHECK(part_o != nullptr && part_ml != nullptr && out != nullptr, "attention_combine: shares and a result");
   SL_CHECK(rows > 0 && nh > 0 && nh <= 65535 && nsplit >= 1 && nsplit <= 64 * COMBINE_PER_LANE, "attention_combine: bad sizes");
-  attention_combine_kernel<false><<<dim3(rows, nh), 64, 0, stream>>>(part_o, part_ml, nsplit, nh, 0, (__bf16*)out, 0);
+  attention_combine<false>(part_o, part_ml, nsplit, nh, rows, 0, (__bf16*)out, 0, stream);
   return sl_launch_status();
 }
