@@ -11,9 +11,9 @@
 //  - Running sums: sixteen blocks, KW parts and E of the four values of a step apart, so that each is as short as in FMAs of a
 //    wavefront or four (64 or 256 sums of K / 64 or K / 256 terms): the error against 64 bits stays what it was, 0.9 to 1.2e-7 of a result, or
 //    shrinks (16 rows of 3584 x 18944 3.2e-7 -> 1.8e-7).
-// us with FMAs / here (matrices in turn, 1.3 GB in all): 17920 x 1536 at 3 / 6 / 16 rows 27 / 37 / 62 -> 21 / 27 / 42; 1536 x 8960 15.8 / 23 / 94 -> 14.3 / 18
-// / 29; 1536 x 1536 5.5 / 8.1 / 27 -> 5.1 / 6.3 / 8.7; 151936 x 1536 165 / 196 / 337 -> 151 / 163 / 281 (6.2 TB/s at three rows); 896 x 4864 7.4 / 11 / 53
-// -> 6.5 / 8.5 / 14; 3584 x 18944 59 / 79 / 186 -> 52 / 62 / 78.
+// us with FMAs / here (matrices in turn, 1.3 GB in all): 17920 x 1536 at 3 / 5 / 16 rows 27 / 37 / 62 -> 22 / 27 / 43; 1536 x 8960 16 / 22 / 94 -> 16
+// / 20 / 31; 1536 x 1536 5.5 / 8.0 / 27 -> 5.3 / 6.3 / 8.7; 151936 x 1536 167 / 196 / 338 -> 152 / 159 / 291 (6.1 TB/s at three rows); 896 x 4864 8.1 / 11 / 53
+// -> 7.9 / 8.8 / 15; 3584 x 18944 58 / 78 / 186 -> 50 / 57 / 84.
 template <int MB, int C, int KW, int U, int E>
 __global__ __launch_bounds__(KW == 8 ? 512 : 256) void gemm_f32_few_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K) {
@@ -98,7 +98,8 @@ __global__ __launch_bounds__(KW == 8 ? 512 : 256) void gemm_f32_few_kernel(
 }
 
 // Which of them, measured for 16 matrices of 896 to 151,936 rows and rows of 64 to 18,944 values: of few columns a wavefront takes four or
-// eight, so that every CU has some; of long rows eight wavefronts share K; of many columns 8 or 16 read a load of x, and of very many two
+// eight, so that every CU has some; of long rows eight wavefronts share K, and of more than 2,048 such columns each takes sixteen (3584 x 18944 at 3 / 16 rows
+// in eight 57 / 111 us, in sixteen 50 / 84; up to eight rows of 2560 x 3072 and 4096 x 4096 sixteen lose up to 7 %); of many columns 8 or 16 read a load of x, and of very many two
 // wavefronts share K (151936 x 896 at three rows 104 us for 91, 17920 x 1536 21 for 22).
 template <int MB>
 static void gemm_f32_few(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, hipStream_t stream) {
@@ -108,7 +109,8 @@ static void gemm_f32_few(const float* x, const float* w, const float* bias, floa
   const bool few = N <= 4096, lengthy = K >= 3072;
   if constexpr (MB <= 2) {
     if (few && lengthy && N < 1024) SL_FEW(1, 8, 2, 4);
-    else if (few && lengthy) SL_FEW(2, 8, 2, 4);
+    else if (few && lengthy && (N <= 2048 || K < 8192)) SL_FEW(2, 8, 2, 4);
+    else if (few && lengthy) SL_FEW(4, 8, 2, 4);
     else if (few) SL_FEW(1, 4, 4, 4);
     else if (N <= 32768) SL_FEW(2, 4, 4, (MB == 1 ? 4 : 2));
     else if constexpr (MB == 1) {
@@ -117,7 +119,8 @@ static void gemm_f32_few(const float* x, const float* w, const float* bias, floa
     } else SL_FEW(4, 2, 2, 2);
   } else {
     if (few && lengthy && N < 1024) SL_FEW(1, 8, 2, 2);
-    else if (few && lengthy) SL_FEW(2, 8, 2, 2);
+    else if (few && lengthy && N <= 2048) SL_FEW(2, 8, 2, 2);
+    else if (few && lengthy) SL_FEW(4, 8, 2, 2);
     else if (N <= 16384) SL_FEW(2, 4, 2, 1);
     else SL_FEW(4, 4, 2, 1);
   }

@@ -11,7 +11,7 @@ DEV = "cuda:0"
 # rows of each form, the last of a block of four and the first of the next, and a second sixteen; columns that no wavefront's divide, each line of the choice of
 # form and its other side; K shorter than a step of 64 and than the parts of K, not a multiple of it, long
 @pytest.mark.parametrize("M", [3, 4, 5, 8, 9, 16, 19])
-@pytest.mark.parametrize("N,K", [(1, 4), (6, 64), (1023, 3072), (1029, 3076), (4096, 196), (4099, 324), (16387, 260), (32771, 132), (32770, 2052)])
+@pytest.mark.parametrize("N,K", [(1, 4), (6, 64), (1023, 3072), (1029, 3076), (2051, 3140), (2051, 8196), (4096, 196), (4099, 324), (16387, 260), (32771, 132), (32770, 2052)])
 def test_sums(M, N, K):
     ops = HipOps(torch.float32, DEV)
     g = torch.Generator(device=DEV).manual_seed(M + N)
