@@ -776,9 +776,8 @@ extern "C" const char* sl_gemm_skinny_shares(const float* shares_o, const float*
 // tile's are used up (a ring of R k-steps per wavefront), so they are in flight
 // during the reduction and the epilogue.  NS is a template argument: the loop is
 // straight-line code whose every wait the compiler can count (with a run-time
-// number of steps it waited for all loads at every step).  Result as
-// gemm_skinny_kernel's CONSUMER forms, bit for bit: the same products in the same
-// order.
+// number of steps it waited for all loads at every step).  The products
+// are those of gemm_few_kernel's CONSUMER forms over whole tiles.
 template <bool GATED, int PARTS, int NS, int R>
 __global__ __launch_bounds__(512) void gemm_resident_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ wt, const float* __restrict__ bias,
@@ -787,7 +786,7 @@ __global__ __launch_bounds__(512) void gemm_resident_kernel(
   static_assert(NS % R == 0, "the ring divides the steps");
   __shared__ f32x4 red[2][WAVES][64];
   __shared__ float wsum[WAVES][16];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);     // (a scalar: see gemm_skinny_kernel)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);     // (a scalar: as in gemm_few_kernel)
   const int lane = threadIdx.x % 64, i = lane & 15, gq = lane >> 4;
   const int ntiles = (N + 15) / 16;
   const int ks0 = NS * wave;
