@@ -5,9 +5,11 @@
 // six products of terms down to 2^-18 of it; the three left out are at most 2^-26 of it together, a quarter of a float's rounding.
 // Products of bfloat16 are exact in float, and a matrix instruction adds 32 of them to the running sum at once.  It rounds that sum down,
 // not to nearest: left so, every result lay 5e-8 to 6e-7 of their spread too low, and the logits of a 6-layer model 3.1e-6 off
-// instead of 2.8e-6.  Hence runs of RUN chunks are summed apart, every other one with x's sign turned, whose sums are
-// subtracted.  Error of a result against 64 bits 2.6e-7 for 4.1e-7 with float32 instructions and sums of 512 terms (30 sizes,
-// inputs of several distributions), of those logits 2.4e-6 for 2.9e-6.
+// instead of 2.8e-6.  Hence runs of chunks are summed apart, every other one with x's sign turned, whose sums are
+// subtracted; runs of either sign are equally many and long, or but one chunk.  Mean offset of two million results, in their spread, no more
+// than that of float32 instructions, 3e-10 (an odd number of chunks: 4e-10 at 544 values of k); with runs of 8 chunks at every k
+// 8.0e-9 at 768, 6.1e-9 at 1,280, 4.6e-9 at 896.  Error of a result against 64 bits 2.4e-7 to 2.6e-7 for 3.7e-7 to 4.1e-7 with float32 instructions
+// and sums of 512 terms, of those logits 2.4e-6 for 2.9e-6.
 // A result that is not finite is worked out again term by term: an infinite operand's rests are NaN.
 //
 // Bound by the matrix units, six instructions of 16 cycles in the place of eight of 32 (16 x 16 results, 32 terms), and their power:
@@ -86,9 +88,12 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
     v[j][1] = *(const split_f32x4*)(src[j] + 4);
     src[j] += CK;
   };
-  // chunks of a run of RUN that are multiplied with -x, from the first on every other run
+  // Runs of RUN chunks, every other one multiplied with -x, from the first on; the chunks behind the last pair of such runs make a
+  // pair of half as many each, an odd one at the end a run of its own.
   constexpr int RUN = 8;
-  auto sign_of = [&](int c) { return (c - first) / RUN & 1 ? 1.f : -1.f; };
+  const int paired = first + (last - first) / (2 * RUN) * (2 * RUN), half = (last - paired) / 2;
+  auto run_end = [&](int c) { return c < paired ? c + RUN : c < paired + half ? paired + half : c < paired + 2 * half ? paired + 2 * half : last; };
+  auto sign_of = [&](int c) { return (c < paired ? ((c - first) / RUN & 1) != 0 : c >= paired + half && c < paired + 2 * half) ? 1.f : -1.f; };
   auto store = [&](int stage, int j) {
     split_bf16x8 terms[3];
     if (j == 0) v[0][0] *= sign_of(first), v[0][1] *= sign_of(first);
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
   __syncthreads();
   int c = first, stage = 0;
   while (c < last) {
-    const int c1 = c + RUN < last ? c + RUN : last;
+    const int c1 = run_end(c);
     const float sign = sign_of(c);
     for (; c < c1; ++c, stage ^= 1) {
       const char* from = stages + stage * STAGE;

@@ -33,6 +33,22 @@ def test_sums_of_terms(M, N, K, spread):
         assert ((got - want).abs() <= bar * size).all()
 
 
+# whole pairs of runs of eight chunks; one chunk more, and two; runs behind the last pair, of even and odd numbers of chunks; a share of its own for them
+@pytest.mark.parametrize("K,shares", [(512, 1), (1024, 2), (544, 1), (576, 2), (608, 1), (672, 1), (768, 1), (768, 2), (896, 1), (1280, 1), (1280, 3)])
+def test_sums_lie_on_neither_side(K, shares):
+    """The matrix unit rounds sums down; that cancels only where as many chunks are summed with either sign."""
+    ops = HipOps(torch.float32, DEV)
+    ops._f32_shares = lambda *_: shares
+    x, w = draws(1024, 2048, K, 0)
+    want = x.double() @ w.double().T
+    off, spread = ops.linear_f32_mfma(x, w, None).double() - want, want.square().mean().sqrt()
+    # float32 instructions are 3.7e-7 to 4.1e-7 off here, and two terms an operand instead of three 4e-6
+    assert off.norm() / want.norm() <= 3.2e-7
+    # The mean over 2 M results, which share 3,072 rows: 3e-10 at whole pairs of runs (float32 instructions: 6e-10 at most).  A run of two chunks
+    # more of one sign than of the other is 1.3e-9.
+    assert abs(off.mean() / spread) <= 9e-10
+
+
 def test_both_widths_are_chosen():
     ops = HipOps(torch.float32, DEV)
     lib = ops._lib["gemm"]
