@@ -1,7 +1,8 @@
 // Float32 products of more than 64 rows on the bfloat16 matrix units: y[M, N] = x[M, K] W[N, K]^T, K % 32 == 0.  Included by gemm.hip.
 //
 // An operand is three bfloat16 terms, each what the ones before left over, rounded to nearest: 8 + 8 + 8 bits of significand, so
-// that together they are the float itself (above 2^-109 in size; below, what a third term loses lies under 2^-133).  A product is the
+// that together they are the float itself.  They are terms of 2^24 times the operand, or what they leave of one below 2^-109 would lie below
+// bfloat16's least value (left at its size, an operand of 2^-116 was 2^-19 off and one of 2^-135 gone).  A product is the
 // six products of terms down to 2^-18 of it; the three left out are at most 2^-26 of it together, a quarter of a float's rounding.
 // Products of bfloat16 are exact in float, and a matrix instruction adds 32 of them to the running sum at once.  It rounds that sum down,
 // not to nearest: left so, every result lay 5e-8 to 6e-7 of their spread too low, and the logits of a 6-layer model 3.1e-6 off
@@ -10,7 +11,7 @@
 // than that of float32 instructions, 3e-10 (an odd number of chunks: 4e-10 at 544 values of k); with runs of 8 chunks at every k
 // 8.0e-9 at 768, 6.1e-9 at 1,280, 4.6e-9 at 896.  Error of a result against 64 bits 2.4e-7 to 2.6e-7 for 3.7e-7 to 4.1e-7 with float32 instructions
 // and sums of 512 terms, of those logits 2.4e-6 for 2.9e-6.
-// A result that is not finite is worked out again term by term: an infinite operand's rests are NaN.
+// A result that is not finite, as a sum of 2^48 times itself, is worked out again term by term: an infinite operand's rests are NaN.
 //
 // Bound by the matrix units, six instructions of 16 cycles in the place of eight of 32 (16 x 16 results, 32 terms), and their power:
 // 2.3 us a chunk of 32 k on all CUs, 1.9 on one.  A workgroup of eight wavefronts, one a CU, owns 128 rows of x by 256 of W, a
@@ -93,10 +94,11 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
   constexpr int RUN = 8;
   const int paired = first + (last - first) / (2 * RUN) * (2 * RUN), half = (last - paired) / 2;
   auto run_end = [&](int c) { return c < paired ? c + RUN : c < paired + half ? paired + half : c < paired + 2 * half ? paired + 2 * half : last; };
-  auto sign_of = [&](int c) { return (c < paired ? ((c - first) / RUN & 1) != 0 : c >= paired + half && c < paired + 2 * half) ? 1.f : -1.f; };
+  constexpr float SCALE = 1 << 24;
   auto store = [&](int stage, int j) {
     split_bf16x8 terms[3];
-    if (j == 0) v[0][0] *= sign_of(first), v[0][1] *= sign_of(first);
+    const float scale = j == 0 ? -SCALE : SCALE;
+    v[j][0] *= scale, v[j][1] *= scale;
     split_terms(v[j], terms);
 #pragma unroll
     for (int p = 0; p < 3; ++p) *(split_bf16x8*)(stages + stage * STAGE + p * PLANE + 8192 * j + 16 * t) = terms[p];
@@ -123,9 +125,8 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
   ++asked;
   __syncthreads();
   int c = first, stage = 0;
-  while (c < last) {
+  for (float sign = -1.f; c < last; sign = -sign) {
     const int c1 = run_end(c);
-    const float sign = sign_of(c);
     for (; c < c1; ++c, stage ^= 1) {
       const char* from = stages + stage * STAGE;
       char* to = stages + (stage ^ 1) * STAGE + 16 * t;
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
         x0[a] = read(0, x_at, a);
       }
       constexpr int P = 24 * B, S = 12 * ITEMS, S0 = 3 * B / 2, SPAN = P - 2 * B;      // products; steps of the conversion, the first one's place
-      const float sign_next = sign_of(c + 1);
+      const float scale_next = c + 1 < c1 ? SCALE * sign : -SCALE * sign;
       unsigned u[3][4];
       split_f32x2 r;
       in_order<P>([&](auto slot) __attribute__((always_inline)) {
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
           constexpr int q = s / 12, e = s / 3 % 4, p = s % 3;
           if constexpr (p == 0) {
             r = split_f32x2{v[q][e >> 1][2 * (e & 1)], v[q][e >> 1][2 * (e & 1) + 1]};
-            if constexpr (q == 0) r *= sign_next;
+            r *= q == 0 ? scale_next : SCALE;
           }
           u[p][e] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, split_bf16x2));
           if constexpr (p < 2) {
@@ -189,9 +190,9 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (n + e >= N) continue;
-        float s = sum[a][b][e];
+        float s = sum[a][b][e] * (1 / (SCALE * SCALE));
         if (!(fabsf(s) < INFINITY)) {
-          // an operand that is not finite, or beyond the largest bfloat16, or a sum past the largest float: term by term
+          // an operand that is not finite, or 2^24 times it beyond the largest bfloat16, or a sum past the largest float: term by term
           s = 0.f;
           const float* xr = x + (size_t)m * K;
           const float* wr = w + (size_t)(n + e) * K;

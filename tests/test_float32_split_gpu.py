@@ -49,6 +49,19 @@ def test_sums_lie_on_neither_side(K, shares):
     assert abs(off.mean() / spread) <= 9e-10
 
 
+# sizes whose third term, second and first lie below the least bfloat16, subnormal floats, the least ones
+@pytest.mark.parametrize("M,N,K", [(130, 300, 1056), (1024, 8192, 512)])
+@pytest.mark.parametrize("e", [-112, -118, -126, -135, -142, -148])
+def test_operands_of_the_least_sizes(M, N, K, e):
+    ops = HipOps(torch.float32, DEV)
+    x, w = draws(M, N, K, 0)
+    small = lambda t: t * 2.0 ** -74 * 2.0 ** (e + 74)
+    for a, b in ((small(x), w * 2.0 ** 40), (x * 2.0 ** 40, small(w))):
+        want = a.double() @ b.double().T
+        # no further off than at ordinary sizes: 2.4e-7 to 2.6e-7 there
+        assert (ops.linear_f32_mfma(a, b, None).double() - want).norm() / want.norm() <= 3.2e-7
+
+
 def test_both_widths_are_chosen():
     ops = HipOps(torch.float32, DEV)
     lib = ops._lib["gemm"]
