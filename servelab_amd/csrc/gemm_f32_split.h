@@ -11,7 +11,7 @@
 // than that of float32 instructions, 3e-10 (an odd number of chunks: 4e-10 at 544 values of k); with runs of 8 chunks at every k
 // 8.0e-9 at 768, 6.1e-9 at 1,280, 4.6e-9 at 896.  Error of a result against 64 bits 2.4e-7 to 2.6e-7 for 3.7e-7 to 4.1e-7 with float32 instructions
 // and sums of 512 terms, of those logits 2.4e-6 for 2.9e-6.
-// A result that is not finite, as a sum of 2^48 times itself, is worked out again term by term: an infinite operand's rests are NaN.
+// A result that is not finite, as a sum of 2^48 times itself, is worked out again by float32 instructions: an infinite operand's rests are NaN.
 //
 // Bound by the matrix units, six instructions of 16 cycles in the place of eight of 32 (16 x 16 results, 32 terms), and their power:
 // 2.3 us a chunk of 32 k on all CUs, 1.9 on one.  A workgroup of eight wavefronts, one a CU, owns 128 rows of x by 256 of W, a
@@ -180,6 +180,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
       }
   }
   // lane: row lane % 16 of x's tile, four rows of W's from 4 (lane / 16) on
+  unsigned long long again = 0;                        // bit 4 (B a + b) + e: a result that is not finite
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     const int m = m0 + 64 * wm + 16 * a + (lane & 15);
@@ -190,16 +191,52 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (n + e >= N) continue;
-        float s = sum[a][b][e] * (1 / (SCALE * SCALE));
-        if (!(fabsf(s) < INFINITY)) {
-          // an operand that is not finite, or 2^24 times it beyond the largest bfloat16, or a sum past the largest float: term by term
-          s = 0.f;
-          const float* xr = x + (size_t)m * K;
-          const float* wr = w + (size_t)(n + e) * K;
-          for (int k = CK * first; k < CK * last; ++k) s = fmaf(xr[k], wr[k], s);
-        }
-        y[(size_t)m * N + n + e] = s + (bias != nullptr ? bias[n + e] : 0.f);
+        const float s = sum[a][b][e] * (1 / (SCALE * SCALE));
+        if (fabsf(s) < INFINITY) y[(size_t)m * N + n + e] = s + (bias != nullptr ? bias[n + e] : 0.f);
+        else again |= 1ull << (4 * (B * a + b) + e);
       }
+    }
+  }
+  // An operand that is not finite, or 2^24 times it beyond the largest bfloat16, or a sum past 2^80: by float32 instructions and sums of
+  // SEGMENT_K terms.  Sixteen rows of x at a time; what is finite beside them stays.
+  for (int a = 0; a < 4; ++a) {
+    const unsigned row = (unsigned)(again >> (4 * B * a)) & ((1u << 4 * B) - 1);
+    if (__builtin_amdgcn_ballot_w64(row != 0) == 0) continue;          // (the whole wavefront)
+    const int mine = m0 + 64 * wm + 16 * a + (lane & 15), wrow = n0 + 16 * B * wn + (lane & 15);
+    const float *xr = x + (size_t)min(mine, M - 1) * K + 4 * (lane >> 4), *wr[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) wr[b] = w + (size_t)min(wrow + 16 * b, N - 1) * K + 4 * (lane >> 4);
+    split_f32x4 total[B], part[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) total[b] = part[b] = split_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = CK * first; k < CK * last; k += CK) {
+      split_f32x4 xv[2], wv[2][B];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        xv[u] = *(const split_f32x4*)(xr + k + 16 * u);
+#pragma unroll
+        for (int b = 0; b < B; ++b) wv[u][b] = *(const split_f32x4*)(wr[b] + k + 16 * u);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int b = 0; b < B; ++b) part[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][b][j], xv[u][j], part[b], 0, 0, 0);
+      if ((k + CK) % SEGMENT_K != 0 && k + CK < CK * last) continue;
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        total[b] += part[b];
+        part[b] = split_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int n = n0 + 16 * B * wn + 16 * b + 4 * (lane >> 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (row >> (4 * b + e) & 1) y[(size_t)mine * N + n + e] = total[b][e] + (bias != nullptr ? bias[n + e] : 0.f);
     }
   }
 }

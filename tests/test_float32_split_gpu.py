@@ -91,3 +91,32 @@ def test_operands_that_are_not_finite_or_hardly(M, N, K, shares):
     there = torch.isfinite(want)
     size = torch.where(torch.isfinite(x), x, 0).double().abs() @ torch.where(torch.isfinite(w), w, 0).double().abs().T
     assert ((got.double() - want).abs()[there] <= (K * 2.0 ** -24 * size)[there]).all() and there.sum() > 0.9 * clean.numel()
+
+
+def test_results_that_are_not_finite_take_no_time_to_speak_of():
+    """A NaN early in a prompt makes every product behind it end in NaN: one row, and all of them."""
+    ops = HipOps(torch.float32, DEV)
+    x, w = draws(849, 1536, 1536, 0)
+    ops._f32_shares = lambda *_: 1
+    clean = ops.linear_f32_mfma(x, w, None)
+
+    def us():
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(4):
+                y = ops.linear_f32_mfma(x, w, None)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 250)
+        return best, y
+    finite, _ = us()
+    x[5, 7] = float("nan")
+    one, y = us()
+    assert torch.isnan(y[5]).all() and torch.equal(torch.cat([y[:5], y[6:]]), torch.cat([clean[:5], clean[6:]]))
+    x[:, 7] = float("nan")
+    all_rows, y = us()
+    assert torch.isnan(y).all()
+    # float32 instructions, at two and a half times the matrix units' time, behind the product; a lane a result took 8 and 90 times it
+    assert one < 4 * finite and all_rows < 8 * finite, (finite, one, all_rows)
