@@ -18,7 +18,8 @@
 // wavefront 64 x 64.  A chunk goes from memory to registers, is split there once for the workgroup, and lies in LDS as three planes of
 // rows of 64 bytes (a wavefront's read of an operand is 1 KB in a row); two stages.  The order of a chunk is laid down
 // instruction by instruction: left to itself the compiler converts in front of all products and loads behind them (294 us
-// below, 272 laid down).  849 rows, 17920 x 1536 444 -> 272 us (172 TFLOP/s), 1536 x 8960 in six shares 205 -> 128; 2,048 rows, 37888 x
+// below, 272 laid down).  A lane stores its four results at once (one by one 266 products
+// took 1.13 times as long, 2,048 rows of 8192 x 256 115 us instead of 56).  849 rows, 17920 x 1536 444 -> 272 us (172 TFLOP/s), 1536 x 8960 in six shares 205 -> 128; 2,048 rows, 37888 x
 // 3584 4,380 -> 2,620 (212); 266 products of 65 to 2,048 rows take 0.72 of the time on average, 0.97 at worst, against
 // v_mfma_f32_32x32x2_f32.
 #pragma once
@@ -26,6 +27,7 @@
 
 typedef __bf16 split_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float split_f32x4 __attribute__((ext_vector_type(4)));
+typedef float split_f32x4_at_4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float split_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 split_bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -188,13 +190,23 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_split_kernel(
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const int n = n0 + 16 * B * wn + 16 * b + 4 * (lane >> 4);
+      if (n >= N) continue;
+      split_f32x4 s = sum[a][b] * (1 / (SCALE * SCALE));
+      unsigned odd = 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        if (n + e >= N) continue;
-        const float s = sum[a][b][e] * (1 / (SCALE * SCALE));
-        if (fabsf(s) < INFINITY) y[(size_t)m * N + n + e] = s + (bias != nullptr ? bias[n + e] : 0.f);
-        else again |= 1ull << (4 * (B * a + b) + e);
+        odd |= fabsf(s[e]) < INFINITY ? 0u : 1u << e;
+        if (bias != nullptr) s[e] += bias[n + e < N ? n + e : N - 1];
       }
+      float* to = y + (size_t)m * N + n;
+      if (odd == 0 && n + 4 <= N) {
+        *(split_f32x4_at_4*)to = s;                    // (one store: rows of 64 to 256 values are bound by them)
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N && !(odd >> e & 1)) to[e] = s[e];
+      again |= (unsigned long long)(n + 4 <= N ? odd : odd & ((1u << (N - n)) - 1)) << 4 * (B * a + b);
     }
   }
   // An operand that is not finite, or 2^24 times it beyond the largest bfloat16, or a sum past 2^80: by float32 instructions and sums of

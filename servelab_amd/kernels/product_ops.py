@@ -706,7 +706,7 @@ class ProductOps:
     F32_MFMA_MIN_M = 17           # float32 products of this many rows or more run on the matrix cores
 
     def linear_f32_mfma(self, x, w, bias):
-        """Float32 product on the matrix cores, K % 16 == 0: more than 64 rows, K % 32 == 0 and 512 at least by products of
+        """Float32 product on the matrix cores, K % 16 == 0: more than 64 rows, K % 32 == 0 and 64 at least by products of
         three bfloat16 terms an operand, which together are the float (gemm_f32_split.h: closer to 64 bits than
         float32 instructions there), else by float32 instructions; float32 sums."""
         if self.act_dtype != torch.float32:

@@ -17,8 +17,8 @@ def draws(M, N, K, spread):
     return x * two(M, K), w * two(N, K)
 
 
-# a row and a column past a tile of 128, past one of 256 (the wide form where many tiles fill the CUs), the shortest rows of three terms and
-# the longest of float32 instructions, a chunk past a segment of 512, a last share of one chunk
+# a row and a column past a tile of 128, past one of 256 (the wide form where many tiles fill the CUs), the rows of one chunk that float32 instructions
+# take, rows below a segment of 512, a whole one, a chunk past a segment of 512, a last share of one chunk
 @pytest.mark.parametrize("M,N,K", [(129, 129, 32), (129, 129, 480), (129, 129, 512), (70, 257, 544), (900, 8193, 608), (1025, 8191, 1056), (128, 256, 1536)])
 @pytest.mark.parametrize("spread", [0, 12])
 def test_sums_of_terms(M, N, K, spread):
@@ -47,6 +47,17 @@ def test_sums_lie_on_neither_side(K, shares):
     # The mean over 2 M results, which share 3,072 rows: 3e-10 at whole pairs of runs (float32 instructions: 6e-10 at most).  A run of two chunks
     # more of one sign than of the other is 1.3e-9.
     assert abs(off.mean() / spread) <= 9e-10
+
+
+@pytest.mark.parametrize("K,bar", [(64, 1.35e-7), (96, 1.5e-7), (128, 1.75e-7), (480, 3.0e-7)])
+def test_short_rows(K, bar):
+    """Three terms an operand from 64 values of k on: closer than float32 instructions, which are 1.44e-7, 1.77e-7, 2.03e-7 and 3.93e-7 off here."""
+    ops = HipOps(torch.float32, DEV)
+    x, w = draws(1024, 2048, K, 0)
+    want = x.double() @ w.double().T
+    off = ops.linear_f32_mfma(x, w, None).double() - want
+    assert off.norm() / want.norm() <= bar
+    assert abs(off.mean()) <= 0.012 * off.square().mean().sqrt()              # (an odd chunk: 1 % of it)
 
 
 # sizes whose third term, second and first lie below the least bfloat16, subnormal floats, the least ones
