@@ -76,8 +76,10 @@ class AttentionOps:
         if N != (nh + 2 * nkv) * D or D % 16 or rot % 16 or not 0 <= rot <= D:
             raise KernelError("qkv_rope_store: weight rows must be (nh + 2 nkv) * D with D % 16 == 0, "
                               "the rotated width a multiple of 16")
+        if weight.shape != (N, K):
+            raise KernelError(f"weight has shape {list(weight.shape)}, x has {K} columns")
         fused = (self.act_dtype == torch.bfloat16 and self.fuse_rope and 0 < M <= self._fused_rows(K)
-                 and weight.tiled is not None and weight.shape == (N, K))
+                 and weight.tiled is not None)
         if not fused:
             plan = None if isinstance(x, ScaledRows) else self._block_plan(M, N, K, weight)
             if plan:
