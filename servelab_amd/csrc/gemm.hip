@@ -750,7 +750,7 @@ extern "C" const char* sl_gemm_skinny_shares(const float* shares_o, const float*
   SL_CHECK(M > 0 && N > 0 && K > 0 && K % 32 == 0, "gemm_skinny_shares: sizes must be positive, K in steps of 32");
   SL_CHECK(head_dim >= 32 && (head_dim & (head_dim - 1)) == 0 && K % head_dim == 0, "gemm_skinny_shares: heads of a power of two, 32 at least");
   SL_CHECK(shares >= 2 && shares <= SL_MAX_SHARES, "gemm_skinny_shares: 2 to 8 shares");
-  SL_CHECK(M <= 8 && M * K <= 16384, "gemm_skinny_shares: at most 8 rows, of 16,384 values together");
+  SL_CHECK(M <= 16 && M * K <= 16384, "gemm_skinny_shares: at most 16 rows, of 16,384 values together");
   SL_CHECK(shares_o != nullptr && shares_ml != nullptr && resid != nullptr && next_w != nullptr && out_parts != nullptr,
            "gemm_skinny_shares: a producer over shares needs them, the stream, the next gain and a parts buffer");
   SL_CHECK(((uintptr_t)shares_o % 16) == 0 && ((uintptr_t)shares_ml % 8) == 0 && ((uintptr_t)wt % 16) == 0, "gemm_skinny_shares: shares and W must be 16-byte aligned");
@@ -759,8 +759,11 @@ extern "C" const char* sl_gemm_skinny_shares(const float* shares_o, const float*
   A.F = NormFusion{nullptr, 0, 0.f, nullptr, resid, next_w, out_parts, 0, y_tiled, th, 0};
   A.S = KeyShares{shares_o, (const float2*)shares_ml, shares, __builtin_ctz(head_dim)};
   const int tiles = (N + th - 1) / th;
-  if (halves) gemm_few_kernel<false, 0, false, false, true, 1, false, 4, 16, true><<<2 * tiles, 1024, 2 * M * K, stream>>>(A);
-  else gemm_few_kernel<false, 1, false, false, true, 1, false, 4, 16, true><<<tiles, 1024, 2 * M * K, stream>>>(A);
+  auto run = [&](auto kernel, int grid) { kernel<<<grid, 1024, 2 * M * K, stream>>>(A); };
+  if (halves && M <= 8) run(gemm_few_kernel<false, 0, false, false, true, 1, false, 4, 16, true>, 2 * tiles);
+  else if (halves) run(gemm_few_kernel<true, 0, false, false, true, 1, false, 4, 16, true>, 2 * tiles);
+  else if (M <= 8) run(gemm_few_kernel<false, 1, false, false, true, 1, false, 4, 16, true>, tiles);
+  else run(gemm_few_kernel<true, 1, false, false, true, 1, false, 4, 16, true>, tiles);
   return sl_launch_status();
 }
 

@@ -36,7 +36,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
   constexpr int NT = TILES == 2 ? 2 : 1;
   static_assert(NT == 1 || WIDE, "two tiles a workgroup share their loads of nine and more rows of x");
   static_assert(!HALF || (!GATED && !ROPE), "a gate and its up, a channel and its partner lie in one tile");
-  static_assert(!SHARES || (PRODUCER && !WIDE), "shares of keys: at most 8 rows, added to the stream");
+  static_assert(!SHARES || PRODUCER, "shares of keys: added to the stream");
   static_assert(!CONSUMER || WAVES == 8, "the shares of the sums of squares are laid out for 512 threads");
   constexpr int C = HALF ? 8 : 16;                           // columns of y a workgroup owns
   constexpr int RM = WIDE ? 16 : 8;                          // rows of x
@@ -130,10 +130,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
     extern __shared__ __bf16 merged[];                       // [M][K]
     constexpr int J = SL_MAX_SHARES;
     const KeyShares& S = A.S;
-    if (p0 < p1) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) load_w(u, p0 + u < p1 ? p0 + u : p1 - 1);
-    }
+    ask_ahead<U>(p0, p1, load_w);
     for (int c = threadIdx.x; c < M * K; c += 64 * WAVES) {
       const size_t at = (size_t)(c >> S.head_bits) * S.shares;        // (rows of K values: whole heads)
       const float* o = S.o + (at << S.head_bits) + (c & ((1 << S.head_bits) - 1));
@@ -162,7 +159,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
       for (int u = 0; u < U; ++u) {
         if (p + u >= p1) break;
         if (p != p0) load_w(u, p + u);
-        b[u] = *(const bf16x8*)(merged + 2 * (p + u) * xstep + xlane);
+        load_x(u, x, p + u);
         multiply(u);
       }
     }

@@ -1,5 +1,5 @@
-// How the wavefronts of a few-rows product share the k-steps (32 values of k each) of a tile of W.  Plain arithmetic, the same on
-// the host.
+// How the wavefronts of a few-rows product share the k-steps (32 values of k each) of a tile of W, or its pairs of k-steps.  Plain
+// arithmetic, the same on the host.
 #pragma once
 
 // Wavefront `wave` of `waves` takes k-steps [first_k_step(wave), first_k_step(wave + 1)) of `steps`; with

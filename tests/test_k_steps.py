@@ -1,4 +1,5 @@
-"""Which k-steps of a weight the wavefronts of a few-rows product read (csrc/k_steps.h), on the host."""
+"""Which k-steps of a weight, or pairs of them, the wavefronts of a few-rows product read, and which they ask for ahead of attention's
+shares (csrc/k_steps.h, gemm_few.h), on the host."""
 import os
 import shutil
 import subprocess
@@ -13,7 +14,7 @@ PROGRAM = """
 #include "k_steps.h"
 int main() {
   for (int waves : {8, 16})
-    for (int steps = 1; steps <= 600; ++steps)
+    for (int steps = 0; steps <= 600; ++steps)           // (none: the pairs of a single k-step)
       for (int wave = 0; wave < waves; ++wave) {
         const int first = first_k_step(steps, wave, waves), behind = first_k_step(steps, wave + 1, waves);
         std::printf("%d %d %d %d %d", waves, steps, wave, first, behind);
@@ -36,5 +37,5 @@ def test_wavefronts_ask_for_their_own_k_steps(tmp_path):
         covered[waves, steps] = behind
         # four of its own k-steps, or none
         assert list(zip(ahead[::2], ahead[1::2])) == [(u, min(first + u, behind - 1)) for u in range(4 if first < behind else 0)]
-    assert len(covered) == 1200 and all(behind == steps for (_, steps), behind in covered.items())
+    assert len(covered) == 1202 and all(behind == steps for (_, steps), behind in covered.items())
 

@@ -4,7 +4,7 @@ import torch
 
 from emulated_ops import EmulatedOps
 from servelab_amd.kernels import HipOps
-from servelab_amd.kernels.values import AttentionShares
+from servelab_amd.kernels.values import AttentionShares, Deferred
 from test_float32_forms_gpu import emu_batch
 from test_kernels_gpu import make_attention_case
 
@@ -42,3 +42,25 @@ def test_shares_of_float32_attention(shares, D):
     want = emu.paged_attention(qkv.cpu(), nh, nkv, D, kc.cpu(), vc.cpu(), page, tables.cpu(), emu_batch(batch), D ** -0.5, None)
     # float32 scores of D products on both sides, and sums of weights that add up to one
     assert float((got.cpu() - want).abs().max()) <= 4e-6 * max(1.0, float(want.abs().max()))
+
+
+# rows of one load of x and of two, the most there are; half a tile a workgroup, a whole one, a lower one; a single k-step, an odd number of them
+@pytest.mark.parametrize("T", [1, 8, 9, 16])
+@pytest.mark.parametrize("nh,D,N", [(1, 32, 40), (5, 32, 2048), (8, 64, 300), (3, 64, 4112), (4, 128, 3600)])
+def test_the_output_projection_merges_them(T, nh, D, N):
+    ops, shares, K = HipOps(torch.bfloat16, DEV), 3, nh * D
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    o = torch.randn(T, nh, shares, D, generator=g, device=DEV)
+    ml = torch.rand(T, nh, shares, 2, generator=g, device=DEV) * 3 + 0.5
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    gain, stream = torch.ones(N, device=DEV), torch.randn(T, N, generator=g, device=DEV)
+    for weight in (ops.prepare_weight(w), ops.prepare_weight(w, residual_delta=True, _th=10)):
+        resid = stream.clone()
+        rows = ops.add_rmsnorm(resid, Deferred(AttentionShares(o, ml), weight, None), gain, 1e-6, fuse=True)
+        x = ops.combine_shares(AttentionShares(o, ml)).double()
+        # the merged rows are bfloat16 in both, rounded alike but for sums in another order: at most one of 2^-8 of a value
+        size = x.abs() @ w.double().abs().T
+        assert ((resid.double() - stream.double() - x @ w.double().T).abs() <= 2.0 ** -8 * size + 1e-6).all()
+        assert float((resid.double() - stream.double() - x @ w.double().T).norm() / (x @ w.double().T).norm()) <= 2.0 ** -10
+        assert torch.allclose(rows.parts.sum(0)[:T], (resid.double() ** 2).sum(1).float(), rtol=1e-5) and not rows.parts[:, T:].any()
+        assert torch.equal(rows.plain_x(), resid.bfloat16())
