@@ -98,9 +98,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
       }
     }
   }
-  f32x4 acc[NT], odd = {0.f, 0.f, 0.f, 0.f};
+  // Running sums: a producer's, whose results are added to the float stream, of every other pair of k-steps apart, so that they are as
+  // short as with the sixteen wavefronts it had (error of a delta of 2048 x 11008 at 8 / 16 rows 1.30e-7 / 1.66e-7; one sum 1.58e-7 / 2.24e-7).
+  constexpr int SUMS = PRODUCER && !SHARES && !(HALF && WIDE) ? 2 : 1;
+  f32x4 acc[SUMS][NT], odd[SUMS];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < SUMS; ++s) {
+    odd[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   bf16x8 a[NT][LW * U], b[LX * U];
   auto load_w = [&](int u, int p) {
 #pragma unroll
@@ -117,8 +124,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
   auto multiply = [&](int u) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][LW * u], b[LX * u], acc[t], 0, 0, 0);
-      f32x4& other = WIDE && !HALF ? acc[t] : odd;           // (whole tiles of 16 rows of x: all of one accumulator is valid)
+      f32x4& even = acc[u % SUMS][t];
+      even = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][LW * u], b[LX * u], even, 0, 0, 0);
+      f32x4& other = WIDE && !HALF ? even : odd[u % SUMS];   // (whole tiles of 16 rows of x: all of one accumulator is valid)
       if (WIDE || !HALF) other = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][LW * u + LW - 1], b[LX * u + LX - 1], other, 0, 0, 0);
     }
   };
@@ -191,20 +199,25 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
     }
     if (WIDE || hi == 0) bx = *(const bf16x8*)(x + 2 * KP * xstep + xlane);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[t], bx, acc[t], 0, 0, 0);
+    for (int t = 0; t < NT; ++t) acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[t], bx, acc[0][t], 0, 0, 0);
+  }
+  if constexpr (SUMS == 2) {
+    odd[0] += odd[1];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[0][t] += acc[1][t];
   }
   // Element r of lane (column of x, quarter of the tile's rows) is a sum of row 4 (quarter) + r of the tile.
   constexpr int QS = WIDE ? 16 : 8;                          // places a quarter takes in LDS: valid columns only
-  if (HALF && WIDE) red[0][wave][lane] = gq < 2 ? acc[0] : odd;      // rows 0..7 of the even k-steps' sums, rows 8..15 of the odd ones'
+  if (HALF && WIDE) red[0][wave][lane] = gq < 2 ? acc[0][0] : odd[0];      // rows 0..7 of the even k-steps' sums, rows 8..15 of the odd ones'
   else if (HALF) {
-    if ((gq >> 1) == hi) red[0][wave][gq * 8 + (i & 7)] = acc[0];
+    if ((gq >> 1) == hi) red[0][wave][gq * 8 + (i & 7)] = acc[0][0];
   } else if (WIDE) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) red[t][wave][lane] = acc[t];
+    for (int t = 0; t < NT; ++t) red[t][wave][lane] = acc[0][t];
   } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) acc[0][r] += __shfl(odd[r], lane + 8, 64);
-    if (hi == 0) red[0][wave][gq * 8 + i] = acc[0];
+    for (int r = 0; r < 4; ++r) acc[0][0][r] += __shfl(odd[0][r], lane + 8, 64);
+    if (hi == 0) red[0][wave][gq * 8 + i] = acc[0][0];
   }
   if (CONSUMER) {                                            // this wavefront's share of the sums of squares, by row
     float sacc = 0.f;
@@ -220,8 +233,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      s += red[t][w][(n / 4) * QS + m][n % 4];
-      if (HALF) s += red[t][w][(2 + n / 4) * QS + m][n % 4];
+      const float even = red[t][w][(n / 4) * QS + m][n % 4];
+      s += HALF ? even + red[t][w][(2 + n / 4) * QS + m][n % 4] : even;
     }
     return s;
   };
