@@ -889,10 +889,11 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(
   const size_t base = ((size_t)r * nh + h) * nsplit;
   const float* po = part_o + base * D;
   // A lane takes channels lane, lane + 64, ...; the partial outputs of BATCH shares are asked for
-  // together, all channels of a lane at once, the first of them with the maxima, the next before the last are added up (a batch
-  // is a trip to memory: with eight shares a batch
+  // together, all channels of a lane at once (a batch is a trip to memory: with eight shares a batch
   // and the channels one after the other, 64 shares took 2 us longer than 32; with the last shares
-  // below a whole batch one by one, 21 took 3 us longer than 16 or 24).  Added in the order of the
+  // below a whole batch one by one, 21 took 3 us longer than 16 or 24).  A batch of four, which is all
+  // there is then, goes with the maxima; sixteen behind the weights (with them 16 rows of 32 heads of 256 in 256 shares took 12.1 us
+  // instead of 10.5, one row of 28 heads of 128 in 16 shares 2.81 instead of 2.65).  Added in the order of the
   // shares, whatever the batches.  (Past the last channel that one again, never stored.)
   constexpr int DI = (D + 63) / 64;
   float v[BATCH][DI];
@@ -904,23 +905,23 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(
       for (int di = 0; di < DI; ++di) v[u][di] = row[64 * di + 64 <= D ? lane + 64 * di : min(lane + 64 * di, D - 1)];
     }
   };
-  float m[COMBINE_PER_LANE], l[COMBINE_PER_LANE];
+  constexpr bool AT_ONCE = BATCH <= 4;
+  float m[COMBINE_PER_LANE], l[COMBINE_PER_LANE], top = -INFINITY;
 #pragma unroll
   for (int i = 0; i < COMBINE_PER_LANE; ++i) {
+    const int j = lane + 64 * i;
     m[i] = -INFINITY;
     l[i] = 0.f;
-    if (64 * i < nsplit) {                              // (the same for all lanes)
-      const size_t at = (base + min(lane + 64 * i, nsplit - 1)) * 2;
+    if (AT_ONCE ? i == 0 : j < nsplit) {                // (at once: no branch in front of the outputs; past the last share that one again)
+      const size_t at = (base + (AT_ONCE ? min(j, nsplit - 1) : j)) * 2;
       m[i] = part_ml[at];
       l[i] = part_ml[at + 1];
     }
-  }
-  ask(0);
-  __builtin_amdgcn_sched_barrier(0);
-  float top = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < COMBINE_PER_LANE; ++i) {
-    if (lane + 64 * i >= nsplit) m[i] = -INFINITY, l[i] = 0.f;
+    if (AT_ONCE && i == 0) {
+      ask(0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (j >= nsplit) m[i] = -INFINITY, l[i] = 0.f;
+    }
     top = fmaxf(top, m[i]);
   }
   const float mx = wave_max(top);
@@ -938,19 +939,14 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(
 #pragma unroll
   for (int di = 0; di < DI; ++di) acc[di] = 0.f;
   for (int j = 0; j < nsplit; j += BATCH) {
-    float now[BATCH][DI];
-#pragma unroll
-    for (int u = 0; u < BATCH; ++u)
-#pragma unroll
-      for (int di = 0; di < DI; ++di) now[u][di] = v[u][di];
-    if (j + BATCH < nsplit) ask(j + BATCH);
+    if (!AT_ONCE) ask(j);
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
       // (no branch here: under one the compiler may move each load down to its use; beyond the last share the
       // weight is 0 and the value that of the last share)
       const float w = j + u < nsplit ? ws[j + u] : 0.f;
 #pragma unroll
-      for (int di = 0; di < DI; ++di) acc[di] += SKIP && w == 0.f ? 0.f : w * now[u][di];
+      for (int di = 0; di < DI; ++di) acc[di] += SKIP && w == 0.f ? 0.f : w * v[u][di];
     }
   }
 #pragma unroll
