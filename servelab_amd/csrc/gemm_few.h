@@ -10,7 +10,8 @@
 //     valid in columns 0..7 of one accumulator, the odd ones' in columns 8..15 of another.
 //   * Half a tile: a load of W is 8 rows at two k-steps, whole cache lines of 128 bytes out of the same layout; up to 8 rows of x
 //     one instruction then multiplies both k-steps (two quadrants of its result are valid).
-//   * Two tiles share every load of x: with 9 to 16 rows those loads are up to half of what a CU pulls.
+//   * Two tiles share every load of x: with 9 to 16 rows those loads are up to half of what a CU pulls.  Their consumers are held to 80
+//     registers, three workgroups a CU: with 82 and two, the 560 of 17920 x 896 took 11.4 us at 16 rows, now 9.8.
 //   * All loads of U pairs of k-steps are asked for before the first product, held there by a scheduling barrier.  Without it the
 //     compiler moves the loads of x down to their products, and a wavefront makes a trip to memory for each of them.
 // Measured in chains of a graph, W cold (us; before: loads left to the compiler, whole tiles; in brackets a plain read of W):
@@ -31,7 +32,7 @@ struct FewRows {
 };
 
 template <bool WIDE, int TILES, bool GATED, bool CONSUMER, bool PRODUCER, int PARTS, bool ROPE, int U, int WAVES = 8, bool SHARES = false>
-__global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
+__global__ __launch_bounds__(64 * WAVES, TILES == 2 && CONSUMER && !ROPE && PARTS == 8 ? 6 : 1) void gemm_few_kernel(const FewRows A) {
   constexpr bool HALF = TILES == 0;
   constexpr int NT = TILES == 2 ? 2 : 1;
   static_assert(NT == 1 || WIDE, "two tiles a workgroup share their loads of nine and more rows of x");
@@ -311,7 +312,10 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_few_kernel(const FewRows A) {
   }
 }
 
-// TILES: 0 half a tile a workgroup, 1, 2.
+// TILES: 0 half a tile a workgroup, 1, 2.  U: pairs of k-steps asked for together.  One tile and 9 to 16 rows: four, and three where there are
+// more than two tiles a CU, so that no more than 80 registers (of consumers of up to 4,096 values and of plain rows) leave room for three
+// workgroups, all tiles at once: 12288 x 1024 7.6 to 9.5 us with four, 6.6 to 7.9 with three, 9728 x 896 6.8 to 8.0 and 5.7 to 6.8; 2048 x 2048, whose
+// wavefronts have four pairs, 5.2 and 5.5.
 template <bool WIDE, int TILES, int U>
 static void launch_few_rows(const FewRows& A, bool gated, bool rope, hipStream_t stream) {
   const bool consumer = A.F.in_parts != nullptr, producer = A.F.resid != nullptr, few = A.F.in_nparts <= 32 * 8;
@@ -329,7 +333,9 @@ static void launch_few_rows(const FewRows& A, bool gated, bool rope, hipStream_t
     if (consumer) return SL_FEW(false, true, false, 16, false);
     if (gated) return SL_FEW(true, false, false, 1, false);
   }
-  if (producer) SL_FEW(false, false, true, 1, false);
-  else SL_FEW(false, false, false, 1, false);
+  if constexpr (U % 2 == 0) {                                // (a producer's two running sums: of pairs in turn)
+    if (producer) return SL_FEW(false, false, true, 1, false);
+  }
+  SL_FEW(false, false, false, 1, false);
 #undef SL_FEW
 }
