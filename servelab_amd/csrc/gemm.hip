@@ -138,6 +138,7 @@ template <int NC>
 static const char* rows_split(const act_t* x, const act_t* w, const float* bias, void* y, int M, int N, int K, hipStream_t stream) {
   const int grid = (N + NC - 1) / NC;
   if (M == 1) gemm_rows_split_kernel<1, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
+  else if (M > 2) gemm_rows_split_kernel<4, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
   else gemm_rows_split_kernel<2, NC><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K);
   return sl_launch_status();
 }
@@ -221,7 +222,10 @@ extern "C" const char* sl_gemm_rows(const void* x, const void* w, const float* b
   const act_t* ww = (const act_t*)w;
 #if defined(SL_F32)
   // Three rows and more go through the matrix units, sixteen at a time (gemm_f32_few.h; two rows there are no faster than here: 17920 x 1536
-  // 20.1 us for 19.4, 1536 x 8960 13.4 for 13.0).
+  // 20.1 us for 19.4, 1536 x 8960 13.4 for 13.0).  Not up to four long rows of more columns than go round the CUs once in fours and fewer than three
+  // quarters of twice that: at 3 / 4 rows 1200 x 16384 26.7 / 27.8 us there, 22.9 / 24.7 here, 1536 x 8960 17.4 / 18.7 and 16.3 / 17.9, 1536 x 6144
+  // 13.1 / 13.8 and 13.0 / 14.0; 2048 x 5632 12.1 / 12.6 and 13.7 / 15.8.
+  if (M > 2 && M <= 4 && N > 1024 && N <= 1536 && K >= 6144) return rows_split<2>(xx, ww, bias, y, M, N, K, stream);
   for (int m0 = 0; M > 2 && m0 < M; m0 += 16) {
     const int rows = min(16, M - m0);
     float* to = (float*)y + (size_t)m0 * N;

@@ -97,9 +97,11 @@ __global__ __launch_bounds__(KW == 8 ? 512 : 256) void gemm_f32_few_kernel(
   }
 }
 
-// Which of them, measured for 16 matrices of 896 to 151,936 rows and rows of 64 to 18,944 values: of few columns a wavefront takes four or
+// Which of them, measured for 37 matrices of 64 to 151,936 rows and rows of 64 to 18,944 values: of few columns a wavefront takes four or
 // eight, so that every CU has some; of long rows eight wavefronts share K, and of more than 2,048 such columns each takes sixteen (3584 x 18944 at 3 / 16 rows
-// in eight 57 / 111 us, in sixteen 50 / 84; up to eight rows of 2560 x 3072 and 4096 x 4096 sixteen lose up to 7 %); of many columns 8 or 16 read a load of x, and of very many two
+// in eight 57 / 111 us, in sixteen 50 / 84; up to eight rows of 2560 x 3072 and 4096 x 4096 sixteen lose up to 7 %), of up to 1,024 four (1024 x 4096 at 3 / 8
+// rows in eight 8.2 / 10.9, in four 6.4 / 8.5); up to four rows of up to 768 columns, from 512 values on, eight wavefronts as well (128 x 896 3.7 -> 3.3, 128 x 2560 4.8 ->
+// 4.7); of many columns 8 or 16 read a load of x, and of very many two
 // wavefronts share K (151936 x 896 at three rows 104 us for 91, 17920 x 1536 21 for 22).
 template <int MB>
 static void gemm_f32_few(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, hipStream_t stream) {
@@ -108,9 +110,10 @@ static void gemm_f32_few(const float* x, const float* w, const float* bias, floa
       <<<(unsigned)((N + 4 * C * (KW == 2 ? 2 : 1) - 1) / (4 * C * (KW == 2 ? 2 : 1))), KW == 8 ? 512 : 256, 0, stream>>>(x, w, bias, y, M, N, K)
   const bool few = N <= 4096, lengthy = K >= 3072;
   if constexpr (MB <= 2) {
-    if (few && lengthy && N < 1024) SL_FEW(1, 8, 2, 4);
+    if (few && lengthy && N <= 1024) SL_FEW(1, 8, 2, 4);
     else if (few && lengthy && (N <= 2048 || K < 8192)) SL_FEW(2, 8, 2, 4);
     else if (few && lengthy) SL_FEW(4, 8, 2, 4);
+    else if (MB == 1 && N <= 768 && K >= 512) SL_FEW(1, 8, 4, 4);
     else if (few) SL_FEW(1, 4, 4, 4);
     else if (N <= 32768) SL_FEW(2, 4, 4, (MB == 1 ? 4 : 2));
     else if constexpr (MB == 1) {
@@ -118,7 +121,7 @@ static void gemm_f32_few(const float* x, const float* w, const float* bias, floa
       else SL_FEW(2, 4, 4, 4);
     } else SL_FEW(4, 2, 2, 2);
   } else {
-    if (few && lengthy && N < 1024) SL_FEW(1, 8, 2, 2);
+    if (few && lengthy && N <= 1024) SL_FEW(1, 8, 2, 2);
     else if (few && lengthy && N <= 2048) SL_FEW(2, 8, 2, 2);
     else if (few && lengthy) SL_FEW(4, 8, 2, 2);
     else if (N <= 16384) SL_FEW(2, 4, 2, 1);

@@ -23,6 +23,13 @@ def test_sums(M, N, K):
     assert ((got - want - b.double()).abs() <= bar + 2.0 ** -24 * got.abs()).all()
 
 
+# the last columns in fours and the first beyond; few columns of short rows; up to four long rows as FMAs, and what lies around them
+@pytest.mark.parametrize("M", [3, 4, 5])
+@pytest.mark.parametrize("N,K", [(1024, 3076), (1025, 3076), (768, 68), (769, 1028), (768, 512), (768, 508), (1025, 6144), (1536, 6148), (1537, 6148), (1536, 6140)])
+def test_sums_at_the_lines_of_few_columns(M, N, K):
+    test_sums(M, N, K)
+
+
 @pytest.mark.parametrize("M", [3, 7, 12])
 def test_what_a_value_reaches(M):
     """NaN and infinities of a row of x or of W stay in that row and that column, also where a step passes the end of K."""
