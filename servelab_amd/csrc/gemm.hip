@@ -529,7 +529,23 @@ extern "C" float sl_gemm_f32_split_us(int M, int N, int terms, int nsplit, int c
 }
 
 constexpr int SPLIT_MIN_K = 64;
-extern "C" int sl_gemm_f32_split_min_k() { return SPLIT_MIN_K; }
+// Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated time, which is the tiles' rounds over
+// the CUs (0.067 us a term of a tile of 128 x 128 results by float32 instructions) plus, for several shares, the traffic of the partial sums and their
+// addition.  (Chosen here and not share by share from Python, which took the host up to 5.6 us a product; 0.3 here.)
+extern "C" int sl_gemm_f32_shares(int M, int N, int K, int cus) {
+  const bool split = M > 64 && K % 32 == 0 && K >= SPLIT_MIN_K;
+  const int rows = M <= 64 ? 32 : 128, segments = (K + SEGMENT_K - 1) / SEGMENT_K;
+  const long long tiles = (long long)((M + rows - 1) / rows) * ((N + 127) / 128);
+  int best = 1;
+  double least = INFINITY;
+  for (int s = 1; s <= min(16, segments); ++s) {
+    const int terms = min(K, (segments + s - 1) / s * SEGMENT_K);      // of the longest share
+    double us = split ? sl_gemm_f32_split_us(M, N, terms, s, cus) : (double)((tiles * s + cus - 1) / max(1, cus)) * terms * 0.067 * (rows / 128.);
+    if (s > 1) us += 5. + (s + 1.) * M * N * 4 / 3e6;
+    if (us < 0.97 * least) best = s, least = us;
+  }
+  return best;
+}
 
 // nsplit > 1: K is cut into that many shares of whole segments, whose sums wait in `part`, [nsplit, M, N].  A product of
 // few tiles (the output projection and the down projection of a short prompt) leaves most CUs idle otherwise: 849 rows

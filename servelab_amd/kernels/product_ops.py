@@ -719,31 +719,9 @@ class ProductOps:
         self._call("gemm", "sl_gemm_f32_mfma", _p(x), _p(w), _p(bias), _p(y), M, N, K, shares, _p(part))
         return y
 
-    F32_SEGMENT = 512             # terms of a running sum of the float32 products: a share of K holds whole ones
-    F32_TILE_US_PER_TERM = 0.067  # a tile of 128 x 128 results takes this long per term of K with a CU to itself (float32 instructions)
-
     def _f32_shares(self, M, N, K):
-        """Into how many shares of K a float32 product on the matrix cores is cut: the number with the least estimated
-        time, which is the tiles' rounds over the CUs plus, for several shares, the traffic of the partial sums and
-        their addition."""
-        rows = 32 if M <= 64 else 128
-        split = M > 64 and K % 32 == 0 and K >= self._lib["gemm"].sl_gemm_f32_split_min_k()
-        tiles = -(-M // rows) * -(-N // 128)
-        best, least, segments = 1, float("inf"), -(-K // self.F32_SEGMENT)
-        if split:
-            estimate = self._lib["gemm"].sl_gemm_f32_split_us
-            estimate.restype = ctypes.c_float
-        for s in range(1, min(16, segments) + 1):
-            terms = min(K, -(-segments // s) * self.F32_SEGMENT)          # of the longest share
-            if split:
-                us = estimate(M, N, terms, s, self._num_cus)
-            else:
-                us = -(-tiles * s // self._num_cus) * terms * self.F32_TILE_US_PER_TERM * (rows / 128)
-            if s > 1:
-                us += 5.0 + (s + 1) * M * N * 4 / 3e6
-            if us < 0.97 * least:
-                best, least = s, us
-        return best
+        """Into how many shares of K a float32 product on the matrix cores is cut (``sl_gemm_f32_shares``)."""
+        return int(self._lib["gemm"].sl_gemm_f32_shares(M, N, K, self._num_cus))
 
     def library_sums(self, x, w, out_dtype=None):
         """x w^T by the library, in bfloat16 or (``out_dtype`` float32) with the
