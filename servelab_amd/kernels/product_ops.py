@@ -258,9 +258,14 @@ class ProductOps:
     def _even_columns(self, M, N, K):
         """Columns of y a workgroup takes in the product of tiles that go round the CUs once (``sl_gemm_even``, 128 rows of x), the
         fewest that do, or 0 where the product is not its own: matrices of 512 rows and more with rows of up to EVEN_MAX_K values,
-        tiles of up to 192 columns, or 224 on nine tenths of the CUs, and with rows of more than EVEN_SHORT_K values seven
-        tenths of the CUs busy.  Of 162 such products (896 to 7,168 rows, 513 to 2,048 rows of x) the library's default pick takes
-        1.32 times as long on average, 0.93 at worst (700 x 4096 x 4096); the shortest wait for the host there, 20 us a call.
+        tiles of up to 192 columns, or 224 on nine tenths of the CUs; with rows of more than EVEN_SHORT_K values seven tenths of the
+        CUs busy, in tiles of 128 columns and more 0.76 of them (GPU time, library / here: three quarters, 700 x 4096 x 4096 31.5 / 34.6,
+        1,536 x 2048 x 3072 in 1.15 of it; at 0.76 to 0.8 in 0.92).  The call is worth having beyond its GPU time, of which 1,966 such
+        products (512 to 6,144 rows, 65 to 8,192 rows of x) take 0.99 of the library's on average: the library's takes the host 20 us,
+        and prompts of up to some 450 tokens wait for the host.  Those take tiles also where few CUs have one (256 x 2048 x 2048 11.9 / 18.5;
+        whole prompts, library / here: twelve layers of the 1.5B shape, 200 / 400 tokens 2,213 / 1,313 and 2,328 / 1,785, of the 3B shape 256 / 400
+        1,674 / 1,670 and 2,044 / 1,999); longer ones with rows of more than EVEN_HOST_K values only on 0.425 of the CUs (the 3B shape at 512
+        tokens, o on 0.34 and q/k/v on 0.42: 2,104 / 2,191; 24 layers of the 0.5B shape, rows of 896, at 512 / 1,000 3,582 / 2,819 and 3,505 / 2,805).
         us, library / here: 2,048 rows of x, 3584 x 3584 52 / 48, 2560 x 2048 26 / 24; 527 rows 4608 x 3584 29 / 26.
         Longer rows and idle CUs: 527 rows, 2048 x 8192 43 / 46, 1536 x 8960 37 / 48; 1,500 rows, 4096 x 4096 49 / 54 in 224
         columns on 0.89 of the CUs; two rounds: 2,048 rows, 4608 x 3584 60 / 76."""
@@ -271,7 +276,12 @@ class ProductOps:
         for columns in range(96, 225, 32):
             fill = rows * -(-N // columns) / self._num_cus
             if fill <= 1:
-                return columns if (columns < 224 or fill >= 0.9) and (K <= self.EVEN_SHORT_K or fill >= 0.7) else 0
+                least = 0.9 if columns == 224 else 0
+                if K > self.EVEN_SHORT_K:
+                    least = max(least, 0.7 if columns == 96 else 0.76)
+                elif K > self.EVEN_HOST_K and M > self.EVEN_HOST_ROWS:
+                    least = max(least, 0.425)
+                return columns if fill >= least else 0
         return 0
 
     def linear_even(self, x, weight, bias, columns, out_f32=False):

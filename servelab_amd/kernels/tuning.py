@@ -96,6 +96,9 @@ class Tuning:
     even_min_n: int = 512
     even_max_k: int = 4096
     even_short_k: int = 2048
+    # ... whatever share of the CUs they fill up to this many rows of x, and beyond with rows of up to so many values
+    even_host_rows: int = 448
+    even_host_k: int = 1024
     # what a million float32 sums of a share cost that are written and read again by the norm (us)
     share_us: float = 0.9
     # gated and activated products of a prompt in the tiles of gemm_rounds.h (measured sides: HipOps._gated_rows): the fewest rows

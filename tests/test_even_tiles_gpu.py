@@ -46,3 +46,15 @@ def test_which_products_take_them():
     want = x.double() @ w.double().T
     for got in (ops.linear(odd, weight, None), ops.linear(x, w, None)):
         assert calls == [] and (got.double() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+def test_idle_cus():
+    ops = HipOps(torch.bfloat16, DEV)
+    ops._num_cus = 256
+    c = ops._even_columns
+    # few CUs: prompts that wait for the host, or short rows; longer ones from 0.425 of them on
+    assert c(448, 2048, 2048) == 96 and c(449, 2048, 2048) == 0 and c(512, 2048, 1024) == 96 and c(512, 2048, 1088) == 0
+    assert c(640, 2048, 1536) == 96 and c(640, 1536, 1536) == 0 and c(2048, 512, 2048) == 0 and c(512, 2560, 2048) == 0
+    # three quarters of them with rows of more than 2,048 values: in tiles of 96 columns, not of 128
+    assert c(512, 4608, 3584) == 96 and c(700, 4096, 4096) == 0 and c(1536, 2048, 2112) == 0 and c(1536, 2048, 2048) == 128
+    assert c(1537, 2048, 4096) == 128
