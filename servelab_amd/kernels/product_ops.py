@@ -374,10 +374,8 @@ class ProductOps:
     def _shares_plan(self, M, N, K, weight):
         """Like ``_block_plan`` for a product of more rows that the norm adds to the stream: two or
         three shares of K in square tiles where they fill the CUs well, two to seven eighths, three to four fifths (GPU
-        time with the norm, library's product / shares: 3584 x 18944, 1,800 / 2,048 rows 351 / 246 and 376 / 272 us in two;
-        2560 x 9728, 2,048 rows 116 / 111 in three, 2560 x 13824 160 / 146; 4096 x 14336, 1,600 / 1,984 rows 343 / 195 and
-        211 / 219).  Less well filled two shares lose: 3584 x 18944, 1,664 rows (0.77) 238 / 253, 3328 x 8192, 2,048 rows (0.81)
-        112 / 129, 3072 x 8192, 2,048 rows (0.75) 107 / 127.  Four shares gain nothing: the norm reads them all."""
+        time with the norm, library's product / shares: 3584 x 18944, 2,048 rows 387 / 236 us in two; 2560 x 9728, 2,048 rows 121 / 107
+        in three, 2560 x 13824 163 / 136; 4096 x 14336, 1,600 / 2,048 rows 344 / 185 and 231 / 212; 4096 x 8192 loses 2 to 5 % but at 1,792)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or weight.w is None
                 or K % 64 or N % 4 or N > self.BLOCK_MAX_N or K < self.BLOCK_SQUARE_MIN_K
                 or not self.BLOCK_SQUARE_MAX_M < M <= self.SHARES_MAX_M):
@@ -390,9 +388,12 @@ class ProductOps:
     def _shares_by_estimate(self, M, N, K, weight):
         """The sizes that ``_shares_plan`` leaves: two to eight shares in wide tiles, as many as take the least time by estimate
         (the product's, ``_tiles_us``, and SHARE_US for every million sums written and read again).  us with the norm that adds
-        them, the library's product / the shares: 2048 x 11008 at 1,792 / 1,930 / 2,048 rows 109 / 82, 105 / 88 and 110 / 92 in
-        four, 2048 x 8192 at 2,048 81 / 76, 1536 x 8960 78 / 67 in five, 3584 x 18944 at 1,792 320 / 216 in two; 3072 x 8192
-        at 1,930 106 / 107.  Rows of 5,632 values and less gain nothing (2048 x 5632 at 2,048 64 / 62, 896 x 4864 34 / 33)."""
+        them, the library's product / the shares: 2048 x 11008 at 1,792 / 1,930 / 2,048 rows 111 / 87, 109 / 92 and 115 / 96 in
+        four, 2048 x 8192 at 2,048 83 / 79, 1536 x 8960 83 / 71 in five, 3584 x 18944 at 1,664 / 1,792 244 / 203 and 321 / 221 in two,
+        64 x 8192 31 / 20 in eight; of 142 sizes from 64 columns on 0.85 of the time on average, 1.05 at worst (one of ``_shares_plan``).  Two shares on
+        three quarters of the CUs or fewer lose and are left to the library (3072 x 8192 at 1,930 / 2,048 109 / 115 and 110 / 115, 3328 x 8192 at 1,792
+        111 / 115, 2880 x 11520 at 1,930 141 / 149); at 0.77 they do not (3584 x 8192 at 1,792 120 / 117).
+        Rows of 5,632 values and less gain nothing (2048 x 5632 at 2,048 64 / 62, 896 x 4864 34 / 33)."""
         if (self.act_dtype != torch.bfloat16 or not self.use_block_products or weight.w is None
                 or K % 64 or N % 4 or N > self.BLOCK_MAX_N or K < self.BLOCK_SQUARE_MIN_K
                 or not self.BLOCK_SQUARE_MAX_M < M <= self.SHARES_MAX_M):
@@ -401,7 +402,10 @@ class ProductOps:
         plans = [ks for ks in range(2, 9) if tiles * ks <= self._num_cus]
         if not plans:
             return None
-        return min(plans, key=lambda ks: self._tiles_us(self._tile_rows(M, N, K, ks), M, N, K, ks) + self.SHARE_US * 1e-6 * ks * M * N), True
+        ks = min(plans, key=lambda ks: self._tiles_us(self._tile_rows(M, N, K, ks), M, N, K, ks) + self.SHARE_US * 1e-6 * ks * M * N)
+        if ks == 2 and 4 * 2 * -(-N // 256) * -(-M // self._tile_rows(M, N, K, 2)) <= 3 * self._num_cus:
+            return None
+        return ks, True
 
     def _gated_rows(self, M, N, K):
         """Rows of x a workgroup takes (192 or 256) for the gated product of a prompt at sizes that take the tiles whatever their

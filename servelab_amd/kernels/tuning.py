@@ -90,7 +90,7 @@ class Tuning:
     # 257 rows of x up to this many (7B shape, down at 768 / 1,024 / 1,536 rows: 83 / 111 / 168 us)
     block_square_min_k: int = 8192
     block_square_max_m: int = 1536
-    # up to how many rows a residual delta of long rows takes two or three shares of K in those tiles
+    # up to how many rows a residual delta of long rows takes two to eight shares of K in those tiles
     shares_max_m: int = 2048
     # products of more rows than the kernels above take in tiles that go round the CUs once (HipOps._even_columns)
     even_min_n: int = 512

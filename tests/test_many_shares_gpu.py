@@ -23,6 +23,15 @@ def test_which_sizes_take_how_many():
     assert plan(2048, 4352, 8192) is None                                                       # 136 tiles: no second share
 
 
+def test_two_shares_on_few_cus_stay_with_the_library():
+    ops = HipOps(torch.bfloat16, DEV)
+    ops._num_cus = 256
+    plan = lambda M, N, K: ops._shares_by_estimate(M, N, K, Rows)
+    # 192 tiles of 256 rows, 182, 196; 234 of 192 rows
+    assert plan(1930, 3072, 8192) is None and plan(1792, 3328, 8192) is None and plan(1792, 3584, 8192) == (2, True)
+    assert plan(1537, 3328, 8192) == (2, True)
+
+
 @pytest.mark.parametrize("M,N,K", [(1537, 260, 8192), (2048, 1024, 8256)])       # part-filled tiles; chunks that do not divide by the shares
 def test_the_sums_of_the_shares(M, N, K):
     ops = HipOps(torch.bfloat16, DEV)
