@@ -919,7 +919,8 @@ static int resident_workgroups(Kernel kernel) {
 // flight), each with the number of k-steps R a wavefront asks for at once.  They are the
 // widths whose consumers have many tiles per CU among the models this was measured on
 // (1536, 2048, 3584, 4096, 5120); every other K, and K = 8192, where this form measured
-// slower, takes sl_gemm_skinny, which gives the same result bit for bit.
+// slower, takes sl_gemm_skinny: the same result with 9 to 16 rows, and up to the order of
+// the float sums with 8 and fewer (there odd k-steps are summed apart).
 #define SL_RESIDENT_WIDTHS(X) X(6, 6) X(8, 8) X(14, 14) X(16, 16) X(20, 10)
 constexpr int resident_parts_per_thread(int NS) { return NS <= 16 ? 8 : 16; }
 
@@ -935,7 +936,7 @@ extern "C" int sl_gemm_resident_parts(int K) {
 }
 
 // The consumer forms of sl_gemm_skinny (x: un-normalised rows) for matrices of
-// many tiles; same arguments, same result.
+// many tiles; same arguments, same products (sums of 8 rows and fewer in another order).
 extern "C" const char* sl_gemm_resident(const void* x, const void* wt, const float* bias, void* y,
                                         int M, int N, int K, int out_f32, int gated,
                                         const float* in_parts, int in_nparts, float eps,

@@ -177,9 +177,11 @@ class ProductOps:
 
         bfloat16, by rows of x: 1..16 the few-rows kernel over the tiled weight,
         17..64 the wide or the LDS-staged kernel (by the size of W; the latter
-        up to 128 rows), more the library, or that many rows at a time through
-        those kernels when the result is wanted in float32.  float32: the wavefront-per-column kernel up to 16 rows, the
-        tiled FMA kernel above; never a library product."""
+        up to 128 rows), more the kernels in tiles, some of them in shares of K (``_block_plan``, ``_shares_plan``,
+        ``_shares_by_estimate``), over the tiled copy where such tiles go round the CUs once (``_even_columns``),
+        or the library, or as many rows as the first ones take at a time when the result is wanted in float32.
+        float32: ``linear_rows`` up to 16 rows (FMAs, from three on the matrix units), ``linear_f32_mfma`` above where
+        K % 16 == 0, else the tiled FMA kernel; never a library product."""
         if not isinstance(weight, LinearWeight):
             weight = LinearWeight(weight)
         if isinstance(x, ScaledRows):
@@ -585,7 +587,8 @@ class ProductOps:
         (x in registers, row scales computed once): matrices with several tiles per CU whose
         row length the kernel is built for (the library says which: ``sl_gemm_resident_parts``,
         the most sums of squares a row its kernel for K adds up, 0 for no kernel).  Every other
-        width takes the workgroup-per-tile kernel, which gives the same result bit for bit."""
+        width takes the workgroup-per-tile kernel: the same result with 9 to 16 rows, and up to the order of the float
+        sums with 8 and fewer."""
         if -(-N // 16) < self.RESIDENT_MIN_ROUNDS * self._num_cus:
             return False
         most = self._resident_k.get(K)

@@ -70,8 +70,8 @@ class Tuning:
     # matrices of fewer elements than this stay off the block kernel (tiles of 256 rows of x) at 129 rows and more
     block_min_elements: int = 8 << 20
 
-    # ---- the wavefront-per-column products (float32 table, bfloat16 fallbacks)
-    # up to 16 rows of x go through LDS once per 32 columns of W instead of through L1 once per 4
+    # ---- the wavefront-per-column products of bfloat16 (matrices without a tiled copy)
+    # 4 to 8 rows of x go through LDS once per 32 columns of W instead of through L1 once per 4
     rows_through_lds: bool = True
 
     # ---- products over the row-major copy in tiles of 256 rows of x by 128 rows of W (gemm_block)

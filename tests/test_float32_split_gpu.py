@@ -1,5 +1,5 @@
 """Float32 products of three bfloat16 terms an operand: both widths of a workgroup at the edges of tiles, chunks and shares, values of
-every size, and operands that are not finite."""
+sizes from the least on, and operands that are not finite."""
 import pytest
 import torch
 

@@ -316,7 +316,7 @@ def test_fused_add_norm_around_few_rows_products(M, H, N2, pairs, th):
     ops, emu = HipOps(torch.bfloat16, "cuda:0", tuning=Tuning(fused_rows_by_width=((1 << 30, 16),))), EmulatedOps(torch.bfloat16)
     if pairs:
         ops._pair_tiles = lambda M, N, K, th=16: True
-    K1 = 128 if H != 3584 else 4160       # (the long one: 224 tiles, sixteen wavefronts a workgroup)
+    K1 = 128 if H != 3584 else 4160       # (the long one: 224 tiles, rows of an odd number of pairs of k-steps)
     x = randn(M, K1, dtype=torch.bfloat16, seed=1)
     if -(-H // th) > 512:
         pytest.skip("more tiles than the readers of the stream add up sums of squares for")
