@@ -39,16 +39,21 @@ class ProductOps:
         two = -(-(-(-tiles // 2)) // self._num_cus) * (2 * w + x)
         return two < 0.97 * one
 
-    def _tiles_a_workgroup(self, M, N, K, th, whole) -> int:
+    def _tiles_a_workgroup(self, M, N, K, th, whole, plain=False) -> int:
         """Tiles of W (``th`` rows each) that a workgroup of a few-rows product owns: 2, 1, or 0 for half of one.
         Halves (not where ``whole``: a gate and its up product, a channel and its partner lie in one tile) as long as
         they go round the CUs once: a CU pulls some 50 GB/s whatever the kernel does, and a matrix of 2,048 rows has tiles
         for half of them (us, whole / half: 2048 x 11008 at 1 / 4 rows 10.6 / 12.1 and 9.2 / 9.8, 2048 x 2048 3.8 / 4.0 and
         3.4 / 3.7, 896 x 4864 5.8 and 4.9, 64 x 2048 3.2 and 2.8).  Beyond, the halves' second round costs more than the
-        idle CUs (2112 x 2048 3.9 and 4.2, 3584 x 18944 at 8 rows 24.0 and 30.8)."""
+        idle CUs (2112 x 2048 3.9 and 4.2, 3584 x 18944 at 8 rows 24.0 and 30.8), until whole tiles are two on some CUs where
+        halves are three: up to four rows then (us at 1 / 4 rows 5120 x 27648 56.4 / 58.9 and 53.1 / 57.8, 4608 x 8192 18.9 / 20.2 and 16.8 / 18.7,
+        4224 x 2048 6.1 / 6.3 and 5.7 / 6.1; at 8 rows x is read again too often, 34.9 and 37.3 of 5120 x 13824).  ``plain``: not a product that
+        adds to the stream, whose readers take 512 sums of squares a row at most."""
         if self._pair_tiles(M, N, K, th):
             return 2
-        return 0 if not whole and th == 16 and 2 * -(-N // 16) <= self._num_cus else 1
+        tiles = -(-N // 16)
+        third = plain and M <= 4 and K >= 1024 and self._num_cus < tiles and 2 * tiles <= 3 * self._num_cus
+        return 0 if not whole and th == 16 and (2 * tiles <= self._num_cus or third) else 1
 
     def _skinny(self, x, weight, bias, y, M, N, K, out_f32=False, gated=False, scaled=None,
                 resid=None, next_gain=None, out_parts=None, rope=None, y_tiled=False, act=0):
@@ -59,7 +64,7 @@ class ProductOps:
             x_tiled, x = x.shape[0], x.data
         # (the product that adds to the stream reads the copy in lower tiles, where the matrix has one)
         wt, th = self._producer_copy(weight, M) if resid is not None else (weight.tiled, 16)
-        tiles = self._tiles_a_workgroup(M, N, K, th, gated or scaled is not None or rope is not None)
+        tiles = self._tiles_a_workgroup(M, N, K, th, gated or scaled is not None or rope is not None, resid is None)
         self._call("gemm", "sl_gemm_skinny", _p(x), _p(wt), _p(bias), _p(y), M, N, K,
                    int(out_f32), int(gated), _p(parts), parts.shape[0] if parts is not None else 0,
                    _c_float(scaled.eps if scaled is not None else 0.0),

@@ -66,3 +66,22 @@ def test_halves_go_round_the_cus_once():
     ops._num_cus = 256
     assert [ops._tiles_a_workgroup(4, N, 2048, 16, False) for N in (64, 2048, 2049, 3584)] == [0, 0, 1, 1]
     assert ops._tiles_a_workgroup(4, 2048, 2048, 16, True) == 1 and ops._tiles_a_workgroup(4, 2048, 2048, 10, False) == 1
+
+
+def test_three_halves_on_a_cu_for_two_tiles():
+    ops = HipOps(torch.bfloat16, DEV)
+    ops._num_cus = 256
+    form = lambda M, N, K, whole=False, plain=True: ops._tiles_a_workgroup(M, N, K, 16, whole, plain)
+    assert [form(4, N, 1024) for N in (4096, 4097, 6144, 6145)] == [1, 0, 0, 1]
+    assert form(5, 5120, 1024) == 1 and form(4, 5120, 992) == 1 and form(4, 5120, 1024, True) == 1 and form(4, 5120, 1024, False, False) == 1
+    # the products, and a delta of as many columns, whose sums of squares are one a whole tile
+    M, N, K = 3, 4136, 1056
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    ops.lower_tiles = False
+    weight, want = ops.prepare_weight(w, residual_delta=True), x.double() @ w.double().T
+    bar = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30
+    assert ((ops.linear(x, weight, None, True).double() - want).abs() <= bar).all()
+    stream = torch.zeros(M, N, device=DEV)
+    rows = ops.add_rmsnorm(stream, ops.linear(x, weight, None, defer=True), torch.ones(N, device=DEV), 1e-6, fuse=True)
+    assert ((stream.double() - want).abs() <= bar).all() and rows.parts.shape[0] == -(-N // 16)
