@@ -264,8 +264,7 @@ template <bool MAX> __device__ __forceinline__ float over_keys(float v) {      /
   auto meet = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
   v = meet(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));   // the other key of two
   v = meet(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true)));   // the other two of four
-  v = meet(v, __shfl_xor(v, 16, 64));
-  return meet(v, __shfl_xor(v, 32, 64));
+  return column_meet(v, meet);
 }
 template <int HD>
 __global__ __launch_bounds__(64) void attention_few_keys_kernel(
@@ -512,8 +511,7 @@ __global__ __launch_bounds__(TILE_THREADS) void attention_general_tile_kernel(
       sc[r] = key >= lo_c && key <= pos_c ? sc[r] * scale : -INFINITY;
       mx = fmaxf(mx, sc[r]);
     }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    mx = row_meet(mx, max_f);
     const float mn = fmaxf(m, mx);
     // a column that has seen no key yet keeps m = -inf: nothing to rescale, nothing to add
     const float alpha = mn == -INFINITY ? 1.f : expf(m - mn);
@@ -524,8 +522,7 @@ __global__ __launch_bounds__(TILE_THREADS) void attention_general_tile_kernel(
       psum += pr;
       ps[col * KB + sub + 16 * r] = pr;
     }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) psum += __shfl_xor(psum, o, 64);
+    psum = row_meet(psum, add_f);
     l = l * alpha + psum;
     m = mn;
     __syncthreads();                                 // ps is complete
@@ -653,8 +650,7 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
         s[kt][i] = key >= lo_c && key <= pos_c ? s[kt][i] * scale : -INFINITY;
         top = fmaxf(top, s[kt][i]);
       }
-    top = fmaxf(top, __shfl_xor(top, 16, 64));
-    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    top = column_meet(top, max_f);
     const float mn = fmaxf(m, top);
     // a column that has seen no key yet keeps m = -inf: nothing to rescale, nothing to add
     const float alpha = mn == -INFINITY ? 1.f : expf(m - mn);
@@ -681,8 +677,7 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
       for (int i = 0; i < 4; ++i) o[dd][i] = fmaf(o[dd][i], alpha, acc[i]);
     }
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = column_meet(l, add_f);
   float odd = 0.f;                                     // (0, or NaN where a result is not finite)
 #pragma unroll
   for (int dd = 0; dd < D / 16; ++dd) odd = fmaf((o[dd][0] + o[dd][1]) + (o[dd][2] + o[dd][3]), 0.f, odd);
@@ -703,8 +698,7 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) sc = fmaf(qf[j][i], kv[i], sc);
       }
-      sc += __shfl_xor(sc, 16, 64);
-      sc += __shfl_xor(sc, 32, 64);
+      sc = column_meet(sc, add_f);
       if (key < lo_c || key > pos_c) continue;
       sc *= scale;
       const float mn = fmaxf(m, sc), alpha = mn == -INFINITY ? 1.f : expf(m - mn), p = sc == -INFINITY ? 0.f : expf(sc - mn);

@@ -28,14 +28,69 @@ template <typename T> __device__ __forceinline__ T from_f(float x);
 template <> __device__ __forceinline__ float from_f<float>(float x) { return x; }
 template <> __device__ __forceinline__ __bf16 from_f<__bf16>(float x) { return (__bf16)x; }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = SL_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, SL_WAVE);
-  return v;
+// The value of lane ^ O, O = 1, 2, 4 or 8, by moves between the lanes of a row of 16 (register to register: 8 cycles, where an
+// exchange through the LDS's crossbar takes about 130).  The source lanes have to be active.
+template <int CTRL, int BANKS = 0xf> __device__ __forceinline__ int row_move(int old, int v) {
+  return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xf, BANKS, false);
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = SL_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, SL_WAVE));
+template <int O> __device__ __forceinline__ float lane_xor(float v) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8, "within a row of 16 lanes");
+  const int x = __float_as_int(v);
+  if (O == 1) return __int_as_float(row_move<0xB1>(0, x));                 // quad_perm [1, 0, 3, 2]
+  if (O == 2) return __int_as_float(row_move<0x4E>(0, x));                 // quad_perm [2, 3, 0, 1]
+  if (O == 8) return __int_as_float(row_move<0x128>(0, x));                // rotated by 8
+  return __int_as_float(row_move<0x114, 0xa>(row_move<0x104, 0x5>(0, x), x));   // quads 0, 2 from the next, 1, 3 from the one before
+}
+// op(v of this lane, v of lane ^ O) in both lanes, O = 16 or 32; op does not mind the order.  (After a swap of a register with
+// itself one result holds the lower partner in every lane and the other the upper one.)
+template <int O, class Op> __device__ __forceinline__ float rows_meet(float v, Op op) {
+  static_assert(O == 16 || O == 32, "rows of 16 lanes, halves of the wavefront");
+  const unsigned x = __float_as_uint(v);
+  if (O == 32) {
+    auto a = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  }
+  auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  return op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+// The value of lane + 32 in lanes 0 .. 31.
+__device__ __forceinline__ float lane_and_32_on(float v) {
+  const unsigned x = __float_as_uint(v);
+  return __uint_as_float(__builtin_amdgcn_permlane32_swap(x, x, false, false)[1]);
+}
+__device__ __forceinline__ float add_f(float a, float b) { return a + b; }
+__device__ __forceinline__ float max_f(float a, float b) { return fmaxf(a, b); }
+
+// Over a wavefront whose lanes are all active, pairs 32, 16, 8, 4, 2, 1 apart in turn; every lane gets the result.  Six exchanges
+// through the LDS's crossbar stood here, in a row: most of the time of a kernel of a few rows is such chains.  (RATES)
+template <class Op> __device__ __forceinline__ float wave_meet(float v, Op op) {
+  v = rows_meet<32>(v, op);
+  v = rows_meet<16>(v, op);
+  v = op(v, lane_xor<8>(v));
+  v = op(v, lane_xor<4>(v));
+  v = op(v, lane_xor<2>(v));
+  return op(v, lane_xor<1>(v));
+}
+// Over the 16 lanes of a row (pairs 8, 4, 2, 1 apart), and over the four lanes l, l + 16, l + 32, l + 48 (16, then 32 apart).
+template <class Op> __device__ __forceinline__ float row_meet(float v, Op op) {
+  v = op(v, lane_xor<8>(v));
+  v = op(v, lane_xor<4>(v));
+  v = op(v, lane_xor<2>(v));
+  return op(v, lane_xor<1>(v));
+}
+template <class Op> __device__ __forceinline__ float column_meet(float v, Op op) { return rows_meet<32>(rows_meet<16>(v, op), op); }
+__device__ __forceinline__ float wave_sum(float v) { return wave_meet(v, add_f); }
+__device__ __forceinline__ float wave_max(float v) { return wave_meet(v, max_f); }
+
+// The sum over this lane and the ones before it, all lanes active: within rows of 16 by shifts of 1, 2, 4 and 8, then the last
+// lanes of rows 0 and 2 to the rows behind them and lane 31 to the upper half.
+__device__ __forceinline__ int sum_up_to(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
   return v;
 }
 

@@ -838,8 +838,7 @@ __global__ __launch_bounds__(512) void gemm_resident_kernel(
     float sacc = 0.f;
 #pragma unroll
     for (int j = 0; j < PARTS; ++j) sacc += pv[j];
-    sacc += __shfl_xor(sacc, 16, 64);
-    sacc += __shfl_xor(sacc, 32, 64);
+    sacc = column_meet(sacc, add_f);
     if (lane < 16) wsum[wave][lane] = sacc;
   }
   __syncthreads();
@@ -1381,7 +1380,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_mid_kernel(
         // rows 0..7 of a tile are gates, 8..15 their ups: lanes gq < 2 fetch the ups from gq + 2
         f32x4 up;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) up[r] = __shfl(acc[t][b][r], lane + 32, 64);
+        for (int r = 0; r < 4; ++r) up[r] = lane_and_32_on(acc[t][b][r]);
         if (gq < 2 && m < M) {
           __bf16* o = (__bf16*)y + (size_t)m * (N / 2) + tile_of[t] * 8 + 4 * gq;
 #pragma unroll

@@ -79,9 +79,12 @@ __global__ __launch_bounds__(KW == 8 ? 512 : 256) void gemm_f32_few_kernel(
       else if constexpr (E == 2) v = sums[0][m][c] + sums[1][m][c];
       else v = sums[0][m][c];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int d = 4; d < 64; d *= 2) v[e] += __shfl_xor(v[e], d);
+      for (int e = 0; e < 4; ++e) {
+        float s = v[e];
+        s += lane_xor<4>(s);
+        s += lane_xor<8>(s);
+        v[e] = column_meet(s, add_f);
+      }
       if (lane < 4) part[wave][m * C + c][lane] = v;
     }
   __syncthreads();

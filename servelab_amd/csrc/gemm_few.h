@@ -217,15 +217,14 @@ __global__ __launch_bounds__(64 * WAVES, TILES == 2 && CONSUMER && !ROPE && PART
     for (int t = 0; t < NT; ++t) red[t][wave][lane] = acc[0][t];
   } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) acc[0][0][r] += __shfl(odd[0][r], lane + 8, 64);
+    for (int r = 0; r < 4; ++r) acc[0][0][r] += lane_xor<8>(odd[0][r]);      // (columns 0..7 are used)
     if (hi == 0) red[0][wave][gq * 8 + i] = acc[0][0];
   }
   if (CONSUMER) {                                            // this wavefront's share of the sums of squares, by row
     float sacc = 0.f;
 #pragma unroll
     for (int j = 0; j < PARTS; ++j) sacc += pv[j];
-    sacc += __shfl_xor(sacc, 16, 64);
-    sacc += __shfl_xor(sacc, 32, 64);
+    sacc = column_meet(sacc, add_f);
     if (lane < 16) wsum[wave][lane] = sacc;
   }
   __syncthreads();
@@ -273,7 +272,7 @@ __global__ __launch_bounds__(64 * WAVES, TILES == 2 && CONSUMER && !ROPE && PART
     if (CONSUMER && live) s *= inv_of(em);
     if constexpr (ROPE) {
       s += b_pre[t];
-      const float partner = __shfl_xor(s, 8, 64);            // the other half of the pair, same row
+      const float partner = lane_xor<8>(s);                  // the other half of the pair, same row
       if (!live) continue;
       const int hd = en / R.D, q = en % R.D;
       if (hd < R.nh + R.nkv) {
@@ -297,8 +296,10 @@ __global__ __launch_bounds__(64 * WAVES, TILES == 2 && CONSUMER && !ROPE && PART
         ((__bf16*)A.y)[at] = (__bf16)(r * g_next[t]);
         sq = r * r;
       }
-#pragma unroll
-      for (int o = C / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);   // over the workgroup's columns of row em
+      if (C == 16) sq += lane_xor<8>(sq);                    // over the workgroup's columns of row em
+      sq += lane_xor<4>(sq);
+      sq += lane_xor<2>(sq);
+      sq += lane_xor<1>(sq);
       if (ec == 0) {
         float* parts = F.out_parts + (size_t)(HALF ? blockIdx.x : tile) * 16 + em;
         parts[0] = sq;

@@ -494,7 +494,7 @@ constexpr int SCAN_ROWS = 8;      // key channels a lane owns: channels 8 p .. 8
 
 // Sum over the P lanes that share a column (P a power of two, the lanes adjacent and aligned); every
 // lane gets the sum.  Within 16 lanes by data-parallel moves (neighbours in a quad, the other pair of
-// the quad, the mirrored half row, the mirrored row), beyond that by shuffles.
+// the quad, the mirrored half row, the mirrored row), beyond that by swaps of rows.
 template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }
@@ -503,7 +503,8 @@ __device__ __forceinline__ float group_sum(float v, int P) {
   if (P >= 4) v += dpp_move<0x4E>(v);          // quad_perm [2, 3, 0, 1]
   if (P >= 8) v += dpp_move<0x141>(v);         // row_half_mirror
   if (P >= 16) v += dpp_move<0x140>(v);        // row_mirror
-  for (int w = 16; w < P; w <<= 1) v += __shfl_xor(v, w, SL_WAVE);
+  if (P >= 32) v = rows_meet<16>(v, add_f);
+  if (P >= 64) v = rows_meet<32>(v, add_f);
   return v;
 }
 struct __attribute__((aligned(16))) scan_f4 { float v[4]; };

@@ -87,7 +87,7 @@ __device__ __forceinline__ int route_token(const Route& r, size_t t, int lane) {
     const float most = wave_max(best);
     unsigned long long holders = __ballot(best == most);
     if (__popcll(holders) == 1) {
-      at = __shfl(at, __ffsll(holders) - 1, SL_WAVE);
+      at = __builtin_amdgcn_readlane(at, __ffsll(holders) - 1);
     } else {
       if (best != most) at = 0x7fffffff;
 #pragma unroll
@@ -116,7 +116,7 @@ __device__ __forceinline__ int route_token(const Route& r, size_t t, int lane) {
     }
     return mine_e;
   }
-  const float top1 = __shfl(mine, 0, SL_WAVE);
+  const float top1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mine)));
   const float w = lane < top ? expf(mine - top1) : 0.f;
   const float sum = wave_sum(w);
   if (lane < top) {
@@ -156,21 +156,13 @@ __device__ __forceinline__ void group_pairs(const Group& g, const int* chosen, i
     int rows = 0, nt = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + tid, c = e < E ? count[e] : 0, tl = e < E_real ? (c + tile_rows - 1) / tile_rows : 0;
-      int up_rows = c, up_tiles = tl;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int a = __shfl_up(up_rows, o, SL_WAVE), b = __shfl_up(up_tiles, o, SL_WAVE);
-        if (tid >= o) {
-          up_rows += a;
-          up_tiles += b;
-        }
-      }
+      const int up_rows = sum_up_to(c), up_tiles = sum_up_to(tl);
       if (e < E) {
         start[e] = rows + up_rows - c;
         tile0[e] = nt + up_tiles - tl;
       }
-      rows += __shfl(up_rows, 63, SL_WAVE);
-      nt += __shfl(up_tiles, 63, SL_WAVE);
+      rows += __builtin_amdgcn_readlane(up_rows, 63);
+      nt += __builtin_amdgcn_readlane(up_tiles, 63);
     }
     if (tid == 0) *g.used = nt;
     for (int i = nt + tid; i < g.max_tiles; i += 64) {

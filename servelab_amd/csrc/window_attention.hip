@@ -131,8 +131,7 @@ __global__ __launch_bounds__(WA_THREADS) void window_attention_kernel(const Wind
       sc[r] = sees ? sv - slope * (float)(pos_c - key) : -INFINITY;
       mx = fmaxf(mx, sc[r]);
     }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    mx = row_meet(mx, max_f);
     const float mn = fmaxf(m, mx);
     // a column that has seen no key yet keeps m = -inf: nothing to rescale, nothing to add
     const float alpha = mn == -INFINITY ? 1.f : expf(m - mn);
@@ -143,8 +142,7 @@ __global__ __launch_bounds__(WA_THREADS) void window_attention_kernel(const Wind
       psum += pr;
       ps[col * KB + sub + 16 * r] = pr;
     }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) psum += __shfl_xor(psum, o, 64);
+    psum = row_meet(psum, add_f);
     l = l * alpha + psum;
     m = mn;
     __syncthreads();                                 // ps is complete
