@@ -748,11 +748,13 @@ extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float
              "gemm_skinny: cache rows need the pages");
   }
   const bool wide = M > 8 || !pair_x || tiles == 2, rp = rope != nullptr;
-  const int pairs = (K / 64 + 7) / 8;            // pairs of k-steps a wavefront takes at most: up to 8 in one trip to memory
+  const int pairs = (K / 64 + 7) / 8;            // pairs of k-steps a wavefront takes at most: up to 8 in one trip to memory, 10 of halves
   if (wide && tiles == 2) launch_few_rows<true, 2, 2>(A, gated, rp, stream);
   else if (wide && tiles == 1 && (N + 15) / 16 > 2 * device_cus() && !producer) launch_few_rows<true, 1, 3>(A, gated, rp, stream);
   else if (wide && tiles == 1) launch_few_rows<true, 1, 4>(A, gated, rp, stream);
+  else if (wide && pairs > 4) launch_few_rows<true, 0, 2>(A, gated, rp, stream);
   else if (wide) launch_few_rows<true, 0, 4>(A, gated, rp, stream);
+  else if (tiles == 0 && pairs > 8 && pairs <= 10) launch_few_rows<false, 0, 10>(A, gated, rp, stream);
   else if (tiles == 0 && pairs > 4 && pairs <= 8) launch_few_rows<false, 0, 8>(A, gated, rp, stream);
   else if (tiles == 0) launch_few_rows<false, 0, 4>(A, gated, rp, stream);
   else if (pairs > 4 && !consumer) launch_few_rows<false, 1, 8>(A, gated, rp, stream);

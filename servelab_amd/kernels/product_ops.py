@@ -44,7 +44,9 @@ class ProductOps:
         Halves (not where ``whole``: a gate and its up product, a channel and its partner lie in one tile) as long as
         they go round the CUs once: a CU pulls some 50 GB/s whatever the kernel does, and a matrix of 2,048 rows has tiles
         for half of them (us, whole / half: 2048 x 11008 at 1 / 4 rows 10.6 / 12.1 and 9.2 / 9.8, 2048 x 2048 3.8 / 4.0 and
-        3.4 / 3.7, 896 x 4864 5.8 and 4.9, 64 x 2048 3.2 and 2.8).  Beyond, the halves' second round costs more than the
+        3.4 / 3.7, 896 x 4864 5.8 and 4.9, 64 x 2048 3.2 and 2.8; products that add to the stream, a copy in tiles of 8 rows / halves,
+        at 1 / 8 / 16 rows: 896 x 4864 5.7 / 6.5 / 8.4 and 4.5 / 5.9 / 7.5, 2048 x 11008 10.7 / 11.8 / 15.8 and 9.4 / 10.9 / 14.8, 2048 x
+        2048 4.1 / 4.4 / 5.2 and 3.7 / 4.1 / 4.9: a load of a tile of 8 rows brings half as much).  Beyond, the halves' second round costs more than the
         idle CUs (2112 x 2048 3.9 and 4.2, 3584 x 18944 at 8 rows 24.0 and 30.8), until whole tiles are two on some CUs where
         halves are three: up to four rows then (us at 1 / 4 rows 5120 x 27648 56.4 / 58.9 and 53.1 / 57.8, 4608 x 8192 18.9 / 20.2 and 16.8 / 18.7,
         4224 x 2048 6.1 / 6.3 and 5.7 / 6.1; at 8 rows x is read again too often, 34.9 and 37.3 of 5120 x 13824).  ``plain``: not a product that
@@ -150,7 +152,9 @@ class ProductOps:
                 self._rows_budget -= 2 * N * K
             self._matrices_with_rows += 1
             weight = LinearWeight(w, tiled)
-        if residual_delta and self.fuse_norms and self.lower_tiles:
+        # (halves of tiles of 16 rows, where they go round the CUs once, are as many workgroups and take the same copy as every
+        # other product: ``_tiles_a_workgroup``)
+        if residual_delta and self.fuse_norms and self.lower_tiles and (_th is not None or 2 * -(-N // 16) > self._num_cus):
             th, lower_from = (_th, 1) if _th is not None else self.producer_tile_height(N)
             if th != 16:
                 weight.lower = torch.empty(-(-N // th) * th * K, dtype=torch.bfloat16, device=self.device)
