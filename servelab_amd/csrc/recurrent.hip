@@ -819,6 +819,168 @@ __global__ void normaliser_kernel(const MatrixScan a) {
   if (threadIdx.x == 0) slot[(size_t)a.H * a.D + h] = from[a.D];
 }
 
+// A step of one token a sequence: the recurrences above, without their LDS.  P lanes share a column of S as there, 256 / P columns side by
+// side and J of them one after the other a lane, so that a lane has up to 2 J pieces of the state on their way at once; what a token
+// brings (q, k, decays, gates) every lane works out for the channels it owns.  Of a column a lane owns channels 4 p .. 4 p + 3 of its
+// first half and of its second: a load of a column's lanes is one run of memory.  The matrix LSTM's n and m are read, and
+// carried on, by every column's lanes; the first ones leave the new values for normaliser_kernel.
+// Bound by streaming the state in and out.  (MEASURED)
+struct Channels8 { float v[8]; };
+typedef float state_v4 __attribute__((ext_vector_type(4)));
+template <int MODE, int J>
+__global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, int P, int lgP, int aligned) {
+  constexpr bool SCALAR = MODE == SCAN_LSTM || MODE == SCAN_SSD || MODE == SCAN_DELTA_HEAD;
+  const int s = blockIdx.x, h = blockIdx.y, g = h / (a.H / a.G);
+  const int p = threadIdx.x & (P - 1), cl = threadIdx.x >> lgP, cols = 256 >> lgP;
+  const int r0 = 4 * p, r1 = 4 * P + 4 * p, D = a.D;
+  const bool fresh = a.positions[s] == 0;
+  float* slot = a.state + (size_t)a.slots[s] * a.state_stride;
+  // the 8 values of a row of D channels that this lane owns
+  auto channels = [&](const float* row, float beyond) {
+    Channels8 c;
+    if (aligned && r1 + 4 <= D) {
+      const scan_f4 x = *(const scan_f4*)(row + r0), y = *(const scan_f4*)(row + r1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c.v[i] = x.v[i], c.v[4 + i] = y.v[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = i < 4 ? r0 + i : r1 + i - 4;
+        c.v[i] = r < D ? row[r] : beyond;
+      }
+    }
+    return c;
+  };
+  const float* row = a.src + (size_t)s * a.src_stride;
+  Channels8 S[J], q = channels(row + a.q_col + g * D, 0.f), k = channels(row + a.k_col + g * D, 0.f), d, n;
+  if (!SCALAR && MODE != SCAN_FORGET) d = channels(a.log_decay + ((size_t)s * a.H + h) * D, 0.f);
+  if (MODE == SCAN_FORGET) d = channels(a.lower + h * D, 0.f);
+  float g0 = 0.f, g1 = 0.f, v[J];
+  if (MODE != SCAN_DECAY && MODE != SCAN_FORGET) {
+    const float* gr = a.gates + (size_t)s * a.gate_stride;
+    g0 = gr[a.i_col + h];
+    if (MODE == SCAN_LSTM || MODE == SCAN_DELTA_HEAD) g1 = gr[a.f_col + h];
+  }
+  const int j0 = blockIdx.z * J * cols + cl;             // columns j0, j0 + cols, ..
+#pragma unroll
+  for (int u = 0; u < J; ++u) {
+    const int j = min(j0 + u * cols, a.Dv - 1);
+    v[u] = row[a.v_col + h * a.Dv + j];
+    const float* col = slot + ((size_t)h * a.Dv + j) * D;
+    if (fresh) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) S[u].v[i] = 0.f;
+    } else if (aligned && r1 + 4 <= D) {
+      const state_v4 x = __builtin_nontemporal_load((const state_v4*)(col + r0)), y = __builtin_nontemporal_load((const state_v4*)(col + r1));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[u].v[i] = x[i], S[u].v[4 + i] = y[i];
+    } else {
+      S[u] = channels(col, 0.f);
+    }
+  }
+  const size_t nS = (size_t)a.H * a.Dv * D;
+  float m = 0.f;
+  if (MODE == SCAN_LSTM) {
+    if (fresh) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) n.v[i] = 0.f;
+    } else {
+      n = channels(slot + nS + (size_t)h * D, 0.f);
+      m = slot[nS + (size_t)a.H * D + h];
+    }
+  }
+  // what the token brings
+  float keep = 0.f, add = 0.f, divisor = 1.f;
+  if (MODE == SCAN_FORGET) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // (as in matrix_scan_kernel: f and 1 - f each from its own side; q passes silu)
+      const bool in = (i < 4 ? r0 + i : r1 + i - 4) < D;
+      const float en = expf(-fabsf(k.v[i])), big = 1.f / (1.f + en), small = en * big, bound = d.v[i];
+      const bool pos = k.v[i] >= 0.f;
+      q.v[i] = q.v[i] * sigmoidf_(q.v[i]) * a.q_scale;
+      k.v[i] = in ? (1.f - bound) * (pos ? small : big) : 0.f;
+      d.v[i] = in ? bound + (1.f - bound) * (pos ? big : small) : 1.f;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      q.v[i] *= a.q_scale;
+      if (!SCALAR) d.v[i] = expf(d.v[i]);
+    }
+  }
+  if (MODE == SCAN_DELTA) add = sigmoidf_(g0);
+  if (MODE == SCAN_DELTA_HEAD) {
+    keep = expf(-expf(a.rates[h]) * softplusf_(g1 + a.step_bias[h]));
+    add = sigmoidf_(g0);
+  }
+  if (MODE == SCAN_SSD) {
+    add = softplusf_(g0 + a.step_bias[h]);
+    keep = expf(-expf(a.rates[h]) * add);
+  }
+  auto sum_of = [&](const float* x) { return group_sum(rows_sum<8>(x), P); };
+  if (MODE == SCAN_LSTM) {
+    const float ig = a.cap * tanhf(g0 / a.cap), fg = logsigmoidf_(a.cap * tanhf(g1 / a.cap));
+    const float top = fmaxf(fg + m, ig);
+    keep = expf(fg + m - top);
+    add = expf(ig - top);
+    float part[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      n.v[i] = keep * n.v[i] + k.v[i] * add;
+      part[i] = n.v[i] * q.v[i];
+    }
+    divisor = fmaxf(fabsf(sum_of(part)), expf(-top)) + 1e-6f;
+    if (a.write && blockIdx.z == 0 && cl == 0) {
+      float* to = a.normaliser + ((size_t)s * a.H + h) * (D + 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = i < 4 ? r0 + i : r1 + i - 4;
+        if (r < D) to[r] = n.v[i];
+      }
+      if (p == 0) to[D] = top;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < J; ++u) {
+    float part[8], in = v[u];
+    if (MODE == SCAN_DELTA) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) part[i] = S[u].v[i] * (d.v[i] * k.v[i]);
+      in = add * (v[u] - sum_of(part));
+    } else if (MODE == SCAN_DELTA_HEAD) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) part[i] = S[u].v[i] * k.v[i];
+      in = add * (v[u] - keep * sum_of(part));
+    } else if (MODE == SCAN_LSTM || MODE == SCAN_SSD) {
+      in = add * v[u];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      S[u].v[i] = (SCALAR ? keep : d.v[i]) * S[u].v[i] + k.v[i] * in;
+      part[i] = S[u].v[i] * q.v[i];
+    }
+    float o = sum_of(part);
+    if (MODE == SCAN_LSTM) o = o / divisor;
+    if (MODE == SCAN_SSD) o += a.skip[h] * v[u];
+    const int j = j0 + u * cols;
+    if (j >= a.Dv) continue;
+    if (p == 0) a.out[((size_t)s * a.H + h) * a.Dv + j] = o;
+    if (!a.write) continue;
+    float* col = slot + ((size_t)h * a.Dv + j) * D;
+    if (aligned && r1 + 4 <= D) {
+      __builtin_nontemporal_store(state_v4{S[u].v[0], S[u].v[1], S[u].v[2], S[u].v[3]}, (state_v4*)(col + r0));
+      __builtin_nontemporal_store(state_v4{S[u].v[4], S[u].v[5], S[u].v[6], S[u].v[7]}, (state_v4*)(col + r1));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = i < 4 ? r0 + i : r1 + i - 4;
+        if (r < D) col[r] = S[u].v[i];
+      }
+    }
+  }
+}
+
 #include "scan_chunks.h"
 
 // Floats of the workspace that a step of T tokens in S sequences needs to be walked in chunks; 0: it cannot be.
@@ -827,7 +989,8 @@ extern "C" long long sl_matrix_scan_workspace(int mode, int T, int S, int H, int
 }
 
 // workspace: sequences of `line` tokens and more are walked in chunks, which are among the first `lead` (of lead_tokens tokens,
-// the longest of max_len); `rest`: there are others, walked token by token as all of them are without a workspace.
+// the longest of max_len); `rest`: there are others, walked token by token as all of them are without a workspace (max_len 1: of at
+// most one token each).
 extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride, int q_col, int k_col, int v_col,
                                       int H, int G, int D, int Dv, const float* log_decay, float q_scale,
                                       const float* gates, int gate_stride, int i_col, int f_col, float cap,
@@ -855,6 +1018,7 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   SL_CHECK(need <= state_stride, "matrix_scan: the state does not fit its slot");
   if (S == 0 || T == 0) return nullptr;
   if (workspace == nullptr) line = INT_MAX;
+  const bool single = workspace == nullptr && max_len == 1 && T == S;     // (sequences of at most one token, as many as tokens)
   const MatrixScan a{src, src_stride, q_col, k_col, v_col, H, G, D, Dv, log_decay, q_scale, gates, gate_stride,
                      i_col, f_col, rates, step_bias, skip, lower, cap, state, state_stride, cu_q, positions, slots, write, out,
                      normaliser, line};
@@ -881,6 +1045,26 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   // the waits, not the products.)
   int P = 1;
   while (P * SCAN_ROWS < D) P <<= 1;
+  if (single) {
+    const int per = 256 / P, wanted = 512;
+    const bool four = (long long)S * H * ((Dv + 4 * per - 1) / (4 * per)) >= wanted;
+    const bool aligned = (uintptr_t)src % 16 == 0 && (uintptr_t)log_decay % 16 == 0 && (uintptr_t)lower % 16 == 0 && (uintptr_t)state % 16 == 0 &&
+                         state_stride % 4 == 0 && src_stride % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 && D % 4 == 0;
+    auto run = [&](auto wide, auto narrow) {
+      if (four) wide<<<dim3(S, H, (Dv + 4 * per - 1) / (4 * per)), 256, 0, stream>>>(a, P, __builtin_ctz(P), aligned);
+      else narrow<<<dim3(S, H, (Dv + per - 1) / per), 256, 0, stream>>>(a, P, __builtin_ctz(P), aligned);
+    };
+    if (mode == SCAN_DECAY) run(matrix_step_kernel<SCAN_DECAY, 4>, matrix_step_kernel<SCAN_DECAY, 1>);
+    else if (mode == SCAN_DELTA) run(matrix_step_kernel<SCAN_DELTA, 4>, matrix_step_kernel<SCAN_DELTA, 1>);
+    else if (mode == SCAN_SSD) run(matrix_step_kernel<SCAN_SSD, 4>, matrix_step_kernel<SCAN_SSD, 1>);
+    else if (mode == SCAN_DELTA_HEAD) run(matrix_step_kernel<SCAN_DELTA_HEAD, 4>, matrix_step_kernel<SCAN_DELTA_HEAD, 1>);
+    else if (mode == SCAN_FORGET) run(matrix_step_kernel<SCAN_FORGET, 4>, matrix_step_kernel<SCAN_FORGET, 1>);
+    else {
+      run(matrix_step_kernel<SCAN_LSTM, 4>, matrix_step_kernel<SCAN_LSTM, 1>);
+      if (write) normaliser_kernel<<<dim3(S, H), 64, 0, stream>>>(a);
+    }
+    return sl_launch_status();
+  }
   const int cols = 256 / P, Dp = P * SCAN_ROWS;
   const int CH = min(min(16, 2048 / Dp), 8 * P);       // 8 values a thread of each kind a chunk
   const bool scalar = mode == SCAN_LSTM || mode == SCAN_SSD || mode == SCAN_DELTA_HEAD;

@@ -220,6 +220,8 @@ class RecurrentOps:
             size.restype = ctypes.c_longlong
             floats = size(mode, lead_tokens, lead, H, G, D, Dv)
             workspace = self._new((floats,), torch.float32) if floats else None
+        elif T == batch.num_seqs and getattr(batch, "max_q_len", T) == 1:
+            longest = 1                       # a token each (one may say so that has none: then there were fewer tokens)
         self._call(lib, "sl_matrix_scan", mode, _p(src), stride, q_col, k_col, v_col, H, G,
                    D, Dv, _p(log_decay), _c_float(q_scale), _p(gates), gate_stride, i_col, f_col, _c_float(cap),
                    _p(rates), _p(step_bias), _p(skip), _p(lower), _p(state), _ll(slot_size), _p(batch.cu_q),
