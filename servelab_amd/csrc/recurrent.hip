@@ -824,7 +824,8 @@ __global__ void normaliser_kernel(const MatrixScan a) {
 // brings (q, k, decays, gates) every lane works out for the channels it owns.  Of a column a lane owns channels 4 p .. 4 p + 3 of its
 // first half and of its second: a load of a column's lanes is one run of memory.  The matrix LSTM's n and m are read, and
 // carried on, by every column's lanes; the first ones leave the new values for normaliser_kernel.
-// Bound by streaming the state in and out.  (MEASURED)
+// Bound by streaming the state in and out: 8 requests of 14 heads of 128 x 256, forget form, 29 MB, cold, 7.4 us (the walking kernel
+// 16; a copy in place 6.3), one request of 8 such heads 2.9 (2.2), 32 requests of 14 28 (20).
 struct Channels8 { float v[8]; };
 typedef float state_v4 __attribute__((ext_vector_type(4)));
 template <int MODE, int J>
@@ -1046,8 +1047,10 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   int P = 1;
   while (P * SCAN_ROWS < D) P <<= 1;
   if (single) {
-    const int per = 256 / P, wanted = 512;
-    const bool four = (long long)S * H * ((Dv + 4 * per - 1) / (4 * per)) >= wanted;
+    // Four columns a lane where that still leaves five workgroups to four CUs: fewer, and a lane's work for a token is shared by too
+    // few (us, cold, one column / four: 448 workgroups of four 10.7 / 7.4, 256 5.1 / 5.8, 128 4.5 / 5.0, 64 3.7 / 5.0).
+    const int per = 256 / P;
+    const bool four = 4ll * S * H * ((Dv + 4 * per - 1) / (4 * per)) >= 5ll * device_cus();
     const bool aligned = (uintptr_t)src % 16 == 0 && (uintptr_t)log_decay % 16 == 0 && (uintptr_t)lower % 16 == 0 && (uintptr_t)state % 16 == 0 &&
                          state_stride % 4 == 0 && src_stride % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 && D % 4 == 0;
     auto run = [&](auto wide, auto narrow) {

@@ -46,39 +46,44 @@ __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-
 // Merges the shares of a (token, head): out = sum_j w_j o_j / (sum_j w_j l_j + sink's term),
 // w_j = exp(m_j - top); a share without keys has m = -inf and drops out.  One
 // wavefront per (token, head, 64 channels); shares are added in their order.
+// Everything a wavefront needs is asked for before anything is used (SHARES shares: for a share that is not there the last one is
+// read, and not used), so that a call is one trip to memory: behind the weights, eight shares a trip, 32 shares took four.
+template <int SHARES>
 __global__ __launch_bounds__(64) void window_attention_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, int nsplit, int nh, int Dv,
     const float* __restrict__ sinks, const act_t* __restrict__ gate, int gate_stride,
     const float* __restrict__ channel_gate, int channel_stride, act_t* __restrict__ out) {
-  __shared__ float ws[64];
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, d = blockIdx.z * 64 + lane, dc = d < Dv ? d : Dv - 1;
   const size_t base = ((size_t)t * nh + h) * nsplit;
+  float v[SHARES];
+#pragma unroll
+  for (int j = 0; j < SHARES; ++j) v[j] = part_o[(base + (j < nsplit ? j : nsplit - 1)) * Dv + dc];
   // lane j holds share j (at most 64 shares)
-  float mj = -INFINITY, lj = 0.f;
-  if (lane < nsplit) {
-    mj = part_ml[(base + lane) * 2];
-    lj = part_ml[(base + lane) * 2 + 1];
-  }
+  const size_t mine = (base + (lane < nsplit ? lane : nsplit - 1)) * 2;
+  const float m_at = part_ml[mine], l_at = part_ml[mine + 1];
   const float sink = sinks != nullptr ? sinks[h] : -INFINITY;
+  const float open = gate != nullptr ? to_f(gate[(size_t)t * gate_stride + h]) : 0.f;
+  const float open_here = channel_gate != nullptr ? channel_gate[(size_t)t * channel_stride + h * Dv + dc] : 0.f;
+  const float mj = lane < nsplit ? m_at : -INFINITY, lj = lane < nsplit ? l_at : 0.f;
   const float top = fmaxf(wave_max(mj), sink);
   const float wj = mj == -INFINITY ? 0.f : expf(mj - top);
   const float denom = wave_sum(wj * lj) + (sinks != nullptr ? expf(sink - top) : 0.f);
-  ws[lane] = wj;
-  __syncthreads();
   float f = 1.f / denom;
-  if (gate != nullptr) f *= sigmoidf_(to_f(gate[(size_t)t * gate_stride + h]));
-  act_t* o = out + ((size_t)t * nh + h) * Dv;
-  const int d = blockIdx.z * 64 + lane;
-  if (d < Dv) {
-    float s = 0.f;
-    for (int j = 0; j < nsplit; j += 8) {              // eight shares asked for together; added in their order
-      float v[8];
+  if (gate != nullptr) f *= sigmoidf_(open);
+  float s = 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = j + u < nsplit ? part_o[(base + j + u) * Dv + d] : 0.f;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += (j + u < nsplit ? ws[j + u] : 0.f) * v[u];
-    }
-    if (channel_gate != nullptr) s *= sigmoidf_(channel_gate[(size_t)t * channel_stride + h * Dv + d]);
-    o[d] = from_f<act_t>(s * f);
-  }
+  for (int j = 0; j < SHARES; ++j) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wj), j)) * (j < nsplit ? v[j] : 0.f);
+  if (channel_gate != nullptr) s *= sigmoidf_(open_here);
+  if (d < Dv) out[((size_t)t * nh + h) * Dv + d] = from_f<act_t>(s * f);
+}
+
+static inline void launch_combine(const WindowAttention& a, int num_tokens, hipStream_t stream) {
+  auto run = [&](auto kernel) {
+    kernel<<<dim3(num_tokens, a.nh, (a.Dv + 63) / 64), 64, 0, stream>>>(a.part_o, a.part_ml, a.nsplit, a.nh, a.Dv, a.sinks, a.gate, a.gate_stride,
+                                                                     a.channel_gate, a.channel_stride, a.out);
+  };
+  if (a.nsplit <= 8) run(window_attention_combine_kernel<8>);
+  else if (a.nsplit <= 16) run(window_attention_combine_kernel<16>);
+  else if (a.nsplit <= 32) run(window_attention_combine_kernel<32>);
+  else run(window_attention_combine_kernel<64>);
 }

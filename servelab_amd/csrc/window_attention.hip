@@ -254,9 +254,7 @@ extern "C" const char* sl_window_attention(
     e = launch_window_attention<16>(a, grid, need(16), stream);
   }
   if (e || nsplit == 1) return e;
-  window_attention_combine_kernel<<<dim3(num_tokens, nh, (Dv + 63) / 64), 64, 0, stream>>>(
-      part_o, part_ml, nsplit, nh, Dv, sinks, (const act_t*)gate, gate_stride, channel_gate, channel_stride,
-      (act_t*)out);
+  launch_combine(a, num_tokens, stream);
   return sl_launch_status();
 }
 

@@ -413,6 +413,8 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
   }
 }
 
+#include "window_step.h"
+
 static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, hipStream_t stream) {
   const size_t bytes = sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW);
   if (bytes > 48 * 1024) {
@@ -423,6 +425,18 @@ static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, h
   window_attention_mfma_kernel<<<grid, THREADS, bytes, stream>>>(a, order);
   return sl_launch_status();
 }
+static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream_t stream) {
+  const size_t bytes = VK ? sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW) : 0;
+  if (bytes > 48 * 1024) {
+    hipError_t e = hipFuncSetAttribute((const void*)window_step_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return hipGetErrorString(e);
+  }
+  window_step_kernel<<<dim3(a.nsplit, a.nkv * ((a.nh / a.nkv + 15) / 16), num_seqs), 64 * STEP_WAVES, bytes, stream>>>(a);
+  return sl_launch_status();
+}
+
+// Blocks of 32 keys that a workgroup of a step of single tokens takes side by side.
+extern "C" int sl_window_attention_mfma_step_blocks() { return STEP_BLOCKS; }
 
 extern "C" int sl_window_attention_mfma_lds_bytes() {
   return (int)(sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW));
@@ -456,6 +470,13 @@ extern "C" const char* sl_window_attention_mfma(
                           cu_q, positions, nh, nkv, Dk, Dv, page, scale, softcap, window, chunk, keep_first, slopes, sinks,
                           (const act_t*)gate, gate_stride, channel_gate, channel_stride, (act_t*)out, nsplit, part_o,
                           part_ml};
+  if (max_q_len == 1 && num_tokens == num_seqs && (nsplit == 1 || (uintptr_t)part_ml % 8 == 0) &&
+      (long long)nkv * ((nh / nkv + 15) / 16) <= 65535) {              // (a token each)
+    const char* e = launch_step(a, num_seqs, stream);
+    if (e || nsplit == 1) return e;
+    launch_combine(a, num_tokens, stream);
+    return sl_launch_status();
+  }
   const long long cols = (long long)max_q_len * (nh / nkv);
   const long long tiles = (cols + COLS - 1) / COLS;
   SL_CHECK(tiles * nsplit <= 1 << 30, "window attention: too many column tiles");
@@ -467,8 +488,6 @@ extern "C" const char* sl_window_attention_mfma(
   const dim3 grid = order == BY_LENGTH ? dim3(nkv, num_seqs, items) : dim3(items, nkv, num_seqs);
   const char* e = launch_mfma(a, grid, order, stream);
   if (e || nsplit == 1) return e;
-  window_attention_combine_kernel<<<dim3(num_tokens, nh, (Dv + 63) / 64), 64, 0, stream>>>(
-      part_o, part_ml, nsplit, nh, Dv, sinks, (const act_t*)gate, gate_stride, channel_gate, channel_stride,
-      (act_t*)out);
+  launch_combine(a, num_tokens, stream);
   return sl_launch_status();
 }

@@ -14,7 +14,7 @@ DEV = "cuda:0"
 # heads of 16, 8, 32 and 64 lanes a column, of channels that no load of four divides and that no lane's eight do; value channels that no
 # workgroup divides; few blocks (one column a lane) and many (four)
 @pytest.mark.parametrize("S,H,G,D,Dv", [(3, 2, 2, 128, 256), (2, 3, 3, 20, 24), (5, 2, 2, 72, 15), (2, 1, 1, 200, 33), (2, 2, 1, 256, 16),
-                                        (1, 4, 2, 64, 40), (3, 2, 2, 50, 7), (2, 1, 1, 512, 9), (40, 8, 8, 128, 130), (70, 16, 8, 60, 64)])
+                                        (1, 4, 2, 64, 40), (3, 2, 2, 50, 7), (2, 1, 1, 512, 9), (40, 8, 8, 128, 130), (70, 16, 8, 60, 64), (10, 8, 8, 128, 250)])
 @pytest.mark.parametrize("mode", ["decay", "delta", "delta, decay a head", "state space", "forget", "lstm"])
 def test_steps_of_one_token(mode, S, H, G, D, Dv, monkeypatch):
     if mode in ("forget", "lstm"):
