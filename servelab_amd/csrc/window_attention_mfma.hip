@@ -10,24 +10,25 @@
 // together are the float exactly, and the weighted sum of the values is three matrix
 // instructions, one per term, on float accumulators.
 //
-// Work layout.  A column is a (token, query head) pair of one sequence and one kv head; a
-// wavefront owns 16 columns, a workgroup of four wavefronts 64 consecutive ones, and walks the
-// blocks of 32 keys any of them sees.  A block is staged in LDS once for the workgroup: the key
-// rows [32][SL_DK], and the values channel-major [SL_DV][32] (copied from the value pages, which
-// are channel-major already, or turned in registers, 8 keys x 8 channels a thread, on their way
+// Work layout of prompts (steps of single tokens: window_step.h).  A column is a (token, query head) pair of one sequence and one kv
+// head; a wavefront owns 16 columns, a workgroup 64 consecutive ones, and walks the blocks of 32 keys any of them sees.  A block is
+// staged in LDS once for the wavefronts that compute on it: the key rows [32][SL_DK], and the values channel-major [SL_DV][32] (copied
+// from the value pages, which are channel-major already, or turned in registers, 8 keys x 8 channels a thread, on their way
 // from the key rows); the next block is on its way from the pages to registers while a block is
 // computed.  Per block and wavefront:
 //   S^T[key, column] = K[key, :] . Q[column, :]          mfma 16x16x32, A = K rows, B = Q (registers)
 //   O^T[d, column] += V^T[d, key] P^T[key, column]       mfma 16x16x32, A = V^T rows, B = the terms of P
 // Row i of score tile m is key 8 (i / 4) + 4 m + i % 4 of the block, so that a lane ends up with
 // the weights of 8 consecutive keys of its column: the B operand of the second product as it is.
-// A step of single tokens has few columns (the heads of a group): its blocks are cut into shares
-// over workgroups, whose wavefronts without a column only help to stage.
 //
-// The widest form (576 / 512) holds one workgroup a CU, 132 matrix instructions a block and wavefront of which the
-// three of a channel tile depend on each other: what it waits for is not hidden by another wavefront, so loads stand
-// behind no condition, four channel tiles go side by side, and the longest tiles start first (two prompts of 945 tokens, 16
-// heads: 248 us before, 160 with the three; 128 / 128, 2,048 tokens: 137 and 112).
+// What bounds it: a block is a chain (stage, scores, maximum, exponentials, terms, sums) of a few thousand cycles, of which the matrix
+// instructions are 500 to 2,100, and the longest tile walks all of its keys; so a workgroup is eight wavefronts: two teams that take every other
+// block and meet at the end, or, where values lie in the key rows (132 matrix instructions a block, more registers than two
+// wavefronts a SIMD have), pairs that share columns, each with half the channels; the longest tiles start first; a
+// block has 150 vector instructions and no branches inside (addresses looked up key by key and a cap chosen score by score were 270 and
+// eight).  us, before / now: 128 / 128, 16 heads on 2, one prompt of 2,048 tokens 104 / 68 (255 TFLOP/s counted once a weight), 1,000 and 889 56 /
+// 38, 1,500 with a window of 1,024 64 / 40; 576 / 512, 16 heads, 1,000 and 889 150 / 137, 2,048 282 / 248.  Tried: blocks of 64
+// keys (a tenth slower at 128, half as slow again at 576), two blocks on their way (registers spill; no gain at 576).
 #include "window_attention.h"
 
 #if defined(SL_F32)
@@ -53,6 +54,11 @@ constexpr bool VK = SL_VK != 0;
 constexpr int KK = DK / 32, DD = DV / 16;
 constexpr int KROW = DK + 8;          // elements of a staged key row (the pad spreads rows over the banks)
 constexpr int VROW = 40;              // elements of a staged channel row: 32 keys and a pad
+constexpr int VPAD = VK ? 32 : 0;     // and more behind every eight of them, where a thread turns eight: neighbouring threads' rows in other banks
+constexpr int VT = DV * VROW + DV / 8 * VPAD;
+__device__ __forceinline__ int channel_row(int d) { return d * VROW + (d >> 3) * VPAD; }
+// Key 8 a + 4 m + b of a block is staged as row 16 m + 4 a + b: the rows of a score tile side by side, which take every bank once.
+__device__ __forceinline__ int staged_row(int key) { return 16 * ((key >> 2) & 1) + 4 * (key >> 3) + (key & 3); }
 constexpr float LOG2E = 1.4426950408889634f;
 
 // Maximum / sum over the four lanes n, n + 16, n + 32, n + 48 that share a column, by the row-swap
@@ -71,7 +77,14 @@ __device__ __forceinline__ float column_sum4(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-constexpr int THREADS = 256, COLS = 64;
+// A prompt's workgroup is eight wavefronts over 64 columns: two teams of four that take every other block and meet at the end, or,
+// where values lie in the key rows, one whose wavefronts share their 16 columns two and two, each with half of the channels.
+constexpr int TEAMS = VK ? 1 : 2, PARTS = VK ? 2 : 1;
+constexpr int THREADS = 256 * PARTS, COLS = 64;         // of a team
+constexpr int KKP = (KK + PARTS - 1) / PARTS, DDP = (DD + PARTS - 1) / PARTS;      // steps of key channels and tiles of value channels a wavefront
+constexpr int MEETS = VK ? 8 * 2 * 64 * 16 : 0;         // bytes in which the parts of the scores meet
+constexpr int STAGE = 32 * KROW + VT;                   // values of a team's staged block
+constexpr int MEET = TEAMS == 2 ? 256 * DV + 512 : 0;   // bytes in which the second team hands over what it has
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
 // what a thread stages of a block: chunks of 8 values (16 bytes)
 constexpr int KCH = DK / 8;                            // chunks of a key row
@@ -91,12 +104,14 @@ constexpr int NR = VK ? (RCH ? cdiv(32 * RCH, THREADS) : 1) : 1;
 // 1,000 410 moved, 463 with early tiles first.)
 enum { IN_ORDER = 0, LATE_FIRST = 1, BY_LENGTH = 2, BY_LENGTH_MOVED = 3 };
 
-// (rows of up to 128 values: four workgroups a CU, which 128 registers allow)
-__global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_mfma_kernel(const WindowAttention a, int order) {
+__global__ __launch_bounds__(TEAMS * THREADS, TEAMS == 1 ? 2 : DK <= 128 && DV <= 128 ? 4 : 2) void window_attention_mfma_kernel(const WindowAttention a, int order) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
-  __bf16* ks = lds16;                                  // [32][KROW]
-  __bf16* vt = ks + 32 * KROW;                         // [DV][VROW]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, gq = lane >> 4;
+  const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
+  __bf16* ks = lds16 + team * STAGE;                   // [32][KROW]
+  __bf16* vt = ks + 32 * KROW;                         // channel_row(d) of channel d
+  f32x4 (*meets)[64] = (f32x4(*)[64])(lds16 + STAGE);  // [2 parts][4 wavefronts][2 tiles of keys]
+  const int tid = threadIdx.x % THREADS, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, n = lane & 15, gq = lane >> 4;
+  const int part = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
   const int page = a.page, nkv = a.nkv;
   int seq = blockIdx.z, kvh = blockIdx.y, item = blockIdx.x;
   if (order == LATE_FIRST) {
@@ -134,7 +149,7 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
   if (firstB < nA) firstB = nA;
   const int nB = kmax / 32 - firstB + 1 > 0 ? kmax / 32 - firstB + 1 : 0;
   const int nblk = nA + nB;
-  const int i0 = (int)((long long)nblk * share / a.nsplit);
+  const int from_block = (int)((long long)nblk * share / a.nsplit), i0 = from_block + team;
   const int i1 = (int)((long long)nblk * (share + 1) / a.nsplit);
   // The blocks are walked from the nearest keys to the farthest (the kept first tokens last): a distance
   // bias makes nearer keys score higher, so the running maximum settles in the first block or two and
@@ -143,7 +158,7 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
     const int b = nblk - 1 - i;
     return (b < nA ? b : firstB + (b - nA)) * 32;
   };
-  auto loadable = [&](int key) { return key <= kmax && (key >= kmin || key < keep); };
+  auto loadable = [&](int key) { return (key <= kmax) & ((key >= kmin) | (key < keep)); };
 
   // this wavefront's columns, and this lane's (a column past the last is computed like the last, never stored)
   const int cw0 = c0 + 16 * wave;
@@ -163,15 +178,15 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
   const bool capped = a.softcap > 0.f;
   const float cap2 = a.softcap * LOG2E, uncap = capped ? a.scale / a.softcap : 0.f;
   const float slope2 = a.slopes != nullptr ? a.slopes[head] * LOG2E : 0.f;
-  bf16x8 qf[KK];
+  bf16x8 qf[KKP];
   {
     const __bf16* qp = a.q + (size_t)(q0 + tok) * a.q_stride + (size_t)head * DK + 8 * gq;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) qf[kk] = *(const bf16x8*)(qp + 32 * kk);
+    for (int kk = 0; kk < KKP; ++kk) qf[kk] = *(const bf16x8*)(qp + 32 * min(part * KKP + kk, KK - 1));
   }
-  f32x4 o[DD];
+  f32x4 o[DDP];
 #pragma unroll
-  for (int dd = 0; dd < DD; ++dd) o[dd] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int dd = 0; dd < DDP; ++dd) o[dd] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;                        // the maximum in units of log 2
   const __bf16 zero = (__bf16)0.f;
 
@@ -185,57 +200,55 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
     const int key = kbase + ((lane & 1) << 4);
     return table[(key <= kmax ? key : kbase) >> page_shift];
   };
-  // A key no column sees is replaced by one of the block that some column does: no load stands behind a
-  // condition (the compiler waits for a load where the two ways meet, and eight rows a block are then eight trips to
-  // memory in turn), and what comes in its place gets no weight.
-  auto seen_in = [&](int key, int kbase) {
-    key = min(key, kmax);
-    return key >= kmin || key < keep ? key : (kmin <= kbase + 31 ? kmin : keep - 1);
-  };
+  // A half of a block (16 keys, of one page) is read where it lies: a place for both halves, which is the same for all threads, and a
+  // thread's own places beside it, which are the same for all blocks.  (Clamped and looked up key by key the addresses were 100 of
+  // a block's 270 vector instructions.)  A half of which no column sees a key may have no page: the other half stands for it.  What
+  // lies in slots no column sees gets no weight, and values there become zeros.  No load stands behind a condition: the
+  // compiler waits for a load where the two ways meet.
   bf16x8 kreg[NKC], vreg[NVC], treg[NT][8], rreg[NR];
   auto fetch = [&](int kbase, int asked) {
     const int pgA = __builtin_amdgcn_readlane(asked, 0), pgB = __builtin_amdgcn_readlane(asked, 1);
-    auto key_row = [&](int kl) {                       // start of the cache row of key kbase + kl
-      const int key = seen_in(kbase + kl, kbase), pg = key < kbase + 16 ? pgA : pgB;
-      return a.kc + (((size_t)pg * nkv + kvh) * page + (key & (page - 1))) * DK;
-    };
+    const bool seenA = kbase + 15 >= kmin || kbase < keep, seenB = kbase + 16 <= kmax && (kbase + 31 >= kmin || kbase + 16 < keep);
+    const size_t headA = (size_t)(seenA ? pgA : pgB) * nkv + kvh, headB = (size_t)(seenB ? pgB : pgA) * nkv + kvh;
+    const int inA = (seenA ? kbase : kbase + 16) & (page - 1), inB = (seenB ? kbase + 16 : kbase) & (page - 1);
+    const __bf16 *keysA = a.kc + (headA * page + inA) * DK, *keysB = a.kc + (headB * page + inB) * DK;
     if constexpr (!VK) {
 #pragma unroll
       for (int i = 0; i < NKC; ++i) {
-        const int idx = min(tid + THREADS * i, 32 * KCH - 1);
-        kreg[i] = *(const bf16x8*)(key_row(idx / KCH) + 8 * (idx % KCH));
+        const int idx = min(tid + THREADS * i, 32 * KCH - 1), kl = idx / KCH;
+        const bool second = 16 * KCH % THREADS == 0 ? THREADS * i >= 16 * KCH : kl >= 16;
+        kreg[i] = *(const bf16x8*)((second ? keysB : keysA) + (kl & 15) * DK + 8 * (idx % KCH));
       }
+      const __bf16 *valuesA = a.vc + headA * DV * page + inA, *valuesB = a.vc + headB * DV * page + inB;
 #pragma unroll
       for (int i = 0; i < NVC; ++i) {
-        const int idx = min(tid + THREADS * i, DV * 4 - 1), d = idx / 4, key0 = kbase + 8 * (idx % 4);
-        // (a chunk of 8 keys with one that is seen, else the chunk of one that is)
-        const int key = key0 <= kmax && (key0 + 7 >= kmin || key0 < keep) ? key0 : seen_in(key0, kbase) & ~7;
-        const int pg = key < kbase + 16 ? pgA : pgB;
-        vreg[i] = *(const bf16x8*)(a.vc + (((size_t)pg * nkv + kvh) * DV + d) * page + (key & (page - 1)));
+        const int idx = min(tid + THREADS * i, DV * 4 - 1);
+        vreg[i] = *(const bf16x8*)((idx & 2 ? valuesB : valuesA) + (idx / 4) * page + 8 * (idx & 1));
       }
     } else {
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         const int idx = min(tid + THREADS * i, (DV / 8) * 4 - 1), cb = idx / 4, kg = idx % 4;
+        const __bf16* at = (kg & 2 ? keysB : keysA) + 8 * (kg & 1) * DK + 8 * cb;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) treg[i][j] = *(const bf16x8*)(key_row(8 * kg + j) + 8 * cb);
+        for (int j = 0; j < 8; ++j) treg[i][j] = *(const bf16x8*)(at + j * DK);
       }
       if constexpr (RCH > 0) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-          const int idx = min(tid + THREADS * i, 32 * RCH - 1), kl = idx / RCH, c8 = DV / 8 + idx % RCH;
-          rreg[i] = *(const bf16x8*)(key_row(kl) + 8 * c8);
+          const int idx = min((tid ^ 256) + THREADS * i, 32 * RCH - 1), kl = idx / RCH, c8 = DV / 8 + idx % RCH;
+          rreg[i] = *(const bf16x8*)((kl >= 16 ? keysB : keysA) + (kl & 15) * DK + 8 * c8);
         }
       }
     }
   };
   auto store = [&](int kbase) {
+    const bool all_seen = kbase + 31 <= kmax && (kbase >= kmin || kbase + 31 < keep);
     if constexpr (!VK) {
-      const bool all_seen = kbase + 31 <= kmax && (kbase >= kmin || kbase + 31 < keep);
 #pragma unroll
       for (int i = 0; i < NKC; ++i) {
         const int idx = tid + THREADS * i, kl = idx / KCH, c8 = idx % KCH;
-        if (idx < 32 * KCH) *(bf16x8*)(ks + kl * KROW + 8 * c8) = kreg[i];
+        if (32 * KCH % THREADS == 0 || idx < 32 * KCH) *(bf16x8*)(ks + staged_row(kl) * KROW + 8 * c8) = kreg[i];
       }
 #pragma unroll
       for (int i = 0; i < NVC; ++i) {
@@ -244,31 +257,36 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
         if (!all_seen) {                               // a slot of the page that holds no visible key may hold anything
 #pragma unroll
           for (int e = 0; e < 8; ++e)
-            if (!loadable(kbase + 8 * k8 + e)) v[e] = zero;
+            v[e] = loadable(kbase + 8 * k8 + e) ? v[e] : zero;
         }
-        if (idx < DV * 4) *(bf16x8*)(vt + d * VROW + 8 * k8) = v;
+        if (DV * 4 % THREADS == 0 || idx < DV * 4) *(bf16x8*)(vt + channel_row(d) + 8 * k8) = v;
       }
     } else {
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         const int idx = tid + THREADS * i, cb = idx / 4, kg = idx % 4;
-        if (idx < (DV / 8) * 4) {
+        if (DV / 2 % THREADS == 0 || idx < (DV / 8) * 4) {
+          if (!all_seen) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) *(bf16x8*)(ks + (8 * kg + j) * KROW + 8 * cb) = treg[i][j];
+            for (int j = 0; j < 8; ++j)
+              if (!loadable(kbase + 8 * kg + j)) treg[i][j] = bf16x8{zero, zero, zero, zero, zero, zero, zero, zero};
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j) *(bf16x8*)(ks + staged_row(8 * kg + j) * KROW + 8 * cb) = treg[i][j];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {                // channel 8 cb + e of the tile's 8 keys
             bf16x8 t;
 #pragma unroll
             for (int j = 0; j < 8; ++j) t[j] = treg[i][j][e];
-            *(bf16x8*)(vt + (8 * cb + e) * VROW + 8 * kg) = t;
+            *(bf16x8*)(vt + channel_row(8 * cb + e) + 8 * kg) = t;
           }
         }
       }
       if constexpr (RCH > 0) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-          const int idx = tid + THREADS * i, kl = idx / RCH, c8 = DV / 8 + idx % RCH;
-          if (idx < 32 * RCH) *(bf16x8*)(ks + kl * KROW + 8 * c8) = rreg[i];
+          const int idx = (tid ^ 256) + THREADS * i, kl = idx / RCH, c8 = DV / 8 + idx % RCH;
+          if (32 * RCH % THREADS == 0 || idx < 32 * RCH) *(bf16x8*)(ks + staged_row(kl) * KROW + 8 * c8) = rreg[i];
         }
       }
     }
@@ -277,63 +295,84 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
   int asked = 0;
   if (i0 < i1) {
     fetch(block_base(i0), ask_pages(block_base(i0)));
-    if (i0 + 1 < i1) asked = ask_pages(block_base(i0 + 1));
+    if (i0 + TEAMS < i1) asked = ask_pages(block_base(i0 + TEAMS));
   }
   // (q, asked for before the first keys, is waited for here: left to the loop, the wait for its first use would be one for the
   // next block's keys as well)
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
-  for (int i = i0; i < i1; ++i) {
+  for (int kk = 0; kk < KKP; ++kk) asm volatile("" : "+v"(qf[kk]));
+  for (int i = i0; i - team < i1; i += TEAMS) {        // (as many rounds for both teams; the second may have no block in the last)
     const int kbase = block_base(i);
     __syncthreads();                                   // the last block's readers are done
-    store(kbase);
+    if (i < i1) store(kbase);
     __syncthreads();
-    if (i + 1 < i1) {
-      fetch(block_base(i + 1), asked);
-      if (i + 2 < i1) asked = ask_pages(block_base(i + 2));
+    if (i + TEAMS < i1) {
+      fetch(block_base(i + TEAMS), asked);
+      if (i + 2 * TEAMS < i1) asked = ask_pages(block_base(i + 2 * TEAMS));
     }
-    if (!wave_live) continue;                          // (a wavefront without columns only helps staging)
+    if (PARTS == 1 && (!wave_live || i >= i1)) continue;             // (a wavefront without columns only helps staging)
 
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-    const __bf16* kp = ks + (8 * (n / 4) + n % 4) * KROW + 8 * gq;
+    const __bf16* kp = ks + n * KROW + 8 * gq;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      const bf16x8 k0 = *(const bf16x8*)(kp + 32 * kk);
-      const bf16x8 k1 = *(const bf16x8*)(kp + 4 * KROW + 32 * kk);
+    for (int kk = 0; kk < KKP; ++kk) {
+      if (KK % PARTS != 0 && part * KKP + kk >= KK) continue;
+      const bf16x8 k0 = *(const bf16x8*)(kp + 32 * (part * KKP + kk));
+      const bf16x8 k1 = *(const bf16x8*)(kp + 16 * KROW + 32 * (part * KKP + kk));
       s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qf[kk], s0, 0, 0, 0);
       s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qf[kk], s1, 0, 0, 0);
     }
+    if constexpr (PARTS == 2) {
+      meets[(part * 4 + wave) * 2][lane] = s0;
+      meets[(part * 4 + wave) * 2 + 1][lane] = s1;
+      __syncthreads();
+      if (!wave_live) continue;
+      s0 = meets[2 * wave][lane] + meets[8 + 2 * wave][lane];
+      s1 = meets[2 * wave + 1][lane] + meets[8 + 2 * wave + 1][lane];
+    }
     // score of key kbase + 8 gq + j: raw * scale - slope * (pos_c - key), in units of log 2
     const float bias0 = -slope2 * (float)(pos_c - kbase - 8 * gq);
-    float s[8], top = -INFINITY;
+    // (a cap takes its own pass: chosen score by score it is eight branches a block, which nothing is scheduled across)
+    float s[8], top = -INFINITY, factor = scale2;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float raw = j < 4 ? s0[j] : s1[j - 4];
-      s[j] = capped ? fmaf(tanhf(raw * uncap), cap2, fmaf(slope2, (float)j, bias0))
-                    : fmaf(raw, scale2, fmaf(slope2, (float)j, bias0));
+    for (int j = 0; j < 8; ++j) s[j] = j < 4 ? s0[j] : s1[j - 4];
+    if (capped) {
+      factor = cap2;
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float t = tanhf((h ? s[4 + j] : s[j]) * uncap);
+          if (h) s[4 + j] = t;
+          else s[j] = t;
+        }
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] = fmaf(s[j], factor, fmaf(slope2, (float)j, bias0));
     const bool whole = kbase + 31 <= pos_lo && (kbase >= lo_hi || kbase + 31 < a.keep_first);
     if (!whole) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int key = kbase + 8 * gq + j;
-        if (!(key <= pos_c && (key >= lo_c || key < a.keep_first))) s[j] = -INFINITY;
+        const bool seen = (key <= pos_c) & ((key >= lo_c) | (key < a.keep_first));      // (no branches)
+        s[j] = seen ? s[j] : -INFINITY;
       }
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) top = fmaxf(top, s[j]);
     const float mn = fmaxf(m, column_max4(top));
+    const float from = mn == -INFINITY ? 0.f : mn;     // (only while no key was seen: exp2(-inf) = 0)
     float p[8], psum = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {                      // exp2(-inf) = 0; mn = -inf only while no key was seen
-      p[j] = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[j] - mn);
+    for (int j = 0; j < 8; ++j) {
+      p[j] = __builtin_amdgcn_exp2f(s[j] - from);
       psum += p[j];
     }
     if (__any(mn > m)) {                               // the maximum of some column moved: rescale
       const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
       l *= alpha;
 #pragma unroll
-      for (int dd = 0; dd < DD; ++dd) o[dd] *= alpha;
+      for (int dd = 0; dd < DDP; ++dd) o[dd] *= alpha;
       m = mn;
     }
     l += column_sum4(psum);
@@ -358,12 +397,13 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
     const bf16x8 p1 = __builtin_bit_cast(bf16x8, w1), p2 = __builtin_bit_cast(bf16x8, w2),
                  p3 = __builtin_bit_cast(bf16x8, w3);
     // (four tiles of channels side by side: the three products of one depend on each other)
-    constexpr int SIDE = DD % 4 == 0 ? 4 : 1;
+    constexpr int SIDE = DDP % 4 == 0 && DD % PARTS == 0 ? 4 : 1;
 #pragma unroll
-    for (int dd = 0; dd < DD; dd += SIDE) {
+    for (int dd = 0; dd < DDP; dd += SIDE) {
+      if (DD % PARTS != 0 && part * DDP + dd >= DD) continue;
       bf16x8 vf[SIDE];
 #pragma unroll
-      for (int u = 0; u < SIDE; ++u) vf[u] = *(const bf16x8*)(vt + (16 * (dd + u) + n) * VROW + 8 * gq);
+      for (int u = 0; u < SIDE; ++u) vf[u] = *(const bf16x8*)(vt + channel_row(16 * (part * DDP + dd + u) + n) + 8 * gq);
 #pragma unroll
       for (int u = 0; u < SIDE; ++u) o[dd + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[u], p3, o[dd + u], 0, 0, 0);
 #pragma unroll
@@ -372,14 +412,34 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
       for (int u = 0; u < SIDE; ++u) o[dd + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[u], p1, o[dd + u], 0, 0, 0);
     }
   }
+  if constexpr (TEAMS == 2) {                          // the first team takes what the second has of its columns
+    f32x4* os = (f32x4*)lds16;
+    float2* ml = (float2*)(os + THREADS * DD);
+    __syncthreads();
+    if (team == 1) {
+#pragma unroll
+      for (int dd = 0; dd < DD; ++dd) os[THREADS * dd + tid] = o[dd];
+      if (gq == 0) ml[16 * wave + n] = make_float2(m, l);
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const float2 other = ml[16 * wave + n];
+    const float both = fmaxf(m, other.x), ours = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - both),
+                theirs = other.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(other.x - both);
+#pragma unroll
+    for (int dd = 0; dd < DD; ++dd) o[dd] = o[dd] * ours + os[THREADS * dd + tid] * theirs;
+    l = l * ours + other.y * theirs;
+    m = both;
+  }
   if (!live) return;
   // this lane holds channels 16 dd + 4 gq .. + 3 of its column
   const size_t row = (size_t)(q0 + tok) * a.nh + head;
   if (a.nsplit > 1) {
-    float* po = a.part_o + (row * a.nsplit + share) * DV + 4 * gq;
+    float* po = a.part_o + (row * a.nsplit + share) * DV + 16 * part * DDP + 4 * gq;
 #pragma unroll
-    for (int dd = 0; dd < DD; ++dd) *(f32x4*)(po + 16 * dd) = o[dd];
-    if (gq == 0) {
+    for (int dd = 0; dd < DDP; ++dd)
+      if (DD % PARTS == 0 || part * DDP + dd < DD) *(f32x4*)(po + 16 * dd) = o[dd];
+    if (gq == 0 && part == 0) {
       a.part_ml[(row * a.nsplit + share) * 2] = m == -INFINITY ? m : m * (1.f / LOG2E);
       a.part_ml[(row * a.nsplit + share) * 2 + 1] = l;
     }
@@ -395,11 +455,12 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
   const float w = __builtin_amdgcn_exp2f(m - top);
   float f = w / (l * w + extra);
   if (a.gate != nullptr) f *= sigmoidf_(to_f(a.gate[(size_t)(q0 + tok) * a.gate_stride + head]));
-  __bf16* op = a.out + row * DV + 4 * gq;
+  __bf16* op = a.out + row * DV + 16 * part * DDP + 4 * gq;
   const float* cg = a.channel_gate != nullptr
-      ? a.channel_gate + (size_t)(q0 + tok) * a.channel_stride + (size_t)head * DV + 4 * gq : nullptr;
+      ? a.channel_gate + (size_t)(q0 + tok) * a.channel_stride + (size_t)head * DV + 16 * part * DDP + 4 * gq : nullptr;
 #pragma unroll
-  for (int dd = 0; dd < DD; ++dd) {
+  for (int dd = 0; dd < DDP; ++dd) {
+    if (DD % PARTS != 0 && part * DDP + dd >= DD) continue;
     bf16x4 r;
     if (cg != nullptr) {
       struct __attribute__((aligned(4))) gates4 { float v[4]; };      // (one load, whatever the rows' alignment)
@@ -416,17 +477,17 @@ __global__ __launch_bounds__(THREADS, DK <= 128 ? 4 : 1) void window_attention_m
 #include "window_step.h"
 
 static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, hipStream_t stream) {
-  const size_t bytes = sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW);
+  const size_t staged = sizeof(__bf16) * TEAMS * STAGE + MEETS, bytes = staged > MEET ? staged : MEET;
   if (bytes > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return hipGetErrorString(e);
   }
-  window_attention_mfma_kernel<<<grid, THREADS, bytes, stream>>>(a, order);
+  window_attention_mfma_kernel<<<grid, TEAMS * THREADS, bytes, stream>>>(a, order);
   return sl_launch_status();
 }
 static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream_t stream) {
-  const size_t bytes = VK ? sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW) : 0;
+  const size_t bytes = VK ? sizeof(__bf16) * ((size_t)32 * KROW + (size_t)VT) : 0;
   if (bytes > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)window_step_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return hipGetErrorString(e);
@@ -439,7 +500,7 @@ static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream
 extern "C" int sl_window_attention_mfma_step_blocks() { return STEP_BLOCKS; }
 
 extern "C" int sl_window_attention_mfma_lds_bytes() {
-  return (int)(sizeof(__bf16) * ((size_t)32 * KROW + (size_t)DV * VROW));
+  return (int)(sizeof(__bf16) * ((size_t)32 * KROW + (size_t)VT));
 }
 
 // The call of sl_window_attention, for Dk == SL_DK, Dv == SL_DV and (vc == nullptr) == SL_VK.
@@ -481,8 +542,7 @@ extern "C" const char* sl_window_attention_mfma(
   const long long tiles = (cols + COLS - 1) / COLS;
   SL_CHECK(tiles * nsplit <= 1 << 30, "window attention: too many column tiles");
   const long long full = (long long)num_seqs * max_q_len;         // tokens if every sequence had as many as the longest
-  const int order = window > 0 || chunk > 0 ? IN_ORDER :
-                    num_tokens == full && tiles * nsplit <= 65535 ? BY_LENGTH :
+  const int order = num_tokens == full && tiles * nsplit <= 65535 ? BY_LENGTH :
                     4ll * num_tokens >= 3 * full ? BY_LENGTH_MOVED : LATE_FIRST;
   const unsigned items = (unsigned)(tiles * nsplit);
   const dim3 grid = order == BY_LENGTH ? dim3(nkv, num_seqs, items) : dim3(items, nkv, num_seqs);

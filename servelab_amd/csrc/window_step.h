@@ -67,23 +67,29 @@ struct StepColumn {
         slope2(a.slopes != nullptr ? a.slopes[head] * LOG2E : 0.f), m(-INFINITY), l(0.f), capped(a.softcap > 0.f), pos(pos_), lo(lo_),
         keep_first(a.keep_first) {}
 
-  __device__ __forceinline__ bool sees(int key) const { return key <= pos && (key >= lo || key < keep_first); }
+  __device__ __forceinline__ bool sees(int key) const { return (key <= pos) & ((key >= lo) | (key < keep_first)); }
   // weights of the lane's keys; returns what the sums before have to be multiplied by
   __device__ __forceinline__ float weights(f32x4 s0, f32x4 s1, int kbase, int gq, float (&p)[8]) {
     const float bias0 = -slope2 * (float)(pos - kbase - 8 * gq);
-    float s[8], top = -INFINITY;
+    float s[8], top = -INFINITY, factor = scale2;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] = j < 4 ? s0[j] : s1[j - 4];
+    if (capped) {
+      factor = cap2;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s[j] = tanhf(s[j] * uncap);
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float raw = j < 4 ? s0[j] : s1[j - 4];
-      s[j] = capped ? fmaf(tanhf(raw * uncap), cap2, fmaf(slope2, (float)j, bias0)) : fmaf(raw, scale2, fmaf(slope2, (float)j, bias0));
-      if (!sees(kbase + 8 * gq + j)) s[j] = -INFINITY;
+      s[j] = fmaf(s[j], factor, fmaf(slope2, (float)j, bias0));
+      s[j] = sees(kbase + 8 * gq + j) ? s[j] : -INFINITY;
       top = fmaxf(top, s[j]);
     }
-    const float mn = fmaxf(m, column_max4(top));
+    const float mn = fmaxf(m, column_max4(top)), from = mn == -INFINITY ? 0.f : mn;
     float psum = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      p[j] = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[j] - mn);
+      p[j] = __builtin_amdgcn_exp2f(s[j] - from);
       psum += p[j];
     }
     const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
@@ -96,7 +102,7 @@ struct StepColumn {
 // What a sequence's token sees: keys [0, keep) and [lo, pos].
 struct StepKeys {
   int pos, lo, keep;
-  __device__ __forceinline__ bool seen(int key) const { return key <= pos && (key >= lo || key < keep); }
+  __device__ __forceinline__ bool seen(int key) const { return (key <= pos) & ((key >= lo) | (key < keep)); }
   __device__ __forceinline__ int instead(int key, int kbase) const {  // the key, or one of the block that is seen
     key = min(key, pos);
     return key >= lo || key < keep ? key : (lo <= kbase + 31 ? lo : keep - 1);
@@ -249,11 +255,12 @@ __global__ __launch_bounds__(64 * STEP_WAVES) void window_step_kernel(const Wind
 #else
 // Values are channels of the key rows: a block is staged in LDS, as rows and turned, by the whole workgroup, whose wavefronts divide the
 // key channels of the scores among them (parts that meet in LDS) and the value channels of the weighted sum.
+constexpr int STEP_NT = cdiv((DV / 8) * 4, 256), STEP_NR = RCH ? cdiv(32 * RCH, 256) : 1;      // as NT, NR: for four wavefronts
 constexpr int STEP_DD = (DD + 3) / 4, STEP_KK = (KK + 3) / 4;          // channel tiles and key-channel steps a wavefront
 __global__ __launch_bounds__(256) void window_step_kernel(const WindowAttention a) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
   __bf16* ks = lds16;                                                  // [32][KROW]
-  __bf16* vt = ks + 32 * KROW;                                         // [DV][VROW]
+  __bf16* vt = ks + 32 * KROW;                                         // channel_row(d) of channel d
   __shared__ f32x4 scores[4][2][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, gq = lane >> 4;
   const int g = a.nh / a.nkv, tiles = (g + 15) / 16, seq = blockIdx.z, share = blockIdx.x;
@@ -275,7 +282,7 @@ __global__ __launch_bounds__(256) void window_step_kernel(const WindowAttention 
   f32x4 o[STEP_DD];
 #pragma unroll
   for (int i = 0; i < STEP_DD; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 treg[NT][8], rreg[NR];
+  bf16x8 treg[STEP_NT][8], rreg[STEP_NR];
   auto fetch = [&](int j) {
     const int kbase = (blocks.r + blocks.R * j) * 32;
     int pgA, pgB;
@@ -285,15 +292,15 @@ __global__ __launch_bounds__(256) void window_step_kernel(const WindowAttention 
       return a.kc + (((size_t)pg * a.nkv + kvh) * page + (key & (page - 1))) * DK;
     };
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int idx = min(tid + THREADS * i, (DV / 8) * 4 - 1), cb = idx / 4, kg = idx % 4;
+    for (int i = 0; i < STEP_NT; ++i) {
+      const int idx = min(tid + 256 * i, (DV / 8) * 4 - 1), cb = idx / 4, kg = idx % 4;
 #pragma unroll
       for (int e = 0; e < 8; ++e) treg[i][e] = *(const bf16x8*)(key_row(8 * kg + e) + 8 * cb);
     }
     if constexpr (RCH > 0) {
 #pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const int idx = min(tid + THREADS * i, 32 * RCH - 1);
+      for (int i = 0; i < STEP_NR; ++i) {
+        const int idx = min(tid + 256 * i, 32 * RCH - 1);
         rreg[i] = *(const bf16x8*)(key_row(idx / RCH) + 8 * (DV / 8 + idx % RCH));
       }
     }
@@ -304,37 +311,37 @@ __global__ __launch_bounds__(256) void window_step_kernel(const WindowAttention 
     const int kbase = (blocks.r + blocks.R * j) * 32, after = blocks.settle(j - 1);
     __syncthreads();                                                   // the last block's readers are done
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int idx = tid + THREADS * i, cb = idx / 4, kg = idx % 4;
+    for (int i = 0; i < STEP_NT; ++i) {
+      const int idx = tid + 256 * i, cb = idx / 4, kg = idx % 4;
       if (idx < (DV / 8) * 4) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) *(bf16x8*)(ks + (8 * kg + e) * KROW + 8 * cb) = treg[i][e];
+        for (int e = 0; e < 8; ++e) *(bf16x8*)(ks + staged_row(8 * kg + e) * KROW + 8 * cb) = treg[i][e];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           bf16x8 t;
 #pragma unroll
           for (int u = 0; u < 8; ++u) t[u] = treg[i][u][e];
-          *(bf16x8*)(vt + (8 * cb + e) * VROW + 8 * kg) = t;
+          *(bf16x8*)(vt + channel_row(8 * cb + e) + 8 * kg) = t;
         }
       }
     }
     if constexpr (RCH > 0) {
 #pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const int idx = tid + THREADS * i;
-        if (idx < 32 * RCH) *(bf16x8*)(ks + (idx / RCH) * KROW + 8 * (DV / 8 + idx % RCH)) = rreg[i];
+      for (int i = 0; i < STEP_NR; ++i) {
+        const int idx = tid + 256 * i;
+        if (idx < 32 * RCH) *(bf16x8*)(ks + staged_row(idx / RCH) * KROW + 8 * (DV / 8 + idx % RCH)) = rreg[i];
       }
     }
     __syncthreads();
     if (after >= 0) fetch(after);
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-    const __bf16* kp = ks + (8 * (n / 4) + n % 4) * KROW + 8 * gq;
+    const __bf16* kp = ks + n * KROW + 8 * gq;
 #pragma unroll
     for (int i = 0; i < STEP_KK; ++i) {
       const int kk = wave + 4 * i;
       if (kk >= KK) break;
       s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(kp + 32 * kk), qf[i], s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(kp + 4 * KROW + 32 * kk), qf[i], s1, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(kp + 16 * KROW + 32 * kk), qf[i], s1, 0, 0, 0);
     }
     scores[wave][0][lane] = s0;
     scores[wave][1][lane] = s1;
@@ -347,7 +354,7 @@ __global__ __launch_bounds__(256) void window_step_kernel(const WindowAttention 
     three_terms(p, p1, p2, p3);
 #pragma unroll
     for (int i = 0; i < STEP_DD; ++i) {
-      v[i] = *(const bf16x8*)(vt + (16 * min(wave * STEP_DD + i, DD - 1) + n) * VROW + 8 * gq);
+      v[i] = *(const bf16x8*)(vt + channel_row(16 * min(wave * STEP_DD + i, DD - 1) + n) + 8 * gq);
       o[i] *= alpha;
     }
 #pragma unroll
