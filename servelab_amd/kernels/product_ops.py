@@ -249,6 +249,8 @@ class ProductOps:
             # few-rows kernels stream W once per `limit` rows, 128 + 16 rows in 236 + 178 us).  Without:
             # those, several times faster than the plain tiled kernel below.
             if weight.w is not None:
+                if bias is not None and self._bias_tiles(M, N, K) and self._block_reads(x, weight):
+                    return self.linear_block(x, weight, bias, True, square=True)
                 sums = self.library_sums(x, weight.w, torch.float32)
                 return sums if bias is None else sums.add_(bias)
             return torch.cat([self.linear_skinny(x[i:i + limit], weight, bias, True)
@@ -477,6 +479,17 @@ class ProductOps:
             return None
         rows = self._tile_rows(M, N, K)
         return rows if 2e-6 * M * N * K >= self.PROMPT_MIN_TFLOPS * self._tiles_us(rows, M, N, K) else None
+
+    def _bias_tiles(self, M, N, K) -> bool:
+        """Whether a prompt's product with float32 results and a bias, which the library leaves to a second pass over
+        them, goes into the tiles: by their estimated rate, as in ``_prompt_tiles``.  us, library and pass / tiles: 6160 x
+        2048 at 1,000 / 2,048 rows 43 / 36 and 74 / 56, 7168 x 3584 at 1,500 / 1,852 85 / 72 and 98 / 91, 10304 x 2048 at 600 / 1,500 46 / 38
+        and 81 / 64; of 33 sizes the slowest 10792 x 3584 at 1,500, 123 / 130; below the rate 6160 x 2048 at 600 33 / 36, 4096 x 2048
+        at 1,000 29 / 34."""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 4
+                or not self.GATED_MIN_M <= M <= self.GATED_MAX_M or K > self.PROMPT_MAX_K):
+            return False
+        return 2e-6 * M * N * K >= self.PROMPT_MIN_TFLOPS * self._tiles_us(self._tile_rows(M, N, K), M, N, K)
 
     def _tuned_for(self, M, N, K) -> bool:
         """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside
