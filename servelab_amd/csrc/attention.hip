@@ -313,9 +313,17 @@ __global__ __launch_bounds__(64) void attention_few_keys_kernel(
   block now;
   if (b0 < b1) {
     now = load(b0);
-    for (int idx = lane; idx < GROUP_HEADS * HD; idx += 64)     // rows past nheads: zeros, results never stored
-      qs[idx / HD][idx % HD] = idx / HD < nheads
-          ? to_f(qkv[(size_t)t * row_stride + (size_t)(h0 + idx / HD) * HD + idx % HD]) : 0.f;
+    // (asked for together and without conditions: a value a trip, this was most of the kernel's time)
+    constexpr int NQ = GROUP_HEADS * HD / 64;
+    act_t q[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int h = (lane + 64 * i) / HD, d = (lane + 64 * i) % HD;
+      q[i] = qkv[(size_t)t * row_stride + (size_t)(h0 + (h < nheads ? h : nheads - 1)) * HD + d];
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)                                // (rows past nheads: the last again, results never stored)
+      qs[(lane + 64 * i) / HD][(lane + 64 * i) % HD] = to_f(q[i]);
   }
   __syncthreads();
   for (int b = b0; b < b1; ++b) {
@@ -568,7 +576,7 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float* ks = lds;                                     // [32][KR]
   float* vt = ks + 32 * KR;                            // [D][VR]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, gq = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, gq = lane >> 4;
   const int seq = blockIdx.z, kvh = blockIdx.y, g = nh / nkv;
   const int q0 = cu_q[seq], qlen = cu_q[seq + 1] - q0, ncols = qlen * g;
   // (tiles of late tokens see the most keys: they come first)
@@ -595,38 +603,50 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
   for (int j = 0; j < D / 16; ++j) o[j] = att_v4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   att_v4 kr[NP], vr[NP];
-  // Keys outside [kmin, kmax] are staged as zeros: a slot that holds no visible key, or a released page, may hold anything.
-  auto fetch = [&](int kbase) {
+  // A half of a block (16 keys, of one page) is read where it lies, its page asked for a block earlier, no load behind a condition (the
+  // compiler waits for a load where the two ways meet: eight loads a thread, each behind its page's, were sixteen trips to memory a
+  // block in turn).  A half of which no column sees a key may have no page: the other half stands for it.  Keys outside
+  // [kmin, kmax] get no weight, and their values are staged as zeros: a slot that holds no visible key may hold anything.
+  auto ask_pages = [&](int kbase) { return table[min(kbase + ((lane & 1) << 4), kmax) / page]; };
+  auto fetch = [&](int kbase, int asked) {
+    const int pgA = __builtin_amdgcn_readlane(asked, 0), pgB = __builtin_amdgcn_readlane(asked, 1);
+    const bool seenA = kbase + 15 >= kmin, seenB = kbase + 16 <= kmax;
+    const size_t headA = (size_t)(seenA ? pgA : pgB) * nkv + kvh, headB = (size_t)(seenB ? pgB : pgA) * nkv + kvh;
+    const int inA = (seenA ? kbase : kbase + 16) % page, inB = (seenB ? kbase + 16 : kbase) % page;
+    const float *keysA = kc + (headA * page + inA) * D, *keysB = kc + (headB * page + inB) * D;
+    const float *valuesA = vc + headA * D * page + inA, *valuesB = vc + headB * D * page + inB;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int idx = tid + 256 * i;
-      const int key = kbase + idx / (D / 4), d4 = idx % (D / 4);
-      kr[i] = att_v4{0.f, 0.f, 0.f, 0.f};
-      if (key >= kmin && key <= kmax)
-        kr[i] = *(const att_v4*)(kc + (((size_t)table[key / page] * nkv + kvh) * page + key % page) * D + 4 * d4);
-      const int d = idx / 8, key0 = kbase + 4 * (idx % 8);
-      vr[i] = att_v4{0.f, 0.f, 0.f, 0.f};
-      if (key0 + 3 >= kmin && key0 <= kmax) {          // (page sizes are multiples of 16: four keys share a page)
-        vr[i] = *(const att_v4*)(vc + (((size_t)table[key0 / page] * nkv + kvh) * D + d) * page + key0 % page);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (key0 + e < kmin || key0 + e > kmax) vr[i][e] = 0.f;
-      }
+      const int idx = tid + 256 * i, kl = idx / (D / 4) & 15, d4 = idx % (D / 4);
+      kr[i] = *(const att_v4*)((i >= NP / 2 ? keysB : keysA) + kl * D + 4 * d4);      // (the first NP / 2 pieces are 16 rows)
+      vr[i] = *(const att_v4*)((idx & 4 ? valuesB : valuesA) + (idx / 8) * page + 4 * (idx & 3));
     }
   };
   const int b0 = kmin / 32, b1 = kmax / 32;
-  fetch(32 * b0);
+  fetch(32 * b0, ask_pages(32 * b0));
+  int asked = b0 < b1 ? ask_pages(32 * b0 + 32) : 0;
   for (int b = b0; b <= b1; ++b) {
     const int kbase = 32 * b;
     __syncthreads();                                   // the last block's readers are done
+    const bool all_seen = kbase >= kmin && kbase + 31 <= kmax;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       const int idx = tid + 256 * i;
+      if (!all_seen) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = kbase + 4 * (idx % 8) + e;
+          vr[i][e] = (key >= kmin) & (key <= kmax) ? vr[i][e] : 0.f;
+        }
+      }
       *(att_v4*)(ks + (idx / (D / 4)) * KR + 4 * (idx % (D / 4))) = kr[i];
       *(att_v4*)(vt + (idx / 8) * VR + 4 * (idx % 8)) = vr[i];
     }
     __syncthreads();
-    if (b < b1) fetch(kbase + 32);
+    if (b < b1) {
+      fetch(kbase + 32, asked);
+      if (b + 1 < b1) asked = ask_pages(kbase + 64);
+    }
     if (!wave_live) continue;                          // (a wavefront without columns only helps staging)
     att_v4 s[2];
 #pragma unroll
@@ -647,7 +667,7 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = kbase + 16 * kt + 4 * gq + i;
-        s[kt][i] = key >= lo_c && key <= pos_c ? s[kt][i] * scale : -INFINITY;
+        s[kt][i] = (key >= lo_c) & (key <= pos_c) ? s[kt][i] * scale : -INFINITY;      // (no branches)
         top = fmaxf(top, s[kt][i]);
       }
     top = column_meet(top, max_f);
