@@ -556,35 +556,37 @@ __global__ __launch_bounds__(TILE_THREADS) void attention_general_tile_kernel(
 #if defined(SL_F32)
 // ---------------------------------------------------------------------------
 // Prompt portions in float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 factors and sums), for head sizes in
-// steps of 16 fixed at compile time.  A workgroup of four wavefronts owns 64 columns, (token, head of the group) pairs of
-// one sequence and one kv head, a wavefront 16 of them, and walks blocks of 32 keys, staged in LDS as K [32][D + 4] and
-// V^T [D][36]; the next block travels from the pages to registers meanwhile.  S^T = K Q^T, softmax with a running
+// steps of 16 fixed at compile time.  A workgroup owns 32 columns, (token, head of the group) pairs of one sequence and one kv
+// head, a wavefront 16 of them; two teams of two wavefronts walk every other block of 32 keys, staged in LDS as K [32][D + 4] and
+// V^T [D][36], and meet at the end; a team's next block travels from the pages to registers meanwhile.  S^T = K Q^T, softmax with a running
 // maximum per column, O^T += V^T P^T: a lane's scores of a 16 x 16 block (keys 4 (lane / 16) .. + 3 of column lane % 16) are the
-// second product's operand as they are.  What bounds it is the matrix instructions: 1.05 MFLOP a block and workgroup at
-// D 128, 0.6 TFLOP/s a CU.  One prompt of 333 tokens and two shorter ones, 12 heads on 2, D 128: 287 us with the FMA tiles,
-// 71 here.  The second product multiplies the zero weights of keys that a column does not see too, which an infinite or NaN
+// second product's operand as they are.  What bounds it is the matrix instructions of the longest tile: 128 a block and
+// wavefront at D 128, 1.7 us.  One prompt of 333 tokens and two shorter ones, 12 heads on 2, D 128: 287 us with the FMA tiles, 74 with
+// four wavefronts over 64 columns and loads behind conditions, 45 without those, 41 with two teams over 64 columns, 32 here.  The second product multiplies the zero weights of keys that a column does not see too, which an infinite or NaN
 // value turns into NaN: a wavefront with a result that is not finite takes its columns again key by key, over seen keys alone.
 // ---------------------------------------------------------------------------
 typedef float att_v4 __attribute__((ext_vector_type(4)));
 
+constexpr int F32_TEAMS = 2, F32_TEAM = 128, F32_COLS = 32;      // teams of two wavefronts, on the same 32 columns and every other block
 template <int D>
-__global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
+__global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kernel(
     const float* __restrict__ qkv, int row_stride, const float* __restrict__ kc, const float* __restrict__ vc,
     const int* __restrict__ block_tables, int max_pages, const int* __restrict__ cu_q, const int* __restrict__ positions,
     int nh, int nkv, int page, float scale, int window, float* __restrict__ out) {
-  constexpr int KR = D + 4, VR = 36, NP = D / 32;      // row lengths; 16-byte pieces of K and of V^T a thread stages of a block
+  constexpr int KR = D + 4, VR = 36, NP = 8 * D / F32_TEAM;      // row lengths; 16-byte pieces of K and of V^T a thread stages of a block
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* ks = lds;                                     // [32][KR]
+  const int team = __builtin_amdgcn_readfirstlane(threadIdx.x / F32_TEAM), tid = threadIdx.x % F32_TEAM;
+  float* ks = lds + team * (32 * KR + D * VR);         // [32][KR]
   float* vt = ks + 32 * KR;                            // [D][VR]
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, gq = lane >> 4;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, gq = lane >> 4;
   const int seq = blockIdx.z, kvh = blockIdx.y, g = nh / nkv;
   const int q0 = cu_q[seq], qlen = cu_q[seq + 1] - q0, ncols = qlen * g;
   // (tiles of late tokens see the most keys: they come first)
-  const int tile = (int)gridDim.x - 1 - (int)blockIdx.x, c0 = tile * 64;
+  const int tile = (int)gridDim.x - 1 - (int)blockIdx.x, c0 = tile * F32_COLS;
   if (c0 >= ncols) return;
   const int pos0 = positions[q0];
   const int* table = block_tables + (size_t)seq * max_pages;
-  const int c_last = min(c0 + 63, ncols - 1);
+  const int c_last = min(c0 + F32_COLS - 1, ncols - 1);
   const int kmax = pos0 + c_last / g;
   const int kmin = window > 0 ? max(0, pos0 + c0 / g - window + 1) : 0;
   const int cw = c0 + 16 * wave;
@@ -617,21 +619,25 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
     const float *valuesA = vc + headA * D * page + inA, *valuesB = vc + headB * D * page + inB;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int idx = tid + 256 * i, kl = idx / (D / 4) & 15, d4 = idx % (D / 4);
+      const int idx = tid + F32_TEAM * i, kl = idx / (D / 4) & 15, d4 = idx % (D / 4);
       kr[i] = *(const att_v4*)((i >= NP / 2 ? keysB : keysA) + kl * D + 4 * d4);      // (the first NP / 2 pieces are 16 rows)
       vr[i] = *(const att_v4*)((idx & 4 ? valuesB : valuesA) + (idx / 8) * page + 4 * (idx & 3));
     }
   };
   const int b0 = kmin / 32, b1 = kmax / 32;
-  fetch(32 * b0, ask_pages(32 * b0));
-  int asked = b0 < b1 ? ask_pages(32 * b0 + 32) : 0;
-  for (int b = b0; b <= b1; ++b) {
+  const int mine = b0 + team;
+  int asked = 0;
+  if (mine <= b1) {
+    fetch(32 * mine, ask_pages(32 * mine));
+    if (mine + F32_TEAMS <= b1) asked = ask_pages(32 * (mine + F32_TEAMS));
+  }
+  for (int b = mine; b - team <= b1; b += F32_TEAMS) {   // (as many rounds for both teams; the second may have no block in the last)
     const int kbase = 32 * b;
     __syncthreads();                                   // the last block's readers are done
     const bool all_seen = kbase >= kmin && kbase + 31 <= kmax;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int idx = tid + 256 * i;
+      const int idx = tid + F32_TEAM * i;
       if (!all_seen) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -643,11 +649,11 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
       *(att_v4*)(vt + (idx / 8) * VR + 4 * (idx % 8)) = vr[i];
     }
     __syncthreads();
-    if (b < b1) {
-      fetch(kbase + 32, asked);
-      if (b + 1 < b1) asked = ask_pages(kbase + 64);
+    if (b + F32_TEAMS <= b1) {
+      fetch(kbase + 32 * F32_TEAMS, asked);
+      if (b + 2 * F32_TEAMS <= b1) asked = ask_pages(kbase + 64 * F32_TEAMS);
     }
-    if (!wave_live) continue;                          // (a wavefront without columns only helps staging)
+    if (!wave_live || b > b1) continue;                          // (a wavefront without columns only helps staging)
     att_v4 s[2];
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
@@ -696,6 +702,29 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[dd][i] = fmaf(o[dd][i], alpha, acc[i]);
     }
+  }
+  // the first team takes what the second has of its columns
+  att_v4* os = (att_v4*)lds;                           // [D / 16][F32_TEAM]
+  float2* ml = (float2*)(os + F32_TEAM * (D / 16));
+  __syncthreads();
+  if (team == 1) {
+#pragma unroll
+    for (int dd = 0; dd < D / 16; ++dd) os[F32_TEAM * dd + tid] = o[dd];
+    ml[tid] = make_float2(m, l);
+  }
+  __syncthreads();
+  if (team == 1) return;
+  {
+    const float2 other = ml[tid];
+    const float both = fmaxf(m, other.x), ours = m == -INFINITY ? 0.f : expf(m - both), theirs = other.x == -INFINITY ? 0.f : expf(other.x - both);
+#pragma unroll
+    for (int dd = 0; dd < D / 16; ++dd) {
+      const att_v4 x = os[F32_TEAM * dd + tid];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[dd][i] = fmaf(x[i], theirs, o[dd][i] * ours);
+    }
+    l = fmaf(other.y, theirs, l * ours);
+    m = both;
   }
   l = column_meet(l, add_f);
   float odd = 0.f;                                     // (0, or NaN where a result is not finite)
@@ -759,12 +788,17 @@ extern "C" const char* sl_attention_general_tiles(
   // (head sizes of the shapes served; from 32 columns on a tile of 64 is filled well enough to win at every length measured)
   if ((D == 64 || D == 128) && cols >= 32 && row_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)kc % 16 == 0 &&
       (uintptr_t)vc % 16 == 0 && (uintptr_t)out % 16 == 0) {
-    const dim3 wide((unsigned)((cols + 63) / 64), nkv, num_seqs);
-    const size_t room = sizeof(float) * ((size_t)32 * (D + 4) + (size_t)D * 36);
+    const dim3 wide((unsigned)((cols + F32_COLS - 1) / F32_COLS), nkv, num_seqs);
+    const size_t room = F32_TEAMS * sizeof(float) * ((size_t)32 * (D + 4) + (size_t)D * 36);
     auto run = [&](auto kernel) {
-      kernel<<<wide, 256, room, stream>>>((const float*)qkv, row_stride, (const float*)kc, (const float*)vc, block_tables,
+      kernel<<<wide, F32_TEAM * F32_TEAMS, room, stream>>>((const float*)qkv, row_stride, (const float*)kc, (const float*)vc, block_tables,
                                           max_pages, cu_q, positions, nh, nkv, page, scale, window, (float*)out);
     };
+    auto grow = [&](const void* kernel) {
+      return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)room);
+    };
+    const hipError_t e = room <= 48 * 1024 ? hipSuccess : grow(D == 64 ? (const void*)attention_f32_mfma_kernel<64> : (const void*)attention_f32_mfma_kernel<128>);
+    if (e != hipSuccess) return hipGetErrorString(e);
     if (D == 64) run(attention_f32_mfma_kernel<64>);
     else run(attention_f32_mfma_kernel<128>);
     return sl_launch_status();
