@@ -62,7 +62,7 @@ __device__ __forceinline__ float add_f(float a, float b) { return a + b; }
 __device__ __forceinline__ float max_f(float a, float b) { return fmaxf(a, b); }
 
 // Over a wavefront whose lanes are all active, pairs 32, 16, 8, 4, 2, 1 apart in turn; every lane gets the result.  Six exchanges
-// through the LDS's crossbar stood here, in a row: most of the time of a kernel of a few rows is such chains.  (RATES)
+// through the LDS's crossbar stood here, in a row: most of the time of a kernel of a few rows is such chains.
 template <class Op> __device__ __forceinline__ float wave_meet(float v, Op op) {
   v = rows_meet<32>(v, op);
   v = rows_meet<16>(v, op);

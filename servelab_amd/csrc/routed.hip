@@ -126,7 +126,56 @@ __device__ __forceinline__ int route_token(const Route& r, size_t t, int lane) {
   return mine_e;
 }
 
-__global__ __launch_bounds__(64) void route_kernel(const Route r) { route_token(r, blockIdx.x, threadIdx.x); }
+// The same for up to 64 experts: a lane has one, and what is compared stays in its register.
+__device__ __forceinline__ int route_token_64(const Route& r, size_t t, int lane) {
+  const int E = r.E, top = r.top;
+  const bool there = lane < E;
+  const float raw = r.logits[t * r.stride + (there ? lane : 0)], add = r.correction != nullptr ? r.correction[there ? lane : 0] : 0.f;
+  float share = 0.f, number = raw;
+  if (r.over_all) {
+    const float zmax = wave_max(there ? raw : -INFINITY);
+    share = there ? expf(raw - zmax) : 0.f;
+    share *= 1.f / wave_sum(share);
+    number = share + add;
+  }
+  number = number == number ? number : -INFINITY;
+  unsigned long long left = __ballot(there);
+  float mine = 0.f;
+  int mine_e = 0;
+  for (int k = 0; k < top; ++k) {
+    const bool in = left >> lane & 1;
+    const float most = wave_max(in ? number : -INFINITY);
+    const int at = __ffsll(__ballot(in && number == most)) - 1;      // (the lowest index among equals)
+    left &= ~(1ull << at);
+    // (a chosen expert's logit, or its share of all; NaN stays what it is)
+    const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.over_all ? share : raw), at));
+    if (lane == k) {
+      mine = v;
+      mine_e = at;
+    }
+  }
+  float w;
+  if (r.over_all) {
+    w = lane < top ? mine : 0.f;
+    w = w / (wave_sum(w) + 1e-20f) * r.scale;
+  } else if (r.sigmoid) {
+    w = 1.f / (1.f + expf(-mine));
+  } else {
+    const float top1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mine)));
+    w = lane < top ? expf(mine - top1) : 0.f;
+    w = w / wave_sum(w);
+  }
+  if (lane < top) {
+    r.chosen[t * top + lane] = mine_e;
+    r.shares[t * top + lane] = w;
+  }
+  return mine_e;
+}
+
+__global__ __launch_bounds__(64) void route_kernel(const Route r) {
+  if (r.E <= 64) route_token_64(r, blockIdx.x, threadIdx.x);
+  else route_token(r, blockIdx.x, threadIdx.x);
+}
 
 // ------------------------------------------------------------------ group
 // One workgroup sorts the n = tokens * top pairs by expert (counting sort in LDS: 3 E numbers at `sh`).
@@ -197,12 +246,14 @@ __global__ __launch_bounds__(1024) void group_kernel(const int* __restrict__ cho
 }
 
 // Both for a step of up to 16 tokens, a wavefront each: the work is a few microseconds of one workgroup, and a second
-// launch costs as much again (2 tokens, 64 experts, 8 choices: 7.5 + 8.3 us in two kernels, 7.2 here).
+// launch costs as much again (2 tokens, 64 experts, 8 choices: 7.5 + 8.3 us in two kernels; 6.2 here with four experts a lane in a loop
+// over all of them, 3.2 with an expert's number in its lane's register).  Pairs placed by looking at all the others, in place of the
+// counters of the sort, took 4.2, and 32 pairs 5.4 against 3.4.
 __global__ __launch_bounds__(1024) void route_group_kernel(const Route r, const Group g) {
   extern __shared__ int sh[];
   int* chosen = sh + 3 * g.E;    // [n]
   const int wave = threadIdx.x / 64, lane = threadIdx.x & 63;
-  const int e = route_token(r, wave, lane);
+  const int e = r.E <= 64 ? route_token_64(r, wave, lane) : route_token(r, wave, lane);
   if (lane < r.top) chosen[wave * r.top + lane] = e;
   __syncthreads();
   group_pairs(g, chosen, sh);
