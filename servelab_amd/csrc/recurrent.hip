@@ -55,6 +55,7 @@ __global__ __launch_bounds__(256) void lowrank_expand_kernel(const float* __rest
   float z[LOW_TOKENS];
 #pragma unroll
   for (int tt = 0; tt < LOW_TOKENS; ++tt) z[tt] = 0.f;
+#pragma unroll 8
   for (int r = 0; r < rank; ++r) {
     const float wr = w[r];
 #pragma unroll
@@ -187,11 +188,20 @@ template <int N>
 __device__ __forceinline__ float conv_channel_taps(const ShortConv& a, int first, int i, bool fresh, float* past, int c) {
   float x[N], w[N];
 #pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int idx = i - (N - 1) + j;
-    w[j] = a.w[(size_t)c * N + j];
-    if (idx >= 0) x[j] = a.buf[(size_t)(first + idx) * a.stride + a.col + c];
-    else x[j] = fresh ? 0.f : past[(size_t)(N - 1 + idx) * a.C + c];
+  for (int j = 0; j < N; ++j) w[j] = a.w[(size_t)c * N + j];
+  if (a.shift) {                             // (one token: which inputs lie where is known, and no load stands behind a condition)
+#pragma unroll
+    for (int j = 0; j < N - 1; ++j) x[j] = past[(size_t)j * a.C + c];
+    x[N - 1] = a.buf[(size_t)first * a.stride + a.col + c];
+#pragma unroll
+    for (int j = 0; j < N - 1; ++j) x[j] = fresh ? 0.f : x[j];
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int idx = i - (N - 1) + j;
+      if (idx >= 0) x[j] = a.buf[(size_t)(first + idx) * a.stride + a.col + c];
+      else x[j] = fresh ? 0.f : past[(size_t)(N - 1 + idx) * a.C + c];
+    }
   }
   float acc = a.bias != nullptr ? a.bias[c] : 0.f;
 #pragma unroll
@@ -230,13 +240,46 @@ __global__ __launch_bounds__(64) void short_conv_kernel(const ShortConv a) {
     c0 = a.unit_heads * a.unit_dim + (b - a.unit_heads) * 256;
     n = min(256, a.C - c0);
   }
-  const int s = a.tok_seq[t];
-  const int first = a.cu_q[s];
+  const int s = a.shift ? t : a.tok_seq[t];                 // (a token a sequence: two trips to memory fewer)
+  const int first = a.shift ? t : a.cu_q[s];
   const int i = t - first;                                  // place of the token in its step
   const bool fresh = a.positions[first] == 0;               // the sequence starts in this step
   float* past = a.state + (size_t)a.slots[s] * a.state_stride + a.state_off;
   float ss = 0.f;
   float y[4];
+  if (a.shift && a.taps == 4) {
+    // (a token each: the slot's new inputs are written behind the loads of all four channels, or a channel would wait for the one before:
+    // one request's 8,192 channels 3.8 us, now 2.5)
+    float past_x[4][3], own[4], w[4][4], add[4];
+    int at[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = at[u] = c0 + min(lane + u * 64, n - 1);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) past_x[u][j] = past[(size_t)j * a.C + c];
+      own[u] = a.buf[(size_t)first * a.stride + a.col + c];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[u][j] = a.w[(size_t)c * 4 + j];
+      add[u] = a.bias != nullptr ? a.bias[c] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float acc = add[u];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        past_x[u][j] = fresh ? 0.f : past_x[u][j];
+        acc += w[u][j] * past_x[u][j];
+      }
+      acc += w[u][3] * own[u];
+      y[u] = a.silu ? acc * sigmoidf_(acc) : acc;
+      if (lane + u * 64 < n) {
+        ss += y[u] * y[u];
+        past[at[u]] = past_x[u][1];
+        past[(size_t)a.C + at[u]] = past_x[u][2];
+        past[2 * (size_t)a.C + at[u]] = own[u];
+      }
+    }
+  } else
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int c = c0 + lane + u * 64;
@@ -363,7 +406,7 @@ __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid,
   const int t = blockIdx.x, H = a.C, back = a.taps - 1;
   float* x = resid + (size_t)t * H;
   const act_t* yr = y != nullptr ? y + (size_t)t * H : nullptr;
-  const int s = a.tok_seq[t];
+  const int s = t;                                     // (a token a sequence)
   const bool fresh = a.positions[t] == 0;
   float* keep_in = a.state + (size_t)a.slots[s] * a.state_stride + a.state_off;
   float v, yv = 0.f, gain = 0.f, w_own;
@@ -1090,6 +1133,9 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
 // One wavefront per (token, head): o / sqrt(mean(o^2) + eps) * w * act(gate); act 0: sigmoid, 1: silu;
 // no gate (nullptr): the norm alone.
 // gate_first: the gate comes before the norm, x = o * act(gate), then x / sqrt(mean(x^2) + eps) * w.
+// N > 0: heads of up to 64 N channels, everything asked for at once (a head of 256 / 512 channels took as many trips to memory twice:
+// one request of 8 heads of 256 3.0 us, now 1.9, two of 512 5.3, now 2.5); 0: wider ones.
+template <int N>
 __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restrict__ o, int H, int Dv,
                                                             const float* __restrict__ w, int per_head, float eps,
                                                             const float* __restrict__ gate, int gate_stride,
@@ -1101,6 +1147,30 @@ __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restr
   const float* gr = gate != nullptr ? gate + t * gate_stride + gate_col + h * Dv : nullptr;
   const float* wr = w + (per_head ? h * Dv : 0);
   float ss = 0.f;
+  if constexpr (N > 0) {
+    const float* zr = gr != nullptr ? gr : x;
+    float v[N], z[N], g[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int d = min(lane + 64 * u, Dv - 1);
+      v[u] = x[d];
+      z[u] = zr[d];
+      g[u] = wr[d];
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      z[u] = act == 0 ? sigmoidf_(z[u]) : z[u] * sigmoidf_(z[u]);
+      if (gate_first && gr != nullptr) v[u] *= z[u];
+      ss += lane + 64 * u < Dv ? v[u] * v[u] : 0.f;
+    }
+    const float inv = 1.f / sqrtf(wave_sum(ss) / (float)Dv + eps);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const float r = v[u] * inv * g[u];
+      if (lane + 64 * u < Dv) out[(t * H + h) * Dv + lane + 64 * u] = from_f<act_t>(gr != nullptr && !gate_first ? r * z[u] : r);
+    }
+    return;
+  }
   for (int d = lane; d < Dv; d += 64) {
     float v = x[d];
     if (gate_first && gr != nullptr) {
@@ -1128,8 +1198,14 @@ extern "C" const char* sl_head_norm_gate(const float* o, int T, int H, int Dv, c
   SL_CHECK(gate == nullptr || (gate_col >= 0 && gate_col + H * Dv <= gate_stride), "head_norm_gate: the gates do not fit their rows");
   SL_CHECK(act == 0 || act == 1, "head_norm_gate: the gate is sigmoid (0) or silu (1)");
   if (T == 0) return nullptr;
-  head_norm_gate_kernel<<<dim3(T, H), 64, 0, stream>>>(o, H, Dv, w, per_head, eps, gate, gate_stride, gate_col,
-                                                       act, gate_first, (act_t*)out);
+  auto run = [&](auto kernel) {
+    kernel<<<dim3(T, H), 64, 0, stream>>>(o, H, Dv, w, per_head, eps, gate, gate_stride, gate_col, act, gate_first, (act_t*)out);
+  };
+  if (Dv <= 64) run(head_norm_gate_kernel<1>);
+  else if (Dv <= 128) run(head_norm_gate_kernel<2>);
+  else if (Dv <= 256) run(head_norm_gate_kernel<4>);
+  else if (Dv <= 512) run(head_norm_gate_kernel<8>);
+  else run(head_norm_gate_kernel<0>);
   return sl_launch_status();
 }
 
@@ -1156,8 +1232,8 @@ __global__ void projnorm_rope_store_kernel(const float* __restrict__ buf, int st
   const size_t t = blockIdx.x;
   const float* row = buf + t * stride;
   if (cv.w != nullptr) {
-    const int s = cv.tok_seq[t];
-    const int first = cv.cu_q[s];
+    const int s = cv.shift ? (int)t : cv.tok_seq[t];
+    const int first = cv.shift ? (int)t : cv.cu_q[s];
     const int i = (int)t - first;
     const bool fresh = cv.positions[first] == 0;
     float* past = cv.state + (size_t)cv.slots[s] * cv.state_stride + cv.state_off;
@@ -1200,6 +1276,123 @@ __global__ void projnorm_rope_store_kernel(const float* __restrict__ buf, int st
   if (slots != nullptr)
     for (int e = threadIdx.x; e < nv; e += blockDim.x)
       vc[((pg * G + e / Dv) * Dv + e % Dv) * page + off] = from_f<act_t>(row[v_col + e]);
+}
+
+// The same for a step of few tokens and rows of at most 4,096 values of q and k and 1,024 of v: what a thread needs is asked for before the
+// first sum (its four values of the row, their gains and their partners', angles, its value of v), and both sums meet at once.  One
+// token, 16 heads on 2 of 128: 4.9 us, now 4.3; behind a convolution of four taps 8.4, now 5.3.
+template <bool CONV>
+__global__ __launch_bounds__(1024) void projnorm_step_kernel(const float* __restrict__ buf, int stride, int H, int G, int D, int Dv,
+                                                             const float* __restrict__ qw, const float* __restrict__ kw, float eps,
+                                                             int rot, const float* __restrict__ cosv, const float* __restrict__ sinv,
+                                                             const int* __restrict__ slots, act_t* __restrict__ kc,
+                                                             act_t* __restrict__ vc, int page, act_t* __restrict__ q_out,
+                                                             int v_col, int lg_D, int lg_Dv, int lg_page, const ShortConv cv) {
+  // (a division by a number of the call is 40 instructions, and ten of them stood here: shifts where the sizes are powers of two)
+  auto over_D = [&](int e) { return lg_D >= 0 ? e >> lg_D : e / D; };
+  __shared__ float of_q[16], of_k[16];
+  extern __shared__ float xs[];              // [nq + nk], or all convolved channels
+  const size_t t = blockIdx.x;
+  const int tid = threadIdx.x, nq = H * D, nqk = nq + G * D, nv = G * Dv, half = rot / 2;
+  const float* row = buf + t * stride;
+  const bool normed = qw != nullptr;
+  const float *gq = normed ? qw : row, *gk = normed && nqk > nq ? kw : gq;
+  float x[4], w[4], wp[4], cs[4], sn[4], v = 0.f;
+  auto gain = [&](int e) { return (e < nq ? gq : gk - nq)[e]; };
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = min(tid + 1024 * u, nqk - 1), d = e - over_D(e) * D;
+    if (!CONV) x[u] = row[e];
+    w[u] = gain(e);
+    cs[u] = 1.f;
+    sn[u] = 0.f;
+    wp[u] = w[u];
+    if (rot > 0) {
+      const int i = d < half ? d : d < rot ? d - half : 0;
+      cs[u] = cosv[t * half + i];
+      sn[u] = sinv[t * half + i];
+      wp[u] = gain(d < half ? e + half : d < rot ? e - half : e);
+    }
+  }
+  if (!CONV && nv > 0) v = row[v_col + min(tid, nv - 1)];
+  const int slot = slots != nullptr ? slots[t] : 0;
+  if constexpr (CONV) {
+    const int s = cv.shift ? (int)t : cv.tok_seq[t], first = cv.shift ? (int)t : cv.cu_q[s];
+    const bool fresh = cv.positions[first] == 0;
+    float* past = cv.state + (size_t)cv.slots[s] * cv.state_stride + cv.state_off;
+    if (cv.shift && cv.taps == 4 && cv.C <= 4096) {                    // (as in short_conv_kernel)
+      float px[4][3], own[4], cw[4][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = min(tid + 1024 * u, cv.C - 1);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) px[u][j] = past[(size_t)j * cv.C + c];
+        own[u] = row[c];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cw[u][j] = cv.w[(size_t)c * 4 + j];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = tid + 1024 * u;
+        if (c >= cv.C) break;
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          px[u][j] = fresh ? 0.f : px[u][j];
+          acc += cw[u][j] * px[u][j];
+        }
+        xs[c] = acc + cw[u][3] * own[u];
+        past[c] = px[u][1];
+        past[(size_t)cv.C + c] = px[u][2];
+        past[2 * (size_t)cv.C + c] = own[u];
+      }
+    } else {
+      for (int c = tid; c < cv.C; c += 1024) xs[c] = conv_channel(cv, first, (int)t - first, fresh, past, c);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = xs[min(tid + 1024 * u, nqk - 1)];
+    if (nv > 0) v = xs[v_col + min(tid, nv - 1)];
+  }
+  float sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = tid + 1024 * u;
+    if (!CONV && e < nqk) xs[e] = x[u];
+    sq += e < nq ? x[u] * x[u] : 0.f;
+    sk += e >= nq && e < nqk ? x[u] * x[u] : 0.f;
+  }
+  sq = wave_sum(sq);
+  sk = wave_sum(sk);
+  if (tid % 64 == 0) {
+    of_q[tid / 64] = sq;
+    of_k[tid / 64] = sk;
+  }
+  __syncthreads();
+  sq = sk = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    sq += of_q[i];
+    sk += of_k[i];
+  }
+  const float iq = normed ? 1.f / sqrtf(sq / (float)nq + eps) : 1.f, ik = normed ? 1.f / sqrtf(sk / (float)max(1, nqk - nq) + eps) : 1.f;
+  const int pg_int = lg_page >= 0 ? slot >> lg_page : slot / page, off = slot - pg_int * page;
+  const size_t pg = pg_int;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = tid + 1024 * u, d = e - over_D(e) * D;
+    if (e >= nqk) break;
+    const float inv = e < nq ? iq : ik;
+    float r = normed ? x[u] * inv * w[u] : x[u];
+    if (d < rot) {
+      const float other = xs[d < half ? e + half : e - half], o = normed ? other * inv * wp[u] : other;
+      r = d < half ? r * cs[u] - o * sn[u] : r * cs[u] + o * sn[u];
+    }
+    if (e < nq) q_out[t * nq + e] = from_f<act_t>(r);
+    else if (slots != nullptr) kc[((pg * G + over_D(e - nq)) * page + off) * D + d] = from_f<act_t>(r);
+  }
+  const int vh = lg_Dv >= 0 ? tid >> lg_Dv : tid / Dv;
+  if (slots != nullptr && tid < nv) vc[((pg * G + vh) * Dv + tid - vh * Dv) * page + off] = from_f<act_t>(v);
 }
 
 // The same without a norm over the projection, where nothing ties a token's heads together (no norm, or
@@ -1320,7 +1513,16 @@ extern "C" const char* sl_projnorm_rope_store(const float* buf, int stride, int 
                                                                    (act_t*)kc, (act_t*)vc, page, (act_t*)q_out, v_col, cv);
   else {   // (a step of few tokens has few blocks: wider ones shorten each block's loops over the row)
     cv.shift = taps_w != nullptr && write_state && taps > 1 && S == T;
-    projnorm_rope_store_kernel<<<T, T <= 64 ? 1024 : 256, lds, stream>>>(buf, stride, H, G, D, Dv, qw, kw, eps, rot, cosv, sinv, slots,
+    const long long nqk = (long long)(H + G) * D;
+    auto lg = [](int n) { return n & (n - 1) ? -1 : __builtin_ctz(n); };
+    auto step = [&](auto kernel, size_t room) {
+      kernel<<<T, 1024, room, stream>>>(buf, stride, H, G, D, Dv, qw, kw, eps, rot, cosv, sinv, slots, (act_t*)kc, (act_t*)vc, page,
+                                        (act_t*)q_out, v_col, lg(D), lg(Dv), lg(page), cv);
+    };
+    if (T <= 64 && nqk <= 4096 && (long long)G * Dv <= 1024) {
+      if (taps_w != nullptr) step(projnorm_step_kernel<true>, lds);
+      else step(projnorm_step_kernel<false>, nqk * sizeof(float));
+    } else projnorm_rope_store_kernel<<<T, T <= 64 ? 1024 : 256, lds, stream>>>(buf, stride, H, G, D, Dv, qw, kw, eps, rot, cosv, sinv, slots,
                                                         (act_t*)kc, (act_t*)vc, page, (act_t*)q_out, v_col, cv);
   }
   if (taps_w != nullptr && write_state && taps > 1 && !cv.shift)
