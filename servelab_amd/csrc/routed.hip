@@ -905,6 +905,52 @@ __global__ __launch_bounds__(256) void routed_combine_kernel(const float* __rest
   out[t * H + c] = from_f<act_t>(v);
 }
 
+// The same, four channels a thread with 16-byte loads, eight choices' rows asked for at once: rows of a multiple of four values and
+// aligned operands.  2,048 tokens of 8 choices, 2,048 channels, 150 MB: 39 us with a channel a thread, 26 here.
+struct __attribute__((aligned(16))) rc_f4 { float v[4]; };
+struct __attribute__((aligned(4 * sizeof(act_t)))) rc_a4 { act_t v[4]; };
+template <bool THROUGH>
+__global__ __launch_bounds__(256) void routed_combine_vec_kernel(const float* __restrict__ y, const int* __restrict__ place_of,
+                                                                 const float* __restrict__ shares, int top,
+                                                                 const act_t* __restrict__ base, const float* __restrict__ base_gate,
+                                                                 int gate_stride, int H, act_t* __restrict__ out,
+                                                                 const int* __restrict__ chosen, int E_real,
+                                                                 const act_t* __restrict__ x) {
+  const size_t t = blockIdx.x;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  if (c >= H) return;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  if (base != nullptr) {
+    const rc_a4 b = *(const rc_a4*)(base + t * H + c);
+    const float g = base_gate != nullptr ? 1.f / (1.f + expf(-base_gate[t * gate_stride])) : 1.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = base_gate != nullptr ? to_f(b.v[j]) * g : to_f(b.v[j]);
+  }
+  for (int k0 = 0; k0 < top; k0 += 8) {
+    rc_f4 r[8];
+    float share[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = min(k0 + u, top - 1);                                               // (the same for the whole workgroup)
+      share[u] = shares != nullptr ? shares[t * top + k] : 1.f;
+      if (THROUGH && chosen[t * top + k] >= E_real) {
+        const rc_a4 a = *(const rc_a4*)(x + t * H + c);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[u].v[j] = to_f(a.v[j]);
+      } else r[u] = *(const rc_f4*)(y + (size_t)place_of[t * top + k] * H + c);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k0 + u < top)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += share[u] * r[u].v[j];
+  }
+  rc_a4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o.v[j] = from_f<act_t>(v[j]);
+  *(rc_a4*)(out + t * H + c) = o;
+}
+
 extern "C" const char* sl_routed_combine(const float* y, const int* place_of, const float* shares, int T, int top,
                                          const void* base, const float* base_gate, int gate_stride, int H,
                                          void* out, const int* chosen, int E_real, const void* x,
@@ -912,6 +958,16 @@ extern "C" const char* sl_routed_combine(const float* y, const int* place_of, co
   SL_CHECK(T >= 0 && top >= 1 && top <= 64 && H > 0, "routed_combine: sizes must be positive, at most 64 choices");
   SL_CHECK(chosen == nullptr || x != nullptr, "routed_combine: experts that hand their input through need the input");
   if (T == 0) return nullptr;
+  if (H % 4 == 0 && (uintptr_t)y % 16 == 0 && ((uintptr_t)base | (uintptr_t)out | (uintptr_t)x) % sizeof(rc_a4) == 0) {
+    const int n = H >= 1024 ? 256 : (H / 4 + 63) / 64 * 64;
+    auto run = [&](auto kernel) {
+      kernel<<<dim3(T, (H / 4 + n - 1) / n), n, 0, stream>>>(y, place_of, shares, top, (const act_t*)base, base_gate, gate_stride, H,
+                                                             (act_t*)out, chosen, E_real, (const act_t*)x);
+    };
+    if (chosen != nullptr) run(routed_combine_vec_kernel<true>);
+    else run(routed_combine_vec_kernel<false>);
+    return sl_launch_status();
+  }
   routed_combine_kernel<<<dim3(T, (H + 255) / 256), 256, 0, stream>>>(y, place_of, shares, top, (const act_t*)base,
                                                                     base_gate, gate_stride, H, (act_t*)out,
                                                                     chosen, E_real, (const act_t*)x);
