@@ -102,9 +102,8 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  float t = 0.f;
-  for (int i = 0; i < nwaves; ++i) t += scratch[i];
-  return t;
+  const float part = scratch[lane & 15];               // (a lane a wavefront's sum: added up in a row they wait for one another)
+  return row_meet((lane & 15) < nwaves ? part : 0.f, add_f);
 }
 
 // Activations by number, as the calls of the kernel table pass them: 1 silu, 2 relu, 3 relu squared,

@@ -67,8 +67,12 @@ struct __attribute__((aligned(16))) a4 { act_t v[4]; };
 struct __attribute__((aligned(8))) a4 { act_t v[4]; };
 #endif
 
-template <int ITERS>
-__global__ void add_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ delta,
+// A step of few rows is one trip to memory and one sum, so all that a row needs is asked for at once, PARTS partial sums a trip (0: there are
+// none), and no load stands behind a condition, which would be waited for where the ways meet (an absent delta is read from the stream
+// and left out); the stream's new row is written behind the sum.  64 rows of 3,584 values
+// with eight partial sums: 5.2 us with the loads in turn, 4.9 here, 2,048 with two: 23.0, now 22.5.
+template <int ITERS, int PARTS>
+__global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ delta,
                                        const SplitDelta sd, const int* __restrict__ rows,
                                        const float* __restrict__ w, act_t* __restrict__ out, int H,
                                        float eps) {
@@ -76,53 +80,83 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* _
   const int r = blockIdx.x;
   const size_t src = rows != nullptr ? (size_t)rows[r] : (size_t)r;
   float* x = resid + src * H;
-  const act_t* d = delta != nullptr ? delta + src * H : nullptr;
-  const float* p = sd.parts != nullptr ? sd.parts + src * H : nullptr;
+  const bool plain = delta != nullptr;
+  const act_t* d = plain ? delta + src * H : (const act_t*)x;
+  const float* p = sd.parts + src * H;
   const int H4 = H / 4;
-  f4 v[ITERS];
-  float ss = 0.f;
+  f4 v[ITERS], wv[ITERS], pv[PARTS > 0 ? PARTS : 1][ITERS];
+  a4 dv[ITERS];
+  auto group = [&](int it) { return min((int)(threadIdx.x + it * blockDim.x), H4 - 1); };
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int i = threadIdx.x + it * blockDim.x;
-    if (i < H4) {
-      v[it] = ((const f4*)x)[i];
-      if (d != nullptr) {
-        const a4 dv = ((const a4*)d)[i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[it].v[j] += to_f(dv.v[j]);
-      }
-      if (p != nullptr) {
-#pragma unroll 4
-        for (int q = 0; q < sd.nparts; ++q) {
-          const f4 pv = ((const f4*)(p + q * sd.stride))[i];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[it].v[j] += pv.v[j];
-        }
-        if (sd.bias != nullptr) {
-          const f4 bv = ((const f4*)sd.bias)[i];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[it].v[j] += bv.v[j];
-        }
-      }
-      if ((d != nullptr || p != nullptr) && rows == nullptr) ((f4*)x)[i] = v[it];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) ss += v[it].v[j] * v[it].v[j];
-    }
+    v[it] = ((const f4*)x)[group(it)];
+    if (PARTS == 0) dv[it] = ((const a4*)d)[group(it)];
+    wv[it] = ((const f4*)w)[group(it)];
   }
+  auto ask = [&](int q0) {
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q)
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) pv[q][it] = ((const f4*)(p + min(q0 + q, sd.nparts - 1) * sd.stride))[group(it)];
+  };
+  auto add = [&](int q0) {
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q)
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[it].v[j] += q0 + q < sd.nparts ? pv[q][it].v[j] : 0.f;
+  };
+  ask(0);
+  if (PARTS > 0 && plain)                              // (rare beside partial sums, as a bias is)
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) dv[it] = ((const a4*)d)[group(it)];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[it].v[j] += plain ? to_f(dv[it].v[j]) : 0.f;
+  add(0);
+  if (PARTS > 0) {
+    for (int q0 = PARTS; q0 < sd.nparts; q0 += PARTS) {
+      ask(q0);
+      add(q0);
+    }
+    if (sd.bias != nullptr)
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const f4 bv = ((const f4*)sd.bias)[group(it)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[it].v[j] += bv.v[j];
+      }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss += threadIdx.x + it * blockDim.x < H4 ? v[it].v[j] * v[it].v[j] : 0.f;
   ss = block_sum(ss, scratch);
   const float inv = rsqrtf(ss / (float)H + eps);
   act_t* o = out + (size_t)r * H;
+  const bool store = (plain || PARTS > 0) && rows == nullptr;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int i = threadIdx.x + it * blockDim.x;
     if (i < H4) {
-      const f4 wv = ((const f4*)w)[i];
       a4 ov;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ov.v[j] = from_f<act_t>(v[it].v[j] * inv * wv.v[j]);
+      for (int j = 0; j < 4; ++j) ov.v[j] = from_f<act_t>(v[it].v[j] * inv * wv[it].v[j]);
+      if (store) ((f4*)x)[i] = v[it];
       ((a4*)o)[i] = ov;
     }
   }
+}
+
+// Rows of n groups of four values (n up to 8 * 512): a workgroup's threads.  A group a thread is the shortest chain, and what a few rows
+// want (8 rows of 3,584 values with their output's norm: 896 threads 2.85 us, 512 with two groups each 3.4 before); with more rows than
+// CUs the waits of one cover another's, and workgroups stay at 512 as they were.
+static int row_threads(int R, int n) {
+  const int most = R <= 256 ? 1024 : 512, turns = (n + most - 1) / most;
+  return ((n + turns - 1) / turns + 63) / 64 * 64;
 }
 
 // parts != nullptr: nparts float partial sums [nparts][T][H] (T rows in each)
@@ -140,15 +174,27 @@ extern "C" const char* sl_add_rmsnorm(float* resid, const void* delta, const flo
                        ((uintptr_t)delta % sizeof(a4)) == 0 && ((uintptr_t)parts % 16) == 0 &&
                        ((uintptr_t)bias % 16) == 0 && ((uintptr_t)w % 16) == 0;
   if (H % 4 == 0 && H <= 4 * 8 * 512 && aligned) {
-    const int H4 = H / 4;
-    const int threads = H4 <= 64 ? 64 : (H4 <= 128 ? 128 : (H4 <= 256 ? 256 : 512));
-    const int iters = (H4 + threads - 1) / threads;
+    const int H4 = H / 4, threads = row_threads(R, H4), iters = (H4 + threads - 1) / threads;
     const act_t* dl = (const act_t*)delta;
     act_t* o = (act_t*)out;
-    if (iters == 1) add_rmsnorm_vec_kernel<1><<<R, threads, 0, stream>>>(resid, dl, sd, rows, w, o, H, eps);
-    else if (iters == 2) add_rmsnorm_vec_kernel<2><<<R, threads, 0, stream>>>(resid, dl, sd, rows, w, o, H, eps);
-    else if (iters <= 4) add_rmsnorm_vec_kernel<4><<<R, threads, 0, stream>>>(resid, dl, sd, rows, w, o, H, eps);
-    else add_rmsnorm_vec_kernel<8><<<R, threads, 0, stream>>>(resid, dl, sd, rows, w, o, H, eps);
+    auto run = [&](auto kernel) { kernel<<<R, threads, 0, stream>>>(resid, dl, sd, rows, w, o, H, eps); };
+    // (as many partial sums a trip as there are: reading one again in place of one that is not there costs many rows what it saves few)
+    if (parts == nullptr) {
+      if (iters == 1) run(add_rmsnorm_vec_kernel<1, 0>);
+      else if (iters == 2) run(add_rmsnorm_vec_kernel<2, 0>);
+      else if (iters <= 4) run(add_rmsnorm_vec_kernel<4, 0>);
+      else run(add_rmsnorm_vec_kernel<8, 0>);
+    } else if (iters == 1) {
+      if (nparts <= 2) run(add_rmsnorm_vec_kernel<1, 2>);
+      else if (nparts == 3) run(add_rmsnorm_vec_kernel<1, 3>);
+      else if (nparts == 4) run(add_rmsnorm_vec_kernel<1, 4>);
+      else run(add_rmsnorm_vec_kernel<1, 8>);
+    } else if (iters == 2) {
+      if (nparts <= 2) run(add_rmsnorm_vec_kernel<2, 2>);
+      else if (nparts == 3) run(add_rmsnorm_vec_kernel<2, 3>);
+      else run(add_rmsnorm_vec_kernel<2, 4>);
+    } else if (iters <= 4) run(add_rmsnorm_vec_kernel<4, 2>);
+    else run(add_rmsnorm_vec_kernel<8, 1>);
     return sl_launch_status();
   }
   const int threads = H >= 2048 ? 512 : 256;
@@ -205,8 +251,9 @@ __global__ void add_layernorm_kernel(float* __restrict__ resid, const act_t* __r
 // The same for rows of up to 4 * 8 * blockDim values that are a multiple of 4 wide: every value
 // is read once with 16-byte loads and stays in registers for the mean, the squared deviations
 // and the output.
+// All of it is asked for at once, as above, and the stream's new row is written behind the sums (4 rows of 2,048 values: 2.8 us before, 2.5 here).
 template <int ITERS>
-__global__ void add_layernorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ d1,
+__global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ d1,
                                          const act_t* __restrict__ d2, const int* __restrict__ rows,
                                          const float* __restrict__ w, const float* __restrict__ bias,
                                          act_t* __restrict__ out, int H, float eps) {
@@ -214,61 +261,55 @@ __global__ void add_layernorm_vec_kernel(float* __restrict__ resid, const act_t*
   const int r = blockIdx.x;
   const size_t src = rows != nullptr ? (size_t)rows[r] : (size_t)r;
   float* x = resid + src * H;
-  const act_t* a = d1 != nullptr ? d1 + src * H : nullptr;
-  const act_t* b = d2 != nullptr ? d2 + src * H : nullptr;
+  const act_t* a = d1 != nullptr ? d1 + src * H : (const act_t*)x;
+  const act_t* b = d2 != nullptr ? d2 + src * H : (const act_t*)x;
+  const float* add = bias != nullptr ? bias : w;
   const int H4 = H / 4;
-  f4 v[ITERS];
+  f4 v[ITERS], wv[ITERS], bv[ITERS];
+  a4 av[ITERS], cv[ITERS];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int i = min((int)(threadIdx.x + it * blockDim.x), H4 - 1);
+    v[it] = ((const f4*)x)[i];
+    av[it] = ((const a4*)a)[i];
+    cv[it] = ((const a4*)b)[i];
+    wv[it] = ((const f4*)w)[i];
+    bv[it] = ((const f4*)add)[i];
+  }
   float sum = 0.f;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int i = threadIdx.x + it * blockDim.x;
-    if (i < H4) {
-      v[it] = ((const f4*)x)[i];
-      if (a != nullptr || b != nullptr) {
-        float d[4] = {0.f, 0.f, 0.f, 0.f};
-        if (a != nullptr) {
-          const a4 av = ((const a4*)a)[i];
+    const bool in = threadIdx.x + it * blockDim.x < H4;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) d[j] = to_f(av.v[j]);
-        }
-        if (b != nullptr) {
-          const a4 bv = ((const a4*)b)[i];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) d[j] += to_f(bv.v[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[it].v[j] += d[j];
-        if (rows == nullptr) ((f4*)x)[i] = v[it];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sum += v[it].v[j];
+    for (int j = 0; j < 4; ++j) {
+      const float first = d1 != nullptr ? to_f(av[it].v[j]) : 0.f, second = d2 != nullptr ? to_f(cv[it].v[j]) : 0.f;
+      v[it].v[j] += first + second;
+      sum += in ? v[it].v[j] : 0.f;
     }
   }
   const float mean = block_sum(sum, scratch) / (float)H;
   float sq = 0.f;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int i = threadIdx.x + it * blockDim.x;
-    if (i < H4) {
+    const bool in = threadIdx.x + it * blockDim.x < H4;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[it].v[j] -= mean;
-        sq += v[it].v[j] * v[it].v[j];
-      }
+    for (int j = 0; j < 4; ++j) {
+      const float dv = v[it].v[j] - mean;
+      sq += in ? dv * dv : 0.f;
     }
   }
   const float inv = 1.f / sqrtf(block_sum(sq, scratch) / (float)H + eps);
   act_t* o = out + (size_t)r * H;
+  const bool store = (d1 != nullptr || d2 != nullptr) && rows == nullptr;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int i = threadIdx.x + it * blockDim.x;
     if (i < H4) {
-      const f4 wv = ((const f4*)w)[i];
-      f4 bv = {{0.f, 0.f, 0.f, 0.f}};
-      if (bias != nullptr) bv = ((const f4*)bias)[i];
       a4 ov;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ov.v[j] = from_f<act_t>(v[it].v[j] * inv * wv.v[j] + bv.v[j]);
+      for (int j = 0; j < 4; ++j)
+        ov.v[j] = from_f<act_t>((v[it].v[j] - mean) * inv * wv[it].v[j] + (bias != nullptr ? bv[it].v[j] : 0.f));
+      if (store) ((f4*)x)[i] = v[it];
       ((a4*)o)[i] = ov;
     }
   }
@@ -283,9 +324,7 @@ extern "C" const char* sl_add_layernorm(float* resid, const void* d1, const void
                        ((uintptr_t)d1 % sizeof(a4)) == 0 && ((uintptr_t)d2 % sizeof(a4)) == 0 &&
                        ((uintptr_t)w % 16) == 0 && ((uintptr_t)bias % 16) == 0;
   if (H % 4 == 0 && H <= 4 * 8 * 512 && aligned) {
-    const int H4 = H / 4;
-    const int nthreads = H4 <= 64 ? 64 : (H4 <= 128 ? 128 : (H4 <= 256 ? 256 : 512));
-    const int iters = (H4 + nthreads - 1) / nthreads;
+    const int H4 = H / 4, nthreads = row_threads(R, H4), iters = (H4 + nthreads - 1) / nthreads;
     const act_t* a = (const act_t*)d1;
     const act_t* b = (const act_t*)d2;
     act_t* o = (act_t*)out;
@@ -350,7 +389,22 @@ __global__ void streams_norm_kernel(const StreamsNorm a) {
   const float i1 = a.g1 != nullptr ? inv_rms(y1, H, a.e1, scratch) : 1.f;
   const float i2 = a.g2 != nullptr ? inv_rms(y2, H, a.e2, scratch) : 1.f;
   const bool writes = y1 != nullptr, store = a.rows == nullptr;
-  auto group = [&](int i) -> fv {
+  // (the copies' weights stand in registers where their number is known: behind a store to the stream they would be
+  // read again: one row of four copies of 2,048 values 3.8 us, now 3.0, with two normed outputs 6.1, now 4.9)
+  float rd[MAXS], ot[MAXS], mx[EXACT ? MAXS : 1][EXACT ? MAXS : 1];
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int t = 0; t < MAXS; ++t) {
+      rd[t] = a.read != nullptr ? a.read[t] : 1.f;
+      ot[t] = writes ? a.out[t] : 0.f;
+#pragma unroll
+      for (int s = 0; s < MAXS; ++s) mx[s][t] = writes ? a.mix[s * MAXS + t] : 0.f;
+    }
+  }
+  auto reads = [&](int t) { return EXACT ? rd[t] : a.read != nullptr ? a.read[t] : 1.f; };
+  auto group = [&](int at) -> fv {
+    const int i = min(at, HV - 1);
+    const bool keeps = store && at < HV;
     fv xs[MAXS], u;
 #pragma unroll
     for (int s = 0; s < MAXS; ++s)
@@ -361,7 +415,7 @@ __global__ void streams_norm_kernel(const StreamsNorm a) {
 #pragma unroll
       for (int s = 0; s < MAXS; ++s)
         if (EXACT || s < S) {
-          const float f = a.read != nullptr ? a.read[s] : 1.f;
+          const float f = reads(s);
 #pragma unroll
           for (int c = 0; c < VEC; ++c) u.v[c] += f * xs[s].v[c];
         }
@@ -385,18 +439,18 @@ __global__ void streams_norm_kernel(const StreamsNorm a) {
 #pragma unroll
     for (int t = 0; t < MAXS; ++t)
       if (EXACT || t < S) {
-        const float f = a.read != nullptr ? a.read[t] : 1.f, ot = a.out[t];
+        const float f = reads(t), o1 = EXACT ? ot[t] : a.out[t];
         fv n;
 #pragma unroll
-        for (int c = 0; c < VEC; ++c) n.v[c] = ot * y.v[c];
+        for (int c = 0; c < VEC; ++c) n.v[c] = o1 * y.v[c];
 #pragma unroll
         for (int s = 0; s < MAXS; ++s)
           if (EXACT || s < S) {
-            const float m = a.mix[s * S + t];
+            const float m = EXACT ? mx[EXACT ? s : 0][EXACT ? t : 0] : a.mix[s * S + t];
 #pragma unroll
             for (int c = 0; c < VEC; ++c) n.v[c] += m * xs[s].v[c];
           }
-        if (store) *(fv*)(x + (size_t)t * H + (size_t)i * VEC) = n;
+        if (keeps) *(fv*)(x + (size_t)t * H + (size_t)i * VEC) = n;
 #pragma unroll
         for (int c = 0; c < VEC; ++c) u.v[c] += f * n.v[c];
       }
@@ -409,11 +463,9 @@ __global__ void streams_norm_kernel(const StreamsNorm a) {
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const int i = threadIdx.x + it * blockDim.x;
-      if (i < HV) {
-        keep[it] = group(i);
+      keep[it] = group(i);
 #pragma unroll
-        for (int c = 0; c < VEC; ++c) sum += keep[it].v[c];
-      }
+      for (int c = 0; c < VEC; ++c) sum += i < HV ? keep[it].v[c] : 0.f;
     }
   } else {
     for (int i = threadIdx.x; i < HV; i += blockDim.x) {      // (VEC 1)
@@ -470,9 +522,7 @@ static const char* launch_streams_norm(const StreamsNorm& a, int R, hipStream_t 
   const uintptr_t f32s = (uintptr_t)a.x | (uintptr_t)a.g1 | (uintptr_t)a.g2 | (uintptr_t)a.w | (uintptr_t)a.bias;
   const uintptr_t acts = (uintptr_t)a.y1 | (uintptr_t)a.y2 | (uintptr_t)a.o;
   if (a.H % 4 == 0 && a.H <= 4 * 8 * 512 && f32s % 16 == 0 && acts % (4 * sizeof(act_t)) == 0) {
-    const int H4 = a.H / 4;
-    const int threads = H4 <= 64 ? 64 : (H4 <= 128 ? 128 : (H4 <= 256 ? 256 : 512));
-    const int iters = (H4 + threads - 1) / threads;
+    const int H4 = a.H / 4, threads = row_threads(R, H4), iters = (H4 + threads - 1) / threads;
     if (iters == 1) streams_norm_kernel<MAXS, EXACT, 4, 1><<<R, threads, 0, stream>>>(a);
     else if (iters == 2) streams_norm_kernel<MAXS, EXACT, 4, 2><<<R, threads, 0, stream>>>(a);
     else if (iters <= 4) streams_norm_kernel<MAXS, EXACT, 4, 4><<<R, threads, 0, stream>>>(a);
@@ -572,11 +622,65 @@ __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __re
   }
 }
 
+// The same for rows of up to 4 * 8 * 512 values that are a multiple of 4 wide, 16-byte loads (8 rows of 3,584 values: 2.5 us with single
+// ones, 2.1 here; one of 2,048 2.1, now 1.7).
+template <int ITERS>
+__global__ __launch_bounds__(1024) void add_postnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
+                                                                const float* __restrict__ w, act_t* __restrict__ out, int H, float eps,
+                                                                float mult) {
+  __shared__ float scratch[16];
+  const size_t r = blockIdx.x;
+  float* x = resid + r * H;
+  const int H4 = H / 4;
+  f4 v[ITERS], wv[ITERS];
+  a4 yv[ITERS];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int i = min((int)(threadIdx.x + it * blockDim.x), H4 - 1);
+    yv[it] = ((const a4*)(y + r * H))[i];
+    v[it] = ((const f4*)x)[i];
+    wv[it] = ((const f4*)w)[i];
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float n = threadIdx.x + it * blockDim.x < H4 ? to_f(yv[it].v[j]) : 0.f;
+      ss += n * n;
+    }
+  const float inv = 1.f / sqrtf(block_sum(ss, scratch) / (float)H + eps);
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int i = threadIdx.x + it * blockDim.x;
+    if (i < H4) {
+      a4 ov;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[it].v[j] += mult * (to_f(yv[it].v[j]) * inv * wv[it].v[j]);
+        ov.v[j] = from_f<act_t>(v[it].v[j]);
+      }
+      ((f4*)x)[i] = v[it];
+      if (out != nullptr) ((a4*)(out + r * H))[i] = ov;
+    }
+  }
+}
+
 extern "C" const char* sl_add_postnorm(float* resid, const void* y, const float* w, void* out, int T, int H,
                                        float eps, float mult, hipStream_t stream) {
   SL_CHECK(T >= 0 && H > 0, "add_postnorm: sizes must be positive");
   SL_CHECK(y != nullptr || out != nullptr, "add_postnorm: nothing to do");
   if (T == 0) return nullptr;
+  if (y != nullptr && H % 4 == 0 && H <= 4 * 8 * 512 && ((uintptr_t)resid | (uintptr_t)w) % 16 == 0 &&
+      ((uintptr_t)y | (uintptr_t)out) % sizeof(a4) == 0) {
+    const int H4 = H / 4, n = row_threads(T, H4), iters = (H4 + n - 1) / n;
+    auto run = [&](auto kernel) { kernel<<<T, n, 0, stream>>>(resid, (const act_t*)y, w, (act_t*)out, H, eps, mult); };
+    if (iters == 1) run(add_postnorm_vec_kernel<1>);
+    else if (iters == 2) run(add_postnorm_vec_kernel<2>);
+    else if (iters <= 4) run(add_postnorm_vec_kernel<4>);
+    else run(add_postnorm_vec_kernel<8>);
+    return sl_launch_status();
+  }
   const int threads = H >= 2048 ? 512 : 256, need = (H + threads - 1) / threads;
   auto run = [&](auto kernel) { kernel<<<T, threads, 0, stream>>>(resid, (const act_t*)y, w, (act_t*)out, H, eps, mult); };
   if (need <= 1) run(add_postnorm_kernel<1>);
@@ -652,12 +756,73 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
   }
 }
 
+// The same with 16-byte loads, as above; the stream's new row is written behind both sums (2 rows of 2,048 values: 3.0 us, now 2.1).
+template <int ITERS>
+__global__ __launch_bounds__(1024) void add_normed_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
+                                                                      const float* __restrict__ wy, float eps_y,
+                                                                      const int* __restrict__ rows, const float* __restrict__ w, float eps,
+                                                                      act_t* __restrict__ out, int H) {
+  __shared__ float scratch[16];
+  const size_t r = rows != nullptr ? (size_t)rows[blockIdx.x] : (size_t)blockIdx.x;
+  float* x = resid + r * H;
+  const int H4 = H / 4;
+  f4 v[ITERS], wv[ITERS], wyv[ITERS];
+  a4 yv[ITERS];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int i = min((int)(threadIdx.x + it * blockDim.x), H4 - 1);
+    yv[it] = ((const a4*)(y + r * H))[i];
+    v[it] = ((const f4*)x)[i];
+    wyv[it] = ((const f4*)wy)[i];
+    wv[it] = ((const f4*)w)[i];
+  }
+  float ss = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float n = threadIdx.x + it * blockDim.x < H4 ? to_f(yv[it].v[j]) : 0.f;
+      ss += n * n;
+    }
+  const float inv_y = 1.f / sqrtf(block_sum(ss, scratch) / (float)H + eps_y);
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[it].v[j] += to_f(yv[it].v[j]) * inv_y * wyv[it].v[j];
+      s2 += threadIdx.x + it * blockDim.x < H4 ? v[it].v[j] * v[it].v[j] : 0.f;
+    }
+  const float inv = 1.f / sqrtf(block_sum(s2, scratch) / (float)H + eps);
+  act_t* o = out + (size_t)blockIdx.x * H;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int i = threadIdx.x + it * blockDim.x;
+    if (i < H4) {
+      a4 ov;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ov.v[j] = from_f<act_t>(v[it].v[j] * inv * wv[it].v[j]);
+      if (rows == nullptr) ((f4*)x)[i] = v[it];
+      ((a4*)o)[i] = ov;
+    }
+  }
+}
+
 extern "C" const char* sl_add_normed_rmsnorm(float* resid, const void* y, const float* wy, float eps_y,
                                              const int* rows, const float* w, float eps, void* out, int R,
                                              int H, hipStream_t stream) {
   SL_CHECK(R >= 0 && H > 0, "add_normed_rmsnorm: sizes must be positive");
   SL_CHECK(y != nullptr && wy != nullptr && w != nullptr, "add_normed_rmsnorm: the output and both gains are required");
   if (R == 0) return nullptr;
+  if (H % 4 == 0 && H <= 4 * 8 * 512 && ((uintptr_t)resid | (uintptr_t)w | (uintptr_t)wy) % 16 == 0 &&
+      ((uintptr_t)y | (uintptr_t)out) % sizeof(a4) == 0) {
+    const int H4 = H / 4, n = row_threads(R, H4), iters = (H4 + n - 1) / n;
+    auto run = [&](auto kernel) { kernel<<<R, n, 0, stream>>>(resid, (const act_t*)y, wy, eps_y, rows, w, eps, (act_t*)out, H); };
+    if (iters == 1) run(add_normed_rmsnorm_vec_kernel<1>);
+    else if (iters == 2) run(add_normed_rmsnorm_vec_kernel<2>);
+    else if (iters <= 4) run(add_normed_rmsnorm_vec_kernel<4>);
+    else run(add_normed_rmsnorm_vec_kernel<8>);
+    return sl_launch_status();
+  }
   const int threads = H >= 2048 ? 512 : 256, need = (H + threads - 1) / threads;
   auto run = [&](auto kernel) {
     kernel<<<R, threads, 0, stream>>>(resid, (const act_t*)y, wy, eps_y, rows, w, eps, (act_t*)out, H);

@@ -394,48 +394,50 @@ __global__ __launch_bounds__(256) void stream_conv_kernel(const ShortConv a, act
 // last inputs, and the slot moved on by one.  A block takes slices of a token's channels, a channel a thread, so that the slot is
 // read and rewritten without a barrier; every block of a token adds up all of its y (7 KB) for the norm.  What bounds it is the
 // trips to memory in a row: all that a channel of the first slice needs is asked for before that sum (8 tokens of 3,584
-// channels, four taps: 10.6 us with a block a token, whose threads took their channels one after the other, 4.8 here).  Tokens that
+// channels, four taps: 10.6 us with a block a token, whose threads took their channels one after the other, 3.6 with loads behind
+// conditions, 3.0 here).  Tokens that
 // fill the chip with fewer blocks get fewer (300 of 3,584, two / four taps: 10.8 / 11.8 us with a slice a block, 7.6 / 10.6
 // with a block a token, 8.2 / 9.9 here).  The sums run in the order of the kernels for longer steps.
 // (LOOP apart from the one slice: a loop about the loads costs that 0.5 us.)
-constexpr int STREAM_KEEP = 8, STREAM_TAPS = 3;
+constexpr int STREAM_KEEP = 4, STREAM_TAPS = 3;
 template <bool LOOP>
 __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid, const act_t* __restrict__ y,
                                    const float* __restrict__ wy, float eps, int write, act_t* __restrict__ out) {
   __shared__ float scratch[16];
   const int t = blockIdx.x, H = a.C, back = a.taps - 1;
   float* x = resid + (size_t)t * H;
-  const act_t* yr = y != nullptr ? y + (size_t)t * H : nullptr;
+  const bool adds = y != nullptr;
+  const act_t* yr = adds ? y + (size_t)t * H : (const act_t*)x;         // (what is absent is read from the row and left out: no load
+  const float* gains = adds ? wy : x;                                   // stands behind a condition)
   const int s = t;                                     // (a token a sequence)
   const bool fresh = a.positions[t] == 0;
   float* keep_in = a.state + (size_t)a.slots[s] * a.state_stride + a.state_off;
-  float v, yv = 0.f, gain = 0.f, w_own;
+  const float* kept = back > 0 ? keep_in : x;
+  float v, yv, gain, w_own;
   float past[STREAM_TAPS], w[STREAM_TAPS];
   auto ask = [&](int c) {
     v = x[c];
-    if (back > 0) {
 #pragma unroll
-      for (int j = 0; j < STREAM_TAPS; ++j) {          // (past the taps: the last again, not used)
-        past[j] = keep_in[(size_t)min(j, back - 1) * H + c];
-        w[j] = a.w[(size_t)min(j, back) * H + c];
-      }
+    for (int j = 0; j < STREAM_TAPS; ++j) {            // (past the taps: the last again, not used)
+      past[j] = kept[(size_t)max(min(j, back - 1), 0) * H + c];
+      w[j] = a.w[(size_t)min(j, back) * H + c];
     }
     w_own = a.w[(size_t)back * H + c];
-    if (yr != nullptr) {
-      yv = to_f(yr[c]);
-      gain = wy[c];
-    }
+    yv = to_f(yr[c]);
+    gain = gains[c];
   };
   const int first = blockIdx.y * blockDim.x + threadIdx.x;
   ask(min(first, H - 1));
   float inv = 0.f;
-  if (yr != nullptr) {
+  if (adds) {
     float ss = 0.f;
+    act_t z[STREAM_KEEP];
+#pragma unroll
+    for (int u = 0; u < STREAM_KEEP; ++u) z[u] = yr[min((int)(threadIdx.x + u * blockDim.x), H - 1)];
 #pragma unroll
     for (int u = 0; u < STREAM_KEEP; ++u) {
-      const int e = threadIdx.x + u * blockDim.x;
-      const float z = e < H ? to_f(yr[e]) : 0.f;
-      ss += z * z;
+      const float n = threadIdx.x + u * blockDim.x < H ? to_f(z[u]) : 0.f;
+      ss += n * n;
     }
     for (int e = threadIdx.x + STREAM_KEEP * blockDim.x; e < H; e += blockDim.x) {
       const float z = to_f(yr[e]);
@@ -445,7 +447,7 @@ __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid,
     inv = 1.f / sqrtf(ss / (float)H + eps);
   }
   auto channel = [&](int c) {
-    if (yr != nullptr) {
+    if (adds) {
       v += yv * inv * gain;
       x[c] = v;
     }
