@@ -189,19 +189,11 @@ __device__ __forceinline__ float conv_channel_taps(const ShortConv& a, int first
   float x[N], w[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) w[j] = a.w[(size_t)c * N + j];
-  if (a.shift) {                             // (one token: which inputs lie where is known, and no load stands behind a condition)
 #pragma unroll
-    for (int j = 0; j < N - 1; ++j) x[j] = past[(size_t)j * a.C + c];
-    x[N - 1] = a.buf[(size_t)first * a.stride + a.col + c];
-#pragma unroll
-    for (int j = 0; j < N - 1; ++j) x[j] = fresh ? 0.f : x[j];
-  } else {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int idx = i - (N - 1) + j;
-      if (idx >= 0) x[j] = a.buf[(size_t)(first + idx) * a.stride + a.col + c];
-      else x[j] = fresh ? 0.f : past[(size_t)(N - 1 + idx) * a.C + c];
-    }
+  for (int j = 0; j < N; ++j) {
+    const int idx = i - (N - 1) + j;
+    if (idx >= 0) x[j] = a.buf[(size_t)(first + idx) * a.stride + a.col + c];
+    else x[j] = fresh ? 0.f : past[(size_t)(N - 1 + idx) * a.C + c];
   }
   float acc = a.bias != nullptr ? a.bias[c] : 0.f;
 #pragma unroll
@@ -229,7 +221,44 @@ __device__ __forceinline__ float conv_channel(const ShortConv& a, int first, int
   return acc;
 }
 
-// One wavefront per (token, head of the unit part | 256 other channels).
+// The N inputs of four channels of a token and the sums over them, everything asked for before the first sum and the slot's new inputs
+// written behind it.  A step's input is a row of the step or of the slot, the same for all lanes: a choice of address, not of loads, which
+// would be waited for where the ways meet.
+template <int N, int U>
+__device__ __forceinline__ void conv_channels(const ShortConv& a, int first, int i, bool fresh, float* past, const int (&at)[U], float (&acc)[U],
+                                              float (&x)[U][N]) {
+  float w[U][N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int idx = i - (N - 1) + j;
+    const float* row = idx >= 0 ? a.buf + (size_t)(first + idx) * a.stride + a.col : past + (size_t)(N - 1 + idx) * a.C;
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u][j] = row[at[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) w[u][j] = a.w[(size_t)at[u] * N + j];
+    acc[u] = a.bias != nullptr ? a.bias[at[u]] : 0.f;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      x[u][j] = fresh && i - (N - 1) + j < 0 ? 0.f : x[u][j];
+      acc[u] += w[u][j] * x[u][j];
+    }
+}
+template <int N, int U>
+__device__ __forceinline__ void conv_shift(const ShortConv& a, float* past, int at, const float (&x)[U][N], int u) {
+#pragma unroll
+  for (int j = 1; j < N; ++j) past[(size_t)(j - 1) * a.C + at] = x[u][j];
+}
+
+// One wavefront per (token, head of the unit part | 256 other channels).  N: the taps, 0 for other numbers (one request's 8,192 channels of four
+// taps 3.8 us with a channel after the other, now 2.5; 2,048 tokens of 6,144
+// channels, 100 MB, 41, now 29).
+template <int N>
 __global__ __launch_bounds__(64) void short_conv_kernel(const ShortConv a) {
   const int t = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
   int c0, n;
@@ -247,36 +276,18 @@ __global__ __launch_bounds__(64) void short_conv_kernel(const ShortConv a) {
   float* past = a.state + (size_t)a.slots[s] * a.state_stride + a.state_off;
   float ss = 0.f;
   float y[4];
-  if (a.shift && a.taps == 4) {
-    // (a token each: the slot's new inputs are written behind the loads of all four channels, or a channel would wait for the one before:
-    // one request's 8,192 channels 3.8 us, now 2.5)
-    float past_x[4][3], own[4], w[4][4], add[4];
+  if constexpr (N > 0) {
+    float x[4][N], acc[4];
     int at[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = at[u] = c0 + min(lane + u * 64, n - 1);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) past_x[u][j] = past[(size_t)j * a.C + c];
-      own[u] = a.buf[(size_t)first * a.stride + a.col + c];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[u][j] = a.w[(size_t)c * 4 + j];
-      add[u] = a.bias != nullptr ? a.bias[c] : 0.f;
-    }
+    for (int u = 0; u < 4; ++u) at[u] = c0 + min(lane + u * 64, n - 1);
+    conv_channels<N, 4>(a, first, i, fresh, past, at, acc, x);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      float acc = add[u];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        past_x[u][j] = fresh ? 0.f : past_x[u][j];
-        acc += w[u][j] * past_x[u][j];
-      }
-      acc += w[u][3] * own[u];
-      y[u] = a.silu ? acc * sigmoidf_(acc) : acc;
+      y[u] = a.silu ? acc[u] * sigmoidf_(acc[u]) : acc[u];
       if (lane + u * 64 < n) {
         ss += y[u] * y[u];
-        past[at[u]] = past_x[u][1];
-        past[(size_t)a.C + at[u]] = past_x[u][2];
-        past[2 * (size_t)a.C + at[u]] = own[u];
+        if (a.shift) conv_shift<N, 4>(a, past, at[u], x, u);
       }
     }
   } else
@@ -342,7 +353,11 @@ extern "C" const char* sl_short_conv(const float* buf, int stride, int col, int 
   const ShortConv a{buf, stride, col, C, taps, w, bias, state, state_stride, state_off, cu_q, positions, tok_seq,
                     slots, unit_heads, unit_dim, scaled_heads, unit_eps, scale, silu, out, (act_t*)rows, shift};
   const int rest = C - unit_heads * unit_dim;
-  short_conv_kernel<<<dim3(T, unit_heads + (rest + 255) / 256), 64, 0, stream>>>(a);
+  auto run = [&](auto kernel) { kernel<<<dim3(T, unit_heads + (rest + 255) / 256), 64, 0, stream>>>(a); };
+  if (taps == 4) run(short_conv_kernel<4>);
+  else if (taps == 3) run(short_conv_kernel<3>);
+  else if (taps == 2) run(short_conv_kernel<2>);
+  else run(short_conv_kernel<0>);
   if (write && taps > 1 && !shift) short_conv_state_kernel<<<dim3(S, (C + 255) / 256), 256, 0, stream>>>(a, S);
   return sl_launch_status();
 }
@@ -1282,7 +1297,8 @@ __global__ void projnorm_rope_store_kernel(const float* __restrict__ buf, int st
 
 // The same for a step of few tokens and rows of at most 4,096 values of q and k and 1,024 of v: what a thread needs is asked for before the
 // first sum (its four values of the row, their gains and their partners', angles, its value of v), and both sums meet at once.  One
-// token, 16 heads on 2 of 128: 4.9 us, now 4.3; behind a convolution of four taps 8.4, now 5.3.
+// token, 16 heads on 2 of 128: 4.9 us, now 4.3; behind a convolution of four taps 8.4, now 5.3. A prompt's 1,500 tokens take 35 us in
+// this form behind a convolution, 30 in the one above.
 template <bool CONV>
 __global__ __launch_bounds__(1024) void projnorm_step_kernel(const float* __restrict__ buf, int stride, int H, int G, int D, int Dv,
                                                              const float* __restrict__ qw, const float* __restrict__ kw, float eps,
@@ -1322,31 +1338,17 @@ __global__ __launch_bounds__(1024) void projnorm_step_kernel(const float* __rest
     const int s = cv.shift ? (int)t : cv.tok_seq[t], first = cv.shift ? (int)t : cv.cu_q[s];
     const bool fresh = cv.positions[first] == 0;
     float* past = cv.state + (size_t)cv.slots[s] * cv.state_stride + cv.state_off;
-    if (cv.shift && cv.taps == 4 && cv.C <= 4096) {                    // (as in short_conv_kernel)
-      float px[4][3], own[4], cw[4][4];
+    if (cv.taps == 4 && cv.C <= 4096) {
+      float px[4][4], acc[4];
+      int at[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) at[u] = min(tid + 1024 * u, cv.C - 1);
+      conv_channels<4, 4>(cv, first, (int)t - first, fresh, past, at, acc, px);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int c = min(tid + 1024 * u, cv.C - 1);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) px[u][j] = past[(size_t)j * cv.C + c];
-        own[u] = row[c];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) cw[u][j] = cv.w[(size_t)c * 4 + j];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int c = tid + 1024 * u;
-        if (c >= cv.C) break;
-        float acc = 0.f;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          px[u][j] = fresh ? 0.f : px[u][j];
-          acc += cw[u][j] * px[u][j];
-        }
-        xs[c] = acc + cw[u][3] * own[u];
-        past[c] = px[u][1];
-        past[(size_t)cv.C + c] = px[u][2];
-        past[2 * (size_t)cv.C + c] = own[u];
+        if (tid + 1024 * u >= cv.C) break;
+        xs[at[u]] = acc[u];
+        if (cv.shift) conv_shift<4, 4>(cv, past, at[u], px, u);
       }
     } else {
       for (int c = tid; c < cv.C; c += 1024) xs[c] = conv_channel(cv, first, (int)t - first, fresh, past, c);
