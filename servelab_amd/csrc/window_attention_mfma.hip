@@ -44,13 +44,19 @@
 #error "values read from key rows cannot be wider than a key"
 #endif
 
+// Values with pages of their own: two teams hold keys, values and sums of up to this width in registers.  Wider ones spill
+// (512 / 512: 158 registers), and some do not fit two staged blocks in a CU: they take one team, whose wavefronts have twice the registers.
+// us, two teams / one, 16 heads on 2, a prompt of 1,024: 128 / 128 33 / 48, 512 / 256 64 / 85, 704 / 256 88 / 101; beyond the line 512 / 512 197 / 119,
+// 384 / 512 123 / 111, 1024 / 112 105 / 102.
+#define SL_NARROW (SL_DK + 2 * SL_DV <= 1216)
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int DK = SL_DK, DV = SL_DV;
-constexpr bool VK = SL_VK != 0;
+constexpr bool VK = SL_VK != 0, NARROW = SL_NARROW;
 constexpr int KK = DK / 32, DD = DV / 16;
 constexpr int KROW = DK + 8;          // elements of a staged key row (the pad spreads rows over the banks)
 constexpr int VROW = 40;              // elements of a staged channel row: 32 keys and a pad
@@ -79,12 +85,14 @@ __device__ __forceinline__ float column_sum4(float x) {
 
 // A prompt's workgroup is eight wavefronts over 64 columns: two teams of four that take every other block and meet at the end, or,
 // where values lie in the key rows, one whose wavefronts share their 16 columns two and two, each with half of the channels.
-constexpr int TEAMS = VK ? 1 : 2, PARTS = VK ? 2 : 1;
+constexpr int TEAMS = VK || !NARROW ? 1 : 2, PARTS = VK ? 2 : 1;
 constexpr int THREADS = 256 * PARTS, COLS = 64;         // of a team
 constexpr int KKP = (KK + PARTS - 1) / PARTS, DDP = (DD + PARTS - 1) / PARTS;      // steps of key channels and tiles of value channels a wavefront
 constexpr int MEETS = VK ? 8 * 2 * 64 * 16 : 0;         // bytes in which the parts of the scores meet
 constexpr int STAGE = 32 * KROW + VT;                   // values of a team's staged block
 constexpr int MEET = TEAMS == 2 ? 256 * DV + 512 : 0;   // bytes in which the second team hands over what it has
+constexpr int STAGED = 2 * TEAMS * STAGE + MEETS, LDS_BYTES = STAGED > MEET ? STAGED : MEET;
+static_assert(LDS_BYTES <= 160 * 1024, "a prompt's workgroup fits a CU");
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
 // what a thread stages of a block: chunks of 8 values (16 bytes)
 constexpr int KCH = DK / 8;                            // chunks of a key row
@@ -104,7 +112,7 @@ constexpr int NR = VK ? (RCH ? cdiv(32 * RCH, THREADS) : 1) : 1;
 // 1,000 410 moved, 463 with early tiles first.)
 enum { IN_ORDER = 0, LATE_FIRST = 1, BY_LENGTH = 2, BY_LENGTH_MOVED = 3 };
 
-__global__ __launch_bounds__(TEAMS * THREADS, TEAMS == 1 ? 2 : DK <= 128 && DV <= 128 ? 4 : 2) void window_attention_mfma_kernel(const WindowAttention a, int order) {
+__global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK && DK <= 128 && DV <= 128 ? 4 : 2) void window_attention_mfma_kernel(const WindowAttention a, int order) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
   const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
   __bf16* ks = lds16 + team * STAGE;                   // [32][KROW]
@@ -477,13 +485,12 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS == 1 ? 2 : DK <= 128 && DV <
 #include "window_step.h"
 
 static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, hipStream_t stream) {
-  const size_t staged = sizeof(__bf16) * TEAMS * STAGE + MEETS, bytes = staged > MEET ? staged : MEET;
-  if (bytes > 48 * 1024) {
+  if (LDS_BYTES > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
     if (e != hipSuccess) return hipGetErrorString(e);
   }
-  window_attention_mfma_kernel<<<grid, TEAMS * THREADS, bytes, stream>>>(a, order);
+  window_attention_mfma_kernel<<<grid, TEAMS * THREADS, LDS_BYTES, stream>>>(a, order);
   return sl_launch_status();
 }
 static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream_t stream) {
@@ -498,10 +505,6 @@ static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream
 
 // Blocks of 32 keys that a workgroup of a step of single tokens takes side by side.
 extern "C" int sl_window_attention_mfma_step_blocks() { return STEP_BLOCKS; }
-
-extern "C" int sl_window_attention_mfma_lds_bytes() {
-  return (int)(sizeof(__bf16) * ((size_t)32 * KROW + (size_t)VT));
-}
 
 // The call of sl_window_attention, for Dk == SL_DK, Dv == SL_DV and (vc == nullptr) == SL_VK.
 // q rows, key rows and value rows must be 16-byte aligned.

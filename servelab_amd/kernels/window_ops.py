@@ -18,17 +18,14 @@ class WindowOps:
     WINDOW_SHARE_KEYS = 256
     WINDOW_MAX_SHARES = 16
     WINDOW_MFMA_MAX_SHARES = 32
-    WINDOW_MFMA_LDS_BYTES = 160 * 1024
 
     def _window_mfma_fits(self, q, q_col, Dk, Dv):
         """The matrix-core kernel takes bfloat16, key widths in steps of 32 and value widths in steps
-        of 16 whose staged block fits LDS, and q rows that are 16-byte aligned; everything else goes
-        to the float kernel."""
+        of 16 (a staged block of the widest fits LDS), and q rows that are 16-byte aligned; everything
+        else goes to the float kernel."""
         if self.act_dtype != torch.bfloat16 or not self.use_mfma_attention:
             return False
         if Dk % 32 or Dv % 16 or Dk > 1024 or Dv > 512:
-            return False
-        if 2 * (32 * (Dk + 8) + Dv * 40) > self.WINDOW_MFMA_LDS_BYTES:
             return False
         return q.shape[1] % 8 == 0 and q_col % 8 == 0 and q.data_ptr() % 16 == 0
 
