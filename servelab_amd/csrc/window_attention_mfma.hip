@@ -102,6 +102,11 @@ constexpr int RCH = VK ? (DK - DV) / 8 : 0;            // chunks of a key row be
 constexpr int NT = VK ? cdiv((DV / 8) * 4, THREADS) : 1;   // 8 keys x 8 channels tiles a thread (turned on their way into LDS)
 constexpr int NR = VK ? (RCH ? cdiv(32 * RCH, THREADS) : 1) : 1;
 
+// A thread's places in a block are the same for all blocks and stay in registers, except where these are short; us, kept / worked out
+// anew: 512 / 256 64 / 69 (no register spilled either way), 896 / 64 145 (50 spilled) / 80; one team: 512 / 512 119 / 135 (none), 640 / 512 146 (13) / 145 and
+// steps of 32 requests 41 / 37, 1024 / 512 241 (76) / 200.
+constexpr bool PLACES_ANEW = !VK && (TEAMS == 2 ? 4 * DK + 5 * DV > 3328 : DK + 2 * DV > 1600);
+
 // Workgroups start in the order of their number, and numbers go to the eight dies in turn and there to the groups of CUs in
 // turn.  Without a window or chunks a tile takes as long as its keys are many, so the late tiles come first:
 // BY_LENGTH, for sequences of one length: of every sequence and head, so that the short ones fill what is left at the end;
@@ -214,7 +219,13 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
   // lies in slots no column sees gets no weight, and values there become zeros.  No load stands behind a condition: the
   // compiler waits for a load where the two ways meet.
   bf16x8 kreg[NKC], vreg[NVC], treg[NT][8], rreg[NR];
+  auto this_thread = [&]() {
+    int x = tid;
+    if (PLACES_ANEW) asm volatile("" : "+v"(x));       // (nothing that follows from it is kept from block to block)
+    return x;
+  };
   auto fetch = [&](int kbase, int asked) {
+    const int tid = this_thread();
     const int pgA = __builtin_amdgcn_readlane(asked, 0), pgB = __builtin_amdgcn_readlane(asked, 1);
     const bool seenA = kbase + 15 >= kmin || kbase < keep, seenB = kbase + 16 <= kmax && (kbase + 31 >= kmin || kbase + 16 < keep);
     const size_t headA = (size_t)(seenA ? pgA : pgB) * nkv + kvh, headB = (size_t)(seenB ? pgB : pgA) * nkv + kvh;
@@ -251,6 +262,7 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
     }
   };
   auto store = [&](int kbase) {
+    const int tid = this_thread();
     const bool all_seen = kbase + 31 <= kmax && (kbase >= kmin || kbase + 31 < keep);
     if constexpr (!VK) {
 #pragma unroll
