@@ -44,10 +44,12 @@
 #error "values read from key rows cannot be wider than a key"
 #endif
 
-// Values with pages of their own: two teams hold keys, values and sums of up to this width in registers.  Wider ones spill
-// (512 / 512: 158 registers), and some do not fit two staged blocks in a CU: they take one team, whose wavefronts have twice the registers.
-// us, two teams / one, 16 heads on 2, a prompt of 1,024: 128 / 128 33 / 48, 512 / 256 64 / 85, 704 / 256 88 / 101; beyond the line 512 / 512 197 / 119,
-// 384 / 512 123 / 111, 1024 / 112 105 / 102.
+// Values with pages of their own: two teams, and the kernel of window_step.h for steps, hold keys, values and sums of up to this
+// width in registers.  Wider ones spill there (512 / 512: 158 and 126 registers), and some do not fit two staged blocks in a CU: they take
+// one team, whose wavefronts have twice the registers, and their steps the same kernel with the keys cut into shares.  us, two teams and step
+// kernel / one team and shares, 16 heads on 2: a prompt of 1,024, and steps of 8 requests at 1,500: 128 / 128 33 / 48 and 7.6 / 10.1, 512 / 256 64 / 85
+// and 13.3 / 16.5, 704 / 256 88 / 101 and 14.8 / 20.0; beyond the line 512 / 512 197 / 119 and 35.6 / 22.4, 384 / 512 123 / 111 and 29.8 /
+// 21.1, 1024 / 112 105 / 102 and 15.7 / 20.6.
 #define SL_NARROW (SL_DK + 2 * SL_DV <= 1216)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -505,6 +507,7 @@ static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, h
   window_attention_mfma_kernel<<<grid, TEAMS * THREADS, LDS_BYTES, stream>>>(a, order);
   return sl_launch_status();
 }
+#if SL_VK || SL_NARROW
 static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream_t stream) {
   const size_t bytes = VK ? sizeof(__bf16) * ((size_t)32 * KROW + (size_t)VT) : 0;
   if (bytes > 48 * 1024) {
@@ -514,8 +517,11 @@ static const char* launch_step(const WindowAttention& a, int num_seqs, hipStream
   window_step_kernel<<<dim3(a.nsplit, a.nkv * ((a.nh / a.nkv + 15) / 16), num_seqs), 64 * STEP_WAVES, bytes, stream>>>(a);
   return sl_launch_status();
 }
+#else
+static const char* launch_step(const WindowAttention&, int, hipStream_t) { return "window attention: no kernel for steps of this width"; }
+#endif
 
-// Blocks of 32 keys that a workgroup of a step of single tokens takes side by side.
+// Blocks of 32 keys that a workgroup of a step of single tokens takes side by side; 0: such steps take the kernel of prompts, cut into shares.
 extern "C" int sl_window_attention_mfma_step_blocks() { return STEP_BLOCKS; }
 
 // The call of sl_window_attention, for Dk == SL_DK, Dv == SL_DV and (vc == nullptr) == SL_VK.
@@ -546,7 +552,7 @@ extern "C" const char* sl_window_attention_mfma(
                           cu_q, positions, nh, nkv, Dk, Dv, page, scale, softcap, window, chunk, keep_first, slopes, sinks,
                           (const act_t*)gate, gate_stride, channel_gate, channel_stride, (act_t*)out, nsplit, part_o,
                           part_ml};
-  if (max_q_len == 1 && num_tokens == num_seqs && (nsplit == 1 || (uintptr_t)part_ml % 8 == 0) &&
+  if (STEP_BLOCKS > 0 && max_q_len == 1 && num_tokens == num_seqs && (nsplit == 1 || (uintptr_t)part_ml % 8 == 0) &&
       (long long)nkv * ((nh / nkv + 15) / 16) <= 65535) {              // (a token each)
     const char* e = launch_step(a, num_seqs, stream);
     if (e || nsplit == 1) return e;

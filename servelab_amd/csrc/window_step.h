@@ -135,9 +135,9 @@ __device__ __forceinline__ void finish_column(const WindowAttention& a, int t, i
 
 // columns are the heads of a kv head, 16 a workgroup; grid (shares, kv heads * tiles of columns, sequences)
 constexpr int STEP_WAVES = VK || DV <= 256 ? 4 : 2;
-constexpr int STEP_BLOCKS = VK ? 1 : STEP_WAVES;                       // classes of blocks a workgroup
+constexpr int STEP_BLOCKS = VK ? 1 : NARROW ? STEP_WAVES : 0;          // classes of blocks a workgroup
 
-#if !SL_VK
+#if !SL_VK && SL_NARROW
 // Keys and values go from the pages to the operands' registers; a wavefront takes blocks of its own and the four of a workgroup add up
 // what they have in LDS, so that a call has a quarter of the shares to merge.
 __global__ __launch_bounds__(64 * STEP_WAVES) void window_step_kernel(const WindowAttention a) {
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(64 * STEP_WAVES) void window_step_kernel(const Wind
     }
   }
 }
-#else
+#elif SL_VK
 // Values are channels of the key rows: a block is staged in LDS, as rows and turned, by the whole workgroup, whose wavefronts divide the
 // key channels of the scores among them (parts that meet in LDS) and the value channels of the weighted sum.
 constexpr int STEP_NT = cdiv((DV / 8) * 4, 256), STEP_NR = RCH ? cdiv(32 * RCH, 256) : 1;      // as NT, NR: for four wavefronts

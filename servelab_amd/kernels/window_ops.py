@@ -37,7 +37,8 @@ class WindowOps:
         return key
 
     def _window_step_blocks(self, Dk, Dv, in_keys):
-        """Blocks of 32 keys that a workgroup of a step of single tokens takes side by side."""
+        """Blocks of 32 keys that a workgroup of a step of single tokens takes side by side; 0 where such steps take
+        the kernel of prompts."""
         return self._lib[self._window_mfma_lib(Dk, Dv, in_keys)].sl_window_attention_mfma_step_blocks()
 
     def _lazy(self, stem):
@@ -245,10 +246,10 @@ class WindowOps:
             span = batch.max_ctx_len
             if window or chunk:
                 span = min(span, min(n for n in (window, chunk) if n) + int(keep_first))
-            if mfma and T == S:
+            blocks = self._window_step_blocks(Dk, Dv, v_cache is None) if mfma and T == S else 0
+            if blocks:
                 # a token each: shares of as many blocks as a workgroup takes side by side, a workgroup for every CU at most
                 columns = S * nkv * -(-(nh // nkv) // 16)
-                blocks = self._window_step_blocks(Dk, Dv, v_cache is None)
                 nsplit = max(1, min(self.WINDOW_MFMA_MAX_SHARES, -(-span // (32 * blocks)), self._num_cus // columns))
             elif mfma:
                 # a workgroup for every CU, a block of 32 keys a share at least
