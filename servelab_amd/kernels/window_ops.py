@@ -249,7 +249,7 @@ class WindowOps:
             blocks = self._window_step_blocks(Dk, Dv, v_cache is None) if mfma and T == S else 0
             if blocks:
                 # a token each: shares of as many blocks as a workgroup takes side by side, a workgroup for every CU at most
-                columns = S * nkv * -(-(nh // nkv) // 16)
+                columns = max(1, S * nkv * -(-(nh // nkv) // 16))
                 nsplit = max(1, min(self.WINDOW_MFMA_MAX_SHARES, -(-span // (32 * blocks)), self._num_cus // columns))
             elif mfma:
                 # a workgroup for every CU, a block of 32 keys a share at least

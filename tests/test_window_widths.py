@@ -1,12 +1,14 @@
 """The matrix-core window attention at wide heads whose values have pages of their own: every width it takes compiles into a workgroup that
-fits a CU (a static assertion of the source), and its kernels keep what a block needs in registers."""
+fits a CU (a static assertion of the source), and its kernels keep what a block needs in registers; shares of steps."""
 import os
 import re
 import subprocess
+from types import SimpleNamespace
 
 import pytest
+import torch
 
-from servelab_amd.kernels import build
+from servelab_amd.kernels import HipOps, build
 
 
 def spilled(Dk, Dv):
@@ -29,3 +31,34 @@ def spilled(Dk, Dv):
 def test_registers(Dk, Dv):
     found = spilled(Dk, Dv)
     assert max(found.values()) <= 25, found
+
+
+class Recorded(HipOps):
+    """The table's host side without a device: what it would launch is written down."""
+
+    def __init__(self):
+        self.act_dtype, self.device, self._num_cus, self.use_mfma_attention = torch.bfloat16, torch.device("cpu"), 256, True
+        self._fn, self._lib, self.shares = {"sl_window_attention_mfma@64.64.0": None}, {}, []
+
+    def _window_step_blocks(self, *a):
+        return 4
+
+    def _window_mfma_lib(self, *a):
+        return "window_attention_mfma"
+
+    def _check(self, *a, **k):
+        pass
+
+    def _call(self, stem, name, *a):
+        self.shares.append(a[-3])
+
+
+@pytest.mark.parametrize("S,shares", [(0, 32), (1, 32), (8, 16), (200, 1)])
+def test_shares_of_a_step(S, shares):
+    """A workgroup for every CU at most; a step without sequences is a call like any other."""
+    ops = Recorded()
+    batch = SimpleNamespace(cu_q=None, positions=None, num_seqs=S, num_tokens=S, max_q_len=1, max_ctx_len=4096)
+    pages = torch.zeros(1, 2, 16, 64, dtype=torch.bfloat16)
+    out = ops.window_attention(torch.zeros(S, 256, dtype=torch.bfloat16), 0, 4, 2, 64, 64, pages, pages, 16,
+                               torch.zeros(S, 256, dtype=torch.int32), batch, 1.0, None)
+    assert out.shape == (S, 256) and ops.shares == [shares]
