@@ -482,14 +482,16 @@ class ProductOps:
 
     def _bias_tiles(self, M, N, K) -> bool:
         """Whether a prompt's product with float32 results and a bias, which the library leaves to a second pass over
-        them, goes into the tiles: by their estimated rate, as in ``_prompt_tiles``.  us, library and pass / tiles: 6160 x
-        2048 at 1,000 / 2,048 rows 43 / 36 and 74 / 56, 7168 x 3584 at 1,500 / 1,852 85 / 72 and 98 / 91, 10304 x 2048 at 600 / 1,500 46 / 38
-        and 81 / 64; of 33 sizes the slowest 10792 x 3584 at 1,500, 123 / 130; below the rate 6160 x 2048 at 600 33 / 36, 4096 x 2048
-        at 1,000 29 / 34."""
-        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 4
-                or not self.GATED_MIN_M <= M <= self.GATED_MAX_M or K > self.PROMPT_MAX_K):
+        them, goes into the tiles: by their estimated rate, from BIAS_MIN_TFLOPS on.  Of 92 products of twelve matrices at 300 to 2,500
+        rows the tiles take 0.87 of the pair's time where this says so, 0.99 at worst (us, library and pass / tiles: 6160 x 2048 at
+        1,000 / 2,048 rows 44 / 37 and 75 / 58, 7168 x 3584 at 1,500 / 1,852 85 / 73 and 101 / 92, 10304 x 2048 at 600 / 1,500 44 / 37 and 82 /
+        65).  The longer the rows, the less the pass is beside the product, and the higher the line: at 750 and more, but below it,
+        10792 x 3584 at 1,500 123 / 133 and 7168 x 3584 at 2,500 134 / 137, 5120 x 5120 at 1,000 62 / 66, 14336 x 4096 at 1,280 148 / 153; 6160 x 2048 at
+        768 35 / 37.  (Whether the shape was tuned is not asked: ``library_tuning`` times no product with float32 results.)"""
+        if (self.act_dtype != torch.bfloat16 or not self.use_block_products or K % 64 or N % 4 or M < self.GATED_MIN_M):
             return False
-        return 2e-6 * M * N * K >= self.PROMPT_MIN_TFLOPS * self._tiles_us(self._tile_rows(M, N, K), M, N, K)
+        least = next((rate for values, rows, rate in self.BIAS_MIN_TFLOPS if K <= values and M <= rows), None)
+        return least is not None and 2e-6 * M * N * K >= least * self._tiles_us(self._tile_rows(M, N, K), M, N, K)
 
     def _tuned_for(self, M, N, K) -> bool:
         """Whether the library's product of this shape has been timed over its candidates (``library_tuning``; inside

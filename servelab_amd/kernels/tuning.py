@@ -115,6 +115,8 @@ class Tuning:
     prompt_min_tflops: float = 750.0
     # ... at this one also where the library's product of the shape was tuned (HipOps._tiles_beat_tuned) ...
     prompt_tuned_tflops: float = 1000.0
+    # ... products with float32 results and a bias (HipOps._bias_tiles): (values a row up to which, rows of x up to which, least rate)
+    bias_min_tflops: tuple = ((2048, 2560, 750.0), (3584, 2048, 950.0), (8192, 2560, 1120.0))
     # ... longer ones, up to gated_long_k values and for so many rows of x, in several rounds, the last filled so far
     gated_long_k: int = 5120
     gated_long_rows: tuple = (1537, 2048)

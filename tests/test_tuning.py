@@ -45,3 +45,14 @@ def test_shapes_among_the_library_tuner_s_results():
                ("GemmTunableOp_BFloat16_NN", "nn_64_64_64_ld_64_64_64", "Gemm_Hipblaslt_2", 0.01),
                ("GemmTunableOp_float_TN", "tn_8_8_8_ld_8_8_8", "Gemm_Rocblas_3", 0.01))
     assert tuned_shapes(results) == {(700, 16384, 2048), (32, 96, 64)} and tuned_shapes(()) == set()
+
+
+# (us measured, the library's product and its pass for the bias / the tiles, beside each)
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (1000, 6160, 2048, True), (600, 10304, 2048, True), (1500, 4096, 2048, True),              # 44 / 37, 44 / 37, 37 / 36
+    (1500, 7168, 3584, True), (1280, 10792, 3584, True), (2048, 14336, 4096, True),            # 85 / 73, 104 / 88, 218 / 198
+    (1500, 10792, 3584, False), (2500, 7168, 3584, False), (1000, 5120, 5120, False),          # 123 / 133, 134 / 137, 62 / 66
+    (1280, 14336, 4096, False), (2500, 14336, 4096, False), (768, 6160, 2048, False)])         # 148 / 153, 280 / 295, 35 / 37
+def test_products_with_a_bias_take_tiles_where_these_are_faster(M, N, K, tiles):
+    from test_qkv_shapes import Recorded
+    assert Recorded()._bias_tiles(M, N, K) is tiles
