@@ -67,12 +67,18 @@ struct __attribute__((aligned(16))) a4 { act_t v[4]; };
 struct __attribute__((aligned(8))) a4 { act_t v[4]; };
 #endif
 
+// The most threads of a workgroup whose threads have ITERS groups of four values each (``row_threads``).  Eight groups, more than 256 rows of more
+// than 8,192 values: no more than 512 threads share the register file, and the gains are asked for behind the sums, so that two workgroups fit a CU
+// (2,048 rows of 10,240 values, us: two partial sums 94 with room for 1,024 threads and gains in registers, which spilled, now 65; layer norm 50, now 41; of
+// 16,384 values, layer norm 111, now 69; float32 181, now 93).
+constexpr int row_most(int iters) { return iters > 4 ? 512 : 1024; }
+
 // A step of few rows is one trip to memory and one sum, so all that a row needs is asked for at once, PARTS partial sums a trip (0: there are
 // none), and no load stands behind a condition, which would be waited for where the ways meet (an absent delta is read from the stream
 // and left out); the stream's new row is written behind the sum.  64 rows of 3,584 values
 // with eight partial sums: 5.2 us with the loads in turn, 4.9 here, 2,048 with two: 23.0, now 22.5.
 template <int ITERS, int PARTS>
-__global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ delta,
+__global__ __launch_bounds__(row_most(ITERS), 4) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ delta,
                                        const SplitDelta sd, const int* __restrict__ rows,
                                        const float* __restrict__ w, act_t* __restrict__ out, int H,
                                        float eps) {
@@ -91,7 +97,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
   for (int it = 0; it < ITERS; ++it) {
     v[it] = ((const f4*)x)[group(it)];
     if (PARTS == 0) dv[it] = ((const a4*)d)[group(it)];
-    wv[it] = ((const f4*)w)[group(it)];
+    if (ITERS <= 4) wv[it] = ((const f4*)w)[group(it)];
   }
   auto ask = [&](int q0) {
 #pragma unroll
@@ -143,6 +149,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
     const int i = threadIdx.x + it * blockDim.x;
     if (i < H4) {
       a4 ov;
+      if (ITERS > 4) wv[it] = ((const f4*)w)[i];
 #pragma unroll
       for (int j = 0; j < 4; ++j) ov.v[j] = from_f<act_t>(v[it].v[j] * inv * wv[it].v[j]);
       if (store) ((f4*)x)[i] = v[it];
@@ -253,7 +260,7 @@ __global__ void add_layernorm_kernel(float* __restrict__ resid, const act_t* __r
 // and the output.
 // All of it is asked for at once, as above, and the stream's new row is written behind the sums (4 rows of 2,048 values: 2.8 us before, 2.5 here).
 template <int ITERS>
-__global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ d1,
+__global__ __launch_bounds__(row_most(ITERS)) void add_layernorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ d1,
                                          const act_t* __restrict__ d2, const int* __restrict__ rows,
                                          const float* __restrict__ w, const float* __restrict__ bias,
                                          act_t* __restrict__ out, int H, float eps) {
@@ -273,8 +280,10 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     v[it] = ((const f4*)x)[i];
     av[it] = ((const a4*)a)[i];
     cv[it] = ((const a4*)b)[i];
-    wv[it] = ((const f4*)w)[i];
-    bv[it] = ((const f4*)add)[i];
+    if (ITERS <= 4) {
+      wv[it] = ((const f4*)w)[i];
+      bv[it] = ((const f4*)add)[i];
+    }
   }
   float sum = 0.f;
 #pragma unroll
@@ -306,6 +315,10 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     const int i = threadIdx.x + it * blockDim.x;
     if (i < H4) {
       a4 ov;
+      if (ITERS > 4) {
+        wv[it] = ((const f4*)w)[i];
+        bv[it] = ((const f4*)add)[i];
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         ov.v[j] = from_f<act_t>((v[it].v[j] - mean) * inv * wv[it].v[j] + (bias != nullptr ? bv[it].v[j] : 0.f));
@@ -625,7 +638,7 @@ __global__ void add_postnorm_kernel(float* __restrict__ resid, const act_t* __re
 // The same for rows of up to 4 * 8 * 512 values that are a multiple of 4 wide, 16-byte loads (8 rows of 3,584 values: 2.5 us with single
 // ones, 2.1 here; one of 2,048 2.1, now 1.7).
 template <int ITERS>
-__global__ __launch_bounds__(1024) void add_postnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
+__global__ __launch_bounds__(row_most(ITERS)) void add_postnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
                                                                 const float* __restrict__ w, act_t* __restrict__ out, int H, float eps,
                                                                 float mult) {
   __shared__ float scratch[16];
@@ -758,7 +771,7 @@ __global__ void add_normed_rmsnorm_kernel(float* __restrict__ resid, const act_t
 
 // The same with 16-byte loads, as above; the stream's new row is written behind both sums (2 rows of 2,048 values: 3.0 us, now 2.1).
 template <int ITERS>
-__global__ __launch_bounds__(1024) void add_normed_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
+__global__ __launch_bounds__(row_most(ITERS)) void add_normed_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ y,
                                                                       const float* __restrict__ wy, float eps_y,
                                                                       const int* __restrict__ rows, const float* __restrict__ w, float eps,
                                                                       act_t* __restrict__ out, int H) {

@@ -11,11 +11,11 @@ import torch
 from servelab_amd.kernels import HipOps, build
 
 
-def spilled(Dk, Dv):
+def spilled(source, *defines):
     """Vector registers that each kernel of the library spills."""
     flags = [f for f in build.BASE_FLAGS if f not in ("-shared", "-fPIC")]
-    out = subprocess.run([build.hipcc()] + flags + [f"-DSL_DK={Dk}", f"-DSL_DV={Dv}", "-DSL_VK=0", "--cuda-device-only", "-S", "-o", os.devnull,
-                          "-Rpass-analysis=kernel-resource-usage", os.path.join(build.CSRC, "window_attention_mfma.hip")],
+    out = subprocess.run([build.hipcc()] + flags + ["-D" + d for d in defines] + ["--cuda-device-only", "-S", "-o", os.devnull,
+                          "-Rpass-analysis=kernel-resource-usage", os.path.join(build.CSRC, source)],
                          check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True).stdout
     names = re.findall(r"Function Name: (\S+)", out)
     counts = [int(n) for n in re.findall(r"VGPRs Spill: (\d+)", out)]
@@ -29,7 +29,7 @@ def spilled(Dk, Dv):
 @pytest.mark.parametrize("Dk,Dv", [(512, 256), (192, 512), (704, 256), (1024, 96), (896, 16), (256, 512), (512, 384), (1024, 112), (512, 512),
                                    (544, 512), (640, 512), (1024, 512)])
 def test_registers(Dk, Dv):
-    found = spilled(Dk, Dv)
+    found = spilled("window_attention_mfma.hip", f"SL_DK={Dk}", f"SL_DV={Dv}", "SL_VK=0")
     assert max(found.values()) <= 25, found
 
 
