@@ -754,7 +754,7 @@ extern "C" const char* sl_gemm_skinny(const void* x, const void* wt, const float
   else if (wide && tiles == 1) launch_few_rows<true, 1, 4>(A, gated, rp, stream);
   else if (wide && pairs > 4) launch_few_rows<true, 0, 2>(A, gated, rp, stream);
   else if (wide) launch_few_rows<true, 0, 4>(A, gated, rp, stream);
-  else if (tiles == 0 && pairs > 8 && pairs <= 10) launch_few_rows<false, 0, 10>(A, gated, rp, stream);
+  else if (tiles == 0 && pairs > 8 && K <= (producer ? 4864 : 5056)) launch_few_rows<false, 0, 10>(A, gated, rp, stream);
   else if (tiles == 0 && pairs > 4 && pairs <= 8) launch_few_rows<false, 0, 8>(A, gated, rp, stream);
   else if (tiles == 0) launch_few_rows<false, 0, 4>(A, gated, rp, stream);
   else if (pairs > 4 && !consumer) launch_few_rows<false, 1, 8>(A, gated, rp, stream);

@@ -316,8 +316,11 @@ __global__ __launch_bounds__(64 * WAVES, TILES == 2 && CONSUMER && !ROPE && PART
 // TILES: 0 half a tile a workgroup, 1, 2.  U: pairs of k-steps asked for together.  One tile and 9 to 16 rows: four, and three where there are
 // more than two tiles a CU, so that no more than 80 registers (of consumers of up to 4,096 values and of plain rows) leave room for three
 // workgroups, all tiles at once: 12288 x 1024 7.6 to 9.5 us with four, 6.6 to 7.9 with three, 9728 x 896 6.8 to 8.0 and 5.7 to 6.8; 2048 x 2048, whose
-// wavefronts have four pairs, 5.2 and 5.5.  Halves: 9 or 10 pairs in one trip, 896 x 4864 at one row 4.8 us in fours and 4.5; 9 to 16 rows and
-// more than four pairs, in twos (896 x 4864 at 9 / 16 rows 6.4 / 8.0 in fours and 6.3 / 7.5, 2048 x 11008 11.8 / 15.2 and 11.5 / 14.8).
+// wavefronts have four pairs, 5.2 and 5.5.  Halves: 9 or 10 pairs in one trip, in fours / tens at one row and
+// at 8: 896 x 4224 4.5 / 4.0 and 5.6 / 5.2, 1536 x 4864 5.0 / 4.7 and 6.1 / 5.9, 2048 x 4864 5.8 / 5.5 and 6.4 / 6.2, 2048 x 5056 5.9 / 5.8 and 6.4 / 6.5,
+// 2048 x 5120, ten pairs for every wavefront, 5.6 / 5.5 and 6.5 / 6.7; products that add to the stream 1536 x 4864 5.3 / 5.1 and 6.3 / 6.2, 2048 x 4864
+// 6.0 / 5.9 and 6.6 / 6.5, 2048 x 4992 6.2 / 6.2 and 6.6 / 6.9, 2048 x 5120 5.9 / 6.2 and 6.8 / 7.2.  9 to 16 rows and more than four pairs, in twos (in
+// fours / twos at 9 and 16 rows: 896 x 4864 6.3 / 6.2 and 8.0 / 7.5, 2048 x 3072 5.2 / 5.2 and 6.3 / 5.9, 1536 x 8960 11.4 / 11.3 and 13.1 / 12.8).
 template <bool WIDE, int TILES, int U>
 static void launch_few_rows(const FewRows& A, bool gated, bool rope, hipStream_t stream) {
   const bool consumer = A.F.in_parts != nullptr, producer = A.F.resid != nullptr, few = A.F.in_nparts <= 32 * 8;
