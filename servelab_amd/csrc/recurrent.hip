@@ -1295,8 +1295,8 @@ __global__ void projnorm_rope_store_kernel(const float* __restrict__ buf, int st
       vc[((pg * G + e / Dv) * Dv + e % Dv) * page + off] = from_f<act_t>(row[v_col + e]);
 }
 
-// The same for a step of few tokens and rows of at most 4,096 values of q and k and 1,024 of v: what a thread needs is asked for before the
-// first sum (its four values of the row, their gains and their partners', angles, its value of v), and both sums meet at once.  One
+// The same for a step of few tokens with a norm over the projection and rows of at most 4,096 values of q and k and 1,024 of v: what a
+// thread needs is asked for before the first sum (its four values of the row, their gains and their partners', angles, its value of v), and both sums meet at once.  One
 // token, 16 heads on 2 of 128: 4.9 us, now 4.3; behind a convolution of four taps 8.4, now 5.3. A prompt's 1,500 tokens take 35 us in
 // this form behind a convolution, 30 in the one above.
 template <bool CONV>
@@ -1313,8 +1313,7 @@ __global__ __launch_bounds__(1024) void projnorm_step_kernel(const float* __rest
   const size_t t = blockIdx.x;
   const int tid = threadIdx.x, nq = H * D, nqk = nq + G * D, nv = G * Dv, half = rot / 2;
   const float* row = buf + t * stride;
-  const bool normed = qw != nullptr;
-  const float *gq = normed ? qw : row, *gk = normed && nqk > nq ? kw : gq;
+  const float *gq = qw, *gk = nqk > nq ? kw : gq;
   float x[4], w[4], wp[4], cs[4], sn[4], v = 0.f;
   auto gain = [&](int e) { return (e < nq ? gq : gk - nq)[e]; };
 #pragma unroll
@@ -1379,7 +1378,7 @@ __global__ __launch_bounds__(1024) void projnorm_step_kernel(const float* __rest
     sq += of_q[i];
     sk += of_k[i];
   }
-  const float iq = normed ? 1.f / sqrtf(sq / (float)nq + eps) : 1.f, ik = normed ? 1.f / sqrtf(sk / (float)max(1, nqk - nq) + eps) : 1.f;
+  const float iq = 1.f / sqrtf(sq / (float)nq + eps), ik = 1.f / sqrtf(sk / (float)max(1, nqk - nq) + eps);
   const int pg_int = lg_page >= 0 ? slot >> lg_page : slot / page, off = slot - pg_int * page;
   const size_t pg = pg_int;
 #pragma unroll
@@ -1387,9 +1386,9 @@ __global__ __launch_bounds__(1024) void projnorm_step_kernel(const float* __rest
     const int e = tid + 1024 * u, d = e - over_D(e) * D;
     if (e >= nqk) break;
     const float inv = e < nq ? iq : ik;
-    float r = normed ? x[u] * inv * w[u] : x[u];
+    float r = x[u] * inv * w[u];
     if (d < rot) {
-      const float other = xs[d < half ? e + half : e - half], o = normed ? other * inv * wp[u] : other;
+      const float o = xs[d < half ? e + half : e - half] * inv * wp[u];
       r = d < half ? r * cs[u] - o * sn[u] : r * cs[u] + o * sn[u];
     }
     if (e < nq) q_out[t * nq + e] = from_f<act_t>(r);
@@ -1523,7 +1522,7 @@ extern "C" const char* sl_projnorm_rope_store(const float* buf, int stride, int 
       kernel<<<T, 1024, room, stream>>>(buf, stride, H, G, D, Dv, qw, kw, eps, rot, cosv, sinv, slots, (act_t*)kc, (act_t*)vc, page,
                                         (act_t*)q_out, v_col, lg(D), lg(Dv), lg(page), cv);
     };
-    if (T <= 64 && nqk <= 4096 && (long long)G * Dv <= 1024) {
+    if (T <= 64 && qw != nullptr && nqk <= 4096 && (long long)G * Dv <= 1024) {
       if (taps_w != nullptr) step(projnorm_step_kernel<true>, lds);
       else step(projnorm_step_kernel<false>, nqk * sizeof(float));
     } else projnorm_rope_store_kernel<<<T, T <= 64 ? 1024 : 256, lds, stream>>>(buf, stride, H, G, D, Dv, qw, kw, eps, rot, cosv, sinv, slots,

@@ -41,7 +41,7 @@ def test_norms_of_heads_and_slices(n, dtype):
 
 # steps of 64 tokens and 65; rows of 4,096 values of q and k and above, of 1,024 of v and above; sizes that are no powers of two; no keys of
 # their own; alone, and behind a convolution of four taps (its row of up to 4,096 channels, and above), of three, of one; single tokens,
-# whose slots move on in the launch, and longer ones
+# whose slots move on in the launch, and longer ones.  (Without a norm: the kernel of a wavefront a head.)
 @pytest.mark.parametrize("T,H,G,D,Dv", [(1, 16, 2, 128, 128), (64, 2, 1, 16, 8), (65, 2, 1, 16, 8), (3, 31, 1, 128, 24), (2, 30, 3, 128, 40),
                                         (5, 5, 3, 20, 341), (4, 5, 3, 20, 342), (3, 24, 8, 96, 128), (2, 3, 2, 9, 7)])
 @pytest.mark.parametrize("taps", [0, 1, 3, 4])
