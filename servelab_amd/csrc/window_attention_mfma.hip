@@ -117,7 +117,7 @@ constexpr bool PLACES_ANEW = !VK && (TEAMS == 2 ? 4 * DK + 5 * DV > 3328 : DK + 
 // prompt's, and with BY_LENGTH all of these are one die's: a prompt of 500 tokens among 31 decoding, 16 heads on 1, 576 / 512:
 // 720 us, 127 in this order; prompts of 1,200, 300, 100 and 20 tokens 413 us, 467 moved, 195; of 1,200 and three of
 // 1,000 410 moved, 463 with early tiles first.)
-enum { IN_ORDER = 0, LATE_FIRST = 1, BY_LENGTH = 2, BY_LENGTH_MOVED = 3 };
+enum { LATE_FIRST, BY_LENGTH, BY_LENGTH_MOVED };
 
 __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK && DK <= 128 && DV <= 128 ? 4 : 2) void window_attention_mfma_kernel(const WindowAttention a, int order) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
@@ -128,10 +128,8 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
   const int tid = threadIdx.x % THREADS, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, n = lane & 15, gq = lane >> 4;
   const int part = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
   const int page = a.page, nkv = a.nkv;
-  int seq = blockIdx.z, kvh = blockIdx.y, item = blockIdx.x;
-  if (order == LATE_FIRST) {
-    item = gridDim.x - 1 - blockIdx.x;
-  } else if (order == BY_LENGTH) {                     // (launched with the heads along x and the tiles along z)
+  int seq = blockIdx.z, kvh = blockIdx.y, item = gridDim.x - 1 - blockIdx.x;
+  if (order == BY_LENGTH) {                     // (launched with the heads along x and the tiles along z)
     seq = blockIdx.y;
     kvh = blockIdx.x;
     item = gridDim.z - 1 - blockIdx.z;

@@ -75,6 +75,28 @@ def test_steps_of_one_token(H, G, Dk, Dv, in_keys, window, keep, chunk, page, sh
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -12 * want.abs().max() + 1e-5).all(), float((got - want).abs().max())
 
 
+@pytest.mark.parametrize("H,G,Dk,Dv,in_keys", [(20, 1, 64, 80, False), (8, 2, 128, 128, False), (3, 1, 64, 48, True), (17, 1, 512, 384, False)])
+@pytest.mark.parametrize("shares", [1, 3, 32])
+def test_a_sequence_without_a_token(H, G, Dk, Dv, in_keys, shares):
+    """Two tokens of three sequences: the kernel of prompts, over shares of the keys."""
+    ops, page, lens = HipOps(torch.bfloat16, "cuda:0"), 16, [300, 40, 75]
+    ops.WINDOW_MFMA_MAX_SHARES = shares
+    gen = torch.Generator().manual_seed(Dk)
+    tables, kc, vc = paged(lens, page, G, Dk, 0 if in_keys else Dv, torch.bfloat16, gen)
+    keys = [torch.randn(n, G, Dk, generator=gen).bfloat16() for n in lens]
+    values = [k[..., :Dv] for k in keys] if in_keys else [torch.randn(n, G, Dv, generator=gen).bfloat16() for n in lens]
+    fill_pages(tables, kc, vc, keys, None if in_keys else values, page)
+    q, sinks = torch.randn(2, H * Dk, generator=gen).bfloat16(), torch.randn(H, generator=gen)
+    i32 = lambda v: dev(torch.tensor(v, dtype=torch.int32))
+    batch = SimpleNamespace(cu_q=i32([0, 1, 1, 2]), positions=i32([299, 74]), num_seqs=3, num_tokens=2, max_q_len=1, max_ctx_len=300)
+    got = ops.window_attention(dev(q), 0, H, G, Dk, Dv, dev(kc), None if in_keys else dev(vc), page, dev(tables), batch, Dk ** -0.5, None, 0, None,
+                               dev(sinks)).view(2, H, Dv).double().cpu()
+    want = torch.stack([exact(q[i].view(H, Dk), keys[s], values[s], lens[s] - 1, Dk ** -0.5, None, 0, None, None, None, sinks)[0]
+                        for i, s in enumerate((0, 2))])
+    # results of a few units rounded to bfloat16 (2^-9 of the value); scores, weights and sums are float32
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -12 * want.abs().max() + 1e-5).all(), float((got - want).abs().max())
+
+
 @pytest.mark.parametrize("shares", [1, 2, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("Dv", [16, 64, 80])
 def test_merging_of_shares(shares, Dv):
