@@ -85,6 +85,30 @@ __device__ __forceinline__ float column_sum4(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// p = p1 + p2 + p3 exactly: each term is the upper 16 bits (a bfloat16) of what the terms before left over, 8 bits of significand a
+// term; two terms of neighbouring keys share a register.
+__device__ __forceinline__ void three_terms(const float (&p)[8], bf16x8& p1, bf16x8& p2, bf16x8& p3) {
+  u32x4 w1, w2, w3;
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    unsigned t1[2], t2[2], t3[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float x = p[j + e];
+      t1[e] = __float_as_uint(x) & 0xffff0000u;
+      const float r1 = x - __uint_as_float(t1[e]);
+      t2[e] = __float_as_uint(r1) & 0xffff0000u;
+      t3[e] = __float_as_uint(r1 - __uint_as_float(t2[e]));
+    }
+    w1[j / 2] = __builtin_amdgcn_perm(t1[1], t1[0], 0x07060302u);
+    w2[j / 2] = __builtin_amdgcn_perm(t2[1], t2[0], 0x07060302u);
+    w3[j / 2] = __builtin_amdgcn_perm(t3[1], t3[0], 0x07060302u);
+  }
+  p1 = __builtin_bit_cast(bf16x8, w1);
+  p2 = __builtin_bit_cast(bf16x8, w2);
+  p3 = __builtin_bit_cast(bf16x8, w3);
+}
+
 // A prompt's workgroup is eight wavefronts over 64 columns: two teams of four that take every other block and meet at the end, or,
 // where values lie in the key rows, one whose wavefronts share their 16 columns two and two, each with half of the channels.
 constexpr int TEAMS = VK || !NARROW ? 1 : 2, PARTS = VK ? 2 : 1;
@@ -396,26 +420,8 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
       m = mn;
     }
     l += column_sum4(psum);
-    // p = p1 + p2 + p3 exactly: each term is the upper 16 bits (a bfloat16) of what the terms before left
-    // over, 8 bits of significand a term; two terms of neighbouring keys share a register
-    u32x4 w1, w2, w3;
-#pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      unsigned t1[2], t2[2], t3[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float x = p[j + e];
-        t1[e] = __float_as_uint(x) & 0xffff0000u;
-        const float r1 = x - __uint_as_float(t1[e]);
-        t2[e] = __float_as_uint(r1) & 0xffff0000u;
-        t3[e] = __float_as_uint(r1 - __uint_as_float(t2[e]));
-      }
-      w1[j / 2] = __builtin_amdgcn_perm(t1[1], t1[0], 0x07060302u);
-      w2[j / 2] = __builtin_amdgcn_perm(t2[1], t2[0], 0x07060302u);
-      w3[j / 2] = __builtin_amdgcn_perm(t3[1], t3[0], 0x07060302u);
-    }
-    const bf16x8 p1 = __builtin_bit_cast(bf16x8, w1), p2 = __builtin_bit_cast(bf16x8, w2),
-                 p3 = __builtin_bit_cast(bf16x8, w3);
+    bf16x8 p1, p2, p3;
+    three_terms(p, p1, p2, p3);
     // (four tiles of channels side by side: the three products of one depend on each other)
     constexpr int SIDE = DDP % 4 == 0 && DD % PARTS == 0 ? 4 : 1;
 #pragma unroll

@@ -33,29 +33,6 @@ struct StepBlocks {
   }
 };
 
-// p = p1 + p2 + p3 exactly, two terms of neighbouring keys a register (see the kernel of prompts)
-__device__ __forceinline__ void three_terms(const float (&p)[8], bf16x8& p1, bf16x8& p2, bf16x8& p3) {
-  u32x4 w1, w2, w3;
-#pragma unroll
-  for (int j = 0; j < 8; j += 2) {
-    unsigned t1[2], t2[2], t3[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const float x = p[j + e];
-      t1[e] = __float_as_uint(x) & 0xffff0000u;
-      const float r1 = x - __uint_as_float(t1[e]);
-      t2[e] = __float_as_uint(r1) & 0xffff0000u;
-      t3[e] = __float_as_uint(r1 - __uint_as_float(t2[e]));
-    }
-    w1[j / 2] = __builtin_amdgcn_perm(t1[1], t1[0], 0x07060302u);
-    w2[j / 2] = __builtin_amdgcn_perm(t2[1], t2[0], 0x07060302u);
-    w3[j / 2] = __builtin_amdgcn_perm(t3[1], t3[0], 0x07060302u);
-  }
-  p1 = __builtin_bit_cast(bf16x8, w1);
-  p2 = __builtin_bit_cast(bf16x8, w2);
-  p3 = __builtin_bit_cast(bf16x8, w3);
-}
-
 // One column's softmax over the blocks it has seen: this lane's 8 keys of a block, from the raw scores s0 (keys 8 gq .. + 3) and s1.
 struct StepColumn {
   float scale2, cap2, uncap, slope2, m, l;
