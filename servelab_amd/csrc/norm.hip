@@ -73,9 +73,8 @@ struct __attribute__((aligned(8))) a4 { act_t v[4]; };
 // 16,384 values, layer norm 111, now 69; float32 181, now 93).
 constexpr int row_most(int iters) { return iters > 4 ? 512 : 1024; }
 
-// A step of few rows is one trip to memory and one sum, so all that a row needs is asked for at once, PARTS partial sums a trip (0: there are
-// none), and no load stands behind a condition, which would be waited for where the ways meet (an absent delta is read from the stream
-// and left out); the stream's new row is written behind the sum.  64 rows of 3,584 values
+// A step of few rows is one trip to memory and one sum, so all that a row needs is asked for at once, PARTS partial sums a trip (0: a
+// delta instead, -1: neither), and no load stands behind a condition, which would be waited for where the ways meet; the stream's new row is written behind the sum.  64 rows of 3,584 values
 // with eight partial sums: 5.2 us with the loads in turn, 4.9 here, 2,048 with two: 23.0, now 22.5.
 template <int ITERS, int PARTS>
 __global__ __launch_bounds__(row_most(ITERS), 4) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const act_t* __restrict__ delta,
@@ -87,7 +86,7 @@ __global__ __launch_bounds__(row_most(ITERS), 4) void add_rmsnorm_vec_kernel(flo
   const size_t src = rows != nullptr ? (size_t)rows[r] : (size_t)r;
   float* x = resid + src * H;
   const bool plain = delta != nullptr;
-  const act_t* d = plain ? delta + src * H : (const act_t*)x;
+  const act_t* d = delta + src * H;
   const float* p = sd.parts + src * H;
   const int H4 = H / 4;
   f4 v[ITERS], wv[ITERS], pv[PARTS > 0 ? PARTS : 1][ITERS];
@@ -120,7 +119,7 @@ __global__ __launch_bounds__(row_most(ITERS), 4) void add_rmsnorm_vec_kernel(flo
 #pragma unroll
   for (int it = 0; it < ITERS; ++it)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[it].v[j] += plain ? to_f(dv[it].v[j]) : 0.f;
+    for (int j = 0; j < 4; ++j) v[it].v[j] += PARTS == 0 || (PARTS > 0 && plain) ? to_f(dv[it].v[j]) : 0.f;
   add(0);
   if (PARTS > 0) {
     for (int q0 = PARTS; q0 < sd.nparts; q0 += PARTS) {
@@ -143,7 +142,7 @@ __global__ __launch_bounds__(row_most(ITERS), 4) void add_rmsnorm_vec_kernel(flo
   ss = block_sum(ss, scratch);
   const float inv = rsqrtf(ss / (float)H + eps);
   act_t* o = out + (size_t)r * H;
-  const bool store = (plain || PARTS > 0) && rows == nullptr;
+  const bool store = PARTS >= 0 && rows == nullptr;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int i = threadIdx.x + it * blockDim.x;
@@ -164,6 +163,17 @@ __global__ __launch_bounds__(row_most(ITERS), 4) void add_rmsnorm_vec_kernel(flo
 static int row_threads(int R, int n) {
   const int most = R <= 256 ? 1024 : 512, turns = (n + most - 1) / most;
   return ((n + turns - 1) / turns + 63) / 64 * 64;
+}
+// Calls f with the number of groups a thread has in a kernel for it (a group that no thread of a workgroup has is read all the same: 700 rows of
+// 5,120 values, three groups, 8.1 us in the kernel for four, 7.3 in one for three; 257 rows with eight partial sums 12.5 and 11.9).
+template <int N> struct Groups { static constexpr int n = N; };
+template <class F> static void with_groups(int n, F f) {
+  if (n <= 1) f(Groups<1>{});
+  else if (n == 2) f(Groups<2>{});
+  else if (n == 3) f(Groups<3>{});
+  else if (n == 4) f(Groups<4>{});
+  else if (n <= 6) f(Groups<6>{});
+  else f(Groups<8>{});
 }
 
 // parts != nullptr: nparts float partial sums [nparts][T][H] (T rows in each)
@@ -186,22 +196,18 @@ extern "C" const char* sl_add_rmsnorm(float* resid, const void* delta, const flo
     act_t* o = (act_t*)out;
     auto run = [&](auto kernel) { kernel<<<R, threads, 0, stream>>>(resid, dl, sd, rows, w, o, H, eps); };
     // (as many partial sums a trip as there are: reading one again in place of one that is not there costs many rows what it saves few)
-    if (parts == nullptr) {
-      if (iters == 1) run(add_rmsnorm_vec_kernel<1, 0>);
-      else if (iters == 2) run(add_rmsnorm_vec_kernel<2, 0>);
-      else if (iters <= 4) run(add_rmsnorm_vec_kernel<4, 0>);
-      else run(add_rmsnorm_vec_kernel<8, 0>);
-    } else if (iters == 1) {
-      if (nparts <= 2) run(add_rmsnorm_vec_kernel<1, 2>);
-      else if (nparts == 3) run(add_rmsnorm_vec_kernel<1, 3>);
-      else if (nparts == 4) run(add_rmsnorm_vec_kernel<1, 4>);
-      else run(add_rmsnorm_vec_kernel<1, 8>);
-    } else if (iters == 2) {
-      if (nparts <= 2) run(add_rmsnorm_vec_kernel<2, 2>);
-      else if (nparts == 3) run(add_rmsnorm_vec_kernel<2, 3>);
-      else run(add_rmsnorm_vec_kernel<2, 4>);
-    } else if (iters <= 4) run(add_rmsnorm_vec_kernel<4, 2>);
-    else run(add_rmsnorm_vec_kernel<8, 1>);
+    with_groups(iters, [&](auto groups) {
+      constexpr int N = decltype(groups)::n;
+      if (parts == nullptr && delta == nullptr) run(add_rmsnorm_vec_kernel<N, -1>);
+      else if (parts == nullptr) run(add_rmsnorm_vec_kernel<N, 0>);
+      else if constexpr (N > 4) run(add_rmsnorm_vec_kernel<N, 1>);
+      else if (N > 2 || nparts <= 2) run(add_rmsnorm_vec_kernel<N, 2>);
+      else if constexpr (N <= 2) {
+        if (nparts == 3) run(add_rmsnorm_vec_kernel<N, 3>);
+        else if (N == 2 || nparts == 4) run(add_rmsnorm_vec_kernel<N, 4>);
+        else run(add_rmsnorm_vec_kernel<N, 8>);
+      }
+    });
     return sl_launch_status();
   }
   const int threads = H >= 2048 ? 512 : 256;
@@ -341,10 +347,9 @@ extern "C" const char* sl_add_layernorm(float* resid, const void* d1, const void
     const act_t* a = (const act_t*)d1;
     const act_t* b = (const act_t*)d2;
     act_t* o = (act_t*)out;
-    if (iters == 1) add_layernorm_vec_kernel<1><<<R, nthreads, 0, stream>>>(resid, a, b, rows, w, bias, o, H, eps);
-    else if (iters == 2) add_layernorm_vec_kernel<2><<<R, nthreads, 0, stream>>>(resid, a, b, rows, w, bias, o, H, eps);
-    else if (iters <= 4) add_layernorm_vec_kernel<4><<<R, nthreads, 0, stream>>>(resid, a, b, rows, w, bias, o, H, eps);
-    else add_layernorm_vec_kernel<8><<<R, nthreads, 0, stream>>>(resid, a, b, rows, w, bias, o, H, eps);
+    with_groups(iters, [&](auto groups) {
+      add_layernorm_vec_kernel<decltype(groups)::n><<<R, nthreads, 0, stream>>>(resid, a, b, rows, w, bias, o, H, eps);
+    });
     return sl_launch_status();
   }
   const int threads = H >= 2048 ? 512 : 256;
@@ -536,10 +541,7 @@ static const char* launch_streams_norm(const StreamsNorm& a, int R, hipStream_t 
   const uintptr_t acts = (uintptr_t)a.y1 | (uintptr_t)a.y2 | (uintptr_t)a.o;
   if (a.H % 4 == 0 && a.H <= 4 * 8 * 512 && f32s % 16 == 0 && acts % (4 * sizeof(act_t)) == 0) {
     const int H4 = a.H / 4, threads = row_threads(R, H4), iters = (H4 + threads - 1) / threads;
-    if (iters == 1) streams_norm_kernel<MAXS, EXACT, 4, 1><<<R, threads, 0, stream>>>(a);
-    else if (iters == 2) streams_norm_kernel<MAXS, EXACT, 4, 2><<<R, threads, 0, stream>>>(a);
-    else if (iters <= 4) streams_norm_kernel<MAXS, EXACT, 4, 4><<<R, threads, 0, stream>>>(a);
-    else streams_norm_kernel<MAXS, EXACT, 4, 8><<<R, threads, 0, stream>>>(a);
+    with_groups(iters, [&](auto groups) { streams_norm_kernel<MAXS, EXACT, 4, decltype(groups)::n><<<R, threads, 0, stream>>>(a); });
     return sl_launch_status();
   }
   SL_CHECK(a.H <= 12288, "streams_norm: rows of odd width hold at most 12,288 values");
@@ -688,10 +690,7 @@ extern "C" const char* sl_add_postnorm(float* resid, const void* y, const float*
       ((uintptr_t)y | (uintptr_t)out) % sizeof(a4) == 0) {
     const int H4 = H / 4, n = row_threads(T, H4), iters = (H4 + n - 1) / n;
     auto run = [&](auto kernel) { kernel<<<T, n, 0, stream>>>(resid, (const act_t*)y, w, (act_t*)out, H, eps, mult); };
-    if (iters == 1) run(add_postnorm_vec_kernel<1>);
-    else if (iters == 2) run(add_postnorm_vec_kernel<2>);
-    else if (iters <= 4) run(add_postnorm_vec_kernel<4>);
-    else run(add_postnorm_vec_kernel<8>);
+    with_groups(iters, [&](auto groups) { run(add_postnorm_vec_kernel<decltype(groups)::n>); });
     return sl_launch_status();
   }
   const int threads = H >= 2048 ? 512 : 256, need = (H + threads - 1) / threads;
@@ -830,10 +829,7 @@ extern "C" const char* sl_add_normed_rmsnorm(float* resid, const void* y, const 
       ((uintptr_t)y | (uintptr_t)out) % sizeof(a4) == 0) {
     const int H4 = H / 4, n = row_threads(R, H4), iters = (H4 + n - 1) / n;
     auto run = [&](auto kernel) { kernel<<<R, n, 0, stream>>>(resid, (const act_t*)y, wy, eps_y, rows, w, eps, (act_t*)out, H); };
-    if (iters == 1) run(add_normed_rmsnorm_vec_kernel<1>);
-    else if (iters == 2) run(add_normed_rmsnorm_vec_kernel<2>);
-    else if (iters <= 4) run(add_normed_rmsnorm_vec_kernel<4>);
-    else run(add_normed_rmsnorm_vec_kernel<8>);
+    with_groups(iters, [&](auto groups) { run(add_normed_rmsnorm_vec_kernel<decltype(groups)::n>); });
     return sl_launch_status();
   }
   const int threads = H >= 2048 ? 512 : 256, need = (H + threads - 1) / threads;
