@@ -30,31 +30,40 @@ __global__ void embed_kernel(const int* __restrict__ ids, const act_t* __restric
   }
 }
 
-// The same for rows of a multiple of 8 values and aligned tables: a thread has eight values, asked for at once (64 rows of 3,584 values:
-// 10.5 us with single loads by one workgroup a row, 5.0 here; 8 rows 3.5, now 1.7; 2,048 rows 17.6, now 13.8).
-struct __attribute__((aligned(16))) e8 { act_t v[8]; };
+// The same for rows of a multiple of 8 values and aligned tables: a thread has eight values, asked for at once, four and four, so that
+// a wavefront's store is one run of memory (us, tables in the caches, single loads by one workgroup a row / here: 64 rows of 3,584 values 4.1 / 3.0,
+// 8 rows 4.0 / 3.2, 2,048 rows 10.0 / 8.2; four copies of 2,048 rows of 2,048 13.8 / 13.1, and 16.2 with a thread's eight values side by side).
+struct __attribute__((aligned(4 * sizeof(act_t)))) e4 { act_t v[4]; };
 template <bool PLACED>
 __global__ __launch_bounds__(256) void embed_vec_kernel(const int* __restrict__ ids, const act_t* __restrict__ table,
                                                         float* __restrict__ out, int H, int V, float scale,
                                                         const int* __restrict__ positions, const act_t* __restrict__ pos_table, int P,
                                                         int copies) {
-  const int t = blockIdx.x, i = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
+  const int t = blockIdx.x, first = (blockIdx.y * 2 * blockDim.x + threadIdx.x) * 4, second = first + 4 * (int)blockDim.x;
   const int id = min(max(ids[t], 0), V - 1);
-  if (i >= H) return;
-  const e8 x = *(const e8*)(table + (size_t)id * H + i);
-  float v[8];
+  if (first >= H) return;
+  const bool both = second < H;
+  const act_t* row = table + (size_t)id * H;
+  const e4 x[2] = {*(const e4*)(row + first), *(const e4*)(row + (both ? second : first))};
+  float4 v[2];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = scale * to_f(x.v[j]);
+  for (int i = 0; i < 2; ++i) v[i] = make_float4(scale * to_f(x[i].v[0]), scale * to_f(x[i].v[1]), scale * to_f(x[i].v[2]), scale * to_f(x[i].v[3]));
   if (PLACED) {
     const int p = min(max(positions[t], 0), P - 1);
-    const e8 y = *(const e8*)(pos_table + (size_t)p * H + i);
+    const act_t* placed = pos_table + (size_t)p * H;
+    const e4 y[2] = {*(const e4*)(placed + first), *(const e4*)(placed + (both ? second : first))};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] += to_f(y.v[j]);
+    for (int i = 0; i < 2; ++i) {
+      v[i].x += to_f(y[i].v[0]);
+      v[i].y += to_f(y[i].v[1]);
+      v[i].z += to_f(y[i].v[2]);
+      v[i].w += to_f(y[i].v[3]);
+    }
   }
-  float* o = out + (size_t)t * copies * H + i;
+  float* o = out + (size_t)t * copies * H;
   for (int s = 0; s < copies; ++s) {
-    *(float4*)(o + (size_t)s * H) = make_float4(v[0], v[1], v[2], v[3]);
-    *(float4*)(o + (size_t)s * H + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    *(float4*)(o + (size_t)s * H + first) = v[0];
+    if (both) *(float4*)(o + (size_t)s * H + second) = v[1];
   }
 }
 
