@@ -906,7 +906,10 @@ __global__ __launch_bounds__(256) void routed_combine_kernel(const float* __rest
 }
 
 // The same, four channels a thread with 16-byte loads, eight choices' rows asked for at once: rows of a multiple of four values and
-// aligned operands.  2,048 tokens of 8 choices, 2,048 channels, 150 MB: 39 us with a channel a thread, 26 here.
+// aligned operands.  2,048 tokens of 8 choices, 2,048 channels, 150 MB: 39 us with a channel a thread, 26 here.  Few tokens are a chain of two
+// trips in either, and the places of eight choices in registers are a longer one than two or ten of them in LDS: from 400,000 values
+// on, and with five to eight choices (us, a channel a thread / here: 64 tokens of 2,048 channels, 2 choices 3.0 / 3.2, 10 3.8 / 3.9, 8 3.5 / 3.2; 200 tokens, 2
+// choices 3.5 / 3.5, 10 4.6 / 4.3; 300 of 896, 2 choices 3.3 / 3.4, 500 3.6 / 3.5; 2,048 of 2,048, 2 choices 18.7 / 9.8).
 struct __attribute__((aligned(16))) rc_f4 { float v[4]; };
 struct __attribute__((aligned(4 * sizeof(act_t)))) rc_a4 { act_t v[4]; };
 template <bool THROUGH>
@@ -958,7 +961,8 @@ extern "C" const char* sl_routed_combine(const float* y, const int* place_of, co
   SL_CHECK(T >= 0 && top >= 1 && top <= 64 && H > 0, "routed_combine: sizes must be positive, at most 64 choices");
   SL_CHECK(chosen == nullptr || x != nullptr, "routed_combine: experts that hand their input through need the input");
   if (T == 0) return nullptr;
-  if (H % 4 == 0 && (uintptr_t)y % 16 == 0 && ((uintptr_t)base | (uintptr_t)out | (uintptr_t)x) % sizeof(rc_a4) == 0) {
+  const bool vec = (long long)T * H >= 400000 || top % 8 == 0 || top % 8 > 4;
+  if (vec && H % 4 == 0 && (uintptr_t)y % 16 == 0 && ((uintptr_t)base | (uintptr_t)out | (uintptr_t)x) % sizeof(rc_a4) == 0) {
     const int n = H >= 1024 ? 256 : (H / 4 + 63) / 64 * 64;
     auto run = [&](auto kernel) {
       kernel<<<dim3(T, (H / 4 + n - 1) / n), n, 0, stream>>>(y, place_of, shares, top, (const act_t*)base, base_gate, gate_stride, H,

@@ -24,12 +24,14 @@ def test_odd_logits(T, E, top, form):
     routes_of_odd_logits(T, E, top, form)
 
 
-# no group of four channels behind the last whole workgroup, one, a width without groups; no choice beside a trip's eight, one, two trips; every form
+# no group of four channels behind the last whole workgroup, one, a width without groups; no choice beside a trip's eight, one, two trips; every form; few
+# tokens, which take four channels a thread for some numbers of choices, and so many that they always do
 @pytest.mark.parametrize("H", [4, 1024, 1028, 2052, 30])
-@pytest.mark.parametrize("top", [1, 8, 9, 17])
-def test_sums_over_the_choices(H, top):
+@pytest.mark.parametrize("top", [1, 4, 5, 8, 9, 13, 17])
+@pytest.mark.parametrize("many", [False, True])
+def test_sums_over_the_choices(H, top, many):
     for dtype in (torch.float32, torch.bfloat16):
-        ops, T, E = HipOps(dtype, "cuda:0"), 3, 5
+        ops, T, E = HipOps(dtype, "cuda:0"), -(-400000 // H) if many else 3, 5
         g = torch.Generator(device="cuda:0").manual_seed(H + top)
         new = lambda *s: torch.randn(*s, generator=g, device="cuda:0")
         y, base, x, gate = new(T * top, H), new(T, H).to(dtype), new(T, H).to(dtype), new(T, 2)
