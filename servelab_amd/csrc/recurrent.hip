@@ -1151,8 +1151,9 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
 // no gate (nullptr): the norm alone.
 // gate_first: the gate comes before the norm, x = o * act(gate), then x / sqrt(mean(x^2) + eps) * w.
 // N > 0: heads of up to 64 N channels, everything asked for at once (a head of 256 / 512 channels took as many trips to memory twice:
-// one request of 8 heads of 256 3.0 us, now 1.9, two of 512 5.3, now 2.5); 0: wider ones.
-template <int N>
+// one request of 8 heads of 256 3.0 us, now 1.9, two of 512 5.3, now 2.5); 0: wider ones.  GATED: there is a gate (2,048 tokens of 4 heads of 512
+// without one, us: 8.8 with the row read in its place, 5.8 now).
+template <int N, bool GATED>
 __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restrict__ o, int H, int Dv,
                                                             const float* __restrict__ w, int per_head, float eps,
                                                             const float* __restrict__ gate, int gate_stride,
@@ -1165,26 +1166,27 @@ __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restr
   const float* wr = w + (per_head ? h * Dv : 0);
   float ss = 0.f;
   if constexpr (N > 0) {
-    const float* zr = gr != nullptr ? gr : x;
     float v[N], z[N], g[N];
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const int d = min(lane + 64 * u, Dv - 1);
       v[u] = x[d];
-      z[u] = zr[d];
+      if (GATED) z[u] = gr[d];
       g[u] = wr[d];
     }
 #pragma unroll
     for (int u = 0; u < N; ++u) {
-      z[u] = act == 0 ? sigmoidf_(z[u]) : z[u] * sigmoidf_(z[u]);
-      if (gate_first && gr != nullptr) v[u] *= z[u];
+      if (GATED) {
+        z[u] = act == 0 ? sigmoidf_(z[u]) : z[u] * sigmoidf_(z[u]);
+        if (gate_first) v[u] *= z[u];
+      }
       ss += lane + 64 * u < Dv ? v[u] * v[u] : 0.f;
     }
     const float inv = 1.f / sqrtf(wave_sum(ss) / (float)Dv + eps);
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const float r = v[u] * inv * g[u];
-      if (lane + 64 * u < Dv) out[(t * H + h) * Dv + lane + 64 * u] = from_f<act_t>(gr != nullptr && !gate_first ? r * z[u] : r);
+      if (lane + 64 * u < Dv) out[(t * H + h) * Dv + lane + 64 * u] = from_f<act_t>(GATED && !gate_first ? r * z[u] : r);
     }
     return;
   }
@@ -1218,11 +1220,12 @@ extern "C" const char* sl_head_norm_gate(const float* o, int T, int H, int Dv, c
   auto run = [&](auto kernel) {
     kernel<<<dim3(T, H), 64, 0, stream>>>(o, H, Dv, w, per_head, eps, gate, gate_stride, gate_col, act, gate_first, (act_t*)out);
   };
-  if (Dv <= 64) run(head_norm_gate_kernel<1>);
-  else if (Dv <= 128) run(head_norm_gate_kernel<2>);
-  else if (Dv <= 256) run(head_norm_gate_kernel<4>);
-  else if (Dv <= 512) run(head_norm_gate_kernel<8>);
-  else run(head_norm_gate_kernel<0>);
+  auto choose = [&](auto gated, auto plain) { run(gate != nullptr ? gated : plain); };
+  if (Dv <= 64) choose(head_norm_gate_kernel<1, true>, head_norm_gate_kernel<1, false>);
+  else if (Dv <= 128) choose(head_norm_gate_kernel<2, true>, head_norm_gate_kernel<2, false>);
+  else if (Dv <= 256) choose(head_norm_gate_kernel<4, true>, head_norm_gate_kernel<4, false>);
+  else if (Dv <= 512) choose(head_norm_gate_kernel<8, true>, head_norm_gate_kernel<8, false>);
+  else run(head_norm_gate_kernel<0, true>);
   return sl_launch_status();
 }
 
