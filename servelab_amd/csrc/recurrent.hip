@@ -896,13 +896,16 @@ __global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, in
   const int r0 = 4 * p, r1 = 4 * P + 4 * p, D = a.D;
   const bool fresh = a.positions[s] == 0;
   float* slot = a.state + (size_t)a.slots[s] * a.state_stride;
+  // (aligned: D is a multiple of four, so that a half is there or not; what is not is read from the last one and left out)
+  const int a0 = min(r0, D - 4), a1 = min(r1, D - 4);
+  const bool all = D == 8 * P;
   // the 8 values of a row of D channels that this lane owns
   auto channels = [&](const float* row, float beyond) {
     Channels8 c;
-    if (aligned && r1 + 4 <= D) {
-      const scan_f4 x = *(const scan_f4*)(row + r0), y = *(const scan_f4*)(row + r1);
+    if (aligned) {
+      const scan_f4 x = *(const scan_f4*)(row + a0), y = *(const scan_f4*)(row + a1);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) c.v[i] = x.v[i], c.v[4 + i] = y.v[i];
+      for (int i = 0; i < 4; ++i) c.v[i] = all || r0 < D ? x.v[i] : beyond, c.v[4 + i] = all || r1 < D ? y.v[i] : beyond;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -931,10 +934,10 @@ __global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, in
     if (fresh) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) S[u].v[i] = 0.f;
-    } else if (aligned && r1 + 4 <= D) {
-      const state_v4 x = __builtin_nontemporal_load((const state_v4*)(col + r0)), y = __builtin_nontemporal_load((const state_v4*)(col + r1));
+    } else if (aligned) {
+      const state_v4 x = __builtin_nontemporal_load((const state_v4*)(col + a0)), y = __builtin_nontemporal_load((const state_v4*)(col + a1));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) S[u].v[i] = x[i], S[u].v[4 + i] = y[i];
+      for (int i = 0; i < 4; ++i) S[u].v[i] = all || r0 < D ? x[i] : 0.f, S[u].v[4 + i] = all || r1 < D ? y[i] : 0.f;
     } else {
       S[u] = channels(col, 0.f);
     }
@@ -1029,9 +1032,9 @@ __global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, in
     if (p == 0) a.out[((size_t)s * a.H + h) * a.Dv + j] = o;
     if (!a.write) continue;
     float* col = slot + ((size_t)h * a.Dv + j) * D;
-    if (aligned && r1 + 4 <= D) {
-      __builtin_nontemporal_store(state_v4{S[u].v[0], S[u].v[1], S[u].v[2], S[u].v[3]}, (state_v4*)(col + r0));
-      __builtin_nontemporal_store(state_v4{S[u].v[4], S[u].v[5], S[u].v[6], S[u].v[7]}, (state_v4*)(col + r1));
+    if (aligned) {
+      if (r0 < D) __builtin_nontemporal_store(state_v4{S[u].v[0], S[u].v[1], S[u].v[2], S[u].v[3]}, (state_v4*)(col + r0));
+      if (r1 < D) __builtin_nontemporal_store(state_v4{S[u].v[4], S[u].v[5], S[u].v[6], S[u].v[7]}, (state_v4*)(col + r1));
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
