@@ -413,9 +413,10 @@ __global__ __launch_bounds__(256) void stream_conv_kernel(const ShortConv a, act
 // conditions, 3.0 here).  Tokens that
 // fill the chip with fewer blocks get fewer (300 of 3,584, two / four taps: 10.8 / 11.8 us with a slice a block, 7.6 / 10.6
 // with a block a token, 8.2 / 9.9 here).  The sums run in the order of the kernels for longer steps.
-// (LOOP apart from the one slice: a loop about the loads costs that 0.5 us.)
+// (LOOP apart from the one slice: a loop about the loads costs that 0.5 us.  BACK: there are taps before the token's own; 64 tokens of 4,096
+// channels without, us: 3.1 with the row read in place of their inputs, 2.9 now.)
 constexpr int STREAM_KEEP = 4, STREAM_TAPS = 3;
-template <bool LOOP>
+template <bool LOOP, bool BACK>
 __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid, const act_t* __restrict__ y,
                                    const float* __restrict__ wy, float eps, int write, act_t* __restrict__ out) {
   __shared__ float scratch[16];
@@ -427,14 +428,13 @@ __global__ void stream_step_kernel(const ShortConv a, float* __restrict__ resid,
   const int s = t;                                     // (a token a sequence)
   const bool fresh = a.positions[t] == 0;
   float* keep_in = a.state + (size_t)a.slots[s] * a.state_stride + a.state_off;
-  const float* kept = back > 0 ? keep_in : x;
   float v, yv, gain, w_own;
   float past[STREAM_TAPS], w[STREAM_TAPS];
   auto ask = [&](int c) {
     v = x[c];
 #pragma unroll
-    for (int j = 0; j < STREAM_TAPS; ++j) {            // (past the taps: the last again, not used)
-      past[j] = kept[(size_t)max(min(j, back - 1), 0) * H + c];
+    for (int j = 0; BACK && j < STREAM_TAPS; ++j) {    // (past the taps: the last again, not used)
+      past[j] = keep_in[(size_t)min(j, back - 1) * H + c];
       w[j] = a.w[(size_t)min(j, back) * H + c];
     }
     w_own = a.w[(size_t)back * H + c];
@@ -511,8 +511,10 @@ extern "C" const char* sl_stream_conv(float* resid, int C, int taps, const float
     auto run = [&](auto kernel) {
       kernel<<<dim3(T, slices), threads, 0, stream>>>(a, resid, (const act_t*)y, wy, eps, write, (act_t*)out);
     };
-    if (slices == all) run(stream_step_kernel<false>);
-    else run(stream_step_kernel<true>);
+    if (slices == all && taps > 1) run(stream_step_kernel<false, true>);
+    else if (slices == all) run(stream_step_kernel<false, false>);
+    else if (taps > 1) run(stream_step_kernel<true, true>);
+    else run(stream_step_kernel<true, false>);
     return sl_launch_status();
   }
   const bool whole = C % 4 == 0 && (uintptr_t)resid % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0;
