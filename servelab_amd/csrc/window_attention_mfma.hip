@@ -569,7 +569,9 @@ extern "C" const char* sl_window_attention_mfma(
   const long long full = (long long)num_seqs * max_q_len;         // tokens if every sequence had as many as the longest
   const int order = num_tokens == full && tiles * nsplit <= 65535 ? BY_LENGTH :
                     4ll * num_tokens >= 3 * full ? BY_LENGTH_MOVED : LATE_FIRST;
-  const unsigned items = (unsigned)(tiles * nsplit);
+  // (sequence by sequence: an odd number of tiles for each, so that the first tiles, which is all that single tokens among prompts have, lie on
+  // all dies; with a multiple of eight they are one die's: a prompt of 1,000 tokens beside 31 single ones, 8 heads on 8, 128 / 128, 190 us and 41 so)
+  const unsigned items = (unsigned)(tiles * nsplit) | (order == LATE_FIRST ? 1u : 0u);
   const dim3 grid = order == BY_LENGTH ? dim3(nkv, num_seqs, items) : dim3(items, nkv, num_seqs);
   const char* e = launch_mfma(a, grid, order, stream);
   if (e || nsplit == 1) return e;
