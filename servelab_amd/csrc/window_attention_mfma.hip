@@ -22,8 +22,8 @@
 // the weights of 8 consecutive keys of its column: the B operand of the second product as it is.
 //
 // What bounds it: a block is a chain (stage, scores, maximum, exponentials, terms, sums) of a few thousand cycles, of which the matrix
-// instructions are 500 to 2,100, and the longest tile walks all of its keys; so a workgroup is eight wavefronts: two teams that take every other
-// block and meet at the end, or, where values lie in the key rows (132 matrix instructions a block, more registers than two
+// instructions are 500 to 2,100, and the longest tile walks all of its keys; so where the chip has few workgroups one is eight wavefronts: two teams that take every
+// other block and meet at the end, or, of a wide latent (132 matrix instructions a block, more registers than two
 // wavefronts a SIMD have), pairs that share columns, each with half the channels; the longest tiles start first; a
 // block has 150 vector instructions and no branches inside (addresses looked up key by key and a cap chosen score by score were 270 and
 // eight).  us, before / now: 128 / 128, 16 heads on 2, one prompt of 2,048 tokens 104 / 68 (255 TFLOP/s counted once a weight), 1,000 and 889 56 /
@@ -109,29 +109,39 @@ __device__ __forceinline__ void three_terms(const float (&p)[8], bf16x8& p1, bf1
   p3 = __builtin_bit_cast(bf16x8, w3);
 }
 
-// A prompt's workgroup is eight wavefronts over 64 columns: two teams of four that take every other block and meet at the end, or,
-// where values lie in the key rows, one whose wavefronts share their 16 columns two and two, each with half of the channels.
-constexpr int TEAMS = VK || !NARROW ? 1 : 2, PARTS = VK ? 2 : 1;
-constexpr int THREADS = 256 * PARTS, COLS = 64;         // of a team
-constexpr int KKP = (KK + PARTS - 1) / PARTS, DDP = (DD + PARTS - 1) / PARTS;      // steps of key channels and tiles of value channels a wavefront
-constexpr int MEETS = VK ? 8 * 2 * 64 * 16 : 0;         // bytes in which the parts of the scores meet
-constexpr int STAGE = 32 * KROW + VT;                   // values of a team's staged block
-constexpr int MEET = TEAMS == 2 ? 256 * DV + 512 : 0;   // bytes in which the second team hands over what it has
-constexpr int STAGED = 2 * TEAMS * STAGE + MEETS, LDS_BYTES = STAGED > MEET ? STAGED : MEET;
-static_assert(LDS_BYTES <= 160 * 1024, "a prompt's workgroup fits a CU");
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
-// what a thread stages of a block: chunks of 8 values (16 bytes)
-constexpr int KCH = DK / 8;                            // chunks of a key row
-constexpr int NKC = VK ? 1 : cdiv(32 * KCH, THREADS);  // key chunks a thread
-constexpr int NVC = VK ? 1 : cdiv(DV * 4, THREADS);    // value chunks (a channel's 8 keys) a thread
-constexpr int RCH = VK ? (DK - DV) / 8 : 0;            // chunks of a key row behind the values
-constexpr int NT = VK ? cdiv((DV / 8) * 4, THREADS) : 1;   // 8 keys x 8 channels tiles a thread (turned on their way into LDS)
-constexpr int NR = VK ? (RCH ? cdiv(32 * RCH, THREADS) : 1) : 1;
+constexpr int COLS = 64;                               // of a workgroup
+constexpr int STAGE = 32 * KROW + VT;                  // values of a staged block
+constexpr int KCH = DK / 8, RCH = VK ? (DK - DV) / 8 : 0;      // chunks of 8 values (16 bytes) of a key row, and of one behind the values
 
-// A thread's places in a block are the same for all blocks and stay in registers, except where these are short; us, kept / worked out
-// anew: 512 / 256 64 / 69 (no register spilled either way), 896 / 64 145 (50 spilled) / 80; one team: 512 / 512 119 / 135 (none), 640 / 512 146 (13) / 145 and
-// steps of 32 requests 41 / 37, 1024 / 512 241 (76) / 200.
-constexpr bool PLACES_ANEW = !VK && (TEAMS == 2 ? 4 * DK + 5 * DV > 3328 : DK + 2 * DV > 1600);
+// A prompt's workgroup owns 64 columns, sixteen for each of four wavefronts; TEAMS 2: twice as many, in two teams that take every other block
+// and meet at the end; PARTS 2: twice as many, two of them for sixteen columns, each with half of the channels (of a latent).
+template <int TEAMS, int PARTS> struct Form {
+  static constexpr int THREADS = 256 * PARTS;          // of a team
+  static constexpr int KKP = cdiv(KK, PARTS), DDP = cdiv(DD, PARTS);      // steps of key channels and tiles of value channels a wavefront
+  static constexpr int MEETS = PARTS == 2 ? 8 * 2 * 64 * 16 : 0;          // bytes in which the parts of the scores meet
+  static constexpr int MEET = TEAMS == 2 ? 256 * DV + 512 : 0;            // bytes in which the second team hands over what it has
+  static constexpr int STAGED = 2 * TEAMS * STAGE + MEETS, LDS_BYTES = STAGED > MEET ? STAGED : MEET;
+  static_assert(LDS_BYTES <= 160 * 1024, "a prompt's workgroup fits a CU");
+  // what a thread stages of a block
+  static constexpr int NKC = VK ? 1 : cdiv(32 * KCH, THREADS);            // chunks of keys
+  static constexpr int NVC = VK ? 1 : cdiv(DV * 4, THREADS);              // chunks of values (a channel's 8 keys)
+  static constexpr int NT = VK ? cdiv((DV / 8) * 4, THREADS) : 1;         // 8 keys x 8 channels tiles (turned on their way into LDS)
+  static constexpr int NR = RCH ? cdiv(32 * RCH, THREADS) : 1;
+  // A thread's places in a block are the same for all blocks and stay in registers, except where these are short; us, kept / worked out
+  // anew: 512 / 256 64 / 69 (no register spilled either way), 896 / 64 145 (50 spilled) / 80; one team: 512 / 512 119 / 135 (none), 640 / 512 146 (13) /
+  // 145 and steps of 32 requests 41 / 37, 1024 / 512 241 (76) / 200.
+  static constexpr bool PLACES_ANEW = !VK && (TEAMS == 2 ? 4 * DK + 5 * DV > 3328 : DK + 2 * DV > 1600);
+  static constexpr int WAVES = TEAMS * PARTS == 1 ? (DK <= 128 && DV <= 128 ? (VK && DK + DV > 192 ? 3 : 4) : DK + DV <= 576 ? 2 : 1)
+                                                  : (!VK && DK <= 128 && DV <= 128 ? 4 : 2);      // a SIMD holds, at least
+};
+
+// Prompts' forms that are built.  FEW: of few workgroups each wants to be short, and has eight wavefronts: two teams, or pairs where the latent is so
+// wide that two teams spill or do not fit.  MANY: of many workgroups the chip wants as many as it can hold at once, four wavefronts each and no
+// meeting; only where those leave room for two on a SIMD (576 / 512: pairs 12 % ahead at every number of workgroups, 256 / 256 64 / 85).
+constexpr bool PAIRS = VK && DK + DV > 576;
+constexpr int FEW_TEAMS = !PAIRS && (VK || NARROW) ? 2 : 1, FEW_PARTS = PAIRS ? 2 : 1;
+constexpr bool MANY = FEW_TEAMS == 2 && DK + DV <= 576;
 
 // Workgroups start in the order of their number, and numbers go to the eight dies in turn and there to the groups of CUs in
 // turn.  Without a window or chunks a tile takes as long as its keys are many, so the late tiles come first:
@@ -143,7 +153,10 @@ constexpr bool PLACES_ANEW = !VK && (TEAMS == 2 ? 4 * DK + 5 * DV > 3328 : DK + 
 // 1,000 410 moved, 463 with early tiles first.)
 enum { LATE_FIRST, BY_LENGTH, BY_LENGTH_MOVED };
 
-__global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK && DK <= 128 && DV <= 128 ? 4 : 2) void window_attention_mfma_kernel(const WindowAttention a, int order) {
+template <int TEAMS, int PARTS>
+__global__ __launch_bounds__(256 * TEAMS * PARTS, (Form<TEAMS, PARTS>::WAVES)) void window_attention_mfma_kernel(const WindowAttention a, int order) {
+  using F = Form<TEAMS, PARTS>;
+  constexpr int THREADS = F::THREADS, KKP = F::KKP, DDP = F::DDP, NKC = F::NKC, NVC = F::NVC, NT = F::NT, NR = F::NR;
   extern __shared__ __attribute__((aligned(16))) __bf16 lds16[];
   const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
   __bf16* ks = lds16 + team * STAGE;                   // [32][KROW]
@@ -245,7 +258,7 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
   bf16x8 kreg[NKC], vreg[NVC], treg[NT][8], rreg[NR];
   auto this_thread = [&]() {
     int x = tid;
-    if (PLACES_ANEW) asm volatile("" : "+v"(x));       // (nothing that follows from it is kept from block to block)
+    if (F::PLACES_ANEW) asm volatile("" : "+v"(x));       // (nothing that follows from it is kept from block to block)
     return x;
   };
   auto fetch = [&](int kbase, int asked) {
@@ -279,7 +292,7 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
       if constexpr (RCH > 0) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-          const int idx = min((tid ^ 256) + THREADS * i, 32 * RCH - 1), kl = idx / RCH, c8 = DV / 8 + idx % RCH;
+          const int idx = min((PARTS == 2 ? tid ^ 256 : tid) + THREADS * i, 32 * RCH - 1), kl = idx / RCH, c8 = DV / 8 + idx % RCH;
           rreg[i] = *(const bf16x8*)((kl >= 16 ? keysB : keysA) + (kl & 15) * DK + 8 * c8);
         }
       }
@@ -329,7 +342,7 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
       if constexpr (RCH > 0) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-          const int idx = (tid ^ 256) + THREADS * i, kl = idx / RCH, c8 = DV / 8 + idx % RCH;
+          const int idx = (PARTS == 2 ? tid ^ 256 : tid) + THREADS * i, kl = idx / RCH, c8 = DV / 8 + idx % RCH;
           if (32 * RCH % THREADS == 0 || idx < 32 * RCH) *(bf16x8*)(ks + staged_row(kl) * KROW + 8 * c8) = rreg[i];
         }
       }
@@ -502,13 +515,13 @@ __global__ __launch_bounds__(TEAMS * THREADS, TEAMS * THREADS == 256 ? 1 : !VK &
 
 #include "window_step.h"
 
-static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, hipStream_t stream) {
-  if (LDS_BYTES > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+template <int TEAMS, int PARTS> static const char* launch_mfma(const WindowAttention& a, dim3 grid, int order, hipStream_t stream) {
+  constexpr int bytes = Form<TEAMS, PARTS>::LDS_BYTES;
+  if (bytes > 48 * 1024) {
+    hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel<TEAMS, PARTS>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return hipGetErrorString(e);
   }
-  window_attention_mfma_kernel<<<grid, TEAMS * THREADS, LDS_BYTES, stream>>>(a, order);
+  window_attention_mfma_kernel<TEAMS, PARTS><<<grid, 256 * TEAMS * PARTS, bytes, stream>>>(a, order);
   return sl_launch_status();
 }
 #if SL_VK || SL_NARROW
@@ -529,13 +542,14 @@ static const char* launch_step(const WindowAttention&, int, hipStream_t) { retur
 extern "C" int sl_window_attention_mfma_step_blocks() { return STEP_BLOCKS; }
 
 // The call of sl_window_attention, for Dk == SL_DK, Dv == SL_DV and (vc == nullptr) == SL_VK.
-// q rows, key rows and value rows must be 16-byte aligned.
+// q rows, key rows and value rows must be 16-byte aligned.  few: the form of few workgroups; step: a step of one token a sequence by
+// the kernel for it (either is a wish: what is not built, or does not fit the call, is the other).
 extern "C" const char* sl_window_attention_mfma(
     const void* q, int q_stride, const void* kc, const void* vc, const int* tables, int max_pages,
     const int* cu_q, const int* positions, int num_seqs, int max_q_len, int num_tokens, int nh,
     int nkv, int Dk, int Dv, int page, float scale, float softcap, int window, int chunk, int keep_first, const float* slopes,
     const float* sinks, const void* gate, int gate_stride, const float* channel_gate, int channel_stride, void* out,
-    int nsplit, float* part_o, float* part_ml, hipStream_t stream) {
+    int few, int step, int nsplit, float* part_o, float* part_ml, hipStream_t stream) {
   SL_CHECK(Dk == DK && Dv == DV && (vc == nullptr) == VK, "window attention (matrix cores): built for other widths");
   SL_CHECK(num_seqs >= 0 && max_q_len >= 1 && nh > 0 && nkv > 0 && nh % nkv == 0,
            "window attention: heads must be a positive multiple of kv heads");
@@ -556,7 +570,7 @@ extern "C" const char* sl_window_attention_mfma(
                           cu_q, positions, nh, nkv, Dk, Dv, page, scale, softcap, window, chunk, keep_first, slopes, sinks,
                           (const act_t*)gate, gate_stride, channel_gate, channel_stride, (act_t*)out, nsplit, part_o,
                           part_ml};
-  if (STEP_BLOCKS > 0 && max_q_len == 1 && num_tokens == num_seqs && (nsplit == 1 || (uintptr_t)part_ml % 8 == 0) &&
+  if (step && STEP_BLOCKS > 0 && max_q_len == 1 && num_tokens == num_seqs && (nsplit == 1 || (uintptr_t)part_ml % 8 == 0) &&
       (long long)nkv * ((nh / nkv + 15) / 16) <= 65535) {              // (a token each)
     const char* e = launch_step(a, num_seqs, stream);
     if (e || nsplit == 1) return e;
@@ -573,7 +587,8 @@ extern "C" const char* sl_window_attention_mfma(
   // all dies; with a multiple of eight they are one die's: a prompt of 1,000 tokens beside 31 single ones, 8 heads on 8, 128 / 128, 190 us and 41 so)
   const unsigned items = (unsigned)(tiles * nsplit) | (order == LATE_FIRST ? 1u : 0u);
   const dim3 grid = order == BY_LENGTH ? dim3(nkv, num_seqs, items) : dim3(items, nkv, num_seqs);
-  const char* e = launch_mfma(a, grid, order, stream);
+  const char* e = few || !MANY ? launch_mfma<FEW_TEAMS, FEW_PARTS>(a, grid, order, stream)
+                               : launch_mfma<MANY ? 1 : FEW_TEAMS, MANY ? 1 : FEW_PARTS>(a, grid, order, stream);
   if (e || nsplit == 1) return e;
   launch_combine(a, num_tokens, stream);
   return sl_launch_status();

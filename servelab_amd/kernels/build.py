@@ -180,7 +180,7 @@ LAZY_STEMS = ("window_attention", "head_gemm", "recurrent", "selective", "routed
 # ahead of use; other widths are compiled when a model first needs them
 WINDOW_MFMA_SIZES = ((128, 128, 0), (64, 64, 0), (576, 512, 1), (32, 16, 0), (64, 48, 1), (96, 64, 0),
                      (96, 64, 1), (96, 80, 1), (64, 32, 1), (64, 32, 0), (96, 96, 0), (32, 48, 0), (32, 32, 0), (64, 80, 0), (128, 256, 0), (192, 272, 0),
-                     (896, 64, 0), (512, 384, 0), (640, 512, 0))
+                     (896, 64, 0), (512, 384, 0), (640, 512, 0), (256, 256, 1))
 
 
 def all_units(head_dims=(32, 64, 96, 128, 192, 256)) -> List[Unit]:

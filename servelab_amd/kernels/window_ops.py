@@ -41,6 +41,23 @@ class WindowOps:
         the kernel of prompts."""
         return self._lib[self._window_mfma_lib(Dk, Dv, in_keys)].sl_window_attention_mfma_step_blocks()
 
+    def _window_few(self, T, S, longest, context, span, nh, nkv, Dk, Dv, in_keys):
+        """Whether a prompt's workgroups have eight wavefronts (two teams, one after the other's block) or four: eight
+        make each one shorter, four let the chip hold twice as many.  By the number of workgroups beside what the chip holds
+        of the eight at once, and by the keys a workgroup walks, on which the teams' meeting is spent; among sequences of very
+        different lengths the short ones' workgroups hold up the long ones'.  Of 1,271 prompts of sixteen widths the form
+        chosen takes 1.003 of the faster one's time on average (us, eight / four: 128 / 128, 16 heads on 2, a prompt of
+        1,024 34 / 43, of 4,096 180 / 184, 4 of 300 16 / 18, 16 of 50 8.1 / 8.0, 64 of 100 32 / 25; 32 on 8, 16 of 200 37 / 30, 4 of 1,000 99 / 92; latent of 96 / 64, 16
+        heads, a prompt of 1,024 37 / 48, 16 of 500 63 / 52; 900, 300, 120, 40 and 10 tokens beside 11 single ones, 128 / 128, 16 on 2 32 / 39, 32 on 8 53 / 46).
+        Wide latents' pairs, and heads of more than 576 channels of keys and values, whose four wavefronts fill a CU's registers as
+        well, have one form."""
+        holds = self._num_cus * (2 if Dk <= 128 and Dv <= 128 and not in_keys else 1)
+        workgroups = nkv * max(S, -(-T * (nh // nkv) // 64))
+        keys = min(span, context - longest // 2)
+        if 4 * T < 3 * S * longest:
+            return workgroups < holds and keys >= 40 + workgroups
+        return workgroups <= 2 * holds and keys >= 40 + max(0, workgroups - 3 * holds // 4)
+
     def _lazy(self, stem):
         """The library of ``stem`` for this table's dtype, compiled and loaded at first use."""
         if stem not in self._lib:
@@ -241,12 +258,13 @@ class WindowOps:
         # 2,048 tokens, two shares a tile save 35 us of attention over four layers and their merging
         # costs 186 us.)
         mfma = self._window_mfma_fits(q, q_col, Dk, Dv)
-        nsplit = 1
+        nsplit, span = 1, batch.max_ctx_len
+        if window or chunk:
+            span = min(span, min(n for n in (window, chunk) if n) + int(keep_first))
+        few = mfma and batch.max_q_len > 1 and self._window_few(T, S, batch.max_q_len, batch.max_ctx_len, span, nh, nkv, Dk, Dv, v_cache is None)
+        step = mfma and T == S and batch.max_q_len == 1
         if batch.max_q_len == 1:
-            span = batch.max_ctx_len
-            if window or chunk:
-                span = min(span, min(n for n in (window, chunk) if n) + int(keep_first))
-            blocks = self._window_step_blocks(Dk, Dv, v_cache is None) if mfma and T == S else 0
+            blocks = self._window_step_blocks(Dk, Dv, v_cache is None) if step else 0
             if blocks:
                 # a token each: shares of as many blocks as a workgroup takes side by side, a workgroup for every CU at most
                 columns = max(1, S * nkv * -(-(nh // nkv) // 16))
@@ -271,6 +289,7 @@ class WindowOps:
                 self._fn[name] = fn
         else:
             lib, name = self._lazy("window_attention"), "sl_window_attention"
+        forms = (int(few), int(step)) if mfma else ()
         self._call(lib, name, _c_void_p(q.data_ptr() + q_col * item), q.shape[1], _p(k_cache),
                    _p(v_cache), _p(block_tables), max_pages, _p(batch.cu_q), _p(batch.positions),
                    S, batch.max_q_len, T, nh, nkv, Dk, Dv, page_size, _c_float(scale),
@@ -278,5 +297,5 @@ class WindowOps:
                    int(keep_first), _p(slopes), _p(sinks),
                    _c_void_p(gate.data_ptr() + gate_col * item) if gate is not None else None, gate_stride,
                    _c_void_p(channel_gate.data_ptr() + 4 * channel_gate_col) if channel_gate is not None else None,
-                   channel_stride, _p(out), nsplit, _p(part_o), _p(part_ml))
+                   channel_stride, _p(out), *forms, nsplit, _p(part_o), _p(part_ml))
         return out

@@ -31,7 +31,8 @@ def exact(q, keys, values, pos, scale, window, keep, chunk, softcap, slopes, sin
 # two (beyond 256 channels of values with pages of their own); widths whose steps take the kernel of prompts
 @pytest.mark.parametrize("H,G,Dk,Dv,in_keys", [(2, 2, 32, 16, False), (8, 2, 128, 128, False), (16, 1, 64, 80, False), (20, 1, 96, 64, False),
                                               (3, 1, 64, 48, True), (32, 1, 576, 512, True), (17, 1, 96, 96, False), (8, 2, 128, 256, False),
-                                              (17, 1, 192, 272, False), (2, 1, 896, 64, False), (17, 1, 512, 384, False), (4, 2, 640, 512, False)])
+                                              (17, 1, 192, 272, False), (2, 1, 896, 64, False), (17, 1, 512, 384, False), (4, 2, 640, 512, False),
+                                              (20, 1, 256, 256, True)])
 @pytest.mark.parametrize("window,keep,chunk,page,shares", [(None, 0, None, 16, 32), (9, 3, None, 16, 32), (40, 33, None, 32, 3), (None, 0, 48, 16, 5),
                                                           (1, 1, None, 64, 32), (700, 4, 512, 16, 1), (None, 0, None, 16, 1)])
 def test_steps_of_one_token(H, G, Dk, Dv, in_keys, window, keep, chunk, page, shares):

@@ -1,5 +1,5 @@
 """Prompts through the matrix-core window attention whose workgroups are two teams of wavefronts (every other block of 32 keys) or pairs
-of them (halves of the channels), or one team where heads are wide: one block, two, an odd number, a last round for one team alone; caps;
+of them (halves of the channels), or one team where heads are wide or workgroups many: one block, two, an odd number, a last round for one team alone; caps;
 channels that no half divides."""
 from types import SimpleNamespace
 
@@ -14,11 +14,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,G,Dk,Dv,in_keys", [(4, 2, 32, 16, False), (3, 1, 64, 80, False), (8, 2, 128, 128, False), (3, 1, 64, 48, True),
-                                              (2, 1, 96, 80, True), (4, 1, 576, 512, True), (4, 2, 128, 256, False), (3, 1, 192, 272, False),
+                                              (2, 1, 96, 80, True), (4, 1, 576, 512, True), (3, 1, 256, 256, True), (4, 2, 128, 256, False), (3, 1, 192, 272, False),
                                               (2, 1, 896, 64, False), (3, 1, 512, 384, False), (4, 2, 640, 512, False)])
 @pytest.mark.parametrize("window,keep,chunk,softcap", [(None, 0, None, None), (37, 5, None, None), (None, 0, 48, 15.0), (None, 3, 64, None)])
-def test_prompts(H, G, Dk, Dv, in_keys, window, keep, chunk, softcap):
+@pytest.mark.parametrize("few", [True, False])
+def test_prompts(H, G, Dk, Dv, in_keys, window, keep, chunk, softcap, few):
     ops, page = HipOps(torch.bfloat16, "cuda:0"), 16
+    ops._window_few = lambda *a: few                                                     # (both forms, whatever the rule takes)
     g = torch.Generator().manual_seed(Dk + H)
     seqs = [(0, 32), (0, 33), (64, 1), (40, 75), (0, 1), (150, 9)]                       # (cached tokens, tokens of this step)
     lens = [a + b for a, b in seqs]

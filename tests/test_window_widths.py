@@ -23,13 +23,15 @@ def spilled(source, *defines):
     return dict(zip(names, counts))
 
 
-# either side of the lines between two teams and one, and between places kept and worked out anew; the widest of each sort.  (Up to 25 spilled
+# either side of the lines between two teams and one, between places kept and worked out anew, and between one form and two, of a latent between
+# teams and pairs; the widest of each sort.  (Up to 25 spilled
 # registers the narrow forms are still the faster ones, from 35 on they are not.)
 @pytest.mark.skipif(not os.path.exists(build.hipcc()), reason="no hipcc")
-@pytest.mark.parametrize("Dk,Dv", [(512, 256), (192, 512), (704, 256), (1024, 96), (896, 16), (256, 512), (512, 384), (1024, 112), (512, 512),
-                                   (544, 512), (640, 512), (1024, 512)])
-def test_registers(Dk, Dv):
-    found = spilled("window_attention_mfma.hip", f"SL_DK={Dk}", f"SL_DV={Dv}", "SL_VK=0")
+@pytest.mark.parametrize("Dk,Dv,in_keys", [(512, 256, 0), (192, 512, 0), (704, 256, 0), (1024, 96, 0), (896, 16, 0), (256, 512, 0), (512, 384, 0), (1024, 112, 0),
+                                           (512, 512, 0), (544, 512, 0), (640, 512, 0), (1024, 512, 0), (128, 128, 0), (320, 256, 0), (64, 512, 0), (544, 32, 0),
+                                           (128, 128, 1), (288, 288, 1), (320, 256, 1), (544, 32, 1), (320, 272, 1), (576, 512, 1), (1024, 512, 1)])
+def test_registers(Dk, Dv, in_keys):
+    found = spilled("window_attention_mfma.hip", f"SL_DK={Dk}", f"SL_DV={Dv}", f"SL_VK={in_keys}")
     assert max(found.values()) <= 25, found
 
 
@@ -62,3 +64,20 @@ def test_shares_of_a_step(S, shares):
     out = ops.window_attention(torch.zeros(S, 256, dtype=torch.bfloat16), 0, 4, 2, 64, 64, pages, pages, 16,
                                torch.zeros(S, 256, dtype=torch.int32), batch, 1.0, None)
     assert out.shape == (S, 256) and ops.shares == [shares]
+
+
+def prompts(lens, heads, kv_heads, Dk, Dv, in_keys, cached=0):
+    context = max(lens) + cached
+    return Recorded()._window_few(sum(lens), len(lens), max(lens), context, context, heads, kv_heads, Dk, Dv, in_keys)
+
+
+# (us measured with eight wavefronts a workgroup / with four beside each)
+@pytest.mark.parametrize("lens,heads,kv_heads,Dk,Dv,in_keys,few", [
+    ([1024], 16, 2, 128, 128, False, True), ([300] * 4, 16, 2, 128, 128, False, True),                    # 34 / 43, 16 / 18
+    ([200] * 16, 32, 8, 128, 128, False, False), ([100] * 64, 16, 2, 128, 128, False, False),             # 37 / 30, 32 / 25
+    ([50] * 64, 8, 8, 64, 64, False, False), ([1000] * 4, 8, 8, 64, 64, False, True),                     # 8.9 / 8.1, 28 / 34
+    ([1024], 16, 1, 96, 64, True, True), ([500] * 16, 16, 1, 96, 64, True, False),                        # 37 / 48, 63 / 52
+    ([2000] + [1] * 31, 32, 8, 64, 64, False, False), ([300] + [1] * 31, 16, 2, 128, 128, False, True),   # 122 / 101, 29 / 33
+    ([2048], 16, 2, 192, 128, False, True), ([4096], 16, 2, 192, 128, False, False), ([300] * 4, 16, 2, 192, 128, False, True)])   # 78 / 93, 256 / 202, 17 / 20
+def test_wavefronts_of_a_prompt_s_workgroups(lens, heads, kv_heads, Dk, Dv, in_keys, few):
+    assert prompts(lens, heads, kv_heads, Dk, Dv, in_keys) is few
