@@ -58,6 +58,20 @@ class WindowOps:
             return workgroups < holds and keys >= 40 + workgroups
         return workgroups <= 2 * holds and keys >= 40 + max(0, workgroups - 3 * holds // 4)
 
+    def _window_takes_step(self, S, span, nh, nkv, Dk, Dv, in_keys):
+        """Whether a step of one token a sequence takes the kernel for it, or the one of prompts over shares of the keys.  Values
+        with pages of their own: always, where it is built.  A latent's workgroup has 16 heads and its four wavefronts share a block, which is the
+        shortest way to one (1,000 keys, 16 heads, 96 / 64 and 576 / 512: 7.9 us and 10, in shares 9.3 and 17), but what more heads and blocks
+        read again: as long as a CU has two blocks of 32 keys, of a wide latent with more than 16 heads counted once for all of them
+        (us, step / shares: 96 / 64, 16 heads, 64 requests at 300 keys 11.0 / 10.0, at 2,000 37 / 28, 40 heads on 2 128 / 50; 576 / 512, 32 heads, 32
+        requests at 200 0.89 of the shares', at 1,000 1.26, 40 on 2, 64 at 2,000 201 / 139; 16 heads ahead at every number)."""
+        if not in_keys:
+            return True
+        blocks, tiles = -(-span // 32), -(-(nh // nkv) // 16)
+        if Dk + Dv <= 320:
+            return S * nkv * blocks * tiles <= 2 * self._num_cus and blocks <= 4 * self.WINDOW_MFMA_MAX_SHARES
+        return tiles == 1 or S * nkv * blocks <= 2 * self._num_cus
+
     def _lazy(self, stem):
         """The library of ``stem`` for this table's dtype, compiled and loaded at first use."""
         if stem not in self._lib:
@@ -262,7 +276,7 @@ class WindowOps:
         if window or chunk:
             span = min(span, min(n for n in (window, chunk) if n) + int(keep_first))
         few = mfma and batch.max_q_len > 1 and self._window_few(T, S, batch.max_q_len, batch.max_ctx_len, span, nh, nkv, Dk, Dv, v_cache is None)
-        step = mfma and T == S and batch.max_q_len == 1
+        step = mfma and T == S and batch.max_q_len == 1 and self._window_takes_step(S, span, nh, nkv, Dk, Dv, v_cache is None)
         if batch.max_q_len == 1:
             blocks = self._window_step_blocks(Dk, Dv, v_cache is None) if step else 0
             if blocks:

@@ -35,9 +35,11 @@ def exact(q, keys, values, pos, scale, window, keep, chunk, softcap, slopes, sin
                                               (20, 1, 256, 256, True)])
 @pytest.mark.parametrize("window,keep,chunk,page,shares", [(None, 0, None, 16, 32), (9, 3, None, 16, 32), (40, 33, None, 32, 3), (None, 0, 48, 16, 5),
                                                           (1, 1, None, 64, 32), (700, 4, 512, 16, 1), (None, 0, None, 16, 1)])
-def test_steps_of_one_token(H, G, Dk, Dv, in_keys, window, keep, chunk, page, shares):
+@pytest.mark.parametrize("step", [True, False])
+def test_steps_of_one_token(H, G, Dk, Dv, in_keys, window, keep, chunk, page, shares, step):
     ops = HipOps(torch.bfloat16, "cuda:0")
     ops.WINDOW_MFMA_MAX_SHARES = shares
+    ops._window_takes_step = lambda *a: step                                       # (the kernel for steps, shares of the one for prompts)
     gen = torch.Generator().manual_seed(Dk + keep)
     # the first token, the ends of a page and of a block, a context of more blocks than a lane asks table entries for
     lens = [1, 16, 32, 33, 75, 4700 if shares == 1 else 1100]

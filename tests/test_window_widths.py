@@ -81,3 +81,13 @@ def prompts(lens, heads, kv_heads, Dk, Dv, in_keys, cached=0):
     ([2048], 16, 2, 192, 128, False, True), ([4096], 16, 2, 192, 128, False, False), ([300] * 4, 16, 2, 192, 128, False, True)])   # 78 / 93, 256 / 202, 17 / 20
 def test_wavefronts_of_a_prompt_s_workgroups(lens, heads, kv_heads, Dk, Dv, in_keys, few):
     assert prompts(lens, heads, kv_heads, Dk, Dv, in_keys) is few
+
+
+# (us measured in the kernel for steps / in shares of the one for prompts beside each)
+@pytest.mark.parametrize("S,keys,heads,kv_heads,Dk,Dv,in_keys,step", [
+    (1, 1000, 16, 1, 96, 64, True, True), (16, 300, 16, 1, 96, 64, True, True), (64, 2000, 16, 1, 96, 64, True, False),     # 7.9 / 9.3, 7.8 / 8.9, 37 / 28
+    (1, 8000, 16, 1, 96, 64, True, False), (64, 300, 40, 2, 192, 128, True, False),                                         # 21 / 17, 25 / 18
+    (256, 500, 16, 1, 576, 512, True, True), (1, 8000, 128, 1, 576, 512, True, True),                                       # 53 / 67, 0.73 of it
+    (64, 2000, 40, 2, 576, 512, True, False), (128, 500, 40, 2, 576, 512, True, False), (64, 2000, 16, 2, 128, 128, False, True)])   # 201 / 139, 102 / 68
+def test_kernel_of_a_step(S, keys, heads, kv_heads, Dk, Dv, in_keys, step):
+    assert Recorded()._window_takes_step(S, keys, heads, kv_heads, Dk, Dv, in_keys) is step
