@@ -64,7 +64,7 @@ class WindowOps:
         shortest way to one (1,000 keys, 16 heads, 96 / 64 and 576 / 512: 7.9 us and 10, in shares 9.3 and 17), but what more heads and blocks
         read again: as long as a CU has two blocks of 32 keys, of a wide latent with more than 16 heads counted once for all of them
         (us, step / shares: 96 / 64, 16 heads, 64 requests at 300 keys 11.0 / 10.0, at 2,000 37 / 28, 40 heads on 2 128 / 50; 576 / 512, 32 heads, 32
-        requests at 200 0.89 of the shares', at 1,000 1.26, 40 on 2, 64 at 2,000 201 / 139; 16 heads ahead at every number)."""
+        requests at 200 0.89 of the shares', at 1,000 1.26, 40 on 2, 64 at 2,000 201 / 120; 16 heads ahead at every number)."""
         if not in_keys:
             return True
         blocks, tiles = -(-span // 32), -(-(nh // nkv) // 16)
