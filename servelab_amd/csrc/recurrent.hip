@@ -881,168 +881,159 @@ __global__ void normaliser_kernel(const MatrixScan a) {
   if (threadIdx.x == 0) slot[(size_t)a.H * a.D + h] = from[a.D];
 }
 
-// A step of one token a sequence: the recurrences above, without their LDS.  P lanes share a column of S as there, 256 / P columns side by
-// side and J of them one after the other a lane, so that a lane has up to 2 J pieces of the state on their way at once; what a token
-// brings (q, k, decays, gates) every lane works out for the channels it owns.  Of a column a lane owns channels 4 p .. 4 p + 3 of its
-// first half and of its second: a load of a column's lanes is one run of memory.  The matrix LSTM's n and m are read, and
-// carried on, by every column's lanes; the first ones leave the new values for normaliser_kernel.
-// Bound by streaming the state in and out: 8 requests of 14 heads of 128 x 256, forget form, 29 MB, cold, 7.4 us (the walking kernel
-// 16; a copy in place 6.3), one request of 8 such heads 2.9 (2.2), 32 requests of 14 28 (20).
+// A step of one token a sequence.  P lanes share a column of S as there, 256 / P columns a workgroup, one a lane.  Of a column a lane owns
+// channels 4 p .. 4 p + 3 of its first half and of its second: a load of a column's lanes is one run of memory.  What the token
+// brings (q, k, decays, gates, the matrix LSTM's n) a thread works out for a channel or two, while the state is on its way, and all columns'
+// lanes read it from LDS.  (Every lane for the eight channels it owns, without LDS, is most of what a SIMD then does: forget form, 8
+// requests of 8 heads of 128 x 256 14.8 us, and 10.5 in the kernel that walks tokens; 4.9 here.)  The matrix LSTM's new n and m are left for
+// normaliser_kernel.
+// Bound by streaming the state in and out, us, cold, in the walking kernel / here, forget form, 128 x 256: one request of
+// 8 heads 4.6 / 3.0, 8 of 14, 29 MB, 23.6 / 13.5, 64 of 14, 235 MB, 151 / 81; the matrix LSTM, 64 of 4 heads of 256 x 512, 268 MB, 173 / 61.
 struct Channels8 { float v[8]; };
 typedef float state_v4 __attribute__((ext_vector_type(4)));
-template <int MODE, int J>
-__global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, int P, int lgP, int aligned) {
+template <int MODE, bool ALIGNED>
+__global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, int P, int lgP) {
   constexpr bool SCALAR = MODE == SCAN_LSTM || MODE == SCAN_SSD || MODE == SCAN_DELTA_HEAD;
+  constexpr bool THIRD = !SCALAR || MODE == SCAN_LSTM;   // decays, or the normaliser n, a channel
   const int s = blockIdx.x, h = blockIdx.y, g = h / (a.H / a.G);
   const int p = threadIdx.x & (P - 1), cl = threadIdx.x >> lgP, cols = 256 >> lgP;
   const int r0 = 4 * p, r1 = 4 * P + 4 * p, D = a.D;
   const bool fresh = a.positions[s] == 0;
   float* slot = a.state + (size_t)a.slots[s] * a.state_stride;
-  // (aligned: D is a multiple of four, so that a half is there or not; what is not is read from the last one and left out)
+  // (ALIGNED: D is a multiple of four, so that a half is there or not; what is not is read from the last one and left out)
   const int a0 = min(r0, D - 4), a1 = min(r1, D - 4);
   const bool all = D == 8 * P;
-  // the 8 values of a row of D channels that this lane owns
-  auto channels = [&](const float* row, float beyond) {
-    Channels8 c;
-    if (aligned) {
-      const scan_f4 x = *(const scan_f4*)(row + a0), y = *(const scan_f4*)(row + a1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c.v[i] = all || r0 < D ? x.v[i] : beyond, c.v[4 + i] = all || r1 < D ? y.v[i] : beyond;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = i < 4 ? r0 + i : r1 + i - 4;
-        c.v[i] = r < D ? row[r] : beyond;
-      }
-    }
-    return c;
-  };
   const float* row = a.src + (size_t)s * a.src_stride;
-  Channels8 S[J], q = channels(row + a.q_col + g * D, 0.f), k = channels(row + a.k_col + g * D, 0.f), d, n;
-  if (!SCALAR && MODE != SCAN_FORGET) d = channels(a.log_decay + ((size_t)s * a.H + h) * D, 0.f);
-  if (MODE == SCAN_FORGET) d = channels(a.lower + h * D, 0.f);
-  float g0 = 0.f, g1 = 0.f, v[J];
+  const size_t nS = (size_t)a.H * a.Dv * D;
+  const float* third = MODE == SCAN_LSTM ? slot + nS + (size_t)h * D : MODE == SCAN_FORGET ? a.lower + h * D : a.log_decay + ((size_t)s * a.H + h) * D;
+  float own[3][2];                                       // q, k and the third of two channels, worked out for the whole workgroup
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int r = min((int)threadIdx.x + 256 * e, D - 1);
+    own[0][e] = row[a.q_col + g * D + r];
+    own[1][e] = row[a.k_col + g * D + r];
+    if (THIRD) own[2][e] = third[r];
+  }
+  float g0 = 0.f, g1 = 0.f;
   if (MODE != SCAN_DECAY && MODE != SCAN_FORGET) {
     const float* gr = a.gates + (size_t)s * a.gate_stride;
     g0 = gr[a.i_col + h];
     if (MODE == SCAN_LSTM || MODE == SCAN_DELTA_HEAD) g1 = gr[a.f_col + h];
   }
-  const int j0 = blockIdx.z * J * cols + cl;             // columns j0, j0 + cols, ..
+  const float m = MODE == SCAN_LSTM ? slot[nS + (size_t)a.H * D + h] : 0.f;
+  const bool stepped = MODE == SCAN_SSD || MODE == SCAN_DELTA_HEAD;
+  const float rate = stepped ? a.rates[h] : 0.f, bias = stepped ? a.step_bias[h] : 0.f;
+  const int j = blockIdx.z * cols + cl, jc = min(j, a.Dv - 1);
+  const float v = row[a.v_col + h * a.Dv + jc];
+  // (a fresh sequence's slot is read as well and left out: its loads would stand behind a condition)
+  float* col = slot + ((size_t)h * a.Dv + jc) * D;
+  state_v4 x, y;
+  if (ALIGNED) {
+    x = __builtin_nontemporal_load((const state_v4*)(col + a0));
+    y = __builtin_nontemporal_load((const state_v4*)(col + a1));
+  } else {
 #pragma unroll
-  for (int u = 0; u < J; ++u) {
-    const int j = min(j0 + u * cols, a.Dv - 1);
-    v[u] = row[a.v_col + h * a.Dv + j];
-    const float* col = slot + ((size_t)h * a.Dv + j) * D;
-    if (fresh) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) S[u].v[i] = 0.f;
-    } else if (aligned) {
-      const state_v4 x = __builtin_nontemporal_load((const state_v4*)(col + a0)), y = __builtin_nontemporal_load((const state_v4*)(col + a1));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) S[u].v[i] = all || r0 < D ? x[i] : 0.f, S[u].v[4 + i] = all || r1 < D ? y[i] : 0.f;
-    } else {
-      S[u] = channels(col, 0.f);
-    }
+    for (int i = 0; i < 4; ++i) x[i] = col[min(r0 + i, D - 1)], y[i] = col[min(r1 + i, D - 1)];
   }
-  const size_t nS = (size_t)a.H * a.Dv * D;
-  float m = 0.f;
+  // what the token brings: gates by one thread, but what the matrix LSTM's n needs by all
+  __shared__ __attribute__((aligned(16))) float token[THIRD ? 3 : 2][512];
+  __shared__ float gated[2];
+  float keep = 0.f, add = 0.f, divisor = 1.f, top = 0.f;
   if (MODE == SCAN_LSTM) {
-    if (fresh) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) n.v[i] = 0.f;
+    const float ig = a.cap * tanhf(g0 / a.cap), fg = logsigmoidf_(a.cap * tanhf(g1 / a.cap)), m0 = fresh ? 0.f : m;
+    top = fmaxf(fg + m0, ig);
+    keep = expf(fg + m0 - top);
+    add = expf(ig - top);
+  } else if (MODE != SCAN_DECAY && MODE != SCAN_FORGET && threadIdx.x == 0) {
+    if (MODE == SCAN_SSD) {
+      add = softplusf_(g0 + bias);
+      keep = expf(-expf(rate) * add);
     } else {
-      n = channels(slot + nS + (size_t)h * D, 0.f);
-      m = slot[nS + (size_t)a.H * D + h];
+      add = sigmoidf_(g0);
+      if (MODE == SCAN_DELTA_HEAD) keep = expf(-expf(rate) * softplusf_(g1 + bias));
     }
+    gated[0] = keep;
+    gated[1] = add;
   }
-  // what the token brings
-  float keep = 0.f, add = 0.f, divisor = 1.f;
-  if (MODE == SCAN_FORGET) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+  for (int e = 0; e < 2; ++e) {
+    const int r = threadIdx.x + 256 * e;
+    if (r >= 8 * P) continue;
+    const bool in = r < D;
+    float qr = own[0][e], kr = own[1][e], x = THIRD ? own[2][e] : 0.f;
+    if (MODE == SCAN_FORGET) {
       // (as in matrix_scan_kernel: f and 1 - f each from its own side; q passes silu)
-      const bool in = (i < 4 ? r0 + i : r1 + i - 4) < D;
-      const float en = expf(-fabsf(k.v[i])), big = 1.f / (1.f + en), small = en * big, bound = d.v[i];
-      const bool pos = k.v[i] >= 0.f;
-      q.v[i] = q.v[i] * sigmoidf_(q.v[i]) * a.q_scale;
-      k.v[i] = in ? (1.f - bound) * (pos ? small : big) : 0.f;
-      d.v[i] = in ? bound + (1.f - bound) * (pos ? big : small) : 1.f;
+      const float en = expf(-fabsf(kr)), big = 1.f / (1.f + en), small = en * big, bound = x;
+      const bool pos = kr >= 0.f;
+      qr *= sigmoidf_(qr);
+      kr = (1.f - bound) * (pos ? small : big);
+      x = bound + (1.f - bound) * (pos ? big : small);
+    } else if (MODE == SCAN_LSTM) {
+      x = keep * (fresh ? 0.f : x) + kr * add;
+      if (a.write && blockIdx.z == 0 && in) a.normaliser[((size_t)s * a.H + h) * (D + 1) + r] = x;
+    } else if (THIRD) {
+      x = expf(x);
     }
+    token[0][r] = in ? qr * a.q_scale : 0.f;
+    token[1][r] = in ? kr : 0.f;
+    if (THIRD) token[THIRD ? 2 : 0][r] = in ? x : MODE == SCAN_LSTM ? 0.f : 1.f;
+  }
+  if (MODE == SCAN_LSTM && a.write && blockIdx.z == 0 && threadIdx.x == 0) a.normaliser[((size_t)s * a.H + h) * (D + 1) + D] = top;
+  __syncthreads();
+  auto owned = [&](const float* t) {
+    Channels8 c;
+    const scan_f4 lo = *(const scan_f4*)(t + r0), hi = *(const scan_f4*)(t + r1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c.v[i] = lo.v[i], c.v[4 + i] = hi.v[i];
+    return c;
+  };
+  const Channels8 q = owned(token[0]), k = owned(token[1]), d = owned(token[THIRD ? 2 : 0]);      // (d: the matrix LSTM's new n)
+  auto sum_of = [&](const float* x) { return group_sum(rows_sum<8>(x), P); };
+  if (MODE == SCAN_LSTM) {
+    float part[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[i] = d.v[i] * q.v[i];
+    divisor = fmaxf(fabsf(sum_of(part)), expf(-top)) + 1e-6f;
+  } else if (MODE != SCAN_DECAY && MODE != SCAN_FORGET) {
+    keep = gated[0];
+    add = gated[1];
+  }
+  float S[8], part[8], in = v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    S[i] = !fresh && (ALIGNED ? all || r0 < D : r0 + i < D) ? x[i] : 0.f;
+    S[4 + i] = !fresh && (ALIGNED ? all || r1 < D : r1 + i < D) ? y[i] : 0.f;
+  }
+  if (MODE == SCAN_DELTA) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[i] = S[i] * (d.v[i] * k.v[i]);
+    in = add * (v - sum_of(part));
+  } else if (MODE == SCAN_DELTA_HEAD) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[i] = S[i] * k.v[i];
+    in = add * (v - keep * sum_of(part));
+  } else if (MODE == SCAN_LSTM || MODE == SCAN_SSD) {
+    in = add * v;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    S[i] = (SCALAR ? keep : d.v[i]) * S[i] + k.v[i] * in;
+    part[i] = S[i] * q.v[i];
+  }
+  float o = sum_of(part);
+  if (MODE == SCAN_LSTM) o = o / divisor;
+  if (MODE == SCAN_SSD) o += a.skip[h] * v;
+  if (j >= a.Dv) return;
+  if (p == 0) a.out[((size_t)s * a.H + h) * a.Dv + j] = o;
+  if (!a.write) return;
+  if (ALIGNED) {
+    if (r0 < D) __builtin_nontemporal_store(state_v4{S[0], S[1], S[2], S[3]}, (state_v4*)(col + r0));
+    if (r1 < D) __builtin_nontemporal_store(state_v4{S[4], S[5], S[6], S[7]}, (state_v4*)(col + r1));
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      q.v[i] *= a.q_scale;
-      if (!SCALAR) d.v[i] = expf(d.v[i]);
-    }
-  }
-  if (MODE == SCAN_DELTA) add = sigmoidf_(g0);
-  if (MODE == SCAN_DELTA_HEAD) {
-    keep = expf(-expf(a.rates[h]) * softplusf_(g1 + a.step_bias[h]));
-    add = sigmoidf_(g0);
-  }
-  if (MODE == SCAN_SSD) {
-    add = softplusf_(g0 + a.step_bias[h]);
-    keep = expf(-expf(a.rates[h]) * add);
-  }
-  auto sum_of = [&](const float* x) { return group_sum(rows_sum<8>(x), P); };
-  if (MODE == SCAN_LSTM) {
-    const float ig = a.cap * tanhf(g0 / a.cap), fg = logsigmoidf_(a.cap * tanhf(g1 / a.cap));
-    const float top = fmaxf(fg + m, ig);
-    keep = expf(fg + m - top);
-    add = expf(ig - top);
-    float part[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      n.v[i] = keep * n.v[i] + k.v[i] * add;
-      part[i] = n.v[i] * q.v[i];
-    }
-    divisor = fmaxf(fabsf(sum_of(part)), expf(-top)) + 1e-6f;
-    if (a.write && blockIdx.z == 0 && cl == 0) {
-      float* to = a.normaliser + ((size_t)s * a.H + h) * (D + 1);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = i < 4 ? r0 + i : r1 + i - 4;
-        if (r < D) to[r] = n.v[i];
-      }
-      if (p == 0) to[D] = top;
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < J; ++u) {
-    float part[8], in = v[u];
-    if (MODE == SCAN_DELTA) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) part[i] = S[u].v[i] * (d.v[i] * k.v[i]);
-      in = add * (v[u] - sum_of(part));
-    } else if (MODE == SCAN_DELTA_HEAD) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) part[i] = S[u].v[i] * k.v[i];
-      in = add * (v[u] - keep * sum_of(part));
-    } else if (MODE == SCAN_LSTM || MODE == SCAN_SSD) {
-      in = add * v[u];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      S[u].v[i] = (SCALAR ? keep : d.v[i]) * S[u].v[i] + k.v[i] * in;
-      part[i] = S[u].v[i] * q.v[i];
-    }
-    float o = sum_of(part);
-    if (MODE == SCAN_LSTM) o = o / divisor;
-    if (MODE == SCAN_SSD) o += a.skip[h] * v[u];
-    const int j = j0 + u * cols;
-    if (j >= a.Dv) continue;
-    if (p == 0) a.out[((size_t)s * a.H + h) * a.Dv + j] = o;
-    if (!a.write) continue;
-    float* col = slot + ((size_t)h * a.Dv + j) * D;
-    if (aligned) {
-      if (r0 < D) __builtin_nontemporal_store(state_v4{S[u].v[0], S[u].v[1], S[u].v[2], S[u].v[3]}, (state_v4*)(col + r0));
-      if (r1 < D) __builtin_nontemporal_store(state_v4{S[u].v[4], S[u].v[5], S[u].v[6], S[u].v[7]}, (state_v4*)(col + r1));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = i < 4 ? r0 + i : r1 + i - 4;
-        if (r < D) col[r] = S[u].v[i];
-      }
+      const int r = i < 4 ? r0 + i : r1 + i - 4;
+      if (r < D) col[r] = S[i];
     }
   }
 }
@@ -1112,23 +1103,21 @@ extern "C" const char* sl_matrix_scan(int mode, const float* src, int src_stride
   int P = 1;
   while (P * SCAN_ROWS < D) P <<= 1;
   if (single) {
-    // Four columns a lane where that still leaves five workgroups to four CUs: fewer, and a lane's work for a token is shared by too
-    // few (us, cold, one column / four: 448 workgroups of four 10.7 / 7.4, 256 5.1 / 5.8, 128 4.5 / 5.0, 64 3.7 / 5.0).
     const int per = 256 / P;
-    const bool four = 4ll * S * H * ((Dv + 4 * per - 1) / (4 * per)) >= 5ll * device_cus();
-    const bool aligned = (uintptr_t)src % 16 == 0 && (uintptr_t)log_decay % 16 == 0 && (uintptr_t)lower % 16 == 0 && (uintptr_t)state % 16 == 0 &&
-                         state_stride % 4 == 0 && src_stride % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 && D % 4 == 0;
-    auto run = [&](auto wide, auto narrow) {
-      if (four) wide<<<dim3(S, H, (Dv + 4 * per - 1) / (4 * per)), 256, 0, stream>>>(a, P, __builtin_ctz(P), aligned);
-      else narrow<<<dim3(S, H, (Dv + per - 1) / per), 256, 0, stream>>>(a, P, __builtin_ctz(P), aligned);
+    const bool aligned = (uintptr_t)state % 16 == 0 && state_stride % 4 == 0 && D % 4 == 0;
+    auto run = [&](auto m) {
+      constexpr int M = decltype(m)::value;
+      const dim3 grid(S, H, (Dv + per - 1) / per);
+      if (aligned) matrix_step_kernel<M, true><<<grid, 256, 0, stream>>>(a, P, __builtin_ctz(P));
+      else matrix_step_kernel<M, false><<<grid, 256, 0, stream>>>(a, P, __builtin_ctz(P));
     };
-    if (mode == SCAN_DECAY) run(matrix_step_kernel<SCAN_DECAY, 4>, matrix_step_kernel<SCAN_DECAY, 1>);
-    else if (mode == SCAN_DELTA) run(matrix_step_kernel<SCAN_DELTA, 4>, matrix_step_kernel<SCAN_DELTA, 1>);
-    else if (mode == SCAN_SSD) run(matrix_step_kernel<SCAN_SSD, 4>, matrix_step_kernel<SCAN_SSD, 1>);
-    else if (mode == SCAN_DELTA_HEAD) run(matrix_step_kernel<SCAN_DELTA_HEAD, 4>, matrix_step_kernel<SCAN_DELTA_HEAD, 1>);
-    else if (mode == SCAN_FORGET) run(matrix_step_kernel<SCAN_FORGET, 4>, matrix_step_kernel<SCAN_FORGET, 1>);
+    if (mode == SCAN_DECAY) run(std::integral_constant<int, SCAN_DECAY>{});
+    else if (mode == SCAN_DELTA) run(std::integral_constant<int, SCAN_DELTA>{});
+    else if (mode == SCAN_SSD) run(std::integral_constant<int, SCAN_SSD>{});
+    else if (mode == SCAN_DELTA_HEAD) run(std::integral_constant<int, SCAN_DELTA_HEAD>{});
+    else if (mode == SCAN_FORGET) run(std::integral_constant<int, SCAN_FORGET>{});
     else {
-      run(matrix_step_kernel<SCAN_LSTM, 4>, matrix_step_kernel<SCAN_LSTM, 1>);
+      run(std::integral_constant<int, SCAN_LSTM>{});
       if (write) normaliser_kernel<<<dim3(S, H), 64, 0, stream>>>(a);
     }
     return sl_launch_status();

@@ -12,7 +12,7 @@ DEV = "cuda:0"
 
 
 # heads of 16, 8, 32 and 64 lanes a column, of channels that no load of four divides and that no lane's eight do; value channels that no
-# workgroup divides; few blocks (one column a lane) and many (four)
+# workgroup divides; few blocks and many
 @pytest.mark.parametrize("S,H,G,D,Dv", [(3, 2, 2, 128, 256), (2, 3, 3, 20, 24), (5, 2, 2, 72, 15), (2, 1, 1, 200, 33), (2, 2, 1, 256, 16),
                                         (1, 4, 2, 64, 40), (3, 2, 2, 50, 7), (2, 1, 1, 512, 9), (40, 8, 8, 128, 130), (70, 16, 8, 60, 64), (10, 8, 8, 128, 250)])
 @pytest.mark.parametrize("mode", ["decay", "delta", "delta, decay a head", "state space", "forget", "lstm"])
@@ -27,7 +27,7 @@ def test_steps_of_one_token(mode, S, H, G, D, Dv, monkeypatch):
     state = torch.randn(S + 2, size + 8, generator=g) * 0.3
     for i in range(S):
         if starts[i] == 0:
-            state[slots[i]] = float("nan")                           # what a fresh sequence's slot holds is not read
+            state[slots[i]] = float("nan")                           # what a fresh sequence's slot holds is left out
     hip, emu = HipOps(torch.float32, DEV), EmulatedOps(torch.float32)
     dev, cpu = sequences([1] * S, starts, slots, DEV), sequences([1] * S, starts, slots, "cpu")
     cpu.q_lens, cpu.starts = [1] * S, starts
