@@ -556,37 +556,37 @@ __global__ __launch_bounds__(TILE_THREADS) void attention_general_tile_kernel(
 #if defined(SL_F32)
 // ---------------------------------------------------------------------------
 // Prompt portions in float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 factors and sums), for head sizes in
-// steps of 16 fixed at compile time.  A workgroup owns 32 columns, (token, head of the group) pairs of one sequence and one kv
-// head, a wavefront 16 of them; two teams of two wavefronts walk every other block of 32 keys, staged in LDS as K [32][D + 4] and
-// V^T [D][36], and meet at the end; a team's next block travels from the pages to registers meanwhile.  S^T = K Q^T, softmax with a running
+// steps of 16 fixed at compile time.  A workgroup of four wavefronts owns columns, (token, head of the group) pairs of one sequence and
+// one kv head, a wavefront 16 of them: 64 columns, or 32 in two teams that walk every other block of keys and meet at the end.  Blocks
+// are 32 keys, staged in LDS as K [32][D + 4] and V^T [D][36]; a team's next one travels from the pages to registers meanwhile.  S^T = K Q^T, softmax with a running
 // maximum per column, O^T += V^T P^T: a lane's scores of a 16 x 16 block (keys 4 (lane / 16) .. + 3 of column lane % 16) are the
 // second product's operand as they are.  What bounds it is the matrix instructions of the longest tile: 128 a block and
 // wavefront at D 128, 1.7 us.  One prompt of 333 tokens and two shorter ones, 12 heads on 2, D 128: 287 us with the FMA tiles, 74 with
-// four wavefronts over 64 columns and loads behind conditions, 45 without those, 41 with two teams over 64 columns, 32 here.  The second product multiplies the zero weights of keys that a column does not see too, which an infinite or NaN
+// four wavefronts over 64 columns and loads behind conditions, 45 without those, 41 with two teams over 64 columns, 31 with two over 32.  The second product multiplies the zero weights of keys that a column does not see too, which an infinite or NaN
 // value turns into NaN: a wavefront with a result that is not finite takes its columns again key by key, over seen keys alone.
 // ---------------------------------------------------------------------------
 typedef float att_v4 __attribute__((ext_vector_type(4)));
 
-constexpr int F32_TEAMS = 2, F32_TEAM = 128, F32_COLS = 32;      // teams of two wavefronts, on the same 32 columns and every other block
-template <int D>
-__global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kernel(
+template <int D, int TEAMS>
+__global__ __launch_bounds__(256) void attention_f32_mfma_kernel(
     const float* __restrict__ qkv, int row_stride, const float* __restrict__ kc, const float* __restrict__ vc,
     const int* __restrict__ block_tables, int max_pages, const int* __restrict__ cu_q, const int* __restrict__ positions,
     int nh, int nkv, int page, float scale, int window, float* __restrict__ out) {
-  constexpr int KR = D + 4, VR = 36, NP = 8 * D / F32_TEAM;      // row lengths; 16-byte pieces of K and of V^T a thread stages of a block
+  constexpr int TEAM = 256 / TEAMS, COLS = 64 / TEAMS; // threads of a team, and the columns that all teams share
+  constexpr int KR = D + 4, VR = 36, NP = 8 * D / TEAM;      // row lengths; 16-byte pieces of K and of V^T a thread stages of a block
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int team = __builtin_amdgcn_readfirstlane(threadIdx.x / F32_TEAM), tid = threadIdx.x % F32_TEAM;
+  const int team = __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM), tid = threadIdx.x % TEAM;
   float* ks = lds + team * (32 * KR + D * VR);         // [32][KR]
   float* vt = ks + 32 * KR;                            // [D][VR]
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, gq = lane >> 4;
   const int seq = blockIdx.z, kvh = blockIdx.y, g = nh / nkv;
   const int q0 = cu_q[seq], qlen = cu_q[seq + 1] - q0, ncols = qlen * g;
   // (tiles of late tokens see the most keys: they come first)
-  const int tile = (int)gridDim.x - 1 - (int)blockIdx.x, c0 = tile * F32_COLS;
+  const int tile = (int)gridDim.x - 1 - (int)blockIdx.x, c0 = tile * COLS;
   if (c0 >= ncols) return;
   const int pos0 = positions[q0];
   const int* table = block_tables + (size_t)seq * max_pages;
-  const int c_last = min(c0 + F32_COLS - 1, ncols - 1);
+  const int c_last = min(c0 + COLS - 1, ncols - 1);
   const int kmax = pos0 + c_last / g;
   const int kmin = window > 0 ? max(0, pos0 + c0 / g - window + 1) : 0;
   const int cw = c0 + 16 * wave;
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kerne
     const float *valuesA = vc + headA * D * page + inA, *valuesB = vc + headB * D * page + inB;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int idx = tid + F32_TEAM * i, kl = idx / (D / 4) & 15, d4 = idx % (D / 4);
+      const int idx = tid + TEAM * i, kl = idx / (D / 4) & 15, d4 = idx % (D / 4);
       kr[i] = *(const att_v4*)((i >= NP / 2 ? keysB : keysA) + kl * D + 4 * d4);      // (the first NP / 2 pieces are 16 rows)
       vr[i] = *(const att_v4*)((idx & 4 ? valuesB : valuesA) + (idx / 8) * page + 4 * (idx & 3));
     }
@@ -629,15 +629,15 @@ __global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kerne
   int asked = 0;
   if (mine <= b1) {
     fetch(32 * mine, ask_pages(32 * mine));
-    if (mine + F32_TEAMS <= b1) asked = ask_pages(32 * (mine + F32_TEAMS));
+    if (mine + TEAMS <= b1) asked = ask_pages(32 * (mine + TEAMS));
   }
-  for (int b = mine; b - team <= b1; b += F32_TEAMS) {   // (as many rounds for both teams; the second may have no block in the last)
+  for (int b = mine; b - team <= b1; b += TEAMS) {   // (as many rounds for both teams; the second may have no block in the last)
     const int kbase = 32 * b;
     __syncthreads();                                   // the last block's readers are done
     const bool all_seen = kbase >= kmin && kbase + 31 <= kmax;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int idx = tid + F32_TEAM * i;
+      const int idx = tid + TEAM * i;
       if (!all_seen) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -649,9 +649,9 @@ __global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kerne
       *(att_v4*)(vt + (idx / 8) * VR + 4 * (idx % 8)) = vr[i];
     }
     __syncthreads();
-    if (b + F32_TEAMS <= b1) {
-      fetch(kbase + 32 * F32_TEAMS, asked);
-      if (b + 2 * F32_TEAMS <= b1) asked = ask_pages(kbase + 64 * F32_TEAMS);
+    if (b + TEAMS <= b1) {
+      fetch(kbase + 32 * TEAMS, asked);
+      if (b + 2 * TEAMS <= b1) asked = ask_pages(kbase + 64 * TEAMS);
     }
     if (!wave_live || b > b1) continue;                          // (a wavefront without columns only helps staging)
     att_v4 s[2];
@@ -704,22 +704,22 @@ __global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kerne
     }
   }
   // the first team takes what the second has of its columns
-  att_v4* os = (att_v4*)lds;                           // [D / 16][F32_TEAM]
-  float2* ml = (float2*)(os + F32_TEAM * (D / 16));
-  __syncthreads();
-  if (team == 1) {
+  if constexpr (TEAMS == 2) {
+    att_v4* os = (att_v4*)lds;                           // [D / 16][TEAM]
+    float2* ml = (float2*)(os + TEAM * (D / 16));
+    __syncthreads();
+    if (team == 1) {
 #pragma unroll
-    for (int dd = 0; dd < D / 16; ++dd) os[F32_TEAM * dd + tid] = o[dd];
-    ml[tid] = make_float2(m, l);
-  }
-  __syncthreads();
-  if (team == 1) return;
-  {
+      for (int dd = 0; dd < D / 16; ++dd) os[TEAM * dd + tid] = o[dd];
+      ml[tid] = make_float2(m, l);
+    }
+    __syncthreads();
+    if (team == 1) return;
     const float2 other = ml[tid];
     const float both = fmaxf(m, other.x), ours = m == -INFINITY ? 0.f : expf(m - both), theirs = other.x == -INFINITY ? 0.f : expf(other.x - both);
 #pragma unroll
     for (int dd = 0; dd < D / 16; ++dd) {
-      const att_v4 x = os[F32_TEAM * dd + tid];
+      const att_v4 x = os[TEAM * dd + tid];
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[dd][i] = fmaf(x[i], theirs, o[dd][i] * ours);
     }
@@ -768,10 +768,10 @@ __global__ __launch_bounds__(F32_TEAM * F32_TEAMS) void attention_f32_mfma_kerne
 #endif
 
 // Sequences [0, num_seqs) of the batch, prompt portions of at most max_q_len
-// tokens each (their tokens come first in the batch).  D % 16 == 0.
+// tokens each, `tokens` in all, that see at most `longest` keys (their tokens come first in the batch).  D % 16 == 0.
 extern "C" const char* sl_attention_general_tiles(
     const void* qkv, int row_stride, const void* kc, const void* vc, const int* block_tables,
-    int max_pages, const int* cu_q, const int* positions, int num_seqs, int max_q_len, int nh,
+    int max_pages, const int* cu_q, const int* positions, int num_seqs, int max_q_len, int tokens, int longest, int nh,
     int nkv, int D, int page, float scale, int window, void* out, hipStream_t stream) {
   SL_CHECK(num_seqs >= 0 && max_q_len >= 1 && nh > 0 && nkv > 0 && nh % nkv == 0,
            "attention tiles: heads must be a positive multiple of kv heads");
@@ -785,23 +785,38 @@ extern "C" const char* sl_attention_general_tiles(
   SL_CHECK(tiles <= 1 << 30, "attention tiles: too many column tiles");
   const dim3 grid((unsigned)tiles, nkv, num_seqs);
 #if defined(SL_F32)
-  // (head sizes of the shapes served; from 32 columns on a tile of 64 is filled well enough to win at every length measured)
+  // (head sizes of the shapes served; from 32 columns on they win at every length measured)
   if ((D == 64 || D == 128) && cols >= 32 && row_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)kc % 16 == 0 &&
       (uintptr_t)vc % 16 == 0 && (uintptr_t)out % 16 == 0) {
-    const dim3 wide((unsigned)((cols + F32_COLS - 1) / F32_COLS), nkv, num_seqs);
-    const size_t room = F32_TEAMS * sizeof(float) * ((size_t)32 * (D + 4) + (size_t)D * 36);
+    // Two teams shorten a workgroup, one lets the chip hold twice as many columns: by the number of one team's workgroups beside the
+    // keys, of which a team of two has none in a context of one block.  Of 438 prompts and batches of seven head shapes the form chosen takes 1.002 of the
+    // faster one's time on average, 1.13 at worst (us, one / two: 14 heads on 2 of 64, 64 prompts of 70 tokens 25 / 36, 16 of 70 11.4 / 12.8, 16 of 150 30 / 25;
+    // 32 on 8 of 128, 32 of 20 15 / 22, 64 of 100 115 / 156, 4 of 700 232 / 240; 12 on 2, three of 512, 100 and 30 64 / 39).
+    const int g = nh / nkv;
+    const long long least = nkv * (((long long)tokens * g + 63) / 64), workgroups = least > (long long)nkv * num_seqs ? least : (long long)nkv * num_seqs;
+    const long long line = device_cus() / 4 + 2ll * longest;
+    const bool few = longest > 32 && workgroups <= (D == 64 ? line + line / 2 : line);
+    const long long columns = few ? 32 : 64;
+    // (among sequences of very different lengths an odd number of places each: workgroups go to the eight dies in turn, and by a multiple of
+    // eight the first tiles of all sequences would be one die's; a prompt of 1,000 tokens beside 15 steps of two at 500 keys, 16 heads of 128, 586 us, 123 so)
+    const bool unequal = 4ll * tokens < 3ll * num_seqs * max_q_len;
+    const dim3 wide((unsigned)((cols + columns - 1) / columns) | (unsigned)unequal, nkv, num_seqs);
+    const size_t room = (few ? 2 : 1) * sizeof(float) * ((size_t)32 * (D + 4) + (size_t)D * 36);
+    const char* failed = nullptr;
     auto run = [&](auto kernel) {
-      kernel<<<wide, F32_TEAM * F32_TEAMS, room, stream>>>((const float*)qkv, row_stride, (const float*)kc, (const float*)vc, block_tables,
+      const hipError_t e = room <= 48 * 1024 ? hipSuccess : hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)room);
+      if (e != hipSuccess) {
+        failed = hipGetErrorString(e);
+        return;
+      }
+      kernel<<<wide, 256, room, stream>>>((const float*)qkv, row_stride, (const float*)kc, (const float*)vc, block_tables,
                                           max_pages, cu_q, positions, nh, nkv, page, scale, window, (float*)out);
     };
-    auto grow = [&](const void* kernel) {
-      return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)room);
-    };
-    const hipError_t e = room <= 48 * 1024 ? hipSuccess : grow(D == 64 ? (const void*)attention_f32_mfma_kernel<64> : (const void*)attention_f32_mfma_kernel<128>);
-    if (e != hipSuccess) return hipGetErrorString(e);
-    if (D == 64) run(attention_f32_mfma_kernel<64>);
-    else run(attention_f32_mfma_kernel<128>);
-    return sl_launch_status();
+    if (few && D == 64) run(attention_f32_mfma_kernel<64, 2>);
+    else if (few) run(attention_f32_mfma_kernel<128, 2>);
+    else if (D == 64) run(attention_f32_mfma_kernel<64, 1>);
+    else run(attention_f32_mfma_kernel<128, 1>);
+    return failed != nullptr ? failed : sl_launch_status();
   }
 #endif
   const int KB = D <= 128 ? 32 : 16;

@@ -280,7 +280,7 @@ class AttentionOps:
             self._check(batch.cu_q, torch.int32, (batch.num_seqs + 1,), "cu_q")
             self._call("attention", "sl_attention_general_tiles", _p(qkv), stride, _p(k_cache),
                        _p(v_cache), _p(block_tables), max_pages, _p(batch.cu_q), _p(batch.positions),
-                       n_pre, batch.max_q_len, nh, nkv, D, page_size, _c_float(scale),
+                       n_pre, batch.max_q_len, n_pre_tok, batch.max_ctx_len, nh, nkv, D, page_size, _c_float(scale),
                        int(window or 0), _p(out))
             first = n_pre_tok
         rest = T - first

@@ -1,5 +1,5 @@
-"""float32 prompts whose two teams of wavefronts take every other block of 32 keys: one block, two, an odd number; NaN where no query sees a
-key, pages without a seen key not in the block table."""
+"""float32 prompts whose two teams of wavefronts take every other block of 32 keys: one block, two, an odd number; prompts of one team: many,
+and of one block; NaN where no query sees a key, pages without a seen key not in the block table."""
 import pytest
 import torch
 
@@ -14,9 +14,11 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("nh,nkv,D", [(6, 1, 128), (14, 2, 64)])
 @pytest.mark.parametrize("page,window", [(16, None), (16, 21), (32, 50)])
-def test_blocks_of_two_teams(nh, nkv, D, page, window):
+@pytest.mark.parametrize("seqs", [[(32, 32), (64, 33), (97, 64), (31, 9), (200, 6)], [(70, 70 - i % 3) for i in range(48)], [(32, 32), (20, 9), (31, 31)],
+                                  [(32, 32)] + [(5, 5)] * 9], ids=["unequal", "many", "one block", "one block, unequal"])
+def test_blocks_of_teams(nh, nkv, D, page, window, seqs):
+    """``seqs``: (context after the step, tokens of it)."""
     ops, emu = HipOps(torch.float32, DEV), EmulatedOps(torch.float32)
-    seqs = [(32, 32), (64, 33), (97, 64), (31, 9), (200, 6)]                              # (context after the step, tokens of it)
     qkv, kc, vc, tables, batch = make_attention_case(torch.float32, nh, nkv, D, page, seqs)[:5]
     want = emu.paged_attention(qkv.cpu(), nh, nkv, D, kc.cpu(), vc.cpu(), page, tables.cpu(), emu_batch(batch), D ** -0.5, window)
     for s, (ctx, n) in enumerate(seqs):
