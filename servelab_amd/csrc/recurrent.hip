@@ -556,15 +556,21 @@ constexpr int SCAN_ROWS = 8;      // key channels a lane owns: channels 8 p .. 8
 
 // Sum over the P lanes that share a column (P a power of two, the lanes adjacent and aligned); every
 // lane gets the sum.  Within 16 lanes by data-parallel moves (neighbours in a quad, the other pair of
-// the quad, the mirrored half row, the mirrored row), beyond that by swaps of rows.
+// the quad, the mirrored half row, the mirrored row), beyond that by exchanges, or by swaps of rows where a token is a chain (SWAPS: two registers more,
+// with which the delta rule's walk has 129 and one workgroup a CU in the place of two: 30 sequences of 3 tokens, 16 heads of 128 x 128, 40 us
+// with exchanges and 72, the others up to a tenth slower).
 template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }
-__device__ __forceinline__ float group_sum(float v, int P) {
+template <bool SWAPS> __device__ __forceinline__ float group_sum(float v, int P) {
   if (P >= 2) v += dpp_move<0xB1>(v);          // quad_perm [1, 0, 3, 2]
   if (P >= 4) v += dpp_move<0x4E>(v);          // quad_perm [2, 3, 0, 1]
   if (P >= 8) v += dpp_move<0x141>(v);         // row_half_mirror
   if (P >= 16) v += dpp_move<0x140>(v);        // row_mirror
+  if (!SWAPS) {
+    for (int w = 16; w < P; w <<= 1) v += __shfl_xor(v, w, SL_WAVE);
+    return v;
+  }
   if (P >= 32) v = rows_meet<16>(v, add_f);
   if (P >= 64) v = rows_meet<32>(v, add_f);
   return v;
@@ -812,7 +818,7 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
         for (int i = 0; i < ROWS; ++i) dk[i] = d[i] * k[i];
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) part[i] = S[i] * dk[i];
-        const float seen = group_sum(rows_sum<ROWS>(part), P);
+        const float seen = group_sum<false>(rows_sum<ROWS>(part), P);
         const float u = sg[tt * 4] * (v - seen);
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
@@ -824,7 +830,7 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) part[i] = S[i] * k[i];
         const float keep = sg[tt * 4];
-        const float u = sg[tt * 4 + 1] * (v - keep * group_sum(rows_sum<ROWS>(part), P));
+        const float u = sg[tt * 4 + 1] * (v - keep * group_sum<false>(rows_sum<ROWS>(part), P));
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
           S[i] = keep * S[i] + k[i] * u;
@@ -838,7 +844,7 @@ __global__ __launch_bounds__(512) void matrix_scan_kernel(const MatrixScan a, in
           part[i] = S[i] * q[i];
         }
       }
-      float o = group_sum(rows_sum<ROWS>(part), P);
+      float o = group_sum<false>(rows_sum<ROWS>(part), P);
       // (the column that carries n leaves the divisor of its token's read-outs)
       if (MODE == SCAN_LSTM && is_n) o = fmaxf(fabsf(o), sg[tt * 4 + 2]) + 1e-6f;
       if (MODE == SCAN_SSD) o += skip_h * v;
@@ -988,7 +994,7 @@ __global__ __launch_bounds__(256) void matrix_step_kernel(const MatrixScan a, in
     return c;
   };
   const Channels8 q = owned(token[0]), k = owned(token[1]), d = owned(token[THIRD ? 2 : 0]);      // (d: the matrix LSTM's new n)
-  auto sum_of = [&](const float* x) { return group_sum(rows_sum<8>(x), P); };
+  auto sum_of = [&](const float* x) { return group_sum<true>(rows_sum<8>(x), P); };
   if (MODE == SCAN_LSTM) {
     float part[8];
 #pragma unroll

@@ -473,8 +473,8 @@ __global__ __launch_bounds__(256) void scan_prepare_channel_kernel(const MatrixS
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      pa[i] = rows_meet<32>(pa[i], add_f);
-      if (DELTA) pm[i] = rows_meet<32>(pm[i], add_f);
+      pa[i] += __shfl_xor(pa[i], 32, SL_WAVE);
+      if (DELTA) pm[i] += __shfl_xor(pm[i], 32, SL_WAVE);
       if (lane < 32) {
         part[(wave * C + u) * 8 + i] = pa[i];
         if (DELTA) part[4 * C * 8 + (wave * C + u) * 8 + i] = pm[i];

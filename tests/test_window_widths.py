@@ -11,14 +11,14 @@ import torch
 from servelab_amd.kernels import HipOps, build
 
 
-def spilled(source, *defines):
-    """Vector registers that each kernel of the library spills."""
+def spilled(source, *defines, what="VGPRs Spill"):
+    """Vector registers that each kernel of the library spills (or another of the compiler's figures)."""
     flags = [f for f in build.BASE_FLAGS if f not in ("-shared", "-fPIC")]
     out = subprocess.run([build.hipcc()] + flags + ["-D" + d for d in defines] + ["--cuda-device-only", "-S", "-o", os.devnull,
                           "-Rpass-analysis=kernel-resource-usage", os.path.join(build.CSRC, source)],
                          check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True).stdout
     names = re.findall(r"Function Name: (\S+)", out)
-    counts = [int(n) for n in re.findall(r"VGPRs Spill: (\d+)", out)]
+    counts = [int(n) for n in re.findall(re.escape(what) + r": (\d+)", out)]
     assert len(names) == len(counts) > 0
     return dict(zip(names, counts))
 
