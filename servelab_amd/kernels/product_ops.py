@@ -106,13 +106,13 @@ class ProductOps:
         LOWER_TILES_MIN_GAIN of it.  Measured on MI355X (us at 1 / 4 / 8 / 16 rows, tiles of 16 against the
         choice): 3584 x 18944, 14 rows (256 tiles on 256 CUs instead of 224): 23.8 / 25.7 / 29.4 / 38.6 against
         25.8 / 26.2 / 28.0 / 33.8; 5120 x 27648, 10 rows (512 tiles instead of 320, two on a quarter of the
-        CUs): 57.6 / 61.2 / 68.9 against 54.1 / 52.6 / 56.1; 2048 x 11008, 8 rows (256 tiles instead of 128):
-        12.3 / 13.5 / 15.5 against 12.1 / 12.6 / 13.7.  Where the busiest CU pulls less W (fewer rounds, or
-        idle CUs put to work at half the tile) the lower tiles win from one row on; where only the re-read
+        CUs): 57.6 / 61.2 / 68.9 against 54.1 / 52.6 / 56.1.  Where the busiest CU pulls less W (fewer rounds, or
+        idle CUs put to work at a lower tile) the lower tiles win from one row on; where only the re-read
         of x per tile of W shrinks (3584), from 8 rows on: below, HBM is the limit, and it streams tiles of
         1 KB a k-step a little faster.  (Timed with x in plain rows; with x laid out by k-step, as the engine
         hands it over, the 3584 case gains nothing end to end, which is why the default minimum gain leaves
-        it at 16 rows.)"""
+        it at 16 rows.  ``prepare_weight`` does not ask about matrices of which halves of tiles of 16 rows go round the CUs once:
+        those are as many workgroups.)"""
         def busiest(th, x):
             return -(-(-(-N // th)) // self._num_cus) * (th + x)
         # (a tile is one sum of squares a row for the products that read the stream next: the kernel that keeps
